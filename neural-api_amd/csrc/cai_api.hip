@@ -60,6 +60,17 @@ int ensure_stage(void** p, size_t* cap, size_t need)
   return CAI_OK;
 }
 
+int ensure_host_stage(size_t need)
+{
+  if (g_ctx.h_stage_cap >= need) return CAI_OK;
+  CAI_HIP(hipStreamSynchronize(g_ctx.stream));
+  if (g_ctx.h_stage) { (void)hipHostFree(g_ctx.h_stage); g_ctx.h_stage = nullptr; g_ctx.h_stage_cap = 0; }
+  const size_t want = need < (1u << 16) ? (1u << 16) : need;
+  CAI_HIP(hipHostMalloc(&g_ctx.h_stage, want, hipHostMallocDefault));
+  g_ctx.h_stage_cap = want;
+  return CAI_OK;
+}
+
 int64_t block_elems(int qt)
 {
   switch (qt) { case CAI_F32: case CAI_F16: case CAI_BF16: case CAI_I8ROW: return 1; case CAI_Q4_0: case CAI_Q8_0: return 32; case CAI_Q4_K: case CAI_Q6_K: return 256; }
@@ -118,6 +129,7 @@ extern "C" int cai_shutdown(void)
   nb_release(); ra_release(); prefill_release(); bf16_release();
   if (c.d_small) (void)hipFree(c.d_small);
   if (c.h_small) (void)hipHostFree(c.h_small);
+  if (c.h_stage) (void)hipHostFree(c.h_stage);
   if (c.tl.buf) (void)hipFree(c.tl.buf);
   (void)hipEventDestroy(c.ev0); (void)hipEventDestroy(c.ev1);
   (void)hipStreamDestroy(c.stream);

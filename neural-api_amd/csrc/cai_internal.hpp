@@ -23,6 +23,7 @@ struct Context {
   void*  stage_in = nullptr;  size_t stage_in_cap = 0;
   void*  stage_out = nullptr; size_t stage_out_cap = 0;
   void*  stage_sample = nullptr; size_t stage_sample_cap = 0;   // a host logits row on its way to cai_sample_candidates
+  void*  h_stage = nullptr; size_t h_stage_cap = 0;      // pinned host memory of calls that wait for their results (kernels read and write it in place)
   int32_t* d_small = nullptr;            // 1024 ints of device scratch for small arguments/results
   int32_t* h_small = nullptr;            // 1024 ints of pinned host memory paired with d_small
   // Step timeline (measurement aid, cai_decoder_timeline): while armed, every instrumented launch gets a record of eight
@@ -68,6 +69,7 @@ struct ApiLock { ApiLock(); ~ApiLock(); ApiLock(const ApiLock&) = delete; ApiLoc
 int  set_error(int code, const char* fmt, ...);
 int  hip_fail(hipError_t e, const char* what, const char* file, int line);
 int  ensure_stage(void** p, size_t* cap, size_t need);
+int  ensure_host_stage(size_t need);   // grows ctx().h_stage; only for calls that do not return before the stream is done with it
 
 #define CAI_HIP(call)                                                        \
   do {                                                                       \

@@ -68,3 +68,38 @@ def test_session_candidates_read_the_resident_row():
     # greedy agreement: the first candidate of the plain row is the arg-max the step reported
     am, lg = dec.step([7, 8], [4, 4])
     assert dec.candidates(1, row=0)[0][0] == am[0] and dec.candidates(1, row=1)[0][0] == am[1]
+
+
+@pytest.mark.parametrize("n", [1, 255, 1024, 1025, 262144, 262145, 300001])
+def test_slices_of_a_row(n):
+    """rows that end inside a slice, fill slices exactly, fill all 256 of them, and need longer ones; m where the values in reach are
+    ranked directly (64) and near the limit (1024)"""
+    from helpers.device import dev
+    cai = dev()
+    rng = np.random.default_rng(n)
+    logits = (rng.standard_normal(n) * 3).astype(np.float32)
+    hist = rng.integers(0, n, 200).tolist()
+    for m in (64, 1024):
+        for kw in (dict(), dict(temperature=0.8, history=hist, repetition=1.2, presence=0.1)):
+            check(cai.sample_candidates(logits, m, **kw), O.sample_candidates(logits, m, **kw))
+
+
+def test_more_equal_values_than_are_ranked_directly():
+    """5000 equal values in reach: the m-th largest is found bit by bit; quotients that underflow; rows with infinities and NaN"""
+    from helpers.device import dev
+    cai = dev()
+    logits = np.full(60000, -3.0, np.float32)
+    tied = np.random.default_rng(1).permutation(60000)[:5000]
+    logits[tied] = 2.0; logits[59999] = 2.5; logits[31] = 2.25
+    for kw in (dict(), dict(temperature=0.7), dict(history=[31, 59999], presence=0.5)):
+        check(cai.sample_candidates(logits, 1000, **kw), O.sample_candidates(logits, 1000, **kw))
+    tok, p = cai.sample_candidates(logits, 300)
+    np.testing.assert_array_equal(tok, np.concatenate([[59999, 31], np.setdiff1d(np.sort(tied), [31, 59999])])[:300])
+    steep = np.full(20000, -200.0, np.float32); steep[::40] = -0.001 * np.arange(500)     # the m-th largest is a zero: every value is in reach
+    check(cai.sample_candidates(steep, 900, temperature=0.5), O.sample_candidates(steep, 900, temperature=0.5))
+    low = np.full(5000, -np.inf, np.float32); low[[7, 4321]] = 1.0
+    tok, p = cai.sample_candidates(low, 4)
+    np.testing.assert_array_equal(tok, [7, 4321, 0, 1]); np.testing.assert_array_equal(p, [0.5, 0.5, 0, 0])
+    low[100] = np.nan                                                # counts as far below the maximum
+    tok, p = cai.sample_candidates(low, 4, temperature=0.9)
+    np.testing.assert_array_equal(tok[:2], [7, 4321]); np.testing.assert_allclose(p[:2], 0.5, rtol=1e-6)
