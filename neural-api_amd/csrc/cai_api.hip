@@ -385,6 +385,7 @@ extern "C" int cai_ffn_gateup(cai_qw_t w, const float* x, const float* gain, flo
   CAI_REQUIRE(w && x && y, "cai_ffn_gateup: null argument");
   CAI_REQUIRE(n_b >= 1 && n_b <= 8, "cai_ffn_gateup: n_b %d outside 1..8", n_b);
   CAI_REQUIRE(w->rows % 2 == 0, "cai_ffn_gateup: %lld rows is not an up|gate pair", (long long)w->rows);
+  if (raw_block_type(w->qtype) && w->qtype != CAI_Q5_K) return set_error(CAI_ERR_UNSUPPORTED, "cai_ffn_gateup: weight type %d", w->qtype);   // (the decoder's batch-1 step alone fuses these)
   Context& c = ctx();
   const int64_t I = w->rows / 2;
   const size_t xb = (size_t)n_b * w->cols * 4, gb = gain ? (size_t)w->cols * 4 : 0, yb = (size_t)n_b * I * 4;

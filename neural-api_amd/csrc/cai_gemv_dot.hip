@@ -1,6 +1,6 @@
 // Persistent streaming matrix-vector kernel for batch-1 decode on gfx950, integer-dot form: Q4_K, and with other requests and
-// block arithmetic in the same walk Q5_K (stored super-blocks), Q4_0 (quants and scales planes) and Q6_K (ql|qh records +
-// planes of scales and d).
+// block arithmetic in the same walk Q5_K (stored super-blocks), Q4_0 (quants and scales planes), Q6_K (ql|qh records +
+// planes of scales and d) and the stored streams of Q2_K, Q3_K, Q4_1, Q5_0 and Q5_1.
 //
 // The weights of a Q4_K sub-block are 4-bit integers with one float scale, so dot(W[a], X) splits into an exact
 // integer part and a handful of float operations per 32 weights once X is held as integers too.  Each
@@ -29,12 +29,40 @@ namespace {
 
 struct Q4kRegs { uint4 h, q0, q1; };
 struct Q5kRegs { uint4 h, q0, q1, e0, e1; };   // Q5_K: + the 32 bytes of the fifth-bit plane (neural/neuralgguf.pas:516-587)
-template <int QT> constexpr int dot_rec_bytes() { return QT == CAI_Q6_K ? 192 : QT == CAI_Q4_0 ? 128 : QT == CAI_Q5_K ? 176 : 144; }
+// Stored streams read as they are, two 32-weight blocks or a quarter of a super-block per lane.  Q3_K blocks of 110 bytes lie at
+// even addresses only: their 16-byte requests are unaligned, which global memory takes (and which costs less than the padding or the
+// narrower requests would: 110 of 112 bytes are used either way).
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef u32x4 __attribute__((aligned(2))) u32x4_a2;
+typedef u32x4 __attribute__((aligned(4))) u32x4_a4;
+typedef u32x3 __attribute__((aligned(4))) u32x3_a4;
+typedef u32x2 __attribute__((aligned(4))) u32x2_a4;
+struct Q3kRegs { u32x4 h0, h1, q0, q1, t; };
+struct Q2kRegs { u32x4 q0, q1; uint32_t sc, dm; };
+struct Q41Regs { u32x4 a, b; u32x2 c; };
+struct Q50Regs { u32x4 a, b; u32x3 c; };
+struct Q51Regs { u32x4 a, b, c; };
+template <int QT> constexpr bool dot_stream() { return QT == CAI_Q2_K || QT == CAI_Q3_K || QT == CAI_Q4_1 || QT == CAI_Q5_0 || QT == CAI_Q5_1; }
+// bytes of 256 weights in the plane the lanes walk
+template <int QT> constexpr int dot_rec_bytes()
+{
+  return QT == CAI_Q6_K ? 192 : QT == CAI_Q4_0 ? 128 : QT == CAI_Q5_K ? 176 : QT == CAI_Q3_K ? 110 : QT == CAI_Q2_K ? 84 : QT == CAI_Q4_1 ? 160 : QT == CAI_Q5_0 ? 176 : QT == CAI_Q5_1 ? 192 : 144;
+}
+// four bits (elements 4w .. 4w + 3 of a block) -> bit 4 of four bytes
+__device__ __forceinline__ uint32_t spread_fifth(uint32_t qh, int w) { return __umul24((qh >> (4 * w)) & 15u, 0x204081u) << 4 & 0x10101010u; }
 
 // LDS slot (in uint4) of the t-th uint4 (t = 0..15) of unit u (64 activations): tiles of 16 units, transposed
 __device__ __forceinline__ int xq_slot(int u, int t) { return (u >> 4) * 256 + t * 16 + (u & 15); }
 
 constexpr float XQ_MAX = 4194303.0f;          // 2^22 - 1
+// The stored streams take the whole range of three balanced digits (127 * (1 + 256 + 65536), less the rounding of the quotient): their
+// 16-weight sums fit 32 bits all the same (16 * 16 * 8355711), and the rounding of the activations is half as large, 2^-24 of the
+// 32-block maximum: 1.4e-7 off 64 bits over widths of 2048 to 5120, the float walk (gemv_raw) 1.1e-7 to 1.7e-7.
+// 18944 x 3584 against that walk, which spends 12 to 25 vector instructions on a weight (here 2 to 2.5): Q3_K 39.2 -> 12.0 us,
+// Q2_K 18.6 -> 10.8, Q4_1 17.8 -> 9.3, Q5_0 27.0 -> 10.9, Q5_1 22.1 -> 10.9; 2048 x 2048 5.0..7.9 -> 4.3.
+constexpr float XQ_MAX_STREAM = 8355710.0f;
 constexpr int NL = 3;                         // balanced base-256 digits per activation
 
 __device__ __forceinline__ float quad_max(float v)
@@ -68,13 +96,13 @@ __device__ __forceinline__ float group_sum(float v)
   return v;
 }
 
-// four rounded activations (as float bit patterns of x*inv + 1.5*2^23) -> one dword per digit
-__device__ __forceinline__ void pack_digits(const float (&f)[4], int (&d)[NL])
+// four rounded activations -> one dword per digit
+__device__ __forceinline__ void pack_digits(const int (&q)[4], int (&d)[NL])
 {
   uint32_t e[4];
 #pragma unroll
   for (int i = 0; i < 4; i++)   // integer value + 0x808080, then flip the digit sign bits: bytes are balanced digits
-    e[i] = (__builtin_bit_cast(uint32_t, f[i]) + (0x00808080u - 0x4B400000u)) ^ 0x00808080u;
+    e[i] = ((uint32_t)q[i] + 0x00808080u) ^ 0x00808080u;
   const uint32_t p01 = __builtin_amdgcn_perm(e[1], e[0], 0x05010400u), p23 = __builtin_amdgcn_perm(e[3], e[2], 0x05010400u);
   const uint32_t h01 = __builtin_amdgcn_perm(e[1], e[0], 0x06020602u), h23 = __builtin_amdgcn_perm(e[3], e[2], 0x06020602u);
   d[0] = (int)__builtin_amdgcn_perm(p23, p01, 0x05040100u);
@@ -90,6 +118,14 @@ __device__ __forceinline__ void pack_digits(const float (&f)[4], int (&d)[NL])
 // 32-byte ql runs and two of the four 2-bit fields of the 32 qh bytes.  Codes 0..63 go to v_dot4 as they are; the - 32
 // offset uses the sums of the lane's integer activations per 16, taken once; each 16 weights have their own scale.
 struct Q6kRegs { uint4 a0, a1, b0, b1, h0, h1; uint2 sc; uint32_t d; };
+template <int QT> struct DotRegs { using type = Q4kRegs; };
+template <> struct DotRegs<CAI_Q5_K> { using type = Q5kRegs; };
+template <> struct DotRegs<CAI_Q6_K> { using type = Q6kRegs; };
+template <> struct DotRegs<CAI_Q3_K> { using type = Q3kRegs; };
+template <> struct DotRegs<CAI_Q2_K> { using type = Q2kRegs; };
+template <> struct DotRegs<CAI_Q4_1> { using type = Q41Regs; };
+template <> struct DotRegs<CAI_Q5_0> { using type = Q50Regs; };
+template <> struct DotRegs<CAI_Q5_1> { using type = Q51Regs; };
 
 // PK > 1 packs PK rows into one wave: a wave then holds 16 / PK super-blocks of PK different row-group streams (lane
 // quarter-groups of 64 / PK lanes), so a width that is not a multiple of 4096 columns leaves no lanes idle - 5120 columns
@@ -132,7 +168,7 @@ __device__ __forceinline__ void gemv_dot_body(const GemvParams& p, const DotHot 
   const int g_first = blockIdx.x * gwv + gslot, g_stride = a.grid * gwv;
   const int n_iters = (n_groups + g_stride - 1) / g_stride;
   const int64_t lane_off = (int64_t)(act ? sb : 0) * dot_rec_bytes<QT>();
-  using WRegs = typename std::conditional<QT == CAI_Q6_K, Q6kRegs, typename std::conditional<QT == CAI_Q5_K, Q5kRegs, Q4kRegs>::type>::type;
+  using WRegs = typename DotRegs<QT>::type;
 
   // group -> segment, first row of the group inside the segment
   auto locate = [&](int g, const GemvSeg*& sg, int& row0) {
@@ -151,7 +187,7 @@ __device__ __forceinline__ void gemv_dot_body(const GemvParams& p, const DotHot 
       if (p.n_seg > 2 && g >= p.seg[1].grp_end) { s = 2; g0 = p.seg[1].grp_end; }
     }
     data = (!MULTISEG || s == 0) ? a.w0 : p.seg[s].data;
-    if (QT == CAI_Q4_K || QT == CAI_Q5_K) aux = nullptr; else aux = p.seg[s].aux;
+    if (QT == CAI_Q4_K || QT == CAI_Q5_K || dot_stream<QT>()) aux = nullptr; else aux = p.seg[s].aux;
     rows = (!MULTISEG || s == 0) ? a.rows0 : p.seg[s].rows;
     row0 = (g - g0) * R;
   };
@@ -203,6 +239,24 @@ __device__ __forceinline__ void gemv_dot_body(const GemvParams& p, const DotHot 
         rg[r].e0 = *reinterpret_cast<const uint4*>(blk + 16); rg[r].e1 = *reinterpret_cast<const uint4*>(blk + 32);
         rg[r].q0 = *reinterpret_cast<const uint4*>(blk + 48 + 32 * cc);
         rg[r].q1 = *reinterpret_cast<const uint4*>(blk + 64 + 32 * cc);
+      } else if constexpr (QT == CAI_Q3_K) {
+        // mask bytes 0..31 (all four lanes), the 32 two-bit bytes of the lane's half, and the last 16 bytes: two of the half's quants,
+        // twelve of scales, d
+        rg[r].h0 = *reinterpret_cast<const u32x4_a2*>(blk);      rg[r].h1 = *reinterpret_cast<const u32x4_a2*>(blk + 16);
+        rg[r].q0 = *reinterpret_cast<const u32x4_a2*>(blk + 32 + 32 * (cc >> 1)); rg[r].q1 = *reinterpret_cast<const u32x4_a2*>(blk + 48 + 32 * (cc >> 1));
+        rg[r].t = *reinterpret_cast<const u32x4_a2*>(blk + 94);
+      } else if constexpr (QT == CAI_Q2_K) {
+        rg[r].sc = *reinterpret_cast<const uint32_t*>(blk + 4 * cc); rg[r].dm = *reinterpret_cast<const uint32_t*>(blk + 80);
+        rg[r].q0 = *reinterpret_cast<const u32x4_a4*>(blk + 16 + 32 * (cc >> 1)); rg[r].q1 = *reinterpret_cast<const u32x4_a4*>(blk + 32 + 32 * (cc >> 1));
+      } else if constexpr (QT == CAI_Q4_1) {   // two blocks of {d, m, 16 bytes}
+        rg[r].a = *reinterpret_cast<const u32x4_a4*>(blk + 40 * cc); rg[r].b = *reinterpret_cast<const u32x4_a4*>(blk + 40 * cc + 16);
+        rg[r].c = *reinterpret_cast<const u32x2_a4*>(blk + 40 * cc + 32);
+      } else if constexpr (QT == CAI_Q5_0) {   // two blocks of {d, four bytes of fifth bits, 16 bytes}
+        rg[r].a = *reinterpret_cast<const u32x4_a4*>(blk + 44 * cc); rg[r].b = *reinterpret_cast<const u32x4_a4*>(blk + 44 * cc + 16);
+        rg[r].c = *reinterpret_cast<const u32x3_a4*>(blk + 44 * cc + 32);
+      } else if constexpr (QT == CAI_Q5_1) {   // two blocks of {d, m, four bytes of fifth bits, 16 bytes}
+        rg[r].a = *reinterpret_cast<const u32x4_a4*>(blk + 48 * cc); rg[r].b = *reinterpret_cast<const u32x4_a4*>(blk + 48 * cc + 16);
+        rg[r].c = *reinterpret_cast<const u32x4_a4*>(blk + 48 * cc + 32);
       } else {
         rg[r].h = *reinterpret_cast<const uint4*>(blk);
         rg[r].q0 = *reinterpret_cast<const uint4*>(blk + 16 + 32 * cc);
@@ -299,15 +353,21 @@ __device__ __forceinline__ void gemv_dot_body(const GemvParams& p, const DotHot 
       const bool ok = m > 0.0f && m < 3.0e38f;           // an all-zero block contributes 0
       // 0 for finite values, NaN when the eight hold an inf or a NaN: carried into the scale so the outputs show it
       const float poison = (((v0.x + v0.y) + (v0.z + v0.w)) + ((v1.x + v1.y) + (v1.z + v1.w))) * 0.0f;
-      const float inv = ok ? XQ_MAX / m : 0.0f, s = ok ? m * (1.0f / XQ_MAX) : 0.0f;
-      const float fa[4] = {fmaf(v0.x, inv, 12582912.0f), fmaf(v0.y, inv, 12582912.0f), fmaf(v0.z, inv, 12582912.0f), fmaf(v0.w, inv, 12582912.0f)};
-      const float fb[4] = {fmaf(v1.x, inv, 12582912.0f), fmaf(v1.y, inv, 12582912.0f), fmaf(v1.z, inv, 12582912.0f), fmaf(v1.w, inv, 12582912.0f)};
-      int da[NL], db[NL];
-      pack_digits(fa, da); pack_digits(fb, db);
-      int isum = 0;
+      constexpr float QM = dot_stream<QT>() ? XQ_MAX_STREAM : XQ_MAX;
+      const float inv = ok ? QM / m : 0.0f, s = ok ? m * (1.0f / QM) : 0.0f;
+      const float va[4] = {v0.x, v0.y, v0.z, v0.w}, vb[4] = {v1.x, v1.y, v1.z, v1.w};
+      int qa[4], qb[4], isum = 0;
 #pragma unroll
-      for (int i = 0; i < 4; i++)
-        isum += (int)(__builtin_bit_cast(uint32_t, fa[i]) - 0x4B400000u) + (int)(__builtin_bit_cast(uint32_t, fb[i]) - 0x4B400000u);
+      for (int i = 0; i < 4; i++) {
+        if constexpr (dot_stream<QT>()) { qa[i] = (int)rintf(va[i] * inv); qb[i] = (int)rintf(vb[i] * inv); }
+        else {   // up to 2^22 the addition of 1.5 * 2^23 rounds
+          qa[i] = (int)(__builtin_bit_cast(uint32_t, fmaf(va[i], inv, 12582912.0f)) - 0x4B400000u);
+          qb[i] = (int)(__builtin_bit_cast(uint32_t, fmaf(vb[i], inv, 12582912.0f)) - 0x4B400000u);
+        }
+        isum += qa[i] + qb[i];
+      }
+      int da[NL], db[NL];
+      pack_digits(qa, da); pack_digits(qb, db);
       isum = quad_sum(isum);
       // n = [unit][half:1][j:2]: the unit's record holds per digit 4 uint4 (2 per 32-block), then one uint4 of
       // {scale A, scale B, s*sum A, s*sum B}
@@ -352,8 +412,9 @@ __device__ __forceinline__ void gemv_dot_body(const GemvParams& p, const DotHot 
       for (int t = 0; t < 16; t++) xq[L][t] = 0;
   }
 
-  float s16[4] = {0.0f, 0.0f, 0.0f, 0.0f};   // Q6_K: the lane's integer activations summed per 16 (first / second 32: groups 0, 1 / 2, 3)
-  if constexpr (QT == CAI_Q6_K) {
+  float s16[4] = {0.0f, 0.0f, 0.0f, 0.0f};   // the lane's integer activations summed per 16 (first / second 32: groups 0, 1 / 2, 3)
+  int i16[4] = {0, 0, 0, 0};
+  if constexpr (QT == CAI_Q6_K || dot_stream<QT>()) {
 #pragma unroll
     for (int gq = 0; gq < 4; gq++) {
       int tot = 0;
@@ -364,7 +425,7 @@ __device__ __forceinline__ void gemv_dot_body(const GemvParams& p, const DotHot 
         for (int w = 0; w < 4; w++) t = __builtin_amdgcn_sdot4(0x01010101, xq[L][4 * gq + w], t, false);
         tot += t << (8 * L);
       }
-      s16[gq] = (float)tot;
+      s16[gq] = (float)tot; i16[gq] = tot;
     }
   }
   timeline_stamp(p.timeline, 4);
@@ -430,6 +491,73 @@ __device__ __forceinline__ void gemv_dot_body(const GemvParams& p, const DotHot 
           const float dA = __half2float(__ushort_as_half((unsigned short)(cur[r].h.x & 0xffffu)));
           const float dB = __half2float(__ushort_as_half((unsigned short)(cur[r].h.x >> 16)));
           acc[r] = dA * fmaf(sA, fa, -8.0f * mA) + dB * fmaf(sB, fb, -8.0f * mB);
+          continue;
+        } else if constexpr (dot_stream<QT>()) {
+          // exact sums of (code - OFFSET) * activation per 16, for Q2_K of (2 code - 3) * activation.  The offset of a type with minima is the
+          // middle of its codes: what the minimum then still adds is small, where a sum of bare codes and its minimum would cancel
+          // (error of Q4_1 against 64 bits 2.6e-7 with bare codes, 1.4e-7 so).
+          constexpr int OFFSET = QT == CAI_Q3_K ? 4 : QT == CAI_Q4_1 ? 8 : QT == CAI_Q2_K ? 3 : 16;
+          float f[4];
+          auto code = [&](int gq, int w) -> uint32_t {      // four codes
+            if constexpr (QT == CAI_Q3_K || QT == CAI_Q2_K) {
+              const uint32_t q = ((gq & 1) ? cur[r].q1[w] : cur[r].q0[w]) >> (4 * (cc & 1));
+              uint32_t c = (gq < 2 ? q : q >> 2) & 0x03030303u;
+              if constexpr (QT == CAI_Q3_K) {               // a clear mask bit stands for - 4
+                const uint32_t h = ((gq & 1) ? cur[r].h1[w] : cur[r].h0[w]) >> (2 * cc);
+                c |= (gq < 2 ? h << 2 : h << 1) & 0x04040404u;
+              }
+              return c;
+            } else {
+              uint32_t q, e = 0;
+              const bool first = gq < 2;
+              if constexpr (QT == CAI_Q4_1) {
+                q = first ? (w == 0 ? cur[r].a.y : w == 1 ? cur[r].a.z : w == 2 ? cur[r].a.w : cur[r].b.x)
+                          : (w == 0 ? cur[r].b.z : w == 1 ? cur[r].b.w : w == 2 ? cur[r].c.x : cur[r].c.y);
+              } else if constexpr (QT == CAI_Q5_0) {        // the first block's bytes start in the middle of a dword
+                const uint32_t lo = w == 0 ? cur[r].a.y : w == 1 ? cur[r].a.z : w == 2 ? cur[r].a.w : cur[r].b.x, hi = w == 0 ? cur[r].a.z : w == 1 ? cur[r].a.w : w == 2 ? cur[r].b.x : cur[r].b.y;
+                q = first ? __builtin_amdgcn_alignbit(hi, lo, 16) : (w == 0 ? cur[r].b.w : w == 1 ? cur[r].c.x : w == 2 ? cur[r].c.y : cur[r].c.z);
+                e = first ? __builtin_amdgcn_alignbit(cur[r].a.y, cur[r].a.x, 16) : cur[r].b.z;
+              } else {
+                q = first ? (w == 0 ? cur[r].a.z : w == 1 ? cur[r].a.w : w == 2 ? cur[r].b.x : cur[r].b.y)
+                          : (w == 0 ? cur[r].c.x : w == 1 ? cur[r].c.y : w == 2 ? cur[r].c.z : cur[r].c.w);
+                e = first ? cur[r].a.y : cur[r].b.w;
+              }
+              const uint32_t c = ((gq & 1) ? q >> 4 : q) & 0x0f0f0f0fu;
+              return QT == CAI_Q4_1 ? c : c | spread_fifth(e, 4 * (gq & 1) + w);
+            }
+          };
+#pragma unroll
+          for (int gq = 0; gq < 4; gq++) {
+            int dg[NL];
+#pragma unroll
+            for (int L = 0; L < NL; L++) dg[L] = 0;
+#pragma unroll
+            for (int w = 0; w < 4; w++) {
+              const int c = (int)code(gq, w);
+#pragma unroll
+              for (int L = 0; L < NL; L++) dg[L] = __builtin_amdgcn_sdot4(c, xq[L][4 * gq + w], dg[L], false);
+            }
+            // (unsigned: the sum of the bare codes may wrap, what is left after the offset fits)
+            const uint32_t tot = (uint32_t)dg[0] + ((uint32_t)dg[1] << 8) + ((uint32_t)dg[2] << 16);
+            f[gq] = (float)(int)((QT == CAI_Q2_K ? 2u * tot : tot) - (uint32_t)OFFSET * (uint32_t)i16[gq]);
+          }
+          auto half_of = [](uint32_t v) { return __half2float(__ushort_as_half((unsigned short)(v & 0xffffu))); };
+          if constexpr (QT == CAI_Q3_K) {
+            const uint32_t s0 = __builtin_amdgcn_alignbit(cur[r].t.y, cur[r].t.x, 16), s1 = __builtin_amdgcn_alignbit(cur[r].t.z, cur[r].t.y, 16), s2 = __builtin_amdgcn_alignbit(cur[r].t.w, cur[r].t.z, 16);
+            const uint32_t sc = ((((cc & 1) ? s1 : s0) >> (4 * (cc >> 1))) & 0x0f0f0f0fu) | (((s2 >> (2 * cc)) & 0x03030303u) << 4);
+            acc[r] = half_of(cur[r].t.w >> 16) * (sA * ((cvt_ub0(sc) - 32.0f) * f[0] + (cvt_ub1(sc) - 32.0f) * f[1]) + sB * ((cvt_ub2(sc) - 32.0f) * f[2] + (cvt_ub3(sc) - 32.0f) * f[3]));
+          } else if constexpr (QT == CAI_Q2_K) {
+            const uint32_t sc = cur[r].sc & 0x0f0f0f0fu, mn = (cur[r].sc >> 4) & 0x0f0f0f0fu;
+            const float d = half_of(cur[r].dm), dmin = half_of(cur[r].dm >> 16), d15 = 1.5f * d;
+            acc[r] = (0.5f * d) * (sA * (cvt_ub0(sc) * f[0] + cvt_ub1(sc) * f[1]) + sB * (cvt_ub2(sc) * f[2] + cvt_ub3(sc) * f[3])) +
+                     sA * (fmaf(d15, cvt_ub0(sc), -dmin * cvt_ub0(mn)) * s16[0] + fmaf(d15, cvt_ub1(sc), -dmin * cvt_ub1(mn)) * s16[1]) +
+                     sB * (fmaf(d15, cvt_ub2(sc), -dmin * cvt_ub2(mn)) * s16[2] + fmaf(d15, cvt_ub3(sc), -dmin * cvt_ub3(mn)) * s16[3]);
+          } else {
+            const uint32_t ha = cur[r].a.x, hb = QT == CAI_Q4_1 ? cur[r].b.y : QT == CAI_Q5_0 ? cur[r].b.y >> 16 : cur[r].b.z;
+            const float dA = half_of(ha), dB = half_of(hb);
+            acc[r] = dA * (sA * (f[0] + f[1])) + dB * (sB * (f[2] + f[3]));
+            if constexpr (QT != CAI_Q5_0) acc[r] += fmaf((float)OFFSET, dA, half_of(ha >> 16)) * mA + fmaf((float)OFFSET, dB, half_of(hb >> 16)) * mB;
+          }
           continue;
         } else if constexpr (QT == CAI_Q5_K) {
           // code = nibble | bit << 4 (0..31): bit 2 cc of plane byte i belongs to weight i of the first 32, bit 2 cc + 1 to the second
@@ -632,6 +760,13 @@ __global__ __launch_bounds__(768, 3) void gemv_q5k_dot(DOT_HOT_ARGS, const GemvP
   gemv_dot_body<R, MODE, MULTISEG, NS, CAI_Q5_K, PK>(p, DOT_HOT_PACK);
 }
 
+template <int QT, int MODE, bool MULTISEG, int PK>
+__global__ __launch_bounds__(768, 3) void gemv_stream_dot(DOT_HOT_ARGS, const GemvParams p)
+{
+  // (two gate|up pairs of Q3_K in flight are 80 registers beside the 48 of the activations: they would spill)
+  gemv_dot_body<1, MODE, MULTISEG, MODE == 1 && QT == CAI_Q3_K ? 1 : 2, QT, PK>(p, DOT_HOT_PACK);
+}
+
 template <int R, int NS>
 __global__ __launch_bounds__(768, 3) void gemv_q6k_dot(DOT_HOT_ARGS, const GemvParams p)
 {
@@ -680,7 +815,8 @@ int launch_q4k_dot(GemvParams& p, const MultiGemv& m, int swiglu_half, hipStream
     if (nsw < 3 || 2 * turns2 <= turns1) R = 2;
     if (packed) R = 2;
   }
-  if (q6k) R = 1;   // (two rows of Q6_K requests in flight twice over do not fit the registers)
+  const bool stream = raw_block_type(m.w[0]->qtype) && m.w[0]->qtype != CAI_Q5_K;
+  if (q6k || stream) R = 1;   // (two rows of Q6_K requests in flight twice over do not fit the registers; the stored streams spend longer on a row than it takes to arrive)
   int cum = 0;
   for (int i = 0; i < m.n; i++) {
     const int64_t rows = swiglu_half ? swiglu_half : m.rows[i];
@@ -717,6 +853,25 @@ int launch_q4k_dot(GemvParams& p, const MultiGemv& m, int swiglu_half, hipStream
     else if (m.n > 1) { if (R == 2) go(gemv_q4k_dot<2, 0, true, NSV, PKV>); else go(gemv_q4k_dot<1, 0, true, NSV, PKV>); }
     else { if (R == 2) go(gemv_q4k_dot<2, 0, false, NSV, PKV>); else go(gemv_q4k_dot<1, 0, false, NSV, PKV>); }
   };
+  auto pick_stream = [&](auto qt, auto pk) {
+    constexpr int Q = decltype(qt)::value, PKV = decltype(pk)::value;
+    if (swiglu_half) go(gemv_stream_dot<Q, 1, false, PKV>);
+    else if (m.n > 1) go(gemv_stream_dot<Q, 0, true, PKV>);
+    else go(gemv_stream_dot<Q, 0, false, PKV>);
+  };
+  if (stream) {
+    auto type = [&](auto pk) {
+      switch (m.w[0]->qtype) {
+        case CAI_Q2_K: pick_stream(std::integral_constant<int, CAI_Q2_K>(), pk); break;
+        case CAI_Q3_K: pick_stream(std::integral_constant<int, CAI_Q3_K>(), pk); break;
+        case CAI_Q4_1: pick_stream(std::integral_constant<int, CAI_Q4_1>(), pk); break;
+        case CAI_Q5_0: pick_stream(std::integral_constant<int, CAI_Q5_0>(), pk); break;
+        default: pick_stream(std::integral_constant<int, CAI_Q5_1>(), pk); break;
+      }
+    };
+    if (packed) type(std::integral_constant<int, PKW>()); else type(std::integral_constant<int, 1>());
+    return CAI_OK;
+  }
   auto pick = [&](auto ns) {
     constexpr int NSV = decltype(ns)::value;
     if (q6k) go(gemv_q6k_dot<1, NSV>);

@@ -74,6 +74,46 @@ def test_gemv_widths_that_are_not_whole_super_blocks(qt, rows, cols):
     w.close()
 
 
+@pytest.mark.parametrize("qt", RAW[1:])
+@pytest.mark.parametrize("rows,cols", [(5, 32768), (6, 33024)])
+def test_gemv_at_the_widest_integer_dot_row_and_past_it(qt, rows, cols):
+    """eight slices of sixteen super-blocks, and one super-block more (the float walk); block bytes of any pattern, one activation far
+    above its block"""
+    from helpers.device import dev, rel_err
+    from test_oracle_codecs_other import random_blocks
+    cai = dev()
+    rng = np.random.default_rng(cols + qt)
+    raw = random_blocks(qt, rows * cols // (256 if qt in (O.Q2_K, O.Q3_K) else 32), seed=50 + qt).reshape(-1)
+    x = rng.standard_normal((1, cols)).astype(np.float32)
+    x[0, 100] = 50.0
+    w = cai.QWeight(qt, rows, cols, raw)
+    want = O.gemv(qt, raw, rows, cols, x, None, 0, 1)
+    assert rel_err(w.gemv(x), want, floor=float(np.abs(O.dequant(qt, raw, rows * cols)).max()) * cols ** 0.5) < TIGHT
+    x[0, 7] = np.nan
+    assert np.isnan(w.gemv(x)).all()
+    w.close()
+    if cols == 32768:
+        w = cai.QWeight(qt, 6, 256, raw[:raw.size * 6 * 256 // (rows * cols)])
+        with pytest.raises(cai.CaiError):                    # fused gate|up by itself stays refused for these types
+            w.ffn_gateup(np.ones((1, 256), np.float32))
+        w.close()
+
+
+@pytest.mark.parametrize("qt", RAW[1:])
+def test_decoder_of_a_stored_stream_type(qt):
+    """the fused walks of a decoding step: q|k|v in one launch, gate|up with norm and SwiGLU, the sums of squares handed on"""
+    from helpers.device import dev, rel_err
+    cai = dev()
+    cfg = dict(n_layers=2, d_model=512, n_q_heads=6, n_kv_heads=2, head_dim=128, ffn=1280, vocab=300, max_ctx=64, eps=1e-5, rope_theta=1e4)
+    spec = synthetic_spec(cfg, qt, head_qtype=O.Q8_0, seed=qt, std=0.05, qkv_bias=True)
+    om, dec = oracle_model(spec, acc64=1), cai.Decoder(spec)
+    for p, t in enumerate((3, 77, 12)):
+        _, want = om.step(t, p)
+        _, got = dec.step(t, p)
+        assert rel_err(got[0], want) < 1e-4, p
+    dec.close()
+
+
 def test_width_that_splits_a_block_is_refused():
     from helpers.device import dev
     cai = dev()
