@@ -126,7 +126,7 @@ extern "C" int cai_shutdown(void)
   if (c.stage_in) (void)hipFree(c.stage_in);
   if (c.stage_out) (void)hipFree(c.stage_out);
   if (c.stage_sample) (void)hipFree(c.stage_sample);
-  nb_release(); ra_release(); prefill_release(); bf16_release();
+  nb_release(); ra_release(); prefill_release(); wide_release(); bf16_release();
   if (c.d_small) (void)hipFree(c.d_small);
   if (c.h_small) (void)hipHostFree(c.h_small);
   if (c.h_stage) (void)hipHostFree(c.h_stage);

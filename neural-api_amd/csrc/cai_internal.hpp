@@ -314,6 +314,10 @@ int launch_gemm_blk_multi(const cai_qw_s* const* ws, const int* y_off, int n_w, 
 bool prefill_multi_supported(const cai_qw_s* const* ws, int n_w);   // one launch of a prompt kernel takes these matrices together
 int launch_gemm_q4k_multi(const cai_qw_s* const* ws, const int* y_off, int n_w, const _Float16* xhi, const _Float16* xlo, const _Float16* sxhi,
                           const _Float16* sxlo, const float* sinv, int n_tok, float* y, int64_t y_stride, const float* residual, int swiglu_half);
+bool gemm_wide_wanted(const cai_qw_s* w, int64_t rows_all, int n_tok);   // prompt product on wide tiles (cai_prefill_wide.hip)
+int launch_gemm_wide(const cai_qw_s* const* ws, const int* y_off, int n_w, const _Float16* xhi, const _Float16* xlo, const _Float16* sxhi,
+                     const _Float16* sxlo, const float* sinv, int n_tok, float* y, int64_t y_stride, const float* residual, int swiglu_half);
+void wide_release();                                           // frees its buffer of partial sums (cai_shutdown)
 bool prefill_gemm_swiglu_supported(const cai_qw_s* w, int n_tok);
 int prefill_gemm_swiglu(const cai_qw_s* w, int n_tok, float* y, int64_t y_stride);   // y[t][i] = up_i * silu(gate_i), on the planes of the last prefill_prep
 

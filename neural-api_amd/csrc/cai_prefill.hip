@@ -201,7 +201,7 @@ __device__ __forceinline__ half4_t bytes_to_half4_pf(uint32_t t)
 
 typedef _Float16 half8_pf __attribute__((ext_vector_type(8)));
 
-// One work-group: 4 waves x RT row tiles of 32 rows x TT * 32 tokens, one super-block (256 columns) per step, on
+// One work-group: 4 waves x RT row tiles of 32 rows x 32 tokens, one super-block (256 columns) per step, on
 // v_mfma_f32_32x32x16_f16 (lane (n, kg) supplies 8 consecutive k of row / column n).
 //   * the weight operand sc_j * q (<= 63 * 15, exact in f16) is built once per super-block per wave and reused by the
 //     token tiles and by the hi and lo activation planes; the matrix cores accumulate across the whole super-block, hi
@@ -215,10 +215,10 @@ typedef _Float16 half8_pf __attribute__((ext_vector_type(8)));
 // per token tile) hit that XCD's L2.  TT = 1 doubles the number of work-groups for matrices with few row groups.
 // QT = CAI_Q5_K: 176-byte super-blocks (neural/neuralgguf.pas:516-587) - the Q4_K header, the 32-byte plane of fifth bits (bit j of byte i
 // belongs to weight i of sub-block j), the nibbles; the weight operand sc * (nibble | bit << 4) <= 63 * 31 stays exact in f16.
-template <int TT, int RT, int QT>
+template <int RT, int QT>
 __global__ __launch_bounds__(256, 2) void gemm_q4k_pf(const GemmParams p)
 {
-  constexpr int BB = QT == CAI_Q5_K ? 176 : 144, QOFF = QT == CAI_Q5_K ? 48 : 16;
+  constexpr int TT = 1, BB = QT == CAI_Q5_K ? 176 : 144, QOFF = QT == CAI_Q5_K ? 48 : 16;
   extern __shared__ __align__(16) unsigned char pf_smem[];
   constexpr int NTOK = TT * 32;
   _Float16* xs_hi = reinterpret_cast<_Float16*>(pf_smem);            // [NTOK][PF_LDX]
@@ -634,12 +634,13 @@ int launch_gemm_q4k_multi(const cai_qw_s* const* ws, const int* y_off, int n_w, 
   if (n_w > 1 && (!gemm_q4k_multi_supported(ws, n_w) || residual)) return set_error(CAI_ERR_UNSUPPORTED, "prefill gemm: %d matrices in one launch", n_w);
   if (swiglu_half && (n_w != 1 || residual || w->qtype == CAI_Q6_K || w->rows != 2 * (int64_t)swiglu_half))
     return set_error(CAI_ERR_UNSUPPORTED, "prefill gemm: fused SwiGLU needs one Q4_K / Q5_K matrix of 2 x %d rows", swiglu_half);
+  int64_t rows_all = 0;
+  for (int i = 0; i < n_w; i++) rows_all += ws[i]->rows;
+  if (gemm_wide_wanted(w, rows_all, n_tok)) return launch_gemm_wide(ws, y_off, n_w, xhi, xlo, sxhi, sxlo, sinv, n_tok, y, y_stride, residual, swiglu_half);
   GemmParams p{};
   p.w = w->data; p.bias = w->bias; p.rows = (int)w->rows; p.cols = (int)w->cols;
   p.xhi = xhi; p.xlo = xlo; p.sxhi = sxhi; p.sxlo = sxlo; p.sinv = sinv; p.n_tok = n_tok; p.y = y + y_off[0]; p.y_stride = y_stride;
   p.residual = residual; p.n_seg = n_w;
-  int64_t rows_all = 0;
-  for (int i = 0; i < n_w; i++) rows_all += ws[i]->rows;
   if (w->qtype == CAI_Q6_K) {
     p.aux = w->aux; p.aux2 = qw_aux2(w);
     const int tt = ((p.rows + 127) / 128) * ((n_tok + 63) / 64) < 2 * ctx().n_cu ? 1 : 2;
@@ -657,15 +658,12 @@ int launch_gemm_q4k_multi(const cai_qw_s* const* ws, const int* y_off, int n_w, 
     else hipLaunchKernelGGL(gemm_q6k_pf<2>, dim3(grid), dim3(256), lds, ctx().stream, p);
     return CAI_OK;
   }
-  // Tiling: two row tiles per wave (256 rows per work-group, 32 tokens) when that still gives every CU several
-  // work-groups; else 128 rows with two token tiles, or with one for matrices with few row groups.
-  const int n_cu = ctx().n_cu;
-  const int wgs_rt2 = (int)((rows_all + 255) / 256) * ((n_tok + 31) / 32);
-  const int wgs_tt2 = (int)((rows_all + 127) / 128) * ((n_tok + 63) / 64);
+  // Tiling: two row tiles per wave (256 rows per work-group, 32 tokens) when that still gives every CU several work-groups, else one
   // (measured on 512-token chunks: 7168 rows = 448 work-groups of two row tiles 107 us against 121 us with one tile; 5120 rows = 320
   // work-groups lose to 640 of one tile, 3584 rows = 224 likewise)
-  const int mode = (swiglu_half || 4 * wgs_rt2 >= 7 * n_cu) ? 3 : (wgs_tt2 < 2 * n_cu ? 1 : 2);   // 1, 2: token tiles; 3: two row tiles
-  const int rt = mode == 3 ? 2 : 1, tt = mode == 2 ? 2 : 1;
+  const int n_cu = ctx().n_cu;
+  const int wgs_rt2 = (int)((rows_all + 255) / 256) * ((n_tok + 31) / 32);
+  const int rt = (swiglu_half || 4 * wgs_rt2 >= 7 * n_cu) ? 2 : 1;
   p.swiglu_half = swiglu_half;
   p.n_row_groups = 0;
   for (int i = 0; i < n_w; i++) {       // every matrix starts a row group of its own
@@ -673,23 +671,20 @@ int launch_gemm_q4k_multi(const cai_qw_s* const* ws, const int* y_off, int n_w, 
     p.n_row_groups += (int)((ws[i]->rows + 128 * rt - 1) / (128 * rt));
   }
   if (swiglu_half) p.n_row_groups = (swiglu_half + 127) / 128;   // 128 up rows and their gate rows per work-group
-  p.n_tok_tiles = (n_tok + tt * 32 - 1) / (tt * 32);
-  const size_t lds = (size_t)tt * 32 * (PF_LDX + 8) * 2 * 2 + (size_t)4 * rt * 2 * 32 * 4;
+  p.n_tok_tiles = (n_tok + 31) / 32;
+  const size_t lds = (size_t)32 * (PF_LDX + 8) * 2 * 2 + (size_t)4 * rt * 2 * 32 * 4;
   static bool attr_done = false;
   if (!attr_done) {
-    const void* ks[6] = {(const void*)gemm_q4k_pf<1, 1, CAI_Q4_K>, (const void*)gemm_q4k_pf<2, 1, CAI_Q4_K>, (const void*)gemm_q4k_pf<1, 2, CAI_Q4_K>,
-                         (const void*)gemm_q4k_pf<1, 1, CAI_Q5_K>, (const void*)gemm_q4k_pf<2, 1, CAI_Q5_K>, (const void*)gemm_q4k_pf<1, 2, CAI_Q5_K>};
+    const void* ks[4] = {(const void*)gemm_q4k_pf<1, CAI_Q4_K>, (const void*)gemm_q4k_pf<2, CAI_Q4_K>, (const void*)gemm_q4k_pf<1, CAI_Q5_K>, (const void*)gemm_q4k_pf<2, CAI_Q5_K>};
     for (const void* k : ks) if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024) != hipSuccess) (void)hipGetLastError();
     attr_done = true;
   }
   const int grid = 8 * p.n_tok_tiles * ((p.n_row_groups + 7) / 8);
   if (w->qtype == CAI_Q5_K) {
-    if (mode == 3) hipLaunchKernelGGL((gemm_q4k_pf<1, 2, CAI_Q5_K>), dim3(grid), dim3(256), lds, ctx().stream, p);
-    else if (mode == 1) hipLaunchKernelGGL((gemm_q4k_pf<1, 1, CAI_Q5_K>), dim3(grid), dim3(256), lds, ctx().stream, p);
-    else hipLaunchKernelGGL((gemm_q4k_pf<2, 1, CAI_Q5_K>), dim3(grid), dim3(256), lds, ctx().stream, p);
-  } else if (mode == 3) hipLaunchKernelGGL((gemm_q4k_pf<1, 2, CAI_Q4_K>), dim3(grid), dim3(256), lds, ctx().stream, p);
-  else if (mode == 1) hipLaunchKernelGGL((gemm_q4k_pf<1, 1, CAI_Q4_K>), dim3(grid), dim3(256), lds, ctx().stream, p);
-  else hipLaunchKernelGGL((gemm_q4k_pf<2, 1, CAI_Q4_K>), dim3(grid), dim3(256), lds, ctx().stream, p);
+    if (rt == 2) hipLaunchKernelGGL((gemm_q4k_pf<2, CAI_Q5_K>), dim3(grid), dim3(256), lds, ctx().stream, p);
+    else hipLaunchKernelGGL((gemm_q4k_pf<1, CAI_Q5_K>), dim3(grid), dim3(256), lds, ctx().stream, p);
+  } else if (rt == 2) hipLaunchKernelGGL((gemm_q4k_pf<2, CAI_Q4_K>), dim3(grid), dim3(256), lds, ctx().stream, p);
+  else hipLaunchKernelGGL((gemm_q4k_pf<1, CAI_Q4_K>), dim3(grid), dim3(256), lds, ctx().stream, p);
   return CAI_OK;
 }
 
@@ -762,6 +757,7 @@ int prefill_gemm_multi(const cai_qw_s* const* ws, const int* y_off, int n_w, int
 // y[t][i] = up_i * silu(gate_i) of the prepared activations through a gate|up matrix of 2 * half rows (Q4_K / Q5_K), one launch
 bool prefill_gemm_swiglu_supported(const cai_qw_s* w, int n_tok)
 {
+  if (gemm_wide_wanted(w, w->rows, n_tok)) return w->rows % 2 == 0;
   // only where the product takes two row tiles per wave anyway (enough work-groups to fill the chip several times over)
   return gemm_mfma_supported(w) && w->qtype != CAI_Q6_K && w->rows % 2 == 0 && (int)((w->rows + 255) / 256) * ((n_tok + 31) / 32) >= 4 * ctx().n_cu;
 }

@@ -374,3 +374,42 @@ def test_blocks_of_denormal_and_huge_activations(qt):
     assert np.isfinite(got).all()
     assert rel_err(got, want) < TIGHT
     w.close()
+
+
+@pytest.mark.parametrize("qt", [O.Q4_K, O.Q5_K])
+@pytest.mark.parametrize("rows,cols,T", [(255, 2560, 17), (256, 2560, 64), (257, 2048, 65), (700, 2816, 129), (33000, 2048, 130)])
+def test_prompt_products_on_wide_tiles(qt, rows, cols, T):
+    """tiles of 256 rows x 64 or 128 tokens: one row short of a tile, exactly one, one more; widths of 8, 10 and 11 super-blocks cut into
+    slices of unequal length; 258 tiles, of which two are left over from a round of 256 and cut"""
+    from helpers.device import dev, rel_err
+    cai = dev()
+    rng = np.random.default_rng(rows + cols + T)
+    base = O.quantize(qt, (rng.standard_normal((min(rows, 700), cols)) * 0.02).astype(np.float32)).reshape(min(rows, 700), -1)
+    raw = np.ascontiguousarray(base[np.arange(rows) % 700])
+    x = (rng.standard_normal((T, cols)) * rng.uniform(0.01, 30.0, (T, 1))).astype(np.float32)
+    x[0, : cols // 2] = 0.0
+    bias = (rng.standard_normal(rows) * 0.1).astype(np.float32)
+    w = cai.QWeight(qt, rows, cols, raw.reshape(-1), bias)
+    got = w.gemm(x)
+    for t in sorted({0, 1, 15, 31, 32, T // 2, 63, 64, T - 2, T - 1} & set(range(T))):
+        want = O.gemv(qt, base.reshape(-1), base.shape[0], cols, x[t:t + 1], None, 0, 1)[0][np.arange(rows) % 700] + bias
+        assert rel_err(got[t], want, floor=0.02 * cols ** 0.5 * float(np.abs(x[t]).mean())) < 2e-5, t
+    w.close()
+
+
+@pytest.mark.parametrize("qt", [O.Q4_K, O.Q5_K])
+def test_prompt_of_a_decoder_on_wide_tiles(qt):
+    """q | k | v in one launch of three row groups, gate | up with SwiGLU in the epilogue and behind the slices, residual on a cut product:
+    a prompt of 70 tokens equals its tokens one by one"""
+    from helpers.device import dev, rel_err
+    from helpers.model_build import synthetic_spec
+    cai = dev()
+    cfg = dict(n_layers=2, d_model=2048, n_q_heads=4, n_kv_heads=1, head_dim=128, ffn=2304, vocab=500, max_ctx=128, eps=1e-5, rope_theta=1e4)
+    spec = synthetic_spec(cfg, qt, head_qtype=O.Q8_0, seed=5, std=0.03, qkv_bias=True)
+    dec = cai.Decoder(spec, max_batch=2)
+    tok = np.random.default_rng(2).integers(0, 500, 70).astype(np.int32)
+    _, got = dec.prefill(tok)
+    for p_, t in enumerate(tok):
+        _, want = dec.step_window([t], p_, seq=1)
+    assert rel_err(got, want[0]) < 1e-4
+    dec.close()
