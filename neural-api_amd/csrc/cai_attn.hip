@@ -1775,7 +1775,13 @@ void kv_geometry(const cai_kv_s* kv, int rows, int* split_len, int* n_splits)
   *split_len = sl; *n_splits = (rows + sl - 1) / sl;
 }
 
-int kv_alloc(cai_kv_s* kv, int n_seq, int n_layers, int kv_heads, int head_dim, int max_ctx, int dtype)
+static __global__ void iota_kernel(int32_t* __restrict__ dst, int n)
+{
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) dst[i] = i;
+}
+
+int kv_alloc(cai_kv_s* kv, int n_seq, int n_layers, int kv_heads, int head_dim, int max_ctx, int dtype, bool positions)
 {
   if (n_seq < 1 || n_layers < 1 || kv_heads < 1 || head_dim < 2 || (head_dim & 1) || (head_dim > 64 && (head_dim & 3)) || head_dim > 128 || max_ctx < 1)
     return set_error(CAI_ERR_INVALID, "kv cache: bad geometry seq=%d layers=%d kv_heads=%d head_dim=%d max_ctx=%d", n_seq, n_layers, kv_heads, head_dim, max_ctx);
@@ -1803,7 +1809,11 @@ int kv_alloc(cai_kv_s* kv, int n_seq, int n_layers, int kv_heads, int head_dim, 
   }
   kv->part_q_heads = kv_heads * 8;
   CAI_HIP(hipMalloc(&kv->part, (size_t)n_seq * kv->part_q_heads * kv->n_splits_alloc * (head_dim + 2) * sizeof(float)));
-  CAI_HIP(hipMalloc(&kv->d_len, sizeof(int32_t) * n_seq));
+  CAI_HIP(hipMalloc(&kv->d_len, sizeof(int32_t) * ((size_t)n_seq + (positions ? max_ctx : 0))));
+  if (positions) {
+    kv->d_iota = kv->d_len + n_seq;
+    hipLaunchKernelGGL(iota_kernel, dim3((max_ctx + 255) / 256), dim3(256), 0, ctx().stream, kv->d_iota, max_ctx);
+  }
   CAI_HIP(hipMalloc((void**)&kv->merge_cnt, sizeof(unsigned) * n_seq * kv->part_q_heads));
   CAI_HIP(hipMemsetAsync(kv->merge_cnt, 0, sizeof(unsigned) * n_seq * kv->part_q_heads, ctx().stream));
   CAI_HIP(hipStreamSynchronize(ctx().stream));
@@ -1824,7 +1834,7 @@ void kv_free(cai_kv_s* kv)
   if (kv->part) (void)hipFree(kv->part);
   if (kv->d_len) (void)hipFree(kv->d_len);
   if (kv->merge_cnt) (void)hipFree(kv->merge_cnt);
-  kv->merge_cnt = nullptr;
+  kv->merge_cnt = nullptr; kv->d_iota = nullptr;
   kv->k = kv->v = nullptr; kv->part = nullptr; kv->d_len = nullptr;
 }
 
@@ -1933,7 +1943,7 @@ extern "C" int cai_kv_create(int n_layers, int kv_heads, int head_dim, int max_c
   CAI_READY();
   CAI_REQUIRE(out, "cai_kv_create: null out");
   cai_kv_s* kv = new cai_kv_s();
-  const int rc = kv_alloc(kv, 1, n_layers, kv_heads, head_dim, max_ctx, kv_dtype);
+  const int rc = kv_alloc(kv, 1, n_layers, kv_heads, head_dim, max_ctx, kv_dtype, true);
   if (rc) { kv_free(kv); delete kv; return rc; }
   *out = kv;
   return CAI_OK;
@@ -2092,15 +2102,29 @@ extern "C" int cai_attn_decode(cai_kv_t kv, int layer, const float* qkv, int q_h
   if (len >= kv->max_ctx && kv->evict_cap == 0) return set_error(CAI_ERR_STATE, "cai_attn_decode: cache full (%d rows)", kv->max_ctx);
   const int hd = kv->head_dim;
   const size_t in_b = (size_t)(q_heads + 2 * kv->kv_heads) * hd * sizeof(float), out_b = (size_t)q_heads * hd * sizeof(float);
-  // the kernel rotates/append from a mutable row: always work on a private device copy
-  int rc = ensure_stage(&c.stage_in, &c.stage_in_cap, in_b); if (rc) return rc;
-  CAI_HIP(hipMemcpyAsync(c.stage_in, qkv, in_b, (flags & CAI_X_DEVICE) ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, c.stream));
+  // The kernels below only read the row (no norm and no rotation in place here), so a device row is used where it lies: its copy
+  // and the upload of the position below were two more launches (40 / 8 heads x 128 behind 8191 int8 rows: 29.4 us with both,
+  // 24.1 without).  It is still copied where the wide loads need an alignment that it lacks,
+  // and where the result is written over it, which would race with work-groups that have yet to read their part.
   float* d_out = out;
+  int rc;
   if (!(flags & CAI_Y_DEVICE)) { rc = ensure_stage(&c.stage_out, &c.stage_out_cap, out_b); if (rc) return rc; d_out = (float*)c.stage_out; }
-  c.h_small[0] = len;
-  CAI_HIP(hipMemcpyAsync(kv->d_len, c.h_small, sizeof(int32_t), hipMemcpyHostToDevice, c.stream));
+  const char *x0 = (const char*)qkv, *y0 = (const char*)d_out;
+  float* d_qkv = const_cast<float*>(qkv);
+  if (!(flags & CAI_X_DEVICE) || ((uintptr_t)qkv & 15) || (x0 < y0 + out_b && y0 < x0 + in_b)) {
+    rc = ensure_stage(&c.stage_in, &c.stage_in_cap, in_b); if (rc) return rc;
+    CAI_HIP(hipMemcpyAsync(c.stage_in, qkv, in_b, (flags & CAI_X_DEVICE) ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, c.stream));
+    d_qkv = (float*)c.stage_in;
+  }
+  // The kernels read the position through a pointer (a captured step moves it on the device): here it is an entry of the cache's
+  // table of positions instead of an upload of four bytes.  A rolling cache counts past the table.
+  const int32_t* d_pos = kv->d_iota && len < kv->max_ctx ? kv->d_iota + len : kv->d_len;
+  if (d_pos == kv->d_len) {
+    c.h_small[0] = len;
+    CAI_HIP(hipMemcpyAsync(kv->d_len, c.h_small, sizeof(int32_t), hipMemcpyHostToDevice, c.stream));
+  }
   kv->geo_rows = kv_bucket_rows(kv, len + 1);
-  rc = launch_attn_step(kv, layer, (float*)c.stage_in, 0, 1, q_heads, window, softcap, nullptr, kv->d_len, d_out, 0, 0, 0, nullptr);
+  rc = launch_attn_step(kv, layer, d_qkv, 0, 1, q_heads, window, softcap, nullptr, d_pos, d_out, 0, 0, 0, nullptr);
   if (rc) return rc;
   if (!(flags & CAI_Y_DEVICE)) CAI_HIP(hipMemcpyAsync(out, d_out, out_b, hipMemcpyDeviceToHost, c.stream));
   CAI_HIP(hipStreamSynchronize(c.stream));

@@ -177,6 +177,7 @@ struct cai_kv_s {
   float* part = nullptr;                  // [seq][q_head][split][head_dim+2] split-K partials
   int part_q_heads = 0;
   int32_t* d_len = nullptr;               // [seq] device scratch: rows live BEFORE the token being decoded
+  int32_t* d_iota = nullptr;              // [max_ctx] 0, 1, 2, ... behind d_len: positions that need no upload (a cache of its own only, not a decoder's)
   unsigned* merge_cnt = nullptr;          // [seq][part_q_heads] arrival counters of the in-kernel merge of the split partials (wrap to 0 by themselves)
   void* pq_hi = nullptr; void* pq_lo = nullptr; size_t pq_cap = 0;   // prompt ingestion: rotated q of a chunk as two f16 planes
   float* pq_part = nullptr; size_t pq_part_cap = 0;                     // prompt ingestion: partial results of a token tile's K splits
@@ -253,7 +254,7 @@ int launch_attn_step(cai_kv_s* kv, int layer, float* qkv, int64_t qkv_stride, in
                      float softcap, const float* theta, const int32_t* pos_dev, float* out, int64_t out_stride, int seq0,
                      int prompt_rows = 0, float* prompt_part = nullptr,
                      const float* qn_gain = nullptr, const float* kn_gain = nullptr, float qk_eps = 0.0f);   // full-width q / k RMSNorm done on the way (null: none)
-int kv_alloc(cai_kv_s* kv, int n_seq, int n_layers, int kv_heads, int head_dim, int max_ctx, int dtype);
+int kv_alloc(cai_kv_s* kv, int n_seq, int n_layers, int kv_heads, int head_dim, int max_ctx, int dtype, bool positions = false);
 void kv_free(cai_kv_s* kv);
 int kv_set_eviction(cai_kv_s* kv, int sinks, int recent);
 int kv_snapshot(cai_kv_s* kv, int seq, cai_kv_snap_s** out);

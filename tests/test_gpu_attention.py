@@ -451,3 +451,33 @@ def test_grouped_matrix_core_attention_rolling_eviction(hkv, G, sinks, recent):
         got = kv.attn_decode(0, rows[pos], hq)
         assert np.max(np.abs(got - want[pos])) < 2e-5 * max(1.0, np.max(np.abs(want[pos]))), pos
 
+
+
+@pytest.mark.parametrize("kvt,hq,hkv,dk,ctx,sinks,recent", [("f32", 6, 2, 80, 40, 0, 0), ("f16", 28, 4, 128, 4096, 0, 0), ("i8", 8, 8, 64, 8192, 0, 0), ("f32", 4, 2, 64, 16, 2, 4)])
+def test_device_rows_are_used_in_place_or_copied(kvt, hq, hkv, dk, ctx, sinks, recent):
+    """A row on the device: aligned (read where it lies), at an odd address, and with the result written over it (both copied
+    first); the last case is a rolling cache that counts past its length, which uploads its position.  Same bits as a host row."""
+    import torch
+    from helpers.device import dev
+    cai = dev()
+    L, C = cai.load(), cai.C
+    rng = np.random.default_rng(hq + ctx)
+    n, width, out_n = 45 if sinks else 38, (hq + 2 * hkv) * dk, hq * dk
+    rows = rng.standard_normal((n, width)).astype(np.float32)
+    caches = [cai.KVCache(1, hkv, dk, ctx, {"f32": cai.KV_F32, "f16": cai.KV_F16, "i8": cai.KV_I8}[kvt]) for _ in range(4)]
+    if sinks:
+        for kv in caches:
+            kv.set_eviction(sinks, recent)
+    buf = torch.zeros(width + 4, device="cuda")
+    res = torch.zeros(out_n, device="cuda")
+    for pos in range(n):
+        want = caches[0].attn_decode(0, rows[pos], hq)
+        for kv, shift, over in ((caches[1], 0, False), (caches[2], 1, False), (caches[3], 0, True)):
+            x = buf[shift:shift + width]
+            x.copy_(torch.from_numpy(rows[pos]))
+            y = x[dk:dk + out_n] if over else res
+            torch.cuda.synchronize()
+            cai.check(L.cai_attn_decode(kv.h, 0, C.c_void_p(x.data_ptr()), hq, 0, 0.0, C.c_void_p(y.data_ptr()), cai.X_DEVICE | cai.Y_DEVICE))
+            np.testing.assert_array_equal(y.cpu().numpy(), want, err_msg=f"row {pos} shift {shift} over {over}")
+            if not over:
+                np.testing.assert_array_equal(x.cpu().numpy(), rows[pos])
