@@ -14,12 +14,13 @@
 // = weights 16 + 8 kg .. + 7), so the two lanes of a row read whole 32- / 16-byte blocks and a row's 256 columns are one
 // contiguous run.
 //
-// Work-group: 4 waves x RT row tiles of 32 rows, TT * 32 tokens, 256 columns (8 blocks) per step staged in LDS; with RT = 2
-// an activation operand (1 KB of LDS traffic per wave and instruction) feeds two MFMAs.  The next step's weights are
-// requested before the current one is consumed.
+// Two forms: work-groups with a large tile of their own (gemm_blk_tile), and, where there are too few of those to fill the chip,
+// work-groups whose waves share one small tile and cut its width (gemm_blk_cut).  Both bring their operands into LDS with
+// asynchronous copies along the rows.
 #include "cai_internal.hpp"
 #include "cai_gemv_common.hpp"
 #include <algorithm>
+#include <type_traits>
 
 namespace cai {
 
@@ -29,8 +30,6 @@ typedef _Float16 half2_b __attribute__((ext_vector_type(2)));
 typedef _Float16 half8_b __attribute__((ext_vector_type(8)));
 typedef float float16_b __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4_b __attribute__((ext_vector_type(4)));   // (arrays of HIP's uint4 struct end up in scratch memory)
-
-constexpr int BL_LDX = 264;   // halfs per staged token row: 256 + pad (row stride = 4 banks mod 64: conflict-free 16-byte reads)
 
 struct BlkGemmParams {
   const uint8_t* q; const uint8_t* d; const float* bias;
@@ -64,16 +63,53 @@ __device__ __forceinline__ half8_b codes8(uint32_t w0, uint32_t w1, int high)
   return half8_b{h0.x, h0.y, h1.x, h1.y, h2.x, h2.y, h3.x, h3.y};
 }
 
+// 64 lanes x 16 bytes from base + voff into 1 KB of LDS at lds (uniform), in lane order.  The compiler does not see the load: the
+// caller waits for it before the barrier that publishes the tile, and before the kernel's LDS could go to another work-group.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"     // (m0 is reserved, and named all the same: the statement changes it)
+__device__ __forceinline__ void copy_chunk(uint32_t lds, uint32_t voff, const void* base)
+{
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
+}
+__device__ __forceinline__ void copy_dword(uint32_t lds, uint32_t voff, const void* base)     // 64 lanes x 4 bytes
+{
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" :: "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
+}
+__device__ __forceinline__ void copy_short(uint32_t lds, uint32_t voff, const void* base)     // 64 lanes x 2 bytes, a dword each in LDS
+{
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_ushort %1, %2" :: "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
 }  // namespace
 
-template <int QT, int TT, int RT>
-__global__ __launch_bounds__(256, 2) void gemm_blk_pf(const BlkGemmParams p)
+// ------------------------------------------------------------------------------------------
+// Large tiles.  Eight waves, 256 weight rows x TT * 32 tokens.  Chunks of 64 columns - token planes, quants, scales, all copied along
+// the rows from memory into LDS - are requested DEPTH - 1 chunks ahead of the one that is multiplied; the waves meet once a chunk.
+// A wave holds 64 rows x 16 TT tokens: what it reads of a chunk from LDS (activations of its tokens, quants of its rows) takes less
+// time than its products, which 32 rows x all tokens does not.  A tile of at most 32 tokens (an expert's run, a short prompt) is
+// neither staged nor multiplied in its other half.
+// What bounds it: a chunk's products (2048 cycles of a SIMD at TT = 4), the folds and codes (about 1800 cycles of VALU) and the LDS
+// reads overlap only in part between the two waves of a SIMD (1.65 us a chunk; without copies 1.4, without folds 1.5, with neither
+// and no codes 1.1).  Operands requested one block ahead, and folds issued between the next block's products, changed nothing.
+// 37888 x 3584 Q8_0, 2048 tokens: 1721 us in tiles of 256 x 64 that staged through registers -> 1273 (TT = 4); 3584 x 18944: 1358 -> 718.
+// Gate | up and down of 64 experts (2048 x 2048, 2048 x 1024), 2040 slots: 199 us a layer -> 149 (82 to read the banks once): with tiles
+// of 64 slots instead of 32 an expert's rows come from memory once.  Two work-groups a CU (two slots of LDS each) take the same time.
+// ------------------------------------------------------------------------------------------
+template <int N> __device__ __forceinline__ void wait_loads()
+{
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
+  asm volatile("" ::: "memory");
+}
+template <int QT, int TT, bool ODD>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_blk_tile(const BlkGemmParams p)
 {
   extern __shared__ __align__(16) unsigned char bl_smem[];
-  constexpr int NTOK = TT * 32;
-  _Float16* xs_hi = reinterpret_cast<_Float16*>(bl_smem);            // [NTOK][BL_LDX]
-  _Float16* xs_lo = xs_hi + NTOK * BL_LDX;
-  __shared__ int s_xrow[NTOK], s_yrow[NTOK];
+  constexpr int NTOK = TT * 32, DEPTH = TT == 2 ? 4 : 3, WROW = QT == CAI_Q8_0 ? 64 : 32;
+  constexpr int PLANE = NTOK * 128, XB = 2 * PLANE, WB = 256 * WROW, SLOT = XB + WB + (ODD ? 2048 : 1024);
+  constexpr int XC = NTOK / 64, WC = WB / 8192, COPIES = 2 * XC + WC + (ODD ? 2 : 1);      // a wave's copies of a chunk
+  __shared__ int s_yrow[NTOK];
   __shared__ float s_sinv[NTOK];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 31, kg = lane >> 5;
@@ -89,159 +125,316 @@ __global__ __launch_bounds__(256, 2) void gemm_blk_pf(const BlkGemmParams p)
     if (rg >= p.n_row_groups) return;
     first = ttile * NTOK; n_here = min(NTOK, p.n_tok - first);
   }
-  if (threadIdx.x < NTOK) {
-    const int m = min((int)threadIdx.x, n_here - 1);     // rows past the end repeat the last token; their results are not written
-    int xr, yr;
-    if (p.perm) { const int slot = p.perm[first + m]; xr = slot / p.x_div; yr = slot; }
-    else { xr = yr = first + m; }
-    s_xrow[threadIdx.x] = xr; s_yrow[threadIdx.x] = yr; s_sinv[threadIdx.x] = p.sinv[xr];
-  }
+  const bool one = TT == 2 && n_here <= 32;              // half a tile: the other half is neither staged (by waves 4 .. 7) nor multiplied
+  const bool x_on = !(one && wave >= 4);
   const uint8_t* qbase = p.q; const uint8_t* dbase = p.d; const float* bias = p.bias; int rows = p.rows, yo = 0, rgl = rg;   // this work-group's matrix (uniform)
   if (p.n_seg > 1 && rg >= p.seg_end[0]) { qbase = p.q2[0]; dbase = p.d2[0]; bias = p.bias2[0]; rows = p.rows2[0]; yo = p.y_off2[0]; rgl = rg - p.seg_end[0]; }
   if (p.n_seg > 2 && rg >= p.seg_end[1]) { qbase = p.q2[1]; dbase = p.d2[1]; bias = p.bias2[1]; rows = p.rows2[1]; yo = p.y_off2[1]; rgl = rg - p.seg_end[1]; }
-  const int R0 = (rgl * 4 + wave) * 32 * RT;
-  const int K = p.cols, nb32 = K >> 5, nsb = (K + 255) >> 8;
-  constexpr int BQ = QT == CAI_Q8_0 ? 32 : 16;          // quant bytes per block
+  const int R0 = rgl * 256, K = p.cols, nb32 = K >> 5, n_chunks = (nb32 + 1) >> 1;
   const int64_t bank_row = (int64_t)expert * p.expert_rows;
-  const uint8_t* qrow[RT]; const uint16_t* drow[RT];
-#pragma unroll
-  for (int rt = 0; rt < RT; rt++) {
-    const int64_t r = bank_row + min(R0 + 32 * rt + n, rows - 1);     // tail rows: re-read the last row, not written
-    qrow[rt] = qbase + r * (int64_t)nb32 * BQ + (BQ / 2) * kg;
-    drow[rt] = reinterpret_cast<const uint16_t*>(dbase) + r * (int64_t)nb32;
+  auto x_row = [&](int m) { const int t = first + min(m, n_here - 1); return p.perm ? p.perm[t] / p.x_div : t; };   // rows past the end repeat the last token; their results are not written
+  if (threadIdx.x < NTOK) {
+    const int t = first + min((int)threadIdx.x, n_here - 1);
+    s_yrow[threadIdx.x] = p.perm ? p.perm[t] : t; s_sinv[threadIdx.x] = p.sinv[x_row(threadIdx.x)];
   }
-  struct WRegs { uint32_t q[4][BQ / 8]; uint32_t d[2]; };               // per row tile: the lane's piece of 4 blocks, their 4 scales
-  // unit u = blocks 4 u .. 4 u + 3 of the row.  Loads carry no branch: past the end the last unit / block is fetched again
-  // (cache hits, not used), a block at or past the width counts with scale zero.
-  auto load_w = [&](int u, WRegs (&w)[RT]) {
-    const int uu = min(u, 2 * nsb - 1);
+  // this lane's part of the copies: copy 8 i + wave takes 8 token rows (128 bytes a plane), 16 or 32 weight rows, 64 rows' scales
+  uint32_t xo[XC], wo[WC], xcut = 0, wcut = 0;
 #pragma unroll
-    for (int rt = 0; rt < RT; rt++) {
+  for (int i = 0; i < XC; i++) {
+    const int t = 8 * (8 * i + wave) + (lane >> 3);
+    const uint32_t piece = (uint32_t)((lane & 7) ^ ((t >> 1) & 7));
+    xo[i] = (uint32_t)x_row(t) * (uint32_t)K * 2u + 16u * piece;
+    if (ODD && piece >= 4) xcut |= 1u << i;
+  }
+  const int rlast = rows - 1 - R0;         // tail rows: the last one again, not written
 #pragma unroll
-      for (int b = 0; b < 4; b++) {
-        const int bi = min(4 * uu + b, nb32 - 1);
-        if constexpr (QT == CAI_Q8_0) {
-          const uint4 v = *reinterpret_cast<const uint4*>(qrow[rt] + (int64_t)bi * 32);
-          w[rt].q[b][0] = v.x; w[rt].q[b][1] = v.y; w[rt].q[b][2] = v.z; w[rt].q[b][3] = v.w;
-        } else {
-          const uint2 v = *reinterpret_cast<const uint2*>(qrow[rt] + (int64_t)bi * 16);
-          w[rt].q[b][0] = v.x; w[rt].q[b][1] = v.y;
-        }
-      }
-#pragma unroll
-      for (int b2 = 0; b2 < 2; b2++) {
-        const int b0 = 4 * uu + 2 * b2;
-        uint32_t lo = drow[rt][min(b0, nb32 - 1)], hi = drow[rt][min(b0 + 1, nb32 - 1)];
-        lo = b0 < nb32 ? lo : 0u; hi = b0 + 1 < nb32 ? hi : 0u;
-        w[rt].d[b2] = lo | (hi << 16);
-      }
+  for (int i = 0; i < WC; i++) {
+    if constexpr (QT == CAI_Q8_0) {
+      const int t = 16 * (8 * i + wave) + (lane >> 2); const uint32_t piece = (uint32_t)((lane & 3) ^ ((t >> 2) & 3));
+      wo[i] = (uint32_t)min(t, rlast) * (uint32_t)K + 16u * piece; if (ODD && piece >= 2) wcut |= 1u << i;
     }
+    else {
+      const int t = 32 * (8 * i + wave) + (lane >> 1); const uint32_t piece = (uint32_t)((lane & 1) ^ ((t >> 3) & 1));
+      wo[i] = (uint32_t)min(t, rlast) * (uint32_t)(K / 2) + 16u * piece; if (ODD && piece) wcut |= 1u << i;
+    }
+  }
+  const uint32_t dof = (uint32_t)min(64 * (wave & 3) + lane, rlast) * (uint32_t)(nb32 * 2);     // (waves 4 .. 7 repeat 0 .. 3: every wave counts the same copies)
+  const uint8_t* const qb = qbase + (bank_row + R0) * (int64_t)nb32 * (WROW / 2);
+  const uint8_t* const db = dbase + (bank_row + R0) * (int64_t)nb32 * 2;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)bl_smem;
+  auto copy = [&](int c, int slot) {
+    const uint32_t dst = lds0 + (uint32_t)(slot * SLOT);
+    const bool half = ODD && c == n_chunks - 1;        // one block is left: the chunk's second half repeats the first and is not used
+    const char* const xh = reinterpret_cast<const char*>(p.xhi) + (int64_t)c * 128;
+    const char* const xl = reinterpret_cast<const char*>(p.xlo) + (int64_t)c * 128;
+    if (x_on)
+#pragma unroll
+      for (int i = 0; i < XC; i++) {
+        const uint32_t o = xo[i] - (half && (xcut >> i & 1) ? 64u : 0u);
+        copy_chunk(dst + 1024 * (8 * i + wave), o, xh);
+        copy_chunk(dst + PLANE + 1024 * (8 * i + wave), o, xl);
+      }
+#pragma unroll
+    for (int i = 0; i < WC; i++) copy_chunk(dst + XB + 1024 * (8 * i + wave), wo[i] - (half && (wcut >> i & 1) ? WROW / 2u : 0u), qb + (int64_t)c * WROW);
+    if constexpr (ODD) {
+      copy_short(dst + XB + WB + 256 * (wave & 3), dof, db + (int64_t)c * 4);
+      copy_short(dst + XB + WB + 1024 + 256 * (wave & 3), dof, db + (int64_t)c * 4 + (half ? 0 : 2));
+    } else copy_dword(dst + XB + WB + 256 * (wave & 3), dof, db + (int64_t)c * 4);
   };
 
-  float16_b Y[RT][TT];
+  const float16_b zero16 = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+  // RW row tiles x TW token tiles of a wave, from row tile r0 and token tile t0 of the work-group's on
+  auto body = [&](auto rw_, auto tw_, int r0, int t0) {
+    constexpr int RW = rw_, TW = tw_;
+    float16_b Y[RW][TW];
+#pragma unroll
+    for (int rt = 0; rt < RW; rt++)
+#pragma unroll
+      for (int tt = 0; tt < TW; tt++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) Y[rt][tt][v] = 0.0f;
+    auto use = [&](int slot, bool half) {
+      const unsigned char* const s0 = bl_smem + slot * SLOT;
+      const unsigned char* const sx = s0 + (32 * t0 + n) * 128;
+      const unsigned char* const sw = s0 + XB + (32 * r0 + n) * WROW;
+      uint32_t dw[RW];
+#pragma unroll
+      for (int rt = 0; rt < RW; rt++) {
+        dw[rt] = *reinterpret_cast<const uint32_t*>(s0 + XB + WB + 4 * (32 * (r0 + rt) + n));
+        if constexpr (ODD) dw[rt] |= *reinterpret_cast<const uint32_t*>(s0 + XB + WB + 1024 + 4 * (32 * (r0 + rt) + n)) << 16;
+      }
+#pragma unroll
+      for (int b = 0; b < 2; b++) {
+        if (ODD && b && half) break;
+        half8_b A[TW][4], W[RW][2];
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+          // Q8_0: the lane's k of step s are columns 16 kg + 8 s .. of the block; Q4_0: 16 s + 8 kg ..
+          const int c = 4 * b + (QT == CAI_Q8_0 ? 2 * kg + s : 2 * s + kg);
+#pragma unroll
+          for (int tt = 0; tt < TW; tt++) {
+            const unsigned char* const a = sx + tt * 4096 + 16 * (c ^ ((n >> 1) & 7));
+            A[tt][2 * s] = *reinterpret_cast<const half8_b*>(a); A[tt][2 * s + 1] = *reinterpret_cast<const half8_b*>(a + PLANE);
+          }
+        }
+#pragma unroll
+        for (int rt = 0; rt < RW; rt++) {
+          const unsigned char* const w = sw + rt * 32 * WROW;
+          if constexpr (QT == CAI_Q8_0) {
+            const u32x4_b q = *reinterpret_cast<const u32x4_b*>(w + 16 * ((2 * b + kg) ^ ((n >> 2) & 3)));
+            W[rt][0] = codes8<QT>(q.x, q.y, 0); W[rt][1] = codes8<QT>(q.z, q.w, 0);
+          } else {
+            const uint2 q = *reinterpret_cast<const uint2*>(w + 16 * (b ^ ((n >> 3) & 1)) + 8 * kg);
+            W[rt][0] = codes8<QT>(q.x, q.y, 0); W[rt][1] = codes8<QT>(q.x, q.y, 1);
+          }
+        }
+#pragma unroll
+        for (int rt = 0; rt < RW; rt++) {
+          const float dv = __half2float(__ushort_as_half((unsigned short)(b ? (dw[rt] >> 16) : (dw[rt] & 0xffffu))));
+          float16_b C[TW];
+#pragma unroll
+          for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int tt = 0; tt < TW; tt++) C[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[tt][k], W[rt][k >> 1], k == 0 ? zero16 : C[tt], 0, 0, 0);
+#pragma unroll
+          for (int tt = 0; tt < TW; tt++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) Y[rt][tt][v] = fmaf(dv, C[tt][v], Y[rt][tt][v]);
+        }
+      }
+    };
+#pragma unroll
+    for (int i = 0; i < DEPTH - 1; i++) if (i < n_chunks) copy(i, i);
+    int slot = 0;
+    for (int c = 0; c < n_chunks; c++) {
+      const int left = n_chunks - 1 - c;               // chunks behind this one
+      if (left >= DEPTH - 2) { if (x_on) wait_loads<(DEPTH - 2) * COPIES>(); else wait_loads<(DEPTH - 2) * (COPIES - 2 * XC)>(); }
+      else wait_loads<0>();
+      __builtin_amdgcn_s_waitcnt(0xC07F);              // lgkmcnt(0): this wave's reads of the slot that is filled next (and the row tables, the first time)
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      if (left >= DEPTH - 1) copy(c + DEPTH - 1, slot == 0 ? DEPTH - 1 : slot - 1);
+      use(slot, ODD && left == 0);
+      slot = slot + 1 == DEPTH ? 0 : slot + 1;
+    }
+    // ---- write: the lane holds weight row n and tokens 8 g + 4 kg + i of each tile: the 32 lanes of a half-wave store 32
+    // consecutive outputs of one token row ----
+#pragma unroll
+    for (int tt = 0; tt < TW; tt++)
+#pragma unroll
+      for (int v = 0; v < 16; v++) {
+        const int m = 32 * (t0 + tt) + 8 * (v >> 2) + 4 * kg + (v & 3);
+        if (m >= n_here) continue;
+        const float si = s_sinv[m];
+        const int64_t o = (int64_t)s_yrow[m] * p.y_stride + yo;
+#pragma unroll
+        for (int rt = 0; rt < RW; rt++) {
+          const int row = R0 + 32 * (r0 + rt) + n;
+          if (row >= rows) continue;
+          float y = Y[rt][tt][v] * si;
+          if (bias) y += bias[bank_row + row];
+          if (p.residual) y += p.residual[o + row];
+          p.y[o + row] = y;
+        }
+      }
+  };
+  if constexpr (TT == 2) {
+    if (one) { body(std::integral_constant<int, 1>(), std::integral_constant<int, 1>(), wave, 0); return; }
+  }
+  body(std::integral_constant<int, 2>(), std::integral_constant<int, TT / 2>(), 2 * (wave & 3), TT / 2 * (wave >> 2));
+}
+
+// ------------------------------------------------------------------------------------------
+// Few tiles: the waves of a work-group share ONE tile of 32 RT rows x 32 tokens and cut its width; their sums meet in LDS at the end.
+// Each wave copies chunks of 64 columns (token planes, quants, scales) along the rows into LDS of its own, one chunk ahead of the one
+// it multiplies, so there is no barrier before the end.  An operand load straight from memory touches 32 rows, a line each, and takes
+// four times the cycles of the same bytes read along the rows: that form, also cut, took 15.2 us where this one takes 10.7.
+// What bounds it: the copies, 66 KB/us into one CU.  576 x 1536, 37 tokens, with the pre-pass of the activations: 23.1 us as 10 uncut
+// tiles of 128 x 32 -> 10.7; 64 x 2048, 255 tokens: 27 -> 14; 2048 x 2048, 255: 31 -> 17.5.
+// Places in LDS: 16-byte piece c of token row t (128 bytes a plane) at c ^ (t / 2 % 8), of Q8_0 weight row n (64 bytes) at c ^ (n / 4 % 4),
+// of Q4_0 row n (32 bytes) at c ^ (n / 8 % 2): the lanes of a read pass then meet different banks.
+// ------------------------------------------------------------------------------------------
+template <int QT, int RT, int NW, bool ODD>     // ODD: rows of an odd number of blocks (scales that are not aligned to 4 bytes, a last chunk of one block)
+__global__ __launch_bounds__(64 * NW) void gemm_blk_cut(const BlkGemmParams p)
+{
+  extern __shared__ __align__(16) unsigned char bl_smem[];
+  constexpr int WROW = QT == CAI_Q8_0 ? 64 : 32, NV = RT * 16;                 // quant bytes of a row's chunk; values of a lane
+  constexpr int XB = 8192, WB = 32 * WROW, SLOT = XB + RT * WB + (ODD ? 512 : 256);          // a chunk: planes hi, lo; quants; scales
+  constexpr int COPIES = 8 + RT * WB / 1024 + (ODD ? 2 : 1);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = lane & 31, kg = lane >> 5;
+  const int L = blockIdx.x;
+  const int rg = (L & 7) + 8 * ((L >> 3) / p.n_tok_tiles), ttile = (L >> 3) % p.n_tok_tiles;
+  if (rg >= p.n_row_groups) return;
+  const int first = ttile * 32;
+  const uint8_t* qbase = p.q; const uint8_t* dbase = p.d; const float* bias = p.bias; int rows = p.rows, yo = 0, rgl = rg;   // this work-group's matrix (uniform)
+  if (p.n_seg > 1 && rg >= p.seg_end[0]) { qbase = p.q2[0]; dbase = p.d2[0]; bias = p.bias2[0]; rows = p.rows2[0]; yo = p.y_off2[0]; rgl = rg - p.seg_end[0]; }
+  if (p.n_seg > 2 && rg >= p.seg_end[1]) { qbase = p.q2[1]; dbase = p.d2[1]; bias = p.bias2[1]; rows = p.rows2[1]; yo = p.y_off2[1]; rgl = rg - p.seg_end[1]; }
+  const int R0 = rgl * 32 * RT, K = p.cols, nb32 = K >> 5;
+  const int n_chunks = (nb32 + 1) >> 1, c0 = n_chunks * wave / NW, c1 = n_chunks * (wave + 1) / NW;     // this wave's chunks
+  // this lane's part of the copies; rows and tokens past the end repeat the last one and are not written
+  uint32_t xo[4], wo[RT * WB / 1024], xcut = 0, wcut = 0;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int t = 8 * i + (lane >> 3);
+    const uint32_t piece = (uint32_t)((lane & 7) ^ ((t >> 1) & 7));
+    xo[i] = (uint32_t)min(first + t, p.n_tok - 1) * (uint32_t)K * 2u + 16u * piece;
+    if (ODD && piece >= 4) xcut |= 1u << i;
+  }
+  const int rlast = rows - 1 - R0;
+#pragma unroll
+  for (int i = 0; i < RT * WB / 1024; i++) {
+    if constexpr (QT == CAI_Q8_0) {
+      const int t = 16 * i + (lane >> 2); const uint32_t piece = (uint32_t)((lane & 3) ^ ((t >> 2) & 3));
+      wo[i] = (uint32_t)min(t, rlast) * (uint32_t)K + 16u * piece; if (ODD && piece >= 2) wcut |= 1u << i;
+    }
+    else {
+      const int t = 32 * i + (lane >> 1); const uint32_t piece = (uint32_t)((lane & 1) ^ ((t >> 3) & 1));
+      wo[i] = (uint32_t)min(t, rlast) * (uint32_t)(K / 2) + 16u * piece; if (ODD && piece) wcut |= 1u << i;
+    }
+  }
+  const uint32_t dof = (uint32_t)min(RT == 2 ? lane : n, rlast) * (uint32_t)(nb32 * 2);
+  const uint8_t* const qb = qbase + (int64_t)R0 * nb32 * (WROW / 2);
+  const uint8_t* const db = dbase + (int64_t)R0 * nb32 * 2;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)bl_smem + (uint32_t)(wave * 2 * SLOT);
+  auto copy = [&](int c, int slot) {
+    const uint32_t dst = lds0 + (uint32_t)(slot * SLOT);
+    const bool half = ODD && c == n_chunks - 1;        // one block is left: the chunk's second half repeats the first and is not used
+    const char* const xh = reinterpret_cast<const char*>(p.xhi) + (int64_t)c * 128;
+    const char* const xl = reinterpret_cast<const char*>(p.xlo) + (int64_t)c * 128;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const uint32_t o = xo[i] - (half && (xcut >> i & 1) ? 64u : 0u);
+      copy_chunk(dst + 1024 * i, o, xh); copy_chunk(dst + 4096 + 1024 * i, o, xl);
+    }
+#pragma unroll
+    for (int i = 0; i < RT * WB / 1024; i++) copy_chunk(dst + XB + 1024 * i, wo[i] - (half && (wcut >> i & 1) ? WROW / 2u : 0u), qb + (int64_t)c * WROW);
+    if constexpr (ODD) {
+      copy_short(dst + XB + RT * WB, dof, db + (int64_t)c * 4);
+      copy_short(dst + XB + RT * WB + 256, dof, db + (int64_t)c * 4 + (half ? 0 : 2));
+    } else copy_dword(dst + XB + RT * WB, dof, db + (int64_t)c * 4);
+  };
+  float16_b Y[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; rt++)
 #pragma unroll
-    for (int tt = 0; tt < TT; tt++)
-#pragma unroll
-      for (int v = 0; v < 16; v++) Y[rt][tt][v] = 0.0f;
-
+    for (int v = 0; v < 16; v++) Y[rt][v] = 0.0f;
   const float16_b zero16 = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-  // four blocks of the staged 256 columns, starting at block b_first of the tile
-  auto compute = [&](const WRegs (&w)[RT], int b_first) {
+  const unsigned char* const mine = bl_smem + wave * 2 * SLOT;
+  auto use = [&](int slot, bool half) {
+    const unsigned char* const s0 = mine + slot * SLOT;
+    uint32_t dw[RT];
 #pragma unroll
-    for (int b = 0; b < 4; b++) {
-      half8_b W[RT][2];
+    for (int rt = 0; rt < RT; rt++) {
+      dw[rt] = *reinterpret_cast<const uint32_t*>(s0 + XB + RT * WB + 4 * (32 * rt + n));
+      if constexpr (ODD) dw[rt] |= *reinterpret_cast<const uint32_t*>(s0 + XB + RT * WB + 256 + 4 * (32 * rt + n)) << 16;
+    }
 #pragma unroll
-      for (int rt = 0; rt < RT; rt++) {
-        if constexpr (QT == CAI_Q8_0) { W[rt][0] = codes8<QT>(w[rt].q[b][0], w[rt].q[b][1], 0); W[rt][1] = codes8<QT>(w[rt].q[b][2], w[rt].q[b][3], 0); }
-        else { W[rt][0] = codes8<QT>(w[rt].q[b][0], w[rt].q[b][1], 0); W[rt][1] = codes8<QT>(w[rt].q[b][0], w[rt].q[b][1], 1); }
+    for (int b = 0; b < 2; b++) {
+      if (ODD && b && half) break;
+      half8_b A[4], W[RT][2];
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        // Q8_0: the lane's k of step s are columns 16 kg + 8 s .. of the block; Q4_0: 16 s + 8 kg ..
+        const int c = 4 * b + (QT == CAI_Q8_0 ? 2 * kg + s : 2 * s + kg);
+        const unsigned char* const a = s0 + n * 128 + 16 * (c ^ ((n >> 1) & 7));
+        A[2 * s] = *reinterpret_cast<const half8_b*>(a); A[2 * s + 1] = *reinterpret_cast<const half8_b*>(a + 4096);
       }
-      float16_b C[RT][TT];
-#pragma unroll
-      for (int s = 0; s < 2; s++)
-#pragma unroll
-        for (int tt = 0; tt < TT; tt++) {
-          // Q8_0: the lane's k of step s are columns 16 kg + 8 s .. of the block; Q4_0: 16 s + 8 kg ..
-          const int koff = QT == CAI_Q8_0 ? 16 * kg + 8 * s : 16 * s + 8 * kg;
-          const int off = (tt * 32 + n) * BL_LDX + 32 * (b_first + b) + koff;
-          const half8_b Ah = *reinterpret_cast<const half8_b*>(xs_hi + off);
-          const half8_b Al = *reinterpret_cast<const half8_b*>(xs_lo + off);
-#pragma unroll
-          for (int rt = 0; rt < RT; rt++) C[rt][tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Ah, W[rt][s], s == 0 ? zero16 : C[rt][tt], 0, 0, 0);
-#pragma unroll
-          for (int rt = 0; rt < RT; rt++) C[rt][tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Al, W[rt][s], C[rt][tt], 0, 0, 0);
-        }
 #pragma unroll
       for (int rt = 0; rt < RT; rt++) {
-        const uint32_t dw = w[rt].d[b >> 1];
-        const float dv = __half2float(__ushort_as_half((unsigned short)((b & 1) ? (dw >> 16) : (dw & 0xffffu))));
+        const unsigned char* const w = s0 + XB + rt * WB + n * WROW;
+        if constexpr (QT == CAI_Q8_0) {
+          const u32x4_b q = *reinterpret_cast<const u32x4_b*>(w + 16 * ((2 * b + kg) ^ ((n >> 2) & 3)));
+          W[rt][0] = codes8<QT>(q.x, q.y, 0); W[rt][1] = codes8<QT>(q.z, q.w, 0);
+        } else {
+          const uint2 q = *reinterpret_cast<const uint2*>(w + 16 * (b ^ ((n >> 3) & 1)) + 8 * kg);
+          W[rt][0] = codes8<QT>(q.x, q.y, 0); W[rt][1] = codes8<QT>(q.x, q.y, 1);
+        }
+      }
 #pragma unroll
-        for (int tt = 0; tt < TT; tt++)
+      for (int rt = 0; rt < RT; rt++) {
+        const float dv = __half2float(__ushort_as_half((unsigned short)(b ? (dw[rt] >> 16) : (dw[rt] & 0xffffu))));
+        float16_b C = zero16;
 #pragma unroll
-          for (int v = 0; v < 16; v++) Y[rt][tt][v] = fmaf(dv, C[rt][tt][v], Y[rt][tt][v]);
+        for (int k = 0; k < 4; k++) C = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[k], W[rt][k >> 1], C, 0, 0, 0);
+#pragma unroll
+        for (int v = 0; v < 16; v++) Y[rt][v] = fmaf(dv, C[v], Y[rt][v]);
       }
     }
   };
-
-  WRegs wa[RT], wb[RT];
-  load_w(0, wa);
-  __syncthreads();                         // the row tables
-  for (int sb = 0; sb < nsb; sb++) {
-    if (sb) __syncthreads();               // the previous step's LDS reads are done
-    {
-      // thread = (token tq + 8 i, 16-byte chunk); columns at or past the width are staged as zeros
-      const int tq = threadIdx.x >> 5, chunk = threadIdx.x & 31;
-      const int col = sb * 256 + chunk * 8;
-      const bool in = col < K;
-      const uint32_t colo = (uint32_t)(in ? col : 0);
-      constexpr int SB = TT == 2 ? 2 : 4;
-#pragma unroll
-      for (int i0 = 0; i0 < NTOK / 8; i0 += SB) {
-        u32x4_b vh[SB], vl[SB];
-#pragma unroll
-        for (int i = 0; i < SB; i++) {
-          const int64_t off = (int64_t)s_xrow[tq + 8 * (i0 + i)] * K + colo;
-          vh[i] = *reinterpret_cast<const u32x4_b*>(p.xhi + off);
-          vl[i] = *reinterpret_cast<const u32x4_b*>(p.xlo + off);
-        }
-#pragma unroll
-        for (int i = 0; i < SB; i++) {
-          const u32x4_b z = {0u, 0u, 0u, 0u};
-          *reinterpret_cast<u32x4_b*>(xs_hi + (tq + 8 * (i0 + i)) * BL_LDX + chunk * 8) = in ? vh[i] : z;
-          *reinterpret_cast<u32x4_b*>(xs_lo + (tq + 8 * (i0 + i)) * BL_LDX + chunk * 8) = in ? vl[i] : z;
-        }
-      }
-    }
-    load_w(2 * sb + 1, wb);
-    __syncthreads();
-    compute(wa, 0);
-    load_w(2 * sb + 2, wa);                // the next step's first half is in flight while this step's second half is consumed
-    compute(wb, 4);
+  if (c0 < c1) copy(c0, 0);
+  for (int c = c0; c < c1; c++) {
+    const int slot = (c - c0) & 1;
+    if (c + 1 < c1) {
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the last reads of the other slot
+      copy(c + 1, slot ^ 1);
+      wait_loads<COPIES>();
+    } else wait_loads<0>();
+    use(slot, ODD && c == n_chunks - 1);
   }
-
-  // ---- write: the lane holds weight row n of each row tile and tokens 8 g + 4 kg + i of each token tile: the 32 lanes of a
-  // half-wave store 32 consecutive outputs of one token row ----
+  __syncthreads();                         // (every wave's copies have been waited for)
+  float* const sacc = reinterpret_cast<float*>(bl_smem);     // [wave][RT 16][64 lanes]
 #pragma unroll
-  for (int tt = 0; tt < TT; tt++)
+  for (int rt = 0; rt < RT; rt++)
 #pragma unroll
-    for (int g = 0; g < 4; g++)
+    for (int v = 0; v < 16; v++) sacc[(wave * NV + rt * 16 + v) * 64 + lane] = Y[rt][v];
+  __syncthreads();
+  // wave w sums the values w, w + NW, ...: the lane's value v of row tile rt is weight row n and token 8 (v / 4) + 4 kg + v % 4
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int m = tt * 32 + 8 * g + 4 * kg + i;
-        if (m >= n_here) continue;
-        const float si = s_sinv[m];
-        const int64_t o = (int64_t)s_yrow[m] * p.y_stride;
+  for (int j0 = 0; j0 < NV; j0 += NW) {
+    const int j = j0 + wave, v = j & 15, rt = j >> 4;
+    if (j >= NV) break;
+    float y = 0.0f;
 #pragma unroll
-        for (int rt = 0; rt < RT; rt++) {
-          const int row = R0 + 32 * rt + n;
-          if (row >= rows) continue;
-          float r = Y[rt][tt][4 * g + i] * si;
-          if (bias) r += bias[bank_row + row];
-          if (p.residual) r += p.residual[o + yo + row];
-          p.y[o + yo + row] = r;
-        }
-      }
+    for (int w = 0; w < NW; w++) y += sacc[(w * NV + j) * 64 + lane];
+    const int t = first + 8 * (v >> 2) + 4 * kg + (v & 3), row = R0 + 32 * rt + n;
+    if (t >= p.n_tok || row >= rows) continue;
+    const int64_t o = (int64_t)t * p.y_stride + yo + row;
+    y *= p.sinv[t];
+    if (bias) y += bias[row];
+    if (p.residual) y += p.residual[o];
+    p.y[o] = y;
+  }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -276,36 +469,83 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int32_t* expert, 
 
 namespace {
 
-template <int QT>
+template <void (*KERNEL)(BlkGemmParams)>
+int launch_lds(int grid, int threads, size_t lds, const BlkGemmParams& p)
+{
+  static bool attr_done = false;
+  if (!attr_done) {
+    CAI_HIP(hipFuncSetAttribute((const void*)KERNEL, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    attr_done = true;
+  }
+  hipLaunchKernelGGL(KERNEL, dim3(grid), dim3(threads), lds, ctx().stream, p);
+  return CAI_OK;
+}
+
+// Row groups of `rows` weight rows (every matrix starts one of its own) x n_tiles token tiles
+int blk_grid(BlkGemmParams& p, int rows, int n_tiles)
+{
+  p.n_row_groups = (p.rows + rows - 1) / rows;
+  for (int i = 1; i < p.n_seg; i++) { p.seg_end[i - 1] = p.n_row_groups; p.n_row_groups += (p.rows2[i - 1] + rows - 1) / rows; }
+  p.n_tok_tiles = n_tiles;
+  return p.tile_tab ? n_tiles * p.n_row_groups : 8 * n_tiles * ((p.n_row_groups + 7) / 8);
+}
+
+template <int QT, bool ODD>
 int launch_blk(const BlkGemmParams& p0, int n_tiles_grouped)
 {
   BlkGemmParams p = p0;
-  const int n_cu = ctx().n_cu;
-  static bool attr_done = false;
-  if (!attr_done) {
-    const void* ks[] = {(const void*)gemm_blk_pf<CAI_Q8_0, 1, 1>, (const void*)gemm_blk_pf<CAI_Q8_0, 1, 2>, (const void*)gemm_blk_pf<CAI_Q8_0, 2, 2>,
-                        (const void*)gemm_blk_pf<CAI_Q4_0, 1, 1>, (const void*)gemm_blk_pf<CAI_Q4_0, 1, 2>, (const void*)gemm_blk_pf<CAI_Q4_0, 2, 2>};
-    for (const void* k : ks) if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024) != hipSuccess) (void)hipGetLastError();
-    attr_done = true;
+  constexpr size_t WROW = QT == CAI_Q8_0 ? 64 : 32;                                    // quant bytes of a row's chunk
+  auto tile = [&](auto tt_, int n_tiles) {
+    constexpr int TT = tt_;
+    return launch_lds<gemm_blk_tile<QT, TT, ODD>>(blk_grid(p, 256, n_tiles), 512, (TT == 2 ? 4 : 3) * (TT * 8192 + 256 * WROW + (ODD ? 2048 : 1024)), p);
+  };
+  auto cut = [&](auto rt_, auto nw_) {
+    constexpr int RT = rt_, NW = nw_;
+    return launch_lds<gemm_blk_cut<QT, RT, NW, ODD>>(blk_grid(p, 32 * RT, (p.n_tok + 31) / 32), 64 * NW, NW * 2 * (8192 + RT * 32 * WROW + (ODD ? 512 : 256)), p);
+  };
+  typedef std::integral_constant<int, 1> One; typedef std::integral_constant<int, 2> Two; typedef std::integral_constant<int, 3> Three;
+  typedef std::integral_constant<int, 4> Four; typedef std::integral_constant<int, 7> Seven;
+  if (p.tile_tab) return tile(Two(), n_tiles_grouped);
+  // A form's time is its rounds over the chip times what a round takes, in ns a column (Q8_0; with a full chip): cut tiles of 32 rows
+  // 3.0, of 64 rows 4.6 (one work-group a CU) or 9.0 (three waves, two work-groups a CU: better from the second round on, 6144 x 2048
+  // and 255 tokens 34.2 us against 35.5), tiles of 256 x 64 18 (13 if half empty), of 256 x 128 27.  At the lines, with the pre-pass:
+  //   2048 x 2048:  128 tokens  32 rows 13.5  64 rows 16.0     255: 20.3, 17.4     1024:  64 rows 51.5  256 x 64 51.7
+  //   6144 x 2048:  511 tokens  64 rows 59.8  256 x 64 51.4   1024: 256 x 64 96, 256 x 128 77
+  //   3072 x 576:   511 tokens  64 rows 18.9  256 x 64 21.6   1024: 30.4, 24.8
+  const int n_cu = ctx().n_cu, tok32 = (p.n_tok + 31) / 32;
+  auto groups = [&](int rows) {
+    int g = (p.rows + rows - 1) / rows;
+    for (int i = 1; i < p.n_seg; i++) g += (p.rows2[i - 1] + rows - 1) / rows;
+    return (int64_t)g;
+  };
+  auto rounds = [](int64_t wgs, int n) { return (double)((wgs + n - 1) / n); };
+  if (groups(32) * tok32 <= n_cu) return cut(One(), Seven());
+  if (groups(64) * tok32 <= n_cu) return cut(Two(), Four());
+  const double c64 = 9.0 * rounds(groups(64) * tok32, 2 * n_cu);
+  const double t64 = (p.n_tok <= 32 ? 13.0 : 18.0) * rounds(groups(256) * ((p.n_tok + 63) / 64), n_cu);
+  const double t128 = 27.0 * rounds(groups(256) * ((p.n_tok + 127) / 128), n_cu);
+  if (c64 <= t64 && c64 <= t128) return cut(Two(), Three());
+  return t128 <= t64 ? tile(Four(), (p.n_tok + 127) / 128) : tile(Two(), (p.n_tok + 63) / 64);
+}
+
+int launch_blk(const cai_qw_s* w, const BlkGemmParams& p0, int n_tiles_grouped)
+{
+  auto go = [&](const BlkGemmParams& p) {
+    const bool odd = (p.cols >> 5) & 1;
+    if (w->qtype == CAI_Q8_0) return odd ? launch_blk<CAI_Q8_0, true>(p, n_tiles_grouped) : launch_blk<CAI_Q8_0, false>(p, n_tiles_grouped);
+    return odd ? launch_blk<CAI_Q4_0, true>(p, n_tiles_grouped) : launch_blk<CAI_Q4_0, false>(p, n_tiles_grouped);
+  };
+  if (p0.tile_tab) return go(p0);
+  // the kernels reach an activation row through a 32-bit byte offset: planes of 4 GiB and more go in pieces of whole tiles
+  const int64_t most = ((int64_t)1 << 31) / p0.cols / 128 * 128;
+  for (int64_t t = 0; t < p0.n_tok; t += most) {
+    BlkGemmParams p = p0;
+    p.n_tok = (int)std::min<int64_t>(most, p0.n_tok - t);
+    p.xhi += t * p0.cols; p.xlo += t * p0.cols; p.sinv += t; p.y += t * p0.y_stride;
+    if (p.residual) p.residual += t * p0.y_stride;
+    const int rc = go(p);
+    if (rc) return rc;
   }
-  // Tiling: two row tiles per wave (256 rows per work-group) whenever that still gives every CU work; two token tiles on top
-  // for long prompts; one row tile for matrices of few rows
-  const int tiles32 = p.tile_tab ? n_tiles_grouped : (p.n_tok + 31) / 32;
-  int rows_all = p.rows;
-  for (int i = 1; i < p.n_seg; i++) rows_all += p.rows2[i - 1];
-  const int wgs_rt2 = ((rows_all + 255) / 256) * tiles32;
-  int rt = wgs_rt2 >= n_cu ? 2 : 1, tt = 1;
-  if (!p.tile_tab && rt == 2 && ((rows_all + 255) / 256) * ((p.n_tok + 63) / 64) >= 2 * n_cu) tt = 2;
-  p.n_row_groups = (p.rows + 128 * rt - 1) / (128 * rt);
-  for (int i = 1; i < p.n_seg; i++) { p.seg_end[i - 1] = p.n_row_groups; p.n_row_groups += (p.rows2[i - 1] + 128 * rt - 1) / (128 * rt); }   // every matrix starts a row group of its own
-  const size_t lds = (size_t)tt * 32 * BL_LDX * 2 * 2;
-  int grid;
-  if (p.tile_tab) { p.n_tok_tiles = n_tiles_grouped; grid = n_tiles_grouped * p.n_row_groups; }
-  else { p.n_tok_tiles = (p.n_tok + tt * 32 - 1) / (tt * 32); grid = 8 * p.n_tok_tiles * ((p.n_row_groups + 7) / 8); }
-  hipStream_t st = ctx().stream;
-  if (tt == 2) hipLaunchKernelGGL((gemm_blk_pf<QT, 2, 2>), dim3(grid), dim3(256), lds, st, p);
-  else if (rt == 2) hipLaunchKernelGGL((gemm_blk_pf<QT, 1, 2>), dim3(grid), dim3(256), lds, st, p);
-  else hipLaunchKernelGGL((gemm_blk_pf<QT, 1, 1>), dim3(grid), dim3(256), lds, st, p);
   return CAI_OK;
 }
 
@@ -322,7 +562,7 @@ int launch_gemm_blk(const cai_qw_s* w, const _Float16* xhi, const _Float16* xlo,
   p.q = w->data; p.d = w->aux; p.bias = w->bias; p.rows = (int)w->rows; p.cols = (int)w->cols;
   p.xhi = xhi; p.xlo = xlo; p.sinv = sinv; p.n_tok = n_tok; p.y = y; p.y_stride = y_stride; p.residual = residual;
   p.x_div = 1; p.expert_rows = 0;
-  return w->qtype == CAI_Q8_0 ? launch_blk<CAI_Q8_0>(p, 0) : launch_blk<CAI_Q4_0>(p, 0);
+  return launch_blk(w, p, 0);
 }
 
 // Up to three matrices of one type and width in one launch: y[t][y_off[i] + r] = (W_i x[t])[r] (+ bias_i)
@@ -342,16 +582,17 @@ int launch_gemm_blk_multi(const cai_qw_s* const* ws, const int* y_off, int n_w, 
   p.xhi = xhi; p.xlo = xlo; p.sinv = sinv; p.n_tok = n_tok; p.y = y + y_off[0]; p.y_stride = y_stride; p.residual = nullptr;
   p.x_div = 1; p.expert_rows = 0; p.n_seg = n_w;
   for (int i = 1; i < n_w; i++) { p.q2[i - 1] = ws[i]->data; p.d2[i - 1] = ws[i]->aux; p.bias2[i - 1] = ws[i]->bias; p.rows2[i - 1] = (int)ws[i]->rows; p.y_off2[i - 1] = y_off[i] - y_off[0]; }
-  return w->qtype == CAI_Q8_0 ? launch_blk<CAI_Q8_0>(p, 0) : launch_blk<CAI_Q4_0>(p, 0);
+  return launch_blk(w, p, 0);
 }
 
 // Token tiles of the grouped launches: every expert may end with a partial tile
-int moe_group_max_tiles(int n_slots, int n_experts) { return (n_slots + 31) / 32 + n_experts; }
+constexpr int MOE_TILE = 64;
+int moe_group_max_tiles(int n_slots, int n_experts) { return (n_slots + MOE_TILE - 1) / MOE_TILE + n_experts; }
 
 int launch_moe_group(const int32_t* expert, int n_slots, int n_experts, int32_t* perm, int32_t* tile_tab)
 {
   if (n_experts > 512) return set_error(CAI_ERR_UNSUPPORTED, "moe grouping: %d experts (up to 512)", n_experts);
-  hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(1024), 0, ctx().stream, expert, n_slots, n_experts, 32, moe_group_max_tiles(n_slots, n_experts), perm, tile_tab);
+  hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(1024), 0, ctx().stream, expert, n_slots, n_experts, MOE_TILE, moe_group_max_tiles(n_slots, n_experts), perm, tile_tab);
   return CAI_OK;
 }
 
@@ -362,12 +603,13 @@ int launch_gemm_blk_grouped(const cai_qw_s* bank, int64_t expert_rows, const _Fl
 {
   if (!gemm_blk_supported(bank)) return set_error(CAI_ERR_UNSUPPORTED, "grouped prompt gemm: weight type %d", bank->qtype);
   if (expert_rows <= 0 || bank->rows != expert_rows * n_experts) return set_error(CAI_ERR_INVALID, "grouped prompt gemm: bank of %lld rows is not %d windows of %lld", (long long)bank->rows, n_experts, (long long)expert_rows);
+  if ((int64_t)((n_slots - 1) / x_div + 1) * bank->cols >= ((int64_t)1 << 31)) return set_error(CAI_ERR_UNSUPPORTED, "grouped prompt gemm: %d slots of width %lld", n_slots, (long long)bank->cols);
   BlkGemmParams p{};
   p.q = bank->data; p.d = bank->aux; p.bias = bank->bias; p.rows = (int)expert_rows; p.cols = (int)bank->cols;
   p.xhi = xhi; p.xlo = xlo; p.sinv = sinv; p.n_tok = n_slots; p.y = y; p.y_stride = y_stride; p.residual = nullptr;
   p.tile_tab = tile_tab; p.perm = perm; p.x_div = x_div; p.expert_rows = expert_rows;
   const int tiles = moe_group_max_tiles(n_slots, n_experts);
-  return bank->qtype == CAI_Q8_0 ? launch_blk<CAI_Q8_0>(p, tiles) : launch_blk<CAI_Q4_0>(p, tiles);
+  return launch_blk(bank, p, tiles);
 }
 
 }  // namespace cai

@@ -397,6 +397,27 @@ def test_prompt_products_on_wide_tiles(qt, rows, cols, T):
     w.close()
 
 
+@pytest.mark.parametrize("qt", [O.Q8_0, O.Q4_0])
+@pytest.mark.parametrize("rows,cols,T", [(40, 96, 17), (8192, 64, 33), (8193, 544, 65), (9000, 128, 255), (40000, 96, 31), (40000, 128, 32), (40000, 96, 64),
+                                         (40000, 128, 63), (40000, 96, 129), (39937, 192, 128), (66000, 32, 100)])
+def test_prompt_products_on_block_tiles(qt, rows, cols, T):
+    """each form of the block product at its edges: cut tiles of 32 and 64 rows (one and two work-groups a CU), tiles of 256 rows x 64 tokens
+    (half empty, full, one token short) and x 128; rows of an odd and an even number of blocks, one block, one chunk"""
+    from helpers.device import dev, rel_err
+    cai = dev()
+    rng = np.random.default_rng(rows + cols + T)
+    base = O.quantize(qt, (rng.standard_normal((min(rows, 700), cols)) * 0.02).astype(np.float32)).reshape(min(rows, 700), -1)
+    raw = np.ascontiguousarray(base[np.arange(rows) % 700])
+    x = (rng.standard_normal((T, cols)) * rng.uniform(0.01, 30.0, (T, 1))).astype(np.float32)
+    bias = (rng.standard_normal(rows) * 0.1).astype(np.float32)
+    w = cai.QWeight(qt, rows, cols, raw.reshape(-1), bias)
+    got = w.gemm(x)
+    for t in sorted({0, 1, 15, 31, 32, T // 2, 63, 64, T - 2, T - 1} & set(range(T))):
+        want = O.gemv(qt, base.reshape(-1), base.shape[0], cols, x[t:t + 1], None, 0, 1)[0][np.arange(rows) % 700] + bias
+        assert rel_err(got[t], want, floor=0.02 * cols ** 0.5 * float(np.abs(x[t]).mean())) < 2e-5, t
+    w.close()
+
+
 @pytest.mark.parametrize("qt", [O.Q4_K, O.Q5_K])
 def test_prompt_of_a_decoder_on_wide_tiles(qt):
     """q | k | v in one launch of three row groups, gate | up with SwiGLU in the epilogue and behind the slices, residual on a cut product:
@@ -408,6 +429,25 @@ def test_prompt_of_a_decoder_on_wide_tiles(qt):
     spec = synthetic_spec(cfg, qt, head_qtype=O.Q8_0, seed=5, std=0.03, qkv_bias=True)
     dec = cai.Decoder(spec, max_batch=2)
     tok = np.random.default_rng(2).integers(0, 500, 70).astype(np.int32)
+    _, got = dec.prefill(tok)
+    for p_, t in enumerate(tok):
+        _, want = dec.step_window([t], p_, seq=1)
+    assert rel_err(got, want[0]) < 1e-4
+    dec.close()
+
+
+@pytest.mark.parametrize("qt,ffn,T", [(O.Q8_0, 352, 100), (O.Q4_0, 64, 40), (O.Q8_0, 320, 150)])
+def test_prompt_of_a_mixture_on_tiles_of_64_slots(qt, ffn, T):
+    """banks of four experts, two a token: runs of about T / 2 slots in tiles of 64 (full, half empty, a remainder), widths of an odd and an
+    even number of blocks, windows of 704, 128 and 640 rows: a prompt equals its tokens one by one"""
+    from helpers.device import dev, rel_err
+    from helpers.model_build import synthetic_spec
+    cai = dev()
+    cfg = dict(n_layers=2, d_model=256, n_q_heads=4, n_kv_heads=2, head_dim=64, ffn=ffn, vocab=300, max_ctx=256, eps=1e-5, rope_theta=1e4,
+               n_experts=4, top_k=2, norm_topk=1)
+    spec = synthetic_spec(cfg, qt, head_qtype=O.Q8_0, seed=T, std=0.05, qkv_bias=False)
+    dec = cai.Decoder(spec, max_batch=2)
+    tok = np.random.default_rng(3).integers(0, 300, T).astype(np.int32)
     _, got = dec.prefill(tok)
     for p_, t in enumerate(tok):
         _, want = dec.step_window([t], p_, seq=1)
