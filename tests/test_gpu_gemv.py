@@ -453,3 +453,26 @@ def test_prompt_of_a_mixture_on_tiles_of_64_slots(qt, ffn, T):
         _, want = dec.step_window([t], p_, seq=1)
     assert rel_err(got, want[0]) < 1e-4
     dec.close()
+
+
+@pytest.mark.parametrize("cols", [32, 1024, 1056, 2048, 2080, 4096, 4128, 8192, 8224, 24576, 24608])
+def test_prompt_rows_at_the_widths_of_the_pre_pass(cols):
+    """the last and the first width of each number of values a thread keeps, and rows that start one float off alignment"""
+    import torch
+    from helpers.device import dev, rel_err
+    cai = dev()
+    rows, T = 40, 18
+    raw, rng = make(O.Q8_0, rows, cols, cols)
+    x = (rng.standard_normal((T, cols)) * rng.uniform(0.01, 30.0, (T, 1))).astype(np.float32)
+    w = cai.QWeight(O.Q8_0, rows, cols, raw)
+    want = O.gemv(O.Q8_0, raw, rows, cols, x, None, 0, 1)
+    buf, y = torch.zeros(T * cols + 1, device="cuda"), torch.zeros((T, rows), device="cuda")
+    for shift in (0, 1):
+        buf[shift:shift + T * cols].copy_(torch.from_numpy(x).reshape(-1))
+        torch.cuda.synchronize()
+        cai.check(cai.load().cai_qgemm(w.h, cai.C.c_void_p(buf.data_ptr() + 4 * shift), T, cai.C.c_void_p(y.data_ptr()), cai.X_DEVICE | cai.Y_DEVICE))
+        torch.cuda.synchronize()
+        got = y.cpu().numpy()
+        for t in range(T):
+            assert rel_err(got[t], want[t], floor=0.02 * cols ** 0.5 * float(np.abs(x[t]).mean())) < TIGHT, (shift, t)
+    w.close()
