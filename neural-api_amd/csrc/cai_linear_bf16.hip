@@ -192,10 +192,29 @@ __global__ __launch_bounds__(64 * GV_WAVES) void gemv_bf16(const uint16_t* __res
 
 // ------------------------------------------------------------------------------------------
 // Prompts: C^T tile = W tile x activations^T on the matrix cores; a lane ends with four consecutive outputs of one token.
-// Both operand tiles are 128 bytes deep per row (64 bfloat16 or 32 floats), double buffered in LDS; the 16-byte chunks of a row
-// are stored at chunk ^ (row & 7), which makes the fragment reads conflict-free.
+// Both operand tiles are 128 bytes deep per row (64 bfloat16 or 32 floats), DEPTH of them in LDS; the 16-byte chunks of a row
+// are stored at chunk ^ (row & 7), which makes the fragment reads conflict-free.  bfloat16 tiles are copied into LDS asynchronously,
+// DEPTH - 1 steps ahead, with one meeting of the waves a step; float ones are widened on the way, through registers.
+// Bound by the matrix cores and the fragment reads of a step together: sixteen waves of 64 x 32 overlap them better than four of
+// 64 x 64 (whole prompt of 2048 tokens through four layers of width 2048: 2798 us with four waves and staging through registers -> 2546).
 // ------------------------------------------------------------------------------------------
-template <typename AT, int BM, int BN, int WM, int WN, bool BANK, int MODE>   // MODE: e.mode (one epilogue a kernel: with all of them the accumulators would leave their registers)
+// 64 lanes x 16 bytes, each from an address of its own, into 1 KB of LDS at lds (uniform), in lane order.  The compiler does not see
+// the load: the caller waits for it before the barrier that publishes the tile.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"     // (m0 is reserved, and named all the same: the statement changes it)
+__device__ __forceinline__ void copy_to_lds(uint32_t lds, const void* from)
+{
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" :: "s"(lds), "v"(from) : "memory", "m0");
+}
+#pragma clang diagnostic pop
+template <int N> __device__ __forceinline__ void wait_copies()
+{
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
+  asm volatile("" ::: "memory");
+}
+
+template <typename AT, int BM, int BN, int WM, int WN, bool BANK, int MODE, int DEPTH = 2>   // MODE: e.mode (one epilogue a kernel: with all of them the accumulators would leave their registers)
 __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16(const uint16_t* __restrict__ W, const AT* __restrict__ X, int n_rows, int ldw, int64_t ldx, int n_tok, int tiles_m, int n_tiles, LinEpi e, BankList l)
 {
   constexpr int NT = 64 * WM * WN;
@@ -203,7 +222,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16(const uint16_t* __rest
   constexpr int TM = BM / WM / 16, TN = BN / WN / 16;
   constexpr int CA = BM * 8 / NT, CW = BN * 8 / NT;  // 16-byte chunks per thread
   static_assert(CA >= 1 && CW >= 1 && BM * 8 % NT == 0 && BN * 8 % NT == 0 && TN % 2 == 0, "tile shape");
-  __shared__ u32x4 sx[2][BM * 8], sw[2][BN * 8];
+  extern __shared__ u32x4 gm_lds[];                 // DEPTH slots of BM + BN rows of 128 bytes
+  u32x4* const sx_ = gm_lds; u32x4* const sw_ = gm_lds + BM * 8;
+  constexpr int SLOT = (BM + BN) * 8;
   // consecutive work-groups go to different XCDs: give each XCD a contiguous run of tiles, token tiles fastest, so that the
   // work-groups of an XCD share weight rows in its L2
   int tile;
@@ -228,48 +249,26 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16(const uint16_t* __rest
     const int c = tid + i * NT;
     int t = min(m0 + (c >> 3), n_tok - 1);
     if constexpr (BANK) { if (l.div) t = l.order[t] / l.div; }
-    xp[i] = X + (int64_t)t * ldx + (c & 7) * (16 / sizeof(AT));
+    xp[i] = X + (int64_t)t * ldx + ((c ^ (c >> 3)) & 7) * (16 / sizeof(AT));
   }
 #pragma unroll
-  for (int i = 0; i < CW; i++) { const int c = tid + i * NT; wp[i] = W + (int64_t)min(n0 + (c >> 3), n_rows - 1) * ldw + (c & 7) * (16 / sizeof(AT)); }
-  u32x4 rx[CA], rw[CW];
-  auto fetch = [&](int k) {
-#pragma unroll
-    for (int i = 0; i < CA; i++) rx[i] = *reinterpret_cast<const u32x4*>(xp[i] + k);
-#pragma unroll
-    for (int i = 0; i < CW; i++) {
-      if constexpr (sizeof(AT) == 2) rw[i] = *reinterpret_cast<const u32x4*>(wp[i] + k);
-      else {
-        const uint2 u = *reinterpret_cast<const uint2*>(wp[i] + k);
-        rw[i] = u32x4{u.x << 16, u.x & 0xffff0000u, u.y << 16, u.y & 0xffff0000u};
-      }
-    }
-  };
-  auto stash = [&](int s) {
-#pragma unroll
-    for (int i = 0; i < CA; i++) { const int c = tid + i * NT, r = c >> 3; sx[s][r * 8 + ((c & 7) ^ (r & 7))] = rx[i]; }
-#pragma unroll
-    for (int i = 0; i < CW; i++) { const int c = tid + i * NT, r = c >> 3; sw[s][r * 8 + ((c & 7) ^ (r & 7))] = rw[i]; }
-  };
+  for (int i = 0; i < CW; i++) { const int c = tid + i * NT; wp[i] = W + (int64_t)min(n0 + (c >> 3), n_rows - 1) * ldw + ((c ^ (c >> 3)) & 7) * (16 / sizeof(AT)); }
   f32x4 acc[TN][TM];
 #pragma unroll
   for (int j = 0; j < TN; j++)
 #pragma unroll
     for (int i = 0; i < TM; i++) acc[j][i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   const int fr = lane & 15, fc = lane >> 4;
-  fetch(0); stash(0);
-  __syncthreads();
   const int nk = ldw / BK;
-  for (int kt = 0; kt < nk; kt++) {
-    const int s = kt & 1;
-    if (kt + 1 < nk) fetch((kt + 1) * BK);
+  auto multiply = [&](int s) {
+    const u32x4 *const sx = sx_ + s * SLOT, *const sw = sw_ + s * SLOT;
 #pragma unroll
     for (int kk = 0; kk < 2; kk++) {
       u32x4 fx[TM], fw[TN];
 #pragma unroll
-      for (int i = 0; i < TM; i++) { const int r = wm + i * 16 + fr; fx[i] = sx[s][r * 8 + ((kk * 4 + fc) ^ (r & 7))]; }
+      for (int i = 0; i < TM; i++) { const int r = wm + i * 16 + fr; fx[i] = sx[r * 8 + ((kk * 4 + fc) ^ (r & 7))]; }
 #pragma unroll
-      for (int j = 0; j < TN; j++) { const int r = wn + j * 16 + fr; fw[j] = sw[s][r * 8 + ((kk * 4 + fc) ^ (r & 7))]; }
+      for (int j = 0; j < TN; j++) { const int r = wn + j * 16 + fr; fw[j] = sw[r * 8 + ((kk * 4 + fc) ^ (r & 7))]; }
 #pragma unroll
       for (int j = 0; j < TN; j++)
 #pragma unroll
@@ -284,8 +283,53 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16(const uint16_t* __rest
           }
         }
     }
-    if (kt + 1 < nk) stash(s ^ 1);
+  };
+  if constexpr (sizeof(AT) == 2) {
+    // the copies of step kt + DEPTH - 1 go out as soon as every wave has read the slot they fill
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) u32x4*)gm_lds;
+    auto copy = [&](int kt) {
+      const uint32_t dst = lds0 + (uint32_t)(kt % DEPTH * SLOT * 16 + wave * 1024);
+#pragma unroll
+      for (int i = 0; i < CA; i++) copy_to_lds(dst + i * NT * 16, xp[i] + kt * BK);
+#pragma unroll
+      for (int i = 0; i < CW; i++) copy_to_lds(dst + BM * 128 + i * NT * 16, wp[i] + kt * BK);
+    };
+#pragma unroll
+    for (int i = 0; i < DEPTH - 1; i++) if (i < nk) copy(i);
+    for (int kt = 0; kt < nk; kt++) {
+      if (kt + DEPTH - 1 <= nk) wait_copies<(DEPTH - 2) * (CA + CW)>(); else wait_copies<0>();
+      __builtin_amdgcn_s_waitcnt(0xC07F);              // lgkmcnt(0): this wave's reads of the slot that is filled next
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      if (kt + DEPTH - 1 < nk) copy(kt + DEPTH - 1);
+      multiply(kt % DEPTH);
+    }
+  } else {
+    u32x4 rx[CA], rw[CW];
+    auto fetch = [&](int k) {
+#pragma unroll
+      for (int i = 0; i < CA; i++) rx[i] = *reinterpret_cast<const u32x4*>(xp[i] + k);
+#pragma unroll
+      for (int i = 0; i < CW; i++) {
+        const uint2 u = *reinterpret_cast<const uint2*>(wp[i] + k);
+        rw[i] = u32x4{u.x << 16, u.x & 0xffff0000u, u.y << 16, u.y & 0xffff0000u};
+      }
+    };
+    auto stash = [&](int s) {
+#pragma unroll
+      for (int i = 0; i < CA; i++) { const int c = tid + i * NT; sx_[s * SLOT + c] = rx[i]; }
+#pragma unroll
+      for (int i = 0; i < CW; i++) { const int c = tid + i * NT; sw_[s * SLOT + c] = rw[i]; }
+    };
+    fetch(0); stash(0);
     __syncthreads();
+    for (int kt = 0; kt < nk; kt++) {
+      const int s = kt & 1;
+      if (kt + 1 < nk) fetch((kt + 1) * BK);
+      multiply(s);
+      if (kt + 1 < nk) stash(s ^ 1);
+      __syncthreads();
+    }
   }
 #pragma unroll
   for (int i = 0; i < TM; i++) {
@@ -336,21 +380,36 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16(const uint16_t* __rest
   }
 }
 
-template <typename AT, int BM, int BN, int WM, int WN>
-static void run_gemm(const cai_qw_s* w, const AT* x, int64_t ldx, int n_tok, const LinEpi& e)
+template <typename AT, int BM, int BN, int WM, int WN, int MODE, int DEPTH>
+static int run_gemm_mode(const cai_qw_s* w, const AT* x, int64_t ldx, int n_tok, const LinEpi& e)
 {
+  constexpr size_t lds = (size_t)DEPTH * (BM + BN) * 128;
+  if constexpr (lds > 65536) {
+    static bool attr_done = false;
+    if (!attr_done) {
+      CAI_HIP(hipFuncSetAttribute((const void*)gemm_bf16<AT, BM, BN, WM, WN, false, MODE, DEPTH>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+      attr_done = true;
+    }
+  }
   const int tm = (n_tok + BM - 1) / BM, tn = ((int)w->rows + BN - 1) / BN;
-#define GEMM(MODE) case MODE: hipLaunchKernelGGL((gemm_bf16<AT, BM, BN, WM, WN, false, MODE>), dim3(tm * tn), dim3(64 * WM * WN), 0, ctx().stream, \
-                              (const uint16_t*)w->data, x, (int)w->rows, (int)w->ld, ldx, n_tok, tm, tm * tn, e, BankList{}); break
+  hipLaunchKernelGGL((gemm_bf16<AT, BM, BN, WM, WN, false, MODE, DEPTH>), dim3(tm * tn), dim3(64 * WM * WN), lds, ctx().stream,
+                     (const uint16_t*)w->data, x, (int)w->rows, (int)w->ld, ldx, n_tok, tm, tm * tn, e, BankList{});
+  return CAI_OK;
+}
+template <typename AT, int BM, int BN, int WM, int WN, int DEPTH = 2>
+static int run_gemm(const cai_qw_s* w, const AT* x, int64_t ldx, int n_tok, const LinEpi& e)
+{
+#define GEMM(MODE) case MODE: return run_gemm_mode<AT, BM, BN, WM, WN, MODE, DEPTH>(w, x, ldx, n_tok, e)
   switch (e.mode) { GEMM(EPI_STORE); GEMM(EPI_GLU); GEMM(EPI_RESIDUAL); GEMM(EPI_SPLIT); GEMM(EPI_JOIN); }
 #undef GEMM
+  return CAI_OK;
 }
 
 template <typename AT, int BM, int BN>
 static void run_bank(const cai_qw_s* w, int mat_rows, const AT* x, int64_t ldx, const BankList& l, const LinEpi& e)
 {
   const int tm = l.max_tiles, tn = (mat_rows + BN - 1) / BN;
-#define GEMM(MODE) case MODE: hipLaunchKernelGGL((gemm_bf16<AT, BM, BN, 2, 2, true, MODE>), dim3(tm * tn), dim3(256), 0, ctx().stream, \
+#define GEMM(MODE) case MODE: hipLaunchKernelGGL((gemm_bf16<AT, BM, BN, 2, 2, true, MODE>), dim3(tm * tn), dim3(256), (size_t)2 * (BM + BN) * 128, ctx().stream, \
                               (const uint16_t*)w->data, x, mat_rows, (int)w->ld, ldx, 0, tm, tm * tn, e, l); break
   switch (e.mode) { GEMM(EPI_STORE); GEMM(EPI_GLU); GEMM(EPI_SPLIT); }
 #undef GEMM
@@ -421,10 +480,14 @@ static int run_lin(const cai_qw_s* w, const AT* x, int64_t ldx, int n_tok, const
     return CAI_OK;
   }
   auto tiles = [&](int bm, int bn) { return (int64_t)((n_tok + bm - 1) / bm) * ((w->rows + bn - 1) / bn); };
-  if (n_tok > 64 && tiles(128, 128) >= ctx().n_cu) run_gemm<AT, 128, 128, 2, 2>(w, x, ldx, n_tok, e);
-  else if (n_tok > 32 && tiles(64, 64) >= ctx().n_cu) run_gemm<AT, 64, 64, 2, 2>(w, x, ldx, n_tok, e);
-  else run_gemm<AT, 32, 64, 2, 2>(w, x, ldx, n_tok, e);
-  return CAI_OK;
+  // (2048 tokens, a 4-layer decoder of width 2048, its whole prompt: 128 x 128 by four waves 2783 us, by eight 2607, 256 x 128 by sixteen
+  // 2546, 256 x 256 by sixteen 3009; where 128 x 128 leaves CUs idle the halved tiles of 64 x 64 are faster: 511 tokens, width 512: 609, 628)
+  if (n_tok > 64 && tiles(128, 128) >= ctx().n_cu) {
+    if constexpr (sizeof(AT) == 2) return run_gemm<AT, 256, 128, 4, 4, 3>(w, x, ldx, n_tok, e);
+    else return run_gemm<AT, 128, 128, 2, 2>(w, x, ldx, n_tok, e);
+  }
+  if (n_tok > 32 && tiles(64, 64) >= ctx().n_cu) return run_gemm<AT, 64, 64, 2, 2>(w, x, ldx, n_tok, e);
+  return run_gemm<AT, 32, 64, 2, 2>(w, x, ldx, n_tok, e);
 }
 
 int launch_lin_rms(int act_t, const float* x, int64_t ldx, int width, float eps, int n_tok, const RmsLin& a, const RmsLin* b)

@@ -93,6 +93,17 @@ def test_mechanism_alone(cai, tmp_path, mech, i, dt):
     dec.close()
 
 
+@pytest.mark.parametrize("tokens, ff", [(129, 16400), (257, 8208), (300, 12000)])
+def test_products_on_tiles_of_256_tokens(cai, tmp_path, tokens, ff):
+    """gate | up matrices whose products fill the chip with large tiles: tokens one past half a tile, one past a tile and inside a second one, rows
+    that end inside a tile; one and a half steps of depth"""
+    m = Model(tmp_path, B.config([B.layer(B.delta(), ff=ff)], width=72, vocab=67), seed=tokens, edit=only("feed-forward"), rank_a=3, rank_g=20)
+    tok = m.tokens(tokens, 1)
+    dec = m.open(cai, 320, 1, "bf16")
+    check(feed(dec, tok, [tokens]), m.ref(tok), "bf16")
+    dec.close()
+
+
 # ---------------------------------------------------------------- whole models
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
 @pytest.mark.parametrize("cuts", [[300], [1], [2], [3, 2, 65, 1, 1, 16, 17, 2], [64], [130, 1], [5, 9, 7]], ids=str)
