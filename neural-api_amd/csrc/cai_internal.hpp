@@ -272,6 +272,9 @@ int prefill_linear(const cai_qw_s* w, const float* x, int64_t x_stride, const fl
                    float* y, int64_t y_stride, const float* residual);
 bool gemm_mfma_supported(const cai_qw_s* w);   // many-token (prompt) matrix-core kernel of the super-block types (Q4_K, Q6_K)
 bool gemm_blk_supported(const cai_qw_s* w);    // many-token (prompt) matrix-core kernel of the 32-weight block types (Q8_0, Q4_0)
+bool gemm_raw_supported(const cai_qw_s* w);    // many-token products of the types kept as their stored stream (but Q5_K)
+int launch_gemm_raw(const cai_qw_s* w, const _Float16* xhi, const _Float16* xlo, const float* sinv, int n_tok, float* y, int64_t y_stride, const float* residual);
+void raw_release();
 inline bool prompt_gemm_supported(const cai_qw_s* w) { return gemm_mfma_supported(w) || gemm_blk_supported(w); }
 int launch_gemm_blk(const cai_qw_s* w, const _Float16* xhi, const _Float16* xlo, const float* sinv, int n_tok, float* y, int64_t y_stride, const float* residual);
 // mixture-of-experts prompt: slots (token * top_k + rank) grouped by expert, then one launch over the bank per projection

@@ -747,6 +747,7 @@ void prefill_release()   // cai_shutdown
   void* q[] = {g_pws.hi, g_pws.lo, g_pws.sinv, g_pws.sxhi, g_pws.sxlo};
   for (void* v : q) if (v) (void)hipFree(v);
   g_pws = PrefillWs();
+  raw_release();
 }
 
 int prefill_prep(const float* x, int64_t x_stride, const float* gain, float eps, int K, int n_tok)
@@ -792,6 +793,7 @@ int prefill_gemm_swiglu(const cai_qw_s* w, int n_tok, float* y, int64_t y_stride
 void prefill_planes(const _Float16** hi, const _Float16** lo, const float** sinv) { *hi = g_pws.hi; *lo = g_pws.lo; *sinv = g_pws.sinv; }
 int prefill_gemm(const cai_qw_s* w, int n_tok, float* y, int64_t y_stride, const float* residual)
 {
+  if (gemm_raw_supported(w)) return launch_gemm_raw(w, g_pws.hi, g_pws.lo, g_pws.sinv, n_tok, y, y_stride, residual);
   if (gemm_blk_supported(w)) return launch_gemm_blk(w, g_pws.hi, g_pws.lo, g_pws.sinv, n_tok, y, y_stride, residual);
   return launch_gemm_q4k(w, g_pws.hi, g_pws.lo, g_pws.sxhi, g_pws.sxlo, g_pws.sinv, n_tok, y, y_stride, residual);
 }
@@ -806,6 +808,7 @@ int prompt_route(const cai_qw_s* w, int n_tok)
 {
   if (gemm_mfma_supported(w)) return n_tok <= 16 && nb_supported(w) ? 1 : 2;
   if (gemm_blk_supported(w) && n_tok > 16) return 2;
+  if (gemm_raw_supported(w) && n_tok > 8) return 2;
   if (nb_supported(w) && w->data_bytes >= ((int64_t)16 << 20)) return 1;
   return 0;
 }

@@ -19,6 +19,7 @@
 // asynchronous copies along the rows.
 #include "cai_internal.hpp"
 #include "cai_gemv_common.hpp"
+#include "cai_blocks_raw.hpp"
 #include <algorithm>
 #include <type_traits>
 
@@ -29,6 +30,7 @@ namespace {
 typedef _Float16 half2_b __attribute__((ext_vector_type(2)));
 typedef _Float16 half8_b __attribute__((ext_vector_type(8)));
 typedef float float16_b __attribute__((ext_vector_type(16)));
+typedef float f32x4_b __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_b __attribute__((ext_vector_type(4)));   // (arrays of HIP's uint4 struct end up in scratch memory)
 
 struct BlkGemmParams {
@@ -46,6 +48,8 @@ struct BlkGemmParams {
   // matrix i + 1, whose rows land y_off2[i] columns into a y row
   int n_seg; int seg_end[2];
   const uint8_t* q2[2]; const uint8_t* d2[2]; const float* bias2[2]; int rows2[2]; int y_off2[2];
+  // types with minima: a weight is d * code + m16 of its sixteen; s16 = sums of sixteen activations [x row][cols / 16] in the planes' scale
+  const float* m16; const float* s16;
 };
 
 // eight codes (two dwords) -> eight exact halfs.  Q8_0: signed bytes; Q4_0: (nibble - 8), low or high nibbles of the bytes
@@ -294,13 +298,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // Places in LDS: 16-byte piece c of token row t (128 bytes a plane) at c ^ (t / 2 % 8), of Q8_0 weight row n (64 bytes) at c ^ (n / 4 % 4),
 // of Q4_0 row n (32 bytes) at c ^ (n / 8 % 2): the lanes of a read pass then meet different banks.
 // ------------------------------------------------------------------------------------------
-template <int QT, int RT, int NW, bool ODD>     // ODD: rows of an odd number of blocks (scales that are not aligned to 4 bytes, a last chunk of one block)
+template <int QT, int RT, int NW, bool ODD, bool MIN = false>     // ODD: rows of an odd number of blocks (scales that are not aligned to 4 bytes, a last chunk of one block)
 __global__ __launch_bounds__(64 * NW) void gemm_blk_cut(const BlkGemmParams p)
 {
   extern __shared__ __align__(16) unsigned char bl_smem[];
   constexpr int WROW = QT == CAI_Q8_0 ? 64 : 32, NV = RT * 16;                 // quant bytes of a row's chunk; values of a lane
-  constexpr int XB = 8192, WB = 32 * WROW, SLOT = XB + RT * WB + (ODD ? 512 : 256);          // a chunk: planes hi, lo; quants; scales
-  constexpr int COPIES = 8 + RT * WB / 1024 + (ODD ? 2 : 1);
+  constexpr int XB = 8192, WB = 32 * WROW, DB = ODD ? 512 : 256, MB = RT * WB + XB + DB, SLOT = MB + (MIN ? 512 + 512 * RT : 0);          // a chunk: planes hi, lo; quants; scales
+  constexpr int COPIES = 8 + RT * WB / 1024 + (ODD ? 2 : 1) + (MIN ? 2 + 2 * RT : 0);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 31, kg = lane >> 5;
   const int L = blockIdx.x;
@@ -336,6 +340,10 @@ __global__ __launch_bounds__(64 * NW) void gemm_blk_cut(const BlkGemmParams p)
   const uint32_t dof = (uint32_t)min(RT == 2 ? lane : n, rlast) * (uint32_t)(nb32 * 2);
   const uint8_t* const qb = qbase + (int64_t)R0 * nb32 * (WROW / 2);
   const uint8_t* const db = dbase + (int64_t)R0 * nb32 * 2;
+  // (MIN) lanes of a copy: token n, sixteen 2 i + kg; rows: RT = 2 row `lane`, sixteen i, RT = 1 row n, sixteen i + kg
+  const uint32_t sof = MIN ? (uint32_t)min(first + n, p.n_tok - 1) * (uint32_t)(K / 4) + 4u * (uint32_t)kg : 0u;
+  const uint32_t mof = MIN ? (uint32_t)min(RT == 2 ? lane : n, rlast) * (uint32_t)(K / 4) + (RT == 2 ? 0u : 4u * (uint32_t)kg) : 0u;
+  const char* const mb = MIN ? reinterpret_cast<const char*>(p.m16) + (int64_t)R0 * (K / 4) : nullptr;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)bl_smem + (uint32_t)(wave * 2 * SLOT);
   auto copy = [&](int c, int slot) {
     const uint32_t dst = lds0 + (uint32_t)(slot * SLOT);
@@ -353,6 +361,14 @@ __global__ __launch_bounds__(64 * NW) void gemm_blk_cut(const BlkGemmParams p)
       copy_short(dst + XB + RT * WB, dof, db + (int64_t)c * 4);
       copy_short(dst + XB + RT * WB + 256, dof, db + (int64_t)c * 4 + (half ? 0 : 2));
     } else copy_dword(dst + XB + RT * WB, dof, db + (int64_t)c * 4);
+    if constexpr (MIN) {                   // [sixteen of the chunk][token or row]; past the width (the last chunk of ODD) the ones before again
+#pragma unroll
+      for (int i = 0; i < 2; i++) copy_dword(dst + MB + 256 * i, sof + (uint32_t)(8 * i), reinterpret_cast<const char*>(p.s16) + (int64_t)c * 16 - (half && i ? 8 : 0));
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        if (RT == 2 || (i & 1) == 0)
+          copy_dword(dst + MB + 512 + 256 * (RT == 2 ? i : i >> 1), mof + (uint32_t)(4 * i), mb + (int64_t)c * 16 - (half && i >= 2 ? 8 : 0));
+    }
   };
   float16_b Y[RT];
 #pragma unroll
@@ -400,6 +416,22 @@ __global__ __launch_bounds__(64 * NW) void gemm_blk_cut(const BlkGemmParams p)
 #pragma unroll
         for (int v = 0; v < 16; v++) Y[rt][v] = fmaf(dv, C[v], Y[rt][v]);
       }
+      if constexpr (MIN)
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+          const int g16 = 2 * b + e;
+          const float* const sp = reinterpret_cast<const float*>(s0 + MB) + 32 * g16 + 4 * kg;
+          const float* const mp = reinterpret_cast<const float*>(s0 + MB + 512);
+          f32x4_b sv[4];
+#pragma unroll
+          for (int g = 0; g < 4; g++) sv[g] = *reinterpret_cast<const f32x4_b*>(sp + 8 * g);
+#pragma unroll
+          for (int rt = 0; rt < RT; rt++) {
+            const float m = mp[32 * RT * g16 + 32 * rt + n];
+#pragma unroll
+            for (int v = 0; v < 16; v++) Y[rt][v] = fmaf(m, sv[v >> 2][v & 3], Y[rt][v]);
+          }
+        }
     }
   };
   if (c0 < c1) copy(c0, 0);
@@ -549,6 +581,128 @@ int launch_blk(const cai_qw_s* w, const BlkGemmParams& p0, int n_tiles_grouped)
   return CAI_OK;
 }
 
+// ------------------------------------------------------------------------------------------
+// Types kept as their stored stream (Q2_K, Q3_K, Q4_1, Q5_0, Q5_1): a panel of rows at a time is rewritten as signed bytes with an f16 scale
+// a block of 32 - and, for the types with minima, a float a sixteen - and multiplied by the kernel above.  Codes and scales are exact:
+// Q5_0 q - 16; Q4_1, Q5_1 q - 8, q - 16 with m + 8 d, m + 16 d; Q3_K (32 - scale) * q with -d; Q2_K scale * (q - 2) with 2 d scale - dmin min.
+// (Codes about zero: with q from 0 up the two parts of a sum cancel, and its error doubles.)
+// In place of passes of eight tokens through the float walk, bound by its VALU work: 18944 x 3584 with 200 tokens Q3_K 2282 -> 166 us,
+// Q4_1 1321 -> 253, with 16 tokens 183 -> 74, 106 -> 90; 3584 x 3584 with 16 tokens 52 -> 24, 39 -> 30.  Rewriting takes about 2 bytes of
+// memory traffic a weight (40 us of the first), the minima half the time of the products; up to eight tokens the walk is one pass and stays.
+// ------------------------------------------------------------------------------------------
+template <int QT>
+__global__ __launch_bounds__(256) void raw_expand_kernel(const uint8_t* __restrict__ raw, int64_t row_bytes, int n_rows, int runs, int8_t* __restrict__ q, uint16_t* __restrict__ d, float* __restrict__ m16)
+{
+  const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (id >= (int64_t)n_rows * runs) return;
+  const int row = (int)(id / runs), run = (int)(id % runs);
+  const uint8_t* const base = raw + row * row_bytes;
+  uint32_t out[4]; float m = 0.0f; uint16_t dh;
+  auto put = [&](int t, int v) { const uint32_t byte = (uint32_t)(v & 255) << (8 * (t & 3)); out[t >> 2] = (t & 3) ? out[t >> 2] | byte : byte; };
+  constexpr int BB = raw_block_bytes(QT);
+  if constexpr (raw_block_elems(QT) == 32) {
+    const uint8_t* const blk = base + (int64_t)(run >> 1) * BB;
+    const int half = run & 1;
+    uint32_t qs[4];
+    raw_load16<QT == CAI_Q5_0 ? 2 : 4>(blk + (QT == CAI_Q4_1 ? 4 : QT == CAI_Q5_0 ? 6 : 8), qs);
+    dh = *reinterpret_cast<const uint16_t*>(blk);
+    const uint32_t qh = QT == CAI_Q4_1 ? 0u : (QT == CAI_Q5_0 ? raw_u32_a2(blk + 2) : *reinterpret_cast<const uint32_t*>(blk + 4)) >> (16 * half);
+#pragma unroll
+    for (int t = 0; t < 16; t++) {
+      const int b = raw_byte(qs, t), nib = half ? (b >> 4) : (b & 15);
+      put(t, QT == CAI_Q4_1 ? nib - 8 : (nib | (int)(((qh >> t) & 1u) << 4)) - 16);
+    }
+    if constexpr (QT != CAI_Q5_0) m = fmaf(raw_half(blk), QT == CAI_Q4_1 ? 8.0f : 16.0f, raw_half(blk + 2));
+  } else {
+    const uint8_t* const blk = base + (int64_t)(run >> 4) * BB;
+    const int r = run & 15, sh = 2 * ((r >> 1) & 3);
+    uint32_t qs[4];
+    if constexpr (QT == CAI_Q2_K) {
+      const int sc = blk[r] & 15, mn = blk[r] >> 4;
+      raw_load16<4>(blk + 16 + (r >> 3) * 32 + 16 * (r & 1), qs);
+      dh = *reinterpret_cast<const uint16_t*>(blk + 80);
+#pragma unroll
+      for (int t = 0; t < 16; t++) put(t, sc * (((raw_byte(qs, t) >> sh) & 3) - 2));
+      m = fmaf(raw_half(blk + 80), (float)(2 * sc), -(raw_half(blk + 82) * (float)mn));
+    } else {
+      const int sc = -q3k_scale(blk + 96, r), bit = r >> 1;
+      uint32_t hm[4];
+      raw_load16<2>(blk + 32 + (r >> 3) * 32 + 16 * (r & 1), qs);
+      raw_load16<2>(blk + 16 * (r & 1), hm);
+      dh = *reinterpret_cast<const uint16_t*>(blk + 108) ^ 0x8000u;
+#pragma unroll
+      for (int t = 0; t < 16; t++) put(t, sc * (((raw_byte(qs, t) >> sh) & 3) - ((((raw_byte(hm, t) >> bit) & 1) ^ 1) << 2)));
+    }
+  }
+  *reinterpret_cast<uint4*>(q + id * 16) = make_uint4(out[0], out[1], out[2], out[3]);
+  if ((run & 1) == 0) d[id >> 1] = dh;
+  if constexpr (QT == CAI_Q2_K || QT == CAI_Q4_1 || QT == CAI_Q5_1) m16[id] = m;
+}
+
+// sums of sixteen neighbours of the activation planes
+__global__ __launch_bounds__(256) void plane_sums_kernel(const _Float16* __restrict__ hi, const _Float16* __restrict__ lo, int64_t n, float* __restrict__ s16)
+{
+  const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;      // eight values each
+  if (id >= n) return;
+  const half8_b h = *reinterpret_cast<const half8_b*>(hi + id * 8), l = *reinterpret_cast<const half8_b*>(lo + id * 8);
+  float s = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 8; i++) s += (float)h[i] + (float)l[i];
+  s += __shfl_xor(s, 1);
+  if ((id & 1) == 0) s16[id >> 1] = s;
+}
+
+struct RawWs { uint8_t* q = nullptr; float* s16 = nullptr; size_t q_cap = 0, s_cap = 0; };
+RawWs g_raw;
+constexpr int64_t RAW_PANEL = (int64_t)64 << 20;       // weights of a panel: its bytes stay in the last-level cache between the two launches
+
+template <int QT>
+int launch_raw(const cai_qw_s* w, const BlkGemmParams& p0)
+{
+  constexpr bool MIN = QT == CAI_Q2_K || QT == CAI_Q4_1 || QT == CAI_Q5_1;
+  const int64_t K = w->cols, rows = w->rows;
+  const int64_t panel = std::min((rows + 63) / 64 * 64, std::max<int64_t>(64, RAW_PANEL / K / 64 * 64));
+  const size_t q_need = (size_t)panel * K * 21 / 16, s_need = MIN ? (size_t)p0.n_tok * K / 16 : 0;    // bytes: code 1, f16 scale 1 / 16, float minimum 4 / 16
+  if (q_need > g_raw.q_cap || s_need > g_raw.s_cap) {
+    CAI_HIP(hipStreamSynchronize(ctx().stream));
+    const size_t qc = std::max(q_need, g_raw.q_cap), sc = std::max(s_need, g_raw.s_cap);
+    raw_release();
+    if (qc) { CAI_HIP(hipMalloc((void**)&g_raw.q, qc)); g_raw.q_cap = qc; }
+    if (sc) { CAI_HIP(hipMalloc((void**)&g_raw.s16, sc * 4)); g_raw.s_cap = sc; }
+  }
+  hipStream_t st = ctx().stream;
+  if (MIN) {
+    const int64_t n8 = (int64_t)p0.n_tok * K / 8;
+    hipLaunchKernelGGL(plane_sums_kernel, dim3((unsigned)((n8 + 255) / 256)), dim3(256), 0, st, p0.xhi, p0.xlo, n8, g_raw.s16);
+  }
+  const int64_t row_bytes = K / raw_block_elems(QT) * raw_block_bytes(QT);
+  const int n_cu = ctx().n_cu, tok32 = (p0.n_tok + 31) / 32;
+  for (int64_t r0 = 0; r0 < rows; r0 += panel) {
+    BlkGemmParams p = p0;
+    const int n = (int)std::min(panel, rows - r0), runs = (int)(K / 16);
+    uint16_t* const d = reinterpret_cast<uint16_t*>(g_raw.q + panel * K);
+    float* const m16 = reinterpret_cast<float*>(g_raw.q + panel * K / 16 * 17);
+    hipLaunchKernelGGL(raw_expand_kernel<QT>, dim3((unsigned)(((int64_t)n * runs + 255) / 256)), dim3(256), 0, st, w->data + r0 * row_bytes, row_bytes, n, runs, (int8_t*)g_raw.q, d, m16);
+    p.q = g_raw.q; p.d = reinterpret_cast<const uint8_t*>(d); p.rows = n; p.m16 = m16; p.s16 = g_raw.s16;
+    if (p.bias) p.bias += r0;
+    p.y += r0;
+    if (p.residual) p.residual += r0;
+    auto cut = [&](auto rt_, auto nw_, auto odd_) {
+      constexpr int RT = rt_, NW = nw_; constexpr bool ODD = odd_;
+      return launch_lds<gemm_blk_cut<CAI_Q8_0, RT, NW, ODD, MIN>>(blk_grid(p, 32 * RT, tok32), 64 * NW, NW * 2 * (8192 + RT * 2048 + (ODD ? 512 : 256) + (MIN ? 512 + 512 * RT : 0)), p);
+    };
+    // (always cut tiles, whose sums are short chains: 1.4e-7 off 64 bits at width 3584, as the float walk of eight tokens a pass; large tiles 2e-7)
+    auto form = [&](auto odd_) {
+      if ((int64_t)((n + 31) / 32) * tok32 <= n_cu) return cut(std::integral_constant<int, 1>(), std::integral_constant<int, 6>(), odd_);
+      if ((int64_t)((n + 63) / 64) * tok32 <= n_cu || MIN) return cut(std::integral_constant<int, 2>(), std::integral_constant<int, 4>(), odd_);
+      return cut(std::integral_constant<int, 2>(), std::integral_constant<int, 3>(), odd_);
+    };
+    const int rc = (K >> 5) & 1 ? form(std::true_type()) : form(std::false_type());
+    if (rc) return rc;
+  }
+  return CAI_OK;
+}
+
 }  // namespace
 
 bool gemm_blk_supported(const cai_qw_s* w) { return (w->qtype == CAI_Q8_0 || w->qtype == CAI_Q4_0) && w->cols % 32 == 0; }
@@ -583,6 +737,37 @@ int launch_gemm_blk_multi(const cai_qw_s* const* ws, const int* y_off, int n_w, 
   p.x_div = 1; p.expert_rows = 0; p.n_seg = n_w;
   for (int i = 1; i < n_w; i++) { p.q2[i - 1] = ws[i]->data; p.d2[i - 1] = ws[i]->aux; p.bias2[i - 1] = ws[i]->bias; p.rows2[i - 1] = (int)ws[i]->rows; p.y_off2[i - 1] = y_off[i] - y_off[0]; }
   return launch_blk(w, p, 0);
+}
+
+bool gemm_raw_supported(const cai_qw_s* w) { return w->qtype == CAI_Q2_K || w->qtype == CAI_Q3_K || w->qtype == CAI_Q4_1 || w->qtype == CAI_Q5_0 || w->qtype == CAI_Q5_1; }
+void raw_release()
+{
+  if (g_raw.q) (void)hipFree(g_raw.q);
+  if (g_raw.s16) (void)hipFree(g_raw.s16);
+  g_raw = RawWs();
+}
+int launch_gemm_raw(const cai_qw_s* w, const _Float16* xhi, const _Float16* xlo, const float* sinv, int n_tok, float* y, int64_t y_stride, const float* residual)
+{
+  if (!gemm_raw_supported(w)) return set_error(CAI_ERR_UNSUPPORTED, "prompt gemm: weight type %d", w->qtype);
+  // (activation rows at 32-bit byte offsets, the sums of sixteen bounded: pieces of whole tiles)
+  const int64_t most = std::max<int64_t>(32, std::min<int64_t>(4096, ((int64_t)1 << 31) / w->cols) / 32 * 32);
+  for (int64_t t = 0; t < n_tok; t += most) {
+    BlkGemmParams p{};
+    p.bias = w->bias; p.cols = (int)w->cols; p.x_div = 1;
+    p.n_tok = (int)std::min<int64_t>(most, n_tok - t);
+    p.xhi = xhi + t * w->cols; p.xlo = xlo + t * w->cols; p.sinv = sinv + t; p.y = y + t * y_stride; p.y_stride = y_stride;
+    p.residual = residual ? residual + t * y_stride : nullptr;
+    int rc;
+    switch (w->qtype) {
+      case CAI_Q2_K: rc = launch_raw<CAI_Q2_K>(w, p); break;
+      case CAI_Q3_K: rc = launch_raw<CAI_Q3_K>(w, p); break;
+      case CAI_Q4_1: rc = launch_raw<CAI_Q4_1>(w, p); break;
+      case CAI_Q5_0: rc = launch_raw<CAI_Q5_0>(w, p); break;
+      default: rc = launch_raw<CAI_Q5_1>(w, p); break;
+    }
+    if (rc) return rc;
+  }
+  return CAI_OK;
 }
 
 // Token tiles of the grouped launches: every expert may end with a partial tile

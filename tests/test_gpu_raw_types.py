@@ -303,3 +303,43 @@ def test_q5_k_m_like_decoder_long_prompt_and_batched_generation():
         for b in range(3):
             assert rel_err(lg[b], lo) < TOL and int(tok[b]) == n_o
     dec.close()
+
+
+@pytest.mark.parametrize("qt", RAW[1:])
+@pytest.mark.parametrize("rows,cols,T", [(1, 256, 9), (65, 512, 33), (300, 3584, 64), (8200, 256, 70), (8300, 512, 40), (17000, 256, 31), (3600, 18944, 10), (40, 4096, 4100)])
+def test_prompt_products_of_a_stored_stream(qt, rows, cols, T):
+    """more tokens than a pass of the float walk: tiles of 32 and 64 rows, row and token remainders, a matrix of more than one panel, more tokens
+    than a piece"""
+    from helpers.device import dev, rel_err
+    cai = dev()
+    rng = np.random.default_rng(rows + cols + T + qt)
+    n = min(rows, 400)
+    base = O.quantize(qt, (rng.standard_normal((n, cols)) * 0.02).astype(np.float32)).reshape(n, -1)
+    raw = np.ascontiguousarray(base[np.arange(rows) % n])
+    x = (rng.standard_normal((T, cols)) * rng.uniform(0.01, 30.0, (T, 1))).astype(np.float32)
+    x[0, : cols // 2] = 0.0
+    bias = (rng.standard_normal(rows) * 0.1).astype(np.float32)
+    w = cai.QWeight(qt, rows, cols, raw.reshape(-1), bias)
+    got = w.gemm(x)
+    for t in sorted({0, 1, 8, 31, 32, T // 2, T - 2, T - 1} & set(range(T))):
+        want = O.gemv(qt, base.reshape(-1), n, cols, x[t:t + 1], None, 0, 1)[0][np.arange(rows) % n] + bias
+        assert rel_err(got[t], want, floor=0.02 * cols ** 0.5 * float(np.abs(x[t]).mean())) < TIGHT, t
+    w.close()
+
+
+@pytest.mark.parametrize("qt,cols", [(q, c) for q in RAW[1:] for c in ((256, 512) if q in (O.Q2_K, O.Q3_K) else (32, 64, 96, 544))])
+def test_prompt_products_of_arbitrary_bytes(qt, cols):
+    """every code, scale and minimum, picked out by unit vectors; widths of an odd and an even number of blocks"""
+    from helpers.device import dev
+    from test_oracle_codecs_other import random_blocks
+    cai = dev()
+    rows, be = 130, 256 if qt in (O.Q2_K, O.Q3_K) else 32
+    raw = random_blocks(qt, rows * cols // be, seed=70 + qt + cols).reshape(-1)
+    w = cai.QWeight(qt, rows, cols, raw)
+    want = O.dequant(qt, raw, rows * cols).reshape(rows, cols)
+    got = w.gemm(np.eye(cols, dtype=np.float32)).T
+    # a weight with a minimum is two products of halves and small integers, each rounded once: 2^-23 of the block's largest part
+    size = np.abs(want).reshape(rows, -1, be).max(2).repeat(be, 1)
+    ok = np.abs(got - want) <= (0.0 if qt in (O.Q3_K, O.Q5_0) else 4e-6) * size
+    assert ok.all(), (int((~ok).sum()), float((np.abs(got - want) / size).max()))
+    w.close()
