@@ -429,10 +429,10 @@ static int enqueue_prefill_chunk(cai_decoder_s* d, int seq, int n)
                                  c.qk_norm_full ? L.v[CAI_V_Q_NORM] : nullptr, c.qk_norm_full ? L.v[CAI_V_K_NORM] : nullptr, c.eps))) return rc;
     if ((rc = linear_rows(L.w[CAI_W_O], false, d->patt, qw, nullptr, 0.0f, n, d->px, dm, d->px))) return rc;
     if (c.n_experts > 0) {
-      // experts differ from token to token.  A chunk of more than 16 tokens whose banks the block prompt kernel takes is
+      // experts differ from token to token.  A chunk of more than 8 tokens whose banks the block prompt kernel takes is
       // sorted by expert and runs each projection as ONE launch over the bank; otherwise the routed half runs on groups of
       // rows (one router / top-k launch per group, the gathered products per token)
-      if (n > 16 && d->pm_gu && gemm_blk_supported(L.w[CAI_W_GATEUP]) && gemm_blk_supported(L.w[CAI_W_DOWN]) &&
+      if (n > 8 && d->pm_gu && gemm_blk_supported(L.w[CAI_W_GATEUP]) && gemm_blk_supported(L.w[CAI_W_DOWN]) &&
           (int64_t)n * c.top_k * I < ((int64_t)1 << 31)) {   // (an activation row of the grouped products lies at a 32-bit byte offset)
         if ((rc = moe_ffn_prompt(d, L, n))) return rc;
         continue;

@@ -801,15 +801,19 @@ int prefill_gemm(const cai_qw_s* w, int n_tok, float* y, int64_t y_stride, const
 // Which kernel family takes n_tok tokens of this matrix: 1 = small-batch matrix-core kernel (passes of up to 8 or 16 tokens;
 // the bandwidth-bound regime), 2 = prompt kernel on prepared activation planes, 0 = matrix-vector kernel in passes of 8.
 //   Q4_K, Q6_K: up to 16 tokens small-batch, above that the prompt kernel;
-//   Q8_0, Q4_0: above 16 tokens the prompt kernel; below, small-batch only for a matrix too large for the cache (a small
-//               one stays resident: one VALU launch per 8 tokens is cheaper than three launches);
+//   Q8_0, Q4_0: above 16 tokens the prompt kernel; below, small-batch for a matrix too large for the cache, and for a small one
+//               the prompt kernel above 8 tokens (16 of 2048 x 2048 9.5 us against 15.5 in passes of 8, of 3584 x 3584 12.7, 44) and
+//               below where the walk over all products (0.18 us a million) is longer than a tile's over the width (3 ns a column)
+//               and the pre-pass: 8 of 3584 x 3584 11.9, 21.7, 4 of them 12.1, 10.5; 8 of 2048 x 2048 9.0, 7.8;
+//   Q2_K, Q3_K, Q4_1, Q5_0, Q5_1: above 8 tokens the prompt kernel on rewritten panels;
 //   per-row int8: small-batch for a large matrix.
 int prompt_route(const cai_qw_s* w, int n_tok)
 {
   if (gemm_mfma_supported(w)) return n_tok <= 16 && nb_supported(w) ? 1 : 2;
-  if (gemm_blk_supported(w) && n_tok > 16) return 2;
+  const bool large = w->data_bytes >= ((int64_t)16 << 20);
+  if (gemm_blk_supported(w) && (n_tok > 16 || (!large && (n_tok > 8 || (n_tok > 1 && n_tok * w->rows * w->cols >= 22000000 + 16000 * w->cols))))) return 2;
   if (gemm_raw_supported(w) && n_tok > 8) return 2;
-  if (nb_supported(w) && w->data_bytes >= ((int64_t)16 << 20)) return 1;
+  if (nb_supported(w) && large) return 1;
   return 0;
 }
 

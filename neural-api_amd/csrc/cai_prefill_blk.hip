@@ -293,13 +293,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // Each wave copies chunks of 64 columns (token planes, quants, scales) along the rows into LDS of its own, one chunk ahead of the one
 // it multiplies, so there is no barrier before the end.  An operand load straight from memory touches 32 rows, a line each, and takes
 // four times the cycles of the same bytes read along the rows: that form, also cut, took 15.2 us where this one takes 10.7.
+// Sums are taken in two steps: one chain over a wave's share of 18944 columns is 1.9e-7 off 64 bits, two short ones 1.2e-7, as the
+// one-token kernels are (1 % of the time).
 // What bounds it: the copies, 66 KB/us into one CU.  576 x 1536, 37 tokens, with the pre-pass of the activations: 23.1 us as 10 uncut
 // tiles of 128 x 32 -> 10.7; 64 x 2048, 255 tokens: 27 -> 14; 2048 x 2048, 255: 31 -> 17.5.
 // Places in LDS: 16-byte piece c of token row t (128 bytes a plane) at c ^ (t / 2 % 8), of Q8_0 weight row n (64 bytes) at c ^ (n / 4 % 4),
 // of Q4_0 row n (32 bytes) at c ^ (n / 8 % 2): the lanes of a read pass then meet different banks.
 // ------------------------------------------------------------------------------------------
 template <int QT, int RT, int NW, bool ODD, bool MIN = false>     // ODD: rows of an odd number of blocks (scales that are not aligned to 4 bytes, a last chunk of one block)
-__global__ __launch_bounds__(64 * NW) void gemm_blk_cut(const BlkGemmParams p)
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_blk_cut(const BlkGemmParams p)
 {
   extern __shared__ __align__(16) unsigned char bl_smem[];
   constexpr int WROW = QT == CAI_Q8_0 ? 64 : 32, NV = RT * 16;                 // quant bytes of a row's chunk; values of a lane
@@ -370,11 +372,11 @@ __global__ __launch_bounds__(64 * NW) void gemm_blk_cut(const BlkGemmParams p)
           copy_dword(dst + MB + 512 + 256 * (RT == 2 ? i : i >> 1), mof + (uint32_t)(4 * i), mb + (int64_t)c * 16 - (half && i >= 2 ? 8 : 0));
     }
   };
-  float16_b Y[RT];
+  float16_b Y[RT], Z[RT];                  // sums of eight (RT = 2: sixteen) blocks, sums of those: see the end of the comment above
 #pragma unroll
   for (int rt = 0; rt < RT; rt++)
 #pragma unroll
-    for (int v = 0; v < 16; v++) Y[rt][v] = 0.0f;
+    for (int v = 0; v < 16; v++) Y[rt][v] = Z[rt][v] = 0.0f;
   const float16_b zero16 = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
   const unsigned char* const mine = bl_smem + wave * 2 * SLOT;
   auto use = [&](int slot, bool half) {
@@ -443,13 +445,18 @@ __global__ __launch_bounds__(64 * NW) void gemm_blk_cut(const BlkGemmParams p)
       wait_loads<COPIES>();
     } else wait_loads<0>();
     use(slot, ODD && c == n_chunks - 1);
+    if (((c - c0) & (RT == 1 ? 3 : 7)) == (RT == 1 ? 3 : 7))
+#pragma unroll
+      for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) { Z[rt][v] += Y[rt][v]; Y[rt][v] = 0.0f; }
   }
   __syncthreads();                         // (every wave's copies have been waited for)
   float* const sacc = reinterpret_cast<float*>(bl_smem);     // [wave][RT 16][64 lanes]
 #pragma unroll
   for (int rt = 0; rt < RT; rt++)
 #pragma unroll
-    for (int v = 0; v < 16; v++) sacc[(wave * NV + rt * 16 + v) * 64 + lane] = Y[rt][v];
+    for (int v = 0; v < 16; v++) sacc[(wave * NV + rt * 16 + v) * 64 + lane] = Z[rt][v] + Y[rt][v];
   __syncthreads();
   // wave w sums the values w, w + NW, ...: the lane's value v of row tile rt is weight row n and token 8 (v / 4) + 4 kg + v % 4
 #pragma unroll

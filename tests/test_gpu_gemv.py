@@ -398,7 +398,7 @@ def test_prompt_products_on_wide_tiles(qt, rows, cols, T):
 
 
 @pytest.mark.parametrize("qt", [O.Q8_0, O.Q4_0])
-@pytest.mark.parametrize("rows,cols,T", [(40, 96, 17), (8192, 64, 33), (8193, 544, 65), (9000, 128, 255), (40000, 96, 31), (40000, 128, 32), (40000, 96, 64),
+@pytest.mark.parametrize("rows,cols,T", [(40, 96, 17), (300, 544, 9), (3584, 3584, 8), (2048, 8192, 16), (8192, 64, 33), (8193, 544, 65), (9000, 128, 255), (40000, 96, 31), (40000, 128, 32), (40000, 96, 64),
                                          (40000, 128, 63), (40000, 96, 129), (39937, 192, 128), (66000, 32, 100)])
 def test_prompt_products_on_block_tiles(qt, rows, cols, T):
     """each form of the block product at its edges: cut tiles of 32 and 64 rows (one and two work-groups a CU), tiles of 256 rows x 64 tokens
