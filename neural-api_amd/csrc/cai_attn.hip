@@ -1311,7 +1311,7 @@ __global__ __launch_bounds__(256) void kv_append_rows_i8_kernel(const AttnParams
 
 // ------------------------------------------------------------------------------------------
 // Prompt ingestion on the matrix cores: every prompt token attends over the cached rows up to its own position.
-// Work-group = (KV head, four query heads of its group, 32 consecutive tokens); wave w takes head h0 + w.  K and V
+// Work-group = (KV head, four query heads of its group, 32 consecutive tokens); wave w takes head h0 + w.  Heads are HD = 128 or 64 wide.  K and V
 // tiles of 32 cached rows are staged in LDS (V transposed) and shared by the four waves.  Per tile and wave:
 //   S^T[row][token] = K . q^T   on v_mfma_f32_32x32x8_f16: the result lane holds ONE token column, so the running
 //                               maximum, the normaliser and the rescaling of the output are per-lane scalars, and the
@@ -1323,14 +1323,14 @@ typedef float pf16_t __attribute__((ext_vector_type(16)));
 
 struct PromptParams {
   const float* qkv; int64_t qkv_stride;      // rows [Q | K | V], K and V already appended to the cache
-  _Float16* qhi; _Float16* qlo;              // [token][q_heads * 128] rotated q, hi + lo
-  const void* kc; const void* vc;            // this sequence's layer plane: [kv_head][max_ctx][128]
+  _Float16* qhi; _Float16* qlo;              // [token][q_heads * HD] rotated q, hi + lo
+  const void* kc; const void* vc;            // this sequence's layer plane: [kv_head][max_ctx][HD]
   const float* ksc; const float* vsc;        // int8 cache: row scales of the same plane, [kv_head][max_ctx]
   int q_heads, kv_heads, max_ctx, n_tok, window;
   float softcap, inv_sqrt;
   const float* theta; const int32_t* pos;
   float* out; int64_t out_stride;
-  float* part;                               // [token][q_head][K split][128 + 2]: unnormalised sums, maximum, normaliser
+  float* part;                               // [token][q_head][K split][HD + 2]: unnormalised sums, maximum, normaliser
 };
 
 constexpr int PA_KT_MIN = 2;     // K tiles (of 32 cached rows) a split takes at least
@@ -1346,13 +1346,14 @@ __device__ __forceinline__ void prompt_k_range(const PromptParams& p, int t0, in
 }
 
 // rotated q (neural/neural.cl:1517-1542) as two f16 planes
+template <int HD>
 __device__ __forceinline__ void prompt_q_row(const PromptParams& p)
 {
-  const int t = blockIdx.x, qw = p.q_heads * 128;
+  const int t = blockIdx.x, qw = p.q_heads * HD;
   const float* row = p.qkv + (int64_t)t * p.qkv_stride;
   const int pos = p.pos[t];
   for (int e = threadIdx.x; e < (qw >> 1); e += 256) {
-    const int d = (2 * e) & 127;
+    const int d = (2 * e) & (HD - 1);
     float x0 = row[2 * e], x1 = row[2 * e + 1];
     if (p.theta) {
       float sn, cs; sincosf((float)pos * p.theta[d >> 1], &sn, &cs);
@@ -1365,22 +1366,24 @@ __device__ __forceinline__ void prompt_q_row(const PromptParams& p)
     p.qlo[(int64_t)t * qw + 2 * e] = l0; p.qlo[(int64_t)t * qw + 2 * e + 1] = l1;
   }
 }
-__global__ __launch_bounds__(256) void prompt_q_kernel(const PromptParams p) { prompt_q_row(p); }
+template <int HD>
+__global__ __launch_bounds__(256) void prompt_q_kernel(const PromptParams p) { prompt_q_row<HD>(p); }
 // one launch per chunk for both: the token's K and V rows into the cache, its rotated q into the planes
-template <typename KV_T>
-__global__ __launch_bounds__(256) void prompt_rows_kernel(const AttnParams p, const PromptParams pp) { kv_append_row<KV_T>(p); prompt_q_row(pp); }
+template <typename KV_T, int HD>
+__global__ __launch_bounds__(256) void prompt_rows_kernel(const AttnParams p, const PromptParams pp) { kv_append_row<KV_T>(p); prompt_q_row<HD>(pp); }
 
-constexpr int PA_LDK = 136;    // halfs per staged K row (128 + pad: rows stay 16-byte aligned for the 8-half operand reads)
 constexpr int PA_LDV = 36;     // halfs per staged V^T row (32 cached rows + pad)
 
-template <typename KV_T>
+template <typename KV_T, int HD>
 __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
 {
   constexpr bool I8P = sizeof(KV_T) == 1;         // int8 rows are dequantised (code * row scale) while they are staged
   constexpr bool F32 = sizeof(KV_T) != 2;         // ... and, like a float cache, split hi + lo
   constexpr int NP = F32 ? 2 : 1;                 // planes of K and V
+  constexpr int PA_LDK = HD + 8;                  // halfs per staged K row (rows stay 16-byte aligned for the 8-half operand reads)
+  constexpr int E = HD / 8;                       // elements of a row that a thread stages
   __shared__ __align__(16) _Float16 sK[NP][32 * PA_LDK];
-  __shared__ __align__(16) _Float16 sV[NP][128 * PA_LDV];
+  __shared__ __align__(16) _Float16 sV[NP][HD * PA_LDV];
   const int G = p.q_heads / p.kv_heads, quads = (G + 3) >> 2;
   const int g = blockIdx.y / quads, h0 = (blockIdx.y % quads) * 4;
   const int t0 = blockIdx.x * 32;
@@ -1402,48 +1405,53 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
     const int a = jt_first + ks * per;
     jt_last = min(jt_last, a + per - 1); jt_first = a;
   }
-  const KV_T* kc = reinterpret_cast<const KV_T*>(p.kc) + (int64_t)g * p.max_ctx * 128;
-  const KV_T* vc = reinterpret_cast<const KV_T*>(p.vc) + (int64_t)g * p.max_ctx * 128;
+  const KV_T* kc = reinterpret_cast<const KV_T*>(p.kc) + (int64_t)g * p.max_ctx * HD;
+  const KV_T* vc = reinterpret_cast<const KV_T*>(p.vc) + (int64_t)g * p.max_ctx * HD;
 
   // this lane's q fragments: token n, dims 16 s + 8 kg .. + 7 of the wave's head
-  ph8_t qh[8], ql[8];
+  ph8_t qh[HD / 16], ql[HD / 16];
   {
-    const int64_t qo = (int64_t)min(tok, p.n_tok - 1) * (p.q_heads * 128) + head * 128 + 8 * kg;
+    const int64_t qo = (int64_t)min(tok, p.n_tok - 1) * (p.q_heads * HD) + head * HD + 8 * kg;
 #pragma unroll
-    for (int s = 0; s < 8; s++) {
+    for (int s = 0; s < HD / 16; s++) {
       qh[s] = *reinterpret_cast<const ph8_t*>(p.qhi + qo + 16 * s);
       ql[s] = *reinterpret_cast<const ph8_t*>(p.qlo + qo + 16 * s);
     }
   }
-  pf16_t O[4];
+  pf16_t O[HD / 32];
 #pragma unroll
-  for (int dt = 0; dt < 4; dt++)
+  for (int dt = 0; dt < HD / 32; dt++)
 #pragma unroll
     for (int v = 0; v < 16; v++) O[dt][v] = 0.0f;
   float m_run = -1e30f, l_run = 0.0f;
 
-  const int srow = tid >> 3, sdim = (tid & 7) * 16;         // staging: 16 consecutive elements of one cached row
+  const int srow = tid >> 3, sdim = (tid & 7) * E;          // staging: E consecutive elements of one cached row
   // The rows of the NEXT tile are requested before the products of the current one and converted into LDS after them: the
   // memory round trip runs behind the matrix-core work instead of in front of it.  Requests are unconditional (rows past the
   // live range are clamped and masked below).
-  struct RawTile { uint4 k[sizeof(KV_T) == 4 ? 4 : 2], v[sizeof(KV_T) == 4 ? 4 : 2]; float ks, vs; };   // (int8: one uint4 each is used)
+  struct RawTile { uint4 k[sizeof(KV_T) == 4 ? E / 4 : 2], v[sizeof(KV_T) == 4 ? E / 4 : 2]; float ks, vs; };   // (int8: one uint4 each is used)
   auto fetch = [&](int jt, RawTile& r) {
     const int j = min(jt * 32 + srow, p.max_ctx - 1);
     if (I8P) {
-      r.k[0] = *reinterpret_cast<const uint4*>(reinterpret_cast<const int8_t*>(kc) + (int64_t)j * 128 + sdim);
-      r.v[0] = *reinterpret_cast<const uint4*>(reinterpret_cast<const int8_t*>(vc) + (int64_t)j * 128 + sdim);
+      if constexpr (E == 16) {
+        r.k[0] = *reinterpret_cast<const uint4*>(reinterpret_cast<const int8_t*>(kc) + (int64_t)j * HD + sdim);
+        r.v[0] = *reinterpret_cast<const uint4*>(reinterpret_cast<const int8_t*>(vc) + (int64_t)j * HD + sdim);
+      } else {
+        const uint2 a = *reinterpret_cast<const uint2*>(reinterpret_cast<const int8_t*>(kc) + (int64_t)j * HD + sdim), b = *reinterpret_cast<const uint2*>(reinterpret_cast<const int8_t*>(vc) + (int64_t)j * HD + sdim);
+        r.k[0] = make_uint4(a.x, a.y, 0u, 0u); r.v[0] = make_uint4(b.x, b.y, 0u, 0u);
+      }
       r.ks = p.ksc[(int64_t)g * p.max_ctx + j]; r.vs = p.vsc[(int64_t)g * p.max_ctx + j];
     } else if (sizeof(KV_T) == 4) {
 #pragma unroll
-      for (int c4 = 0; c4 < 4; c4++) {
-        r.k[c4] = *reinterpret_cast<const uint4*>(reinterpret_cast<const float*>(kc) + (int64_t)j * 128 + sdim + 4 * c4);
-        r.v[c4] = *reinterpret_cast<const uint4*>(reinterpret_cast<const float*>(vc) + (int64_t)j * 128 + sdim + 4 * c4);
+      for (int c4 = 0; c4 < E / 4; c4++) {
+        r.k[c4] = *reinterpret_cast<const uint4*>(reinterpret_cast<const float*>(kc) + (int64_t)j * HD + sdim + 4 * c4);
+        r.v[c4] = *reinterpret_cast<const uint4*>(reinterpret_cast<const float*>(vc) + (int64_t)j * HD + sdim + 4 * c4);
       }
     } else {
 #pragma unroll
-      for (int c8 = 0; c8 < 2; c8++) {
-        r.k[c8] = *reinterpret_cast<const uint4*>(reinterpret_cast<const __half*>(kc) + (int64_t)j * 128 + sdim + 8 * c8);
-        r.v[c8] = *reinterpret_cast<const uint4*>(reinterpret_cast<const __half*>(vc) + (int64_t)j * 128 + sdim + 8 * c8);
+      for (int c8 = 0; c8 < E / 8; c8++) {
+        r.k[c8] = *reinterpret_cast<const uint4*>(reinterpret_cast<const __half*>(kc) + (int64_t)j * HD + sdim + 8 * c8);
+        r.v[c8] = *reinterpret_cast<const uint4*>(reinterpret_cast<const __half*>(vc) + (int64_t)j * HD + sdim + 8 * c8);
       }
     }
   };
@@ -1452,13 +1460,13 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
   for (int jt = jt_first; jt <= jt_last; jt++) {
     __syncthreads();                                        // the previous tile has been consumed
     {
-      float kv[16], vv[16];
+      float kv[E], vv[E];
       if (I8P) {
         const uint4 a = raw.k[0], b = raw.v[0];
         const float ks = raw.ks, vs = raw.vs;
         const int aw[4] = {(int)a.x, (int)a.y, (int)a.z, (int)a.w}, bw[4] = {(int)b.x, (int)b.y, (int)b.z, (int)b.w};
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < E / 4; i++) {
           kv[4 * i] = (float)((aw[i] << 24) >> 24) * ks; kv[4 * i + 1] = (float)((aw[i] << 16) >> 24) * ks;
           kv[4 * i + 2] = (float)((aw[i] << 8) >> 24) * ks; kv[4 * i + 3] = (float)(aw[i] >> 24) * ks;
           vv[4 * i] = (float)((bw[i] << 24) >> 24) * vs; vv[4 * i + 1] = (float)((bw[i] << 16) >> 24) * vs;
@@ -1466,7 +1474,7 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
         }
       } else if (sizeof(KV_T) == 4) {
 #pragma unroll
-        for (int c4 = 0; c4 < 4; c4++) {
+        for (int c4 = 0; c4 < E / 4; c4++) {
           const uint4 a = raw.k[c4], b = raw.v[c4];
           kv[4 * c4] = __builtin_bit_cast(float, a.x); kv[4 * c4 + 1] = __builtin_bit_cast(float, a.y); kv[4 * c4 + 2] = __builtin_bit_cast(float, a.z); kv[4 * c4 + 3] = __builtin_bit_cast(float, a.w);
           vv[4 * c4] = __builtin_bit_cast(float, b.x); vv[4 * c4 + 1] = __builtin_bit_cast(float, b.y); vv[4 * c4 + 2] = __builtin_bit_cast(float, b.z); vv[4 * c4 + 3] = __builtin_bit_cast(float, b.w);
@@ -1474,7 +1482,7 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
       }
       if constexpr (sizeof(KV_T) == 2) {                  // a half cache goes in as it is
 #pragma unroll
-        for (int c8 = 0; c8 < 2; c8++) {
+        for (int c8 = 0; c8 < E / 8; c8++) {
           const uint4 a = raw.k[c8], b = raw.v[c8];
           *reinterpret_cast<uint2*>(&sK[0][srow * PA_LDK + sdim + 8 * c8]) = make_uint2(a.x, a.y);
           *reinterpret_cast<uint2*>(&sK[0][srow * PA_LDK + sdim + 8 * c8 + 4]) = make_uint2(a.z, a.w);
@@ -1487,7 +1495,7 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
         }
       } else {
 #pragma unroll
-      for (int i4 = 0; i4 < 4; i4++) {                    // K rows stay row-major: 8-byte stores
+      for (int i4 = 0; i4 < E / 4; i4++) {                    // K rows stay row-major: 8-byte stores
         ph4_t kh, kl;
 #pragma unroll
         for (int i = 0; i < 4; i++) { _Float16 a, b; split_f16(kv[4 * i4 + i], a, b); kh[i] = a; kl[i] = b; }
@@ -1495,7 +1503,7 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
         if (F32) *reinterpret_cast<ph4_t*>(&sK[NP - 1][srow * PA_LDK + sdim + 4 * i4]) = kl;
       }
 #pragma unroll
-      for (int i = 0; i < 16; i++) {                      // V goes in transposed
+      for (int i = 0; i < E; i++) {                       // V goes in transposed
         _Float16 vh, vl; split_f16(vv[i], vh, vl);
         sV[0][(sdim + i) * PA_LDV + srow] = vh;
         if (F32) sV[NP - 1][(sdim + i) * PA_LDV + srow] = vl;
@@ -1511,7 +1519,7 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
 #pragma unroll
     for (int v = 0; v < 16; v++) C[v] = 0.0f;
 #pragma unroll
-    for (int s = 0; s < 8; s++) {
+    for (int s = 0; s < HD / 16; s++) {
       const ph8_t a = *reinterpret_cast<const ph8_t*>(&sK[0][n * PA_LDK + 16 * s + 8 * kg]);
       C = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qh[s], C, 0, 0, 0);
       C = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, ql[s], C, 0, 0, 0);
@@ -1541,7 +1549,7 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
     l_run = l_run * corr + psum; m_run = m_new;
     if (__builtin_amdgcn_ballot_w64(corr != 1.0f)) {      // (after the first tiles a new maximum is rare: the whole wave skips the rescaling)
 #pragma unroll
-      for (int dt = 0; dt < 4; dt++)
+      for (int dt = 0; dt < HD / 32; dt++)
 #pragma unroll
         for (int v = 0; v < 16; v++) O[dt][v] *= corr;
     }
@@ -1555,7 +1563,7 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
 #pragma unroll
       for (int i = 0; i < 8; i++) { _Float16 hv, lv; split_f16(C[8 * s2 + i], hv, lv); ph[i] = hv; pl[i] = lv; }
 #pragma unroll
-      for (int dt = 0; dt < 4; dt++) {
+      for (int dt = 0; dt < HD / 32; dt++) {
         const ph4_t a0 = *reinterpret_cast<const ph4_t*>(&sV[0][(32 * dt + n) * PA_LDV + 16 * s2 + 4 * kg]);
         const ph4_t a1 = *reinterpret_cast<const ph4_t*>(&sV[0][(32 * dt + n) * PA_LDV + 16 * s2 + 8 + 4 * kg]);
         const ph8_t a = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
@@ -1572,21 +1580,21 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
   }
   if (!head_on || !tok_on) return;
   if (splits > 1) {        // this piece's unnormalised sums, maximum and normaliser; prompt_merge_kernel adds the pieces
-    float* pt = p.part + (((int64_t)tok * p.q_heads + head) * gridDim.z + ks) * 130;
+    float* pt = p.part + (((int64_t)tok * p.q_heads + head) * gridDim.z + ks) * (HD + 2);
 #pragma unroll
-    for (int dt = 0; dt < 4; dt++)
+    for (int dt = 0; dt < HD / 32; dt++)
 #pragma unroll
       for (int g4 = 0; g4 < 4; g4++) {
-        float* q4 = pt + 32 * dt + 8 * g4 + 4 * kg;       // (130-float records: 8-byte aligned only)
+        float* q4 = pt + 32 * dt + 8 * g4 + 4 * kg;       // (records of HD + 2 floats: 8-byte aligned only)
         q4[0] = O[dt][4 * g4]; q4[1] = O[dt][4 * g4 + 1]; q4[2] = O[dt][4 * g4 + 2]; q4[3] = O[dt][4 * g4 + 3];
       }
-    if (kg == 0) { pt[128] = m_run; pt[129] = l_run; }
+    if (kg == 0) { pt[HD] = m_run; pt[HD + 1] = l_run; }
     return;
   }
   const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
-  float* dst = p.out + (int64_t)tok * p.out_stride + head * 128;
+  float* dst = p.out + (int64_t)tok * p.out_stride + head * HD;
 #pragma unroll
-  for (int dt = 0; dt < 4; dt++)
+  for (int dt = 0; dt < HD / 32; dt++)
 #pragma unroll
     for (int g4 = 0; g4 < 4; g4++)
       *reinterpret_cast<float4*>(dst + 32 * dt + 8 * g4 + 4 * kg) =
@@ -1595,17 +1603,18 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
 
 // out[token][head] = sum of the K splits of a token tile, folded with a running maximum in split order (a tile walked by one
 // work-group was written by it and is left alone)
+template <int HD>
 __global__ __launch_bounds__(512) void prompt_merge_kernel(const PromptParams p, int n_ks)
 {
   const int tok = blockIdx.x, head = blockIdx.y * 4 + (threadIdx.x >> 7), d = threadIdx.x & 127;   // four heads per work-group
   int jt0, jt1, splits;
   prompt_k_range(p, (tok >> 5) << 5, n_ks, jt0, jt1, splits);
-  if (splits <= 1 || head >= p.q_heads) return;
-  const float* pt = p.part + (((int64_t)tok * p.q_heads + head) * n_ks) * 130;
+  if (splits <= 1 || head >= p.q_heads || d >= HD) return;
+  const float* pt = p.part + (((int64_t)tok * p.q_heads + head) * n_ks) * (HD + 2);
   float M = -1e30f, L = 0.0f, A = 0.0f;
   float ms[PA_KS_MAX], ls[PA_KS_MAX], as[PA_KS_MAX];                     // all requests first (a split past the count repeats the last one; not used)
 #pragma unroll
-  for (int s = 0; s < PA_KS_MAX; s++) { const int sc = min(s, splits - 1); ms[s] = pt[sc * 130 + 128]; ls[s] = pt[sc * 130 + 129]; as[s] = pt[sc * 130 + d]; }
+  for (int s = 0; s < PA_KS_MAX; s++) { const int sc = min(s, splits - 1); ms[s] = pt[sc * (HD + 2) + HD]; ls[s] = pt[sc * (HD + 2) + HD + 1]; as[s] = pt[sc * (HD + 2) + d]; }
 #pragma unroll
   for (int s = 0; s < PA_KS_MAX; s++) {
     if (s < splits && ls[s] > 0.0f) {
@@ -1613,14 +1622,17 @@ __global__ __launch_bounds__(512) void prompt_merge_kernel(const PromptParams p,
       A = A * c0 + as[s] * c1; L = L * c0 + ls[s] * c1; M = mn;
     }
   }
-  p.out[(int64_t)tok * p.out_stride + head * 128 + d] = L > 0.0f ? A * (1.0f / L) : 0.0f;
+  p.out[(int64_t)tok * p.out_stride + head * HD + d] = L > 0.0f ? A * (1.0f / L) : 0.0f;
 }
 
 // Whether n prompt rows of this cache go to the matrix-core prompt kernel (it needs no per-slice partial results).
+// Heads of 128: from 8 rows on.  Heads of 64: from 256 on, where the per-row kernel's reads of the cache outgrow its launch (9 / 3
+// heads, six layers, float cache: 128 tokens 383 us per row, 395 here; 300: 772, 452; 1500: 3799, 1727; 8 / 8 heads, three layers,
+// 200 tokens: 261, 272).
 bool attn_prompt_is_flash(const cai_kv_s* kv, int n)
 {
   static const int flash_on = []() { const char* e = getenv("CAIHIP_PROMPT_FLASH"); return e ? atoi(e) : 1; }();
-  return flash_on && kv->head_dim == 128 && kv->evict_cap == 0 && n >= 8;
+  return flash_on && kv->evict_cap == 0 && ((kv->head_dim == 128 && n >= 8) || (kv->head_dim == 64 && n >= 256));
 }
 
 int launch_attn_step(cai_kv_s* kv, int layer, float* qkv, int64_t qkv_stride, int n_seq, int q_heads, int window,
@@ -1664,7 +1676,7 @@ int launch_attn_step(cai_kv_s* kv, int layer, float* qkv, int64_t qkv_stride, in
     if (!prompt_rows && !grouped) { p.qn_gain = qn_gain; p.kn_gain = kn_gain; p.qk_eps = qk_eps; }
     else if ((rc = launch_rmsnorm_pair(qkv, qn_gain, qw, kn_gain, kw, n_seq, qk_eps, qkv_stride))) return rc;
   }
-  // prompts over a 128-wide cache: matrix-core kernel, 32 tokens x 4 heads per work-group
+  // prompts over a 128- or 64-wide cache: matrix-core kernel, 32 tokens x 4 heads per work-group
   const bool flash = prompt_rows == 1 && attn_prompt_is_flash(kv, n_seq);
   const bool rows_fused = flash && kv->dtype != CAI_KV_I8;     // the append and the q planes share a launch (below)
   if (prompt_rows && kv->dtype == CAI_KV_I8) {
@@ -1676,7 +1688,7 @@ int launch_attn_step(cai_kv_s* kv, int layer, float* qkv, int64_t qkv_stride, in
     else hipLaunchKernelGGL(kv_append_rows_kernel<float>, dim3(n_seq), dim3(256), 0, c.stream, p);
   }
   if (flash) {
-    const size_t need = (size_t)n_seq * q_heads * 128;
+    const size_t need = (size_t)n_seq * q_heads * p.hd;
     if (need > kv->pq_cap) {
       CAI_HIP(hipStreamSynchronize(c.stream));
       if (kv->pq_hi) (void)hipFree(kv->pq_hi);
@@ -1703,7 +1715,7 @@ int launch_attn_step(cai_kv_s* kv, int layer, float* qkv, int64_t qkv_stride, in
     // 50.8 + 11.6 with three; on 512-token chunks of the 32B shape (256 work-groups) splitting loses (365 -> 373 + 16 us).
     const int n_ks = std::max(1, std::min(PA_KS_MAX, c.n_cu / wgs));
     if (n_ks > 1) {
-      const size_t pneed = (size_t)n_seq * q_heads * n_ks * 130;
+      const size_t pneed = (size_t)n_seq * q_heads * n_ks * (p.hd + 2);
       if (pneed > kv->pq_part_cap) {
         CAI_HIP(hipStreamSynchronize(c.stream));
         if (kv->pq_part) (void)hipFree(kv->pq_part);
@@ -1713,14 +1725,18 @@ int launch_attn_step(cai_kv_s* kv, int layer, float* qkv, int64_t qkv_stride, in
       }
     }
     pp.part = kv->pq_part;
-    if (!rows_fused) hipLaunchKernelGGL(prompt_q_kernel, dim3(n_seq), dim3(256), 0, c.stream, pp);
-    else if (kv->dtype == CAI_KV_F16) hipLaunchKernelGGL(prompt_rows_kernel<__half>, dim3(n_seq), dim3(256), 0, c.stream, p, pp);
-    else hipLaunchKernelGGL(prompt_rows_kernel<float>, dim3(n_seq), dim3(256), 0, c.stream, p, pp);
     const dim3 grid((n_seq + 31) / 32, kv->kv_heads * ((G + 3) / 4), n_ks);
-    if (kv->dtype == CAI_KV_F16) hipLaunchKernelGGL(attn_prompt_kernel<__half>, grid, dim3(256), 0, c.stream, pp);
-    else if (kv->dtype == CAI_KV_I8) hipLaunchKernelGGL(attn_prompt_kernel<int8_t>, grid, dim3(256), 0, c.stream, pp);
-    else hipLaunchKernelGGL(attn_prompt_kernel<float>, grid, dim3(256), 0, c.stream, pp);
-    if (n_ks > 1) hipLaunchKernelGGL(prompt_merge_kernel, dim3(n_seq, (q_heads + 3) / 4), dim3(512), 0, c.stream, pp, n_ks);
+    auto go = [&](auto hd_) {
+      constexpr int HD = hd_;
+      if (!rows_fused) hipLaunchKernelGGL(prompt_q_kernel<HD>, dim3(n_seq), dim3(256), 0, c.stream, pp);
+      else if (kv->dtype == CAI_KV_F16) hipLaunchKernelGGL((prompt_rows_kernel<__half, HD>), dim3(n_seq), dim3(256), 0, c.stream, p, pp);
+      else hipLaunchKernelGGL((prompt_rows_kernel<float, HD>), dim3(n_seq), dim3(256), 0, c.stream, p, pp);
+      if (kv->dtype == CAI_KV_F16) hipLaunchKernelGGL((attn_prompt_kernel<__half, HD>), grid, dim3(256), 0, c.stream, pp);
+      else if (kv->dtype == CAI_KV_I8) hipLaunchKernelGGL((attn_prompt_kernel<int8_t, HD>), grid, dim3(256), 0, c.stream, pp);
+      else hipLaunchKernelGGL((attn_prompt_kernel<float, HD>), grid, dim3(256), 0, c.stream, pp);
+      if (n_ks > 1) hipLaunchKernelGGL(prompt_merge_kernel<HD>, dim3(n_seq, (q_heads + 3) / 4), dim3(512), 0, c.stream, pp, n_ks);
+    };
+    if (p.hd == 64) go(std::integral_constant<int, 64>()); else go(std::integral_constant<int, 128>());
     return CAI_OK;
   }
   // one work-group per (slice, KV head) serving the whole group of query heads, or one per (slice, query head)

@@ -393,6 +393,29 @@ def test_prompt_attention_on_matrix_cores_equals_steps(kv, window):
     assert rel_err(lg, last[0]) < tol
 
 
+@pytest.mark.parametrize("kv,window,hq,hkv", [("f32", 0, 6, 2), ("f16", 90, 5, 1), ("i8", 0, 4, 4), ("f32", 300, 8, 1)])
+def test_prompt_attention_of_64_wide_heads_on_matrix_cores(kv, window, hq, hkv):
+    """256 rows and more of a 64-wide cache: one row past a token tile, a continuation from position 256, groups of 1, 3, 5 and 8 heads;
+    equal to the same prompt in pieces of 100 rows, which go to the per-row kernels"""
+    from helpers.device import dev, rel_err
+    cai = dev()
+    cfg = dict(n_layers=2, d_model=256, n_q_heads=hq, n_kv_heads=hkv, head_dim=64, ffn=512, vocab=300, max_ctx=640, eps=1e-5, rope_theta=1e4, window=window)
+    spec = synthetic_spec(cfg, O.Q8_0, head_qtype=O.Q8_0, seed=hq, std=0.05, qkv_bias=True)
+    dec = cai.Decoder(spec, max_batch=2, kv_dtype={"f32": cai.KV_F32, "f16": cai.KV_F16, "i8": cai.KV_I8}[kv])
+    toks = np.random.default_rng(hkv).integers(0, 300, 513).astype(np.int32)
+    tol = 5e-3 if kv == "i8" else 2e-4       # (int8: now and then a code lands one step apart)
+    for n, cuts in ((257, [257]), (513, [256, 257])):
+        dec.reset(0); dec.reset(1)
+        for seq, pieces in ((0, [100] * (n // 100) + [n % 100]), (1, cuts)):
+            p = 0
+            for m in pieces:
+                _, lg = dec.prefill(toks[p:p + m], p, seq=seq)
+                p += m
+            if seq == 0: want = lg
+        assert rel_err(lg, want) < tol, (n, rel_err(lg, want))
+    dec.close()
+
+
 @pytest.mark.parametrize("name", ["qwen7b_like_q4k", "olmoe_like_q8"])
 def test_per_class_timing_leaves_the_session_as_it_found_it(name):
     """cai_decoder_profile (a measurement aid without a counterpart in the reference) replays whole steps and steps without one
