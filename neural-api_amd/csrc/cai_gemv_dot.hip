@@ -57,13 +57,15 @@ __device__ __forceinline__ uint32_t spread_fifth(uint32_t qh, int w) { return __
 __device__ __forceinline__ int xq_slot(int u, int t) { return (u >> 4) * 256 + t * 16 + (u & 15); }
 
 constexpr float XQ_MAX = 4194303.0f;          // 2^22 - 1
-// The stored streams take the whole range of three balanced digits (127 * (1 + 256 + 65536), less the rounding of the quotient): their
-// 16-weight sums fit 32 bits all the same (16 * 16 * 8355711), and the rounding of the activations is half as large, 2^-24 of the
-// 32-block maximum: 1.4e-7 off 64 bits over widths of 2048 to 5120, the float walk (gemv_raw) 1.1e-7 to 1.7e-7.
-// 18944 x 3584 against that walk, which spends 12 to 25 vector instructions on a weight (here 2 to 2.5): Q3_K 39.2 -> 12.0 us,
-// Q2_K 18.6 -> 10.8, Q4_1 17.8 -> 9.3, Q5_0 27.0 -> 10.9, Q5_1 22.1 -> 10.9; 2048 x 2048 5.0..7.9 -> 4.3.
-constexpr float XQ_MAX_STREAM = 8355710.0f;
-constexpr int NL = 3;                         // balanced base-256 digits per activation
+// The stored streams take four digits and a power of two as the scale of 32 neighbours: x * 2^k, k chosen so that the largest lies in [2^29, 2^30),
+// is a whole number for everything within 2^-6 of the largest and off by 2^-31 of it at most below, so an activation is held as well as in
+// 32 bits over any range, denormals and the largest finite values included.  Three digits of the largest / 8355710 (2^-24 of the largest a
+// value) were 1.3..1.5e-7 off 64 bits at widths of 512 to 3584, 2.0e-7 where the activations spread widely; the float walk (gemv_raw)
+// is 0.9..1.5e-7 (3e-7 at 18944), this form 0.7..0.9e-7 (1e-7).
+// 18944 x 3584 against that walk, which spends 12 to 25 vector instructions on a weight (here 2.5 to 3): Q3_K 41.1 -> 13.6 us, Q2_K 18.4 -> 11.8,
+// Q4_1 18.0 -> 10.9, Q5_0 28.1 -> 12.7, Q5_1 24.1 -> 12.8; 3584 x 18944 Q3_K 62 -> 16; 2048 x 2048 Q3_K 8.2 -> 5.2, Q4_1 5.8 -> 5.3
+// (three digits: 9 % less at the large sizes).
+template <int QT> constexpr int dot_digits() { return dot_stream<QT>() ? 4 : 3; }   // balanced base-256 digits per activation
 
 __device__ __forceinline__ float quad_max(float v)
 {
@@ -97,17 +99,20 @@ __device__ __forceinline__ float group_sum(float v)
 }
 
 // four rounded activations -> one dword per digit
+template <int NL>
 __device__ __forceinline__ void pack_digits(const int (&q)[4], int (&d)[NL])
 {
+  constexpr uint32_t mid = NL == 4 ? 0x80808080u : 0x00808080u, top = NL == 4 ? 0x07030602u : 0x06020602u;
   uint32_t e[4];
 #pragma unroll
   for (int i = 0; i < 4; i++)   // integer value + 0x808080, then flip the digit sign bits: bytes are balanced digits
-    e[i] = ((uint32_t)q[i] + 0x00808080u) ^ 0x00808080u;
+    e[i] = ((uint32_t)q[i] + mid) ^ mid;
   const uint32_t p01 = __builtin_amdgcn_perm(e[1], e[0], 0x05010400u), p23 = __builtin_amdgcn_perm(e[3], e[2], 0x05010400u);
-  const uint32_t h01 = __builtin_amdgcn_perm(e[1], e[0], 0x06020602u), h23 = __builtin_amdgcn_perm(e[3], e[2], 0x06020602u);
+  const uint32_t h01 = __builtin_amdgcn_perm(e[1], e[0], top), h23 = __builtin_amdgcn_perm(e[3], e[2], top);
   d[0] = (int)__builtin_amdgcn_perm(p23, p01, 0x05040100u);
   d[1] = (int)__builtin_amdgcn_perm(p23, p01, 0x07060302u);
   d[2] = (int)__builtin_amdgcn_perm(h23, h01, 0x05040100u);
+  if constexpr (NL == 4) d[3] = (int)__builtin_amdgcn_perm(h23, h01, 0x07060302u);
 }
 
 }  // namespace
@@ -152,6 +157,7 @@ __device__ __forceinline__ void gemv_dot_body(const GemvParams& p, const DotHot 
   const unsigned long long tl0 = timeline_now();
   constexpr int RR = MODE == 1 ? 2 * R : R;
   constexpr int TS = 16 / PK;                 // super-blocks of a row held by one wave
+  constexpr int NL = dot_digits<QT>();
   static_assert(PK == 1 || PK == 2 || PK == 4 || PK == 8, "rows packed per wave");
   __shared__ float s_ss[16];
   constexpr int CH = 4;                       // row groups between two meetings of the slice waves
@@ -267,6 +273,7 @@ __device__ __forceinline__ void gemv_dot_body(const GemvParams& p, const DotHot 
 
   WRegs buf[NS][RR];
 
+  float* const stream_scales = reinterpret_cast<float*>(xq4 + ((cols + 1023) >> 10) * 256);
   // ---- activation -> block-float integers, once per work-group, through LDS ----
   {
     float inv_rms = 1.0f;
@@ -353,24 +360,38 @@ __device__ __forceinline__ void gemv_dot_body(const GemvParams& p, const DotHot 
       const bool ok = m > 0.0f && m < 3.0e38f;           // an all-zero block contributes 0
       // 0 for finite values, NaN when the eight hold an inf or a NaN: carried into the scale so the outputs show it
       const float poison = (((v0.x + v0.y) + (v0.z + v0.w)) + ((v1.x + v1.y) + (v1.z + v1.w))) * 0.0f;
-      constexpr float QM = dot_stream<QT>() ? XQ_MAX_STREAM : XQ_MAX;
-      const float inv = ok ? QM / m : 0.0f, s = ok ? m * (1.0f / QM) : 0.0f;
       const float va[4] = {v0.x, v0.y, v0.z, v0.w}, vb[4] = {v1.x, v1.y, v1.z, v1.w};
       int qa[4], qb[4], isum = 0;
+      float s;
+      if constexpr (dot_stream<QT>()) {
+        const int k = min(30 - __builtin_amdgcn_frexp_expf(m), 149);   // (2^-149 is the smallest step of a float)
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        if constexpr (dot_stream<QT>()) { qa[i] = (int)rintf(va[i] * inv); qb[i] = (int)rintf(vb[i] * inv); }
-        else {   // up to 2^22 the addition of 1.5 * 2^23 rounds
+        for (int i = 0; i < 4; i++) { qa[i] = (int)rintf(ldexpf(va[i], k)); qb[i] = (int)rintf(ldexpf(vb[i], k)); }
+        s = ldexpf(1.0f, -k);
+        if (quad_poison(poison) != 0.0f) {       // an infinity: its sign times the scale infinity, beside which finite values vanish; a NaN is the scale
+          const float inf = __builtin_inff();
+          float nan = 0.0f;
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            qa[i] = (va[i] == inf) - (va[i] == -inf); qb[i] = (vb[i] == inf) - (vb[i] == -inf);
+            if (va[i] != va[i] || vb[i] != vb[i]) nan = __builtin_nanf("");
+          }
+          s = inf + quad_poison(nan);
+        }
+      } else {
+        const float inv = ok ? XQ_MAX / m : 0.0f;
+        s = ok ? m * (1.0f / XQ_MAX) : 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {            // up to 2^22 the addition of 1.5 * 2^23 rounds
           qa[i] = (int)(__builtin_bit_cast(uint32_t, fmaf(va[i], inv, 12582912.0f)) - 0x4B400000u);
           qb[i] = (int)(__builtin_bit_cast(uint32_t, fmaf(vb[i], inv, 12582912.0f)) - 0x4B400000u);
+          isum += qa[i] + qb[i];
         }
-        isum += qa[i] + qb[i];
       }
       int da[NL], db[NL];
       pack_digits(qa, da); pack_digits(qb, db);
-      isum = quad_sum(isum);
       // n = [unit][half:1][j:2]: the unit's record holds per digit 4 uint4 (2 per 32-block), then one uint4 of
-      // {scale A, scale B, s*sum A, s*sum B}
+      // {scale A, scale B, s*sum A, s*sum B}; four digits fill it, and the scales of all units lie behind the records
       const int u = n >> 3, hb = (n >> 2) & 1, j = n & 3;
       uint32_t* rec = reinterpret_cast<uint32_t*>(xq4);
 #pragma unroll
@@ -378,11 +399,16 @@ __device__ __forceinline__ void gemv_dot_body(const GemvParams& p, const DotHot 
         uint32_t* dst = rec + (size_t)xq_slot(u, L * 4 + hb * 2 + (j >> 1)) * 4 + (j & 1) * 2;
         dst[0] = (uint32_t)da[L]; dst[1] = (uint32_t)db[L];
       }
-      // the block's scale must be poisoned by any of its four threads
-      const float s_blk = s + quad_poison(poison);
-      if (j == 0) {
-        float* fr = reinterpret_cast<float*>(rec + (size_t)xq_slot(u, NL * 4) * 4);
-        fr[hb] = s_blk; fr[2 + hb] = s_blk * (float)isum;
+      if constexpr (dot_stream<QT>()) {
+        if (j == 0) stream_scales[2 * u + hb] = s;
+      } else {
+        isum = quad_sum(isum);
+        // the block's scale must be poisoned by any of its four threads
+        const float s_blk = s + quad_poison(poison);
+        if (j == 0) {
+          float* fr = reinterpret_cast<float*>(rec + (size_t)xq_slot(u, NL * 4) * 4);
+          fr[hb] = s_blk; fr[2 + hb] = s_blk * (float)isum;
+        }
       }
       }
      }
@@ -402,9 +428,12 @@ __device__ __forceinline__ void gemv_dot_body(const GemvParams& p, const DotHot 
         xq[L][4 * t] = (int)v.x; xq[L][4 * t + 1] = (int)v.y; xq[L][4 * t + 2] = (int)v.z; xq[L][4 * t + 3] = (int)v.w;
       }
     }
-    const uint4 v = xq4[xq_slot(u, NL * 4)];
-    sA = __builtin_bit_cast(float, v.x); sB = __builtin_bit_cast(float, v.y);
-    mA = __builtin_bit_cast(float, v.z); mB = __builtin_bit_cast(float, v.w);
+    if constexpr (dot_stream<QT>()) { sA = stream_scales[2 * u]; sB = stream_scales[2 * u + 1]; }
+    else {
+      const uint4 v = xq4[xq_slot(u, NL * 4)];
+      sA = __builtin_bit_cast(float, v.x); sB = __builtin_bit_cast(float, v.y);
+      mA = __builtin_bit_cast(float, v.z); mB = __builtin_bit_cast(float, v.w);
+    }
   } else {
 #pragma unroll
     for (int L = 0; L < NL; L++)
@@ -412,20 +441,21 @@ __device__ __forceinline__ void gemv_dot_body(const GemvParams& p, const DotHot 
       for (int t = 0; t < 16; t++) xq[L][t] = 0;
   }
 
-  float s16[4] = {0.0f, 0.0f, 0.0f, 0.0f};   // the lane's integer activations summed per 16 (first / second 32: groups 0, 1 / 2, 3)
-  int i16[4] = {0, 0, 0, 0};
+  // the lane's integer activations summed per 16 (first / second 32: groups 0, 1 / 2, 3); four digits as two sums, of the lower and the upper two
+  float s16[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  int i16[4] = {0, 0, 0, 0}, j16[4] = {0, 0, 0, 0};
   if constexpr (QT == CAI_Q6_K || dot_stream<QT>()) {
 #pragma unroll
     for (int gq = 0; gq < 4; gq++) {
-      int tot = 0;
+      int t[NL];
 #pragma unroll
       for (int L = 0; L < NL; L++) {
-        int t = 0;
+        t[L] = 0;
 #pragma unroll
-        for (int w = 0; w < 4; w++) t = __builtin_amdgcn_sdot4(0x01010101, xq[L][4 * gq + w], t, false);
-        tot += t << (8 * L);
+        for (int w = 0; w < 4; w++) t[L] = __builtin_amdgcn_sdot4(0x01010101, xq[L][4 * gq + w], t[L], false);
       }
-      s16[gq] = (float)tot; i16[gq] = tot;
+      if constexpr (NL == 4) { i16[gq] = t[0] + (t[1] << 8); j16[gq] = t[2] + (t[3] << 8); s16[gq] = fmaf(65536.0f, (float)j16[gq], (float)i16[gq]); }
+      else s16[gq] = (float)(t[0] + (t[1] << 8) + (t[2] << 16));
     }
   }
   timeline_stamp(p.timeline, 4);
@@ -493,7 +523,7 @@ __device__ __forceinline__ void gemv_dot_body(const GemvParams& p, const DotHot 
           acc[r] = dA * fmaf(sA, fa, -8.0f * mA) + dB * fmaf(sB, fb, -8.0f * mB);
           continue;
         } else if constexpr (dot_stream<QT>()) {
-          // exact sums of (code - OFFSET) * activation per 16, for Q2_K of (2 code - 3) * activation.  The offset of a type with minima is the
+          // sums of (code - OFFSET) * activation per 16, rounded once, for Q2_K of (2 code - 3) * activation.  The offset of a type with minima is the
           // middle of its codes: what the minimum then still adds is small, where a sum of bare codes and its minimum would cancel
           // (error of Q4_1 against 64 bits 2.6e-7 with bare codes, 1.4e-7 so).
           constexpr int OFFSET = QT == CAI_Q3_K ? 4 : QT == CAI_Q4_1 ? 8 : QT == CAI_Q2_K ? 3 : 16;
@@ -537,26 +567,30 @@ __device__ __forceinline__ void gemv_dot_body(const GemvParams& p, const DotHot 
 #pragma unroll
               for (int L = 0; L < NL; L++) dg[L] = __builtin_amdgcn_sdot4(c, xq[L][4 * gq + w], dg[L], false);
             }
-            // (unsigned: the sum of the bare codes may wrap, what is left after the offset fits)
-            const uint32_t tot = (uint32_t)dg[0] + ((uint32_t)dg[1] << 8) + ((uint32_t)dg[2] << 16);
-            f[gq] = (float)(int)((QT == CAI_Q2_K ? 2u * tot : tot) - (uint32_t)OFFSET * (uint32_t)i16[gq]);
+            // (two digits of sixteen codes, the offset taken off or not, fit 24 bits: both conversions are exact and the sum is rounded once)
+            constexpr int TWICE = QT == CAI_Q2_K ? 1 : 0;
+            const int lo = ((dg[0] + (dg[1] << 8)) << TWICE) - OFFSET * i16[gq], hi = ((dg[2] + (dg[3] << 8)) << TWICE) - OFFSET * j16[gq];
+            f[gq] = fmaf(65536.0f, (float)hi, (float)lo);
           }
           auto half_of = [](uint32_t v) { return __half2float(__ushort_as_half((unsigned short)(v & 0xffffu))); };
           if constexpr (QT == CAI_Q3_K) {
             const uint32_t s0 = __builtin_amdgcn_alignbit(cur[r].t.y, cur[r].t.x, 16), s1 = __builtin_amdgcn_alignbit(cur[r].t.z, cur[r].t.y, 16), s2 = __builtin_amdgcn_alignbit(cur[r].t.w, cur[r].t.z, 16);
             const uint32_t sc = ((((cc & 1) ? s1 : s0) >> (4 * (cc >> 1))) & 0x0f0f0f0fu) | (((s2 >> (2 * cc)) & 0x03030303u) << 4);
-            acc[r] = half_of(cur[r].t.w >> 16) * (sA * ((cvt_ub0(sc) - 32.0f) * f[0] + (cvt_ub1(sc) - 32.0f) * f[1]) + sB * ((cvt_ub2(sc) - 32.0f) * f[2] + (cvt_ub3(sc) - 32.0f) * f[3]));
+            const float d = half_of(cur[r].t.w >> 16);     // (before the scale of the activations: the sums of codes alone leave the range of floats)
+            acc[r] = sA * (d * ((cvt_ub0(sc) - 32.0f) * f[0] + (cvt_ub1(sc) - 32.0f) * f[1])) + sB * (d * ((cvt_ub2(sc) - 32.0f) * f[2] + (cvt_ub3(sc) - 32.0f) * f[3]));
           } else if constexpr (QT == CAI_Q2_K) {
             const uint32_t sc = cur[r].sc & 0x0f0f0f0fu, mn = (cur[r].sc >> 4) & 0x0f0f0f0fu;
             const float d = half_of(cur[r].dm), dmin = half_of(cur[r].dm >> 16), d15 = 1.5f * d;
-            acc[r] = (0.5f * d) * (sA * (cvt_ub0(sc) * f[0] + cvt_ub1(sc) * f[1]) + sB * (cvt_ub2(sc) * f[2] + cvt_ub3(sc) * f[3])) +
-                     sA * (fmaf(d15, cvt_ub0(sc), -dmin * cvt_ub0(mn)) * s16[0] + fmaf(d15, cvt_ub1(sc), -dmin * cvt_ub1(mn)) * s16[1]) +
-                     sB * (fmaf(d15, cvt_ub2(sc), -dmin * cvt_ub2(mn)) * s16[2] + fmaf(d15, cvt_ub3(sc), -dmin * cvt_ub3(mn)) * s16[3]);
+            acc[r] = sA * ((0.5f * d) * (cvt_ub0(sc) * f[0] + cvt_ub1(sc) * f[1]) +
+                           (fmaf(d15, cvt_ub0(sc), -dmin * cvt_ub0(mn)) * s16[0] + fmaf(d15, cvt_ub1(sc), -dmin * cvt_ub1(mn)) * s16[1])) +
+                     sB * ((0.5f * d) * (cvt_ub2(sc) * f[2] + cvt_ub3(sc) * f[3]) +
+                           (fmaf(d15, cvt_ub2(sc), -dmin * cvt_ub2(mn)) * s16[2] + fmaf(d15, cvt_ub3(sc), -dmin * cvt_ub3(mn)) * s16[3]));
           } else {
             const uint32_t ha = cur[r].a.x, hb = QT == CAI_Q4_1 ? cur[r].b.y : QT == CAI_Q5_0 ? cur[r].b.y >> 16 : cur[r].b.z;
             const float dA = half_of(ha), dB = half_of(hb);
-            acc[r] = dA * (sA * (f[0] + f[1])) + dB * (sB * (f[2] + f[3]));
-            if constexpr (QT != CAI_Q5_0) acc[r] += fmaf((float)OFFSET, dA, half_of(ha >> 16)) * mA + fmaf((float)OFFSET, dB, half_of(hb >> 16)) * mB;
+            float a = dA * (f[0] + f[1]), b = dB * (f[2] + f[3]);
+            if constexpr (QT != CAI_Q5_0) { a = fmaf(fmaf((float)OFFSET, dA, half_of(ha >> 16)), s16[0] + s16[1], a); b = fmaf(fmaf((float)OFFSET, dB, half_of(hb >> 16)), s16[2] + s16[3], b); }
+            acc[r] = sA * a + sB * b;
           }
           continue;
         } else if constexpr (QT == CAI_Q5_K) {
@@ -800,7 +834,8 @@ int launch_q4k_dot(GemvParams& p, const MultiGemv& m, int swiglu_half, hipStream
   int64_t total = 0;
   for (int i = 0; i < m.n; i++) total += swiglu_half ? swiglu_half : m.rows[i];
   const int waves_per_wg = nsw * gquads;
-  const size_t lds = (size_t)((cols + 1023) / 1024 * 1024) * 4;   // 16 uint4 per 64 activations
+  const bool stream = raw_block_type(m.w[0]->qtype) && m.w[0]->qtype != CAI_Q5_K;
+  const size_t lds = (size_t)((cols + 1023) / 1024 * 1024) * 4 + (stream ? cols / 32 * 4 : 0);   // 16 uint4 per 64 activations; scales of the four-digit form
   int wg_per_cu = W / waves_per_wg; if (wg_per_cu < 1) wg_per_cu = 1;
   { const int lds_fit = (int)((160 * 1024 - 4096) / (lds + 1024)); if (wg_per_cu > lds_fit) wg_per_cu = lds_fit < 1 ? 1 : lds_fit; }
   const int max_wgs = c.n_cu * wg_per_cu;
@@ -815,7 +850,6 @@ int launch_q4k_dot(GemvParams& p, const MultiGemv& m, int swiglu_half, hipStream
     if (nsw < 3 || 2 * turns2 <= turns1) R = 2;
     if (packed) R = 2;
   }
-  const bool stream = raw_block_type(m.w[0]->qtype) && m.w[0]->qtype != CAI_Q5_K;
   if (q6k || stream) R = 1;   // (two rows of Q6_K requests in flight twice over do not fit the registers; the stored streams spend longer on a row than it takes to arrive)
   int cum = 0;
   for (int i = 0; i < m.n; i++) {

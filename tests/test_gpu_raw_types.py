@@ -114,6 +114,53 @@ def test_decoder_of_a_stored_stream_type(qt):
     dec.close()
 
 
+@pytest.mark.parametrize("qt", RAW[1:])
+@pytest.mark.parametrize("cols", [512, 2048])
+def test_gemv_of_one_row_holds_activations_as_in_32_bits(qt, cols):
+    """Activations of even and of widely differing sizes.  With the activations held as well as in 32 bits what is left are the roundings of the
+    sums: about ten in a row, each even within 2^-24 of a partial sum, sqrt(10 / 3) * 2^-24 = 1.1e-7 of the result in the mean (2-norm); activations
+    rounded to 2^-24 of the largest of 32 neighbours are 1.35e-7 to 2.0e-7 away"""
+    from helpers.device import dev
+    cai = dev()
+    rng = np.random.default_rng(cols + qt)
+    raw = O.quantize(qt, (rng.standard_normal((1500, cols)) * 0.02).astype(np.float32))
+    w, full = cai.QWeight(qt, 1500, cols, raw), O.dequant(qt, raw, 1500 * cols).reshape(1500, cols).astype(np.float64)
+    for spread in (0.0, 1.5):
+        errs = []
+        for _ in range(6):
+            x = (rng.standard_normal((1, cols)) * np.exp(spread * rng.standard_normal((1, cols)))).astype(np.float32)
+            want = full @ x[0].astype(np.float64)
+            errs.append(np.linalg.norm(w.gemv(x)[0] - want) / np.linalg.norm(want))
+        assert np.mean(errs) < 1.15e-7, (spread, errs)
+    w.close()
+
+
+@pytest.mark.parametrize("qt", RAW[1:])
+def test_gemv_of_one_row_at_the_ends_of_the_number_range(qt):
+    """the largest finite values, values whose reciprocals overflow, denormals, and an infinity, which takes the sign of its weight"""
+    from helpers.device import dev
+    cai = dev()
+    rows, cols = 300, 768
+    rng = np.random.default_rng(qt)
+    raw = O.quantize(qt, (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32))
+    w, full = cai.QWeight(qt, rows, cols, raw), O.dequant(qt, raw, rows * cols).reshape(rows, cols)
+    normal = rng.standard_normal((1, cols)).astype(np.float32)
+    huge = normal.copy(); huge[0, 100] = np.float32(3.3e38)
+    for x in (huge, normal * np.float32(1e36), normal * np.float32(1e-33), normal * np.float32(1e-36)):
+        want = full.astype(np.float64) @ x[0].astype(np.float64)
+        got = w.gemv(x)[0].astype(np.float64)
+        assert np.abs(got - want).max() < TIGHT * np.abs(want).max()
+    x = normal * np.float32(1e-40)               # whole multiples of 2^-149: the result is within a few steps of that
+    assert np.abs(w.gemv(x)[0].astype(np.float64) - full.astype(np.float64) @ x[0].astype(np.float64)).max() < cols * 2.0 ** -149
+    clear = np.abs(full[:, 37]) > 1e-4
+    for inf in (np.inf, -np.inf):
+        x = normal.copy(); x[0, 37] = inf
+        np.testing.assert_array_equal(w.gemv(x)[0][clear], np.sign(full[clear, 37]) * inf)
+        x[0, 38] = np.nan
+        assert np.isnan(w.gemv(x)).all()
+    w.close()
+
+
 def test_width_that_splits_a_block_is_refused():
     from helpers.device import dev
     cai = dev()
