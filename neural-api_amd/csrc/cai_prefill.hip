@@ -22,11 +22,24 @@ typedef float float16_t __attribute__((ext_vector_type(16)));
 
 // ------------------------------------------------------------------------------------------
 // Activation pre-pass (one work-group per token): optional RMSNorm (neural/neural.cl:1047-1085), then
-//   s = 2^e with max|x|*s in [2^13, 2^14),  hi = f16(x*s),  lo = f16(x*s - hi),
+//   s = 2^e with max|x|*s in [2^13, 2^14) over the finite values (the largest floats and denormals too),  hi = f16(x*s),  lo = f16(x*s - hi),
 //   sxhi[b] + sxlo[b] = (sum of x over 32-block b) * s / 32 as two halfs (the block sums go to the matrix cores too).
 // SWIGLU: the row holds up | gate (K values each) and the value is up * silu(gate) - the feed-forward's middle step folded into
 // the pre-pass of the down projection (no norm in that case).
+// An infinity is hi = infinity and lo = 0, so that a product shows it with the sign of its weight; a NaN stays one.
 // ------------------------------------------------------------------------------------------
+__device__ __forceinline__ float finite_abs(float v) { const float a = fabsf(v); return a < __builtin_inff() ? a : 0.0f; }
+__device__ __forceinline__ int plane_exponent(float a)      // a = m*2^ex, m in [0.5,1) -> a*2^e in [2^13, 2^14)
+{
+  int e = 0;
+  if (a > 0.0f) { int ex; frexpf(a, &ex); e = 14 - ex; }
+  return min(e, 126);                                       // (2^-126 is the smallest normal reciprocal: 2^-149 is then 2^-23, above the steps of a half)
+}
+__device__ __forceinline__ void split_plane(float x, _Float16& hi, _Float16& lo)
+{
+  split_f16(x, hi, lo);
+  if (fabsf(x) == __builtin_inff()) lo = (_Float16)0.0f;
+}
 template <bool SWIGLU, int NT>     // NT threads per token
 __global__ __launch_bounds__(NT) void xprep_kernel(const float* x, int64_t x_stride, const float* gain, float eps, int K,
                                                     _Float16* hi, _Float16* lo, float* sinv, _Float16* sxhi, _Float16* sxlo)
@@ -53,7 +66,7 @@ __global__ __launch_bounds__(NT) void xprep_kernel(const float* x, int64_t x_str
   for_strided8(xr, second, threadIdx.x, K, NT, [&](float v, float g, int) {
     if (SWIGLU) v = silu_mul(v, g);
     else if (gain) v = g * (v * inv);
-    amax = fmaxf(amax, fabsf(v));
+    amax = fmaxf(amax, finite_abs(v));
   });
   for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
   if (lane == 0) red[wave] = amax;
@@ -62,9 +75,7 @@ __global__ __launch_bounds__(NT) void xprep_kernel(const float* x, int64_t x_str
     float a = 0.0f;
 #pragma unroll
     for (int w4 = 0; w4 < NT / 64; w4++) a = fmaxf(a, red[w4]);
-    int e = 0;
-    if (a > 0.0f && a < 3.0e38f) { int ex; frexpf(a, &ex); e = 14 - ex; }   // a = m*2^ex, m in [0.5,1) -> a*2^e in [2^13, 2^14)
-    if (e > 60) e = 60; if (e < -60) e = -60;
+    const int e = plane_exponent(a);
     s_scale = ldexpf(1.0f, e);
     sinv[t] = ldexpf(1.0f, -e);
   }
@@ -75,13 +86,13 @@ __global__ __launch_bounds__(NT) void xprep_kernel(const float* x, int64_t x_str
     if (SWIGLU) v = silu_mul(v, g);
     else if (gain) v = g * (v * inv);
     const float vs = v * s;
-    _Float16 h, l; split_f16(vs, h, l);
+    _Float16 h, l; split_plane(vs, h, l);
     hi[(int64_t)t * K + i] = h; lo[(int64_t)t * K + i] = l;
     float sum = v;
     for (int off = 16; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
     if ((i & 31) == 0) {   // the block sum in the scaled domain of hi/lo, divided by 32 so that it stays inside the half range
       const float ss = sum * s * 0.03125f;
-      _Float16 sh, sl; split_f16(ss, sh, sl);
+      _Float16 sh, sl; split_plane(ss, sh, sl);
       sxhi[(int64_t)t * (K >> 5) + (i >> 5)] = sh; sxlo[(int64_t)t * (K >> 5) + (i >> 5)] = sl;
     }
   });
@@ -147,16 +158,14 @@ __global__ __launch_bounds__(NT) void xprep_regs_kernel(const float* x, int64_t 
 #pragma unroll
   for (int e = 0; e < V; e++)
 #pragma unroll
-    for (int i = 0; i < 4; i++) amax = fmaxf(amax, fabsf(v[e][i]));
+    for (int i = 0; i < 4; i++) amax = fmaxf(amax, finite_abs(v[e][i]));
   amax = wave_abs_max(amax);
   if (lane == 63) red_m[wave] = amax;
   __syncthreads();
   float a = 0.0f;
 #pragma unroll
   for (int w4 = 0; w4 < NT / 64; w4++) a = fmaxf(a, red_m[w4]);
-  int ex2 = 0;
-  if (a > 0.0f && a < 3.0e38f) { int ex; frexpf(a, &ex); ex2 = 14 - ex; }
-  if (ex2 > 60) ex2 = 60; if (ex2 < -60) ex2 = -60;
+  const int ex2 = plane_exponent(a);
   const float s = ldexpf(1.0f, ex2);
   if (threadIdx.x == 0) sinv[t] = ldexpf(1.0f, -ex2);
 #pragma unroll
@@ -165,7 +174,7 @@ __global__ __launch_bounds__(NT) void xprep_regs_kernel(const float* x, int64_t 
     if (j >= K) break;                              // K is a multiple of 32: the eight threads of a block are inside or outside together
     half4_p h, l;
 #pragma unroll
-    for (int i = 0; i < 4; i++) { _Float16 a16, b16; split_f16(v[e][i] * s, a16, b16); h[i] = a16; l[i] = b16; }
+    for (int i = 0; i < 4; i++) { _Float16 a16, b16; split_plane(v[e][i] * s, a16, b16); h[i] = a16; l[i] = b16; }
     *reinterpret_cast<half4_p*>(hi + (int64_t)t * K + j) = h;
     *reinterpret_cast<half4_p*>(lo + (int64_t)t * K + j) = l;
     float sum = (v[e][0] + v[e][1]) + (v[e][2] + v[e][3]);
@@ -173,7 +182,7 @@ __global__ __launch_bounds__(NT) void xprep_regs_kernel(const float* x, int64_t 
     for (int off = 4; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
     if ((j & 31) == 0) {
       const float ss = sum * s * 0.03125f;
-      _Float16 sh, sl; split_f16(ss, sh, sl);
+      _Float16 sh, sl; split_plane(ss, sh, sl);
       sxhi[(int64_t)t * (K >> 5) + (j >> 5)] = sh; sxlo[(int64_t)t * (K >> 5) + (j >> 5)] = sl;
     }
   }

@@ -469,6 +469,18 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
     const int t = first + 8 * (v >> 2) + 4 * kg + (v & 3), row = R0 + 32 * rt + n;
     if (t >= p.n_tok || row >= rows) continue;
     const int64_t o = (int64_t)t * p.y_stride + yo + row;
+    if constexpr (MIN)
+      if (!(fabsf(y) < __builtin_inff())) {         // an infinity among the activations: its two parts may differ in sign, the weight's own counts
+        float sum = 0.0f; bool any = false;
+        for (int k = 0; k < K; k++) {
+          const float x = (float)p.xhi[(int64_t)t * K + k] + (float)p.xlo[(int64_t)t * K + k];
+          if (fabsf(x) < __builtin_inff()) continue;
+          const int64_t at = (int64_t)row * K + k;
+          const float d = (float)__builtin_bit_cast(_Float16, reinterpret_cast<const uint16_t*>(dbase)[at >> 5]);
+          sum += fmaf(d, (float)reinterpret_cast<const int8_t*>(qbase)[at], p.m16[at >> 4]) * x; any = true;
+        }
+        if (any) y = sum;
+      }
     y *= p.sinv[t];
     if (bias) y += bias[row];
     if (p.residual) y += p.residual[o];

@@ -418,6 +418,34 @@ def test_prompt_products_on_block_tiles(qt, rows, cols, T):
     w.close()
 
 
+@pytest.mark.parametrize("qt", [O.Q8_0, O.Q4_0, O.Q2_K, O.Q3_K, O.Q4_1, O.Q5_0, O.Q5_1])
+@pytest.mark.parametrize("T", [9, 70])
+def test_prompt_rows_at_the_ends_of_the_number_range(qt, T):
+    """the largest finite values, very small ones, denormals, an infinity (which takes the sign of its weight) and a NaN, each in a token of its own"""
+    from helpers.device import dev
+    cai = dev()
+    rows, cols = 300, 768
+    raw, rng = make(qt, rows, cols, qt)
+    w, full = cai.QWeight(qt, rows, cols, raw), O.dequant(qt, raw, rows * cols).reshape(rows, cols)
+    x = rng.standard_normal((T, cols)).astype(np.float32)
+    x[0, 100] = 3.3e38
+    for t, scale in ((1, 1e36), (2, 1e-20), (3, 1e-33), (4, 1e-36), (5, 1e-40)):
+        x[t] *= np.float32(scale)
+    x[6, 37], x[7, 37], x[8, 37] = np.inf, -np.inf, np.nan
+    got = w.gemm(x)
+    for t in (0, 1, 2, 3, 4, 5, T - 1):
+        if t == 8:
+            continue
+        want = full.astype(np.float64) @ x[t].astype(np.float64)
+        slack = cols * 2.0 ** -149 if t == 5 else TIGHT * np.abs(want).max()        # (denormals: whole multiples of 2^-149)
+        assert np.abs(got[t].astype(np.float64) - want).max() <= slack, t
+    clear = np.abs(full[:, 37]) > 1e-4
+    np.testing.assert_array_equal(got[6, clear], np.sign(full[clear, 37]) * np.inf)
+    np.testing.assert_array_equal(got[7, clear], np.sign(full[clear, 37]) * -np.inf)
+    assert np.isnan(got[8]).all()
+    w.close()
+
+
 @pytest.mark.parametrize("qt", [O.Q4_K, O.Q5_K])
 def test_prompt_of_a_decoder_on_wide_tiles(qt):
     """q | k | v in one launch of three row groups, gate | up with SwiGLU in the epilogue and behind the slices, residual on a cut product:
