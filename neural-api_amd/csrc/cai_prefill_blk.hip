@@ -50,6 +50,7 @@ struct BlkGemmParams {
   const uint8_t* q2[2]; const uint8_t* d2[2]; const float* bias2[2]; int rows2[2]; int y_off2[2];
   // types with minima: a weight is d * code + m16 of its sixteen; s16 = sums of sixteen activations [x row][cols / 16] in the planes' scale
   const float* m16; const float* s16;
+  float post;                           // the results' last factor (gemm_blk_cut)
 };
 
 // eight codes (two dwords) -> eight exact halfs.  Q8_0: signed bytes; Q4_0: (nibble - 8), low or high nibbles of the bytes
@@ -300,7 +301,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // Places in LDS: 16-byte piece c of token row t (128 bytes a plane) at c ^ (t / 2 % 8), of Q8_0 weight row n (64 bytes) at c ^ (n / 4 % 4),
 // of Q4_0 row n (32 bytes) at c ^ (n / 8 % 2): the lanes of a read pass then meet different banks.
 // ------------------------------------------------------------------------------------------
-template <int QT, int RT, int NW, bool ODD, bool MIN = false>     // ODD: rows of an odd number of blocks (scales that are not aligned to 4 bytes, a last chunk of one block)
+// FINE (panels of the stored streams): the lo halves and the minima are summed apart from the large parts.  A matrix instruction that adds them to the
+// block's sum rounds it once more each (and cuts what lies below the largest of its products off downwards): 1.04e-7 off 64 bits for Q2_K and
+// 0.91e-7 for Q3_K at width 512, where the float walk of eight tokens is 0.96e-7 and 0.88e-7; apart 0.80e-7 both (3584: 1.28e-7 -> 0.95e-7, walk
+// 1.52e-7) for 3 to 5 % of the time.  Q8_0 and Q4_0 are as near as their walk without it (0.92e-7, 0.99e-7 at 512; 1.07e-7 both at 3584).
+template <int QT, int RT, int NW, bool ODD, bool FINE = false, bool MIN = false>     // ODD: rows of an odd number of blocks (scales that are not aligned to 4 bytes, a last chunk of one block)
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_blk_cut(const BlkGemmParams p)
 {
   extern __shared__ __align__(16) unsigned char bl_smem[];
@@ -372,11 +377,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
           copy_dword(dst + MB + 512 + 256 * (RT == 2 ? i : i >> 1), mof + (uint32_t)(4 * i), mb + (int64_t)c * 16 - (half && i >= 2 ? 8 : 0));
     }
   };
-  float16_b Y[RT], Z[RT];                  // sums of eight (RT = 2: sixteen) blocks, sums of those: see the end of the comment above
+  float16_b Y[RT], Z[RT], U[RT];           // sums of eight (RT = 2: sixteen) blocks, sums of those: see the comment above; FINE: the small parts
 #pragma unroll
   for (int rt = 0; rt < RT; rt++)
 #pragma unroll
-    for (int v = 0; v < 16; v++) Y[rt][v] = Z[rt][v] = 0.0f;
+    for (int v = 0; v < 16; v++) Y[rt][v] = Z[rt][v] = U[rt][v] = 0.0f;
   const float16_b zero16 = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
   const unsigned char* const mine = bl_smem + wave * 2 * SLOT;
   auto use = [&](int slot, bool half) {
@@ -412,11 +417,19 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
       for (int rt = 0; rt < RT; rt++) {
         const float dv = __half2float(__ushort_as_half((unsigned short)(b ? (dw[rt] >> 16) : (dw[rt] & 0xffffu))));
-        float16_b C = zero16;
+        float16_b C = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[0], W[rt][0], zero16, 0, 0, 0);
+        if constexpr (FINE) {
+          float16_b D = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[1], W[rt][0], zero16, 0, 0, 0);
+          C = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[2], W[rt][1], C, 0, 0, 0);
+          D = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[3], W[rt][1], D, 0, 0, 0);
 #pragma unroll
-        for (int k = 0; k < 4; k++) C = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[k], W[rt][k >> 1], C, 0, 0, 0);
+          for (int v = 0; v < 16; v++) { Y[rt][v] = fmaf(dv, C[v], Y[rt][v]); U[rt][v] = fmaf(dv, D[v], U[rt][v]); }
+        } else {
 #pragma unroll
-        for (int v = 0; v < 16; v++) Y[rt][v] = fmaf(dv, C[v], Y[rt][v]);
+          for (int k = 1; k < 4; k++) C = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[k], W[rt][k >> 1], C, 0, 0, 0);
+#pragma unroll
+          for (int v = 0; v < 16; v++) Y[rt][v] = fmaf(dv, C[v], Y[rt][v]);
+        }
       }
       if constexpr (MIN)
 #pragma unroll
@@ -431,7 +444,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
           for (int rt = 0; rt < RT; rt++) {
             const float m = mp[32 * RT * g16 + 32 * rt + n];
 #pragma unroll
-            for (int v = 0; v < 16; v++) Y[rt][v] = fmaf(m, sv[v >> 2][v & 3], Y[rt][v]);
+            for (int v = 0; v < 16; v++) U[rt][v] = fmaf(m, sv[v >> 2][v & 3], U[rt][v]);
           }
         }
     }
@@ -456,7 +469,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
   for (int rt = 0; rt < RT; rt++)
 #pragma unroll
-    for (int v = 0; v < 16; v++) sacc[(wave * NV + rt * 16 + v) * 64 + lane] = Z[rt][v] + Y[rt][v];
+    for (int v = 0; v < 16; v++) sacc[(wave * NV + rt * 16 + v) * 64 + lane] = FINE ? Z[rt][v] + (Y[rt][v] + U[rt][v]) : Z[rt][v] + Y[rt][v];
   __syncthreads();
   // wave w sums the values w, w + NW, ...: the lane's value v of row tile rt is weight row n and token 8 (v / 4) + 4 kg + v % 4
 #pragma unroll
@@ -481,7 +494,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
         }
         if (any) y = sum;
       }
-    y *= p.sinv[t];
+    y *= p.sinv[t] * p.post;
     if (bias) y += bias[row];
     if (p.residual) y += p.residual[o];
     p.y[o] = y;
@@ -611,7 +624,8 @@ int launch_blk(const cai_qw_s* w, const BlkGemmParams& p0, int n_tiles_grouped)
 // ------------------------------------------------------------------------------------------
 // Types kept as their stored stream (Q2_K, Q3_K, Q4_1, Q5_0, Q5_1): a panel of rows at a time is rewritten as signed bytes with an f16 scale
 // a block of 32 - and, for the types with minima, a float a sixteen - and multiplied by the kernel above.  Codes and scales are exact:
-// Q5_0 q - 16; Q4_1, Q5_1 q - 8, q - 16 with m + 8 d, m + 16 d; Q3_K (32 - scale) * q with -d; Q2_K scale * (q - 2) with 2 d scale - dmin min.
+// Q5_0 q - 16; Q4_1, Q5_1 q - 8, q - 16 with m + 8 d, m + 16 d; Q3_K (32 - scale) * q with -d; Q2_K, all doubled, scale * (2 q - c) with c d scale - 2 dmin min,
+// c the whole number of 0 .. 6 next to 2 dmin min / (d scale).
 // (Codes about zero: with q from 0 up the two parts of a sum cancel, and its error doubles.)
 // In place of passes of eight tokens through the float walk, bound by its VALU work: 18944 x 3584 with 200 tokens Q3_K 2282 -> 175 us,
 // Q4_1 1321 -> 252, with 16 tokens 183 -> 74, 106 -> 90; 3584 x 3584 with 16 tokens 52 -> 24, 39 -> 30.  Rewriting takes about 2 bytes of
@@ -646,11 +660,13 @@ __global__ __launch_bounds__(256) void raw_expand_kernel(const uint8_t* __restri
     uint32_t qs[4];
     if constexpr (QT == CAI_Q2_K) {
       const int sc = blk[r] & 15, mn = blk[r] >> 4;
+      const float ds = raw_half(blk + 80) * (float)sc, dm = raw_half(blk + 82) * (float)(2 * mn);
+      const int c = (int)fminf(fmaxf(rintf(dm / ds), 0.0f), 6.0f);      // (0 / 0 counts as 0)
       raw_load16<4>(blk + 16 + (r >> 3) * 32 + 16 * (r & 1), qs);
       dh = *reinterpret_cast<const uint16_t*>(blk + 80);
 #pragma unroll
-      for (int t = 0; t < 16; t++) put(t, sc * (((raw_byte(qs, t) >> sh) & 3) - 2));
-      m = fmaf(raw_half(blk + 80), (float)(2 * sc), -(raw_half(blk + 82) * (float)mn));
+      for (int t = 0; t < 16; t++) put(t, sc * (2 * ((raw_byte(qs, t) >> sh) & 3) - c));
+      m = fmaf(ds, (float)c, -dm);
     } else {
       const int sc = -q3k_scale(blk + 96, r), bit = r >> 1;
       uint32_t hm[4];
@@ -716,9 +732,9 @@ int launch_raw(const cai_qw_s* w, const BlkGemmParams& p0)
     if (p.residual) p.residual += r0;
     auto cut = [&](auto rt_, auto nw_, auto odd_) {
       constexpr int RT = rt_, NW = nw_; constexpr bool ODD = odd_;
-      return launch_lds<gemm_blk_cut<CAI_Q8_0, RT, NW, ODD, MIN>>(blk_grid(p, 32 * RT, tok32), 64 * NW, NW * 2 * (8192 + RT * 2048 + (ODD ? 512 : 256) + (MIN ? 512 + 512 * RT : 0)), p);
+      return launch_lds<gemm_blk_cut<CAI_Q8_0, RT, NW, ODD, true, MIN>>(blk_grid(p, 32 * RT, tok32), 64 * NW, NW * 2 * (8192 + RT * 2048 + (ODD ? 512 : 256) + (MIN ? 512 + 512 * RT : 0)), p);
     };
-    // (always cut tiles, whose sums are short chains: 1.4e-7 off 64 bits at width 3584, as the float walk of eight tokens a pass; large tiles 2e-7)
+    // (always cut tiles, whose sums are short chains: 0.95e-7 off 64 bits at width 3584, the float walk of eight tokens a pass 1.5e-7; large tiles 2e-7)
     auto form = [&](auto odd_) {
       if ((int64_t)((n + 31) / 32) * tok32 <= n_cu) return cut(std::integral_constant<int, 1>(), std::integral_constant<int, 6>(), odd_);
       if ((int64_t)((n + 63) / 64) * tok32 <= n_cu || MIN) return cut(std::integral_constant<int, 2>(), std::integral_constant<int, 4>(), odd_);
@@ -742,7 +758,7 @@ int launch_gemm_blk(const cai_qw_s* w, const _Float16* xhi, const _Float16* xlo,
   BlkGemmParams p{};
   p.q = w->data; p.d = w->aux; p.bias = w->bias; p.rows = (int)w->rows; p.cols = (int)w->cols;
   p.xhi = xhi; p.xlo = xlo; p.sinv = sinv; p.n_tok = n_tok; p.y = y; p.y_stride = y_stride; p.residual = residual;
-  p.x_div = 1; p.expert_rows = 0;
+  p.x_div = 1; p.expert_rows = 0; p.post = 1.0f;
   return launch_blk(w, p, 0);
 }
 
@@ -761,7 +777,7 @@ int launch_gemm_blk_multi(const cai_qw_s* const* ws, const int* y_off, int n_w, 
   BlkGemmParams p{};
   p.q = w->data; p.d = w->aux; p.bias = w->bias; p.rows = (int)w->rows; p.cols = (int)w->cols;
   p.xhi = xhi; p.xlo = xlo; p.sinv = sinv; p.n_tok = n_tok; p.y = y + y_off[0]; p.y_stride = y_stride; p.residual = nullptr;
-  p.x_div = 1; p.expert_rows = 0; p.n_seg = n_w;
+  p.x_div = 1; p.expert_rows = 0; p.post = 1.0f; p.n_seg = n_w;
   for (int i = 1; i < n_w; i++) { p.q2[i - 1] = ws[i]->data; p.d2[i - 1] = ws[i]->aux; p.bias2[i - 1] = ws[i]->bias; p.rows2[i - 1] = (int)ws[i]->rows; p.y_off2[i - 1] = y_off[i] - y_off[0]; }
   return launch_blk(w, p, 0);
 }
@@ -780,7 +796,7 @@ int launch_gemm_raw(const cai_qw_s* w, const _Float16* xhi, const _Float16* xlo,
   const int64_t most = std::max<int64_t>(32, std::min<int64_t>(4096, ((int64_t)1 << 31) / w->cols) / 32 * 32);
   for (int64_t t = 0; t < n_tok; t += most) {
     BlkGemmParams p{};
-    p.bias = w->bias; p.cols = (int)w->cols; p.x_div = 1;
+    p.bias = w->bias; p.cols = (int)w->cols; p.x_div = 1; p.post = w->qtype == CAI_Q2_K ? 0.5f : 1.0f;
     p.n_tok = (int)std::min<int64_t>(most, n_tok - t);
     p.xhi = xhi + t * w->cols; p.xlo = xlo + t * w->cols; p.sinv = sinv + t; p.y = y + t * y_stride; p.y_stride = y_stride;
     p.residual = residual ? residual + t * y_stride : nullptr;
