@@ -1418,6 +1418,7 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
       ql[s] = *reinterpret_cast<const ph8_t*>(p.qlo + qo + 16 * s);
     }
   }
+  const int last = p.pos[p.n_tok - 1];            // rows behind it hold what an earlier sequence left: not multiplied, not even by zero
   pf16_t O[HD / 32];
 #pragma unroll
   for (int dt = 0; dt < HD / 32; dt++)
@@ -1461,6 +1462,11 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
     __syncthreads();                                        // the previous tile has been consumed
     {
       float kv[E], vv[E];
+      if (jt * 32 + srow > last) {
+#pragma unroll
+        for (int i = 0; i < (int)(sizeof(raw.v) / sizeof(uint4)); i++) raw.v[i] = make_uint4(0u, 0u, 0u, 0u);
+        raw.vs = 0.0f;
+      }
       if (I8P) {
         const uint4 a = raw.k[0], b = raw.v[0];
         const float ks = raw.ks, vs = raw.vs;

@@ -416,6 +416,31 @@ def test_prompt_attention_of_64_wide_heads_on_matrix_cores(kv, window, hq, hkv):
     dec.close()
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("kv", ["f32", "f16", "i8"])
+def test_prompt_attention_leaves_alone_what_an_earlier_sequence_left(kv, hd):
+    """a prompt of NaN rows, reset, then a healthy one whose last tile of 32 cached rows ends inside what is left of it"""
+    from helpers.device import dev
+    cai = dev()
+    cfg = dict(n_layers=1, d_model=256, n_q_heads=4, n_kv_heads=2, head_dim=hd, ffn=256, vocab=300, max_ctx=640, eps=1e-5, rope_theta=1e4)
+    spec = synthetic_spec(cfg, O.Q8_0, head_qtype=O.Q8_0, seed=3, std=0.05)
+    spec["vecs"][(0, O.V_ATTN_NORM)] = np.ones(256, np.float32)
+    t = spec["tensors"][(-1, O.W_EMBED)]
+    raw = t["raw"].reshape(300, -1)
+    raw[299, 0:2] = np.array([np.inf], np.float16).view(np.uint8)       # token 299: the scale of its first block
+    t["raw"] = raw.reshape(-1)
+    dec = cai.Decoder(spec, kv_dtype={"f32": cai.KV_F32, "f16": cai.KV_F16, "i8": cai.KV_I8}[kv])
+    toks = np.random.default_rng(hd).integers(0, 299, 257).astype(np.int32)
+    _, want = dec.prefill(toks)
+    dec.reset(0)
+    _, bad = dec.prefill(np.full(400, 299, np.int32))
+    assert not np.isfinite(bad).any()
+    dec.reset(0)
+    _, got = dec.prefill(toks)
+    np.testing.assert_array_equal(got, want)
+    dec.close()
+
+
 @pytest.mark.parametrize("name", ["qwen7b_like_q4k", "olmoe_like_q8"])
 def test_per_class_timing_leaves_the_session_as_it_found_it(name):
     """cai_decoder_profile (a measurement aid without a counterpart in the reference) replays whole steps and steps without one
