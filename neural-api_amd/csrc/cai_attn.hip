@@ -1318,6 +1318,10 @@ __global__ __launch_bounds__(256) void kv_append_rows_i8_kernel(const AttnParams
 //                               result registers of k-step s are exactly the B operand of step s of the next product;
 //   O^T[dim][token] += V^T . P^T   with P split hi + lo into two f16 (22 bits), like q; a float cache is split too.
 // Same arithmetic as the decode kernels up to the order of the sums (tests: < 1e-4 of token-at-a-time ingestion).
+// A pair of halfs ends at 65504 and loses bits below 2^-14, so heads of 64, whose per-row kernel holds floats, scale every operand by a power of
+// two first: q per token and head, the rows of a float cache each (int8 codes are exact halfs; their scales count as the row's), the weights
+// times the value rows' scales per token and tile, whose sums are then added to O as floats; over a half cache only q and, by 2^14, the
+// weights.  9 / 3 heads, float cache, six layers of a 511-token prompt: 593 us without, 630; values of 1e-5 were 7e-5 off and such past 65504 NaN.
 // ------------------------------------------------------------------------------------------
 typedef float pf16_t __attribute__((ext_vector_type(16)));
 
@@ -1331,6 +1335,7 @@ struct PromptParams {
   const float* theta; const int32_t* pos;
   float* out; int64_t out_stride;
   float* part;                               // [token][q_head][K split][HD + 2]: unnormalised sums, maximum, normaliser
+  float* qsc;                                // HD = 64: [token][q_head] what the head's planes are to be multiplied by
 };
 
 constexpr int PA_KT_MIN = 2;     // K tiles (of 32 cached rows) a split takes at least
@@ -1361,7 +1366,14 @@ __device__ __forceinline__ void prompt_q_row(const PromptParams& p)
       x0 = y0; x1 = y1;
     }
     _Float16 h0, h1, l0, l1;
-    split_f16(x0, h0, l0); split_f16(x1, h1, l1);
+    if constexpr (HD == 64) {               // (32 neighbouring lanes hold a head)
+      float m = fmaxf(finite_abs(x0), finite_abs(x1));
+#pragma unroll
+      for (int off = 1; off < 32; off <<= 1) m = fmaxf(m, __shfl_xor(m, off));
+      const int ex = plane_exponent(m);
+      split_plane(ldexpf(x0, ex), h0, l0); split_plane(ldexpf(x1, ex), h1, l1);
+      if ((e & 31) == 0) p.qsc[(int64_t)t * p.q_heads + (e >> 5)] = ldexpf(1.0f, -ex);
+    } else { split_f16(x0, h0, l0); split_f16(x1, h1, l1); }
     p.qhi[(int64_t)t * qw + 2 * e] = h0; p.qhi[(int64_t)t * qw + 2 * e + 1] = h1;
     p.qlo[(int64_t)t * qw + 2 * e] = l0; p.qlo[(int64_t)t * qw + 2 * e + 1] = l1;
   }
@@ -1377,13 +1389,16 @@ constexpr int PA_LDV = 36;     // halfs per staged V^T row (32 cached rows + pad
 template <typename KV_T, int HD>
 __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
 {
-  constexpr bool I8P = sizeof(KV_T) == 1;         // int8 rows are dequantised (code * row scale) while they are staged
-  constexpr bool F32 = sizeof(KV_T) != 2;         // ... and, like a float cache, split hi + lo
+  constexpr bool I8P = sizeof(KV_T) == 1;         // int8 rows: HD = 128: dequantised (code * row scale) while they are staged
+  constexpr bool SC = HD == 64;                   // every operand holds what a float holds, whatever its size: see the comment above
+  constexpr bool F32 = SC ? sizeof(KV_T) == 4 : sizeof(KV_T) != 2;         // ... and, like a float cache, split hi + lo
+  constexpr bool ROWS = SC && sizeof(KV_T) != 2;  // row scales
   constexpr int NP = F32 ? 2 : 1;                 // planes of K and V
   constexpr int PA_LDK = HD + 8;                  // halfs per staged K row (rows stay 16-byte aligned for the 8-half operand reads)
   constexpr int E = HD / 8;                       // elements of a row that a thread stages
   __shared__ __align__(16) _Float16 sK[NP][32 * PA_LDK];
   __shared__ __align__(16) _Float16 sV[NP][HD * PA_LDV];
+  __shared__ __align__(16) float sKS[ROWS ? 32 : 4], sVS[ROWS ? 32 : 4];      // of each cached row: what its staged K and V are to be multiplied by
   const int G = p.q_heads / p.kv_heads, quads = (G + 3) >> 2;
   const int g = blockIdx.y / quads, h0 = (blockIdx.y % quads) * 4;
   const int t0 = blockIdx.x * 32;
@@ -1418,6 +1433,7 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
       ql[s] = *reinterpret_cast<const ph8_t*>(p.qlo + qo + 16 * s);
     }
   }
+  const float qs = SC ? p.qsc[(int64_t)min(tok, p.n_tok - 1) * p.q_heads + head] * p.inv_sqrt : p.inv_sqrt;
   const int last = p.pos[p.n_tok - 1];            // rows behind it hold what an earlier sequence left: not multiplied, not even by zero
   pf16_t O[HD / 32];
 #pragma unroll
@@ -1469,7 +1485,8 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
       }
       if (I8P) {
         const uint4 a = raw.k[0], b = raw.v[0];
-        const float ks = raw.ks, vs = raw.vs;
+        const float ks = ROWS ? 1.0f : raw.ks, vs = ROWS ? 1.0f : raw.vs;     // (codes are exact halfs)
+        if (ROWS && (tid & 7) == 0) { sKS[srow] = raw.ks; sVS[srow] = raw.vs; }
         const int aw[4] = {(int)a.x, (int)a.y, (int)a.z, (int)a.w}, bw[4] = {(int)b.x, (int)b.y, (int)b.z, (int)b.w};
 #pragma unroll
         for (int i = 0; i < E / 4; i++) {
@@ -1484,6 +1501,17 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
           const uint4 a = raw.k[c4], b = raw.v[c4];
           kv[4 * c4] = __builtin_bit_cast(float, a.x); kv[4 * c4 + 1] = __builtin_bit_cast(float, a.y); kv[4 * c4 + 2] = __builtin_bit_cast(float, a.z); kv[4 * c4 + 3] = __builtin_bit_cast(float, a.w);
           vv[4 * c4] = __builtin_bit_cast(float, b.x); vv[4 * c4 + 1] = __builtin_bit_cast(float, b.y); vv[4 * c4 + 2] = __builtin_bit_cast(float, b.z); vv[4 * c4 + 3] = __builtin_bit_cast(float, b.w);
+        }
+        if constexpr (ROWS) {                             // (the eight threads of a row are neighbours)
+          float mk = 0.0f, mv = 0.0f;
+#pragma unroll
+          for (int i = 0; i < E; i++) { mk = fmaxf(mk, finite_abs(kv[i])); mv = fmaxf(mv, finite_abs(vv[i])); }
+#pragma unroll
+          for (int off = 1; off < 8; off <<= 1) { mk = fmaxf(mk, __shfl_xor(mk, off)); mv = fmaxf(mv, __shfl_xor(mv, off)); }
+          const int ek = plane_exponent(mk), ev = plane_exponent(mv);
+#pragma unroll
+          for (int i = 0; i < E; i++) { kv[i] = ldexpf(kv[i], ek); vv[i] = ldexpf(vv[i], ev); }
+          if ((tid & 7) == 0) { sKS[srow] = ldexpf(1.0f, -ek); sVS[srow] = ldexpf(1.0f, -ev); }
         }
       }
       if constexpr (sizeof(KV_T) == 2) {                  // a half cache goes in as it is
@@ -1504,13 +1532,14 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
       for (int i4 = 0; i4 < E / 4; i4++) {                    // K rows stay row-major: 8-byte stores
         ph4_t kh, kl;
 #pragma unroll
-        for (int i = 0; i < 4; i++) { _Float16 a, b; split_f16(kv[4 * i4 + i], a, b); kh[i] = a; kl[i] = b; }
+        for (int i = 0; i < 4; i++) { _Float16 a, b; if (SC) split_plane(kv[4 * i4 + i], a, b); else split_f16(kv[4 * i4 + i], a, b); kh[i] = a; kl[i] = b; }
         *reinterpret_cast<ph4_t*>(&sK[0][srow * PA_LDK + sdim + 4 * i4]) = kh;
         if (F32) *reinterpret_cast<ph4_t*>(&sK[NP - 1][srow * PA_LDK + sdim + 4 * i4]) = kl;
       }
 #pragma unroll
       for (int i = 0; i < E; i++) {                       // V goes in transposed
-        _Float16 vh, vl; split_f16(vv[i], vh, vl);
+        _Float16 vh, vl;
+        if (SC) split_plane(vv[i], vh, vl); else split_f16(vv[i], vh, vl);
         sV[0][(sdim + i) * PA_LDV + srow] = vh;
         if (F32) sV[NP - 1][(sdim + i) * PA_LDV + srow] = vl;
       }
@@ -1537,10 +1566,15 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
     // ---- this token's column: mask, running maximum, weights ----
     float tmax = -1e30f;
     bool ok[16];
+    float4 rs[ROWS ? 4 : 1];
+    if constexpr (ROWS)
+#pragma unroll
+      for (int i = 0; i < 4; i++) rs[i] = *reinterpret_cast<const float4*>(&sKS[8 * i + 4 * kg]);
+    auto row_scale = [&](int v) { const float4 r = rs[ROWS ? v >> 2 : 0]; return (v & 3) == 0 ? r.x : (v & 3) == 1 ? r.y : (v & 3) == 2 ? r.z : r.w; };
 #pragma unroll
     for (int v = 0; v < 16; v++) {
       const int krow = jt * 32 + 8 * (v >> 2) + 4 * kg + (v & 3);
-      float sc = C[v] * p.inv_sqrt;
+      float sc = C[v] * (ROWS ? row_scale(v) * qs : qs);
       if (p.softcap > 0.0f) sc = p.softcap * tanhf(sc / p.softcap);
       ok[v] = krow <= pos_n && krow >= jstart_n;
       C[v] = sc;
@@ -1550,7 +1584,7 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
     const float m_new = fmaxf(m_run, tmax), corr = expf(m_run - m_new);
     float psum = 0.0f;
 #pragma unroll
-    for (int v = 0; v < 16; v++) { C[v] = ok[v] ? expf(C[v] - m_new) : 0.0f; psum += C[v]; }
+    for (int v = 0; v < 16; v++) { C[v] = ok[v] ? (SC && !ROWS ? 16384.0f : 1.0f) * expf(C[v] - m_new) : 0.0f; psum += C[v]; }   // (half cache: weights of 2^-39 on stay)
     psum += __shfl_xor(psum, 32, 64);
     l_run = l_run * corr + psum; m_run = m_new;
     if (__builtin_amdgcn_ballot_w64(corr != 1.0f)) {      // (after the first tiles a new maximum is rare: the whole wave skips the rescaling)
@@ -1558,6 +1592,25 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
       for (int dt = 0; dt < HD / 32; dt++)
 #pragma unroll
         for (int v = 0; v < 16; v++) O[dt][v] *= corr;
+    }
+    // row scales: the weights take them, and a power of two per token and tile brings the largest to 2^13
+    float back = 1.0f;
+    pf16_t T[ROWS ? HD / 32 : 1];
+    if constexpr (ROWS) {
+      float wmax = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 4; i++) rs[i] = *reinterpret_cast<const float4*>(&sVS[8 * i + 4 * kg]);
+#pragma unroll
+      for (int v = 0; v < 16; v++) { C[v] = ok[v] ? C[v] * row_scale(v) : 0.0f; wmax = fmaxf(wmax, finite_abs(C[v])); }
+      wmax = fmaxf(wmax, __shfl_xor(wmax, 32, 64));
+      const int e = plane_exponent(wmax);
+      back = ldexpf(1.0f, -e);
+#pragma unroll
+      for (int v = 0; v < 16; v++) C[v] = ldexpf(C[v], e);
+#pragma unroll
+      for (int dt = 0; dt < HD / 32; dt++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) T[dt][v] = 0.0f;
     }
     // ---- O^T += V^T . P^T ----
     // The score registers 8 s2 .. 8 s2 + 7 of a lane are cached rows 16 s2 + 4 kg + (0..3) and 16 s2 + 8 + 4 kg + (0..3): taken as
@@ -1573,16 +1626,22 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
         const ph4_t a0 = *reinterpret_cast<const ph4_t*>(&sV[0][(32 * dt + n) * PA_LDV + 16 * s2 + 4 * kg]);
         const ph4_t a1 = *reinterpret_cast<const ph4_t*>(&sV[0][(32 * dt + n) * PA_LDV + 16 * s2 + 8 + 4 * kg]);
         const ph8_t a = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
-        O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, ph, O[dt], 0, 0, 0);
-        O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pl, O[dt], 0, 0, 0);
+        pf16_t& S = ROWS ? T[ROWS ? dt : 0] : O[dt];
+        S = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, ph, S, 0, 0, 0);
+        S = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pl, S, 0, 0, 0);
         if (F32) {
           const ph4_t b0 = *reinterpret_cast<const ph4_t*>(&sV[NP - 1][(32 * dt + n) * PA_LDV + 16 * s2 + 4 * kg]);
           const ph4_t b1 = *reinterpret_cast<const ph4_t*>(&sV[NP - 1][(32 * dt + n) * PA_LDV + 16 * s2 + 8 + 4 * kg]);
           const ph8_t al = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
-          O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, ph, O[dt], 0, 0, 0);
+          S = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, ph, S, 0, 0, 0);
         }
       }
     }
+    if constexpr (ROWS)
+#pragma unroll
+      for (int dt = 0; dt < HD / 32; dt++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) O[dt][v] = fmaf(T[dt][v], back, O[dt][v]);
   }
   if (!head_on || !tok_on) return;
   if (splits > 1) {        // this piece's unnormalised sums, maximum and normaliser; prompt_merge_kernel adds the pieces
@@ -1632,9 +1691,9 @@ __global__ __launch_bounds__(512) void prompt_merge_kernel(const PromptParams p,
 }
 
 // Whether n prompt rows of this cache go to the matrix-core prompt kernel (it needs no per-slice partial results).
-// Heads of 128: from 8 rows on.  Heads of 64: from 256 on, where the per-row kernel's reads of the cache outgrow its launch (9 / 3
-// heads, six layers, float cache: 128 tokens 383 us per row, 395 here; 300: 772, 452; 1500: 3799, 1727; 8 / 8 heads, three layers,
-// 200 tokens: 261, 272).
+// Heads of 128: from 8 rows on.  Heads of 64: from 256 on, where the per-row kernel's reads of the cache outgrow its launch (first chunks of
+// 9 / 3 heads, a whole prompt through six layers, float cache: 128 tokens 383 us per row, 395 here (with operands that were not scaled
+// yet); 256: 929, 486; 511: 1317, 630; 1500: 4313, 1878; int8 6698, 1873; 8 / 8 heads, three layers, 200 tokens: 261, 272).
 bool attn_prompt_is_flash(const cai_kv_s* kv, int n)
 {
   static const int flash_on = []() { const char* e = getenv("CAIHIP_PROMPT_FLASH"); return e ? atoi(e) : 1; }();
@@ -1701,11 +1760,12 @@ int launch_attn_step(cai_kv_s* kv, int layer, float* qkv, int64_t qkv_stride, in
       if (kv->pq_lo) (void)hipFree(kv->pq_lo);
       kv->pq_hi = kv->pq_lo = nullptr; kv->pq_cap = 0;
       CAI_HIP(hipMalloc(&kv->pq_hi, need * 2));
-      CAI_HIP(hipMalloc(&kv->pq_lo, need * 2));
+      CAI_HIP(hipMalloc(&kv->pq_lo, need * 2 + need / p.hd * 4));
       kv->pq_cap = need;
     }
     PromptParams pp{};
     pp.qkv = qkv; pp.qkv_stride = qkv_stride; pp.qhi = (_Float16*)kv->pq_hi; pp.qlo = (_Float16*)kv->pq_lo;
+    pp.qsc = (float*)(pp.qlo + kv->pq_cap);
     const size_t plane = ((size_t)seq0 * kv->seq_elems() + (size_t)layer * kv->layer_elems()) * kv->elem();
     pp.kc = (const char*)kv->k + plane; pp.vc = (const char*)kv->v + plane;
     if (kv->dtype == CAI_KV_I8) {

@@ -100,6 +100,18 @@ __device__ __forceinline__ void split_f16(float x, _Float16& hi, _Float16& lo)
   const float h = __builtin_bit_cast(float, (b + 0xFFFu + ((b >> 13) & 1u)) & 0xFFFFE000u);
   hi = (_Float16)h; lo = (_Float16)(x - h);
 }
+// The pair over the whole number range of a float: values that belong together are multiplied by 2^e, e = plane_exponent of the largest
+// finite one, before they are split; an infinity is hi = infinity and lo = 0.
+__device__ __forceinline__ float finite_abs(float v) { const float a = fabsf(v); return a < __builtin_inff() ? a : 0.0f; }
+__device__ __forceinline__ int plane_exponent(float a)      // a = m*2^ex, m in [0.5,1) -> a*2^e in [2^13, 2^14)
+{
+  return a > 0.0f ? min(14 - __builtin_amdgcn_frexp_expf(a), 126) : 0;   // (2^-126 is the smallest normal reciprocal: 2^-149 is then 2^-23, above the steps of a half)
+}
+__device__ __forceinline__ void split_plane(float x, _Float16& hi, _Float16& lo)
+{
+  split_f16(x, hi, lo);
+  if (fabsf(x) == __builtin_inff()) lo = (_Float16)0.0f;
+}
 
 // Walks x[i0], x[i0 + step], ... (< n, n >= 1) and hands every value to f(value, index) in index order.  Eight requests go out
 // before the first value is used: a loop that uses each value as it arrives pays one cache round trip per element, which is
@@ -179,7 +191,7 @@ struct cai_kv_s {
   int32_t* d_len = nullptr;               // [seq] device scratch: rows live BEFORE the token being decoded
   int32_t* d_iota = nullptr;              // [max_ctx] 0, 1, 2, ... behind d_len: positions that need no upload (a cache of its own only, not a decoder's)
   unsigned* merge_cnt = nullptr;          // [seq][part_q_heads] arrival counters of the in-kernel merge of the split partials (wrap to 0 by themselves)
-  void* pq_hi = nullptr; void* pq_lo = nullptr; size_t pq_cap = 0;   // prompt ingestion: rotated q of a chunk as two f16 planes
+  void* pq_hi = nullptr; void* pq_lo = nullptr; size_t pq_cap = 0;   // prompt ingestion: rotated q of a chunk as two f16 planes; behind the lo plane (of pq_cap halfs) a scale per head
   float* pq_part = nullptr; size_t pq_part_cap = 0;                     // prompt ingestion: partial results of a token tile's K splits
   size_t elem() const { return dtype == CAI_KV_F16 ? 2 : dtype == CAI_KV_I8 ? 1 : 4; }
   int64_t layer_rows() const { return (int64_t)kv_heads * max_ctx; }

@@ -28,18 +28,6 @@ typedef float float16_t __attribute__((ext_vector_type(16)));
 // the pre-pass of the down projection (no norm in that case).
 // An infinity is hi = infinity and lo = 0, so that a product shows it with the sign of its weight; a NaN stays one.
 // ------------------------------------------------------------------------------------------
-__device__ __forceinline__ float finite_abs(float v) { const float a = fabsf(v); return a < __builtin_inff() ? a : 0.0f; }
-__device__ __forceinline__ int plane_exponent(float a)      // a = m*2^ex, m in [0.5,1) -> a*2^e in [2^13, 2^14)
-{
-  int e = 0;
-  if (a > 0.0f) { int ex; frexpf(a, &ex); e = 14 - ex; }
-  return min(e, 126);                                       // (2^-126 is the smallest normal reciprocal: 2^-149 is then 2^-23, above the steps of a half)
-}
-__device__ __forceinline__ void split_plane(float x, _Float16& hi, _Float16& lo)
-{
-  split_f16(x, hi, lo);
-  if (fabsf(x) == __builtin_inff()) lo = (_Float16)0.0f;
-}
 template <bool SWIGLU, int NT>     // NT threads per token
 __global__ __launch_bounds__(NT) void xprep_kernel(const float* x, int64_t x_stride, const float* gain, float eps, int K,
                                                     _Float16* hi, _Float16* lo, float* sinv, _Float16* sxhi, _Float16* sxlo)

@@ -416,6 +416,35 @@ def test_prompt_attention_of_64_wide_heads_on_matrix_cores(kv, window, hq, hkv):
     dec.close()
 
 
+@pytest.mark.parametrize("kv,gain,std_qk,std_v,std_o", [("f32", 1e-4, 600.0, 0.05, 60.0), ("f32", 2e4, 5e-6, 0.4, 1e-5), ("i8", 2e4, 5e-6, 0.4, 1e-5), ("f16", 1e-4, 600.0, 600.0, 6e-3)])
+def test_prompt_attention_of_64_wide_heads_at_any_size_of_its_values(kv, gain, std_qk, std_v, std_o):
+    """values of 1e-5 and of 1e5, the latter past the largest half, with scores of ordinary size; the attention's output outweighs the stream.
+    A float cache keeps them as floats, so the logits are those of the oracle to the roundings of a 32-bit pass (1e-6, measured 1e-6 with values
+    of size one); an int8 cache may store a code one step apart now and then"""
+    from helpers.device import dev, rel_err
+    from helpers.model_build import _t
+    cai = dev()
+    cfg = dict(n_layers=1, d_model=256, n_q_heads=6, n_kv_heads=2, head_dim=64, ffn=256, vocab=300, max_ctx=640, eps=1e-5, rope_theta=1e4)
+    spec = synthetic_spec(cfg, O.Q8_0, head_qtype=O.Q8_0, seed=7, std=0.05)
+    rng = np.random.default_rng(8)
+    for slot, rows, cols, std in ((O.W_Q, 384, 256, std_qk), (O.W_K, 128, 256, std_qk), (O.W_V, 128, 256, std_v), (O.W_O, 256, 384, std_o)):
+        spec["tensors"][(0, slot)] = _t((rng.standard_normal((rows, cols)) * std).astype(np.float32), O.Q8_0)
+    spec["vecs"][(0, O.V_ATTN_NORM)] = np.full(256, gain, np.float32)
+    om, dec = oracle_model(spec, acc64=1), cai.Decoder(spec, max_batch=2, kv_dtype={"f32": cai.KV_F32, "f16": cai.KV_F16, "i8": cai.KV_I8}[kv])
+    toks = rng.integers(0, 300, 257).astype(np.int32)
+    _, got = dec.prefill(toks)
+    assert np.isfinite(got).all()
+    if kv == "f32":
+        for p, t in enumerate(toks): _, want = om.step(int(t), p)
+        assert rel_err(got, want) < 1e-5
+    p = 0
+    for m in (100, 100, 57):                       # the same prompt through the per-row kernels
+        _, rows = dec.prefill(toks[p:p + m], p, seq=1)
+        p += m
+    assert rel_err(got, rows) < {"f32": 1e-5, "f16": 1e-3, "i8": 5e-3}[kv]
+    dec.close()
+
+
 @pytest.mark.parametrize("hd", [64, 128])
 @pytest.mark.parametrize("kv", ["f32", "f16", "i8"])
 def test_prompt_attention_leaves_alone_what_an_earlier_sequence_left(kv, hd):
