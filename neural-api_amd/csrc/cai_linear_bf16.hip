@@ -480,11 +480,18 @@ static int run_lin(const cai_qw_s* w, const AT* x, int64_t ldx, int n_tok, const
     return CAI_OK;
   }
   auto tiles = [&](int bm, int bn) { return (int64_t)((n_tok + bm - 1) / bm) * ((w->rows + bn - 1) / bn); };
-  // (2048 tokens, a 4-layer decoder of width 2048, its whole prompt: 128 x 128 by four waves 2783 us, by eight 2607, 256 x 128 by sixteen
-  // 2546, 256 x 256 by sixteen 3009; where 128 x 128 leaves CUs idle the halved tiles of 64 x 64 are faster: 511 tokens, width 512: 609, 628)
+  // 256 x 128 by sixteen waves, one work-group a CU, or 128 x 128 by eight, two a CU: whichever takes less time by rounds over the chip.  A
+  // full round takes 32 us of the one and 37 of the other (at a depth of 2048), one of at most a work-group a CU 28.  Products alone, us,
+  // 256 x 128 | 128 x 128 (by four waves, staged through registers, before): 11264 rows, 300 tokens 30.8 | 31.9 (40.7), 640: 57.1 | 35.6
+  // (46.2), 768: 59.0 | 57.1, 1024: 63.5 | 67.5, 2048: 98.6 | 110.2 (127); 32800 rows, 128 tokens 57.6 | 43.9 (45.4); 49152 rows, 100: 61.1 | 50.4.
+  // (Where 128 x 128 leaves CUs idle the halved tiles of 64 x 64 are faster: whole prompt of 511 tokens, width 512: 609, 628.)
   if (n_tok > 64 && tiles(128, 128) >= ctx().n_cu) {
-    if constexpr (sizeof(AT) == 2) return run_gemm<AT, 256, 128, 4, 4, 3>(w, x, ldx, n_tok, e);
-    else return run_gemm<AT, 128, 128, 2, 2>(w, x, ldx, n_tok, e);
+    if constexpr (sizeof(AT) == 2) {
+      const int64_t n_cu = ctx().n_cu, large = tiles(256, 128), small = tiles(128, 128), left = small % (2 * n_cu);
+      if (32 * ((large + n_cu - 1) / n_cu) <= 37 * (small / (2 * n_cu)) + (left == 0 ? 0 : left <= n_cu && small > n_cu ? 28 : 37))
+        return run_gemm<AT, 256, 128, 4, 4, 3>(w, x, ldx, n_tok, e);
+    }
+    return run_gemm<AT, 128, 128, 2, sizeof(AT) == 2 ? 4 : 2>(w, x, ldx, n_tok, e);
   }
   if (n_tok > 32 && tiles(64, 64) >= ctx().n_cu) return run_gemm<AT, 64, 64, 2, 2>(w, x, ldx, n_tok, e);
   return run_gemm<AT, 32, 64, 2, 2>(w, x, ldx, n_tok, e);

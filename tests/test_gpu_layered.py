@@ -104,6 +104,17 @@ def test_products_on_tiles_of_256_tokens(cai, tmp_path, tokens, ff):
     dec.close()
 
 
+@pytest.mark.parametrize("tokens, ff, width", [(300, 12000, 448), (700, 12000, 320), (129, 16400, 448), (600, 5632, 320)])
+def test_products_on_large_tiles_of_many_steps(cai, tmp_path, tokens, ff, width):
+    """the same products seven and five steps of 64 deep, so that every slot of the tiles' rings is filled again and the last fill lies in another
+    slot than the first: tiles of 256 x 128 (12000) and of 128 x 128 (the others)"""
+    m = Model(tmp_path, B.config([B.layer(B.delta(), ff=ff)], width=width, vocab=67), seed=tokens, edit=only("feed-forward"), rank_a=3, rank_g=20)
+    tok = m.tokens(tokens, 1)
+    dec = m.open(cai, 768, 1, "bf16")
+    check(feed(dec, tok, [tokens]), m.ref(tok), "bf16")
+    dec.close()
+
+
 # ---------------------------------------------------------------- whole models
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
 @pytest.mark.parametrize("cuts", [[300], [1], [2], [3, 2, 65, 1, 1, 16, 17, 2], [64], [130, 1], [5, 9, 7]], ids=str)
