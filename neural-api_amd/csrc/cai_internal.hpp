@@ -330,7 +330,11 @@ int launch_gemm_blk_multi(const cai_qw_s* const* ws, const int* y_off, int n_w, 
 bool prefill_multi_supported(const cai_qw_s* const* ws, int n_w);   // one launch of a prompt kernel takes these matrices together
 int launch_gemm_q4k_multi(const cai_qw_s* const* ws, const int* y_off, int n_w, const _Float16* xhi, const _Float16* xlo, const _Float16* sxhi,
                           const _Float16* sxlo, const float* sinv, int n_tok, float* y, int64_t y_stride, const float* residual, int swiglu_half);
-bool gemm_wide_wanted(const cai_qw_s* w, int64_t rows_all, int n_tok);   // prompt product on wide tiles (cai_prefill_wide.hip)
+bool gemm_wide_wanted(const cai_qw_s* const* ws, int n_w, int n_tok);   // prompt product on wide tiles (cai_prefill_wide.hip)
+// Its kernels reach a token of the planes and a row of each matrix through 32-bit byte offsets: a plane of less than 2 GiB, a matrix of less than
+// 4000 MiB (whose last row begins below 2^32).
+constexpr bool wide_offsets_fit(int64_t n_tok, int64_t cols, int64_t data_bytes) { return n_tok * cols < (int64_t)1 << 30 && data_bytes < (int64_t)4000 << 20; }
+static_assert(wide_offsets_fit(2048, 18944, (int64_t)3999 << 20) && !wide_offsets_fit(2048, 18944, (int64_t)4000 << 20) && !wide_offsets_fit(1 << 15, 1 << 15, 1), "the last byte a tile reads lies below 2^32");
 int launch_gemm_wide(const cai_qw_s* const* ws, const int* y_off, int n_w, const _Float16* xhi, const _Float16* xlo, const _Float16* sxhi,
                      const _Float16* sxlo, const float* sinv, int n_tok, float* y, int64_t y_stride, const float* residual, int swiglu_half);
 void wide_release();                                           // frees its buffer of partial sums (cai_shutdown)

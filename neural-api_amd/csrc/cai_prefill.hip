@@ -654,9 +654,9 @@ int launch_gemm_q4k_multi(const cai_qw_s* const* ws, const int* y_off, int n_w, 
   if (n_w > 1 && (!gemm_q4k_multi_supported(ws, n_w) || residual)) return set_error(CAI_ERR_UNSUPPORTED, "prefill gemm: %d matrices in one launch", n_w);
   if (swiglu_half && (n_w != 1 || residual || w->qtype == CAI_Q6_K || w->rows != 2 * (int64_t)swiglu_half))
     return set_error(CAI_ERR_UNSUPPORTED, "prefill gemm: fused SwiGLU needs one Q4_K / Q5_K matrix of 2 x %d rows", swiglu_half);
+  if (gemm_wide_wanted(ws, n_w, n_tok)) return launch_gemm_wide(ws, y_off, n_w, xhi, xlo, sxhi, sxlo, sinv, n_tok, y, y_stride, residual, swiglu_half);
   int64_t rows_all = 0;
   for (int i = 0; i < n_w; i++) rows_all += ws[i]->rows;
-  if (gemm_wide_wanted(w, rows_all, n_tok)) return launch_gemm_wide(ws, y_off, n_w, xhi, xlo, sxhi, sxlo, sinv, n_tok, y, y_stride, residual, swiglu_half);
   GemmParams p{};
   p.w = w->data; p.bias = w->bias; p.rows = (int)w->rows; p.cols = (int)w->cols;
   p.xhi = xhi; p.xlo = xlo; p.sxhi = sxhi; p.sxlo = sxlo; p.sinv = sinv; p.n_tok = n_tok; p.y = y + y_off[0]; p.y_stride = y_stride;
@@ -778,7 +778,7 @@ int prefill_gemm_multi(const cai_qw_s* const* ws, const int* y_off, int n_w, int
 // y[t][i] = up_i * silu(gate_i) of the prepared activations through a gate|up matrix of 2 * half rows (Q4_K / Q5_K), one launch
 bool prefill_gemm_swiglu_supported(const cai_qw_s* w, int n_tok)
 {
-  if (gemm_wide_wanted(w, w->rows, n_tok)) return w->rows % 2 == 0;
+  if (gemm_wide_wanted(&w, 1, n_tok)) return w->rows % 2 == 0;
   // only where the product takes two row tiles per wave anyway (enough work-groups to fill the chip several times over)
   return gemm_mfma_supported(w) && w->qtype != CAI_Q6_K && w->rows % 2 == 0 && (int)((w->rows + 255) / 256) * ((n_tok + 31) / 32) >= 4 * ctx().n_cu;
 }

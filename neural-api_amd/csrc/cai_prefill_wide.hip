@@ -375,17 +375,22 @@ int go_wide(const WideParams& p)
 }
 }  // namespace
 
-// Wide tiles or those of 128 rows x 32 tokens (gemm_q4k_pf), whose work-groups walk the whole width: for rows_all rows of w's type and
+// Wide tiles or those of 128 rows x 32 tokens (gemm_q4k_pf), whose work-groups walk the whole width: for n_w matrices of one type and
 // width together.  The lines, us of a call by tiles of that kernel | super-blocks of the width, Q4_K, 256 CUs, that kernel -> this one:
 //   many tiles (4 per CU on): 37888 x 3584 x 511 tokens 358 -> 300, x 2048 1540 -> 1213; 28672 x 1024 x 200 48.1 -> 46.0;
 //   long widths: 3584 x 18944 x 20 152 -> 47, x 511 253 -> 184, 4608 x 3584 x 256 47 -> 40, 3584 x 3584 x 511 54 -> 49;
 //   few tiles: 2048 x 2048 x 20 22.1 -> 17.0, x 200 24.8 -> 21.7 (the width is cut; nothing to cut below eight super-blocks, for Q5_K four);
 //   in between that kernel is the faster one: 11264 x 2048 x 200 42.1, here 43.6; 4096 x 1024 x 200 15.9 and 20.1;
 //   one token tile of it that fills the chip: 37888 x 3584 x 20 44, here 61 (a tile takes 64 tokens).
-bool gemm_wide_wanted(const cai_qw_s* w, int64_t rows_all, int n_tok)
+bool gemm_wide_wanted(const cai_qw_s* const* ws, int n_w, int n_tok)
 {
+  const cai_qw_s* w = ws[0];
+  int64_t rows_all = 0;
+  for (int i = 0; i < n_w; i++) {
+    if (!wide_offsets_fit(n_tok, ws[i]->cols, ws[i]->data_bytes)) return false;
+    rows_all += ws[i]->rows;
+  }
   if ((w->qtype != CAI_Q4_K && w->qtype != CAI_Q5_K) || w->cols % 256 || n_tok <= 16) return false;
-  if ((int64_t)n_tok * w->cols >= (int64_t)1 << 30 || w->data_bytes >= (int64_t)4000 << 20) return false;   // (32-bit byte offsets into the planes and the matrix)
   const int n_cu = ctx().n_cu, nsb = (int)(w->cols >> 8);
   const int64_t tiles = (rows_all + 127) / 128 * ((n_tok + 31) / 32);
   if (n_tok <= 32 && tiles >= n_cu) return false;
