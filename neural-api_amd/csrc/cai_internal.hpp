@@ -283,6 +283,11 @@ void kv_geometry(const cai_kv_s* kv, int rows, int* split_len, int* n_splits);
 int prefill_linear(const cai_qw_s* w, const float* x, int64_t x_stride, const float* gain, float eps, int n_tok,
                    float* y, int64_t y_stride, const float* residual);
 bool gemm_mfma_supported(const cai_qw_s* w);   // many-token (prompt) matrix-core kernel of the super-block types (Q4_K, Q6_K)
+// The kernels of the block types and of the stored streams reach activation rows and the rows of a tile through 32-bit byte offsets: widths up to
+// BLK_MAX_COLS, and token pieces of whole tiles whose plane ends below 2^32.
+constexpr int64_t BLK_MAX_COLS = (int64_t)1 << 24;
+constexpr int64_t blk_piece(int64_t cols) { return ((int64_t)1 << 31) / cols / 128 * 128; }
+static_assert(blk_piece(BLK_MAX_COLS) >= 128 && blk_piece(BLK_MAX_COLS) * BLK_MAX_COLS * 2 <= (int64_t)1 << 32 && 256 * BLK_MAX_COLS <= (int64_t)1 << 32, "a piece is at least a tile, and its offsets and those of 256 rows fit");
 bool gemm_blk_supported(const cai_qw_s* w);    // many-token (prompt) matrix-core kernel of the 32-weight block types (Q8_0, Q4_0)
 bool gemm_raw_supported(const cai_qw_s* w);    // many-token products of the types kept as their stored stream (but Q5_K)
 int launch_gemm_raw(const cai_qw_s* w, const _Float16* xhi, const _Float16* xlo, const float* sinv, int n_tok, float* y, int64_t y_stride, const float* residual);

@@ -608,8 +608,7 @@ int launch_blk(const cai_qw_s* w, const BlkGemmParams& p0, int n_tiles_grouped)
     return odd ? launch_blk<CAI_Q4_0, true>(p, n_tiles_grouped) : launch_blk<CAI_Q4_0, false>(p, n_tiles_grouped);
   };
   if (p0.tile_tab) return go(p0);
-  // the kernels reach an activation row through a 32-bit byte offset: planes of 4 GiB and more go in pieces of whole tiles
-  const int64_t most = ((int64_t)1 << 31) / p0.cols / 128 * 128;
+  const int64_t most = blk_piece(p0.cols);
   for (int64_t t = 0; t < p0.n_tok; t += most) {
     BlkGemmParams p = p0;
     p.n_tok = (int)std::min<int64_t>(most, p0.n_tok - t);
@@ -748,7 +747,7 @@ int launch_raw(const cai_qw_s* w, const BlkGemmParams& p0)
 
 }  // namespace
 
-bool gemm_blk_supported(const cai_qw_s* w) { return (w->qtype == CAI_Q8_0 || w->qtype == CAI_Q4_0) && w->cols % 32 == 0; }
+bool gemm_blk_supported(const cai_qw_s* w) { return (w->qtype == CAI_Q8_0 || w->qtype == CAI_Q4_0) && w->cols % 32 == 0 && w->cols <= BLK_MAX_COLS; }
 
 // Dense: y[t][rows] = W x[t] (+ bias) (+ residual) for the n_tok prepared activation rows.
 int launch_gemm_blk(const cai_qw_s* w, const _Float16* xhi, const _Float16* xlo, const float* sinv, int n_tok, float* y, int64_t y_stride,
@@ -782,7 +781,10 @@ int launch_gemm_blk_multi(const cai_qw_s* const* ws, const int* y_off, int n_w, 
   return launch_blk(w, p, 0);
 }
 
-bool gemm_raw_supported(const cai_qw_s* w) { return w->qtype == CAI_Q2_K || w->qtype == CAI_Q3_K || w->qtype == CAI_Q4_1 || w->qtype == CAI_Q5_0 || w->qtype == CAI_Q5_1; }
+bool gemm_raw_supported(const cai_qw_s* w)
+{
+  return (w->qtype == CAI_Q2_K || w->qtype == CAI_Q3_K || w->qtype == CAI_Q4_1 || w->qtype == CAI_Q5_0 || w->qtype == CAI_Q5_1) && w->cols <= BLK_MAX_COLS;
+}
 void raw_release()
 {
   if (g_raw.q) (void)hipFree(g_raw.q);
@@ -792,8 +794,7 @@ void raw_release()
 int launch_gemm_raw(const cai_qw_s* w, const _Float16* xhi, const _Float16* xlo, const float* sinv, int n_tok, float* y, int64_t y_stride, const float* residual)
 {
   if (!gemm_raw_supported(w)) return set_error(CAI_ERR_UNSUPPORTED, "prompt gemm: weight type %d", w->qtype);
-  // (activation rows at 32-bit byte offsets, the sums of sixteen bounded: pieces of whole tiles)
-  const int64_t most = std::max<int64_t>(32, std::min<int64_t>(4096, ((int64_t)1 << 31) / w->cols) / 32 * 32);
+  const int64_t most = std::min<int64_t>(4096, blk_piece(w->cols));     // (4096: the sums of sixteen are bounded)
   for (int64_t t = 0; t < n_tok; t += most) {
     BlkGemmParams p{};
     p.bias = w->bias; p.cols = (int)w->cols; p.x_div = 1; p.post = w->qtype == CAI_Q2_K ? 0.5f : 1.0f;
