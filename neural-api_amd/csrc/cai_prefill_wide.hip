@@ -367,7 +367,7 @@ int go_wide(const WideParams& p)
   constexpr size_t lds = 3 * BN * 256 + 3 * 256 * 32 + 2 * 256 * HB + 2 * 2 * BN * 16;
   static_assert(lds <= 160 * 1024, "LDS of a CU");
   static bool raised = false;
-  if (!raised) { if (hipFuncSetAttribute((const void*)gemm_wide_pf<QT, TT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) (void)hipGetLastError(); raised = true; }
+  if (!raised) { CAI_HIP(hipFuncSetAttribute((const void*)gemm_wide_pf<QT, TT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); raised = true; }
   const int n_cut = p.n_row_groups * p.n_tok_tiles - p.n_whole;
   hipLaunchKernelGGL((gemm_wide_pf<QT, TT>), dim3(p.n_whole + n_cut * p.n_splits), dim3(512), lds, ctx().stream, p);
   if (n_cut) hipLaunchKernelGGL(gemm_wide_sum<BN>, dim3(n_cut, (std::min(BN, p.n_tok) + 7) / 8), dim3(256), 0, ctx().stream, p);
