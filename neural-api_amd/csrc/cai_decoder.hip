@@ -325,6 +325,11 @@ static int ensure_prefill_buffers(cai_decoder_s* d, int n)
     CAI_HIP(hipMalloc((void**)&d->pm_gu, S * 2 * c.ffn * 4)); CAI_HIP(hipMalloc((void**)&d->pm_part, S * c.d_model * 4));
   }
   d->pf_cap = cap;
+  size_t raw[2] = {0, 0};                    // panels of the stored streams, sized once for the largest matrix (growing inside a prompt would wait for the stream each time)
+  for (auto& L : d->layers)
+    for (int slot : {CAI_W_Q, CAI_W_K, CAI_W_V, CAI_W_O, CAI_W_ROUTER, CAI_W_GATEUP, CAI_W_DOWN})
+      if (L.w[slot] && (c.n_experts == 0 || (slot != CAI_W_GATEUP && slot != CAI_W_DOWN))) raw_needs(L.w[slot], cap, raw);
+  const int rc = raw_reserve(raw); if (rc) return rc;
   // the activation planes of the prompt products, sized once for the widest row (a mixture-of-experts chunk prepares one row per slot)
   const int plane_rows = c.n_experts > 0 ? cap * std::max(c.top_k, 1) : cap;
   return prefill_reserve_rows(plane_rows, std::max(std::max(c.d_model, d->qw()), c.ffn));

@@ -291,6 +291,8 @@ static_assert(blk_piece(BLK_MAX_COLS) >= 128 && blk_piece(BLK_MAX_COLS) * BLK_MA
 bool gemm_blk_supported(const cai_qw_s* w);    // many-token (prompt) matrix-core kernel of the 32-weight block types (Q8_0, Q4_0)
 bool gemm_raw_supported(const cai_qw_s* w);    // many-token products of the types kept as their stored stream (but Q5_K)
 int launch_gemm_raw(const cai_qw_s* w, const _Float16* xhi, const _Float16* xlo, const float* sinv, int n_tok, float* y, int64_t y_stride, const float* residual);
+void raw_needs(const cai_qw_s* w, int n_tok, size_t (&need)[2]);   // workspace of that product; raw_reserve grows to it
+int  raw_reserve(const size_t (&need)[2]);
 void raw_release();
 inline bool prompt_gemm_supported(const cai_qw_s* w) { return gemm_mfma_supported(w) || gemm_blk_supported(w); }
 int launch_gemm_blk(const cai_qw_s* w, const _Float16* xhi, const _Float16* xlo, const float* sinv, int n_tok, float* y, int64_t y_stride, const float* residual);

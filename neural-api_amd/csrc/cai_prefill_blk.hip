@@ -698,20 +698,15 @@ struct RawWs { uint8_t* q = nullptr; float* s16 = nullptr; size_t q_cap = 0, s_c
 RawWs g_raw;
 constexpr int64_t RAW_PANEL = (int64_t)64 << 20;       // weights of a panel: its bytes stay in the last-level cache between the two launches
 
+constexpr bool raw_has_minima(int qt) { return qt == CAI_Q2_K || qt == CAI_Q4_1 || qt == CAI_Q5_1; }
+int64_t raw_panel(const cai_qw_s* w) { return std::min((w->rows + 63) / 64 * 64, std::max<int64_t>(64, RAW_PANEL / w->cols / 64 * 64)); }
+int64_t raw_piece(const cai_qw_s* w) { return std::min<int64_t>(4096, blk_piece(w->cols)); }     // (4096: the sums of sixteen are bounded)
+
 template <int QT>
 int launch_raw(const cai_qw_s* w, const BlkGemmParams& p0)
 {
-  constexpr bool MIN = QT == CAI_Q2_K || QT == CAI_Q4_1 || QT == CAI_Q5_1;
-  const int64_t K = w->cols, rows = w->rows;
-  const int64_t panel = std::min((rows + 63) / 64 * 64, std::max<int64_t>(64, RAW_PANEL / K / 64 * 64));
-  const size_t q_need = (size_t)panel * K * 21 / 16, s_need = MIN ? (size_t)p0.n_tok * K / 16 : 0;    // bytes: code 1, f16 scale 1 / 16, float minimum 4 / 16
-  if (q_need > g_raw.q_cap || s_need > g_raw.s_cap) {
-    CAI_HIP(hipStreamSynchronize(ctx().stream));
-    const size_t qc = std::max(q_need, g_raw.q_cap), sc = std::max(s_need, g_raw.s_cap);
-    raw_release();
-    if (qc) { CAI_HIP(hipMalloc((void**)&g_raw.q, qc)); g_raw.q_cap = qc; }
-    if (sc) { CAI_HIP(hipMalloc((void**)&g_raw.s16, sc * 4)); g_raw.s_cap = sc; }
-  }
+  constexpr bool MIN = raw_has_minima(QT);
+  const int64_t K = w->cols, rows = w->rows, panel = raw_panel(w);
   hipStream_t st = ctx().stream;
   if (MIN) {
     const int64_t n8 = (int64_t)p0.n_tok * K / 8;
@@ -791,10 +786,35 @@ void raw_release()
   if (g_raw.s16) (void)hipFree(g_raw.s16);
   g_raw = RawWs();
 }
+// bytes of a panel (code 1, f16 scale 1 / 16, float minimum 4 / 16 a weight) and floats of a piece's sums: the larger of what need[] holds and this
+void raw_needs(const cai_qw_s* w, int n_tok, size_t (&need)[2])
+{
+  if (!gemm_raw_supported(w)) return;
+  need[0] = std::max(need[0], (size_t)raw_panel(w) * w->cols * 21 / 16);
+  if (raw_has_minima(w->qtype)) need[1] = std::max(need[1], (size_t)std::min<int64_t>(n_tok, raw_piece(w)) * w->cols / 16);
+}
+int raw_reserve(const size_t (&need)[2])      // (prompts are not captured: the buffers may move between two of them)
+{
+  if (need[0] > g_raw.q_cap || need[1] > g_raw.s_cap) CAI_HIP(hipStreamSynchronize(ctx().stream));
+  if (need[0] > g_raw.q_cap) {
+    if (g_raw.q) (void)hipFree(g_raw.q);
+    g_raw.q = nullptr; g_raw.q_cap = 0;
+    CAI_HIP(hipMalloc((void**)&g_raw.q, need[0])); g_raw.q_cap = need[0];
+  }
+  if (need[1] > g_raw.s_cap) {
+    if (g_raw.s16) (void)hipFree(g_raw.s16);
+    g_raw.s16 = nullptr; g_raw.s_cap = 0;
+    CAI_HIP(hipMalloc((void**)&g_raw.s16, need[1] * 4)); g_raw.s_cap = need[1];
+  }
+  return CAI_OK;
+}
 int launch_gemm_raw(const cai_qw_s* w, const _Float16* xhi, const _Float16* xlo, const float* sinv, int n_tok, float* y, int64_t y_stride, const float* residual)
 {
   if (!gemm_raw_supported(w)) return set_error(CAI_ERR_UNSUPPORTED, "prompt gemm: weight type %d", w->qtype);
-  const int64_t most = std::min<int64_t>(4096, blk_piece(w->cols));     // (4096: the sums of sixteen are bounded)
+  size_t need[2] = {0, 0};
+  raw_needs(w, n_tok, need);
+  const int rc0 = raw_reserve(need); if (rc0) return rc0;
+  const int64_t most = raw_piece(w);
   for (int64_t t = 0; t < n_tok; t += most) {
     BlkGemmParams p{};
     p.bias = w->bias; p.cols = (int)w->cols; p.x_div = 1; p.post = w->qtype == CAI_Q2_K ? 0.5f : 1.0f;

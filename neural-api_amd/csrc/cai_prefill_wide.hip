@@ -344,20 +344,15 @@ __global__ __launch_bounds__(256) void gemm_wide_sum(const WideParams p)
   }
 }
 
-// partial sums of products whose width is cut over work-groups: grown on demand, given back with the other prompt buffers.  All prompt
-// work runs on the one stream of the library under its lock, so one buffer serves every decoder.
+// partial sums of products whose width is cut over work-groups: allocated once for any product (no more than one slice of a tile per CU), given
+// back with the other prompt buffers.  All prompt work runs on the one stream of the library under its lock, so one buffer serves every decoder.
 static float* g_wide_part = nullptr;
-static size_t g_wide_cap = 0;
-static int wide_reserve(size_t floats)
+static int wide_reserve()
 {
-  if (floats <= g_wide_cap) return CAI_OK;
-  CAI_HIP(hipStreamSynchronize(ctx().stream));
-  if (g_wide_part) { (void)hipFree(g_wide_part); g_wide_part = nullptr; g_wide_cap = 0; }
-  CAI_HIP(hipMalloc((void**)&g_wide_part, floats * 4));
-  g_wide_cap = floats;
+  if (!g_wide_part) CAI_HIP(hipMalloc((void**)&g_wide_part, (size_t)ctx().n_cu * 256 * 128 * sizeof(float)));
   return CAI_OK;
 }
-void wide_release() { if (g_wide_part) (void)hipFree(g_wide_part); g_wide_part = nullptr; g_wide_cap = 0; }
+void wide_release() { if (g_wide_part) (void)hipFree(g_wide_part); g_wide_part = nullptr; }
 
 namespace {
 template <int QT, int TT>
@@ -426,7 +421,8 @@ int launch_gemm_wide(const cai_qw_s* const* ws, const int* y_off, int n_w, const
   }
   const int n_cut = p.n_row_groups * p.n_tok_tiles - p.n_whole;
   if (n_cut) {
-    const int rc = wide_reserve((size_t)n_cut * p.n_splits * BM * BN); if (rc) return rc;
+    if (n_cut * p.n_splits > slots) return set_error(CAI_ERR_INVALID, "prompt gemm: %d tiles cut into %d slices for %d work-groups", n_cut, p.n_splits, slots);
+    const int rc = wide_reserve(); if (rc) return rc;
     p.part = g_wide_part;
   }
   const bool q5 = ws[0]->qtype == CAI_Q5_K;
