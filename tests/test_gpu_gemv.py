@@ -483,6 +483,41 @@ def test_prompt_of_a_mixture_on_tiles_of_64_slots(qt, ffn, T):
     dec.close()
 
 
+@pytest.mark.parametrize("qt", [O.Q8_0, O.Q4_0])
+@pytest.mark.parametrize("rows,cols,T", [(39937, 544, 128), (39937, 576, 100)])
+def test_large_block_tiles_of_many_chunks(qt, rows, cols, T):
+    """tiles of 256 rows x 128 tokens nine chunks of 64 columns deep, whose ring of three is filled three times; an odd and an even number of blocks"""
+    from helpers.device import dev, rel_err
+    cai = dev()
+    rng = np.random.default_rng(cols + qt)
+    base = O.quantize(qt, (rng.standard_normal((700, cols)) * 0.02).astype(np.float32)).reshape(700, -1)
+    raw = np.ascontiguousarray(base[np.arange(rows) % 700])
+    x = rng.standard_normal((T, cols)).astype(np.float32)
+    w = cai.QWeight(qt, rows, cols, raw.reshape(-1))
+    got = w.gemm(x)
+    want = x.astype(np.float64) @ O.dequant(qt, base.reshape(-1), 700 * cols).reshape(700, cols).astype(np.float64).T
+    assert rel_err(got, want[:, np.arange(rows) % 700]) < TIGHT
+    w.close()
+
+
+@pytest.mark.parametrize("experts,T", [(130, 40), (500, 70)])
+def test_prompt_of_a_mixture_of_more_experts_than_a_wave(experts, T):
+    """slots grouped by expert where the sums over the experts before one run over several waves: a prompt equals its tokens one by one"""
+    from helpers.device import dev, rel_err
+    from helpers.model_build import synthetic_spec
+    cai = dev()
+    cfg = dict(n_layers=2, d_model=128, n_q_heads=4, n_kv_heads=2, head_dim=32, ffn=64, vocab=300, max_ctx=128, eps=1e-5, rope_theta=1e4,
+               n_experts=experts, top_k=2, norm_topk=1)
+    spec = synthetic_spec(cfg, O.Q8_0, head_qtype=O.Q8_0, seed=T, std=0.05, qkv_bias=False)
+    dec = cai.Decoder(spec, max_batch=2)
+    tok = np.random.default_rng(3).integers(0, 300, T).astype(np.int32)
+    _, got = dec.prefill(tok)
+    for p_, t in enumerate(tok):
+        _, want = dec.step_window([t], p_, seq=1)
+    assert rel_err(got, want[0]) < 1e-4
+    dec.close()
+
+
 @pytest.mark.parametrize("cols", [32, 1024, 1056, 2048, 2080, 4096, 4128, 8192, 8224, 24576, 24608])
 def test_prompt_rows_at_the_widths_of_the_pre_pass(cols):
     """the last and the first width of each number of values a thread keeps, and rows that start one float off alignment"""
