@@ -203,9 +203,6 @@ struct GemmParams {
   // matrix i + 1, whose rows land y_off2[i] columns into a y row (gemm_q4k_pf only)
   int n_seg; int seg_end[2];
   const uint8_t* w2[2]; const float* bias2[2]; int rows2[2]; int y_off2[2];
-  // fused feed-forward front half (gemm_q4k_pf with two row tiles per wave): rows [0, half) are up, [half, 2 half) gate; a wave's
-  // two tiles are 32 up rows and THEIR gate rows, and y[t][i] = up_i * silu(gate_i) is written (y rows are half wide)
-  int swiglu_half;
 };
 
 constexpr int PF_LDX = 264;       // halfs per staged token row: 256 + pad (stride = 4 banks mod 64: 16-byte reads)
@@ -224,23 +221,23 @@ typedef _Float16 half8_pf __attribute__((ext_vector_type(8)));
 // One work-group: 4 waves x RT row tiles of 32 rows x 32 tokens, one super-block (256 columns) per step, on
 // v_mfma_f32_32x32x16_f16 (lane (n, kg) supplies 8 consecutive k of row / column n).
 //   * the weight operand sc_j * q (<= 63 * 15, exact in f16) is built once per super-block per wave and reused by the
-//     token tiles and by the hi and lo activation planes; the matrix cores accumulate across the whole super-block, hi
-//     and lo planes into the same accumulator (the chains of the tiles interleave);
+//     hi and lo activation planes; the matrix cores accumulate across the whole super-block, hi and lo planes into the
+//     same accumulator;
 //   * -dmin * mn_j * sum_{k in j} x_k is one more MFMA step per plane (k = the 8 sub-blocks);
 //   * d and dmin are applied once per super-block (2 FMAs per value), the token scale once at the end.
 // Every MFMA takes its activation operand from LDS (1 KB per wave and instruction): with one row tile per wave the LDS
 // pipe, not the matrix cores, sets the pace.  RT = 2 lets one activation operand serve two row tiles (half the LDS reads
 // per FLOP); it needs 256 rows per work-group and is used for matrices with enough row groups to fill the chip.
 // Work-group ids are laid out so that the token tiles of one row group run on one XCD: the re-reads of its weights (one
-// per token tile) hit that XCD's L2.  TT = 1 doubles the number of work-groups for matrices with few row groups.
+// per token tile) hit that XCD's L2.
 // QT = CAI_Q5_K: 176-byte super-blocks (neural/neuralgguf.pas:516-587) - the Q4_K header, the 32-byte plane of fifth bits (bit j of byte i
 // belongs to weight i of sub-block j), the nibbles; the weight operand sc * (nibble | bit << 4) <= 63 * 31 stays exact in f16.
 template <int RT, int QT>
 __global__ __launch_bounds__(256, 2) void gemm_q4k_pf(const GemmParams p)
 {
-  constexpr int TT = 1, BB = QT == CAI_Q5_K ? 176 : 144, QOFF = QT == CAI_Q5_K ? 48 : 16;
+  constexpr int BB = QT == CAI_Q5_K ? 176 : 144, QOFF = QT == CAI_Q5_K ? 48 : 16;
   extern __shared__ __align__(16) unsigned char pf_smem[];
-  constexpr int NTOK = TT * 32;
+  constexpr int NTOK = 32;
   _Float16* xs_hi = reinterpret_cast<_Float16*>(pf_smem);            // [NTOK][PF_LDX]
   _Float16* xs_lo = xs_hi + NTOK * PF_LDX;
   _Float16* sx_hi = xs_lo + NTOK * PF_LDX;                            // [NTOK][8]
@@ -254,16 +251,12 @@ __global__ __launch_bounds__(256, 2) void gemm_q4k_pf(const GemmParams p)
   const uint8_t* wbase = p.w; const float* bias = p.bias; int rows = p.rows, yo = 0, rgl = rg;   // this work-group's matrix (uniform)
   if (p.n_seg > 1 && rg >= p.seg_end[0]) { wbase = p.w2[0]; bias = p.bias2[0]; rows = p.rows2[0]; yo = p.y_off2[0]; rgl = rg - p.seg_end[0]; }
   if (p.n_seg > 2 && rg >= p.seg_end[1]) { wbase = p.w2[1]; bias = p.bias2[1]; rows = p.rows2[1]; yo = p.y_off2[1]; rgl = rg - p.seg_end[1]; }
-  const int half = RT == 2 ? p.swiglu_half : 0;
-  const int R0 = half ? (rgl * 4 + wave) * 32 : (rgl * 4 + wave) * 32 * RT, T0 = ttile * NTOK;
+  const int R0 = (rgl * 4 + wave) * 32 * RT, T0 = ttile * NTOK;
   const int K = p.cols, nsb = K >> 8, nb32 = K >> 5;
   const int64_t row_bytes = (int64_t)nsb * BB;
   const uint8_t* wrow[RT];
 #pragma unroll
-  for (int rt = 0; rt < RT; rt++) {     // tail rows: re-read the last row, not written
-    const int row = half ? min(R0 + n, half - 1) + rt * half : min(R0 + 32 * rt + n, rows - 1);
-    wrow[rt] = wbase + (int64_t)row * row_bytes;
-  }
+  for (int rt = 0; rt < RT; rt++) wrow[rt] = wbase + (int64_t)min(R0 + 32 * rt + n, rows - 1) * row_bytes;     // tail rows: re-read the last row, not written
 
   struct WRegs { uint4 h, q[4], e[QT == CAI_Q5_K ? 2 : 1]; };   // e: Q5_K's bit plane (all 32 bytes: the lane needs four bits of each)
   auto load_w = [&](int sb, WRegs (&r)[RT]) {
@@ -278,13 +271,11 @@ __global__ __launch_bounds__(256, 2) void gemm_q4k_pf(const GemmParams p)
       }
     }
   };
-  float16_t Y[RT][TT];
+  float16_t Y[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; rt++)
 #pragma unroll
-    for (int tt = 0; tt < TT; tt++)
-#pragma unroll
-      for (int v = 0; v < 16; v++) Y[rt][tt][v] = 0.0f;
+    for (int v = 0; v < 16; v++) Y[rt][v] = 0.0f;
 
   WRegs wcur[RT], wnxt[RT];
   load_w(0, wcur);
@@ -296,7 +287,7 @@ __global__ __launch_bounds__(256, 2) void gemm_q4k_pf(const GemmParams p)
       // the end repeat the last token (their results are never written), so the loads carry no branch and issue together.
       const int tq = threadIdx.x >> 5, chunk = threadIdx.x & 31;
       const uint32_t colo = (uint32_t)(sb * 256 + chunk * 8);
-      constexpr int SB = (TT == 2 || RT == 2) ? 1 : 4;     // loads in flight per plane (measured: with two tiles the registers are worth more than the overlap)
+      constexpr int SB = RT == 2 ? 1 : 4;     // loads in flight per plane (measured: with two row tiles the registers are worth more than the overlap)
 #pragma unroll
       for (int i0 = 0; i0 < NTOK / 8; i0 += SB) {
         uint4 vh[SB], vl[SB];
@@ -363,47 +354,42 @@ __global__ __launch_bounds__(256, 2) void gemm_q4k_pf(const GemmParams p)
         }
       }
     }
-    float16_t C[RT][TT], Cm[RT][TT];
+    float16_t C[RT], Cm[RT];
     const float16_t zero16 = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int j = 0; j < 4; j++)
 #pragma unroll
-      for (int t = 0; t < 4; t++)
+      for (int t = 0; t < 4; t++) {
+        const int off = n * PF_LDX + 128 * kg + 32 * j + 8 * t;
+        const half8_pf Bh = *reinterpret_cast<const half8_pf*>(xs_hi + off);
+        const half8_pf Bl = *reinterpret_cast<const half8_pf*>(xs_lo + off);
 #pragma unroll
-        for (int tt = 0; tt < TT; tt++) {
-          const int off = (tt * 32 + n) * PF_LDX + 128 * kg + 32 * j + 8 * t;
-          const half8_pf Bh = *reinterpret_cast<const half8_pf*>(xs_hi + off);
-          const half8_pf Bl = *reinterpret_cast<const half8_pf*>(xs_lo + off);
-#pragma unroll
-          for (int rt = 0; rt < RT; rt++) {
-            if (j == 0 && t == 0) C[rt][tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[rt][j][t], Bh, zero16, 0, 0, 0);   // a fresh accumulator per super-block
-            else C[rt][tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[rt][j][t], Bh, C[rt][tt], 0, 0, 0);
-          }
-#pragma unroll
-          for (int rt = 0; rt < RT; rt++) C[rt][tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[rt][j][t], Bl, C[rt][tt], 0, 0, 0);
+        for (int rt = 0; rt < RT; rt++) {
+          if (j == 0 && t == 0) C[rt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[rt][j][t], Bh, zero16, 0, 0, 0);   // a fresh accumulator per super-block
+          else C[rt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[rt][j][t], Bh, C[rt], 0, 0, 0);
         }
-    __builtin_amdgcn_wave_barrier();       // s_d was written by this wave's own lanes above; LDS operations of a wave complete in order
 #pragma unroll
-    for (int tt = 0; tt < TT; tt++) {
-      const half4_t Bmh = *reinterpret_cast<const half4_t*>(sx_hi + (tt * 32 + n) * 8 + 4 * kg);
-      const half4_t Bml = *reinterpret_cast<const half4_t*>(sx_lo + (tt * 32 + n) * 8 + 4 * kg);
-#pragma unroll
-      for (int rt = 0; rt < RT; rt++) {
-        Cm[rt][tt] = __builtin_amdgcn_mfma_f32_32x32x8f16(mnv[rt], Bmh, zero16, 0, 0, 0);
-        Cm[rt][tt] = __builtin_amdgcn_mfma_f32_32x32x8f16(mnv[rt], Bml, Cm[rt][tt], 0, 0, 0);
+        for (int rt = 0; rt < RT; rt++) C[rt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[rt][j][t], Bl, C[rt], 0, 0, 0);
       }
+    __builtin_amdgcn_wave_barrier();       // s_d was written by this wave's own lanes above; LDS operations of a wave complete in order
+    const half4_t Bmh = *reinterpret_cast<const half4_t*>(sx_hi + n * 8 + 4 * kg);
+    const half4_t Bml = *reinterpret_cast<const half4_t*>(sx_lo + n * 8 + 4 * kg);
 #pragma unroll
-      for (int rt = 0; rt < RT; rt++)
-#pragma unroll
-        for (int g = 0; g < 4; g++) {
-          const float4 d4 = *reinterpret_cast<const float4*>(&s_d[((wave * RT + rt) * 2 + 0) * 32 + 8 * g + 4 * kg]);
-          const float4 m4 = *reinterpret_cast<const float4*>(&s_d[((wave * RT + rt) * 2 + 1) * 32 + 8 * g + 4 * kg]);
-          Y[rt][tt][4 * g + 0] += d4.x * C[rt][tt][4 * g + 0] - m4.x * Cm[rt][tt][4 * g + 0];
-          Y[rt][tt][4 * g + 1] += d4.y * C[rt][tt][4 * g + 1] - m4.y * Cm[rt][tt][4 * g + 1];
-          Y[rt][tt][4 * g + 2] += d4.z * C[rt][tt][4 * g + 2] - m4.z * Cm[rt][tt][4 * g + 2];
-          Y[rt][tt][4 * g + 3] += d4.w * C[rt][tt][4 * g + 3] - m4.w * Cm[rt][tt][4 * g + 3];
-        }
+    for (int rt = 0; rt < RT; rt++) {
+      Cm[rt] = __builtin_amdgcn_mfma_f32_32x32x8f16(mnv[rt], Bmh, zero16, 0, 0, 0);
+      Cm[rt] = __builtin_amdgcn_mfma_f32_32x32x8f16(mnv[rt], Bml, Cm[rt], 0, 0, 0);
     }
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        const float4 d4 = *reinterpret_cast<const float4*>(&s_d[((wave * RT + rt) * 2 + 0) * 32 + 8 * g + 4 * kg]);
+        const float4 m4 = *reinterpret_cast<const float4*>(&s_d[((wave * RT + rt) * 2 + 1) * 32 + 8 * g + 4 * kg]);
+        Y[rt][4 * g + 0] += d4.x * C[rt][4 * g + 0] - m4.x * Cm[rt][4 * g + 0];
+        Y[rt][4 * g + 1] += d4.y * C[rt][4 * g + 1] - m4.y * Cm[rt][4 * g + 1];
+        Y[rt][4 * g + 2] += d4.z * C[rt][4 * g + 2] - m4.z * Cm[rt][4 * g + 2];
+        Y[rt][4 * g + 3] += d4.w * C[rt][4 * g + 3] - m4.w * Cm[rt][4 * g + 3];
+      }
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int rt = 0; rt < RT; rt++) wcur[rt] = wnxt[rt];
@@ -413,60 +399,31 @@ __global__ __launch_bounds__(256, 2) void gemm_q4k_pf(const GemmParams p)
   // row go out as one 16-byte store (bias and residual come in the same way) when the addresses allow it ----
   const bool vec = ((p.y_stride | yo) & 3) == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0 &&
                    (!p.residual || (reinterpret_cast<uintptr_t>(p.residual) & 15) == 0) && (!bias || (reinterpret_cast<uintptr_t>(bias) & 15) == 0);
-  if constexpr (RT == 2) if (half) {
+  const int t = T0 + n;
+  if (t >= p.n_tok) return;
+  const float si = p.sinv[t];
 #pragma unroll
-    for (int tt = 0; tt < TT; tt++) {
-      const int t = T0 + tt * 32 + n;
-      if (t >= p.n_tok) continue;
-      const float si = p.sinv[t];
+  for (int rt = 0; rt < RT; rt++)
 #pragma unroll
-      for (int g = 0; g < 4; g++) {
-        const int row = R0 + 8 * g + 4 * kg;
-        const int64_t o = (int64_t)t * p.y_stride + row;
-        float r[4];
+    for (int g = 0; g < 4; g++) {
+      const int row = R0 + 32 * rt + 8 * g + 4 * kg;
+      const int64_t o = (int64_t)t * p.y_stride + yo + row;
+      if (vec && row + 3 < rows) {
+        float4 r = make_float4(Y[rt][4 * g] * si, Y[rt][4 * g + 1] * si, Y[rt][4 * g + 2] * si, Y[rt][4 * g + 3] * si);
+        if (bias) { const float4 b = *reinterpret_cast<const float4*>(bias + row); r.x += b.x; r.y += b.y; r.z += b.z; r.w += b.w; }
+        if (p.residual) { const float4 q = *reinterpret_cast<const float4*>(p.residual + o); r.x += q.x; r.y += q.y; r.z += q.z; r.w += q.w; }
+        *reinterpret_cast<float4*>(p.y + o) = r;
+      } else {
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          float up = Y[0][tt][4 * g + i] * si, gate = Y[1][tt][4 * g + i] * si;
-          if (bias && row + i < half) { up += bias[row + i]; gate += bias[half + row + i]; }
-          r[i] = silu_mul(up, gate);
-        }
-        if (vec && row + 3 < half) *reinterpret_cast<float4*>(p.y + o) = make_float4(r[0], r[1], r[2], r[3]);
-        else {
-#pragma unroll
-          for (int i = 0; i < 4; i++) if (row + i < half) p.y[o + i] = r[i];
+          if (row + i >= rows) continue;
+          float r = Y[rt][4 * g + i] * si;
+          if (bias) r += bias[row + i];
+          if (p.residual) r += p.residual[o + i];
+          p.y[o + i] = r;
         }
       }
     }
-    return;
-  }
-#pragma unroll
-  for (int tt = 0; tt < TT; tt++) {
-    const int t = T0 + tt * 32 + n;
-    if (t >= p.n_tok) continue;
-    const float si = p.sinv[t];
-#pragma unroll
-    for (int rt = 0; rt < RT; rt++)
-#pragma unroll
-      for (int g = 0; g < 4; g++) {
-        const int row = R0 + 32 * rt + 8 * g + 4 * kg;
-        const int64_t o = (int64_t)t * p.y_stride + yo + row;
-        if (vec && row + 3 < rows) {
-          float4 r = make_float4(Y[rt][tt][4 * g] * si, Y[rt][tt][4 * g + 1] * si, Y[rt][tt][4 * g + 2] * si, Y[rt][tt][4 * g + 3] * si);
-          if (bias) { const float4 b = *reinterpret_cast<const float4*>(bias + row); r.x += b.x; r.y += b.y; r.z += b.z; r.w += b.w; }
-          if (p.residual) { const float4 q = *reinterpret_cast<const float4*>(p.residual + o); r.x += q.x; r.y += q.y; r.z += q.z; r.w += q.w; }
-          *reinterpret_cast<float4*>(p.y + o) = r;
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; i++) {
-            if (row + i >= rows) continue;
-            float r = Y[rt][tt][4 * g + i] * si;
-            if (bias) r += bias[row + i];
-            if (p.residual) r += p.residual[o + i];
-            p.y[o + i] = r;
-          }
-        }
-      }
-  }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -654,7 +611,9 @@ int launch_gemm_q4k_multi(const cai_qw_s* const* ws, const int* y_off, int n_w, 
   if (n_w > 1 && (!gemm_q4k_multi_supported(ws, n_w) || residual)) return set_error(CAI_ERR_UNSUPPORTED, "prefill gemm: %d matrices in one launch", n_w);
   if (swiglu_half && (n_w != 1 || residual || w->qtype == CAI_Q6_K || w->rows != 2 * (int64_t)swiglu_half))
     return set_error(CAI_ERR_UNSUPPORTED, "prefill gemm: fused SwiGLU needs one Q4_K / Q5_K matrix of 2 x %d rows", swiglu_half);
-  if (gemm_wide_wanted(ws, n_w, n_tok)) return launch_gemm_wide(ws, y_off, n_w, xhi, xlo, sxhi, sxlo, sinv, n_tok, y, y_stride, residual, swiglu_half);
+  const bool wide = gemm_wide_wanted(ws, n_w, n_tok);
+  if (swiglu_half && !wide) return set_error(CAI_ERR_UNSUPPORTED, "prefill gemm: fused SwiGLU of %d tokens", n_tok);
+  if (wide) return launch_gemm_wide(ws, y_off, n_w, xhi, xlo, sxhi, sxlo, sinv, n_tok, y, y_stride, residual, swiglu_half);
   int64_t rows_all = 0;
   for (int i = 0; i < n_w; i++) rows_all += ws[i]->rows;
   GemmParams p{};
@@ -683,14 +642,12 @@ int launch_gemm_q4k_multi(const cai_qw_s* const* ws, const int* y_off, int n_w, 
   // work-groups lose to 640 of one tile, 3584 rows = 224 likewise)
   const int n_cu = ctx().n_cu;
   const int wgs_rt2 = (int)((rows_all + 255) / 256) * ((n_tok + 31) / 32);
-  const int rt = (swiglu_half || 4 * wgs_rt2 >= 7 * n_cu) ? 2 : 1;
-  p.swiglu_half = swiglu_half;
+  const int rt = 4 * wgs_rt2 >= 7 * n_cu ? 2 : 1;
   p.n_row_groups = 0;
   for (int i = 0; i < n_w; i++) {       // every matrix starts a row group of its own
     if (i > 0) { p.seg_end[i - 1] = p.n_row_groups; p.w2[i - 1] = ws[i]->data; p.bias2[i - 1] = ws[i]->bias; p.rows2[i - 1] = (int)ws[i]->rows; p.y_off2[i - 1] = y_off[i] - y_off[0]; }
     p.n_row_groups += (int)((ws[i]->rows + 128 * rt - 1) / (128 * rt));
   }
-  if (swiglu_half) p.n_row_groups = (swiglu_half + 127) / 128;   // 128 up rows and their gate rows per work-group
   p.n_tok_tiles = (n_tok + 31) / 32;
   const size_t lds = (size_t)32 * (PF_LDX + 8) * 2 * 2 + (size_t)4 * rt * 2 * 32 * 4;
   static bool attr_done = false;
@@ -775,13 +732,8 @@ int prefill_gemm_multi(const cai_qw_s* const* ws, const int* y_off, int n_w, int
   }
   return CAI_OK;
 }
-// y[t][i] = up_i * silu(gate_i) of the prepared activations through a gate|up matrix of 2 * half rows (Q4_K / Q5_K), one launch
-bool prefill_gemm_swiglu_supported(const cai_qw_s* w, int n_tok)
-{
-  if (gemm_wide_wanted(&w, 1, n_tok)) return w->rows % 2 == 0;
-  // only where the product takes two row tiles per wave anyway (enough work-groups to fill the chip several times over)
-  return gemm_mfma_supported(w) && w->qtype != CAI_Q6_K && w->rows % 2 == 0 && (int)((w->rows + 255) / 256) * ((n_tok + 31) / 32) >= 4 * ctx().n_cu;
-}
+// y[t][i] = up_i * silu(gate_i) of the prepared activations through a gate|up matrix of 2 * half rows (Q4_K / Q5_K), one launch: on wide tiles
+bool prefill_gemm_swiglu_supported(const cai_qw_s* w, int n_tok) { return w->rows % 2 == 0 && gemm_wide_wanted(&w, 1, n_tok); }
 int prefill_gemm_swiglu(const cai_qw_s* w, int n_tok, float* y, int64_t y_stride)
 {
   const int zero = 0;
