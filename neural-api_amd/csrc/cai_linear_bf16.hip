@@ -9,6 +9,7 @@
 // streaming kernel takes float rows (the stream's) through an RMS norm itself, and runs two products in one launch.  The matrix-core kernel also runs over a
 // bank of equal matrices with a list of activation rows for each (mixtures of experts).
 #include "cai_lin_epilogue.hpp"
+#include "cai_async_copy.hpp"
 
 #include <algorithm>
 
@@ -198,22 +199,6 @@ __global__ __launch_bounds__(64 * GV_WAVES) void gemv_bf16(const uint16_t* __res
 // Bound by the matrix cores and the fragment reads of a step together: sixteen waves of 64 x 32 overlap them better than four of
 // 64 x 64 (whole prompt of 2048 tokens through four layers of width 2048: 2798 us with four waves and staging through registers -> 2546).
 // ------------------------------------------------------------------------------------------
-// 64 lanes x 16 bytes, each from an address of its own, into 1 KB of LDS at lds (uniform), in lane order.  The compiler does not see
-// the load: the caller waits for it before the barrier that publishes the tile.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"     // (m0 is reserved, and named all the same: the statement changes it)
-__device__ __forceinline__ void copy_to_lds(uint32_t lds, const void* from)
-{
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" :: "s"(lds), "v"(from) : "memory", "m0");
-}
-#pragma clang diagnostic pop
-template <int N> __device__ __forceinline__ void wait_copies()
-{
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
-  asm volatile("" ::: "memory");
-}
-
 template <typename AT, int BM, int BN, int WM, int WN, bool BANK, int MODE, int DEPTH = 2>   // MODE: e.mode (one epilogue a kernel: with all of them the accumulators would leave their registers)
 __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16(const uint16_t* __restrict__ W, const AT* __restrict__ X, int n_rows, int ldw, int64_t ldx, int n_tok, int tiles_m, int n_tiles, LinEpi e, BankList l)
 {
@@ -290,9 +275,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16(const uint16_t* __rest
     auto copy = [&](int kt) {
       const uint32_t dst = lds0 + (uint32_t)(kt % DEPTH * SLOT * 16 + wave * 1024);
 #pragma unroll
-      for (int i = 0; i < CA; i++) copy_to_lds(dst + i * NT * 16, xp[i] + kt * BK);
+      for (int i = 0; i < CA; i++) copy16_to_lds(dst + i * NT * 16, xp[i] + kt * BK);
 #pragma unroll
-      for (int i = 0; i < CW; i++) copy_to_lds(dst + BM * 128 + i * NT * 16, wp[i] + kt * BK);
+      for (int i = 0; i < CW; i++) copy16_to_lds(dst + BM * 128 + i * NT * 16, wp[i] + kt * BK);
     };
 #pragma unroll
     for (int i = 0; i < DEPTH - 1; i++) if (i < nk) copy(i);

@@ -20,6 +20,7 @@
 #include "cai_internal.hpp"
 #include "cai_gemv_common.hpp"
 #include "cai_blocks_raw.hpp"
+#include "cai_async_copy.hpp"
 #include <algorithm>
 #include <type_traits>
 
@@ -68,24 +69,6 @@ __device__ __forceinline__ half8_b codes8(uint32_t w0, uint32_t w1, int high)
   return half8_b{h0.x, h0.y, h1.x, h1.y, h2.x, h2.y, h3.x, h3.y};
 }
 
-// 64 lanes x 16 bytes from base + voff into 1 KB of LDS at lds (uniform), in lane order.  The compiler does not see the load: the
-// caller waits for it before the barrier that publishes the tile, and before the kernel's LDS could go to another work-group.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"     // (m0 is reserved, and named all the same: the statement changes it)
-__device__ __forceinline__ void copy_chunk(uint32_t lds, uint32_t voff, const void* base)
-{
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
-}
-__device__ __forceinline__ void copy_dword(uint32_t lds, uint32_t voff, const void* base)     // 64 lanes x 4 bytes
-{
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" :: "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
-}
-__device__ __forceinline__ void copy_short(uint32_t lds, uint32_t voff, const void* base)     // 64 lanes x 2 bytes, a dword each in LDS
-{
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_ushort %1, %2" :: "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
 }  // namespace
 
 // ------------------------------------------------------------------------------------------
@@ -101,12 +84,6 @@ __device__ __forceinline__ void copy_short(uint32_t lds, uint32_t voff, const vo
 // Gate | up and down of 64 experts (2048 x 2048, 2048 x 1024), 2040 slots: 199 us a layer -> 149 (82 to read the banks once): with tiles
 // of 64 slots instead of 32 an expert's rows come from memory once.  Two work-groups a CU (two slots of LDS each) take the same time.
 // ------------------------------------------------------------------------------------------
-template <int N> __device__ __forceinline__ void wait_loads()
-{
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
-  asm volatile("" ::: "memory");
-}
 template <int QT, int TT, bool ODD>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_blk_tile(const BlkGemmParams p)
 {
@@ -176,15 +153,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
       for (int i = 0; i < XC; i++) {
         const uint32_t o = xo[i] - (half && (xcut >> i & 1) ? 64u : 0u);
-        copy_chunk(dst + 1024 * (8 * i + wave), o, xh);
-        copy_chunk(dst + PLANE + 1024 * (8 * i + wave), o, xl);
+        copy16_to_lds(dst + 1024 * (8 * i + wave), o, xh);
+        copy16_to_lds(dst + PLANE + 1024 * (8 * i + wave), o, xl);
       }
 #pragma unroll
-    for (int i = 0; i < WC; i++) copy_chunk(dst + XB + 1024 * (8 * i + wave), wo[i] - (half && (wcut >> i & 1) ? WROW / 2u : 0u), qb + (int64_t)c * WROW);
+    for (int i = 0; i < WC; i++) copy16_to_lds(dst + XB + 1024 * (8 * i + wave), wo[i] - (half && (wcut >> i & 1) ? WROW / 2u : 0u), qb + (int64_t)c * WROW);
     if constexpr (ODD) {
-      copy_short(dst + XB + WB + 256 * (wave & 3), dof, db + (int64_t)c * 4);
-      copy_short(dst + XB + WB + 1024 + 256 * (wave & 3), dof, db + (int64_t)c * 4 + (half ? 0 : 2));
-    } else copy_dword(dst + XB + WB + 256 * (wave & 3), dof, db + (int64_t)c * 4);
+      copy2_to_lds(dst + XB + WB + 256 * (wave & 3), dof, db + (int64_t)c * 4);
+      copy2_to_lds(dst + XB + WB + 1024 + 256 * (wave & 3), dof, db + (int64_t)c * 4 + (half ? 0 : 2));
+    } else copy4_to_lds(dst + XB + WB + 256 * (wave & 3), dof, db + (int64_t)c * 4);
   };
 
   const float16_b zero16 = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
@@ -253,8 +230,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     int slot = 0;
     for (int c = 0; c < n_chunks; c++) {
       const int left = n_chunks - 1 - c;               // chunks behind this one
-      if (left >= DEPTH - 2) { if (x_on) wait_loads<(DEPTH - 2) * COPIES>(); else wait_loads<(DEPTH - 2) * (COPIES - 2 * XC)>(); }
-      else wait_loads<0>();
+      if (left >= DEPTH - 2) { if (x_on) wait_copies<(DEPTH - 2) * COPIES>(); else wait_copies<(DEPTH - 2) * (COPIES - 2 * XC)>(); }
+      else wait_copies<0>();
       __builtin_amdgcn_s_waitcnt(0xC07F);              // lgkmcnt(0): this wave's reads of the slot that is filled next (and the row tables, the first time)
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
@@ -360,21 +337,21 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       const uint32_t o = xo[i] - (half && (xcut >> i & 1) ? 64u : 0u);
-      copy_chunk(dst + 1024 * i, o, xh); copy_chunk(dst + 4096 + 1024 * i, o, xl);
+      copy16_to_lds(dst + 1024 * i, o, xh); copy16_to_lds(dst + 4096 + 1024 * i, o, xl);
     }
 #pragma unroll
-    for (int i = 0; i < RT * WB / 1024; i++) copy_chunk(dst + XB + 1024 * i, wo[i] - (half && (wcut >> i & 1) ? WROW / 2u : 0u), qb + (int64_t)c * WROW);
+    for (int i = 0; i < RT * WB / 1024; i++) copy16_to_lds(dst + XB + 1024 * i, wo[i] - (half && (wcut >> i & 1) ? WROW / 2u : 0u), qb + (int64_t)c * WROW);
     if constexpr (ODD) {
-      copy_short(dst + XB + RT * WB, dof, db + (int64_t)c * 4);
-      copy_short(dst + XB + RT * WB + 256, dof, db + (int64_t)c * 4 + (half ? 0 : 2));
-    } else copy_dword(dst + XB + RT * WB, dof, db + (int64_t)c * 4);
+      copy2_to_lds(dst + XB + RT * WB, dof, db + (int64_t)c * 4);
+      copy2_to_lds(dst + XB + RT * WB + 256, dof, db + (int64_t)c * 4 + (half ? 0 : 2));
+    } else copy4_to_lds(dst + XB + RT * WB, dof, db + (int64_t)c * 4);
     if constexpr (MIN) {                   // [sixteen of the chunk][token or row]; past the width (the last chunk of ODD) the ones before again
 #pragma unroll
-      for (int i = 0; i < 2; i++) copy_dword(dst + MB + 256 * i, sof + (uint32_t)(8 * i), reinterpret_cast<const char*>(p.s16) + (int64_t)c * 16 - (half && i ? 8 : 0));
+      for (int i = 0; i < 2; i++) copy4_to_lds(dst + MB + 256 * i, sof + (uint32_t)(8 * i), reinterpret_cast<const char*>(p.s16) + (int64_t)c * 16 - (half && i ? 8 : 0));
 #pragma unroll
       for (int i = 0; i < 4; i++)
         if (RT == 2 || (i & 1) == 0)
-          copy_dword(dst + MB + 512 + 256 * (RT == 2 ? i : i >> 1), mof + (uint32_t)(4 * i), mb + (int64_t)c * 16 - (half && i >= 2 ? 8 : 0));
+          copy4_to_lds(dst + MB + 512 + 256 * (RT == 2 ? i : i >> 1), mof + (uint32_t)(4 * i), mb + (int64_t)c * 16 - (half && i >= 2 ? 8 : 0));
     }
   };
   float16_b Y[RT], Z[RT], U[RT];           // sums of eight (RT = 2: sixteen) blocks, sums of those: see the comment above; FINE: the small parts
@@ -455,8 +432,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
     if (c + 1 < c1) {
       __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the last reads of the other slot
       copy(c + 1, slot ^ 1);
-      wait_loads<COPIES>();
-    } else wait_loads<0>();
+      wait_copies<COPIES>();
+    } else wait_copies<0>();
     use(slot, ODD && c == n_chunks - 1);
     if (((c - c0) & (RT == 1 ? 3 : 7)) == (RT == 1 ? 3 : 7))
 #pragma unroll

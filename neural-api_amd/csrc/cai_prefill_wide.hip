@@ -12,6 +12,7 @@
 // The weights are the B operand: a lane then holds results of ONE row, and that row's d and dmin are values it loaded itself.
 #include "cai_layered.hpp"
 #include "cai_gemv_common.hpp"
+#include "cai_async_copy.hpp"
 #include <algorithm>
 
 namespace cai {
@@ -57,16 +58,6 @@ __device__ __forceinline__ void wide_tile(const WideParams& p, int i, int& rg, i
   if (i < body) { rg = (i & 7) + 8 * ((i >> 3) / p.n_tok_tiles); tt = (i >> 3) % p.n_tok_tiles; }
   else { const int j = i - body, r = p.n_row_groups - whole8; rg = whole8 + j % r; tt = j / r; }
 }
-
-// 64 lanes copy 16 bytes each from base + voff to 1 KB of LDS at lds (a wave-uniform byte address).  No registers are written; the
-// copies are counted by vmcnt and the caller waits for all of them before the barrier that publishes the tile.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"     // (m0 is reserved, and named all the same: the statement changes it)
-__device__ __forceinline__ void copy_to_lds(uint32_t lds, uint32_t voff, const void* base)
-{
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
-}
-#pragma clang diagnostic pop
 
 __device__ __forceinline__ half2_w pk_codes(uint32_t v, uint32_t sel, half2_w s2, half2_w c2)
 {
@@ -132,17 +123,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   auto copy_x = [&](int step, int b) {        // past the last step the last one again, into a buffer nobody reads
     const int st = min(step, n_steps - 1), col = sb0 * 256 + st * 64;
 #pragma unroll
-    for (int i = 0; i < XCOP; i++) copy_to_lds(lds0 + (uint32_t)(b * BUF + (wave * XCOP + i) * 1024), voff[i], xplane + col);
-    copy_to_lds(lds0 + (uint32_t)(QOFS + b * QBUF + wave * 1024), qoff, wbase + (int64_t)(sb0 + (st >> 2)) * BB + (st & 3) * 32);
+    for (int i = 0; i < XCOP; i++) copy16_to_lds(lds0 + (uint32_t)(b * BUF + (wave * XCOP + i) * 1024), voff[i], xplane + col);
+    copy16_to_lds(lds0 + (uint32_t)(QOFS + b * QBUF + wave * 1024), qoff, wbase + (int64_t)(sb0 + (st >> 2)) * BB + (st & 3) * 32);
   };
   auto copy_h = [&](int sb) {                 // HCOP copies per wave: waves 4..7 take the block sums in the round that the headers leave to them
     const int b = (sb - sb0) & 1, s = min(sb, sb1 - 1);
     const uint8_t* const blk = wbase + (int64_t)s * BB;
-    if constexpr (HCOP == 2) copy_to_lds(lds0 + (uint32_t)(HOFS + b * HBUF + wave * 1024), hoff[0], blk);
-    if (wave < 4) copy_to_lds(lds0 + (uint32_t)(HOFS + b * HBUF + (HCOP - 1) * 8192 + wave * 1024), hoff[HCOP - 1], blk);
+    if constexpr (HCOP == 2) copy16_to_lds(lds0 + (uint32_t)(HOFS + b * HBUF + wave * 1024), hoff[0], blk);
+    if (wave < 4) copy16_to_lds(lds0 + (uint32_t)(HOFS + b * HBUF + (HCOP - 1) * 8192 + wave * 1024), hoff[HCOP - 1], blk);
     else {                                    // (of 64 tokens twice: every wave issues the same number of copies)
       const int k = (wave - 4) % (2 * BN / 64);
-      copy_to_lds(lds0 + (uint32_t)(SOFS + b * SXBUF + k * 1024), soff, (k < BN / 64 ? p.sxhi : p.sxlo) + s * 8);
+      copy16_to_lds(lds0 + (uint32_t)(SOFS + b * SXBUF + k * 1024), soff, (k < BN / 64 ? p.sxhi : p.sxlo) + s * 8);
     }
   };
   // operand of k-step (hl, t): columns 32 hl + 16 kg + 8 t .. + 7 of the 64
