@@ -9,9 +9,9 @@
 //
 // The row is cut into at most 256 slices, one work-group each, and every stage that needs a number of the whole row is a launch
 // boundary: slice maxima and sums -> [penalised probabilities] -> last values and a histogram of their leading 12 bits -> the few
-// values at or above the bin that holds the m-th largest -> one work-group that ranks these.  What bounds it is launches (five, four
-// without a penalty), not bytes: a 152k row with penalties and temperature takes 30 us in five launches (48 us a call), 244 us (284) as one work-group that
-// walked the row ten times out of L2 at the 40 GB/s one compute unit gets.
+// values at or above the bin that holds the m-th largest -> their ranking, by one work-group up to 32 candidates and sixteen for more.
+// What bounds it is launches (five, four without a penalty), not bytes: a 152k row with penalties, temperature and 40 candidates takes 44 us a call, 284 as
+// one work-group that walked the row ten times out of L2 at the 40 GB/s one compute unit gets.
 #include "cai_internal.hpp"
 #include <algorithm>
 #include <string.h>
@@ -203,8 +203,8 @@ __global__ __launch_bounds__(SL_T) void candidates_reach_kernel(const SamplePara
   float inv = smp_sum<SL_T>(s2, red);
   inv = warm ? 1.0f / (inv <= 0.0f ? 1.0f : inv) : 1.0f;
   smp_crossing<SL_T>(p.bins, min(p.m, p.n), redi, sel);
-  // A division by the sum keeps the order but can make neighbours equal, and equal ones go by token: two steps below the bin are still
-  // in reach.  Where the quotients lose bits to the end of the number range everything is.
+  // A division by the sum keeps the order but can make neighbours equal, and equal ones go by token: a quotient rounds two steps of its
+  // dividend together at most, and with the rounding of the reciprocal values up to four steps below the bin are still in reach.  Where the quotients lose bits to the end of the number range everything is.
   uint32_t floor_bits = (uint32_t)sel[0] << 20;
   floor_bits = warm && __uint_as_float(floor_bits) * inv < 1.0e-36f ? 0u : floor_bits < 4u ? 0u : floor_bits - 4u;
   int mine = 0, total;
@@ -292,8 +292,9 @@ __global__ __launch_bounds__(SMP_T) void candidates_rank_kernel(const SamplePara
   for (int o = tid >> 3; o < n_own; o += SMP_T / 8) {
     const int e = mine[o], t = ct[e];
     const float v = cp[e];
+    const uint32_t u = __float_as_uint(v);       // (values are not negative, so their bits order like they do; a NaN is the largest and has a rank like any other)
     int rank = 0;
-    for (int j = tid & 7; j < total; j += 8) rank += (cp[j] > v) || (cp[j] == v && ct[j] < t);
+    for (int j = tid & 7; j < total; j += 8) { const uint32_t w = __float_as_uint(cp[j]); rank += w > u || (w == u && ct[j] < t); }
     rank += __shfl_xor(rank, 1); rank += __shfl_xor(rank, 2); rank += __shfl_xor(rank, 4);
     if ((tid & 7) == 0 && rank < m) { p.tok_out[rank] = t; p.p_out[rank] = v; }
   }

@@ -103,3 +103,16 @@ def test_more_equal_values_than_are_ranked_directly():
     low[100] = np.nan                                                # counts as far below the maximum
     tok, p = cai.sample_candidates(low, 4, temperature=0.9)
     np.testing.assert_array_equal(tok[:2], [7, 4321]); np.testing.assert_allclose(p[:2], 0.5, rtol=1e-6)
+
+
+@pytest.mark.parametrize("m", [8, 300])
+def test_a_probability_that_overflows_leaves_the_other_ranks_alone(m):
+    """exp(100) is past the largest float: the token's share is NaN, and it still has one rank, the first, so that every place holds a token of this row"""
+    from helpers.device import dev
+    cai = dev()
+    logits = np.random.default_rng(m).standard_normal(5000).astype(np.float32)
+    cai.sample_candidates(logits, 1000)              # (what an earlier call left)
+    tok, p = cai.sample_candidates(logits, m, history=[4321], presence=-100.0)
+    assert tok[0] == 4321 and np.isnan(p[0])
+    np.testing.assert_array_equal(tok[1:], np.arange(m - 1))
+    np.testing.assert_array_equal(p[1:], np.zeros(m - 1))
