@@ -518,6 +518,44 @@ def test_prompt_of_a_mixture_of_more_experts_than_a_wave(experts, T):
     dec.close()
 
 
+def test_short_prompt_of_a_mixture_sums_its_width_in_steps():
+    """12 tokens through experts whose weights and activations are all positive, so that a chain over the width rounds at the size of the whole
+    sum: the last of 128 blocks in one chain is added at 128 times its own size, in steps of sixteen at 16 times.  What the two add to the other
+    roundings of the block (1.6e-7, the walks of the tokens one by one) is 2.0e-7 and 0.3e-7: the bound lies between their sums.
+    The reference is the same block in 64 bits; the attention is switched off by a zero output projection"""
+    from helpers.device import dev
+    from helpers.model_build import _t, synthetic_spec
+    cai = dev()
+    d, I, E, V = 4096, 32, 4, 256
+    cfg = dict(n_layers=1, d_model=d, n_q_heads=2, n_kv_heads=1, head_dim=64, ffn=I, vocab=V, max_ctx=64, eps=1e-5, rope_theta=1e4, n_experts=E, top_k=2, norm_topk=1)
+    spec = synthetic_spec(cfg, O.Q8_0, head_qtype=O.Q8_0, seed=1, std=0.02)
+    rng = np.random.default_rng(2)
+    T = spec["tensors"]
+    put = lambda key, w: T.__setitem__(key, _t(w.astype(np.float32), O.Q8_0))
+    put((-1, O.W_EMBED), rng.uniform(0.5, 1.5, (V, d))); put((0, O.W_O), np.zeros((d, 128)))
+    put((0, O.W_GATEUP), rng.uniform(0.0, 2.0 / d, (2 * I * E, d))); put((0, O.W_DOWN), rng.standard_normal((E * d, I)))
+    w = {k: O.dequant(O.Q8_0, np.asarray(t["raw"]).reshape(-1), t["rows"] * t["cols"]).reshape(t["rows"], t["cols"]).astype(np.float64) for k, t in T.items()}
+    dec = cai.Decoder(spec)
+    rms = lambda x: x / np.sqrt(np.mean(x * x) + np.float64(np.float32(1e-5)))
+    err = size = 0.0
+    for seed in range(8):
+        tok = np.random.default_rng(10 + seed).integers(0, V, 12).astype(np.int32)
+        dec.reset()
+        _, got = dec.prefill(tok)
+        x = w[(-1, O.W_EMBED)][tok[-1]]
+        u = rms(x)
+        s = w[(0, O.W_ROUTER)] @ u
+        top = np.argsort(-s)[:2]
+        g = np.exp(s[top] - s[top].max()); g /= g.sum()
+        for e, ge in zip(top, g):
+            gu = w[(0, O.W_GATEUP)][e * 2 * I:(e + 1) * 2 * I] @ u
+            x = x + ge * (w[(0, O.W_DOWN)][e * d:(e + 1) * d] @ (gu[:I] * gu[I:] / (1.0 + np.exp(-gu[I:]))))
+        want = w[(-1, O.W_HEAD)] @ rms(x)
+        err += np.sum((got - want) ** 2); size += np.sum(want ** 2)
+    dec.close()
+    assert np.sqrt(err / size) < 2.1e-7
+
+
 @pytest.mark.parametrize("cols", [32, 1024, 1056, 2048, 2080, 4096, 4128, 8192, 8224, 24576, 24608])
 def test_prompt_rows_at_the_widths_of_the_pre_pass(cols):
     """the last and the first width of each number of values a thread keeps, and rows that start one float off alignment"""
