@@ -54,18 +54,19 @@ struct BlkGemmParams {
   float post;                           // the results' last factor (gemm_blk_cut)
 };
 
-// eight codes (two dwords) -> eight exact halfs.  Q8_0: signed bytes; Q4_0: (nibble - 8), low or high nibbles of the bytes
+// eight codes (two dwords) -> eight exact halfs, negated or not.  Q8_0: signed bytes; Q4_0: (nibble - 8), low or high nibbles of the bytes
 template <int QT>
-__device__ __forceinline__ half8_b codes8(uint32_t w0, uint32_t w1, int high)
+__device__ __forceinline__ half8_b codes8(uint32_t w0, uint32_t w1, int high, bool neg = false)
 {
   uint32_t a, b; _Float16 off;
   if (QT == CAI_Q8_0) { a = w0 ^ 0x80808080u; b = w1 ^ 0x80808080u; off = (_Float16)(-1152.0f); }   // byte + 128 as 1024 + u, minus 1152
   else { a = (high ? (w0 >> 4) : w0) & 0x0f0f0f0fu; b = (high ? (w1 >> 4) : w1) & 0x0f0f0f0fu; off = (_Float16)(-1032.0f); }
   const half2_b o2 = {off, off};
-  const half2_b h0 = __builtin_bit_cast(half2_b, __builtin_amdgcn_perm(0x64646464u, a, 0x04010400u)) + o2;
-  const half2_b h1 = __builtin_bit_cast(half2_b, __builtin_amdgcn_perm(0x64646464u, a, 0x04030402u)) + o2;
-  const half2_b h2 = __builtin_bit_cast(half2_b, __builtin_amdgcn_perm(0x64646464u, b, 0x04010400u)) + o2;
-  const half2_b h3 = __builtin_bit_cast(half2_b, __builtin_amdgcn_perm(0x64646464u, b, 0x04030402u)) + o2;
+  auto half_pair = [&](uint32_t v, uint32_t sel) {
+    const half2_b h = __builtin_bit_cast(half2_b, __builtin_amdgcn_perm(0x64646464u, v, sel));
+    return neg ? -o2 - h : h + o2;
+  };
+  const half2_b h0 = half_pair(a, 0x04010400u), h1 = half_pair(a, 0x04030402u), h2 = half_pair(b, 0x04010400u), h3 = half_pair(b, 0x04030402u);
   return half8_b{h0.x, h0.y, h1.x, h1.y, h2.x, h2.y, h3.x, h3.y};
 }
 
@@ -293,10 +294,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // Places in LDS: 16-byte piece c of token row t (128 bytes a plane) at c ^ (t / 2 % 8), of Q8_0 weight row n (64 bytes) at c ^ (n / 4 % 4),
 // of Q4_0 row n (32 bytes) at c ^ (n / 8 % 2): the lanes of a read pass then meet different banks.
 // ------------------------------------------------------------------------------------------
-// FINE (panels of the stored streams): the lo halves and the minima are summed apart from the large parts.  A matrix instruction that adds them to the
-// block's sum rounds it once more each (and cuts what lies below the largest of its products off downwards): 1.04e-7 off 64 bits for Q2_K and
-// 0.91e-7 for Q3_K at width 512, where the float walk of eight tokens is 0.96e-7 and 0.88e-7; apart 0.80e-7 both (3584: 1.28e-7 -> 0.95e-7, walk
-// 1.52e-7) for 3 to 5 % of the time.  Q8_0 and Q4_0 are as near as their walk without it (0.92e-7, 0.99e-7 at 512; 1.07e-7 both at 3584).
+// FINE (panels of the stored streams, and up to 16 tokens of Q8_0 and Q4_0: what went through the 32-bit walks otherwise): the lo halves and the
+// minima are summed apart from the large parts.  A matrix instruction that adds them to the block's sum rounds it once more each, and cuts what
+// lies below the largest of its products off downwards (so every second block goes in with its sign changed): 1.04e-7 off 64 bits for Q2_K and 0.91e-7 for Q3_K at width 512, where the walk of
+// eight tokens is 0.96e-7 and 0.88e-7; apart 0.80e-7 both (3584: 1.28e-7 -> 0.95e-7, walk 1.52e-7) for 3 to 5 % of the time.  Q8_0, nine
+// tokens: 0.92e-7 -> 0.82e-7 at 512, walk 0.99e-7; at 3584 1.06e-7 -> 0.97e-7, walk 1.07e-7, and with activations that spread over decades
+// 1.14e-7 -> 1.04e-7, walk 1.05e-7.
 template <int QT, int RT, int NW, bool ODD, bool FINE = false, bool MIN = false>     // ODD: rows of an odd number of blocks (scales that are not aligned to 4 bytes, a last chunk of one block)
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_blk_cut(const BlkGemmParams p)
 {
@@ -387,6 +390,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
     for (int b = 0; b < 2; b++) {
       if (ODD && b && half) break;
+      const bool neg = FINE && b;           // (the second block's products and scale change sign, and with it the side to which the small ones are cut off)
       half8_b A[4], W[RT][2];
 #pragma unroll
       for (int s = 0; s < 2; s++) {
@@ -400,15 +404,15 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
         const unsigned char* const w = s0 + XB + rt * WB + n * WROW;
         if constexpr (QT == CAI_Q8_0) {
           const u32x4_b q = *reinterpret_cast<const u32x4_b*>(w + 16 * ((2 * b + kg) ^ ((n >> 2) & 3)));
-          W[rt][0] = codes8<QT>(q.x, q.y, 0); W[rt][1] = codes8<QT>(q.z, q.w, 0);
+          W[rt][0] = codes8<QT>(q.x, q.y, 0, neg); W[rt][1] = codes8<QT>(q.z, q.w, 0, neg);
         } else {
           const uint2 q = *reinterpret_cast<const uint2*>(w + 16 * (b ^ ((n >> 3) & 1)) + 8 * kg);
-          W[rt][0] = codes8<QT>(q.x, q.y, 0); W[rt][1] = codes8<QT>(q.x, q.y, 1);
+          W[rt][0] = codes8<QT>(q.x, q.y, 0, neg); W[rt][1] = codes8<QT>(q.x, q.y, 1, neg);
         }
       }
 #pragma unroll
       for (int rt = 0; rt < RT; rt++) {
-        const float dv = __half2float(__ushort_as_half((unsigned short)(b ? (dw[rt] >> 16) : (dw[rt] & 0xffffu))));
+        const float dh = __half2float(__ushort_as_half((unsigned short)(b ? (dw[rt] >> 16) : (dw[rt] & 0xffffu)))), dv = neg ? -dh : dh;
         float16_b C = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[0], W[rt][0], zero16, 0, 0, 0);
         if constexpr (FINE) {
           float16_b D = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[1], W[rt][0], zero16, 0, 0, 0);
@@ -565,7 +569,9 @@ int launch_blk(const BlkGemmParams& p0, int n_tiles_grouped)
   };
   auto cut = [&](auto rt_, auto nw_) {
     constexpr int RT = rt_, NW = nw_;
-    return launch_lds<gemm_blk_cut<QT, RT, NW, ODD>>(blk_grid(p, 32 * RT, (p.n_tok + 31) / 32), 64 * NW, NW * 2 * (8192 + RT * 32 * WROW + (ODD ? 512 : 256)), p);
+    const int grid = blk_grid(p, 32 * RT, (p.n_tok + 31) / 32), lds = NW * 2 * (8192 + RT * 32 * WROW + (ODD ? 512 : 256));
+    if (p.n_tok <= 16) return launch_lds<gemm_blk_cut<QT, RT, NW, ODD, true>>(grid, 64 * NW, lds, p);
+    return launch_lds<gemm_blk_cut<QT, RT, NW, ODD>>(grid, 64 * NW, lds, p);
   };
   typedef std::integral_constant<int, 1> One; typedef std::integral_constant<int, 2> Two; typedef std::integral_constant<int, 3> Three;
   typedef std::integral_constant<int, 4> Four; typedef std::integral_constant<int, 7> Seven;
