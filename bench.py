@@ -221,7 +221,7 @@ def gemv_sweep(cai, synth, torch, with_cpu):
 
 def gemm_sweep(cai, synth, torch):
     """One JSON line per (type, shape, tokens): the prompt product cai_qgemm with device pointers (activation pre-pass + matrix-core
-    kernel: gemm_q4k_pf / gemm_q6k_pf / gemm_blk_pf), HIP-event time per call over 10 calls."""
+    kernel: gemm_wide_pf, gemm_q4k_pf, gemm_q6k_pf, gemm_blk_tile or gemm_blk_cut), HIP-event time per call over 10 calls."""
     lib = cai.load()
     gen = torch.Generator(device="cuda"); gen.manual_seed(424242)
     for name, qt in (("Q8_0", cai.Q8_0), ("Q4_0", cai.Q4_0), ("Q4_K", cai.Q4_K), ("Q5_K", cai.Q5_K), ("Q6_K", cai.Q6_K)):

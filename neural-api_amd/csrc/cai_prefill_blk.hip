@@ -290,7 +290,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // Sums are taken in two steps: one chain over a wave's share of 18944 columns is 1.9e-7 off 64 bits, two short ones 1.2e-7, as the
 // one-token kernels are (1 % of the time).
 // What bounds it: the copies, 66 KB/us into one CU.  576 x 1536, 37 tokens, with the pre-pass of the activations: 23.1 us as 10 uncut
-// tiles of 128 x 32 -> 9.6; 64 x 2048, 255 tokens: 27 -> 14; 2048 x 2048, 255: 31 -> 16.
+// tiles of 128 x 32 -> 10.7; 64 x 2048, 255 tokens: 27 -> 14; 2048 x 2048, 255: 31 -> 17.
 // Places in LDS: 16-byte piece c of token row t (128 bytes a plane) at c ^ (t / 2 % 8), of Q8_0 weight row n (64 bytes) at c ^ (n / 4 % 4),
 // of Q4_0 row n (32 bytes) at c ^ (n / 8 % 2): the lanes of a read pass then meet different banks.
 // ------------------------------------------------------------------------------------------
@@ -624,8 +624,8 @@ int launch_blk(const cai_qw_s* w, const BlkGemmParams& p0, int n_tiles_grouped)
 // Q5_0 q - 16; Q4_1, Q5_1 q - 8, q - 16 with m + 8 d, m + 16 d; Q3_K (32 - scale) * q with -d; Q2_K, all doubled, scale * (2 q - c) with c d scale - 2 dmin min,
 // c the whole number of 0 .. 6 next to 2 dmin min / (d scale).
 // (Codes about zero: with q from 0 up the two parts of a sum cancel, and its error doubles.)
-// In place of passes of eight tokens through the float walk, bound by its VALU work: 18944 x 3584 with 200 tokens Q3_K 2282 -> 175 us,
-// Q4_1 1321 -> 252, with 16 tokens 183 -> 74, 106 -> 90; 3584 x 3584 with 16 tokens 52 -> 24, 39 -> 30.  Rewriting takes about 2 bytes of
+// In place of passes of eight tokens through the float walk, bound by its VALU work: 18944 x 3584 with 200 tokens Q3_K 2282 -> 186 us,
+// Q4_1 1321 -> 269, with 16 tokens 183 -> 77, 106 -> 95; 3584 x 3584 with 16 tokens 52 -> 26, 39 -> 31.  Rewriting takes about 2 bytes of
 // memory traffic a weight (40 us of the first), the minima half the time of the products; up to eight tokens the walk is one pass and stays.
 // ------------------------------------------------------------------------------------------
 template <int QT>

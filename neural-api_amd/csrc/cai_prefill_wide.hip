@@ -71,8 +71,8 @@ __device__ __forceinline__ half2_w pk_codes(uint32_t v, uint32_t sel, half2_w s2
 // into one of three buffers, the headers of the super-blocks and the block sums one super-block ahead - so that the loop holds no load
 // whose arrival the compiler would wait for, and the waits count the copies.  The copies are what costs most beside the MFMAs: with 128
 // rows a work-group needs 32 KB of activations for half the products, 37888 x 3584 x 2048 tokens took 1370 us instead of 1213
-// (useful 398 and 458 TFLOP/s; a library product of 4096 f16 rows, the same MFMAs, takes 874 us).  x 511 tokens: 287 us beside 7.6 for the
-// planes and 9.5 for the sums of cut tiles, the kernel of narrow tiles 369; 3584 x 18944 144 + 24 + 9 us, 229 + 24.
+// (useful 398 and 458 TFLOP/s; a library product of 4096 f16 rows, the same MFMAs, takes 874 us).  x 511 tokens, by launch: 286 us beside 7.6 for the
+// planes and 9.6 for the sums of cut tiles, the kernel of narrow tiles 369; 3584 x 18944 143 + 24 + 8.5 us, 229 + 24.
 template <int QT, int TT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_wide_pf(const WideParams p)
 {

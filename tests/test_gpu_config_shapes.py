@@ -203,7 +203,7 @@ def test_olmoe_width_prompt_grouped_by_expert_against_the_oracle():
 @pytest.mark.parametrize("name,n_tok", [("qwen2.5-7b", 230), ("qwen2.5-32b", 150)])
 def test_full_width_prompt_pass_equals_token_at_a_time(name, n_tok):
     """A prompt long enough for the full-width prompt pass to take its large-tile forms (q | k | v as one launch with biases,
-    SwiGLU in the epilogue of the gate|up product - engaged from 193 tokens at 37888 rows, from 129 at 55296 -, the
+    SwiGLU in the epilogue of the gate|up product - on wide tiles, from 33 tokens on at 37888 and 55296 rows -, the
     register-resident pre-pass of the 18944- / 27648-wide row) against the same tokens ingested one step at a time, whose
     kernels the test above pins to the oracle at these widths: last-token logits within 2e-4 of the row's largest logit, same
     arg-max, and the decode step that follows agrees too (the caches hold the same rows)."""

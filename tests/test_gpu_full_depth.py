@@ -84,8 +84,8 @@ def test_qwen7b_all_28_blocks_64_greedy_tokens_against_the_oracle():
 
 def test_large_tile_prompt_pass_of_one_full_width_block_against_the_oracle():
     """A 256-token prompt through ONE block of the 7B width (vocabulary cut to 1024 rows so that the oracle's 257 steps stay
-    short): the prompt pass takes its large-tile forms - q | k | v as one launch with biases, the gate|up product with two row
-    tiles per wave and SwiGLU in its epilogue (engaged from 193 tokens at 37888 rows), the register-resident pre-pass of the
+    short): the prompt pass takes its large-tile forms - q | k | v as one launch with biases, the gate|up product on wide tiles
+    with SwiGLU in its epilogue (from 33 tokens on at 37888 rows), the register-resident pre-pass of the
     18944-wide row, matrix-core prompt attention - and is compared DIRECTLY with the oracle stepping token by token: last-token
     logits within 1e-3 of the row's largest logit, same arg-max, and the decode step that follows (it reads the cache rows the
     prompt pass wrote) as well."""
