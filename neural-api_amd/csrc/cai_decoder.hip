@@ -467,6 +467,8 @@ static int enqueue_prefill_chunk(cai_decoder_s* d, int seq, int n)
 }
 
 // `rows_needed`: cache rows the step's attention must cover (largest position + 1 over its rows)
+// The host's tokens and positions (h_io) are read by the step's first launch, a node of its graph: a copy in front of the graph cost 12 us of
+// waiting between the two.
 static int run_step(cai_decoder_s* d, int n_b, int rows_needed, bool window = false, int seq0 = 0)
 {
   Context& c = ctx();
@@ -486,12 +488,13 @@ static int run_step(cai_decoder_s* d, int n_b, int rows_needed, bool window = fa
   const int bucket = kv_bucket_rows(&d->kv, rows_needed);
   d->kv.geo_rows = bucket;
   // (a captured graph holds the sequence index: only sequence 0 has one)
-  if (!d->use_graph || seq0 != 0) { const int rc = enqueue_step(d, n_b, seq0, ~0u, window); if (rc) return rc; CAI_HIP(hipGetLastError()); return CAI_OK; }
+  auto body = [&]() -> int { launch_words_copy(d->h_io, d->d_tokens, 16); return enqueue_step(d, n_b, seq0, ~0u, window); };
+  if (!d->use_graph || seq0 != 0) { const int rc = body(); if (rc) return rc; CAI_HIP(hipGetLastError()); return CAI_OK; }
   hipGraphExec_t& ge = d->graphs[cai_decoder_s::graph_key(window ? 1 : 0, n_b, bucket)];
   if (!ge) {
     hipGraph_t g = nullptr;
     CAI_HIP(hipStreamBeginCapture(c.stream, hipStreamCaptureModeThreadLocal));
-    const int rc = enqueue_step(d, n_b, 0, ~0u, window);
+    const int rc = body();
     const hipError_t e = hipStreamEndCapture(c.stream, &g);
     if (rc) { if (g) (void)hipGraphDestroy(g); return rc; }
     if (e != hipSuccess) return hip_fail(e, "hipStreamEndCapture", __FILE__, __LINE__);
@@ -501,6 +504,13 @@ static int run_step(cai_decoder_s* d, int n_b, int rows_needed, bool window = fa
   }
   CAI_HIP(hipGraphLaunch(ge, c.stream));
   return CAI_OK;
+}
+
+// What a step left, to the caller (either may be null); waits for the stream.
+static int fetch_step(cai_decoder_s* d, int n_b, float* logits, int32_t* argmax)
+{
+  const HostCopy out[2] = {{logits, d->logits, logits ? (size_t)n_b * d->cfg.vocab * 4 : 0}, {argmax, d->d_argmax, argmax ? (size_t)n_b * 4 : 0}};
+  return fetch_to_host(out, 2);
 }
 
 // `steps` greedy batch-1 steps of sequence 0, each followed by the hand-over kernel, as ONE graph launch (steps = 1 or
@@ -767,19 +777,12 @@ extern "C" int cai_decoder_step(cai_decoder_t d, const int32_t* tokens, const in
     if (pos[b] != d->kv.len_at(b, 0)) return set_error(CAI_ERR_STATE, "cai_decoder_step: sequence %d is at position %d, got %d", b, d->kv.len_at(b, 0), pos[b]);
     if (pos[b] >= c.max_ctx && d->kv.evict_cap == 0) return set_error(CAI_ERR_STATE, "cai_decoder_step: sequence %d reached max_ctx %d", b, c.max_ctx);
   }
-  Context& cx = ctx();
   for (int b = 0; b < n_b; b++) { d->h_io[b] = tokens[b]; d->h_io[8 + b] = pos[b]; }
-  CAI_HIP(hipMemcpyAsync(d->d_tokens, d->h_io, 16 * sizeof(int32_t), hipMemcpyHostToDevice, cx.stream));
   int rows_needed = 0;
   for (int b = 0; b < n_b; b++) rows_needed = std::max(rows_needed, pos[b] + 1);
   if ((rc = run_step(d, n_b, rows_needed))) return rc;
-  if (logits) CAI_HIP(hipMemcpyAsync(logits, d->logits, (size_t)n_b * c.vocab * 4, hipMemcpyDeviceToHost, cx.stream));
-  CAI_HIP(hipMemcpyAsync(d->h_io + 16, d->d_argmax, 8 * sizeof(int32_t), hipMemcpyDeviceToHost, cx.stream));
-  CAI_HIP(hipStreamSynchronize(cx.stream));
-  for (int b = 0; b < n_b; b++) {
-    for (int l = 0; l < c.n_layers; l++) d->kv.len_at(b, l) = pos[b] + 1;
-    if (argmax) argmax[b] = d->h_io[16 + b];
-  }
+  if ((rc = fetch_step(d, n_b, logits, argmax))) return rc;
+  for (int b = 0; b < n_b; b++) for (int l = 0; l < c.n_layers; l++) d->kv.len_at(b, l) = pos[b] + 1;
   return CAI_OK;
 }
 
@@ -808,13 +811,9 @@ extern "C" int cai_decoder_step_window(cai_decoder_t d, int seq, const int32_t* 
   if (n > 1 && (rc = ensure_wpart(d))) return rc;
   CAI_HIP(hipStreamSynchronize(cx.stream));   // h_io is reused
   for (int i = 0; i < n; i++) { d->h_io[i] = tokens[i]; d->h_io[8 + i] = pos0 + i; }
-  CAI_HIP(hipMemcpyAsync(d->d_tokens, d->h_io, 16 * sizeof(int32_t), hipMemcpyHostToDevice, cx.stream));
   if ((rc = run_step(d, n, pos0 + n, n > 1, seq))) return rc;
-  if (logits) CAI_HIP(hipMemcpyAsync(logits, d->logits, (size_t)n * c.vocab * 4, hipMemcpyDeviceToHost, cx.stream));
-  CAI_HIP(hipMemcpyAsync(d->h_io + 16, d->d_argmax, 8 * sizeof(int32_t), hipMemcpyDeviceToHost, cx.stream));
-  CAI_HIP(hipStreamSynchronize(cx.stream));
+  if ((rc = fetch_step(d, n, logits, argmax))) return rc;
   for (int l = 0; l < c.n_layers; l++) d->kv.len_at(seq, l) = pos0 + n;
-  if (argmax) for (int i = 0; i < n; i++) argmax[i] = d->h_io[16 + i];
   return CAI_OK;
 }
 
@@ -1055,7 +1054,6 @@ extern "C" int cai_decoder_prefill(cai_decoder_t d, int seq, const int32_t* toke
     for (int i = 0; i < n; i++) {
       CAI_HIP(hipStreamSynchronize(cx.stream));   // h_io is reused
       d->h_io[0] = tokens[i]; d->h_io[8] = pos0 + i;
-      CAI_HIP(hipMemcpyAsync(d->d_tokens, d->h_io, 16 * sizeof(int32_t), hipMemcpyHostToDevice, cx.stream));
       if ((rc = run_step(d, 1, pos0 + i + 1, false, seq))) return rc;
     }
   } else {
@@ -1082,11 +1080,8 @@ extern "C" int cai_decoder_prefill(cai_decoder_t d, int seq, const int32_t* toke
       }
     }
   }
-  if (last_logits) CAI_HIP(hipMemcpyAsync(last_logits, d->logits, (size_t)c.vocab * 4, hipMemcpyDeviceToHost, cx.stream));
-  CAI_HIP(hipMemcpyAsync(d->h_io + 16, d->d_argmax, 8 * sizeof(int32_t), hipMemcpyDeviceToHost, cx.stream));
-  CAI_HIP(hipStreamSynchronize(cx.stream));
+  if ((rc = fetch_step(d, 1, last_logits, argmax))) return rc;
   for (int l = 0; l < c.n_layers; l++) d->kv.len_at(seq, l) = pos0 + n;
-  if (argmax) *argmax = d->h_io[16];
   return CAI_OK;
 }
 

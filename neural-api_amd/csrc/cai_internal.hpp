@@ -26,6 +26,7 @@ struct Context {
   void*  h_stage = nullptr; size_t h_stage_cap = 0;      // pinned host memory of calls that wait for their results (kernels read and write it in place)
   int32_t* d_small = nullptr;            // 1024 ints of device scratch for small arguments/results
   int32_t* h_small = nullptr;            // 1024 ints of pinned host memory paired with d_small
+  hipEvent_t  piece_ev[8] = {};          // pieces of a result on their way to the host (fetch_to_host)
   // Step timeline (measurement aid, cai_decoder_timeline): while armed, every instrumented launch gets a record of eight
   // wall-clock stamps per work-group (0 entry .. 7 exit, the ones between are the kernel's own) and a descriptor (class,
   // work-groups, offset)
@@ -70,6 +71,10 @@ int  set_error(int code, const char* fmt, ...);
 int  hip_fail(hipError_t e, const char* what, const char* file, int line);
 int  ensure_stage(void** p, size_t* cap, size_t need);
 int  ensure_host_stage(size_t need);   // grows ctx().h_stage; only for calls that do not return before the stream is done with it
+// A call's results: `bytes` (whole words) at the device address src for the caller's memory dst.  fetch_to_host waits for the stream.
+struct HostCopy { void* dst; const void* src; size_t bytes; };
+int  fetch_to_host(const HostCopy* c, int n);
+void launch_words_copy(const void* src, void* dst, int words);   // a few words between device and pinned memory, either way, as a launch of the stream (or node of a graph)
 
 #define CAI_HIP(call)                                                        \
   do {                                                                       \

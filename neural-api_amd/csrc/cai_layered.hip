@@ -797,6 +797,7 @@ static int run_captured(LayeredNet* n, int R, int steps, bool gen, int end)
   if (reach >= n->pool.keep) reach = std::max(n->pool.keep, 1);
   const StepRows r = dec_rows(n, R, reach);
   auto body = [&]() -> int {
+    if (!gen) launch_words_copy(n->h_dec, n->d_dec, 9 * DEC_ROWS);      // (a node of the graph: a copy in front of it cost 12 us of waiting between the two)
     for (int i = 0; i < steps; i++) {
       const int rc = enqueue_net(n, r, true, StepLists(), nullptr, R);
       if (rc) return rc;
@@ -858,7 +859,6 @@ int net_step(LayeredNet* n, int n_ent, const int32_t* seq, const int32_t* count,
       hd[e] = tokens[e]; hd[DEC_ROWS + e] = pos; hd[2 * DEC_ROWS + e] = seq[e]; hd[3 * DEC_ROWS + e] = e; hd[4 * DEC_ROWS + e] = e;
       int32_t* en = hd + 5 * DEC_ROWS + 4 * e; en[0] = seq[e]; en[1] = e; en[2] = 1; en[3] = pos;
     }
-    CAI_HIP(hipMemcpyAsync(n->d_dec, hd, 9 * DEC_ROWS * sizeof(int32_t), hipMemcpyHostToDevice, st));
     if ((rc = run_captured(n, R, 1, false, end))) return rc;
     n->row_of = wrows; n->rows_gathered = false;
   } else {
@@ -915,14 +915,15 @@ int net_step(LayeredNet* n, int n_ent, const int32_t* seq, const int32_t* count,
     for (int k = 0; k < W; k++) n->row_of.push_back(k);
     n->rows_gathered = true;
   }
+  std::vector<HostCopy> out;
   for (int k = 0; k < W; k++) {
     // (consecutive logits rows come back in one copy)
     int k2 = k; while (k2 + 1 < W && n->row_of[k2 + 1] == n->row_of[k2] + 1) k2++;
-    if (logits_host) CAI_HIP(hipMemcpyAsync(logits_host + (size_t)k * n->s.vocab, n->logits + (size_t)n->row_of[k] * n->s.vocab, (size_t)(k2 - k + 1) * n->s.vocab * 4, hipMemcpyDeviceToHost, st));
-    if (argmax_host) CAI_HIP(hipMemcpyAsync(argmax_host + k, n->best + n->row_of[k], (size_t)(k2 - k + 1) * 4, hipMemcpyDeviceToHost, st));
+    if (logits_host) out.push_back({logits_host + (size_t)k * n->s.vocab, n->logits + (size_t)n->row_of[k] * n->s.vocab, (size_t)(k2 - k + 1) * n->s.vocab * 4});
+    if (argmax_host) out.push_back({argmax_host + k, n->best + n->row_of[k], (size_t)(k2 - k + 1) * 4});
     k = k2;
   }
-  CAI_HIP(hipStreamSynchronize(st));
+  if ((rc = fetch_to_host(out.data(), (int)out.size()))) return rc;
   for (int e = 0; e < n_ent; e++) { n->pool.seq[seq[e]].len += count[e]; n->pool.trim(seq[e]); }
   return CAI_OK;
 }

@@ -592,3 +592,34 @@ def test_rotary_positions_far_beyond_32768_in_a_rolling_session():
             assert rel_err(ld[0], lo) < 1e-3, (pos, rel_err(ld[0], lo))
             pos += 1; toks.append(int(am[0]))
     dec.close()
+
+
+@pytest.mark.parametrize("vocab, n_b, tokens", [(5001, 1, 1), (5001, 3, 1), (70001, 8, 1), (70001, 8, 8), (262149, 1, 1), (262147, 8, 8)])
+def test_logits_reach_the_callers_memory_whole(vocab, n_b, tokens):
+    """Rows of odd lengths in one piece, in eight, and past what is staged (8 MB): every word arrives and nothing beside them is written.
+    The arg-max is taken on the device, the rows of a batch or window are those of single steps."""
+    import ctypes as C
+    from helpers.device import dev, rel_err
+    cai = dev()
+    cfg = dict(n_layers=1, d_model=64, n_q_heads=1, n_kv_heads=1, head_dim=64, ffn=64, vocab=vocab, max_ctx=256, eps=1e-5, rope_theta=1e4)
+    dec = cai.Decoder(synthetic_spec(cfg, O.Q8_0, std=0.05), max_batch=8)
+    ids = np.random.default_rng(vocab).integers(0, vocab, n_b).astype(np.int32)
+    rows = np.full((n_b + 2, vocab), np.nan, np.float32)
+    got, am = rows[1:-1], np.full(n_b, -1, np.int32)
+    if tokens == 1:
+        pos = np.zeros(n_b, np.int32)
+        cai.check(cai.load().cai_decoder_step(dec.h, ids.ctypes.data, pos.ctypes.data, n_b, C.c_void_p(got.ctypes.data), C.c_void_p(am.ctypes.data)))
+    else:
+        cai.check(cai.load().cai_decoder_step_window(dec.h, 0, ids.ctypes.data, n_b, 0, C.c_void_p(got.ctypes.data), C.c_void_p(am.ctypes.data)))
+    assert np.isnan(rows[0]).all() and np.isnan(rows[-1]).all() and np.isfinite(got).all()
+    assert am.tolist() == got.argmax(1).tolist()
+    for b in range(n_b):
+        if tokens == 1:
+            dec.reset(b)
+    if tokens > 1:
+        dec.reset(0)
+    for b in range(n_b):
+        if tokens == 1:
+            dec.reset(0)
+        one = dec.step(ids[b], 0 if tokens == 1 else b)[1]
+        assert rel_err(one[0], got[b]) < 1e-5
