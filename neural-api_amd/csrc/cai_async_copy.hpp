@@ -18,6 +18,11 @@ __device__ __forceinline__ void copy16_to_lds(uint32_t lds, uint32_t voff, const
 {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
 }
+// of what is read once: not kept in the caches
+__device__ __forceinline__ void copy16_to_lds_once(uint32_t lds, uint32_t voff, const void* base)
+{
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" :: "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
+}
 __device__ __forceinline__ void copy4_to_lds(uint32_t lds, uint32_t voff, const void* base)
 {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" :: "s"(lds), "v"(voff), "s"(base) : "memory", "m0");

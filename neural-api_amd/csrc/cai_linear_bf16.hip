@@ -16,7 +16,8 @@
 namespace cai {
 
 // ------------------------------------------------------------------------------------------
-// Decode: NB activation rows.  A wave owns R weight rows (of a gated matrix R / 2 outputs) or, with ksplit > 1, every ksplit-th
+// Decode, every product in 32 bits: float activations, an RMS norm on the way, two products in one, and bfloat16 rows of more than 8192 columns.
+// NB activation rows.  A wave owns R weight rows (of a gated matrix R / 2 outputs) or, with ksplit > 1, every ksplit-th
 // 512-wide turn of them; the activations are staged in LDS as float in panels, the weights stream past once.
 // GV_RMS: the activations are the float stream, RMS-normed on the way (the gain while they are staged, the root at the end), and the
 // work-groups from q.blocks on do the same for a second matrix with a gain of its own.
@@ -188,6 +189,106 @@ __global__ __launch_bounds__(64 * GV_WAVES) void gemv_bf16(const uint16_t* __res
   } else if (i < R && grp * R + i < n_rows) {
     if constexpr (KIND == GV_RMS) { if (e.mode == EPI_SPLIT) epi_as<AT, EPI_SPLIT>(e, grp * R + i, b, mine); else epi_as<AT, EPI_STORE>(e, grp * R + i, b, mine); }
     else epi_one<AT>(e, grp * R + i, b, mine);
+  }
+}
+
+// ------------------------------------------------------------------------------------------
+// Decode over bfloat16 activations, and their shortest prompts: the matrix cores multiply eight weight rows (twice: a tile has sixteen) and up to
+// 16 activation rows (lanes past the last one repeat it; what they make is not read), so a weight costs no more at sixteen rows than at one, and
+// what is left is the stream of weights.  A work-group owns MC_H rows (of a gated matrix so many gate and up rows) at a time, its KS waves every
+// KS-th slot of 256 columns of them.  A wave copies its slots (two rows of 512 bytes a request; requests of 64 bytes a row, the shape of the
+// operands, reached half the rate) into a ring of its own in LDS without meeting anyone, and keeps its part of the activations in registers from
+// tile to tile.  16-byte chunk q of row r lies at q ^ r, which makes the operand reads conflict-free.  The sums of a tile meet once, in one of two
+// areas in turn.  Weights are read past the caches' replacement ("nt"): a step's do not fit the memory-side cache, and kept there one by one
+// they push each other out.
+// Per launch at 4 rows, us, by the 32-bit walk below | here: 11264 x 2048 gated 14.2 | 10.8; 2048 x 5632 10.9 | 9.3; 6200 x 2048 9.2 | 7.6;
+// 32768 x 2048 33.7 | 24.6 (5.4 TB/s).  Sixteen rows a tile: 128 work-groups for 2048 rows, 9.9 for 2048 x 5632; a ring of one slot
+// loses 2 % of a step; without "nt" 13.2 and 10.6.
+// ------------------------------------------------------------------------------------------
+constexpr int MC_WAVES = 8, MC_ROWS = 16, MC_H = 8, MC_SLOT = MC_H * 512, MC_SLOTS = 4;      // (at most MC_SLOTS slots of a row a wave)
+constexpr int mc_depth(int sb) { return sb < 2 ? 2 : sb; }  // slots of a wave's ring: a tile's, and the next one's where that is one
+template <bool GLU, int SB>
+__global__ __launch_bounds__(64 * MC_WAVES) void gemv_bf16_mc(const uint16_t* __restrict__ W, const bf16_t* __restrict__ x, int n_rows, int ldw, int64_t ldx, int n_tok, int n_tiles, LinEpi e)
+{
+  constexpr int T = GLU ? 2 : 1, DEPTH = mc_depth(SB), COPIES = MC_H / 2;
+  extern __shared__ u32x4 mc_lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), KS = blockDim.x >> 6;
+  const int r = lane & 15, c = lane >> 4, hi = lane >> 5;
+  const int slots = (ldw + 255) >> 8, mine = wave < slots ? (slots - wave + KS - 1) / KS : 0;       // slots of a row, of this wave
+  float* const parts = reinterpret_cast<float*>(mc_lds) + KS * (DEPTH * MC_SLOT / 4);
+  const int part_len = n_tok * T * 16;                                                              // of one wave: [token][row]
+  const char* const ring = reinterpret_cast<const char*>(mc_lds) + wave * (DEPTH * MC_SLOT);
+  const uint32_t ring0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) u32x4*)mc_lds + wave * (DEPTH * MC_SLOT);
+  auto first_row = [](int tile, int t) { return !GLU ? tile * MC_H : (tile >> 1) * 32 + t * 16 + (tile & 1) * MC_H; };
+  // the next slot to request: slot q_s of this wave, of part q_t of tile q_tile
+  int q_tile = blockIdx.x, q_t = 0, q_s = 0, q_ring = 0;
+  auto request = [&]() {
+    const int row0 = first_row(q_tile, q_t), k0 = (wave + q_s * KS) * 256, chunks = min(32, (ldw - k0) >> 3);
+    const char* const base = reinterpret_cast<const char*>(W + (int64_t)row0 * ldw + k0);
+    const int last = n_rows - 1 - row0;
+#pragma unroll
+    for (int i = 0; i < COPIES; i++) {
+      const int row = 2 * i + hi;
+      copy16_to_lds_once(ring0 + q_ring * MC_SLOT + i * 1024, (uint32_t)(min(row, last) * ldw * 2 + min((lane & 31) ^ row, chunks - 1) * 16), base);
+    }
+    q_ring = q_ring + 1 == DEPTH ? 0 : q_ring + 1;
+    if (++q_s == mine) { q_s = 0; if (++q_t == T) { q_t = 0; q_tile += gridDim.x; } }
+  };
+  int ahead = 0;
+  if (mine) {
+#pragma unroll
+    for (int i = 0; i < DEPTH; i++) if (q_tile < n_tiles) { request(); ahead++; }
+  }
+  u32x4 b[SB][8];
+#pragma unroll
+  for (int s = 0; s < SB; s++)
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      const int k = min((wave + s * KS) * 256 + u * 32, ldw - 32);
+      b[s][u] = *reinterpret_cast<const u32x4*>(x + min(r, n_tok - 1) * ldx + k + c * 8);
+    }
+  int at = 0, parity = 0;
+  for (int tile = blockIdx.x, turn = 0; tile < n_tiles; tile += gridDim.x, turn++) {
+    f32x4 acc[T];
+#pragma unroll
+    for (int t = 0; t < T; t++) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int t = 0; t < T; t++)
+#pragma unroll
+      for (int s = 0; s < SB; s++)
+        if (s < mine) {
+          if (ahead == DEPTH) wait_copies<(DEPTH - 1) * COPIES>(); else wait_copies<0>();
+          const char* const slot = ring + at * MC_SLOT;
+          u32x4 w[8];
+#pragma unroll
+          for (int u = 0; u < 8; u++) { const int row = r & (MC_H - 1); w[u] = *reinterpret_cast<const u32x4*>(slot + row * 512 + (((u * 4 + c) ^ row) << 4)); }
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the slot has been read
+          at = at + 1 == DEPTH ? 0 : at + 1;
+          if (q_tile < n_tiles) request(); else ahead--;
+          const int left = (ldw - (wave + s * KS) * 256) >> 5;
+          if (left >= 8) {
+#pragma unroll
+            for (int u = 0; u < 8; u++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[u]), __builtin_bit_cast(bf16x8, b[s][u]), acc[t], 0, 0, 0);
+          } else {
+#pragma unroll
+            for (int u = 0; u < 8; u++) if (u < left) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[u]), __builtin_bit_cast(bf16x8, b[s][u]), acc[t], 0, 0, 0);
+          }
+        }
+    float* const area = parts + parity * KS * part_len;
+    parity ^= 1;
+    if (r < n_tok)
+#pragma unroll
+      for (int t = 0; t < T; t++) *reinterpret_cast<f32x4*>(area + wave * part_len + r * (T * 16) + t * 16 + c * 4) = acc[t];
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // (no wait for the copies on their way)
+    // (another wave's turn from tile to tile: a result's own loads wait for the copies requested before them)
+    for (int o = (tid + turn * 64) & (blockDim.x - 1); o < MC_H * n_tok; o += blockDim.x) {
+      const int i = o & (MC_H - 1), tok = o / MC_H, n = first_row(tile, 0) + i;
+      const float* p = area + tok * (T * 16) + i;
+      float v = 0.0f, up = 0.0f;
+      for (int w = 0; w < KS; w++) { v += p[w * part_len]; if (GLU) up += p[w * part_len + 16]; }
+      if constexpr (GLU) put_act<bf16_t>(e.h, tok * e.ldh + tile * MC_H + i, glu_pair(e.glu, e.limit, v, up));
+      else if (n < n_rows) epi_one<bf16_t>(e, n, tok, v);
+    }
   }
 }
 
@@ -455,9 +556,39 @@ static void run_gemv_rows(int n_tok, const cai_qw_s* w, const void* x, int64_t l
   }
 }
 
+template <bool GLU, int SB>
+static int run_mc(const cai_qw_s* w, const bf16_t* x, int64_t ldx, int n_tok, const LinEpi& e, int ks)
+{
+  constexpr int T = GLU ? 2 : 1;
+  auto lds_of = [](int waves, int rows) { return (size_t)waves * (mc_depth(SB) * MC_SLOT + 2 * rows * T * 16 * 4); };
+  static bool attr_done = false;
+  if (!attr_done) {
+    CAI_HIP(hipFuncSetAttribute((const void*)gemv_bf16_mc<GLU, SB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_of(MC_WAVES, MC_ROWS)));
+    attr_done = true;
+  }
+  const int tiles = ((int)w->rows + T * MC_H - 1) / (T * MC_H);
+  const size_t lds = lds_of(ks, n_tok);
+  const int per_cu = std::min((int)(160 * 1024 / lds), 16 / ks);      // (sixteen waves of these registers fill a CU)
+  hipLaunchKernelGGL((gemv_bf16_mc<GLU, SB>), dim3(std::min(tiles, std::max(1, per_cu) * ctx().n_cu)), dim3(64 * ks), lds, ctx().stream,
+                     (const uint16_t*)w->data, x, (int)w->rows, (int)w->ld, ldx, n_tok, tiles, e);
+  return CAI_OK;
+}
+static int run_gemv_mc(const cai_qw_s* w, const bf16_t* x, int64_t ldx, int n_tok, const LinEpi& e)
+{
+  const int slots = ((int)w->ld + 255) / 256;
+  int ks = 1;
+  while (ks < MC_WAVES && ks < slots) ks *= 2;
+#define MC(SB) return e.mode == EPI_GLU ? run_mc<true, SB>(w, x, ldx, n_tok, e, ks) : run_mc<false, SB>(w, x, ldx, n_tok, e, ks)
+  switch ((slots + ks - 1) / ks) { case 1: MC(1); case 2: MC(2); case 3: MC(3); default: MC(4); }
+#undef MC
+}
+
 template <typename AT>
 static int run_lin(const cai_qw_s* w, const AT* x, int64_t ldx, int n_tok, const LinEpi& e)
 {
+  if constexpr (sizeof(AT) == 2) {
+    if (n_tok <= MC_ROWS && w->ld <= 256 * MC_WAVES * MC_SLOTS) return run_gemv_mc(w, x, ldx, n_tok, e);
+  }
   if (n_tok <= LIN_FEW) {
     const bool glu = e.mode == EPI_GLU;
     const GvShape s = gv_shape((int)w->rows, gv_turns(w), glu);

@@ -115,6 +115,19 @@ def test_products_on_large_tiles_of_many_steps(cai, tmp_path, tokens, ff, width)
     dec.close()
 
 
+@pytest.mark.parametrize("width, ff, vocab", [(72, 17, 61), (192, 300, 131), (264, 520, 9), (776, 1100, 1003), (2056, 2120, 67), (328, 4200, 67), (72, 8192, 67), (72, 8200, 67)])
+def test_streamed_bf16_products(cai, tmp_path, width, ff, vocab):
+    """One to sixteen rows: one partial slot of 256 columns, a last slot of 8 to 200 columns, one to four waves of a row with and without work, two
+    to four slots a wave, widths of 8192 columns and past them (another kernel); rows that end inside a tile; fewer tiles than work-groups and more."""
+    m = Model(tmp_path, B.config([B.layer(B.delta(), ff=ff)], width=width, vocab=vocab), seed=width, edit=only("feed-forward"), rank_a=3, rank_g=20)
+    tok = m.tokens(40, 1)
+    dec = m.open(cai, 64, 1, "bf16")
+    for cuts in ([1], [2, 3, 5, 7, 8], [9, 16, 15]):
+        check(feed(dec, tok, cuts), m.ref(tok), "bf16")
+        dec.reset()
+    dec.close()
+
+
 # ---------------------------------------------------------------- whole models
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
 @pytest.mark.parametrize("cuts", [[300], [1], [2], [3, 2, 65, 1, 1, 16, 17, 2], [64], [130, 1], [5, 9, 7]], ids=str)
