@@ -41,32 +41,37 @@ template <> __device__ __forceinline__ float kv_from_float<float>(float v) { ret
 template <> __device__ __forceinline__ __half kv_from_float<__half>(float v) { return __float2half_rn(v); }
 
 
-// DS consecutive cache elements as floats with ONE vector load (the head width is a multiple of DS, so a lane's
-// DS-wide slot is either wholly inside the row or wholly outside it)
-template <int DS, typename KV_T> __device__ __forceinline__ void load_row_vec(const KV_T* src, float (&o)[DS]);
-template <> __device__ __forceinline__ void load_row_vec<1, float>(const float* s, float (&o)[1]) { o[0] = s[0]; }
-template <> __device__ __forceinline__ void load_row_vec<2, float>(const float* s, float (&o)[2]) { const float2 v = *reinterpret_cast<const float2*>(s); o[0] = v.x; o[1] = v.y; }
-template <> __device__ __forceinline__ void load_row_vec<4, float>(const float* s, float (&o)[4]) { const float4 v = *reinterpret_cast<const float4*>(s); o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w; }
-template <> __device__ __forceinline__ void load_row_vec<1, __half>(const __half* s, float (&o)[1]) { o[0] = __half2float(s[0]); }
-template <> __device__ __forceinline__ void load_row_vec<2, __half>(const __half* s, float (&o)[2]) { const __half2 v = *reinterpret_cast<const __half2*>(s); o[0] = __low2float(v); o[1] = __high2float(v); }
-template <> __device__ __forceinline__ void load_row_vec<4, __half>(const __half* s, float (&o)[4])
+// VW (2 or 4) consecutive cache elements with one load, kept as they lie until they are used: a conversion beside the load would wait for it
+// before the next goes out
+template <int VW, typename KV_T> struct RowVec;
+template <> struct RowVec<2, float> { typedef float type __attribute__((ext_vector_type(2), aligned(4))); };
+template <> struct RowVec<4, float> { typedef float type __attribute__((ext_vector_type(4), aligned(4))); };
+template <> struct RowVec<2, __half> { using type = uint32_t; };
+template <> struct RowVec<4, __half> { using type = uint2; };
+template <> struct RowVec<2, int8_t> { using type = uint16_t; };
+template <> struct RowVec<4, int8_t> { using type = uint32_t; };
+template <int VW, typename KV_T> using row_vec = typename RowVec<VW, KV_T>::type;
+template <int VW, typename KV_T>
+__device__ __forceinline__ void row_floats(const row_vec<VW, KV_T>& r, float* o)
 {
-  const uint2 r = *reinterpret_cast<const uint2*>(s);
-  const __half2 a = __builtin_bit_cast(__half2, r.x), b = __builtin_bit_cast(__half2, r.y);
-  o[0] = __low2float(a); o[1] = __high2float(a); o[2] = __low2float(b); o[3] = __high2float(b);
+  if constexpr (sizeof(KV_T) == 4) {
+#pragma unroll
+    for (int i = 0; i < VW; i++) o[i] = r[i];
+  } else if constexpr (sizeof(KV_T) == 2) {
+    if constexpr (VW == 2) { const __half2 h = __builtin_bit_cast(__half2, r); o[0] = __low2float(h); o[1] = __high2float(h); }
+    else {
+      const __half2 h = __builtin_bit_cast(__half2, r.x), g = __builtin_bit_cast(__half2, r.y);
+      o[0] = __low2float(h); o[1] = __high2float(h); o[2] = __low2float(g); o[3] = __high2float(g);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < VW; i++) o[i] = (float)((int)((uint32_t)r << (24 - 8 * i)) >> 24);
+  }
 }
-
-template <> __device__ __forceinline__ void load_row_vec<1, int8_t>(const int8_t* s, float (&o)[1]) { o[0] = (float)s[0]; }
-template <> __device__ __forceinline__ void load_row_vec<2, int8_t>(const int8_t* s, float (&o)[2])
-{
-  const int r = *reinterpret_cast<const short*>(s);
-  o[0] = (float)(int8_t)(r & 0xff); o[1] = (float)(int8_t)((r >> 8) & 0xff);
-}
-template <> __device__ __forceinline__ void load_row_vec<4, int8_t>(const int8_t* s, float (&o)[4])
-{
-  const int r = *reinterpret_cast<const int*>(s);
-  o[0] = (float)((r << 24) >> 24); o[1] = (float)((r << 16) >> 24); o[2] = (float)((r << 8) >> 24); o[3] = (float)(r >> 24);
-}
+// sum / maximum over each row of 16 lanes, in every lane of it
+#define ROW_ROR(v, n) __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, (v)), 0x120 + (n), 0xf, 0xf, false))
+__device__ __forceinline__ float row16_sum(float v) { v += ROW_ROR(v, 8); v += ROW_ROR(v, 4); v += ROW_ROR(v, 2); v += ROW_ROR(v, 1); return v; }
+__device__ __forceinline__ float row16_max(float v) { v = fmaxf(v, ROW_ROR(v, 8)); v = fmaxf(v, ROW_ROR(v, 4)); v = fmaxf(v, ROW_ROR(v, 2)); v = fmaxf(v, ROW_ROR(v, 1)); return v; }
 
 // max over each half-wave (32 lanes), result in every lane of that half
 __device__ __forceinline__ float half_wave_allmax(float v)
@@ -78,8 +83,8 @@ __device__ __forceinline__ float half_wave_allmax(float v)
 // One cached row of an int8 cache from DS elements per lane of a half-wave (neural/neural.cl:2549-2578): the maximum
 // over FINITE magnitudes, zero codes and unit scale when that maximum is zero or denormal, else scale = max / 127 and
 // code = clamp(rint(v * (1/max) * 127)), NaN -> 0.  Lanes beyond the head width pass zeros.  On return v[] holds the
-// codes as floats.
-template <int DS> __device__ __forceinline__ float quantise_row_i8(float (&v)[DS])
+// codes as floats.  ROW16: 16 lanes hold the row.
+template <int DS, bool ROW16 = false> __device__ __forceinline__ float quantise_row_i8(float (&v)[DS])
 {
   float m = 0.0f;
 #pragma unroll
@@ -87,7 +92,7 @@ template <int DS> __device__ __forceinline__ float quantise_row_i8(float (&v)[DS
     const float a = fabsf(v[i]);
     if (__builtin_bit_cast(uint32_t, a) <= 0x7F7FFFFFu) m = fmaxf(m, a);
   }
-  m = half_wave_allmax(m);
+  m = ROW16 ? row16_max(m) : half_wave_allmax(m);
   const bool usable = __builtin_bit_cast(uint32_t, m) >= 0x00800000u;
   const float recip = usable ? 1.0f / m : 0.0f;
 #pragma unroll
@@ -116,6 +121,7 @@ struct AttnParams {
   float* part_override;        // split partials buffer when more rows than cache sequences are in flight
   float* ksc; float* vsc;      // int8 caches: row scales [seq][layer][kv_head][max_ctx]
   int64_t seq_rows, layer_row_off;
+  int64_t scale_row0;          // the per-head kernel: row of the scales where this layer of sequence seq0 begins
   int evict_sinks, evict_cap;  // cap > 0: only the first `sinks` positions and the latest cap - sinks stay cached
   const float* qn_gain; const float* kn_gain; float qk_eps;   // full-width RMSNorm of q and of k applied while they are read (null: rows are used as they are)
   unsigned* merge_cnt;         // decode steps: arrival counters [seq][head]; the work-group that completes the last slice merges (null: a merge launch follows)
@@ -128,6 +134,7 @@ struct AttnParams {
 // stores to be acknowledged and then counts itself in; the one that counts last reads all partials back at agent scope and
 // writes the finished rows.  The counter wraps to zero on the last arrival, so it needs no clearing between launches.  No
 // cache-wide fence is involved (a __threadfence per work-group measured several times the merge launch it saves).
+__device__ __forceinline__ float lane_value(float v, int lane) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane)); }
 __device__ __forceinline__ void part_store(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ float part_load(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
@@ -143,8 +150,8 @@ __device__ __forceinline__ float part_load(const float* p) { return __hip_atomic
 #if defined(__HIP_DEVICE_COMPILE__) && !defined(CAI_MERGE_RELACQ) && !defined(__gfx950__) && !defined(__gfx942__)
 #error "merge_if_last: the relaxed hand-over is only valid on gfx942 / gfx950; build with -DCAI_MERGE_RELACQ"
 #endif
-// heads qh0 .. qh0 + n_heads - 1 of sequence `seq`; every thread of the work-group calls it after its partial stores
-__device__ __forceinline__ void merge_if_last(const AttnParams& p, int seq, int qh0, int n_heads, int s_first, int n_active, int counter)
+// head qh of sequence `seq`; every thread of the work-group calls it after its partial stores
+__device__ __forceinline__ void merge_if_last(const AttnParams& p, int seq, int qh, int s_first, int n_active, int counter)
 {
   __shared__ int s_is_last;
   __builtin_amdgcn_s_waitcnt(0x0F70);           // vmcnt(0): this thread's partial stores have been acknowledged
@@ -161,30 +168,42 @@ __device__ __forceinline__ void merge_if_last(const AttnParams& p, int seq, int 
 #ifdef CAI_MERGE_RELACQ
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
 #endif
-  // One round trip per MB slices: every thread requests, per slice, its value and the slice's maximum and sum together (the
-  // latter two are the same addresses in all threads), then folds the slices in order with a running maximum.
-  constexpr int MB = 12;
-  const int hd = p.hd;
-  for (int o = threadIdx.x; o < n_heads * hd; o += blockDim.x) {
-    const int qh = qh0 + o / hd, d = o % hd;
-    const float* pt = p.part + (((int64_t)seq * p.q_heads + qh) * p.n_splits + s_first) * (hd + 2);
+  // One round trip per MB slices: every thread requests its value of each slice, lane u of every wave the maximum and the sum of slice u.  The
+  // slices are folded in order with a running maximum; what that scales by depends on the maxima alone, so lane u works it out for slice u
+  // and the fold reads it from there (every thread by itself, two exponentials a slice: half a microsecond at ten slices).
+  constexpr int MB = 12;                  // (at most the 16 lanes of a row)
+  const int hd = p.hd, lane = threadIdx.x & 63;
+  const float* const pt = p.part + (((int64_t)seq * p.q_heads + qh) * p.n_splits + s_first) * (hd + 2);
+  for (int o = threadIdx.x; o - lane < hd; o += blockDim.x) {      // (whole waves)
+    const int d = min(o, hd - 1);
     float A = 0.0f, L = 0.0f, M = -1e30f;
     for (int s0 = 0; s0 < n_active; s0 += MB) {
-      float v[MB], ms[MB], ls[MB];
+      float v[MB];
+      const float* pu = pt + (int64_t)min(s0 + min(lane, MB - 1), n_active - 1) * (hd + 2);
+      const float mu = part_load(pu + hd), lu = part_load(pu + hd + 1);
 #pragma unroll
-      for (int u = 0; u < MB; u++) {
-        const float* ps = pt + (int64_t)min(s0 + u, n_active - 1) * (hd + 2);
-        v[u] = part_load(ps + d); ms[u] = part_load(ps + hd); ls[u] = part_load(ps + hd + 1);
+      for (int u = 0; u < MB; u++) v[u] = part_load(pt + (int64_t)min(s0 + u, n_active - 1) * (hd + 2) + d);
+      const bool on = s0 + lane < n_active && lane < MB && lu > 0.0f;
+      float top = on ? mu : -1e30f;                                            // the running maximum up to this lane's slice
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const int t = __builtin_bit_cast(int, top);
+        top = fmaxf(top, __builtin_bit_cast(float, k == 0 ? __builtin_amdgcn_update_dpp(t, t, 0x111, 0xf, 0xf, false) : k == 1 ? __builtin_amdgcn_update_dpp(t, t, 0x112, 0xf, 0xf, false)
+                                                 : k == 2 ? __builtin_amdgcn_update_dpp(t, t, 0x114, 0xf, 0xf, false) : __builtin_amdgcn_update_dpp(t, t, 0x118, 0xf, 0xf, false)));   // row_shr
       }
+      top = fmaxf(top, M);
+      const float before = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, M), __builtin_bit_cast(int, top), 0x111, 0xf, 0xf, false));
+      const float c0 = expf(before - top), c1 = on ? expf(mu - top) : 0.0f;
 #pragma unroll
       for (int u = 0; u < MB; u++) {
-        if (s0 + u < n_active && ls[u] > 0.0f) {
-          const float mn = fmaxf(M, ms[u]), c0 = expf(M - mn), c1 = expf(ms[u] - mn);
-          A = fmaf(v[u], c1, A * c0); L = fmaf(ls[u], c1, L * c0); M = mn;
+        if (lane_value(on ? 1.0f : 0.0f, u) != 0.0f) {
+          const float e0 = lane_value(c0, u), e1 = lane_value(c1, u);
+          A = fmaf(v[u], e1, A * e0); L = fmaf(lane_value(lu, u), e1, L * e0);
         }
       }
+      M = lane_value(top, MB - 1);
     }
-    p.out[(int64_t)seq * p.out_stride + qh * hd + d] = L > 0.0f ? A * (1.0f / L) : 0.0f;
+    if (o < hd) p.out[(int64_t)seq * p.out_stride + qh * hd + d] = L > 0.0f ? A * (1.0f / L) : 0.0f;
   }
 }
 
@@ -929,176 +948,212 @@ __global__ __launch_bounds__(512) void attn_merge_kernel(const int32_t* hpos, co
 // ---- short caches: one work-group per (split, QUERY head).  The G heads of a group each re-read the slice (from
 //      L2: their work-groups are numbered so that they land on the same XCD), but no work-group loops over heads:
 //      with one wave per SIMD that loop is a chain of dependent DPP/exp/LDS latencies and dominated the step.
-//      Running state lives in registers; LDS is used once, for the meeting of the 8 half-waves. ----
-// The leading scalar arguments are the ones the first requests need (position, the step's q | k | v row, rotary frequencies,
-// grid geometry): they arrive preloaded in scalar registers (see the Makefile), so the position request leaves at once and the
-// rest of the parameter block is fetched while it is on its way.  hheads = query heads | KV heads << 16, hgeo = slices | head
-// width << 16.
-template <int DS, typename KV_T>
-__global__ __launch_bounds__(256) void attn_split_head_kernel(const int32_t* hpos, const float* hqkv, const float* htheta, const long long hqkv_stride,
-                                                              const int hheads, const int hgeo, const AttnParams p)
+//      Running state lives in registers; LDS is used once, for the meeting of the groups of 16 lanes. ----
+// What bounds it is round trips to memory, one after another: the step's q | k | v, the frequencies and the first 64 or 128 rows of the slice are
+// requested unconditionally and before anything waits, the rows before the position has arrived (a slice begins where it begins unless a
+// sliding window cuts it; rows past the live range are read as they lie and dropped).  With requests under branches and rows turned to floats
+// beside them it was four to eight round trips: 28 / 4 heads of 128, 600 float rows 10.0 us a launch (7.8 here), eight sequences of 200 half
+// rows 15.5 (9.6), 9 / 3 heads of 64 and 100 float rows 7.4 (4.8).
+// The leading scalar arguments are all that these first requests need: they arrive preloaded in scalar registers (see the Makefile), and
+// the rest of the parameter block is fetched while the requests are on their way.  hk, hv: this layer's keys and values of activation row 0's
+// sequence, hseq_rows: rows from one sequence to the next (0: all activation rows share one), hheads = query heads | KV heads << 16, hgeo =
+// slices | head width << 16, hsl = rows of a slice.
+// QN: q and k carry an RMS norm over their whole rows.
+// 16 lanes hold a row: of NV x 16 VW elements lane l has VW from 16 VW i + VW l on.  What is not waiting is instructions, one wave a SIMD: with
+// 32 lanes a row, sums of five steps and two scalar reads, 64 rows cost 1.5 us (0.5 here); sine and cosine are worked out once a wave
+// and not once a group, the exponentials of the meeting once a lane.  More waves (8, 16 a work-group) took longer to start and to meet
+// (100 half rows of 128: 5.5 us with four, 6.3, 9.6; 200: 7.2, 7.2, 9.6).  NCH: chunks of 64 rows on their way at once.
+template <int VW, int NV, typename KV_T, int NCH, bool QN>
+__global__ __launch_bounds__(256) void attn_split_head_kernel(const int32_t* hpos, const float* hqkv, const void* hk, const void* hv, const int hqkv_stride,
+                                                                  const int hheads, const int hgeo, const int hsl, const int hmax_ctx, const int hseq_rows, const AttnParams p)
 {
+  constexpr int DS = VW * NV, NG = 16;         // groups of 16 lanes: row j of the slice belongs to group j % NG
   const unsigned long long tl0 = timeline_now();
   const int q_heads = hheads & 0xffff, kv_heads = hheads >> 16, n_splits = hgeo & 0xffff, hd = hgeo >> 16;
   const int G = q_heads / kv_heads;
-  // linear id = item_lo + 8 * (h + G * item_hi), item = split + n_splits * kv_head: consecutive ids rotate over the XCDs
-  const int L = blockIdx.x, item = (L & 7) + 8 * ((L >> 3) / G), h = (L >> 3) % G;
-  if (item >= n_splits * kv_heads) return;
-  const int split = item % n_splits, g = item / n_splits, seq = blockIdx.y;
-  const int pos = hpos[seq];
-  // the query elements and the frequencies do not depend on the position: requested behind it, before anything waits
-  const int tid = threadIdx.x, hw = tid >> 5, l32 = tid & 31;
+  // linear id = item_lo + 8 * (h + G * item_hi), item = split + n_splits * kv_head: consecutive ids rotate over the XCDs, and a sequence
+  // starts on the XCD behind the last one's (four items a sequence would leave half of the chip idle)
+  const int L = blockIdx.x, seq = blockIdx.y, n_items = n_splits * kv_heads;
+  const int item = ((L - seq * n_items) & 7) + 8 * ((L >> 3) / G), h = (L >> 3) % G;
+  if (item >= n_items) return;
+  const int split = item % n_splits, g = item / n_splits;
+  // (a vector load: a scalar one would be waited for together with the parameter block, in front of the requests for the rows)
+  int lane0 = 0;
+  asm volatile("" : "+v"(lane0));
+  const int pos_v = hpos[seq + lane0];
+  const int tid = threadIdx.x, grp = tid >> 4, l16 = tid & 15;
   const int qw = q_heads * hd, kw = kv_heads * hd;
-  const int d0 = l32 * DS;
+  int dc[NV]; bool in_row[NV];                // (lanes beyond the head width read its last elements; the values are dropped)
+#pragma unroll
+  for (int i = 0; i < NV; i++) { const int d = 16 * VW * i + VW * l16; in_row[i] = d < hd; dc[i] = min(d, hd - VW); }
   const float* row = hqkv + (int64_t)seq * hqkv_stride;
-  float qraw[DS], qmate = 0.0f, th[(DS + 1) / 2];
-  {
-    const float* qp = row + (g * G + h) * hd;
+  using FV = row_vec<VW, float>;
+  using CV = row_vec<VW, KV_T>;
+  const float* const qp = row + (g * G + h) * hd; const float* const kp = row + qw + g * hd; const float* const vp = kp + kw;
+  FV qv[NV], kv[NV], vv[NV];
 #pragma unroll
-    for (int i = 0; i < DS; i++) qraw[i] = qp[min(d0 + i, hd - 1)];          // (lanes beyond the head width read its last element; the values are dropped)
-    if (DS == 1) qmate = qp[min(d0 ^ 1, hd - 1)];
-#pragma unroll
-    for (int i = 0; i < (DS + 1) / 2; i++) th[i] = htheta ? htheta[min(d0 + 2 * i, hd - 1) >> 1] : 0.0f;
-  }
-  const LiveRows lr = live_rows(p, pos);
-  const int len = lr.len, j_start = lr.j_start, slot = lr.slot;
-  const int s_begin = max(j_start, split * p.split_len), s_end = min(len, (split + 1) * p.split_len);
-  if (s_begin >= s_end) return;   // whole work-group leaves together, before any barrier
-  const int s_first = j_start / p.split_len, s_last = (len - 1) / p.split_len;
-  const int n_active = s_last - s_first + 1;
-  timeline_put(p.timeline, 0, tl0);
-  timeline_stamp(p.timeline, 1);
+  for (int i = 0; i < NV; i++) { qv[i] = *reinterpret_cast<const FV*>(qp + dc[i]); kv[i] = *reinterpret_cast<const FV*>(kp + dc[i]); vv[i] = *reinterpret_cast<const FV*>(vp + dc[i]); }
 
-  KV_T* kc = reinterpret_cast<KV_T*>(p.kc) + (seq * p.seq_mul + p.seq0) * p.seq_elems + p.layer_off + (int64_t)g * p.max_ctx * hd;
-  KV_T* vc = reinterpret_cast<KV_T*>(p.vc) + (seq * p.seq_mul + p.seq0) * p.seq_elems + p.layer_off + (int64_t)g * p.max_ctx * hd;
-
+  const int64_t plane_row = (int64_t)seq * hseq_rows + (int64_t)g * hmax_ctx;
+  KV_T* const kc = reinterpret_cast<KV_T*>(const_cast<void*>(hk)) + plane_row * hd;
+  KV_T* const vc = reinterpret_cast<KV_T*>(const_cast<void*>(hv)) + plane_row * hd;
   // int8 cache: codes enter the dot products as they are; the K row scale multiplies the finished score and the V row
   // scale the softmax weight (neural/neural.cl:2639-2640, 2683-2684), so nothing is dequantised per element
   constexpr bool I8 = sizeof(KV_T) == 1;
-  const float* ksc = nullptr; const float* vsc = nullptr;
-  if (I8) {
-    const int64_t r0 = (seq * p.seq_mul + p.seq0) * p.seq_rows + p.layer_row_off + (int64_t)g * p.max_ctx;
-    ksc = p.ksc + r0; vsc = p.vsc + r0;
-  }
-
   constexpr int PCH = 4;
-  struct Chunk { float k[PCH][DS], v[PCH][DS], ks[PCH], vs[PCH]; };
-  Chunk cA = {}, cB = {};
-  auto load_chunk = [&](Chunk& ch, int j0) {
-    if (j0 >= s_end || d0 >= hd) return;       // lanes beyond the head width keep their zeros
+  struct Chunk { CV k[PCH][NV], v[PCH][NV]; float ks[PCH], vs[PCH]; };
+  Chunk ch[NCH];
+  auto load_k = [&](Chunk& ch, int j0, int last) {
 #pragma unroll
-    for (int c = 0; c < PCH; c++) {
-      const int j = min(j0 + 8 * c, s_end - 1);
-      // (the slot of the row being appended may hold stale values: reduce_chunk replaces it from registers)
-      load_row_vec<DS, KV_T>(kc + (int64_t)j * hd + d0, ch.k[c]);
-      load_row_vec<DS, KV_T>(vc + (int64_t)j * hd + d0, ch.v[c]);
-      if (I8) { ch.ks[c] = ksc[j]; ch.vs[c] = vsc[j]; }
+    for (int c = 0; c < PCH; c++)
+#pragma unroll
+      for (int i = 0; i < NV; i++) ch.k[c][i] = *reinterpret_cast<const CV*>(kc + (int64_t)min(j0 + NG * c, last) * hd + dc[i]);
+  };
+  auto load_v = [&](Chunk& ch, int j0, int last) {
+#pragma unroll
+    for (int c = 0; c < PCH; c++)
+#pragma unroll
+      for (int i = 0; i < NV; i++) ch.v[c][i] = *reinterpret_cast<const CV*>(vc + (int64_t)min(j0 + NG * c, last) * hd + dc[i]);
+  };
+  const int split_len = hsl & 0xffff, row0 = split * split_len;
+  const bool ahead = !(hsl >> 16);                               // no sliding window
+  const int last0 = ahead ? min(row0 + split_len, hmax_ctx) - 1 : row0;   // (a window's first rows are asked for again once the position is known)
+#pragma unroll
+  for (int n = 0; n < NCH; n++) load_k(ch[n], row0 + grp + n * NG * PCH, last0);
+  const float th = (p.theta ? p.theta : row)[min(tid & 63, (hd >> 1) - 1)];      // lane a turns pair a (no rotation: any readable address)
+#pragma unroll
+  for (int n = 0; n < NCH; n++) load_v(ch[n], row0 + grp + n * NG * PCH, last0);
+  float* const ksc = p.ksc + plane_row + p.scale_row0; float* const vsc = p.vsc + plane_row + p.scale_row0;      // (int8 only)
+  auto load_scales = [&](Chunk& ch, int j0, int last) {
+    if constexpr (I8) {
+#pragma unroll
+      for (int c = 0; c < PCH; c++) { const int j = min(j0 + NG * c, last); ch.ks[c] = ksc[j]; ch.vs[c] = vsc[j]; }
     }
   };
-  // Requests return in the order they were issued: the step's own q, k, v elements and the rotary frequencies go out first, the
-  // cached rows behind them, so that the rotation (sine and cosine of an exact angle) runs while the rows are on their way
-  // instead of after them.
-  const bool owns_new = !p.appended && slot >= s_begin && slot < s_end;
-  float kraw[DS], vraw[DS], kmate = 0.0f;
-  {
-    const float* kp = row + qw + g * hd; const float* vp = row + qw + kw + g * hd;
 #pragma unroll
-    for (int i = 0; i < DS; i++) {
-      const int d = min(d0 + i, hd - 1);
-      kraw[i] = owns_new ? kp[d] : 0.0f; vraw[i] = owns_new ? vp[d] : 0.0f;
-    }
-    if (DS == 1) kmate = owns_new ? kp[min(d0 ^ 1, hd - 1)] : 0.0f;
+  for (int n = 0; n < NCH; n++) load_scales(ch[n], row0 + grp + n * NG * PCH, last0);
+  FV qg[NV], kg[NV];
+  if constexpr (QN) {
+#pragma unroll
+    for (int i = 0; i < NV; i++) { qg[i] = *reinterpret_cast<const FV*>(p.qn_gain + (g * G + h) * hd + dc[i]); kg[i] = *reinterpret_cast<const FV*>(p.kn_gain + g * hd + dc[i]); }
   }
-  load_chunk(cA, s_begin + hw);
-  load_chunk(cB, s_begin + hw + 8 * PCH);
+  __builtin_amdgcn_sched_barrier(0);      // (nothing waits before the last of these requests is out)
+  const int pos = __builtin_amdgcn_readfirstlane(pos_v);
+  const LiveRows lr = live_rows(p, pos);
+  const int len = lr.len, j_start = lr.j_start, slot = lr.slot;
+  const int s_begin = max(j_start, row0), s_end = min(len, row0 + split_len);
+  if (s_begin >= s_end) return;   // whole work-group leaves together, before any barrier
+  const int s_first = j_start / split_len, s_last = (len - 1) / split_len;
+  const int n_active = s_last - s_first + 1;
+  timeline_put(p.timeline, 0, tl0);
+  timeline_stamp(p.timeline, 1);
+  auto load_chunk = [&](Chunk& ch, int j0) { load_k(ch, j0, s_end - 1); load_v(ch, j0, s_end - 1); load_scales(ch, j0, s_end - 1); };
+  if (!ahead)
+#pragma unroll
+    for (int n = 0; n < NCH; n++) load_chunk(ch[n], s_begin + grp + n * NG * PCH);
+  const bool owns_new = !p.appended && slot >= s_begin && slot < s_end;
+  const int skip = owns_new ? slot : -1;        // the row being appended: what lies in the cache there is stale
 
   // Full-width RMSNorm of q and k (neural/neuralpretrained.pas:16511-16530) folded into this kernel: every work-group
   // sums the squares of the whole q and k rows itself (same order as the stand-alone kernel: strided per thread, wave
   // totals, (w0 + w1) + (w2 + w3)) and scales the elements it reads.
   float inv_q = 1.0f, inv_k = 1.0f;
-  if (p.qn_gain) {
+  if constexpr (QN) {
     __shared__ float nred[8];
-    float sq = 0.0f, sk = 0.0f;
-    for_strided8(row, tid, qw, 256, [&](float v, int) { sq = fmaf(v, v, sq); });
-    for_strided8(row + qw, tid, kw, 256, [&](float v, int) { sk = fmaf(v, v, sk); });
-    sq = wave_sum(sq); sk = wave_sum(sk);
-    if ((tid & 63) == 63) { nred[tid >> 6] = sq; nred[4 + (tid >> 6)] = sk; }
+    {
+      float sq = 0.0f, sk = 0.0f;
+      for_strided8(row, tid, qw, 256, [&](float v, int) { sq = fmaf(v, v, sq); });
+      for_strided8(row + qw, tid, kw, 256, [&](float v, int) { sk = fmaf(v, v, sk); });
+      sq = wave_sum(sq); sk = wave_sum(sk);
+      if ((tid & 63) == 63) { nred[tid >> 6] = sq; nred[4 + (tid >> 6)] = sk; }
+    }
     __syncthreads();
     inv_q = 1.0f / sqrtf(((nred[0] + nred[1]) + (nred[2] + nred[3])) / (float)qw + p.qk_eps);
     inv_k = 1.0f / sqrtf(((nred[4] + nred[5]) + (nred[6] + nred[7])) / (float)kw + p.qk_eps);
   }
-  float rs[(DS + 1) / 2], rc[(DS + 1) / 2];
+  float rs[DS / 2], rc[DS / 2];
+  {
+    float sn = 0.0f, cs = 1.0f;
+    if (p.theta) sincosf((float)pos * th, &sn, &cs);       // (one pair a lane, and from there to the lanes that need it)
 #pragma unroll
-  for (int i = 0; i < (DS + 1) / 2; i++) {
-    rs[i] = 0.0f; rc[i] = 1.0f;
-    const int d = d0 + 2 * i;
-    if (p.theta && d < hd) { const float angle = (float)pos * th[i]; sincosf(angle, &rs[i], &rc[i]); }
+    for (int i = 0; i < DS / 2; i++) {
+      const int from = (dc[2 * i / VW] + 2 * i % VW) << 1;       // 4 bytes a lane
+      rs[i] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(from, __builtin_bit_cast(int, sn)));
+      rc[i] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(from, __builtin_bit_cast(int, cs)));
+    }
   }
-  // raw elements (own DS, for DS = 1 also the pair's other element) -> optional RMSNorm gain -> optional rotation
-  auto finish_rot = [&](const float (&raw)[DS], float mate_raw, float (&o)[DS], bool rotate, const float* gain, float inv) {
-    auto elem = [&](float v, int d) { return d < hd ? (gain ? gain[d] * (v * inv) : v) : 0.0f; };
-    if (DS >= 2) {
+  // raw elements -> RMSNorm gain of QN -> optional rotation
+  auto finish_rot = [&](const FV (&raw)[NV], const FV (&gain)[NV], float inv, float (&o)[DS]) {
 #pragma unroll
-      for (int i = 0; i < DS; i += 2) {
-        const int d = d0 + i;
-        const float x0 = elem(raw[i], d), x1 = elem(raw[i + (DS > 1 ? 1 : 0)], d + 1);
-        if (rotate) { o[i] = rc[i / 2] * x0 - rs[i / 2] * x1; o[i + (DS > 1 ? 1 : 0)] = rs[i / 2] * x0 + rc[i / 2] * x1; }
-        else { o[i] = x0; o[i + (DS > 1 ? 1 : 0)] = x1; }
-      }
-    } else {
-      const int d = d0;
-      const float own = elem(raw[0], d), mate = elem(mate_raw, d ^ 1);
-      if (rotate) o[0] = (d & 1) ? (rs[0] * mate + rc[0] * own) : (rc[0] * own - rs[0] * mate);
-      else o[0] = own;
+    for (int i = 0; i < DS; i += 2) {
+      const int n = i / VW, e = i % VW;
+      float x0 = raw[n][e], x1 = raw[n][e + 1];
+      if constexpr (QN) { x0 = gain[n][e] * (x0 * inv); x1 = gain[n][e + 1] * (x1 * inv); }
+      if (!in_row[n]) x0 = x1 = 0.0f;
+      o[i] = x0; o[i + 1] = x1;
+      if (p.theta) { o[i] = rc[i / 2] * x0 - rs[i / 2] * x1; o[i + 1] = rs[i / 2] * x0 + rc[i / 2] * x1; }
     }
   };
-  float q[DS], knew[DS], vnew[DS], acc[DS];
-  finish_rot(qraw, qmate, q, p.theta != nullptr, p.qn_gain ? p.qn_gain + (g * G + h) * hd : nullptr, inv_q);
+  float q[DS], acc[DS], m = -1e30f, l = 0.0f;
+  finish_rot(qv, qg, inv_q, q);
 #pragma unroll
-  for (int i = 0; i < DS; i++) { acc[i] = 0.0f; knew[i] = 0.0f; vnew[i] = 0.0f; }
-  // every work-group whose slice holds `pos` keeps the new row in registers; the group's first head appends it
-  float knew_s = 1.0f, vnew_s = 1.0f;
+  for (int i = 0; i < DS; i++) acc[i] = 0.0f;
+  auto score = [&](float dot, float k_scale) {
+    const float s = row16_sum(dot) * (I8 ? k_scale * p.inv_sqrt : p.inv_sqrt);
+    return p.softcap > 0.0f ? p.softcap * tanhf(s / p.softcap) : s;
+  };
+  // The work-group whose slice holds the new row has it in registers: its first group starts from it, and the group's first head appends it
   if (owns_new) {
-    finish_rot(kraw, kmate, knew, p.theta != nullptr, p.kn_gain ? p.kn_gain + g * hd : nullptr, inv_k);
-    finish_rot(vraw, 0.0f, vnew, false, nullptr, 1.0f);
-    if constexpr (I8) {
-      knew_s = quantise_row_i8<DS>(knew);
-      vnew_s = quantise_row_i8<DS>(vnew);
-      if (h == 0 && hw == 0) {
+    float knew[DS], vnew[DS], knew_s = 1.0f, vnew_s = 1.0f;
+    finish_rot(kv, kg, inv_k, knew);
 #pragma unroll
-        for (int i = 0; i < DS; i++)
-          if (d0 + i < hd) { kc[(int64_t)slot * hd + d0 + i] = (int8_t)knew[i]; vc[(int64_t)slot * hd + d0 + i] = (int8_t)vnew[i]; }
-        if (l32 == 0) { p.ksc[(ksc - p.ksc) + slot] = knew_s; p.vsc[(vsc - p.vsc) + slot] = vnew_s; }
-      }
-    } else {
+    for (int i = 0; i < DS; i++) vnew[i] = in_row[i / VW] ? vv[i / VW][i % VW] : 0.0f;
+    if constexpr (I8) { knew_s = quantise_row_i8<DS, true>(knew); vnew_s = quantise_row_i8<DS, true>(vnew); }
+    if (h == 0 && grp == 0) {
 #pragma unroll
-      for (int i = 0; i < DS; i++) {
-        vnew[i] = kv_to_float<KV_T>(kv_from_float<KV_T>(vnew[i]));
-        knew[i] = kv_to_float<KV_T>(kv_from_float<KV_T>(knew[i]));
-        if (h == 0 && hw == 0 && d0 + i < hd) {
-          kc[(int64_t)slot * hd + d0 + i] = kv_from_float<KV_T>(knew[i]);
-          vc[(int64_t)slot * hd + d0 + i] = kv_from_float<KV_T>(vnew[i]);
+      for (int i = 0; i < DS; i++)
+        if (in_row[i / VW]) {
+          const int64_t at = (int64_t)slot * hd + dc[i / VW] + i % VW;
+          if constexpr (I8) { kc[at] = (int8_t)knew[i]; vc[at] = (int8_t)vnew[i]; }
+          else { kc[at] = kv_from_float<KV_T>(knew[i]); vc[at] = kv_from_float<KV_T>(vnew[i]); }
         }
-      }
+      if constexpr (I8) if (l16 == 0) { ksc[slot] = knew_s; vsc[slot] = vnew_s; }
+    }
+    float dot = 0.0f;
+#pragma unroll
+    for (int i = 0; i < DS; i++) {
+      if constexpr (!I8) { knew[i] = kv_to_float<KV_T>(kv_from_float<KV_T>(knew[i])); vnew[i] = kv_to_float<KV_T>(kv_from_float<KV_T>(vnew[i])); }
+      dot = fmaf(q[i], knew[i], dot);
+    }
+    const float s = score(dot, knew_s);
+    if (grp == 0) {
+      m = s; l = 1.0f;
+#pragma unroll
+      for (int i = 0; i < DS; i++) acc[i] = I8 ? vnew_s * vnew[i] : vnew[i];
     }
   }
-  float m = -1e30f, l = 0.0f;
   timeline_stamp_after(p.timeline, 4, q[0]);
-  auto reduce_chunk = [&](Chunk& ch, int j0) {
+  auto reduce_chunk = [&](const Chunk& ch, int j0) {
     float sc[PCH], cmax = -1e30f;
 #pragma unroll
     for (int c = 0; c < PCH; c++) {
-      if (owns_new && min(j0 + 8 * c, s_end - 1) == slot) {
+      float kf[DS], dot = 0.0f;
 #pragma unroll
-        for (int i = 0; i < DS; i++) { ch.k[c][i] = knew[i]; ch.v[c][i] = vnew[i]; }
-        if (I8) { ch.ks[c] = knew_s; ch.vs[c] = vnew_s; }
-      }
-      float s = 0.0f;
+      for (int i = 0; i < NV; i++) row_floats<VW, KV_T>(ch.k[c][i], kf + VW * i);
 #pragma unroll
-      for (int i = 0; i < DS; i++) s = fmaf(q[i], ch.k[c][i], s);
-      s = half_wave_allsum(s) * (I8 ? ch.ks[c] * p.inv_sqrt : p.inv_sqrt);
-      if (p.softcap > 0.0f) s = p.softcap * tanhf(s / p.softcap);
-      sc[c] = (j0 + 8 * c < s_end) ? s : -1e30f;
+      for (int i = 0; i < DS; i++) dot = fmaf(q[i], kf[i], dot);       // (q is 0 beyond the head width)
+      sc[c] = row16_sum(dot) * (I8 ? ch.ks[c] * p.inv_sqrt : p.inv_sqrt);
+    }
+    if (p.softcap > 0.0f) {
+#pragma unroll
+      for (int c = 0; c < PCH; c++) sc[c] = p.softcap * tanhf(sc[c] / p.softcap);
+    }
+    bool live[PCH];
+#pragma unroll
+    for (int c = 0; c < PCH; c++) {
+      const int j = j0 + NG * c;
+      live[c] = j < s_end && j != skip;
+      if (!live[c]) sc[c] = -1e30f;           // (whatever a row that is not live holds ends here and at its values below)
       cmax = fmaxf(cmax, sc[c]);
     }
     const float mn = fmaxf(m, cmax), corr = expf(m - mn);
@@ -1107,44 +1162,51 @@ __global__ __launch_bounds__(256) void attn_split_head_kernel(const int32_t* hpo
     for (int i = 0; i < DS; i++) acc[i] *= corr;
 #pragma unroll
     for (int c = 0; c < PCH; c++) {
-      const float pj = (j0 + 8 * c < s_end) ? expf(sc[c] - mn) : 0.0f;
+      const float pj = live[c] ? expf(sc[c] - mn) : 0.0f;
       lsum += pj;
-      const float pv = I8 ? pj * ch.vs[c] : pj;
+      const float pv = I8 ? (live[c] ? pj * ch.vs[c] : 0.0f) : pj;
+      float vf[DS];
 #pragma unroll
-      for (int i = 0; i < DS; i++) acc[i] = fmaf(pv, ch.v[c][i], acc[i]);
+      for (int i = 0; i < NV; i++) row_floats<VW, KV_T>(live[c] ? ch.v[c][i] : CV{}, vf + VW * i);
+#pragma unroll
+      for (int i = 0; i < DS; i++) acc[i] = fmaf(pv, vf[i], acc[i]);
     }
     l = l * corr + lsum; m = mn;
   };
-  for (int j0 = s_begin + hw; j0 < s_end; j0 += 16 * PCH) {
-    reduce_chunk(cA, j0);
-    if (j0 + 16 * PCH < s_end) load_chunk(cA, j0 + 16 * PCH);
-    if (j0 + 8 * PCH < s_end) {
-      reduce_chunk(cB, j0 + 8 * PCH);
-      if (j0 + 24 * PCH < s_end) load_chunk(cB, j0 + 24 * PCH);
-    }
+  for (int b = s_begin; b < s_end; b += NCH * NG * PCH) {
+#pragma unroll
+    for (int n = 0; n < NCH; n++)
+      if (b + n * NG * PCH < s_end) {
+        reduce_chunk(ch[n], b + grp + n * NG * PCH);
+        if (b + (n + NCH) * NG * PCH < s_end) load_chunk(ch[n], b + grp + (n + NCH) * NG * PCH);
+      }
   }
 
-  // ---- meeting of the 8 half-waves ----
+  // ---- meeting of the groups ----
   timeline_stamp(p.timeline, 5);
-  __shared__ float sm[8], sl[8];
-  __shared__ float sacc[8][32 * DS];
-  if (l32 == 0) { sm[hw] = m; sl[hw] = l; }
+  __shared__ float sm[NG], sl[NG];
+  __shared__ __attribute__((aligned(16))) float sacc[NG][16 * DS];
+  if (l16 == 0) { sm[grp] = m; sl[grp] = l; }
 #pragma unroll
-  for (int i = 0; i < DS; i++) sacc[hw][d0 + i] = acc[i];
+  for (int i = 0; i < DS; i++) sacc[grp][16 * VW * (i / VW) + VW * l16 + i % VW] = acc[i];
   __syncthreads();
-  if (tid < hd) {
-    const int d = tid;
-    float M = -1e30f;
+  if ((tid & ~63) < hd) {                                    // (whole waves)
+    const int d = min(tid, hd - 1), lane = tid & 63;
+    const float mw = lane < NG ? sm[lane] : -1e30f, lw = lane < NG ? sl[lane] : 0.0f;      // group `lane`'s maximum and sum
+    const float Mr = row16_max(mw);
+    float M = lane_value(Mr, 0);
 #pragma unroll
-    for (int w = 0; w < 8; w++) M = fmaxf(M, sm[w]);
+    for (int r = 1; r < NG / 16; r++) M = fmaxf(M, lane_value(Mr, 16 * r));
+    const float ew = lw > 0.0f ? expf(mw - M) : 0.0f;
     float Ls = 0.0f, A = 0.0f;
 #pragma unroll
-    for (int w = 0; w < 8; w++) {
-      const float e = sl[w] > 0.0f ? expf(sm[w] - M) : 0.0f;
-      Ls = fmaf(sl[w], e, Ls); A = fmaf(sacc[w][d], e, A);
+    for (int w = 0; w < NG; w++) {
+      const float e = lane_value(ew, w);
+      Ls = fmaf(lane_value(lw, w), e, Ls); A = fmaf(sacc[w][d], e, A);
     }
     const int qh = g * G + h;
-    if (n_active == 1) {
+    if (tid >= hd) {
+    } else if (n_active == 1) {
       p.out[(int64_t)seq * p.out_stride + qh * hd + d] = Ls > 0.0f ? A * (1.0f / Ls) : 0.0f;
     } else {
       float* pt = p.part + (((int64_t)seq * p.q_heads + qh) * p.n_splits + split) * (hd + 2);
@@ -1152,7 +1214,7 @@ __global__ __launch_bounds__(256) void attn_split_head_kernel(const int32_t* hpo
       else { pt[d] = A; if (d == 0) { pt[hd] = M; pt[hd + 1] = Ls; } }
     }
   }
-  if (n_active > 1 && p.merge_cnt) merge_if_last(p, seq, g * G + h, 1, s_first, n_active, seq * p.kv_heads * 8 + g * G + h);
+  if (n_active > 1 && p.merge_cnt) merge_if_last(p, seq, g * G + h, s_first, n_active, seq * p.kv_heads * 8 + g * G + h);
   timeline_stamp(p.timeline, 7);
 }
 
@@ -1164,13 +1226,29 @@ static int launch_split_head(const AttnParams& p0, int n_seq, hipStream_t st)
   const int items = p.n_splits * p.kv_heads;
   const dim3 grid(8 * G * ((items + 7) / 8), n_seq);
   p.timeline = timeline_next((int)(grid.x * grid.y));
-  const int hheads = p.q_heads | p.kv_heads << 16, hgeo = p.n_splits | p.hd << 16;
-  if (p.q_heads > 0xffff || p.kv_heads > 0x7fff || p.n_splits > 0xffff) return set_error(CAI_ERR_UNSUPPORTED, "attention: %d query heads, %d slices", p.q_heads, p.n_splits);
-  const long long qs = (long long)p.qkv_stride;
-  if (p.hd <= 32) hipLaunchKernelGGL((attn_split_head_kernel<1, KV_T>), grid, dim3(256), 0, st, p.pos, (const float*)p.qkv, p.theta, qs, hheads, hgeo, p);
-  else if (p.hd <= 64) hipLaunchKernelGGL((attn_split_head_kernel<2, KV_T>), grid, dim3(256), 0, st, p.pos, (const float*)p.qkv, p.theta, qs, hheads, hgeo, p);
-  else if (p.hd <= 128) hipLaunchKernelGGL((attn_split_head_kernel<4, KV_T>), grid, dim3(256), 0, st, p.pos, (const float*)p.qkv, p.theta, qs, hheads, hgeo, p);
-  else return set_error(CAI_ERR_UNSUPPORTED, "attention: head_dim %d > 128", p.hd);
+  const int hheads = p.q_heads | p.kv_heads << 16, hgeo = p.n_splits | p.hd << 16, hsl = p.split_len | (p.window > 0 ? 1 << 16 : 0);
+  const int64_t seq_rows = p.seq_mul ? p.seq_elems / p.hd : 0;
+  if (p.q_heads > 0xffff || p.kv_heads > 0x7fff || p.n_splits > 0xffff || p.split_len > 0xffff || seq_rows > 0x7fffffff || p.qkv_stride > 0x7fffffff)
+    return set_error(CAI_ERR_UNSUPPORTED, "attention: %d query heads, %d slices of %d rows, sequences of %lld rows", p.q_heads, p.n_splits, p.split_len, (long long)seq_rows);
+  if (p.hd > 128) return set_error(CAI_ERR_UNSUPPORTED, "attention: head_dim %d > 128", p.hd);
+  const int64_t at = (p.seq0 * p.seq_elems + p.layer_off) * (int64_t)sizeof(KV_T);
+  const void* hk = (const char*)p.kc + at; const void* hv = (const char*)p.vc + at;
+  p.scale_row0 = p.seq0 * p.seq_rows + p.layer_row_off;
+  auto put = [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, p.pos, (const float*)p.qkv, hk, hv, (int)p.qkv_stride, hheads, hgeo, hsl, p.max_ctx, (int)seq_rows, p);
+  };
+  auto go = [&](auto vw, auto nv) {
+    constexpr int VW = decltype(vw)::value, NV = decltype(nv)::value;
+    // a slice of up to 64 rows is one chunk; longer ones have 128 rows on their way (256: 0.1 us less at 200 rows, 0.5 more at 100)
+    constexpr int LONG = 2;
+    if (p.split_len <= 64) { if (p.qn_gain) put(attn_split_head_kernel<VW, NV, KV_T, 1, true>); else put(attn_split_head_kernel<VW, NV, KV_T, 1, false>); }
+    else if (p.qn_gain) put(attn_split_head_kernel<VW, NV, KV_T, LONG, true>);
+    else put(attn_split_head_kernel<VW, NV, KV_T, LONG, false>);
+  };
+  using std::integral_constant;
+  if (p.hd > 64) go(integral_constant<int, 4>(), integral_constant<int, 2>());       // (widths past 64 are whole fours, all are even)
+  else if (p.hd % 4 == 0) go(integral_constant<int, 4>(), integral_constant<int, 1>());
+  else go(integral_constant<int, 2>(), integral_constant<int, 2>());
   return CAI_OK;
 }
 
@@ -1729,7 +1807,13 @@ int launch_attn_step(cai_kv_s* kv, int layer, float* qkv, int64_t qkv_stride, in
   const int group_min = c.n_cu;   // smallest grid that fills the chip with one work-group per (slice, KV head)
   // (a cache short enough to be ONE slice may be up to 2048 rows long: the grouped kernel's per-slice score arrays in LDS are
   // sized for ordinary slices, the per-head kernel keeps its state in registers)
-  const bool grouped = (kv->head_dim & 7) == 0 && p.split_len <= 256 && n_seq * kv->kv_heads * p.n_splits >= group_min;
+  // Few work-groups either way, or heads that share nothing (half and int8 rows; the float rows of many sequences are better off where requests
+  // stay in flight), are better off with the per-head kernel, which needs no merge launch and norms q and k itself.  us a launch per head |
+  // grouped: 16 / 16 heads of 128, float, 300 rows 7.3 | 10.0, 4000 16.6 | 18.1; half, 300 7.2 | 9.6; 16 / 16 of 64, 4000 10.7 | 15.6; a block of a
+  // decoder with four sequences, 16 / 16, half, 300 rows 46.3 | 51.8, eight 54.1 | 57.9; 28 / 4 heads, four 53.1 | 49.1.
+  const int64_t per_head_wgs = (int64_t)n_seq * q_heads * p.n_splits;
+  const bool per_head = !prompt_rows && p.n_splits <= 16 && (per_head_wgs <= 512 || (q_heads == kv->kv_heads && kv->dtype != CAI_KV_F32 && per_head_wgs <= 2048));
+  const bool grouped = !per_head && (kv->head_dim & 7) == 0 && p.split_len <= 256 && n_seq * kv->kv_heads * p.n_splits >= group_min;
   // The per-head kernel merges its slices itself (one work-group per head does a head's merge).  A prompt has more rows in
   // flight than the counters cover, and in the per-KV-head kernel the last arriver would fold a whole group of heads over
   // many slices alone (32B shape, 33 slices x 5 heads: 37.7 us against 30.7 us with the merge launch): those keep the launch.

@@ -50,6 +50,28 @@ def test_long_context_many_splits_and_f16_cache():
                 assert np.max(np.abs(got - want[pos])) < tol, (dtype, pos)
 
 
+@pytest.mark.parametrize("hq,hkv,dk,ctx", [(3, 1, 2, 150), (4, 2, 34, 300), (4, 4, 62, 300), (6, 2, 64, 256), (2, 2, 68, 140), (28, 4, 128, 300), (5, 1, 100, 1040), (3, 3, 128, 1100)])
+@pytest.mark.parametrize("dtype", ["f32", "f16", "i8"])
+def test_rows_at_the_edges_of_chunks(hq, hkv, dk, ctx, dtype):
+    """Rows that end before, at and behind 16, 64, 128 and a slice; widths that leave lanes idle; slices of one chunk and more.  The cache held
+    NaNs and infinities before: rows past the live range are read ahead and must not be seen."""
+    from helpers.device import dev
+    cai = dev()
+    rng = np.random.default_rng(hq * 1000 + dk)
+    width = (hq + 2 * hkv) * dk
+    n = min(ctx, 270)
+    kv = cai.KVCache(1, hkv, dk, ctx, {"f32": cai.KV_F32, "f16": cai.KV_F16, "i8": cai.KV_I8}[dtype])
+    for p in range(n):
+        kv.attn_decode(0, np.full(width, np.nan if p % 2 else np.inf, np.float32), hq)
+    kv.reset()
+    rows = rng.standard_normal((n, width)).astype(np.float32)
+    want = oracle_run_i8(rows, hq, hkv, dk, ctx)[0] if dtype == "i8" else oracle_run(rows, hq, hkv, dk, ctx, 0, int(dtype == "f16"))
+    for p in range(n):
+        got = kv.attn_decode(0, rows[p], hq)
+        if p + 1 in (1, 2, 15, 16, 17, 31, 32, 33, 63, 64, 65, 66, 127, 128, 129, 130, 191, 192, 193, 255, 256, 257, n):
+            assert np.max(np.abs(got - want[p])) < 1e-5, p + 1
+
+
 def test_softcap():
     from helpers.device import dev
     cai = dev()
