@@ -153,7 +153,7 @@ static int enqueue_step(cai_decoder_s* d, int n_b, int seq0, unsigned classes = 
     for (int sl : slots) if (!nb_supported(L.w[sl]) || L.w[sl]->qtype == CAI_I8ROW) return false;   // (per-row int8 products need the plain reduction for their row scale)
     return true;
   };
-  // ... and when all six are Q4_K of widths the register-resident form takes, a linear layer is ONE launch: activations
+  // ... and when all six are Q4_K or Q6_K of widths the register-resident form takes, a linear layer is ONE launch: activations
   // quantised by the product itself, norm factor, bias, residual and SwiGLU in its epilogue (CAIHIP_SMALL_BATCH_PLANES=1
   // keeps the form with activation planes and slice partials)
   static const bool ra_on = []() { const char* e = getenv("CAIHIP_SMALL_BATCH_PLANES"); return !(e && e[0] == '1'); }();
@@ -271,8 +271,17 @@ static int enqueue_step(cai_decoder_s* d, int n_b, int seq0, unsigned classes = 
   tl_cls = 6;
   if (classes & 64u) {
     cai_qw_s* hw = d->head ? d->head : d->embed;   // tied head (neural/neuralpretrained.pas:15555-)
+    const cai_qw_s* hwc = hw;
+    // (Q6_K: one launch of 123 us for 152064 x 3584 and eight sequences, where planes, product and reduction are 143)
+    if (ra_on && n_b >= 2 && n_b <= 8 && hw->qtype == CAI_Q6_K && ra_supported(&hwc, 1, true, 0)) {
+      if (down_pending && (rc = nb_prep_residual(d->x, dm, nullptr, 0.0f, dm, n_b))) return rc;
+      const int zero = 0;
+      if ((rc = ra_gemm(&hwc, &zero, 1, n_b, d->x, dm, d->final_norm, c.eps, 0, d->logits, c.vocab, nullptr))) return rc;
+      launch_argmax(d->logits, c.vocab, n_b, d->d_argmax, d->am_v, d->am_i);
+      return CAI_OK;
+    }
     if (n_b >= 2 && nb_supported(hw)) {
-      const int zero = 0; const cai_qw_s* hwc = hw;
+      const int zero = 0;
       if (down_pending) rc = nb_prep_residual(d->x, dm, d->final_norm, c.eps, dm, n_b);
       else rc = nb_prep_plain(d->x, dm, d->final_norm, c.eps, dm, n_b);
       if (rc || (rc = nb_gemm(&hwc, &zero, 1, n_b)) || (rc = nb_reduce(d->logits, c.vocab, nullptr))) return rc;

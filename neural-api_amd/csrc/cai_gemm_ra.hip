@@ -1,10 +1,11 @@
-// Small-batch (2..8 tokens) Q4_K linear layer on the matrix cores, register-resident form: the decode step of a few sequences
+// Small-batch (2..8 tokens) Q4_K and Q6_K linear layer on the matrix cores, register-resident form: the decode step of a few sequences
 // with ONE launch per linear layer (no activation pre-pass, no slice reduction launch).
 //
 // The arithmetic is that of gemm_q4k_nb (cai_gemm_nb.hip): A operand = sc_j * q (exact in f16), B operand = the activations
 // of up to 8 tokens, scaled per (token, 256-block) by a power of two and split hi + lo into two f16 = the 16 columns of
 // v_mfma_f32_16x16x32_f16, one more MFMA per row set and super-block for the - dmin * mn_j * sum_j(x) term
-// (Q4_K: neural/neuralgguf.pas:472-514).  What differs is who holds what:
+// (Q4_K: neural/neuralgguf.pas:472-514); for Q6_K that of gemm_q6k_nb: one v_mfma_f32_16x16x16_f16 a scale group of 16 weights, activations
+// as the rows of the result, so that a lane multiplies by the scale it loaded itself.  What differs is who holds what:
 //   * a WAVE owns two super-blocks (512 columns) of EVERY row its work-group walks, so the B operands of its 16 MFMA steps
 //     never change: it reads its 8 x 512 activations as fp32 once, applies the RMSNorm gain, finds the block scales, splits
 //     hi + lo and keeps the operands in 64 registers for the whole launch - no activation planes in memory, no LDS traffic
@@ -20,24 +21,29 @@
 #include "cai_internal.hpp"
 #include "cai_gemv_common.hpp"
 #include <algorithm>
+#include <type_traits>
 
 namespace cai {
 
 namespace {
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t uint2_t __attribute__((ext_vector_type(2)));
 
 constexpr int RA_TK = 8;         // tokens per launch
 constexpr int RA_NW = 8;         // waves per work-group at most
 constexpr int RA_SBW = 2;        // super-blocks of a row per wave
 constexpr int RA_SMAX = RA_NW * RA_SBW;   // super-blocks per column slice at most
 constexpr int RA_BB = 144;       // bytes of a Q4_K super-block
+constexpr int RA_B6 = 192;       // bytes of a Q6_K record of codes (16 scales and d lie in planes of their own)
 constexpr int RA_PART_BATCH = 8; // slices of an element the last arriver requests at once (times 2 elements, times 2 for SwiGLU)
 constexpr int RA_XLD = RA_SBW * 256 + 8;          // halfs per operand column in LDS (+8: 16 columns x 16-byte reads tile the banks)
 constexpr int RA_WAVE_LDS = 16 * RA_XLD * 2 + 16 * 16 * 2 + RA_SBW * RA_TK * 4 + 192;   // = 17408 bytes per wave
 
-struct RaSeg { const uint8_t* w; const float* bias; int rows; int y_off; int pair_end; };   // pair_end: cumulative 32-row pairs
+struct RaSeg { const uint8_t* w; const uint8_t* aux; const uint8_t* aux2; const float* bias; int rows; int y_off; int pair_end; };   // pair_end: cumulative 32-row pairs
 
 struct RaParams {
   RaSeg seg[3]; int n_seg;                       // up to three matrices of equal width share a launch (q | k | v)
@@ -70,6 +76,11 @@ template <bool HIGH> __device__ __forceinline__ half8_t ra_weights(uint32_t d0, 
   const half2_t a3 = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, (e1 & M) | (kreg & ~M)), s2, c2);
   return half8_t{a0.x, a0.y, a1.x, a1.y, a2.x, a2.y, a3.x, a3.y};
 }
+__device__ __forceinline__ half2_t ra_halves(float a, float b)
+{
+  typedef float float2_t __attribute__((ext_vector_type(2)));
+  return __builtin_convertvector((float2_t{a, b}), half2_t);
+}
 // all-reduce over the 16 lanes of a row: lane ^ 1, lane ^ 2, then the mirror images within 8 and within 16
 #define RA_DPP(v, ctrl) __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, (v)), (ctrl), 0xf, 0xf, false))
 __device__ __forceinline__ float ra_row_max(float v)
@@ -101,11 +112,12 @@ __device__ __forceinline__ uint32_t ra_ror8(uint32_t v) { return (uint32_t)__bui
 // the 8 of them at 8 j (in the order 0, 2, 1, 3, 4, 6, 5, 7: see ra_weights).  For the min term lane kg stands for the two sub-blocks 2 g + 4 c1, + 1 (each lane pair kg, kg ^ 1
 // holds the halves of four sub-blocks' activations, so their sums are one exchange away).
 // (what the first requests need travels as leading scalar arguments, preloaded in scalar registers)
+// Q6_K: see gemm_q6k_nb for which bytes make which group; the operands of group g are columns 16 g + 4 kg .. + 3, in the order 0, 2, 1, 3.
 // HH: 16-row sets per unit of rows (2: pairs - what SwiGLU needs and what long walks take; 1 halves the unit, for products
 // with fewer pairs than compute units or an uneven number per work-group).  GAIN: the activations carry an RMSNorm gain.
-template <int HH, bool GAIN>
-__global__ __launch_bounds__(64 * RA_NW) void gemm_q4k_ra(const float* hsrc, const long long hstride, const float* hgain, const int hcols, const int hntok,
-                                                          const int hnpairs, const int hS, const RaParams p)
+#define RA_ARGS const float* hsrc, const long long hstride, const float* hgain, const int hcols, const int hntok, const int hnpairs, const int hS
+template <int QT, int HH, bool GAIN>
+__device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, const RaParams& p)      // row group bx of n_bx
 {
   // per wave RA_WAVE_LDS bytes: the operand columns [16][RA_XLD] halfs while the activations are converted (each wave converts
   // and reads back only its own columns: no work-group barrier), their sub-block sums [16][16] halfs and 1 / scale [2][8]; once
@@ -122,8 +134,8 @@ __global__ __launch_bounds__(64 * RA_NW) void gemm_q4k_ra(const float* hsrc, con
   const int nwa = (nS + RA_SBW - 1) / RA_SBW;                              // waves of this work-group with columns to cover
   const int nsw = max(0, min(RA_SBW, nS - RA_SBW * wave));                  // super-blocks of this wave
   const int sbw0 = sb0 + min(RA_SBW * wave, nS - 1);                        // its first one (an idle wave re-reads the last)
-  const int64_t row_bytes = (int64_t)nsb * RA_BB;
-  const int npw = (int)blockIdx.x < hnpairs ? (hnpairs - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x : 0;   // pairs of this work-group
+  constexpr bool Q6 = QT == CAI_Q6_K;
+  const int npw = bx < hnpairs ? (hnpairs - bx + n_bx - 1) / n_bx : 0;   // pairs of this work-group
   const int nq = RA_SBW * npw;                                              // (pair, super-block) items of a wave
   const int tok = n & (RA_TK - 1), tokc = min(tok, hntok - 1);
   const bool tok_on = tok < hntok;
@@ -139,19 +151,31 @@ __global__ __launch_bounds__(64 * RA_NW) void gemm_q4k_ra(const float* hsrc, con
     else { r0 = (pair - t0) * 16 * HH; r1 = r0 + 16; }
   };
 
-  struct WRegs { uint4 h[HH], q[HH][2]; };
+  struct W4 { uint4 h[HH], q[HH][2]; };
+  struct W6 { u32x4_t ql[HH][2], qh[HH], sc[HH]; uint32_t d[HH]; };
+  using WRegs = std::conditional_t<Q6, W6, W4>;
   // weights of item q = (pair q / 2, super-block q % 2 of this wave): for the rows n of both row sets the header and this
   // lane's 2 x 16 quant bytes.  Loads are never conditional: past the last item the last one is fetched again (a cache hit).
   auto load_w = [&](int q, WRegs& r) __attribute__((always_inline)) {
     const int qc = max(min(q, nq - 1), 0);
-    const int pair = min((int)blockIdx.x + (qc >> 1) * (int)gridDim.x, hnpairs - 1), sb = sbw0 + min(qc & 1, max(nsw, 1) - 1);
+    const int pair = min(bx + (qc >> 1) * n_bx, hnpairs - 1), sb = sbw0 + min(qc & 1, max(nsw, 1) - 1);
     const RaSeg* sg; int r0, r1; locate(pair, sg, r0, r1);
 #pragma unroll
     for (int hh = 0; hh < HH; hh++) {
-      const uint8_t* blk = sg->w + (int64_t)min((hh ? r1 : r0) + n, sg->rows - 1) * row_bytes + (int64_t)sb * RA_BB;   // tail rows: re-read the last row
-      r.h[hh] = *reinterpret_cast<const uint4*>(blk);
-      r.q[hh][0] = *reinterpret_cast<const uint4*>(blk + 16 + 16 * kg);
-      r.q[hh][1] = *reinterpret_cast<const uint4*>(blk + 80 + 16 * kg);
+      const int64_t b = (int64_t)min((hh ? r1 : r0) + n, sg->rows - 1) * nsb + sb;   // tail rows: re-read the last row
+      if constexpr (Q6) {
+        const uint8_t* blk = sg->w + b * RA_B6;
+        r.ql[hh][0] = *reinterpret_cast<const u32x4_t*>(blk + 16 * kg);
+        r.ql[hh][1] = *reinterpret_cast<const u32x4_t*>(blk + 64 + 16 * kg);
+        r.qh[hh] = *reinterpret_cast<const u32x4_t*>(blk + 128 + 16 * kg);
+        r.sc[hh] = *reinterpret_cast<const u32x4_t*>(sg->aux + b * 16);
+        r.d[hh] = *reinterpret_cast<const uint16_t*>(sg->aux2 + b * 2);
+      } else {
+        const uint8_t* blk = sg->w + b * RA_BB;
+        r.h[hh] = *reinterpret_cast<const uint4*>(blk);
+        r.q[hh][0] = *reinterpret_cast<const uint4*>(blk + 16 + 16 * kg);
+        r.q[hh][1] = *reinterpret_cast<const uint4*>(blk + 80 + 16 * kg);
+      }
     }
   };
   WRegs wa, wb, wc, wd;
@@ -207,18 +231,18 @@ __global__ __launch_bounds__(64 * RA_NW) void gemm_q4k_ra(const float* hsrc, con
       const float s = on ? ldexpf(1.0f, e) : 0.0f;      // (an absent token's columns: zeros)
 #pragma unroll
       for (int m = 0; m < 4; m++) {
-        // vs = h + l to 21 bits, both parts converted two at a time towards zero (v_cvt_pkrtz_f16_f32: the pair comes out packed, and
+        // vs = h + l to 22 bits, both parts rounded two at a time (v_cvt_pk_f16_f32: the pair comes out packed, and
         // in the operand's order - inside a group of 8 that order is 0, 2, 1, 3, 4, 6, 5, 7 (ra_weights): the middle two of every four
-        // swap); l = vs - h is exact in fp32 and has the sign of vs
+        // swap); l = vs - h is exact in fp32
         float vs[4], sm = 0.0f;
 #pragma unroll
         for (int u = 0; u < 4; u++) { vs[u] = v[m][u] * s; sm += vs[u]; }
-        typedef __fp16 pk2_t __attribute__((ext_vector_type(2)));
-        const pk2_t h02 = __builtin_amdgcn_cvt_pkrtz(vs[0], vs[2]), h13 = __builtin_amdgcn_cvt_pkrtz(vs[1], vs[3]);
-        const pk2_t l02 = __builtin_amdgcn_cvt_pkrtz(vs[0] - (float)h02.x, vs[2] - (float)h02.y), l13 = __builtin_amdgcn_cvt_pkrtz(vs[1] - (float)h13.x, vs[3] - (float)h13.y);
+        const half2_t h02 = ra_halves(vs[0], vs[2]), h13 = ra_halves(vs[1], vs[3]);
+        const half2_t l02 = ra_halves(vs[0] - (float)h02.x, vs[2] - (float)h02.y), l13 = ra_halves(vs[1] - (float)h13.x, vs[3] - (float)h13.y);
         *reinterpret_cast<uint2*>(xw + t8 * RA_XLD + j * 256 + 64 * m + 4 * ii) = make_uint2(__builtin_bit_cast(uint32_t, h02), __builtin_bit_cast(uint32_t, h13));
         *reinterpret_cast<uint2*>(xw + (8 + t8) * RA_XLD + j * 256 + 64 * m + 4 * ii) = make_uint2(__builtin_bit_cast(uint32_t, l02), __builtin_bit_cast(uint32_t, l13));
         // sub-block 2 m + i / 8 of the block: the sum of 8 lanes' values, / 32, hi + lo
+        if constexpr (Q6) continue;
         sm = ra_oct_sum(sm) * 0.03125f;
         const _Float16 qh = (_Float16)sm, ql = (_Float16)(sm - (float)qh);
         if ((ii & 7) == 0) { sxw[t8 * 16 + j * 8 + 2 * m + (ii >> 3)] = qh; sxw[(8 + t8) * 16 + j * 8 + 2 * m + (ii >> 3)] = ql; }
@@ -230,24 +254,30 @@ __global__ __launch_bounds__(64 * RA_NW) void gemm_q4k_ra(const float* hsrc, con
     }
   __builtin_amdgcn_wave_barrier();    // LDS operations of a wave complete in order: its own columns are there
   // the operands in MFMA order: column n, this lane's 8 k of every step
-  half8_t Bx[RA_SBW][8]; half2_t bm[RA_SBW]; float sinv[RA_SBW];
+  half8_t Bx[Q6 ? 1 : RA_SBW][8]; half4_t Xg[Q6 ? RA_SBW : 1][16]; half2_t bm[RA_SBW]; float sinv[RA_SBW]; float4 sinv4[RA_SBW];
 #pragma unroll
   for (int j = 0; j < RA_SBW; j++) {
+    if constexpr (Q6) {
 #pragma unroll
-    for (int t = 0; t < 8; t++)
-      Bx[j][t] = *reinterpret_cast<const half8_t*>(xw + n * RA_XLD + j * 256 + 64 * g + 16 * c1 + 128 * (t >> 2) + 32 * ((t >> 1) & 1) + 8 * (t & 1));
-    bm[j] = *reinterpret_cast<const half2_t*>(sxw + n * 16 + j * 8 + 2 * g + 4 * c1);    // sub-blocks 2 g + 4 c1, + 1
+      for (int gi = 0; gi < 16; gi++) Xg[j][gi] = *reinterpret_cast<const half4_t*>(xw + n * RA_XLD + j * 256 + 16 * gi + 4 * kg);
+      sinv4[j] = *reinterpret_cast<const float4*>(sinvw + j * RA_TK + 4 * c1);      // row 4 kg + i of a result: token (4 kg + i) % 8
+    } else {
+#pragma unroll
+      for (int t = 0; t < 8; t++)
+        Bx[j][t] = *reinterpret_cast<const half8_t*>(xw + n * RA_XLD + j * 256 + 64 * g + 16 * c1 + 128 * (t >> 2) + 32 * ((t >> 1) & 1) + 8 * (t & 1));
+      bm[j] = *reinterpret_cast<const half2_t*>(sxw + n * 16 + j * 8 + 2 * g + 4 * c1);    // sub-blocks 2 g + 4 c1, + 1
+    }
     sinv[j] = sinvw[j * RA_TK + tok];
   }
   __builtin_amdgcn_wave_barrier();    // (the region is written again as the wave's shares of a pair)
-  load_w(2, wc);
+  if constexpr (!Q6) load_w(2, wc);
   timeline_stamp_after(p.timeline, 3, sinv[RA_SBW - 1]);
   timeline_stamp(p.timeline, 4);
   // what the finishing wave of a pair adds to the rows (bias, residual) is requested when the pair starts: by every wave, so
   // that the requests stay unconditional (a kilobyte per wave and pair), and from a harmless address when there is none
   struct Extra { float4 bias[HH], res[HH]; };
   auto prefetch = [&](int i, Extra& f) __attribute__((always_inline)) {
-    const int pair = min((int)blockIdx.x + min(i, max(npw, 1) - 1) * (int)gridDim.x, hnpairs - 1);
+    const int pair = min(bx + min(i, max(npw, 1) - 1) * n_bx, hnpairs - 1);
     const RaSeg* sg; int r0, r1; locate(pair, sg, r0, r1);
 #pragma unroll
     for (int hh = 0; hh < HH; hh++) {
@@ -272,6 +302,45 @@ __global__ __launch_bounds__(64 * RA_NW) void gemm_q4k_ra(const float* hsrc, con
         for (int i = 0; i < 4; i++) acc[hh][i] = 0.0f;
     }
     if (j >= nsw) return;
+    if constexpr (Q6) {
+      const float4_t z4 = {0.0f, 0.0f, 0.0f, 0.0f};
+      const half2_t o2 = {(_Float16)(-1056.0f), (_Float16)(-1056.0f)};   // 1024 + q - 1056 = q - 32
+#pragma unroll
+      for (int hh = 0; hh < HH; hh++) {
+        // dword kg of every 16-byte chunk: ql chunks 0..7 in lq[0..7], qh chunks 0..3 in hq[0..3]
+        uint32_t lq[8], hq[4];
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+          const u32x4_t v = a < 2 ? r.ql[hh][a] : r.qh[hh];
+          const uint2_t t02 = __builtin_amdgcn_permlane32_swap(v.x, v.z, false, false);
+          const uint2_t t13 = __builtin_amdgcn_permlane32_swap(v.y, v.w, false, false);
+          const uint2_t u01 = __builtin_amdgcn_permlane16_swap(t02.x, t13.x, false, false);
+          const uint2_t u23 = __builtin_amdgcn_permlane16_swap(t02.y, t13.y, false, false);
+          uint32_t* dst = a < 2 ? lq + 4 * a : hq;
+          dst[0] = u01.x; dst[1] = u01.y; dst[2] = u23.x; dst[3] = u23.y;
+        }
+        const float d = __half2float(__ushort_as_half((unsigned short)r.d[hh]));
+        const uint32_t scw[4] = {r.sc[hh].x, r.sc[hh].y, r.sc[hh].z, r.sc[hh].w};
+        float gs[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int gi = 0; gi < 16; gi++) {
+          const int nh = gi >> 3, jq = (gi >> 1) & 3, h = gi & 1;
+          const uint32_t lo = (lq[4 * nh + 2 * (jq & 1) + h] >> (4 * (jq >> 1))) & 0x0f0f0f0fu;
+          const uint32_t hf = hq[2 * nh + h];
+          const uint32_t hi = (jq == 0 ? (hf << 4) : jq == 1 ? (hf << 2) : jq == 2 ? hf : (hf >> 2)) & 0x30303030u;
+          const uint32_t c = lo | hi;
+          const half2_t w02 = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, c, 0x04020400u)) + o2;
+          const half2_t w13 = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, c, 0x04030401u)) + o2;
+          const half4_t W = {w02.x, w02.y, w13.x, w13.y};
+          const float ds = d * (float)(int)(int8_t)((scw[gi >> 2] >> (8 * (gi & 3))) & 0xffu);
+          const float4_t C = __builtin_amdgcn_mfma_f32_16x16x16f16(Xg[j][gi], W, z4, 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < 4; i++) gs[i] = fmaf(ds, C[i], gs[i]);
+        }
+        acc[hh][0] = fmaf(sinv4[j].x, gs[0], acc[hh][0]); acc[hh][1] = fmaf(sinv4[j].y, gs[1], acc[hh][1]);
+        acc[hh][2] = fmaf(sinv4[j].z, gs[2], acc[hh][2]); acc[hh][3] = fmaf(sinv4[j].w, gs[3], acc[hh][3]);
+      }
+    } else {
     float4_t C[HH], Cm[HH];
     half2_t s2[HH][4], c2[HH][4];
 #pragma unroll
@@ -324,12 +393,22 @@ __global__ __launch_bounds__(64 * RA_NW) void gemm_q4k_ra(const float* hsrc, con
       acc[hh][3] += sinv[j] * (d4.w * C[hh][3] - m4.w * Cm[hh][3]);
     }
     __builtin_amdgcn_wave_barrier();
+    }
   };
 
   // ---- end of a pair: every wave leaves its share (column t hi + column 8 + t lo), one wave finishes the rows ----
   auto pair_end = [&](int i, const Extra& f) __attribute__((always_inline)) {
     const int slot = i & 1;
-    if (nsw > 0) {
+    if (Q6 && nsw > 0) {     // result row 4 kg + i = token (4 kg + i) % 8, hi (kg < 2) or lo: they meet across kg ^ 2; column n = weight row n
+#pragma unroll
+      for (int hh = 0; hh < HH; hh++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          const float t = acc[hh][k] + __shfl_xor(acc[hh][k], 32, 64);
+          if (kg < 2) reinterpret_cast<float*>(wl)[(slot * 32 + (n >> 2) * 8 + 4 * kg + k) * 8 + 4 * hh + (n & 3)] = t;
+        }
+    }
+    if (!Q6 && nsw > 0) {
       float tot[4 * HH];
 #pragma unroll
       for (int hh = 0; hh < HH; hh++)
@@ -351,7 +430,7 @@ __global__ __launch_bounds__(64 * RA_NW) void gemm_q4k_ra(const float* hsrc, con
       if constexpr (HH == 2) { const float4 b = *reinterpret_cast<const float4*>(src + 4); t8[4] += b.x; t8[5] += b.y; t8[6] += b.z; t8[7] += b.w; }
     }
     if (!tok_on) return;
-    const int pair = (int)blockIdx.x + i * (int)gridDim.x;
+    const int pair = bx + i * n_bx;
     const RaSeg* sg; int r0, r1; locate(pair, sg, r0, r1);
     if (p.n_slices > 1) {     // a slice's share of the rows (finished by the last slice to arrive, below)
 #pragma unroll
@@ -396,7 +475,14 @@ __global__ __launch_bounds__(64 * RA_NW) void gemm_q4k_ra(const float* hsrc, con
     }
   };
 
-  for (int q = 0; q < nq; q += 4) {
+  if constexpr (Q6)       // (two items on their way are what the registers hold)
+    for (int i = 0; i < npw; i++) {
+      prefetch(i, ea);
+      compute(wa, 0); load_w(2 * i + 2, wa);
+      compute(wb, 1); load_w(2 * i + 3, wb);
+      pair_end(i, ea);
+    }
+  else for (int q = 0; q < nq; q += 4) {
     prefetch(q >> 1, ea);
     load_w(q + 3, wd); compute(wa, 0);
     load_w(q + 4, wa); compute(wb, 1);
@@ -413,7 +499,7 @@ __global__ __launch_bounds__(64 * RA_NW) void gemm_q4k_ra(const float* hsrc, con
     __builtin_amdgcn_s_waitcnt(0x0F70);
     __syncthreads();
     if (threadIdx.x == 0)
-      s_is_last = __builtin_amdgcn_atomic_inc32(p.counters + blockIdx.x, (unsigned)p.n_slices - 1, __ATOMIC_RELAXED, "agent") == (unsigned)p.n_slices - 1;
+      s_is_last = __builtin_amdgcn_atomic_inc32(p.counters + bx, (unsigned)p.n_slices - 1, __ATOMIC_RELAXED, "agent") == (unsigned)p.n_slices - 1;
     __syncthreads();
     timeline_stamp(p.timeline, 6);
     if (!s_is_last) { timeline_stamp(p.timeline, 7); return; }
@@ -430,7 +516,7 @@ __global__ __launch_bounds__(64 * RA_NW) void gemm_q4k_ra(const float* hsrc, con
         const int e = min(e0 + b * (int)blockDim.x, total - 1);
         on[b] = e0 + b * (int)blockDim.x < total;
         const int rl = e % rpu, t = (e / rpu) % hntok, i = (e / rpu) / hntok;
-        const RaSeg* sg; int r0, r1; locate((int)blockIdx.x + i * (int)gridDim.x, sg, r0, r1);
+        const RaSeg* sg; int r0, r1; locate(bx + i * n_bx, sg, r0, r1);
         src[b] = p.part + (int64_t)t * p.part_stride + sg->y_off + r0 + rl;
         out[b] = (int64_t)t * p.y_stride + sg->y_off + r0 + rl;
         bias[b] = sg->bias ? sg->bias[r0 + rl] : 0.0f;
@@ -453,6 +539,20 @@ __global__ __launch_bounds__(64 * RA_NW) void gemm_q4k_ra(const float* hsrc, con
     }
   }
   timeline_stamp(p.timeline, 7);
+}
+
+template <int QT, int HH, bool GAIN>
+__global__ __launch_bounds__(64 * RA_NW) void gemm_ra(RA_ARGS, const RaParams p)
+{
+  ra_body<QT, HH, GAIN>(hsrc, hstride, hgain, hcols, hntok, hnpairs, hS, blockIdx.x, gridDim.x, p);
+}
+// Normed products over the same activations whose matrices are of both types (attn_q and attn_k beside the attn_v of a mixed file): the first
+// hn4 work-groups take the Q4_K rows in pairs of row sets, the others the Q6_K rows.  Both launches by themselves spend most of their time on
+// the activations (7B shape, eight sequences: 11.1 + 11.2 us, 12.9 here).
+__global__ __launch_bounds__(64 * RA_NW) void gemm_ra_two(RA_ARGS, const int hnpairs6, const int hn4, const RaParams p, const RaParams p6)
+{
+  if ((int)blockIdx.x < hn4) ra_body<CAI_Q4_K, 2, true>(hsrc, hstride, hgain, hcols, hntok, hnpairs, hS, blockIdx.x, hn4, p);
+  else ra_body<CAI_Q6_K, 1, true>(hsrc, hstride, hgain, hcols, hntok, hnpairs6, hS, blockIdx.x - hn4, gridDim.x - hn4, p6);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -523,20 +623,53 @@ size_t ra_part_floats(int64_t rows, int64_t cols)
   return (size_t)ns_max * RA_TK * (size_t)((rows + 3) / 4 * 4);
 }
 
-// Whether ra_gemm takes these matrices: Q4_K, one width of whole super-blocks, whole 16-row sets,
+// Whether ra_gemm takes these matrices: Q4_K or Q6_K, one width of whole super-blocks, whole 16-row sets,
 // one column slice when the product carries an RMSNorm or SwiGLU.
 bool ra_supported(const cai_qw_s* const* ws, int n_w, bool normed, int swiglu_half)
 {
   if (n_w < 1 || n_w > 3 || (swiglu_half > 0 && n_w != 1)) return false;
   for (int i = 0; i < n_w; i++) {
     const cai_qw_s* w = ws[i];
-    if (w->qtype != CAI_Q4_K || w->cols != ws[0]->cols || w->cols % 256 || w->cols < 256 || w->rows % 16) return false;
+    if ((w->qtype != CAI_Q4_K && w->qtype != CAI_Q6_K) || w->cols != ws[0]->cols || w->cols % 256 || w->cols < 256 || w->rows % 16) return false;
   }
   if (swiglu_half > 0 && (ws[0]->rows != 2 * (int64_t)swiglu_half || swiglu_half % 16)) return false;
   // a product with an RMSNorm or SwiGLU must be one column slice (its finishing wave needs the whole row's sum of squares and
   // both halves' rows); measured on 5120 columns a sliced form with those exchanged through memory lost to the plane form
   const int nsb = (int)(ws[0]->cols >> 8);
   return !((normed || swiglu_half > 0) && nsb > RA_SMAX);
+}
+
+static int ra_check(const cai_qw_s* const* ws, const int* y_off, int n_w, const float* x, int64_t x_stride, const float* gain, const float* y, int64_t y_stride, const float* residual)
+{
+  if ((x_stride & 3) || (reinterpret_cast<uintptr_t>(x) & 15) || (gain && (reinterpret_cast<uintptr_t>(gain) & 15)))
+    return set_error(CAI_ERR_INVALID, "small-batch product (register form): activations must be 16-byte aligned rows");
+  if ((y_stride & 3) || (reinterpret_cast<uintptr_t>(y) & 15) || (residual && (reinterpret_cast<uintptr_t>(residual) & 15)))
+    return set_error(CAI_ERR_INVALID, "small-batch product (register form): results must be 16-byte aligned rows");
+  for (int i = 0; i < n_w; i++)
+    if ((y_off[i] & 3) || (ws[i]->bias && (reinterpret_cast<uintptr_t>(ws[i]->bias) & 15)))
+      return set_error(CAI_ERR_INVALID, "small-batch product (register form): output offsets and biases must be 16-byte aligned");
+  return CAI_OK;
+}
+static RaSeg ra_seg(const cai_qw_s* w, int y_off, int end) { return RaSeg{w->data, w->aux, w->qtype == CAI_Q6_K ? qw_aux2(w) : nullptr, w->bias, (int)w->rows, y_off, end}; }
+static int ra_two(const cai_qw_s* const* ws, const int* y_off, int n_w, int n_tok, const float* x, int64_t x_stride, const float* gain, float eps, float* y, int64_t y_stride)
+{
+  int rc = ra_check(ws, y_off, n_w, x, x_stride, gain, y, y_stride, nullptr);
+  if (rc) return rc;
+  RaParams p[2] = {};
+  int units[2] = {0, 0};        // pairs of row sets of Q4_K, row sets of Q6_K
+  for (int i = 0; i < n_w; i++) {
+    const int six = ws[i]->qtype == CAI_Q6_K;
+    units[six] += (int)(ws[i]->rows / (six ? 16 : 32));
+    p[six].seg[p[six].n_seg++] = ra_seg(ws[i], y_off[i], units[six]);
+  }
+  for (RaParams& q : p) { q.eps = eps; q.y = y; q.y_stride = y_stride; q.n_slices = 1; }
+  const int nsb = (int)(ws[0]->cols >> 8), nw = (nsb + RA_SBW - 1) / RA_SBW, all = units[0] + units[1], slots = std::max(2, ctx().n_cu * (RA_NW / nw));
+  const int n4 = all <= slots ? units[0] : std::max(1, std::min(slots - 1, (int)((int64_t)slots * units[0] / all))), n6 = all <= slots ? units[1] : std::max(1, std::min(units[1], slots - n4));
+  p[0].timeline = p[1].timeline = timeline_next(n4 + n6);
+  static bool attr_done = false;
+  if (!attr_done) { CAI_HIP(hipFuncSetAttribute((const void*)gemm_ra_two, hipFuncAttributeMaxDynamicSharedMemorySize, RA_NW * RA_WAVE_LDS)); attr_done = true; }
+  hipLaunchKernelGGL(gemm_ra_two, dim3(n4 + n6), dim3(64 * nw), (size_t)nw * RA_WAVE_LDS, ctx().stream, x, (long long)x_stride, gain, (int)ws[0]->cols, n_tok, units[0], nsb, units[1], n4, p[0], p[1]);
+  return CAI_OK;
 }
 
 // y[t][y_off_i + r] = W_i (gain . x_t) / rms(x_t) + bias_i [+ residual]   for t < n_tok <= 8, or, with swiglu_half > 0,
@@ -546,13 +679,17 @@ int ra_gemm(const cai_qw_s* const* ws, const int* y_off, int n_w, int n_tok, con
 {
   if (n_tok < 1 || n_tok > RA_TK || !ra_supported(ws, n_w, gain != nullptr, swiglu_half))
     return set_error(CAI_ERR_UNSUPPORTED, "small-batch product (register form): %d matrices, %d tokens", n_w, n_tok);
-  if ((x_stride & 3) || (reinterpret_cast<uintptr_t>(x) & 15) || (gain && (reinterpret_cast<uintptr_t>(gain) & 15)))
-    return set_error(CAI_ERR_INVALID, "small-batch product (register form): activations must be 16-byte aligned rows");
-  if ((y_stride & 3) || (reinterpret_cast<uintptr_t>(y) & 15) || (residual && (reinterpret_cast<uintptr_t>(residual) & 15)))
-    return set_error(CAI_ERR_INVALID, "small-batch product (register form): results must be 16-byte aligned rows");
-  for (int i = 0; i < n_w; i++)
-    if ((y_off[i] & 3) || (ws[i]->bias && (reinterpret_cast<uintptr_t>(ws[i]->bias) & 15)))
-      return set_error(CAI_ERR_INVALID, "small-batch product (register form): output offsets and biases must be 16-byte aligned");
+  if (gain && swiglu_half == 0 && !residual) {
+    bool four = false, six = false, pairs = true;
+    for (int i = 0; i < n_w; i++) { (ws[i]->qtype == CAI_Q6_K ? six : four) = true; pairs = pairs && (ws[i]->qtype == CAI_Q6_K || ws[i]->rows % 32 == 0); }
+    if (four && six && pairs) return ra_two(ws, y_off, n_w, n_tok, x, x_stride, gain, eps, y, y_stride);
+  }
+  for (int i = 1; i < n_w; i++)
+    if (ws[i]->qtype != ws[0]->qtype) {      // (one type after the other)
+      int rc = ra_gemm(ws, y_off, i, n_tok, x, x_stride, gain, eps, swiglu_half, y, y_stride, residual);
+      return rc ? rc : ra_gemm(ws + i, y_off + i, n_w - i, n_tok, x, x_stride, gain, eps, swiglu_half, y, y_stride, residual);
+    }
+  { int rc = ra_check(ws, y_off, n_w, x, x_stride, gain, y, y_stride, residual); if (rc) return rc; }
   RaParams p{};
   p.n_seg = n_w; p.eps = eps; p.swiglu_half = swiglu_half; p.y = y; p.y_stride = y_stride; p.residual = residual;
   const int cols = (int)ws[0]->cols, nsb = cols >> 8;
@@ -572,7 +709,7 @@ int ra_gemm(const cai_qw_s* const* ws, const int* y_off, int n_w, int n_tok, con
   int cum = 0; int64_t width = 0;
   for (int i = 0; i < n_w; i++) {
     cum += swiglu_half > 0 ? swiglu_half / 16 : (int)(ws[i]->rows / (16 * HH));
-    p.seg[i] = RaSeg{ws[i]->data, ws[i]->bias, (int)ws[i]->rows, y_off[i], cum};
+    p.seg[i] = ra_seg(ws[i], y_off[i], cum);
     width = std::max<int64_t>(width, y_off[i] + ws[i]->rows);
   }
   p.n_slices = n_slices;
@@ -586,14 +723,17 @@ int ra_gemm(const cai_qw_s* const* ws, const int* y_off, int n_w, int n_tok, con
   p.timeline = timeline_next(gx * n_slices);
   const dim3 grid(gx, n_slices), block(64 * nw);
   const size_t lds = (size_t)nw * RA_WAVE_LDS;
-#define RA_LAUNCH(HHv, GAINv) do { \
+#define RA_LAUNCH(QTv, HHv, GAINv) do { \
     static bool attr_done = false; \
-    if (!attr_done) { CAI_HIP(hipFuncSetAttribute((const void*)gemm_q4k_ra<HHv, GAINv>, hipFuncAttributeMaxDynamicSharedMemorySize, RA_NW * RA_WAVE_LDS)); attr_done = true; } \
-    hipLaunchKernelGGL((gemm_q4k_ra<HHv, GAINv>), grid, block, lds, ctx().stream, x, (long long)x_stride, gain, cols, n_tok, units, S, p); } while (0)
-  if (HH == 2 && gain) RA_LAUNCH(2, true);
-  else if (HH == 2) RA_LAUNCH(2, false);
-  else if (gain) RA_LAUNCH(1, true);
-  else RA_LAUNCH(1, false);
+    if (!attr_done) { CAI_HIP(hipFuncSetAttribute((const void*)gemm_ra<QTv, HHv, GAINv>, hipFuncAttributeMaxDynamicSharedMemorySize, RA_NW * RA_WAVE_LDS)); attr_done = true; } \
+    hipLaunchKernelGGL((gemm_ra<QTv, HHv, GAINv>), grid, block, lds, ctx().stream, x, (long long)x_stride, gain, cols, n_tok, units, S, p); } while (0)
+#define RA_TYPE(QTv) do { \
+    if (HH == 2 && gain) RA_LAUNCH(QTv, 2, true); \
+    else if (HH == 2) RA_LAUNCH(QTv, 2, false); \
+    else if (gain) RA_LAUNCH(QTv, 1, true); \
+    else RA_LAUNCH(QTv, 1, false); } while (0)
+  if (ws[0]->qtype == CAI_Q6_K) RA_TYPE(CAI_Q6_K); else RA_TYPE(CAI_Q4_K);
+#undef RA_TYPE
 #undef RA_LAUNCH
   return CAI_OK;
 }

@@ -187,6 +187,36 @@ def test_batched_decode_and_prompt_of_a_q4k_q6k_mix_equal_single_steps():
     assert rel_err(lg, last) < 1e-3 and am == int(np.argmax(last))
 
 
+@pytest.mark.parametrize("types", ["444444", "666666", "446466", "664644", "646446"])      # q, k, v, gate|up, down, head
+@pytest.mark.parametrize("d,heads,kv,ffn,vocab", [(512, 8, 2, 1024, 608), (256, 16, 2, 512, 601), (768, 16, 2, 4352, 1296)])
+def test_batched_decode_of_q4k_and_q6k_matrices_equals_single(types, d, heads, kv, ffn, vocab):
+    """One to three super-blocks a row (waves with one, with none), 17 (slices), matrices of both types over one set of
+    activations, vocabularies that are no whole row sets; 2, 3 and 8 sequences.  Two layers of sums whose operands are held to 22 bits."""
+    from helpers.device import dev
+    cai = dev()
+    cfg = dict(n_layers=2, d_model=d, n_q_heads=heads, n_kv_heads=kv, head_dim=d // heads, ffn=ffn, vocab=vocab, max_ctx=64, eps=1e-5, rope_theta=1e4)
+    t = [O.Q4_K if c == "4" else O.Q6_K for c in types]
+    spec = synthetic_spec(cfg, t[0], head_qtype=t[5], seed=7, std=0.05, qkv_bias=True)
+    rng = np.random.default_rng(8)
+    for l in range(2):
+        for slot, qt in ((O.W_K, t[1]), (O.W_V, t[2]), (O.W_GATEUP, t[3]), (O.W_DOWN, t[4])):
+            m = spec["tensors"][(l, slot)]
+            m.update(type=qt, raw=O.quantize(qt, (rng.standard_normal((m["rows"], m["cols"])) * 0.05).astype(np.float32)))
+    dec = cai.Decoder(spec, max_batch=8)
+    toks = rng.integers(0, vocab, (8, 5))
+    singles = []
+    for b in range(8):
+        dec.reset(0)
+        singles.append([dec.step(int(toks[b, p]), p)[1][0].copy() for p in range(5)])
+    for n in (2, 3, 8):
+        for b in range(n):
+            dec.reset(b)
+        for p in range(5):
+            _, lg = dec.step(toks[:n, p], np.full(n, p))
+            for b in range(n):
+                assert np.max(np.abs(lg[b] - singles[b][p])) <= 2e-5 * np.max(np.abs(singles[b][p])), (n, p, b)
+
+
 @pytest.mark.parametrize("name,n", [("olmoe_like_q8", 11), ("olmoe_like_q8", 45), ("moe_like_q6k", 29)])
 def test_moe_prefill_equals_sequential_steps(name, n):
     """Mixture-of-experts prompts: attention half on the whole chunk, routed half per group of rows (router and top-k once
