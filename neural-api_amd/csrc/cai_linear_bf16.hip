@@ -609,8 +609,13 @@ static int run_lin(const cai_qw_s* w, const AT* x, int64_t ldx, int n_tok, const
     }
     return run_gemm<AT, 128, 128, 2, sizeof(AT) == 2 ? 4 : 2>(w, x, ldx, n_tok, e);
   }
-  if (n_tok > 32 && tiles(64, 64) >= ctx().n_cu) return run_gemm<AT, 64, 64, 2, 2>(w, x, ldx, n_tok, e);
-  return run_gemm<AT, 32, 64, 2, 2>(w, x, ldx, n_tok, e);
+  // Small tiles: a step is a hundred nanoseconds of work and a round trip to memory is a microsecond, so copies go out several steps ahead, as
+  // far as the LDS of the work-groups that share a CU allows (two slots: 5632 columns, 162 tokens 46 us a product of 2048 rows, six 20).  Whole prompt through
+  // four layers, us, two slots | these: width 2048, 20 tokens 884 | 569, 100: 962 | 687, 250: 1045 | 805, 400: 1116 | 976; 1024, 64: 653 | 496; 512, 250: 500 | 472.
+  // 64 x 64 with four and with six slots: 833, 854 at 250 tokens; 32 x 64 with four and with eight: within 2 %.
+  constexpr bool BF = sizeof(AT) == 2;
+  if (n_tok > 32 && tiles(64, 64) >= ctx().n_cu) return run_gemm<AT, 64, 64, 2, 2, BF ? 3 : 2>(w, x, ldx, n_tok, e);
+  return run_gemm<AT, 32, 64, 2, 2, BF ? 6 : 2>(w, x, ldx, n_tok, e);
 }
 
 int launch_lin_rms(int act_t, const float* x, int64_t ldx, int width, float eps, int n_tok, const RmsLin& a, const RmsLin* b)

@@ -128,6 +128,18 @@ def test_streamed_bf16_products(cai, tmp_path, width, ff, vocab):
     dec.close()
 
 
+@pytest.mark.parametrize("width, ff, vocab", [(64, 17, 61), (72, 130, 131), (192, 300, 520), (320, 390, 67), (384, 448, 67), (448, 1100, 67), (264, 8200, 67)])
+def test_small_tiles_of_few_steps(cai, tmp_path, width, ff, vocab):
+    """Tiles of 32 and 64 tokens whose copies run five and two steps ahead: products of one to eight steps, and of many; a token past a tile."""
+    m = Model(tmp_path, B.config([B.layer(B.delta(), ff=ff)], width=width, vocab=vocab), seed=width, edit=only("feed-forward"), rank_a=3, rank_g=20)
+    tok = m.tokens(130, 1)
+    dec = m.open(cai, 192, 1, "bf16")
+    for cuts in ([17, 33, 80], [32, 65, 33], [130]):
+        check(feed(dec, tok, cuts), m.ref(tok), "bf16")
+        dec.reset()
+    dec.close()
+
+
 # ---------------------------------------------------------------- whole models
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
 @pytest.mark.parametrize("cuts", [[300], [1], [2], [3, 2, 65, 1, 1, 16, 17, 2], [64], [130, 1], [5, 9, 7]], ids=str)
