@@ -370,7 +370,7 @@ def gateup_kernel_name(qtype, cols):
     """Name of the batch-1 fused gate|up kernel the library launches for this weight type and width (rows of 17..24
     super-blocks are packed four to a wave: the fifth template argument, else 1)."""
     if qtype not in ("Q4_K", "Q5_K"):
-        return "gemv_fast<%s>" % qtype
+        return "%s<%s>" % ("gemv_one" if cols <= 4096 else "gemv_fast", qtype)
     packed = cols % 256 == 0 and 16 < cols // 256 <= 24
     return "gemv_%s_dot<1,1,false,2,%d>" % ("q4k" if qtype == "Q4_K" else "q5k", 4 if packed else 1)
 

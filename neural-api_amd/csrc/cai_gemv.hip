@@ -10,6 +10,7 @@
 // (reference: neural/neuralvolume.pas:12127-12423, 12693-12745; fused tail neural/neural.cl:111-146).
 #include "cai_internal.hpp"
 #include "cai_gemv_common.hpp"
+#include <type_traits>
 #include "cai_blocks_raw.hpp"
 
 namespace cai {
@@ -212,91 +213,7 @@ __global__ __launch_bounds__(256) void gemv_fast(const GemvParams p)
       }
       const int xb0 = lds_unit_base<QT>(u);
 
-      if (NB == 1) {
-        // x unit in registers, reused for every row of the wave
-        float xv[UW];
-#pragma unroll
-        for (int t = 0; t < T; t++) {
-          const float4 v = xs4[xb0 + t * 16];
-          xv[4 * t] = v.x; xv[4 * t + 1] = v.y; xv[4 * t + 2] = v.z; xv[4 * t + 3] = v.w;
-        }
-        if (QT == CAI_Q4_K) {
-          float sxlo = 0.0f, sxhi = 0.0f;
-#pragma unroll
-          for (int i = 0; i < 16; i++) { sxlo += xv[i]; sxhi += xv[16 + i]; }
-          const int cc = (u & 7) >> 1;
-#pragma unroll
-          for (int r = 0; r < RR; r++) {
-            const uint32_t qw[4] = {q[r].x, q[r].y, q[r].z, q[r].w};
-            float slo = 0.0f, shi = 0.0f;
-#pragma unroll
-            for (int w = 0; w < 4; w++) {
-              const uint32_t lo = qw[w] & 0x0f0f0f0fu, hi = (qw[w] >> 4) & 0x0f0f0f0fu;
-              slo = fmaf(cvt_ub0(lo), xv[4 * w], slo);     slo = fmaf(cvt_ub1(lo), xv[4 * w + 1], slo);
-              slo = fmaf(cvt_ub2(lo), xv[4 * w + 2], slo); slo = fmaf(cvt_ub3(lo), xv[4 * w + 3], slo);
-              shi = fmaf(cvt_ub0(hi), xv[16 + 4 * w], shi);     shi = fmaf(cvt_ub1(hi), xv[16 + 4 * w + 1], shi);
-              shi = fmaf(cvt_ub2(hi), xv[16 + 4 * w + 2], shi); shi = fmaf(cvt_ub3(hi), xv[16 + 4 * w + 3], shi);
-            }
-            uint32_t sc, mn; q4k_scale_pair(hdr[r].y, hdr[r].z, hdr[r].w, cc, sc, mn);
-            const float d = __half2float(__ushort_as_half((unsigned short)(hdr[r].x & 0xffffu)));
-            const float dmin = __half2float(__ushort_as_half((unsigned short)(hdr[r].x >> 16)));
-            const float part = d * (cvt_ub0(sc) * slo + cvt_ub1(sc) * shi) - dmin * (cvt_ub0(mn) * sxlo + cvt_ub1(mn) * sxhi);
-            acc[r][0] += part;
-          }
-        } else if (QT == CAI_Q6_K) {
-          float sx[4];
-#pragma unroll
-          for (int j = 0; j < 4; j++) sx[j] = (xv[4 * j] + xv[4 * j + 1]) + (xv[4 * j + 2] + xv[4 * j + 3]);
-          const int hs = (u & 4) ? 8 : 0;    // positions 16..31 of a 32-run use the odd scale of the pair
-#pragma unroll
-          for (int r = 0; r < RR; r++) {
-            uint32_t cj[4]; q6k_codes(q[r].x, q[r].y, q[r].z, cj);
-            const uint32_t s01 = hdr[r].x >> hs, s23 = hdr[r].y >> hs;
-            const float sc[4] = {(float)(int8_t)(s01 & 0xff), (float)(int8_t)((s01 >> 16) & 0xff), (float)(int8_t)(s23 & 0xff), (float)(int8_t)((s23 >> 16) & 0xff)};
-            float part = 0.0f;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-              float sq = cvt_ub0(cj[j]) * xv[4 * j];
-              sq = fmaf(cvt_ub1(cj[j]), xv[4 * j + 1], sq); sq = fmaf(cvt_ub2(cj[j]), xv[4 * j + 2], sq); sq = fmaf(cvt_ub3(cj[j]), xv[4 * j + 3], sq);
-              part = fmaf(sc[j], fmaf(-32.0f, sx[j], sq), part);
-            }
-            acc[r][0] = fmaf(__half2float(__ushort_as_half(dh[r])), part, acc[r][0]);
-          }
-        } else if (QT == CAI_Q4_0) {
-          float sx = 0.0f;
-#pragma unroll
-          for (int i = 0; i < 32; i++) sx += xv[i];
-#pragma unroll
-          for (int r = 0; r < RR; r++) {
-            const uint32_t qw[4] = {q[r].x, q[r].y, q[r].z, q[r].w};
-            float sq = 0.0f;
-#pragma unroll
-            for (int w = 0; w < 4; w++) {
-              const uint32_t lo = qw[w] & 0x0f0f0f0fu, hi = (qw[w] >> 4) & 0x0f0f0f0fu;
-              sq = fmaf(cvt_ub0(lo), xv[4 * w], sq);     sq = fmaf(cvt_ub1(lo), xv[4 * w + 1], sq);
-              sq = fmaf(cvt_ub2(lo), xv[4 * w + 2], sq); sq = fmaf(cvt_ub3(lo), xv[4 * w + 3], sq);
-              sq = fmaf(cvt_ub0(hi), xv[16 + 4 * w], sq);     sq = fmaf(cvt_ub1(hi), xv[16 + 4 * w + 1], sq);
-              sq = fmaf(cvt_ub2(hi), xv[16 + 4 * w + 2], sq); sq = fmaf(cvt_ub3(hi), xv[16 + 4 * w + 3], sq);
-            }
-            const float d = __half2float(__ushort_as_half(dh[r]));
-            acc[r][0] = fmaf(d, sq - 8.0f * sx, acc[r][0]);
-          }
-        } else {  // Q8_0
-#pragma unroll
-          for (int r = 0; r < RR; r++) {
-            const uint32_t qw[4] = {q[r].x, q[r].y, q[r].z, q[r].w};
-            float sq = 0.0f;
-#pragma unroll
-            for (int w = 0; w < 4; w++) {
-              sq = fmaf((float)(int8_t)(qw[w] & 0xff), xv[4 * w], sq);
-              sq = fmaf((float)(int8_t)((qw[w] >> 8) & 0xff), xv[4 * w + 1], sq);
-              sq = fmaf((float)(int8_t)((qw[w] >> 16) & 0xff), xv[4 * w + 2], sq);
-              sq = fmaf((float)(int8_t)(qw[w] >> 24), xv[4 * w + 3], sq);
-            }
-            acc[r][0] = fmaf(__half2float(__ushort_as_half(dh[r])), sq, acc[r][0]);
-          }
-        }
-      } else {
+      {
         // small batch: dequantize the unit of every row once (unscaled integer values as floats),
         // then stream the NB activation units from LDS
         float wf[RR][UW];
@@ -431,6 +348,236 @@ __global__ __launch_bounds__(256) void gemv_fast(const GemvParams p)
           yout[(int64_t)b * p.y_stride + sg.y_off + row] = silu_mul(up, gate);
         }
       }
+    }
+  }
+  timeline_stamp(p.timeline, 7);
+}
+
+// ------------------------------------------------------------------------------------------
+// One activation row of up to 4096 columns: Q4_K (expert banks), Q4_0, Q8_0, per-row int8, Q6_K.  MODE, R as above; BANK: blockIdx.y is a slot whose expert id selects the rows.
+// What bounds it at the sizes of a small model is round trips to memory, one after another, so everything that does not depend on anything goes
+// out first: the activation with its gains, the first PF steps of the rows (a step: 64 units, a lane each), bias and residual of the
+// row that the lane finishes.  us a launch, weights after the staging | here: 576 x 576
+// in a step 3.5 | 3.0, 6144 x 2048 normed 7.6 | 6.3, 8 experts of 2048 x 2048 10.8 | 9.7, 49152 x 576 14.8 | 10.7; back to back 12000 x 3584 11.7 | 9.3, 36000 x 2048 17.1 | 13.5.
+// The leading scalar arguments are what these requests need of a launch of one matrix; they arrive preloaded (see the Makefile).
+// ------------------------------------------------------------------------------------------
+template <int QT> struct Unit { uint4 q, hdr; uint16_t dh; };
+template <int QT>
+__device__ __forceinline__ void load_unit(const uint8_t* rp, const uint8_t* ap, const uint8_t* dp, int un, Unit<QT>& w)
+{
+  if constexpr (QT == CAI_Q4_K) {
+    const uint8_t* blk = rp + (int64_t)(un >> 3) * 144;
+    w.hdr = *reinterpret_cast<const uint4*>(blk);
+    w.q = *reinterpret_cast<const uint4*>(blk + 16 + 16 * (un & 7));
+  } else if constexpr (QT == CAI_Q6_K) {
+    const int sb = un >> 4, nh = (un >> 3) & 1, l4 = (un & 7) * 4;
+    const uint8_t* blk = rp + (int64_t)sb * 192;
+    w.q.x = *reinterpret_cast<const uint32_t*>(blk + 64 * nh + l4);
+    w.q.y = *reinterpret_cast<const uint32_t*>(blk + 64 * nh + 32 + l4);
+    w.q.z = *reinterpret_cast<const uint32_t*>(blk + 128 + 32 * nh + l4);
+    const uint2 sc2 = *reinterpret_cast<const uint2*>(ap + sb * 16 + 8 * nh);
+    w.hdr.x = sc2.x; w.hdr.y = sc2.y;
+    w.dh = *reinterpret_cast<const uint16_t*>(dp + sb * 2);
+  } else if constexpr (QT == CAI_Q4_0) {
+    w.q = *reinterpret_cast<const uint4*>(rp + (int64_t)un * 16);
+    w.dh = *reinterpret_cast<const uint16_t*>(ap + un * 2);
+  } else {
+    w.q = *reinterpret_cast<const uint4*>(rp + (int64_t)un * 16);
+    w.dh = QT == CAI_I8ROW ? (uint16_t)0x3C00 : *reinterpret_cast<const uint16_t*>(ap + (un >> 1) * 2);   // per-row int8: block scale 1
+  }
+}
+// acc + the unit's part of the sum; un: the unit's place in the row
+template <int QT>
+__device__ __forceinline__ float unit_dot(const Unit<QT>& w, const float (&xv)[QTraits<QT>::UW], int un, float acc)
+{
+  const uint32_t qw[4] = {w.q.x, w.q.y, w.q.z, w.q.w};
+  if constexpr (QT == CAI_Q4_K) {
+    float sxlo = 0.0f, sxhi = 0.0f, slo = 0.0f, shi = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; i++) { sxlo += xv[i]; sxhi += xv[16 + i]; }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const uint32_t lo = qw[k] & 0x0f0f0f0fu, hi = (qw[k] >> 4) & 0x0f0f0f0fu;
+      slo = fmaf(cvt_ub0(lo), xv[4 * k], slo);     slo = fmaf(cvt_ub1(lo), xv[4 * k + 1], slo);
+      slo = fmaf(cvt_ub2(lo), xv[4 * k + 2], slo); slo = fmaf(cvt_ub3(lo), xv[4 * k + 3], slo);
+      shi = fmaf(cvt_ub0(hi), xv[16 + 4 * k], shi);     shi = fmaf(cvt_ub1(hi), xv[16 + 4 * k + 1], shi);
+      shi = fmaf(cvt_ub2(hi), xv[16 + 4 * k + 2], shi); shi = fmaf(cvt_ub3(hi), xv[16 + 4 * k + 3], shi);
+    }
+    uint32_t sc, mn; q4k_scale_pair(w.hdr.y, w.hdr.z, w.hdr.w, (un & 7) >> 1, sc, mn);
+    const float d = __half2float(__ushort_as_half((unsigned short)(w.hdr.x & 0xffffu)));
+    const float dmin = __half2float(__ushort_as_half((unsigned short)(w.hdr.x >> 16)));
+    return acc + (d * (cvt_ub0(sc) * slo + cvt_ub1(sc) * shi) - dmin * (cvt_ub0(mn) * sxlo + cvt_ub1(mn) * sxhi));
+  } else if constexpr (QT == CAI_Q6_K) {
+    uint32_t cj[4]; q6k_codes(w.q.x, w.q.y, w.q.z, cj);
+    const int hs = (un & 4) ? 8 : 0;    // positions 16..31 of a 32-run use the odd scale of the pair
+    const uint32_t s01 = w.hdr.x >> hs, s23 = w.hdr.y >> hs;
+    const float sc[4] = {(float)(int8_t)(s01 & 0xff), (float)(int8_t)((s01 >> 16) & 0xff), (float)(int8_t)(s23 & 0xff), (float)(int8_t)((s23 >> 16) & 0xff)};
+    float part = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const float sx = (xv[4 * j] + xv[4 * j + 1]) + (xv[4 * j + 2] + xv[4 * j + 3]);
+      float sq = cvt_ub0(cj[j]) * xv[4 * j];
+      sq = fmaf(cvt_ub1(cj[j]), xv[4 * j + 1], sq); sq = fmaf(cvt_ub2(cj[j]), xv[4 * j + 2], sq); sq = fmaf(cvt_ub3(cj[j]), xv[4 * j + 3], sq);
+      part = fmaf(sc[j], fmaf(-32.0f, sx, sq), part);
+    }
+    return fmaf(__half2float(__ushort_as_half(w.dh)), part, acc);
+  } else if constexpr (QT == CAI_Q4_0) {
+    float sx = 0.0f, sq = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 32; i++) sx += xv[i];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const uint32_t lo = qw[k] & 0x0f0f0f0fu, hi = (qw[k] >> 4) & 0x0f0f0f0fu;
+      sq = fmaf(cvt_ub0(lo), xv[4 * k], sq);     sq = fmaf(cvt_ub1(lo), xv[4 * k + 1], sq);
+      sq = fmaf(cvt_ub2(lo), xv[4 * k + 2], sq); sq = fmaf(cvt_ub3(lo), xv[4 * k + 3], sq);
+      sq = fmaf(cvt_ub0(hi), xv[16 + 4 * k], sq);     sq = fmaf(cvt_ub1(hi), xv[16 + 4 * k + 1], sq);
+      sq = fmaf(cvt_ub2(hi), xv[16 + 4 * k + 2], sq); sq = fmaf(cvt_ub3(hi), xv[16 + 4 * k + 3], sq);
+    }
+    return fmaf(__half2float(__ushort_as_half(w.dh)), sq - 8.0f * sx, acc);
+  } else {
+    float sq = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      sq = fmaf((float)(int8_t)(qw[k] & 0xff), xv[4 * k], sq);
+      sq = fmaf((float)(int8_t)((qw[k] >> 8) & 0xff), xv[4 * k + 1], sq);
+      sq = fmaf((float)(int8_t)((qw[k] >> 16) & 0xff), xv[4 * k + 2], sq);
+      sq = fmaf((float)(int8_t)(qw[k] >> 24), xv[4 * k + 3], sq);
+    }
+    return fmaf(__half2float(__ushort_as_half(w.dh)), sq, acc);
+  }
+}
+
+template <int QT, int R, int MODE, bool BANK, int SV>
+__global__ __launch_bounds__(256) void gemv_one(const float* hx, const uint8_t* hw0, const uint8_t* haux0, const float* hgain, const float* hres, const int hcols, const int hrows0, const int hgrp0, const int hnseg, const GemvParams p)
+{
+  extern __shared__ float4 xs4[];          // [kp/4]
+  const unsigned long long tl0 = timeline_now();
+  constexpr int UW = QTraits<QT>::UW, T = QTraits<QT>::T;
+  constexpr int RR = MODE == 1 ? 2 * R : R;  // weight rows per wave
+  constexpr int PF = RR == 1 ? 4 : MODE == 0 && R == 4 ? 1 : 2;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int grp = blockIdx.x * 4 + wave, cols = hcols;
+  const float* xin = hx; float* yout = p.y;
+  int64_t bank_row = 0;
+  if constexpr (BANK) { xin += (int64_t)blockIdx.y * p.x_slot_stride; yout += (int64_t)blockIdx.y * p.y_slot_stride; }
+  // the activation (up to 1024 SV columns)
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  const int n4 = cols >> 2;
+  f4 v[SV], g[SV];
+  {
+    const f4* gp = reinterpret_cast<const f4*>(hgain ? hgain : xin);      // (no gain: any readable values)
+#pragma unroll
+    for (int u = 0; u < SV; u++) { const int n = min((int)threadIdx.x + u * 256, n4 - 1); v[u] = reinterpret_cast<const f4*>(xin)[n]; g[u] = gp[n]; }
+  }
+  // segment lookup (groups never straddle segments)
+  int s = 0, grp0 = 0;
+  if (hnseg > 1 && grp >= hgrp0) { s = 1; grp0 = hgrp0; }
+  if (hnseg > 2 && grp >= p.seg[1].grp_end) { s = 2; grp0 = p.seg[1].grp_end; }
+  const uint8_t* data = hw0; const uint8_t* aux = haux0; int rows = hrows0;
+  if (s) { data = p.seg[s].data; aux = p.seg[s].aux; rows = p.seg[s].rows; }
+  const int row_first = (grp - grp0) * R;
+  const bool wave_live = s ? grp < p.seg[hnseg - 1].grp_end : grp < hgrp0;
+  if constexpr (BANK)
+    bank_row = (int64_t)min(max(p.slot_expert[blockIdx.y], 0), p.bank_experts - 1) * p.expert_rows;   // an id outside the bank (a router fed NaN) must not address memory
+  int64_t row_bytes, aux_row_bytes = 0;
+  if (QT == CAI_Q4_K) row_bytes = (int64_t)(cols >> 8) * 144;
+  else if (QT == CAI_Q6_K) { row_bytes = (int64_t)(cols >> 8) * 192; aux_row_bytes = (cols >> 8) * 16; }
+  else if (QT == CAI_Q4_0) { row_bytes = cols >> 1; aux_row_bytes = (cols >> 5) * 2; }
+  else if (QT == CAI_I8ROW) row_bytes = cols;
+  else { row_bytes = cols; aux_row_bytes = (cols >> 5) * 2; }
+  const uint8_t* rp[RR]; const uint8_t* ap[RR]; const uint8_t* dp[RR];
+#pragma unroll
+  for (int r = 0; r < RR; r++) {
+    int row = row_first + (MODE == 1 ? (r >> 1) : r);
+    if (!(wave_live && row < rows)) row = 0;
+    if (MODE == 1 && (r & 1)) row += rows;
+    rp[r] = data + (bank_row + row) * row_bytes;
+    ap[r] = aux + (bank_row + row) * aux_row_bytes;
+    dp[r] = QT == CAI_Q6_K ? p.seg_aux2[s] + (bank_row + row) * (int64_t)(cols >> 8) * 2 : nullptr;
+  }
+  const int n_units = cols / UW, n_steps = (n_units + 63) >> 6;
+  Unit<QT> w[PF][RR];
+  auto load_step = [&](int st, Unit<QT> (&to)[RR]) {
+    const int un = min(st * 64 + lane, n_units - 1);
+#pragma unroll
+    for (int r = 0; r < RR; r++) load_unit<QT>(rp[r], ap[r], dp[r], un, to[r]);
+  };
+#pragma unroll
+  for (int k = 0; k < PF; k++) load_step(k, w[k]);
+  // lane l < R finishes row l of the wave's
+  const int er = min(lane, R - 1), erow = row_first + er;
+  const bool eon = lane < R && wave_live && erow < rows;
+  const int eclamp = wave_live ? min(erow, rows - 1) : 0;
+  const GemvSeg& sg = p.seg[s];
+  const int64_t eo = sg.y_off + eclamp;
+  const float eres = MODE == 0 && hres ? hres[eo] : 0.0f;
+  const float ebias = sg.bias ? sg.bias[bank_row + eclamp] : 0.0f, ebias2 = MODE == 1 && sg.bias ? sg.bias[bank_row + rows + eclamp] : 0.0f;
+  const float escale = QT == CAI_I8ROW ? reinterpret_cast<const float*>(aux)[bank_row + eclamp] : 1.0f;
+
+  // fused RMSNorm statistics (neural/neural.cl:1047-1085): inv = 1/sqrt(mean(x^2)+eps)
+  float inv_rms = 1.0f;
+  if (hgain) {
+    __shared__ float red[4];
+    float ss = 0.0f;
+#pragma unroll
+    for (int u = 0; u < SV; u++)
+      if ((int)threadIdx.x + u * 256 < n4)
+#pragma unroll
+        for (int i = 0; i < 4; i++) ss = fmaf(v[u][i], v[u][i], ss);
+    ss = wave_sum(ss);
+    if (lane == 63) red[wave] = ss;
+    __syncthreads();
+    inv_rms = 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)cols + p.norm_eps);
+  }
+#pragma unroll
+  for (int u = 0; u < SV; u++) {
+    const int n = threadIdx.x + u * 256;
+    if (n < n4) {
+      float4 t = make_float4(v[u][0], v[u][1], v[u][2], v[u][3]);
+      if (hgain) { t.x = g[u][0] * (t.x * inv_rms); t.y = g[u][1] * (t.y * inv_rms); t.z = g[u][2] * (t.z * inv_rms); t.w = g[u][3] * (t.w * inv_rms); }
+      xs4[lds_slot<QT>(n)] = t;
+    }
+  }
+  __syncthreads();
+  timeline_put(p.timeline, 0, tl0); timeline_stamp(p.timeline, 4);
+  float acc[RR];
+#pragma unroll
+  for (int r = 0; r < RR; r++) acc[r] = 0.0f;
+  for (int st0 = 0; st0 < n_steps; st0 += PF) {
+#pragma unroll
+    for (int k = 0; k < PF; k++) {
+      const int un = (st0 + k) * 64 + lane;
+      if (st0 + k < n_steps && un < n_units) {
+        const int xb0 = lds_unit_base<QT>(un);
+        float xv[UW];
+#pragma unroll
+        for (int t = 0; t < T; t++) { const float4 x = xs4[xb0 + t * 16]; xv[4 * t] = x.x; xv[4 * t + 1] = x.y; xv[4 * t + 2] = x.z; xv[4 * t + 3] = x.w; }
+#pragma unroll
+        for (int r = 0; r < RR; r++) acc[r] = unit_dot<QT>(w[k][r], xv, un, acc[r]);
+      }
+      if (st0 + k + PF < n_steps) load_step(st0 + k + PF, w[k]);
+    }
+  }
+  timeline_stamp(p.timeline, 5);
+  float mine[MODE == 1 ? 2 : 1];
+#pragma unroll
+  for (int r = 0; r < RR; r++) {
+    const float t = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wave_sum(acc[r])), 63));
+    if (MODE == 1) { if (r < 2 || lane == r >> 1) mine[MODE == 1 ? r & 1 : 0] = t; }
+    else if (r == 0 || lane == r) mine[0] = t;
+  }
+  if (eon) {
+    if (MODE == 0) {
+      float y = mine[0];
+      if (QT == CAI_I8ROW) y *= escale;    // (sum code * x) * scale, then bias (neural/neuralvolume.pas:12693-12745)
+      if (sg.bias) y += ebias;
+      y = act_apply(y, p.act);
+      if (hres) y += eres;
+      yout[eo] = y;
+    } else {
+      float up = mine[0], gate = mine[MODE == 1 ? 1 : 0];
+      if (sg.bias) { up += ebias; gate += ebias2; }
+      yout[eo] = silu_mul(up, gate);
     }
   }
   timeline_stamp(p.timeline, 7);
@@ -616,6 +763,9 @@ static int panel_len(int cols, int nb)
   return kp;
 }
 
+// (longer rows: what is held of them would be registers, and read in panels behind the weights they take longer than before them: 2000 x 12800
+// of Q8_0 12.4 us, 9.8 as gemv_fast)
+constexpr int ONE_COLS = 4096;
 template <int QT, int NB, int MODE>
 static int launch_fast_r(const GemvParams& p0, int n_groups_r, int R, int n_slots, hipStream_t st)
 {
@@ -623,6 +773,25 @@ static int launch_fast_r(const GemvParams& p0, int n_groups_r, int R, int n_slot
   const size_t lds = (size_t)NB * p.kp_lds * 4;
   const dim3 grid((n_groups_r + 3) / 4, n_slots);
   p.timeline = timeline_next((int)(grid.x * grid.y));
+  if constexpr (NB == 1) if (p.cols <= ONE_COLS) {
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, p.x, p.seg[0].data, p.seg[0].aux, p.norm_gain, p.residual, p.cols, p.seg[0].rows, p.seg[0].grp_end, p.n_seg, p);
+    };
+    auto rows = [&](auto bank, auto sv) {
+      constexpr bool BANK = decltype(bank)::value;
+      constexpr int SV = decltype(sv)::value;
+      if constexpr (MODE == 0) { if (R == 4) { go(gemv_one<QT, 4, MODE, BANK, SV>); return; } }
+      if (R == 2) go(gemv_one<QT, 2, MODE, BANK, SV>); else go(gemv_one<QT, 1, MODE, BANK, SV>);
+    };
+    auto width = [&](auto bank) {
+      using std::integral_constant;
+      if (p.cols <= 1024) rows(bank, integral_constant<int, 1>());
+      else if (p.cols <= 2048) rows(bank, integral_constant<int, 2>());
+      else rows(bank, integral_constant<int, 4>());
+    };
+    if (p.slot_expert) width(std::true_type()); else width(std::false_type());
+    return CAI_OK;
+  }
   if constexpr (NB == 1 && MODE == 0) {
     if (R == 4) { hipLaunchKernelGGL((gemv_fast<QT, NB, 4, MODE>), grid, dim3(256), lds, st, p); return CAI_OK; }
   }

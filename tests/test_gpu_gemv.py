@@ -263,6 +263,26 @@ def test_small_batch_gemm_q6_k_on_matrix_cores(rows, cols, T):
     assert rel_err(w.gemm(x), want, floor=0.02 * cols ** 0.5 * float(np.abs(x).mean())) < TIGHT   # the dispatcher's own choice
 
 
+@pytest.mark.parametrize("qt", [O.Q8_0, O.Q4_0, O.I8ROW])
+@pytest.mark.parametrize("rows,cols", [(1, 32), (3, 1024), (5, 1056), (7, 2048), (6, 2080), (9, 4064), (5, 4096), (5, 4128), (8195, 96), (8195, 2080), (32771, 160), (32771, 1056)])
+def test_one_row_of_activations_at_the_edges_of_what_a_launch_holds(qt, rows, cols):
+    """Widths around one, two and four activations a thread and past them (another kernel), one to nine steps of 64 units, rows that end inside a group
+    of one, two and four."""
+    from helpers.device import dev, rel_err
+    cai = dev()
+    scales = None
+    rng = np.random.default_rng(rows + cols)
+    if qt == O.I8ROW:
+        raw, scales = O.quant_int8_rows((rng.standard_normal((rows, cols)) * 0.02).astype(np.float32))
+    else:
+        raw, rng = make(qt, rows, cols, 1)
+    x = rng.standard_normal((1, cols)).astype(np.float32)
+    bias = (rng.standard_normal(rows) * 0.1).astype(np.float32)
+    w = cai.QWeight(qt, rows, cols, raw, bias, scales)
+    want = O.gemv(qt, raw.view(np.uint8), rows, cols, x, bias, 0, 1, scales) if qt == O.I8ROW else O.gemv(qt, raw, rows, cols, x, bias, 0, 1)
+    assert rel_err(w.gemv(x), want, floor=0.02 * cols ** 0.5) < TIGHT
+
+
 @pytest.mark.parametrize("qt,rows,cols", [(O.Q8_0, 4101, 4096), (O.Q4_0, 8203, 4096), (O.Q4_K, 8203, 4096), (O.Q6_K, 5003, 4096), (O.I8ROW, 4101, 4096), (O.I8ROW, 7001, 2400)])
 @pytest.mark.parametrize("nb", [2, 4, 8])
 def test_gemv_batch_on_large_matrix_goes_to_matrix_cores(qt, rows, cols, nb):
