@@ -1,10 +1,21 @@
 // Elementwise layer math, block dequantization, embedding gather, arg-max and the MoE router for gfx950.
 #include "cai_layered.hpp"
 #include "cai_blocks_raw.hpp"
+#include "cai_gemv_common.hpp"
 #include <string.h>
 #include <math.h>
 
 namespace cai {
+
+__device__ __forceinline__ float last_lane(float v) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63)); }
+// maximum of the wave, valid in lane 63 (wave_sum's steps; a lane without a partner keeps its own)
+__device__ __forceinline__ float wave_max(float v)
+{
+#define STEP(ctrl, rows) { const int t = __builtin_bit_cast(int, v); v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(t, t, ctrl, rows, 0xf, false))); }
+  STEP(0x111, 0xf) STEP(0x112, 0xf) STEP(0x114, 0xf) STEP(0x118, 0xf) STEP(0x142, 0xa) STEP(0x143, 0xc)
+#undef STEP
+  return v;
+}
 
 __device__ __forceinline__ float wave_sum_all(float v)
 {
@@ -308,7 +319,8 @@ int launch_moe_combine(float* x, const float* part, const float* gate, int k, in
 // a wave takes R output rows for ALL selected experts - the R x k weight rows (a lane 16 values of each per 1024 columns), the
 // k SwiGLU rows and the gates are requested together, one round trip behind the expert ids - and adds
 // sum_j gate_j * (row of expert j . mid_j) to the residual row in place (neural/neuralpretrained.pas:15372-15388).  Takes the
-// place of the gathered matrix-vector launch, its k partial rows and the mixture launch.
+// place of the gathered matrix-vector launch, its k partial rows and the mixture launch.  The residual is requested first: behind the sums it was one
+// more round trip (2048 x 1024, eight experts: 8.15 -> 7.65 us).
 template <int R>
 __global__ __launch_bounds__(256) void moe_down_mix_kernel(const int8_t* wq, const __half* wsc, const int bank_experts, const int dm, const int cols,
                                                            const float* mid, const int32_t* experts, const float* gates, const int k, float* x)
@@ -316,6 +328,7 @@ __global__ __launch_bounds__(256) void moe_down_mix_kernel(const int8_t* wq, con
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int row0 = (blockIdx.x * 4 + w) * R;
   if (row0 >= dm) return;               // (no barrier in this kernel)
+  const float before = x[min(row0 + min(lane, R - 1), dm - 1)];      // lane r < R finishes row r
   int e[8]; float g[8];
 #pragma unroll
   for (int j = 0; j < 8; j++) {
@@ -358,12 +371,10 @@ __global__ __launch_bounds__(256) void moe_down_mix_kernel(const int8_t* wq, con
         }
     }
   }
+  float mine = 0.0f;
 #pragma unroll
-  for (int r = 0; r < R; r++) {
-    float a = acc[r];
-    for (int m = 32; m >= 1; m >>= 1) a += __shfl_xor(a, m, 64);
-    if (lane == 0 && row0 + r < dm) x[row0 + r] += a;
-  }
+  for (int r = 0; r < R; r++) { const float a = last_lane(wave_sum(acc[r])); if (lane == r) mine = a; }
+  if (lane < R && row0 + lane < dm) x[row0 + lane] = before + mine;
 }
 bool moe_down_mix_supported(const cai_qw_s* w, int dm, int k)
 {
@@ -468,12 +479,10 @@ __device__ __forceinline__ uint32_t router_key(float p, bool candidate)
 __device__ __forceinline__ float router_select64(float logit, int n, int k, int renorm, int lane, int& expert_j, float& gate_j)
 {
   float v = lane < n ? logit : -3.0e38f;
-  float mx = v;
-  for (int m = 32; m >= 1; m >>= 1) mx = fmaxf(mx, __shfl_xor(mx, m, 64));
+  const float mx = last_lane(wave_max(v));
   float a = v - mx; a = a > 4000.0f ? 4000.0f : (a < -4000.0f ? -4000.0f : a);
   v = lane < n ? expf(a) : 0.0f;
-  float tot = v;
-  for (int m = 32; m >= 1; m >>= 1) tot += __shfl_xor(tot, m, 64);
+  const float tot = last_lane(wave_sum(v));
   const float inv = tot > 0.0f ? 1.0f / tot : 1.0f;
   v *= inv;
   const float pv = lane < n ? v : -1.0f;      // -1 marks "not a candidate"
@@ -563,7 +572,7 @@ int launch_router_topk(const float* logits, int n, int k, int renorm, int n_toke
 // The router of up to 64 experts in ONE launch: a work-group of four waves per four experts and token (one work-group for all
 // the rows measured slower than the two launches it replaced: a single CU streams the 128 KB of a 64 x 2048 router at about
 // 20 GB/s).  Every wave sums the squares of the row itself (no meeting before the products), takes one Q8_0 router row (a lane
-// one 32-value block per 2048 columns; the factor 1 / rms multiplies the finished sum) and stores its logit at agent scope; the
+// four of every 256 columns: with a block of 32 to a lane each request touched 64 lines, 9.6 us a launch of 64 x 2048, 8.7 here; the factor 1 / rms multiplies the finished sum) and stores its logit at agent scope; the
 // work-group that arrives last (wrapping counter per token, the hand-over of the attention merge: agent-scope stores
 // acknowledged under vmcnt(0), work-group barrier, agent-scope increment, agent-scope loads) selects (router_select64).  Takes the
 // place of the matrix-vector launch and the selection launch of a decode step (TNNetPointwiseSoftMax + TNNetTopKGate behind the
@@ -581,26 +590,28 @@ __global__ __launch_bounds__(256) void router_fused_kernel(const float* x, const
   const float* xb = x + (int64_t)t * x_stride;
   const int nblk = cols >> 5;
   float acc = 0.0f, ss = 0.0f;
-  for (int c0 = 0; c0 < nblk; c0 += 64) {
-    const bool on = c0 + lane < nblk;
-    const int blk = on ? c0 + lane : nblk - 1;
-    const uint4* src = reinterpret_cast<const uint4*>(wq + (int64_t)r * cols + 32 * blk);
-    const uint4 q0 = src[0], q1 = src[1];
-    const float sc = __half2float(wsc[(int64_t)r * nblk + blk]);
-    const uint32_t wd[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
-    float d = 0.0f;
+  for (int b0 = 0; b0 < cols; b0 += 2048) {       // eight steps of 256 columns, four to a lane: every request is contiguous, and all leave before the first is used
+    uint32_t q[8]; uint16_t sc[8]; float4 v[8], g[8];
 #pragma unroll
-    for (int q = 0; q < 8; q++) {
-      const float4 v = reinterpret_cast<const float4*>(xb + 32 * blk)[q], g = reinterpret_cast<const float4*>(gain + 32 * blk)[q];
-      const float xv[4] = {on ? v.x : 0.0f, on ? v.y : 0.0f, on ? v.z : 0.0f, on ? v.w : 0.0f};
-      const int c4 = (int)wd[q];
-      ss = fmaf(xv[0], xv[0], ss); ss = fmaf(xv[1], xv[1], ss); ss = fmaf(xv[2], xv[2], ss); ss = fmaf(xv[3], xv[3], ss);
-      d = fmaf(g.x * xv[0], (float)((c4 << 24) >> 24), d); d = fmaf(g.y * xv[1], (float)((c4 << 16) >> 24), d);
-      d = fmaf(g.z * xv[2], (float)((c4 << 8) >> 24), d); d = fmaf(g.w * xv[3], (float)(c4 >> 24), d);
+    for (int u = 0; u < 8; u++) {
+      const int c = min(b0 + 256 * u + 4 * lane, cols - 4);
+      v[u] = *reinterpret_cast<const float4*>(xb + c); g[u] = *reinterpret_cast<const float4*>(gain + c);
+      q[u] = *reinterpret_cast<const uint32_t*>(wq + (int64_t)r * cols + c);
+      sc[u] = reinterpret_cast<const uint16_t*>(wsc)[(int64_t)r * nblk + (c >> 5)];
     }
-    acc = fmaf(d, sc, acc);
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      const bool on = b0 + 256 * u + 4 * lane < cols;
+      const float xv[4] = {on ? v[u].x : 0.0f, on ? v[u].y : 0.0f, on ? v[u].z : 0.0f, on ? v[u].w : 0.0f};
+      const int c4 = (int)q[u];
+      ss = fmaf(xv[0], xv[0], ss); ss = fmaf(xv[1], xv[1], ss); ss = fmaf(xv[2], xv[2], ss); ss = fmaf(xv[3], xv[3], ss);
+      float d = (g[u].x * xv[0]) * (float)((c4 << 24) >> 24);
+      d = fmaf(g[u].y * xv[1], (float)((c4 << 16) >> 24), d);
+      d = fmaf(g[u].z * xv[2], (float)((c4 << 8) >> 24), d); d = fmaf(g[u].w * xv[3], (float)(c4 >> 24), d);
+      acc = fmaf(d, __half2float(__ushort_as_half(sc[u])), acc);
+    }
   }
-  for (int m = 32; m >= 1; m >>= 1) { ss += __shfl_xor(ss, m, 64); acc += __shfl_xor(acc, m, 64); }
+  ss = last_lane(wave_sum(ss)); acc = last_lane(wave_sum(acc));
   const float logit = acc * (1.0f / sqrtf(ss / (float)cols + eps));
   if (lane == 0 && r_own < n) __hip_atomic_store(logits_out + (int64_t)t * n + r_own, logit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __builtin_amdgcn_s_waitcnt(0x0F70);           // vmcnt(0): the logit store has been acknowledged
