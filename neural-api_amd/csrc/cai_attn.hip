@@ -1227,15 +1227,15 @@ static int launch_split_head(const AttnParams& p0, int n_seq, hipStream_t st)
   const dim3 grid(8 * G * ((items + 7) / 8), n_seq);
   p.timeline = timeline_next((int)(grid.x * grid.y));
   const int hheads = p.q_heads | p.kv_heads << 16, hgeo = p.n_splits | p.hd << 16, hsl = p.split_len | (p.window > 0 ? 1 << 16 : 0);
-  const int64_t seq_rows = p.seq_mul ? p.seq_elems / p.hd : 0;
-  if (p.q_heads > 0xffff || p.kv_heads > 0x7fff || p.n_splits > 0xffff || p.split_len > 0xffff || seq_rows > 0x7fffffff || p.qkv_stride > 0x7fffffff)
+  const int64_t seq_rows = p.seq_mul && n_seq > 1 ? p.seq_elems / p.hd : 0, qkv_stride = n_seq > 1 ? p.qkv_stride : 0;
+  if (p.q_heads > 0xffff || p.kv_heads > 0x7fff || p.n_splits > 0xffff || p.split_len > 0xffff || seq_rows > 0x7fffffff || qkv_stride > 0x7fffffff)
     return set_error(CAI_ERR_UNSUPPORTED, "attention: %d query heads, %d slices of %d rows, sequences of %lld rows", p.q_heads, p.n_splits, p.split_len, (long long)seq_rows);
   if (p.hd > 128) return set_error(CAI_ERR_UNSUPPORTED, "attention: head_dim %d > 128", p.hd);
   const int64_t at = (p.seq0 * p.seq_elems + p.layer_off) * (int64_t)sizeof(KV_T);
   const void* hk = (const char*)p.kc + at; const void* hv = (const char*)p.vc + at;
   p.scale_row0 = p.seq0 * p.seq_rows + p.layer_row_off;
   auto put = [&](auto kern) {
-    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, p.pos, (const float*)p.qkv, hk, hv, (int)p.qkv_stride, hheads, hgeo, hsl, p.max_ctx, (int)seq_rows, p);
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, p.pos, (const float*)p.qkv, hk, hv, (int)qkv_stride, hheads, hgeo, hsl, p.max_ctx, (int)seq_rows, p);
   };
   auto go = [&](auto vw, auto nv) {
     constexpr int VW = decltype(vw)::value, NV = decltype(nv)::value;
