@@ -1,11 +1,12 @@
-// Small-batch (2..8 tokens) Q4_K and Q6_K linear layer on the matrix cores, register-resident form: the decode step of a few sequences
+// Small-batch (2..8 tokens) Q4_K, Q6_K and Q8_0 linear layer on the matrix cores, register-resident form: the decode step of a few sequences
 // with ONE launch per linear layer (no activation pre-pass, no slice reduction launch).
 //
 // The arithmetic is that of gemm_q4k_nb (cai_gemm_nb.hip): A operand = sc_j * q (exact in f16), B operand = the activations
 // of up to 8 tokens, scaled per (token, 256-block) by a power of two and split hi + lo into two f16 = the 16 columns of
 // v_mfma_f32_16x16x32_f16, one more MFMA per row set and super-block for the - dmin * mn_j * sum_j(x) term
 // (Q4_K: neural/neuralgguf.pas:472-514); for Q6_K that of gemm_q6k_nb: one v_mfma_f32_16x16x16_f16 a scale group of 16 weights, activations
-// as the rows of the result, so that a lane multiplies by the scale it loaded itself.  What differs is who holds what:
+// as the rows of the result, so that a lane multiplies by the scale it loaded itself; for Q8_0 that of gemm_blk_nb, the same with one
+// v_mfma_f32_16x16x32_f16 a block.  What differs is who holds what:
 //   * a WAVE owns two super-blocks (512 columns) of EVERY row its work-group walks, so the B operands of its 16 MFMA steps
 //     never change: it reads its 8 x 512 activations as fp32 once, applies the RMSNorm gain, finds the block scales, splits
 //     hi + lo and keeps the operands in 64 registers for the whole launch - no activation planes in memory, no LDS traffic
@@ -134,7 +135,7 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
   const int nwa = (nS + RA_SBW - 1) / RA_SBW;                              // waves of this work-group with columns to cover
   const int nsw = max(0, min(RA_SBW, nS - RA_SBW * wave));                  // super-blocks of this wave
   const int sbw0 = sb0 + min(RA_SBW * wave, nS - 1);                        // its first one (an idle wave re-reads the last)
-  constexpr bool Q6 = QT == CAI_Q6_K;
+  constexpr bool Q6 = QT == CAI_Q6_K, Q8 = QT == CAI_Q8_0, SWAPPED = Q6 || Q8;      // SWAPPED: the activations are the rows of a result
   const int npw = bx < hnpairs ? (hnpairs - bx + n_bx - 1) / n_bx : 0;   // pairs of this work-group
   const int nq = RA_SBW * npw;                                              // (pair, super-block) items of a wave
   const int tok = n & (RA_TK - 1), tokc = min(tok, hntok - 1);
@@ -153,7 +154,8 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
 
   struct W4 { uint4 h[HH], q[HH][2]; };
   struct W6 { u32x4_t ql[HH][2], qh[HH], sc[HH]; uint32_t d[HH]; };
-  using WRegs = std::conditional_t<Q6, W6, W4>;
+  struct W8 { u32x4_t q[HH][4], sc[HH]; };
+  using WRegs = std::conditional_t<Q6, W6, std::conditional_t<Q8, W8, W4>>;
   // weights of item q = (pair q / 2, super-block q % 2 of this wave): for the rows n of both row sets the header and this
   // lane's 2 x 16 quant bytes.  Loads are never conditional: past the last item the last one is fetched again (a cache hit).
   auto load_w = [&](int q, WRegs& r) __attribute__((always_inline)) {
@@ -170,6 +172,10 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
         r.qh[hh] = *reinterpret_cast<const u32x4_t*>(blk + 128 + 16 * kg);
         r.sc[hh] = *reinterpret_cast<const u32x4_t*>(sg->aux + b * 16);
         r.d[hh] = *reinterpret_cast<const uint16_t*>(sg->aux2 + b * 2);
+      } else if constexpr (Q8) {           // 256 codes; the scales of their eight blocks
+#pragma unroll
+        for (int i = 0; i < 4; i++) r.q[hh][i] = *reinterpret_cast<const u32x4_t*>(sg->w + b * 256 + 64 * i + 16 * kg);
+        r.sc[hh] = *reinterpret_cast<const u32x4_t*>(sg->aux + b * 16);
       } else {
         const uint8_t* blk = sg->w + b * RA_BB;
         r.h[hh] = *reinterpret_cast<const uint4*>(blk);
@@ -242,7 +248,7 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
         *reinterpret_cast<uint2*>(xw + t8 * RA_XLD + j * 256 + 64 * m + 4 * ii) = make_uint2(__builtin_bit_cast(uint32_t, h02), __builtin_bit_cast(uint32_t, h13));
         *reinterpret_cast<uint2*>(xw + (8 + t8) * RA_XLD + j * 256 + 64 * m + 4 * ii) = make_uint2(__builtin_bit_cast(uint32_t, l02), __builtin_bit_cast(uint32_t, l13));
         // sub-block 2 m + i / 8 of the block: the sum of 8 lanes' values, / 32, hi + lo
-        if constexpr (Q6) continue;
+        if constexpr (SWAPPED) continue;
         sm = ra_oct_sum(sm) * 0.03125f;
         const _Float16 qh = (_Float16)sm, ql = (_Float16)(sm - (float)qh);
         if ((ii & 7) == 0) { sxw[t8 * 16 + j * 8 + 2 * m + (ii >> 3)] = qh; sxw[(8 + t8) * 16 + j * 8 + 2 * m + (ii >> 3)] = ql; }
@@ -261,6 +267,10 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
 #pragma unroll
       for (int gi = 0; gi < 16; gi++) Xg[j][gi] = *reinterpret_cast<const half4_t*>(xw + n * RA_XLD + j * 256 + 16 * gi + 4 * kg);
       sinv4[j] = *reinterpret_cast<const float4*>(sinvw + j * RA_TK + 4 * c1);      // row 4 kg + i of a result: token (4 kg + i) % 8
+    } else if constexpr (Q8) {             // block t: what the exchange of halves below leaves in this lane, weights 16 c1 + 8 g .. + 7
+#pragma unroll
+      for (int t = 0; t < 8; t++) Bx[j][t] = *reinterpret_cast<const half8_t*>(xw + n * RA_XLD + j * 256 + 32 * t + 16 * c1 + 8 * g);
+      sinv4[j] = *reinterpret_cast<const float4*>(sinvw + j * RA_TK + 4 * c1);
     } else {
 #pragma unroll
       for (int t = 0; t < 8; t++)
@@ -270,7 +280,7 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
     sinv[j] = sinvw[j * RA_TK + tok];
   }
   __builtin_amdgcn_wave_barrier();    // (the region is written again as the wave's shares of a pair)
-  if constexpr (!Q6) load_w(2, wc);
+  if constexpr (!SWAPPED) load_w(2, wc);
   timeline_stamp_after(p.timeline, 3, sinv[RA_SBW - 1]);
   timeline_stamp(p.timeline, 4);
   // what the finishing wave of a pair adds to the rows (bias, residual) is requested when the pair starts: by every wave, so
@@ -340,6 +350,34 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
         acc[hh][0] = fmaf(sinv4[j].x, gs[0], acc[hh][0]); acc[hh][1] = fmaf(sinv4[j].y, gs[1], acc[hh][1]);
         acc[hh][2] = fmaf(sinv4[j].z, gs[2], acc[hh][2]); acc[hh][3] = fmaf(sinv4[j].w, gs[3], acc[hh][3]);
       }
+    } else if constexpr (Q8) {
+      const float4_t z4 = {0.0f, 0.0f, 0.0f, 0.0f};
+      const half2_t o2 = {(_Float16)(-1152.0f), (_Float16)(-1152.0f)};   // 1024 + (code + 128) - 1152
+#pragma unroll
+      for (int hh = 0; hh < HH; hh++) {
+        float gs[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          // lanes kg 0, 1 asked for block 2 i, kg 2, 3 for block 2 i + 1: the halves change places, and each block is in all four
+          const u32x4_t v = r.q[hh][i];
+          const uint2_t xz = __builtin_amdgcn_permlane32_swap(v.x, v.z, false, false);
+          const uint2_t yw = __builtin_amdgcn_permlane32_swap(v.y, v.w, false, false);
+          const uint32_t scw = i == 0 ? r.sc[hh].x : i == 1 ? r.sc[hh].y : i == 2 ? r.sc[hh].z : r.sc[hh].w;
+#pragma unroll
+          for (int e = 0; e < 2; e++) {
+            const uint32_t c0 = (e ? xz.y : xz.x) ^ 0x80808080u, c1w = (e ? yw.y : yw.x) ^ 0x80808080u;
+            const half2_t a = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, c0, 0x04020400u)) + o2, b = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, c0, 0x04030401u)) + o2;
+            const half2_t c = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, c1w, 0x04020400u)) + o2, d = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, c1w, 0x04030401u)) + o2;
+            const half8_t W = {a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
+            const float ds = __half2float(__ushort_as_half((unsigned short)(e ? scw >> 16 : scw & 0xffffu)));
+            const float4_t C = __builtin_amdgcn_mfma_f32_16x16x32_f16(Bx[j][2 * i + e], W, z4, 0, 0, 0);
+#pragma unroll
+            for (int k = 0; k < 4; k++) gs[k] = fmaf(ds, C[k], gs[k]);
+          }
+        }
+        acc[hh][0] = fmaf(sinv4[j].x, gs[0], acc[hh][0]); acc[hh][1] = fmaf(sinv4[j].y, gs[1], acc[hh][1]);
+        acc[hh][2] = fmaf(sinv4[j].z, gs[2], acc[hh][2]); acc[hh][3] = fmaf(sinv4[j].w, gs[3], acc[hh][3]);
+      }
     } else {
     float4_t C[HH], Cm[HH];
     half2_t s2[HH][4], c2[HH][4];
@@ -399,7 +437,7 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
   // ---- end of a pair: every wave leaves its share (column t hi + column 8 + t lo), one wave finishes the rows ----
   auto pair_end = [&](int i, const Extra& f) __attribute__((always_inline)) {
     const int slot = i & 1;
-    if (Q6 && nsw > 0) {     // result row 4 kg + i = token (4 kg + i) % 8, hi (kg < 2) or lo: they meet across kg ^ 2; column n = weight row n
+    if (SWAPPED && nsw > 0) {     // result row 4 kg + i = token (4 kg + i) % 8, hi (kg < 2) or lo: they meet across kg ^ 2; column n = weight row n
 #pragma unroll
       for (int hh = 0; hh < HH; hh++)
 #pragma unroll
@@ -408,7 +446,7 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
           if (kg < 2) reinterpret_cast<float*>(wl)[(slot * 32 + (n >> 2) * 8 + 4 * kg + k) * 8 + 4 * hh + (n & 3)] = t;
         }
     }
-    if (!Q6 && nsw > 0) {
+    if (!SWAPPED && nsw > 0) {
       float tot[4 * HH];
 #pragma unroll
       for (int hh = 0; hh < HH; hh++)
@@ -475,7 +513,7 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
     }
   };
 
-  if constexpr (Q6)       // (two items on their way are what the registers hold)
+  if constexpr (SWAPPED)       // (two items on their way are what the registers hold)
     for (int i = 0; i < npw; i++) {
       prefetch(i, ea);
       compute(wa, 0); load_w(2 * i + 2, wa);
@@ -623,14 +661,14 @@ size_t ra_part_floats(int64_t rows, int64_t cols)
   return (size_t)ns_max * RA_TK * (size_t)((rows + 3) / 4 * 4);
 }
 
-// Whether ra_gemm takes these matrices: Q4_K or Q6_K, one width of whole super-blocks, whole 16-row sets,
+// Whether ra_gemm takes these matrices: Q4_K, Q6_K or Q8_0, one width of whole super-blocks, whole 16-row sets,
 // one column slice when the product carries an RMSNorm or SwiGLU.
 bool ra_supported(const cai_qw_s* const* ws, int n_w, bool normed, int swiglu_half)
 {
   if (n_w < 1 || n_w > 3 || (swiglu_half > 0 && n_w != 1)) return false;
   for (int i = 0; i < n_w; i++) {
     const cai_qw_s* w = ws[i];
-    if ((w->qtype != CAI_Q4_K && w->qtype != CAI_Q6_K) || w->cols != ws[0]->cols || w->cols % 256 || w->cols < 256 || w->rows % 16) return false;
+    if ((w->qtype != CAI_Q4_K && w->qtype != CAI_Q6_K && w->qtype != CAI_Q8_0) || w->cols != ws[0]->cols || w->cols % 256 || w->cols < 256 || w->rows % 16) return false;
   }
   if (swiglu_half > 0 && (ws[0]->rows != 2 * (int64_t)swiglu_half || swiglu_half % 16)) return false;
   // a product with an RMSNorm or SwiGLU must be one column slice (its finishing wave needs the whole row's sum of squares and
@@ -680,9 +718,12 @@ int ra_gemm(const cai_qw_s* const* ws, const int* y_off, int n_w, int n_tok, con
   if (n_tok < 1 || n_tok > RA_TK || !ra_supported(ws, n_w, gain != nullptr, swiglu_half))
     return set_error(CAI_ERR_UNSUPPORTED, "small-batch product (register form): %d matrices, %d tokens", n_w, n_tok);
   if (gain && swiglu_half == 0 && !residual) {
-    bool four = false, six = false, pairs = true;
-    for (int i = 0; i < n_w; i++) { (ws[i]->qtype == CAI_Q6_K ? six : four) = true; pairs = pairs && (ws[i]->qtype == CAI_Q6_K || ws[i]->rows % 32 == 0); }
-    if (four && six && pairs) return ra_two(ws, y_off, n_w, n_tok, x, x_stride, gain, eps, y, y_stride);
+    bool four = false, six = false, other = false;
+    for (int i = 0; i < n_w; i++) {
+      (ws[i]->qtype == CAI_Q6_K ? six : four) = true;
+      other = other || ws[i]->qtype == CAI_Q8_0 || (ws[i]->qtype == CAI_Q4_K && ws[i]->rows % 32);
+    }
+    if (four && six && !other) return ra_two(ws, y_off, n_w, n_tok, x, x_stride, gain, eps, y, y_stride);
   }
   for (int i = 1; i < n_w; i++)
     if (ws[i]->qtype != ws[0]->qtype) {      // (one type after the other)
@@ -732,7 +773,9 @@ int ra_gemm(const cai_qw_s* const* ws, const int* y_off, int n_w, int n_tok, con
     else if (HH == 2) RA_LAUNCH(QTv, 2, false); \
     else if (gain) RA_LAUNCH(QTv, 1, true); \
     else RA_LAUNCH(QTv, 1, false); } while (0)
-  if (ws[0]->qtype == CAI_Q6_K) RA_TYPE(CAI_Q6_K); else RA_TYPE(CAI_Q4_K);
+  if (ws[0]->qtype == CAI_Q6_K) RA_TYPE(CAI_Q6_K);
+  else if (ws[0]->qtype == CAI_Q8_0) RA_TYPE(CAI_Q8_0);
+  else RA_TYPE(CAI_Q4_K);
 #undef RA_TYPE
 #undef RA_LAUNCH
   return CAI_OK;

@@ -187,15 +187,15 @@ def test_batched_decode_and_prompt_of_a_q4k_q6k_mix_equal_single_steps():
     assert rel_err(lg, last) < 1e-3 and am == int(np.argmax(last))
 
 
-@pytest.mark.parametrize("types", ["444444", "666666", "446466", "664644", "646446"])      # q, k, v, gate|up, down, head
+@pytest.mark.parametrize("types", ["444444", "666666", "446466", "664644", "646446", "888888", "848684", "468848"])      # q, k, v, gate|up, down, head
 @pytest.mark.parametrize("d,heads,kv,ffn,vocab", [(512, 8, 2, 1024, 608), (256, 16, 2, 512, 601), (768, 16, 2, 4352, 1296)])
-def test_batched_decode_of_q4k_and_q6k_matrices_equals_single(types, d, heads, kv, ffn, vocab):
-    """One to three super-blocks a row (waves with one, with none), 17 (slices), matrices of both types over one set of
+def test_batched_decode_of_q4k_q6k_and_q8_matrices_equals_single(types, d, heads, kv, ffn, vocab):
+    """One to three super-blocks a row (waves with one, with none), 17 (slices), matrices of several types over one set of
     activations, vocabularies that are no whole row sets; 2, 3 and 8 sequences.  Two layers of sums whose operands are held to 22 bits."""
     from helpers.device import dev
     cai = dev()
     cfg = dict(n_layers=2, d_model=d, n_q_heads=heads, n_kv_heads=kv, head_dim=d // heads, ffn=ffn, vocab=vocab, max_ctx=64, eps=1e-5, rope_theta=1e4)
-    t = [O.Q4_K if c == "4" else O.Q6_K for c in types]
+    t = [{"4": O.Q4_K, "6": O.Q6_K, "8": O.Q8_0}[c] for c in types]
     spec = synthetic_spec(cfg, t[0], head_qtype=t[5], seed=7, std=0.05, qkv_bias=True)
     rng = np.random.default_rng(8)
     for l in range(2):
