@@ -272,8 +272,8 @@ static int enqueue_step(cai_decoder_s* d, int n_b, int seq0, unsigned classes = 
   if (classes & 64u) {
     cai_qw_s* hw = d->head ? d->head : d->embed;   // tied head (neural/neuralpretrained.pas:15555-)
     const cai_qw_s* hwc = hw;
-    // (Q6_K: one launch of 123 us for 152064 x 3584 and eight sequences, where planes, product and reduction are 143)
-    if (ra_on && n_b >= 2 && n_b <= 8 && hw->qtype == CAI_Q6_K && ra_supported(&hwc, 1, true, 0)) {
+    // (one launch instead of planes, product and reduction: 152064 x 3584 of Q6_K and eight sequences 143 -> 123 us, Q8_0 100000 x 3584 28 us less)
+    if (ra_on && n_b >= 2 && n_b <= 8 && (hw->qtype == CAI_Q6_K || hw->qtype == CAI_Q8_0) && ra_supported(&hwc, 1, true, 0)) {
       if (down_pending && (rc = nb_prep_residual(d->x, dm, nullptr, 0.0f, dm, n_b))) return rc;
       const int zero = 0;
       if ((rc = ra_gemm(&hwc, &zero, 1, n_b, d->x, dm, d->final_norm, c.eps, 0, d->logits, c.vocab, nullptr))) return rc;
