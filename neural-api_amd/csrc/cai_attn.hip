@@ -953,7 +953,7 @@ __global__ __launch_bounds__(512) void attn_merge_kernel(const int32_t* hpos, co
 // requested unconditionally and before anything waits, the rows before the position has arrived (a slice begins where it begins unless a
 // sliding window cuts it; rows past the live range are read as they lie and dropped).  With requests under branches and rows turned to floats
 // beside them it was four to eight round trips: 28 / 4 heads of 128, 600 float rows 10.0 us a launch (7.8 here), eight sequences of 200 half
-// rows 15.5 (9.6), 9 / 3 heads of 64 and 100 float rows 7.4 (4.8).
+// rows 15.5 (8.9), 9 / 3 heads of 64 and 100 float rows 7.4 (4.8).
 // The leading scalar arguments are all that these first requests need: they arrive preloaded in scalar registers (see the Makefile), and
 // the rest of the parameter block is fetched while the requests are on their way.  hk, hv: this layer's keys and values of activation row 0's
 // sequence, hseq_rows: rows from one sequence to the next (0: all activation rows share one), hheads = query heads | KV heads << 16, hgeo =
