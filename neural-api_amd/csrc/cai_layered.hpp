@@ -51,7 +51,7 @@ __host__ __device__ inline int glu_row(int j, int up) { return (j >> 4) * 32 + u
 
 // y = W x for n_tok activation rows x[t][ldx] (zero padded to LIN_PAD columns, element type act_t); W is a CAI_BF16 matrix.
 int launch_lin(const cai_qw_s* w, int act_t, const void* x, int64_t ldx, int n_tok, const LinEpi& e);
-constexpr int LIN_FEW = 8;                  // up to so many rows take the streaming kernel
+constexpr int LIN_FEW = 8;                  // up to so many float rows take the 32-bit streaming kernel
 // Up to LIN_FEW rows of float columns x[t][ldx] through an RMS norm over the first `width` and a matrix, with one launch also through a second norm and
 // matrix (null: none).  normed: where the normed rows themselves go, ldn apart and zero padded (null: nowhere; both ldn alike).
 struct RmsLin { const cai_qw_s* w; const float* gain; LinEpi e; void* normed = nullptr; int64_t ldn = 0; };

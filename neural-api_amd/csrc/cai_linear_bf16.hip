@@ -1,4 +1,4 @@
-// Linear layers over bfloat16 weights: a streaming matrix-vector kernel for up to eight activation rows (decode) and a
+// Linear layers over bfloat16 weights: streaming kernels for up to sixteen bfloat16 or eight float activation rows (decode) and a
 // matrix-core kernel for more (prompts and mixed batches).
 //
 // Weights are row-major [out][padded in], the padding zero.  Activations are bfloat16 (matrix cores multiply bfloat16 with
@@ -12,6 +12,7 @@
 #include "cai_async_copy.hpp"
 
 #include <algorithm>
+#include <string.h>
 
 namespace cai {
 
@@ -201,9 +202,13 @@ __global__ __launch_bounds__(64 * GV_WAVES) void gemv_bf16(const uint16_t* __res
 // tile to tile.  16-byte chunk q of row r lies at q ^ r, which makes the operand reads conflict-free.  The sums of a tile meet once, in one of two
 // areas in turn.  Weights are read past the caches' replacement ("nt"): a step's do not fit the memory-side cache, and kept there one by one
 // they push each other out.
-// Per launch at 4 rows, us, by the 32-bit walk below | here: 11264 x 2048 gated 14.2 | 10.8; 2048 x 5632 10.9 | 9.3; 6200 x 2048 9.2 | 7.6;
-// 32768 x 2048 33.7 | 24.6 (5.4 TB/s).  Sixteen rows a tile: 128 work-groups for 2048 rows, 9.9 for 2048 x 5632; a ring of one slot
-// loses 2 % of a step; without "nt" 13.2 and 10.6.
+// A matrix instruction cuts what lies below the largest of its products off downwards, and a chain of them does so again at the size of the running
+// sum: whole chains were 1.4 (512 columns) to 2.3 times (8192) as far off 64 bits as the 32-bit walk above.  So each starts from zero, every second one
+// with its activations' sign changed, the difference of two joins a 64-bit sum, and the waves' parts are added in 64 bits: 0.89 times the walk's distance
+// at 512 columns, 0.73 at 2048, 0.62 at 8192 (5.3e-8; one instruction or two, 64 columns: 0.99, all products positive 1.02), for 2 to 4 % of the time.
+// Per launch at 4 rows, us, by the 32-bit walk | whole chains | here (the last two from the trace of a step, whose launches wait for what they read):
+// 11264 x 2048 gated 14.2 | 11.0 | 11.2; 2048 x 5632 10.9 | 9.3 | 9.5; 6200 x 2048 9.2 | 8.7 | 9.0; 32768 x 2048 33.7 | 25.8 | 26.9 (5.0 TB/s).
+// Sixteen rows a tile: 128 work-groups for 2048 rows, 9.9 for 2048 x 5632; a ring of one slot loses 2 % of a step; without "nt" 13.2 and 10.6 (whole chains).
 // ------------------------------------------------------------------------------------------
 constexpr int MC_WAVES = 8, MC_ROWS = 16, MC_H = 8, MC_SLOT = MC_H * 512, MC_SLOTS = 4;      // (at most MC_SLOTS slots of a row a wave)
 constexpr int mc_depth(int sb) { return sb < 2 ? 2 : sb; }  // slots of a wave's ring: a tile's, and the next one's where that is one
@@ -246,12 +251,11 @@ __global__ __launch_bounds__(64 * MC_WAVES) void gemv_bf16_mc(const uint16_t* __
     for (int u = 0; u < 8; u++) {
       const int k = min((wave + s * KS) * 256 + u * 32, ldw - 32);
       b[s][u] = *reinterpret_cast<const u32x4*>(x + min(r, n_tok - 1) * ldx + k + c * 8);
+      if (u & 1) b[s][u] ^= 0x80008000u;
     }
   int at = 0, parity = 0;
   for (int tile = blockIdx.x, turn = 0; tile < n_tiles; tile += gridDim.x, turn++) {
-    f32x4 acc[T];
-#pragma unroll
-    for (int t = 0; t < T; t++) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    double sum[T][4] = {};
 #pragma unroll
     for (int t = 0; t < T; t++)
 #pragma unroll
@@ -265,29 +269,37 @@ __global__ __launch_bounds__(64 * MC_WAVES) void gemv_bf16_mc(const uint16_t* __
           asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the slot has been read
           at = at + 1 == DEPTH ? 0 : at + 1;
           if (q_tile < n_tiles) request(); else ahead--;
-          const int left = (ldw - (wave + s * KS) * 256) >> 5;
+          const int left = (ldw - (wave + s * KS) * 256) >> 5;       // (even: rows are padded to 64 columns)
+          auto pair = [&](int u) {
+            const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+            const f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[u]), __builtin_bit_cast(bf16x8, b[s][u]), zero, 0, 0, 0);
+            const f32x4 n = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[u + 1]), __builtin_bit_cast(bf16x8, b[s][u + 1]), zero, 0, 0, 0);
+#pragma unroll
+            for (int q = 0; q < 4; q++) sum[t][q] += (double)(d[q] - n[q]);
+          };
           if (left >= 8) {
 #pragma unroll
-            for (int u = 0; u < 8; u++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[u]), __builtin_bit_cast(bf16x8, b[s][u]), acc[t], 0, 0, 0);
+            for (int u = 0; u < 8; u += 2) pair(u);
           } else {
 #pragma unroll
-            for (int u = 0; u < 8; u++) if (u < left) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[u]), __builtin_bit_cast(bf16x8, b[s][u]), acc[t], 0, 0, 0);
+            for (int u = 0; u < 8; u += 2) if (u < left) pair(u);
           }
         }
     float* const area = parts + parity * KS * part_len;
     parity ^= 1;
     if (r < n_tok)
 #pragma unroll
-      for (int t = 0; t < T; t++) *reinterpret_cast<f32x4*>(area + wave * part_len + r * (T * 16) + t * 16 + c * 4) = acc[t];
+      for (int t = 0; t < T; t++)
+        *reinterpret_cast<f32x4*>(area + wave * part_len + r * (T * 16) + t * 16 + c * 4) = f32x4{(float)sum[t][0], (float)sum[t][1], (float)sum[t][2], (float)sum[t][3]};
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // (no wait for the copies on their way)
     // (another wave's turn from tile to tile: a result's own loads wait for the copies requested before them)
     for (int o = (tid + turn * 64) & (blockDim.x - 1); o < MC_H * n_tok; o += blockDim.x) {
       const int i = o & (MC_H - 1), tok = o / MC_H, n = first_row(tile, 0) + i;
       const float* p = area + tok * (T * 16) + i;
-      float v = 0.0f, up = 0.0f;
+      double v = 0.0, up = 0.0;
       for (int w = 0; w < KS; w++) { v += p[w * part_len]; if (GLU) up += p[w * part_len + 16]; }
-      if constexpr (GLU) put_act<bf16_t>(e.h, tok * e.ldh + tile * MC_H + i, glu_pair(e.glu, e.limit, v, up));
-      else if (n < n_rows) epi_one<bf16_t>(e, n, tok, v);
+      if constexpr (GLU) put_act<bf16_t>(e.h, tok * e.ldh + tile * MC_H + i, glu_pair(e.glu, e.limit, (float)v, (float)up));
+      else if (n < n_rows) epi_one<bf16_t>(e, n, tok, (float)v);
     }
   }
 }
@@ -716,3 +728,36 @@ int bf16_linear_f32(const cai_qw_s* w, const float* x, int64_t ldx, int n_tok, f
 }
 
 }  // namespace cai
+
+using namespace cai;
+
+// One product over bfloat16 activation rows by itself, as a layered decoder's sublayers run it, on host memory: the rows of x are rounded to
+// bfloat16.  gated: w holds blocks of 16 gate and 16 up rows, y[t][rows / 2] = relu(gate) * up rounded to bfloat16.  For the tests of the
+// products (whole models bound them by a few percent only); not part of the interface in caihip.h.
+extern "C" int cai_bf16_rows(cai_qw_t w, const float* x, int n_tok, int gated, float* y)
+{
+  CAI_ENTER();
+  CAI_READY();
+  CAI_REQUIRE(w && x && y && n_tok >= 1 && w->qtype == CAI_BF16, "cai_bf16_rows: bad argument");
+  const hipStream_t st = ctx().stream;
+  const int64_t outs = gated ? w->rows / 2 : w->rows;
+  const size_t xb = (size_t)n_tok * w->cols * 4, hb = (size_t)n_tok * w->ld * 2, yb = (size_t)n_tok * outs * 4;
+  auto round = [](size_t b) { return (b + 255) / 256 * 256; };
+  char* d = nullptr;
+  CAI_HIP(hipMalloc((void**)&d, round(xb) + round(hb) + yb));
+  char* const dh = d + round(xb); char* const dy = dh + round(hb);
+  hipError_t err = hipMemcpyAsync(d, x, xb, hipMemcpyHostToDevice, st);
+  int rc = err == hipSuccess ? launch_pack_rows((const float*)d, w->cols, 0, (int)w->cols, n_tok, ACT_T_BF16, dh, w->ld) : CAI_OK;
+  LinEpi e; e.bias = w->bias;
+  if (gated) { e.mode = EPI_GLU; e.h = dy; e.ldh = outs; } else { e.y = (float*)dy; e.ldy = outs; }
+  if (err == hipSuccess && !rc) rc = launch_lin(w, ACT_T_BF16, dh, w->ld, n_tok, e);
+  if (err == hipSuccess && !rc) err = hipMemcpyAsync(y, dy, gated ? yb / 2 : yb, hipMemcpyDeviceToHost, st);
+  if (err == hipSuccess) err = hipStreamSynchronize(st);
+  (void)hipFree(d);
+  if (err != hipSuccess) return hip_fail(err, "cai_bf16_rows", __FILE__, __LINE__);
+  if (gated && !rc) {                      // (widened in place, from the last)
+    const uint16_t* h = reinterpret_cast<const uint16_t*>(y);
+    for (int64_t i = (int64_t)n_tok * outs; i-- > 0;) { const uint32_t v = (uint32_t)h[i] << 16; memcpy(y + i, &v, 4); }
+  }
+  return rc;
+}
