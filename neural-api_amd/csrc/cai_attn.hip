@@ -1106,6 +1106,17 @@ __global__ __launch_bounds__(256) void attn_split_head_kernel(const int32_t* hpo
   finish_rot(qv, qg, inv_q, q);
 #pragma unroll
   for (int i = 0; i < DS; i++) acc[i] = 0.0f;
+  // a lane's part of a score, VW elements a chain (one of 8 for two of 4: 2 % further from 64 bits)
+  auto dot_of = [&](const float (&k)[DS]) {
+    float d[NV];
+#pragma unroll
+    for (int n = 0; n < NV; n++) {
+      d[n] = q[VW * n] * k[VW * n];
+#pragma unroll
+      for (int e = 1; e < VW; e++) d[n] = fmaf(q[VW * n + e], k[VW * n + e], d[n]);
+    }
+    return NV == 2 ? d[0] + d[NV - 1] : d[0];
+  };
   auto score = [&](float dot, float k_scale) {
     const float s = row16_sum(dot) * (I8 ? k_scale * p.inv_sqrt : p.inv_sqrt);
     return p.softcap > 0.0f ? p.softcap * tanhf(s / p.softcap) : s;
@@ -1127,13 +1138,10 @@ __global__ __launch_bounds__(256) void attn_split_head_kernel(const int32_t* hpo
         }
       if constexpr (I8) if (l16 == 0) { ksc[slot] = knew_s; vsc[slot] = vnew_s; }
     }
-    float dot = 0.0f;
+    if constexpr (!I8)
 #pragma unroll
-    for (int i = 0; i < DS; i++) {
-      if constexpr (!I8) { knew[i] = kv_to_float<KV_T>(kv_from_float<KV_T>(knew[i])); vnew[i] = kv_to_float<KV_T>(kv_from_float<KV_T>(vnew[i])); }
-      dot = fmaf(q[i], knew[i], dot);
-    }
-    const float s = score(dot, knew_s);
+      for (int i = 0; i < DS; i++) { knew[i] = kv_to_float<KV_T>(kv_from_float<KV_T>(knew[i])); vnew[i] = kv_to_float<KV_T>(kv_from_float<KV_T>(vnew[i])); }
+    const float s = score(dot_of(knew), knew_s);
     if (grp == 0) {
       m = s; l = 1.0f;
 #pragma unroll
@@ -1145,12 +1153,10 @@ __global__ __launch_bounds__(256) void attn_split_head_kernel(const int32_t* hpo
     float sc[PCH], cmax = -1e30f;
 #pragma unroll
     for (int c = 0; c < PCH; c++) {
-      float kf[DS], dot = 0.0f;
+      float kf[DS];
 #pragma unroll
       for (int i = 0; i < NV; i++) row_floats<VW, KV_T>(ch.k[c][i], kf + VW * i);
-#pragma unroll
-      for (int i = 0; i < DS; i++) dot = fmaf(q[i], kf[i], dot);       // (q is 0 beyond the head width)
-      sc[c] = row16_sum(dot) * (I8 ? ch.ks[c] * p.inv_sqrt : p.inv_sqrt);
+      sc[c] = row16_sum(dot_of(kf)) * (I8 ? ch.ks[c] * p.inv_sqrt : p.inv_sqrt);       // (q is 0 beyond the head width)
     }
     if (p.softcap > 0.0f) {
 #pragma unroll
@@ -1206,12 +1212,14 @@ __global__ __launch_bounds__(256) void attn_split_head_kernel(const int32_t* hpo
 #pragma unroll
     for (int r = 1; r < NG / 16; r++) M = fmaxf(M, lane_value(Mr, 16 * r));
     const float ew = lw > 0.0f ? expf(mw - M) : 0.0f;
-    float Ls = 0.0f, A = 0.0f;
+    // (four short sums: one of sixteen is up to 15 % further from 64 bits, 30 rows of 64 1.39e-7 instead of 1.16e-7)
+    float Lp[4] = {0.0f, 0.0f, 0.0f, 0.0f}, Ap[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int w = 0; w < NG; w++) {
       const float e = lane_value(ew, w);
-      Ls = fmaf(lane_value(lw, w), e, Ls); A = fmaf(sacc[w][d], e, A);
+      Lp[w & 3] = fmaf(lane_value(lw, w), e, Lp[w & 3]); Ap[w & 3] = fmaf(sacc[w][d], e, Ap[w & 3]);
     }
+    const float Ls = (Lp[0] + Lp[1]) + (Lp[2] + Lp[3]), A = (Ap[0] + Ap[1]) + (Ap[2] + Ap[3]);
     const int qh = g * G + h;
     if (tid >= hd) {
     } else if (n_active == 1) {
