@@ -1304,11 +1304,33 @@ static int launch_group(const AttnParams& p, int n_seq, hipStream_t st)
   return CAI_OK;
 }
 
-// Whether the grouped launch of this cache takes the matrix-core kernel (CAIHIP_ATTN_GROUP_MFMA=0 keeps the VALU form).
-static bool group_takes_mfma(const AttnParams& p, int dtype)
+// Which kernel attends: one work-group per (slice, query head), or per (slice, KV head) with the whole group of query heads, that one on vector
+// instructions or on the matrix cores (half and int8 rows of 128; CAIHIP_ATTN_GROUP_MFMA=0 keeps the vector form).
+enum { ATTN_PER_HEAD = 0, ATTN_GROUPED = 1, ATTN_GROUPED_CORES = 2 };
+static int attn_form(const cai_kv_s* kv, int q_heads, int n_seq, int split_len, int n_splits, bool prompt_rows, bool normed)
 {
-  static const bool on = []() { const char* e = getenv("CAIHIP_ATTN_GROUP_MFMA"); return !(e && e[0] == '0'); }();
-  return on && (dtype == CAI_KV_F16 || dtype == CAI_KV_I8) && p.hd == 128 && p.q_heads / p.kv_heads <= 16 && p.split_len <= 256;
+  static const bool cores_on = []() { const char* e = getenv("CAIHIP_ATTN_GROUP_MFMA"); return !(e && e[0] == '0'); }();
+  const int group_min = ctx().n_cu;   // smallest grid that fills the chip with one work-group per (slice, KV head)
+  // (a cache short enough to be ONE slice may be up to 2048 rows long: the grouped kernel's per-slice score arrays in LDS are
+  // sized for ordinary slices, the per-head kernel keeps its state in registers)
+  if ((kv->head_dim & 7) != 0 || split_len > 256 || (int64_t)n_seq * kv->kv_heads * n_splits < group_min) return ATTN_PER_HEAD;
+  const bool cores = cores_on && kv->dtype != CAI_KV_F32 && kv->head_dim == 128 && q_heads / kv->kv_heads <= 16;
+  // Where both can run, the per-head kernel saves the merge launch, and the norm launch of normed q and k; the grouped one reads a row once for
+  // all its heads.  us of a layer of a decoding step, per head minus grouped, least and most over 4 to 32 KV heads, one to eight sequences and
+  // slices of 32 to 256 rows (one slice of 256: the same):
+  //   float rows, and half and int8 rows of 64: up to 512 work-groups per head -8.9 .. +0.1 (one query head a KV head, two); half and int8 rows of 64 with a
+  //     query head a KV head, up to 2048 -20 .. -0.1
+  //   half and int8 rows of 128 (grouped: on the matrix cores), a query head a KV head: slices of up to 64 rows, 1024 work-groups -5.1 .. -0.1 (2048: -1.4 ..
+  //     +0.4); int8 slices of 256, up to 2048, -2.8 .. +0.1; others -1.5 .. +3.5; two query heads a KV head -1.2 .. +2.6
+  //   the same with normed q and k: up to 512 work-groups -5.2 .. +0.3, slices of 64 up to 2048 -6.1 .. -0.5, the others -2.1 .. +7.7
+  const int64_t wgs = (int64_t)n_seq * q_heads * n_splits;
+  const bool alone = q_heads == kv->kv_heads;         // heads that share nothing
+  bool per_head;
+  if (!cores) per_head = wgs <= 512 || (alone && kv->dtype != CAI_KV_F32 && wgs <= 2048);
+  else if (normed) per_head = wgs <= 512 || (alone && split_len <= 64 && wgs <= 2048);
+  else per_head = alone && (split_len <= 64 ? wgs <= 1024 : kv->dtype == CAI_KV_I8 && split_len > 128 && n_splits > 1 && wgs <= 2048);
+  if (per_head && !prompt_rows && n_splits <= 16) return ATTN_PER_HEAD;
+  return cores ? ATTN_GROUPED_CORES : ATTN_GROUPED;
 }
 template <typename KV_T>
 static int launch_group_mfma(const AttnParams& p0, int n_seq, hipStream_t st)
@@ -1820,16 +1842,8 @@ int launch_attn_step(cai_kv_s* kv, int layer, float* qkv, int64_t qkv_stride, in
   p.evict_sinks = kv->evict_sinks; p.evict_cap = kv->evict_cap;
   p.ksc = kv->ks; p.vsc = kv->vs; p.seq_rows = kv->seq_rows(); p.layer_row_off = (int64_t)layer * kv->layer_rows();
   int rc;
-  const int group_min = c.n_cu;   // smallest grid that fills the chip with one work-group per (slice, KV head)
-  // (a cache short enough to be ONE slice may be up to 2048 rows long: the grouped kernel's per-slice score arrays in LDS are
-  // sized for ordinary slices, the per-head kernel keeps its state in registers)
-  // Few work-groups either way, or heads that share nothing (half and int8 rows; the float rows of many sequences are better off where requests
-  // stay in flight), are better off with the per-head kernel, which needs no merge launch and norms q and k itself.  us a launch per head |
-  // grouped: 16 / 16 heads of 128, float, 300 rows 7.3 | 10.0, 4000 16.6 | 18.1; half, 300 7.2 | 9.6; 16 / 16 of 64, 4000 10.7 | 15.6; a block of a
-  // decoder with four sequences, 16 / 16, half, 300 rows 46.3 | 51.8, eight 54.1 | 57.9; 28 / 4 heads, four 53.1 | 49.1.
-  const int64_t per_head_wgs = (int64_t)n_seq * q_heads * p.n_splits;
-  const bool per_head = !prompt_rows && p.n_splits <= 16 && (per_head_wgs <= 512 || (q_heads == kv->kv_heads && kv->dtype != CAI_KV_F32 && per_head_wgs <= 2048));
-  const bool grouped = !per_head && (kv->head_dim & 7) == 0 && p.split_len <= 256 && n_seq * kv->kv_heads * p.n_splits >= group_min;
+  const int form = attn_form(kv, q_heads, n_seq, p.split_len, p.n_splits, prompt_rows != 0, qn_gain != nullptr);
+  const bool grouped = form != ATTN_PER_HEAD;
   // The per-head kernel merges its slices itself (one work-group per head does a head's merge).  A prompt has more rows in
   // flight than the counters cover, and in the per-KV-head kernel the last arriver would fold a whole group of heads over
   // many slices alone (32B shape, 33 slices x 5 heads: 37.7 us against 30.7 us with the merge launch): those keep the launch.
@@ -1907,7 +1921,7 @@ int launch_attn_step(cai_kv_s* kv, int layer, float* qkv, int64_t qkv_stride, in
   }
   // one work-group per (slice, KV head) serving the whole group of query heads, or one per (slice, query head)
   // (the first fetches K and V once but has G times fewer work-groups: it needs a grid that fills the chip by itself)
-  if (grouped && group_takes_mfma(p, kv->dtype))
+  if (form == ATTN_GROUPED_CORES)
     rc = kv->dtype == CAI_KV_I8 ? launch_group_mfma<int8_t>(p, n_seq, c.stream) : launch_group_mfma<__half>(p, n_seq, c.stream);
   else if (grouped)
     rc = kv->dtype == CAI_KV_I8 ? launch_group<int8_t>(p, n_seq, c.stream) : kv->dtype == CAI_KV_F16 ? launch_group<__half>(p, n_seq, c.stream) : launch_group<float>(p, n_seq, c.stream);
@@ -2312,4 +2326,17 @@ extern "C" int cai_attn_decode(cai_kv_t kv, int layer, const float* qkv, int q_h
   CAI_HIP(hipStreamSynchronize(c.stream));
   kv->len_at(0, layer) = len + 1;
   return CAI_OK;
+}
+
+// The kernel (ATTN_PER_HEAD, ATTN_GROUPED, ATTN_GROUPED_CORES) that a decoding step of n_seq sequences over caches of `rows` rows takes.  For the tests of the
+// kernels, which say by it what they reach; host only, not part of the interface in caihip.h.
+extern "C" int cai_attn_form(int n_seq, int q_heads, int kv_heads, int head_dim, int rows, int kv_dtype, int normed)
+{
+  CAI_ENTER();
+  CAI_REQUIRE(n_seq >= 1 && kv_heads >= 1 && q_heads >= kv_heads && head_dim >= 2 && rows >= 1, "cai_attn_form: bad argument");
+  cai_kv_s kv;
+  kv.kv_heads = kv_heads; kv.head_dim = head_dim; kv.max_ctx = rows; kv.dtype = kv_dtype;
+  int split_len, n_splits;
+  kv_geometry(&kv, 0, &split_len, &n_splits);
+  return attn_form(&kv, q_heads, n_seq, split_len, n_splits, false, normed != 0);
 }
