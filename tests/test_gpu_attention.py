@@ -9,6 +9,14 @@ from helpers import oracle_lib as O
 pytestmark = pytest.mark.gpu
 
 
+PER_HEAD, GROUPED, GROUPED_CORES = 0, 1, 2
+
+
+def form(cai, hq, hkv, dk, rows, dtype):
+    """the kernel a step of one sequence takes over a cache of `rows` rows (1024, 2048, ... as the length needs, or a rolling cache's own)"""
+    return cai.load().cai_attn_form(1, hq, hkv, dk, rows, {"f32": cai.KV_F32, "f16": cai.KV_F16, "i8": cai.KV_I8}[dtype], 0)
+
+
 def oracle_run(rows, hq, hkv, dk, ctx, window=0, kv_f16=0, softcap=0.0):
     kc = np.zeros((hkv, ctx, dk), np.float32); vc = np.zeros_like(kc)
     outs = []
@@ -279,13 +287,14 @@ def oracle_run_evict(rows, hq, hkv, dk, sinks, recent, kv_f16=0):
     return np.array(outs)
 
 
-@pytest.mark.parametrize("hq,hkv,dk,ctx,sinks,recent", [(4, 2, 64, 16, 2, 4), (28, 4, 128, 128, 4, 90), (32, 16, 128, 1024, 3, 300), (6, 2, 4, 64, 0, 33)])
+@pytest.mark.parametrize("hq,hkv,dk,ctx,sinks,recent", [(4, 2, 64, 16, 2, 4), (28, 4, 128, 128, 4, 90), (32, 16, 128, 1024, 3, 300), (48, 16, 128, 1024, 3, 300), (6, 2, 4, 64, 0, 33)])
 def test_sink_and_window_eviction_matches_oracle_past_max_ctx(hq, hkv, dk, ctx, sinks, recent):
     """EnableEviction (neural/neuraldecode.pas:1257-1276, tests/TestNeuralDecode.pas:3863-3990): bit-identical to the
-    unbounded cache up to the cap, rows pinned at the cap beyond it, and the stream runs past max_ctx.  The third shape
-    takes the one-work-group-per-KV-head kernel, the others the per-query-head kernel."""
+    unbounded cache up to the cap, rows pinned at the cap beyond it, and the stream runs past max_ctx.  The shape of 48
+    heads takes the one-work-group-per-KV-head kernel (five live slices of 64 rows), the others the per-query-head kernel."""
     from helpers.device import dev
     cai = dev()
+    assert form(cai, hq, hkv, dk, ctx, "f32") == (GROUPED if hq == 48 else PER_HEAD)
     rng = np.random.default_rng(ctx + sinks)
     cap = sinks + recent
     n = max(ctx + 40, 2 * cap + 7) if ctx <= 128 else cap + 150
@@ -334,14 +343,15 @@ def test_eviction_int8_cache_tracks_fp32_cache():
     assert q.rows(0) == sinks + recent
 
 
-@pytest.mark.parametrize("hq,hkv,ctx", [(40, 8, 8192), (56, 8, 8192), (32, 16, 1024), (8, 8, 8192)])
+@pytest.mark.parametrize("hq,hkv,ctx", [(40, 8, 8192), (56, 8, 8192), (32, 16, 1024), (8, 8, 8192), (80, 16, 8192), (112, 16, 1024), (72, 72, 1024)])
 @pytest.mark.parametrize("kv", ["f16", "i8"])
 def test_grouped_decode_attention_fp16_int8(hq, hkv, ctx, kv):
-    """Grids that fill the chip (KV heads x slices >= 256) take the one-work-group-per-KV-head slice kernel (groups of
-    5, 7, 2 and 1 query heads here) with fp16 and int8 caches: same bar as the per-head kernel, int8 codes and scales
-    still exact, with a sliding window and a soft cap."""
+    """Grids that fill the chip (KV heads x slices >= 256: 16 slices of 64 rows for lengths up to 1024) take the one-work-group-per-KV-head slice
+    kernel (groups of 2, 5, 7 and 1 query heads here) with fp16 and int8 caches; the caches of 8 KV heads take the per-head kernel.  Same bar for
+    both, int8 codes and scales still exact, with a sliding window and a soft cap."""
     from helpers.device import dev
     cai = dev()
+    assert form(cai, hq, hkv, 128, 1024, kv) == (PER_HEAD if hkv == 8 else GROUPED_CORES)
     rng = np.random.default_rng(hq + ctx)
     dk, n = 128, 150
     rows = rng.standard_normal((n, (hq + 2 * hkv) * dk)).astype(np.float32)
@@ -445,7 +455,7 @@ def test_grouped_matrix_core_attention_random_geometry(seed):
     """The one-work-group-per-KV-head kernel on the matrix cores (fp16 and int8 caches of 128-wide heads) over random geometries:
     8 / 16 / 32 KV heads, 1..8 query heads per KV head, caches of 1024..12000 rows filled to a random length from the host (so the
     live range ends anywhere inside a slice, in any of its 16-row tiles), window, soft cap; a few tokens decoded on top against the
-    oracle's kernel over the same rows."""
+    oracle's kernel over the same rows.  (Four of the twelve lengths need too few slices to fill the chip and take the per-head kernel.)"""
     from helpers.device import dev
     cai = dev()
     rng = np.random.default_rng(5000 + seed)
@@ -483,12 +493,13 @@ def test_grouped_matrix_core_attention_random_geometry(seed):
         assert np.max(np.abs(got - out)) < 2e-5 * max(1.0, np.max(np.abs(out))), (i,) + what
 
 
-@pytest.mark.parametrize("hkv,G,sinks,recent", [(16, 2, 3, 130), (32, 1, 0, 300), (16, 3, 17, 40)])
+@pytest.mark.parametrize("hkv,G,sinks,recent", [(16, 2, 3, 130), (72, 1, 0, 300), (16, 3, 17, 40), (16, 3, 5, 300)])
 def test_grouped_matrix_core_attention_rolling_eviction(hkv, G, sinks, recent):
     """Sink + recent-window eviction on a half-precision cache through the same kernel: the appended row's slot lies in the middle of the
     ring, every cached row stays live."""
     from helpers.device import dev
     cai = dev()
+    assert form(cai, hkv * G, hkv, 128, 1024, "f16") == GROUPED_CORES
     rng = np.random.default_rng(hkv + sinks)
     dk, ctx, hq = 128, 1024, hkv * G
     n = sinks + recent + 40

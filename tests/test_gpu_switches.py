@@ -68,8 +68,10 @@ from helpers.model_build import oracle_model, synthetic_spec
 from helpers.device import dev, rel_err
 cai = dev()
 # 16 KV heads x 16 slices of 64 rows = 256 work-groups: the decode attention of this cache is the one-work-group-per-KV-head kernel
-cfg = dict(n_layers=2, d_model=256, n_q_heads=32, n_kv_heads=16, head_dim=128, ffn=96, vocab=512, max_ctx=1024, eps=1e-5, rope_theta=1e4,
+cfg = dict(n_layers=2, d_model=256, n_q_heads=48, n_kv_heads=16, head_dim=128, ffn=96, vocab=512, max_ctx=1024, eps=1e-5, rope_theta=1e4,
            n_experts=8, top_k=3, norm_topk=1)
+import os
+assert cai.load().cai_attn_form(1, 48, 16, 128, 1024, cai.KV_F16, 0) == (1 if os.environ.get("CAIHIP_ATTN_GROUP_MFMA") == "0" else 2)
 spec = synthetic_spec(cfg, O.Q8_0, std=0.05)
 om, dec = oracle_model(spec, kv_f16=1), cai.Decoder(spec, kv_dtype=cai.KV_F16)
 prompt = np.random.default_rng(11).integers(0, cfg["vocab"], 70).tolist()      # crosses a slice boundary
@@ -101,7 +103,9 @@ sys.path.insert(0, %(root)r); sys.path.insert(0, %(tests)r)
 from helpers.device import dev
 from test_gpu_attention import oracle_run, oracle_run_i8
 cai = dev()
-hq, hkv, dk, ctx, n = 40, 8, 128, 8192, 90          # 8 KV heads x 33 slices: the one-work-group-per-KV-head kernel
+hq, hkv, dk, ctx, n = 80, 16, 128, 8192, 90          # 16 KV heads x 16 slices: the one-work-group-per-KV-head kernel
+for dtype in (cai.KV_F16, cai.KV_I8):
+    assert cai.load().cai_attn_form(1, hq, hkv, dk, 1024, dtype, 0) == 1
 rows = np.random.default_rng(5).standard_normal((n, (hq + 2 * hkv) * dk)).astype(np.float32)
 for kv, window, softcap in (("f16", 0, 0.0), ("i8", 70, 25.0)):
     if kv == "i8":
