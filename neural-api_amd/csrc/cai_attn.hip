@@ -956,7 +956,7 @@ __global__ __launch_bounds__(512) void attn_merge_kernel(const int32_t* hpos, co
 // rows 15.5 (8.9), 9 / 3 heads of 64 and 100 float rows 7.4 (4.8).
 // The leading scalar arguments are all that these first requests need: they arrive preloaded in scalar registers (see the Makefile), and
 // the rest of the parameter block is fetched while the requests are on their way.  hk, hv: this layer's keys and values of activation row 0's
-// sequence, hseq_rows: rows from one sequence to the next (0: all activation rows share one), hheads = query heads | KV heads << 16, hgeo =
+// sequence, hseq_planes: planes of max_ctx rows from one sequence to the next (0: all activation rows share one), hheads = query heads | KV heads << 16, hgeo =
 // slices | head width << 16, hsl = rows of a slice.
 // QN: q and k carry an RMS norm over their whole rows, whose first 2048 elements are among the first requests (16 / 16 heads of 128: 8.7 -> 8.1 us a launch).
 // 16 lanes hold a row: of NV x 16 VW elements lane l has VW from 16 VW i + VW l on.  What is not waiting is instructions, one wave a SIMD: with
@@ -965,7 +965,7 @@ __global__ __launch_bounds__(512) void attn_merge_kernel(const int32_t* hpos, co
 // (100 half rows of 128: 5.5 us with four, 6.3, 9.6; 200: 7.2, 7.2, 9.6).  NCH: chunks of 64 rows on their way at once.
 template <int VW, int NV, typename KV_T, int NCH, bool QN>
 __global__ __launch_bounds__(256) void attn_split_head_kernel(const int32_t* hpos, const float* hqkv, const void* hk, const void* hv, const int hqkv_stride,
-                                                                  const int hheads, const int hgeo, const int hsl, const int hmax_ctx, const int hseq_rows, const AttnParams p)
+                                                                  const int hheads, const int hgeo, const int hsl, const int hmax_ctx, const int hseq_planes, const AttnParams p)
 {
   constexpr int DS = VW * NV, NG = 16;         // groups of 16 lanes: row j of the slice belongs to group j % NG
   const unsigned long long tl0 = timeline_now();
@@ -1000,7 +1000,7 @@ __global__ __launch_bounds__(256) void attn_split_head_kernel(const int32_t* hpo
     for (int u = 0; u < 8; u++) { tq[u] = row[min(tid + 256 * u, qw - 1)]; tk[u] = row[qw + min(tid + 256 * u, kw - 1)]; }
   }
 
-  const int64_t plane_row = (int64_t)seq * hseq_rows + (int64_t)g * hmax_ctx;
+  const int64_t plane_row = ((int64_t)seq * hseq_planes + g) * hmax_ctx;
   KV_T* const kc = reinterpret_cast<KV_T*>(const_cast<void*>(hk)) + plane_row * hd;
   KV_T* const vc = reinterpret_cast<KV_T*>(const_cast<void*>(hv)) + plane_row * hd;
   // int8 cache: codes enter the dot products as they are; the K row scale multiplies the finished score and the V row
@@ -1243,15 +1243,15 @@ static int launch_split_head(const AttnParams& p0, int n_seq, hipStream_t st)
   const dim3 grid(8 * G * ((items + 7) / 8), n_seq);
   p.timeline = timeline_next((int)(grid.x * grid.y));
   const int hheads = p.q_heads | p.kv_heads << 16, hgeo = p.n_splits | p.hd << 16, hsl = p.split_len | (p.window > 0 ? 1 << 16 : 0);
-  const int64_t seq_rows = p.seq_mul && n_seq > 1 ? p.seq_elems / p.hd : 0, qkv_stride = n_seq > 1 ? p.qkv_stride : 0;
-  if (p.q_heads > 0xffff || p.kv_heads > 0x7fff || p.n_splits > 0xffff || p.split_len > 0xffff || seq_rows > 0x7fffffff || qkv_stride > 0x7fffffff)
-    return set_error(CAI_ERR_UNSUPPORTED, "attention: %d query heads, %d slices of %d rows, sequences of %lld rows", p.q_heads, p.n_splits, p.split_len, (long long)seq_rows);
+  const int64_t seq_planes = p.seq_mul && n_seq > 1 ? p.seq_elems / ((int64_t)p.hd * p.max_ctx) : 0, qkv_stride = n_seq > 1 ? p.qkv_stride : 0;
+  if (p.q_heads > 0xffff || p.kv_heads > 0x7fff || p.n_splits > 0xffff || p.split_len > 0xffff || seq_planes > 0x7fffffff || qkv_stride > 0x7fffffff)
+    return set_error(CAI_ERR_UNSUPPORTED, "attention: %d query heads, %d slices of %d rows, rows of %lld", p.q_heads, p.n_splits, p.split_len, (long long)qkv_stride);
   if (p.hd > 128) return set_error(CAI_ERR_UNSUPPORTED, "attention: head_dim %d > 128", p.hd);
   const int64_t at = (p.seq0 * p.seq_elems + p.layer_off) * (int64_t)sizeof(KV_T);
   const void* hk = (const char*)p.kc + at; const void* hv = (const char*)p.vc + at;
   p.scale_row0 = p.seq0 * p.seq_rows + p.layer_row_off;
   auto put = [&](auto kern) {
-    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, p.pos, (const float*)p.qkv, hk, hv, (int)qkv_stride, hheads, hgeo, hsl, p.max_ctx, (int)seq_rows, p);
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, p.pos, (const float*)p.qkv, hk, hv, (int)qkv_stride, hheads, hgeo, hsl, p.max_ctx, (int)seq_planes, p);
   };
   auto go = [&](auto vw, auto nv) {
     constexpr int VW = decltype(vw)::value, NV = decltype(nv)::value;

@@ -653,3 +653,19 @@ def test_logits_reach_the_callers_memory_whole(vocab, n_b, tokens):
             dec.reset(0)
         one = dec.step(ids[b], 0 if tokens == 1 else b)[1]
         assert rel_err(one[0], got[b]) < 1e-5
+
+
+def test_sequences_of_more_than_2_31_cached_rows():
+    """Two sequences whose caches lie 129 layers x 128 heads x 131072 rows apart (rows of two halfs: 35 GB): steps of both equal steps of one, up to
+    elements on the edge between two halves, which the rounding of a batch may move by 2^-11 of themselves (5e-4; a row of another plane is 1)."""
+    from helpers.device import dev, rel_err
+    cai = dev()
+    cfg = dict(n_layers=129, d_model=256, n_q_heads=128, n_kv_heads=128, head_dim=2, ffn=64, vocab=300, max_ctx=131072, eps=1e-5, rope_theta=1e4)
+    dec = cai.Decoder(synthetic_spec(cfg, O.Q8_0, std=0.05), max_batch=2, kv_dtype=cai.KV_F16)
+    toks = np.random.default_rng(3).integers(0, 300, (2, 4))
+    both = [dec.step(toks[:, p], np.full(2, p))[1].copy() for p in range(4)]
+    for b in range(2):
+        dec.reset(0)
+        for p in range(4):
+            assert rel_err(dec.step(int(toks[b, p]), p)[1][0], both[p][b]) < 1e-3, (b, p)
+    dec.close()
