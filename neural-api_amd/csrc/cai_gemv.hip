@@ -59,6 +59,95 @@ __device__ __forceinline__ void q6k_codes(uint32_t ql0, uint32_t ql1, uint32_t q
 }
 
 // ------------------------------------------------------------------------------------------
+// A lane's share of one step of 64: UW weights of a row
+// ------------------------------------------------------------------------------------------
+template <int QT> struct Unit { uint4 q, hdr; uint16_t dh; };
+template <int QT>
+__device__ __forceinline__ void load_unit(const uint8_t* rp, const uint8_t* ap, const uint8_t* dp, int un, Unit<QT>& w)
+{
+  if constexpr (QT == CAI_Q4_K) {
+    const uint8_t* blk = rp + (int64_t)(un >> 3) * 144;
+    w.hdr = *reinterpret_cast<const uint4*>(blk);
+    w.q = *reinterpret_cast<const uint4*>(blk + 16 + 16 * (un & 7));
+  } else if constexpr (QT == CAI_Q6_K) {
+    const int sb = un >> 4, nh = (un >> 3) & 1, l4 = (un & 7) * 4;
+    const uint8_t* blk = rp + (int64_t)sb * 192;
+    w.q.x = *reinterpret_cast<const uint32_t*>(blk + 64 * nh + l4);
+    w.q.y = *reinterpret_cast<const uint32_t*>(blk + 64 * nh + 32 + l4);
+    w.q.z = *reinterpret_cast<const uint32_t*>(blk + 128 + 32 * nh + l4);
+    const uint2 sc2 = *reinterpret_cast<const uint2*>(ap + sb * 16 + 8 * nh);
+    w.hdr.x = sc2.x; w.hdr.y = sc2.y;
+    w.dh = *reinterpret_cast<const uint16_t*>(dp + sb * 2);
+  } else if constexpr (QT == CAI_Q4_0) {
+    w.q = *reinterpret_cast<const uint4*>(rp + (int64_t)un * 16);
+    w.dh = *reinterpret_cast<const uint16_t*>(ap + un * 2);
+  } else {
+    w.q = *reinterpret_cast<const uint4*>(rp + (int64_t)un * 16);
+    w.dh = QT == CAI_I8ROW ? (uint16_t)0x3C00 : *reinterpret_cast<const uint16_t*>(ap + (un >> 1) * 2);   // per-row int8: block scale 1
+  }
+}
+// acc + the unit's part of the sum; un: the unit's place in the row
+template <int QT>
+__device__ __forceinline__ float unit_dot(const Unit<QT>& w, const float (&xv)[QTraits<QT>::UW], int un, float acc)
+{
+  const uint32_t qw[4] = {w.q.x, w.q.y, w.q.z, w.q.w};
+  if constexpr (QT == CAI_Q4_K) {
+    float sxlo = 0.0f, sxhi = 0.0f, slo = 0.0f, shi = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; i++) { sxlo += xv[i]; sxhi += xv[16 + i]; }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const uint32_t lo = qw[k] & 0x0f0f0f0fu, hi = (qw[k] >> 4) & 0x0f0f0f0fu;
+      slo = fmaf(cvt_ub0(lo), xv[4 * k], slo);     slo = fmaf(cvt_ub1(lo), xv[4 * k + 1], slo);
+      slo = fmaf(cvt_ub2(lo), xv[4 * k + 2], slo); slo = fmaf(cvt_ub3(lo), xv[4 * k + 3], slo);
+      shi = fmaf(cvt_ub0(hi), xv[16 + 4 * k], shi);     shi = fmaf(cvt_ub1(hi), xv[16 + 4 * k + 1], shi);
+      shi = fmaf(cvt_ub2(hi), xv[16 + 4 * k + 2], shi); shi = fmaf(cvt_ub3(hi), xv[16 + 4 * k + 3], shi);
+    }
+    uint32_t sc, mn; q4k_scale_pair(w.hdr.y, w.hdr.z, w.hdr.w, (un & 7) >> 1, sc, mn);
+    const float d = __half2float(__ushort_as_half((unsigned short)(w.hdr.x & 0xffffu)));
+    const float dmin = __half2float(__ushort_as_half((unsigned short)(w.hdr.x >> 16)));
+    return acc + (d * (cvt_ub0(sc) * slo + cvt_ub1(sc) * shi) - dmin * (cvt_ub0(mn) * sxlo + cvt_ub1(mn) * sxhi));
+  } else if constexpr (QT == CAI_Q6_K) {
+    uint32_t cj[4]; q6k_codes(w.q.x, w.q.y, w.q.z, cj);
+    const int hs = (un & 4) ? 8 : 0;    // positions 16..31 of a 32-run use the odd scale of the pair
+    const uint32_t s01 = w.hdr.x >> hs, s23 = w.hdr.y >> hs;
+    const float sc[4] = {(float)(int8_t)(s01 & 0xff), (float)(int8_t)((s01 >> 16) & 0xff), (float)(int8_t)(s23 & 0xff), (float)(int8_t)((s23 >> 16) & 0xff)};
+    float part = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const float sx = (xv[4 * j] + xv[4 * j + 1]) + (xv[4 * j + 2] + xv[4 * j + 3]);
+      float sq = cvt_ub0(cj[j]) * xv[4 * j];
+      sq = fmaf(cvt_ub1(cj[j]), xv[4 * j + 1], sq); sq = fmaf(cvt_ub2(cj[j]), xv[4 * j + 2], sq); sq = fmaf(cvt_ub3(cj[j]), xv[4 * j + 3], sq);
+      part = fmaf(sc[j], fmaf(-32.0f, sx, sq), part);
+    }
+    return fmaf(__half2float(__ushort_as_half(w.dh)), part, acc);
+  } else if constexpr (QT == CAI_Q4_0) {
+    float sx = 0.0f, sq = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 32; i++) sx += xv[i];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const uint32_t lo = qw[k] & 0x0f0f0f0fu, hi = (qw[k] >> 4) & 0x0f0f0f0fu;
+      sq = fmaf(cvt_ub0(lo), xv[4 * k], sq);     sq = fmaf(cvt_ub1(lo), xv[4 * k + 1], sq);
+      sq = fmaf(cvt_ub2(lo), xv[4 * k + 2], sq); sq = fmaf(cvt_ub3(lo), xv[4 * k + 3], sq);
+      sq = fmaf(cvt_ub0(hi), xv[16 + 4 * k], sq);     sq = fmaf(cvt_ub1(hi), xv[16 + 4 * k + 1], sq);
+      sq = fmaf(cvt_ub2(hi), xv[16 + 4 * k + 2], sq); sq = fmaf(cvt_ub3(hi), xv[16 + 4 * k + 3], sq);
+    }
+    return fmaf(__half2float(__ushort_as_half(w.dh)), sq - 8.0f * sx, acc);
+  } else {
+    float sq = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      sq = fmaf((float)(int8_t)(qw[k] & 0xff), xv[4 * k], sq);
+      sq = fmaf((float)(int8_t)((qw[k] >> 8) & 0xff), xv[4 * k + 1], sq);
+      sq = fmaf((float)(int8_t)((qw[k] >> 16) & 0xff), xv[4 * k + 2], sq);
+      sq = fmaf((float)(int8_t)(qw[k] >> 24), xv[4 * k + 3], sq);
+    }
+    return fmaf(__half2float(__ushort_as_half(w.dh)), sq, acc);
+  }
+}
+
+// ------------------------------------------------------------------------------------------
 // Fast kernel: Q4_K / Q4_0 / Q8_0 / per-row int8.  MODE 0: plain rows.  MODE 1: SwiGLU pairs (row i and row half+i).
 // ------------------------------------------------------------------------------------------
 template <int QT, int NB, int R, int MODE>
@@ -174,6 +263,18 @@ __global__ __launch_bounds__(256) void gemv_fast(const GemvParams p)
 
     const int n_units = kp / UW;
     for (int u = lane; u < n_units; u += 64) {
+      if constexpr (NB == 1) {        // (rows of more than ONE_COLS columns: gemv_one's sums; the batch below loads as it always did, 1 to 12 % slower through load_unit)
+        const int un = k0 / UW + u;
+        Unit<QT> w[RR];
+#pragma unroll
+        for (int r = 0; r < RR; r++) load_unit<QT>(rp[r], ap[r], dp[r], un, w[r]);
+        float xv[UW];
+#pragma unroll
+        for (int t = 0; t < T; t++) { const float4 v = xs4[lds_unit_base<QT>(u) + t * 16]; xv[4 * t] = v.x; xv[4 * t + 1] = v.y; xv[4 * t + 2] = v.z; xv[4 * t + 3] = v.w; }
+#pragma unroll
+        for (int r = 0; r < RR; r++) acc[r][0] = unit_dot<QT>(w[r], xv, un, acc[r][0]);
+        continue;
+      }
       // ---- issue all weight loads of this step first ----
       uint4 q[RR]; uint4 hdr[RR]; uint16_t dh[RR];
       if (QT == CAI_Q4_K) {
@@ -361,92 +462,6 @@ __global__ __launch_bounds__(256) void gemv_fast(const GemvParams p)
 // in a step 3.5 | 3.0, 6144 x 2048 normed 7.6 | 6.3, 8 experts of 2048 x 2048 10.8 | 9.7, 49152 x 576 14.8 | 10.7; back to back 12000 x 3584 11.7 | 9.3, 36000 x 2048 17.1 | 13.5.
 // The leading scalar arguments are what these requests need of a launch of one matrix; they arrive preloaded (see the Makefile).
 // ------------------------------------------------------------------------------------------
-template <int QT> struct Unit { uint4 q, hdr; uint16_t dh; };
-template <int QT>
-__device__ __forceinline__ void load_unit(const uint8_t* rp, const uint8_t* ap, const uint8_t* dp, int un, Unit<QT>& w)
-{
-  if constexpr (QT == CAI_Q4_K) {
-    const uint8_t* blk = rp + (int64_t)(un >> 3) * 144;
-    w.hdr = *reinterpret_cast<const uint4*>(blk);
-    w.q = *reinterpret_cast<const uint4*>(blk + 16 + 16 * (un & 7));
-  } else if constexpr (QT == CAI_Q6_K) {
-    const int sb = un >> 4, nh = (un >> 3) & 1, l4 = (un & 7) * 4;
-    const uint8_t* blk = rp + (int64_t)sb * 192;
-    w.q.x = *reinterpret_cast<const uint32_t*>(blk + 64 * nh + l4);
-    w.q.y = *reinterpret_cast<const uint32_t*>(blk + 64 * nh + 32 + l4);
-    w.q.z = *reinterpret_cast<const uint32_t*>(blk + 128 + 32 * nh + l4);
-    const uint2 sc2 = *reinterpret_cast<const uint2*>(ap + sb * 16 + 8 * nh);
-    w.hdr.x = sc2.x; w.hdr.y = sc2.y;
-    w.dh = *reinterpret_cast<const uint16_t*>(dp + sb * 2);
-  } else if constexpr (QT == CAI_Q4_0) {
-    w.q = *reinterpret_cast<const uint4*>(rp + (int64_t)un * 16);
-    w.dh = *reinterpret_cast<const uint16_t*>(ap + un * 2);
-  } else {
-    w.q = *reinterpret_cast<const uint4*>(rp + (int64_t)un * 16);
-    w.dh = QT == CAI_I8ROW ? (uint16_t)0x3C00 : *reinterpret_cast<const uint16_t*>(ap + (un >> 1) * 2);   // per-row int8: block scale 1
-  }
-}
-// acc + the unit's part of the sum; un: the unit's place in the row
-template <int QT>
-__device__ __forceinline__ float unit_dot(const Unit<QT>& w, const float (&xv)[QTraits<QT>::UW], int un, float acc)
-{
-  const uint32_t qw[4] = {w.q.x, w.q.y, w.q.z, w.q.w};
-  if constexpr (QT == CAI_Q4_K) {
-    float sxlo = 0.0f, sxhi = 0.0f, slo = 0.0f, shi = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 16; i++) { sxlo += xv[i]; sxhi += xv[16 + i]; }
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-      const uint32_t lo = qw[k] & 0x0f0f0f0fu, hi = (qw[k] >> 4) & 0x0f0f0f0fu;
-      slo = fmaf(cvt_ub0(lo), xv[4 * k], slo);     slo = fmaf(cvt_ub1(lo), xv[4 * k + 1], slo);
-      slo = fmaf(cvt_ub2(lo), xv[4 * k + 2], slo); slo = fmaf(cvt_ub3(lo), xv[4 * k + 3], slo);
-      shi = fmaf(cvt_ub0(hi), xv[16 + 4 * k], shi);     shi = fmaf(cvt_ub1(hi), xv[16 + 4 * k + 1], shi);
-      shi = fmaf(cvt_ub2(hi), xv[16 + 4 * k + 2], shi); shi = fmaf(cvt_ub3(hi), xv[16 + 4 * k + 3], shi);
-    }
-    uint32_t sc, mn; q4k_scale_pair(w.hdr.y, w.hdr.z, w.hdr.w, (un & 7) >> 1, sc, mn);
-    const float d = __half2float(__ushort_as_half((unsigned short)(w.hdr.x & 0xffffu)));
-    const float dmin = __half2float(__ushort_as_half((unsigned short)(w.hdr.x >> 16)));
-    return acc + (d * (cvt_ub0(sc) * slo + cvt_ub1(sc) * shi) - dmin * (cvt_ub0(mn) * sxlo + cvt_ub1(mn) * sxhi));
-  } else if constexpr (QT == CAI_Q6_K) {
-    uint32_t cj[4]; q6k_codes(w.q.x, w.q.y, w.q.z, cj);
-    const int hs = (un & 4) ? 8 : 0;    // positions 16..31 of a 32-run use the odd scale of the pair
-    const uint32_t s01 = w.hdr.x >> hs, s23 = w.hdr.y >> hs;
-    const float sc[4] = {(float)(int8_t)(s01 & 0xff), (float)(int8_t)((s01 >> 16) & 0xff), (float)(int8_t)(s23 & 0xff), (float)(int8_t)((s23 >> 16) & 0xff)};
-    float part = 0.0f;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const float sx = (xv[4 * j] + xv[4 * j + 1]) + (xv[4 * j + 2] + xv[4 * j + 3]);
-      float sq = cvt_ub0(cj[j]) * xv[4 * j];
-      sq = fmaf(cvt_ub1(cj[j]), xv[4 * j + 1], sq); sq = fmaf(cvt_ub2(cj[j]), xv[4 * j + 2], sq); sq = fmaf(cvt_ub3(cj[j]), xv[4 * j + 3], sq);
-      part = fmaf(sc[j], fmaf(-32.0f, sx, sq), part);
-    }
-    return fmaf(__half2float(__ushort_as_half(w.dh)), part, acc);
-  } else if constexpr (QT == CAI_Q4_0) {
-    float sx = 0.0f, sq = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 32; i++) sx += xv[i];
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-      const uint32_t lo = qw[k] & 0x0f0f0f0fu, hi = (qw[k] >> 4) & 0x0f0f0f0fu;
-      sq = fmaf(cvt_ub0(lo), xv[4 * k], sq);     sq = fmaf(cvt_ub1(lo), xv[4 * k + 1], sq);
-      sq = fmaf(cvt_ub2(lo), xv[4 * k + 2], sq); sq = fmaf(cvt_ub3(lo), xv[4 * k + 3], sq);
-      sq = fmaf(cvt_ub0(hi), xv[16 + 4 * k], sq);     sq = fmaf(cvt_ub1(hi), xv[16 + 4 * k + 1], sq);
-      sq = fmaf(cvt_ub2(hi), xv[16 + 4 * k + 2], sq); sq = fmaf(cvt_ub3(hi), xv[16 + 4 * k + 3], sq);
-    }
-    return fmaf(__half2float(__ushort_as_half(w.dh)), sq - 8.0f * sx, acc);
-  } else {
-    float sq = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-      sq = fmaf((float)(int8_t)(qw[k] & 0xff), xv[4 * k], sq);
-      sq = fmaf((float)(int8_t)((qw[k] >> 8) & 0xff), xv[4 * k + 1], sq);
-      sq = fmaf((float)(int8_t)((qw[k] >> 16) & 0xff), xv[4 * k + 2], sq);
-      sq = fmaf((float)(int8_t)(qw[k] >> 24), xv[4 * k + 3], sq);
-    }
-    return fmaf(__half2float(__ushort_as_half(w.dh)), sq, acc);
-  }
-}
-
 template <int QT, int R, int MODE, bool BANK, int SV>
 __global__ __launch_bounds__(256) void gemv_one(const float* hx, const uint8_t* hw0, const uint8_t* haux0, const float* hgain, const float* hres, const int hcols, const int hrows0, const int hgrp0, const int hnseg, const GemvParams p)
 {

@@ -264,10 +264,10 @@ def test_small_batch_gemm_q6_k_on_matrix_cores(rows, cols, T):
 
 
 @pytest.mark.parametrize("qt", [O.Q8_0, O.Q4_0, O.I8ROW])
-@pytest.mark.parametrize("rows,cols", [(1, 32), (3, 1024), (5, 1056), (7, 2048), (6, 2080), (9, 4064), (5, 4096), (5, 4128), (8195, 96), (8195, 2080), (32771, 160), (32771, 1056)])
+@pytest.mark.parametrize("rows,cols", [(1, 32), (3, 1024), (5, 1056), (7, 2048), (6, 2080), (9, 4064), (5, 4096), (5, 4128), (8195, 96), (8195, 2080), (32771, 160), (32771, 1056), (8195, 4128), (32771, 5152), (5, 18912)])
 def test_one_row_of_activations_at_the_edges_of_what_a_launch_holds(qt, rows, cols):
-    """Widths around one, two and four activations a thread and past them (another kernel), one to nine steps of 64 units, rows that end inside a group
-    of one, two and four."""
+    """Widths around one, two and four activations a thread and past them (another kernel, up to three panels), one to nine steps of 64 units, rows that end
+    inside a group of one, two and four."""
     from helpers.device import dev, rel_err
     cai = dev()
     scales = None
