@@ -20,19 +20,6 @@
 
 namespace cai {
 
-// sum over each half-wave (32 lanes), result in every lane of that half
-__device__ __forceinline__ float half_wave_allsum(float v)
-{
-  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x111, 0xf, 0xf, true));
-  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x112, 0xf, 0xf, true));
-  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x114, 0xf, 0xf, true));
-  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x118, 0xf, 0xf, true));
-  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x142, 0xa, 0xf, true));
-  const float lo = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 31));
-  const float hi = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
-  return (threadIdx.x & 32) ? hi : lo;
-}
-
 template <typename T> __device__ __forceinline__ float kv_to_float(T v);
 template <> __device__ __forceinline__ float kv_to_float<float>(float v) { return v; }
 template <> __device__ __forceinline__ float kv_to_float<__half>(__half v) { return __half2float(v); }
@@ -967,7 +954,7 @@ template <int VW, int NV, typename KV_T, int NCH, bool QN>
 __global__ __launch_bounds__(256) void attn_split_head_kernel(const int32_t* hpos, const float* hqkv, const void* hk, const void* hv, const int hqkv_stride,
                                                                   const int hheads, const int hgeo, const int hsl, const int hmax_ctx, const int hseq_planes, const AttnParams p)
 {
-  constexpr int DS = VW * NV, NG = 16;         // groups of 16 lanes: row j of the slice belongs to group j % NG
+  constexpr int DS = VW * NV, NG = 16;         // groups of 16 lanes, four waves: row j of the slice belongs to group j % NG
   const unsigned long long tl0 = timeline_now();
   const int q_heads = hheads & 0xffff, kv_heads = hheads >> 16, n_splits = hgeo & 0xffff, hd = hgeo >> 16;
   const int G = q_heads / kv_heads;
@@ -1207,10 +1194,7 @@ __global__ __launch_bounds__(256) void attn_split_head_kernel(const int32_t* hpo
   if ((tid & ~63) < hd) {                                    // (whole waves)
     const int d = min(tid, hd - 1), lane = tid & 63;
     const float mw = lane < NG ? sm[lane] : -1e30f, lw = lane < NG ? sl[lane] : 0.0f;      // group `lane`'s maximum and sum
-    const float Mr = row16_max(mw);
-    float M = lane_value(Mr, 0);
-#pragma unroll
-    for (int r = 1; r < NG / 16; r++) M = fmaxf(M, lane_value(Mr, 16 * r));
+    const float M = lane_value(row16_max(mw), 0);      // (the groups are one row of lanes)
     const float ew = lw > 0.0f ? expf(mw - M) : 0.0f;
     // (four short sums: one of sixteen is up to 15 % further from 64 bits, 30 rows of 64 1.39e-7 instead of 1.16e-7)
     float Lp[4] = {0.0f, 0.0f, 0.0f, 0.0f}, Ap[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -1221,10 +1205,9 @@ __global__ __launch_bounds__(256) void attn_split_head_kernel(const int32_t* hpo
     }
     const float Ls = (Lp[0] + Lp[1]) + (Lp[2] + Lp[3]), A = (Ap[0] + Ap[1]) + (Ap[2] + Ap[3]);
     const int qh = g * G + h;
-    if (tid >= hd) {
-    } else if (n_active == 1) {
+    if (tid < hd && n_active == 1) {
       p.out[(int64_t)seq * p.out_stride + qh * hd + d] = Ls > 0.0f ? A * (1.0f / Ls) : 0.0f;
-    } else {
+    } else if (tid < hd) {
       float* pt = p.part + (((int64_t)seq * p.q_heads + qh) * p.n_splits + split) * (hd + 2);
       if (p.merge_cnt) { part_store(pt + d, A); if (d == 0) { part_store(pt + hd, M); part_store(pt + hd + 1, Ls); } }
       else { pt[d] = A; if (d == 0) { pt[hd] = M; pt[hd + 1] = Ls; } }
