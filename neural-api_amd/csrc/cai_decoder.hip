@@ -153,7 +153,7 @@ static int enqueue_step(cai_decoder_s* d, int n_b, int seq0, unsigned classes = 
     for (int sl : slots) if (!nb_supported(L.w[sl]) || L.w[sl]->qtype == CAI_I8ROW) return false;   // (per-row int8 products need the plain reduction for their row scale)
     return true;
   };
-  // ... and when all six are Q4_K or Q6_K of widths the register-resident form takes, a linear layer is ONE launch: activations
+  // ... and when all six are Q4_K, Q6_K or Q8_0 of widths the register-resident form takes, a linear layer is ONE launch: activations
   // quantised by the product itself, norm factor, bias, residual and SwiGLU in its epilogue (CAIHIP_SMALL_BATCH_PLANES=1
   // keeps the form with activation planes and slice partials)
   static const bool ra_on = []() { const char* e = getenv("CAIHIP_SMALL_BATCH_PLANES"); return !(e && e[0] == '1'); }();

@@ -1018,7 +1018,7 @@ int nb_pass_tokens(const cai_qw_s* w) { return w->qtype == CAI_Q6_K ? NB_TMAX : 
 int nb_linear(const cai_qw_s* w, const float* x, int64_t x_stride, const float* gain, float eps, int n_tok, float* y, int64_t y_stride, const float* residual)
 {
   int rc;
-  // Q4_K matrices of whole row sets, and Q6_K up to 8 tokens (9 to 16 are one pass here): the one-launch form (cai_gemm_ra.hip), 8 tokens per launch
+  // Q4_K matrices of whole row sets, and Q6_K and Q8_0 up to 8 tokens (9 to 16 are one pass here): the one-launch form (cai_gemm_ra.hip), 8 tokens per launch
   if (ra_supported(&w, 1, gain != nullptr, 0) && (w->qtype == CAI_Q4_K || n_tok <= 8) && !(x_stride & 3) && !(y_stride & 3) && !(reinterpret_cast<uintptr_t>(x) & 15) && !(reinterpret_cast<uintptr_t>(y) & 15) &&
       !(residual && (reinterpret_cast<uintptr_t>(residual) & 15)) && !(gain && (reinterpret_cast<uintptr_t>(gain) & 15)) && !(w->bias && (reinterpret_cast<uintptr_t>(w->bias) & 15))) {
     if ((rc = ra_reserve(ra_part_floats(w->rows, w->cols)))) return rc;

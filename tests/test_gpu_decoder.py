@@ -669,3 +669,22 @@ def test_sequences_of_more_than_2_31_cached_rows():
         for p in range(4):
             assert rel_err(dec.step(int(toks[b, p]), p)[1][0], both[p][b]) < 1e-3, (b, p)
     dec.close()
+
+
+@pytest.mark.parametrize("d,hq,hkv", [(2080, 20, 20), (4064, 32, 8)])
+def test_mixture_whose_rows_are_longer_than_2048(d, hq, hkv):
+    """Whole-row norms of q rows of 2560 and 4096 (and k rows of 2560 and 1024), of which the attention requests 2048 elements ahead, and a router of 2080 and 4064
+    columns, which takes 2048 a turn; gains that differ from element to element; against the oracle."""
+    from helpers.device import dev, rel_err
+    cai = dev()
+    cfg = dict(n_layers=1, d_model=d, n_q_heads=hq, n_kv_heads=hkv, head_dim=128, ffn=64, vocab=300, max_ctx=64, eps=1e-5, rope_theta=1e4, n_experts=8, top_k=3, norm_topk=0, qk_norm_full=1)
+    spec = synthetic_spec(cfg, O.Q8_0, std=0.05, seed=d)
+    rng = np.random.default_rng(d)
+    for slot, n in ((O.V_Q_NORM, hq * 128), (O.V_K_NORM, hkv * 128), (O.V_MLP_NORM, d)):
+        spec["vecs"][(0, slot)] = (1.0 + 0.3 * rng.standard_normal(n)).astype(np.float32)
+    om, dec = oracle_model(spec, acc64=1), cai.Decoder(spec)
+    for p, t in enumerate(rng.integers(0, 300, 6)):
+        tok, lo = om.step(int(t), p)
+        am, ld = dec.step(int(t), p)
+        assert rel_err(ld[0], lo) < 1e-3 and int(am[0]) == tok, (p, rel_err(ld[0], lo))
+    dec.close()

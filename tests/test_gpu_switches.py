@@ -21,7 +21,7 @@ from helpers.model_build import oracle_model, synthetic_spec
 from helpers.device import dev, rel_err
 cai = dev()
 cfg = dict(n_layers=2, d_model=512, n_q_heads=14, n_kv_heads=2, head_dim=128, ffn=1024, vocab=2048, max_ctx=96, eps=1e-6, rope_theta=1e6)
-spec = synthetic_spec(cfg, O.Q4_K, head_qtype=O.Q8_0, qkv_bias=True, std=0.05)
+spec = synthetic_spec(cfg, O.%(body)s, head_qtype=O.%(head)s, qkv_bias=True, std=0.05)
 om, dec = oracle_model(spec, acc64=1), cai.Decoder(spec)
 prompt = np.random.default_rng(7).integers(0, cfg["vocab"], 40).tolist()
 for p, t in enumerate(prompt):
@@ -52,11 +52,18 @@ print("CHILD_OK")
                                       # batched / window steps of a Q4_K model through the form with activation planes and slice
                                       # partials (the one-launch form takes them otherwise)
                                       {"CAIHIP_SMALL_BATCH_PLANES": "1"}])
-def test_switch_selected_path_matches_the_oracle(switches):
+def test_switch_selected_path_matches_the_oracle(switches, body="Q4_K", head="Q8_0"):
     env = dict(os.environ); env.update(switches)
-    code = CHILD % dict(root=ROOT, tests=os.path.join(ROOT, "tests"))
+    code = CHILD % dict(root=ROOT, tests=os.path.join(ROOT, "tests"), body=body, head=head)
     r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and "CHILD_OK" in r.stdout, r.stdout[-2000:] + r.stderr[-4000:]
+
+
+@pytest.mark.parametrize("planes", ["0", "1"])
+@pytest.mark.parametrize("body, head", [("Q6_K", "Q6_K"), ("Q8_0", "Q8_0"), ("Q8_0", "Q6_K")])
+def test_window_steps_of_the_other_types_with_and_without_planes(body, head, planes):
+    """the same session of Q6_K and Q8_0 models, whose window steps take the one-launch form, and the form with planes under its switch"""
+    test_switch_selected_path_matches_the_oracle({"CAIHIP_SMALL_BATCH_PLANES": planes}, body, head)
 
 
 MOE_CHILD = r"""
