@@ -17,7 +17,8 @@
 namespace cai {
 
 // ------------------------------------------------------------------------------------------
-// Decode, every product in 32 bits: float activations, an RMS norm on the way, two products in one, and bfloat16 rows of more than 8192 columns.
+// Decode, every product in 32 bits: float activations, an RMS norm on the way, two products in one, bfloat16 rows of more than 8192 columns and one or two
+// (run_lin) of smaller matrices.
 // NB activation rows.  A wave owns R weight rows (of a gated matrix R / 2 outputs) or, with ksplit > 1, every ksplit-th
 // 512-wide turn of them; the activations are staged in LDS as float in panels, the weights stream past once.
 // GV_RMS: the activations are the float stream, RMS-normed on the way (the gain while they are staged, the root at the end), and the
@@ -580,7 +581,9 @@ static int run_mc(const cai_qw_s* w, const bf16_t* x, int64_t ldx, int n_tok, co
   }
   const int tiles = ((int)w->rows + T * MC_H - 1) / (T * MC_H);
   const size_t lds = lds_of(ks, n_tok);
-  const int per_cu = std::min((int)(160 * 1024 / lds), 16 / ks);      // (sixteen waves of these registers fill a CU)
+  // as many as a CU holds at once: sixteen waves of the registers of one slot of a row a wave, eight of more (147 registers and up).  Twice that many
+  // work-groups began anew half way: width 4096, one to eight rows of 4096 outputs 12.1 .. 14.6 us a launch, 11.2 .. 12.3 with what fits; 18720 outputs 30.2 | 28.6
+  const int per_cu = std::min((int)(160 * 1024 / lds), (SB == 1 ? 16 : 8) / ks);
   hipLaunchKernelGGL((gemv_bf16_mc<GLU, SB>), dim3(std::min(tiles, std::max(1, per_cu) * ctx().n_cu)), dim3(64 * ks), lds, ctx().stream,
                      (const uint16_t*)w->data, x, (int)w->rows, (int)w->ld, ldx, n_tok, tiles, e);
   return CAI_OK;
@@ -599,7 +602,13 @@ template <typename AT>
 static int run_lin(const cai_qw_s* w, const AT* x, int64_t ldx, int n_tok, const LinEpi& e)
 {
   if constexpr (sizeof(AT) == 2) {
-    if (n_tok <= MC_ROWS && w->ld <= 256 * MC_WAVES * MC_SLOTS) return run_gemv_mc(w, x, ldx, n_tok, e);
+    // The 32-bit walk costs more with every row, this form hardly.  Of fewer than 8192 outputs (the walk's two-row form) one and two rows are the walk's, and up to
+    // four between 2048 and 4096 columns, where a wave has two slots a tile and the walk one panel.  us a launch, walk | here: 2048 x 5632, one row 7.85 | 9.15, two
+    // 8.7 | 9.35, three 10.8 | 9.5; 5120 x 2048 6.9 | 8.0, 7.5 | 7.9, 8.1 | 7.9; 2048 x 2048 5.2 | 5.2, 5.5 | 5.3, 6.05 | 5.4; 4096 x 4096 9.0 | 11.2, 10.2 | 11.3,
+    // 10.8 | 11.4, four 11.5 | 11.5, eight 16.9 | 12.3; 18720 x 4096, one row 35.7 | 28.6; 32768 x 2048 27.7 | 26.8
+    const bool few_outputs = (int)w->rows / 4 < ctx().n_cu * 8;
+    const bool walk = few_outputs && (n_tok <= 2 || (n_tok <= 4 && w->ld > 2048 && w->ld <= 4096));
+    if (!walk && n_tok <= MC_ROWS && w->ld <= 256 * MC_WAVES * MC_SLOTS) return run_gemv_mc(w, x, ldx, n_tok, e);
   }
   if (n_tok <= LIN_FEW) {
     const bool glu = e.mode == EPI_GLU;

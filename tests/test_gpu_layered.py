@@ -72,7 +72,21 @@ def test_products_over_bf16_rows(cai, rows, cols):
     q.close()
 
 
-@pytest.mark.parametrize("rows, cols", [(32, 64), (96, 320), (5664, 72), (2144, 2112), (64, 8192), (160, 264), (64, 8200)])
+@pytest.mark.parametrize("rows, cols", [(8193, 72), (8201, 2120), (8198, 4616), (8195, 6160)])
+def test_few_rows_of_many_outputs_over_bf16_rows(cai, rows, cols):
+    """the same of one to four and sixteen rows where the ring kernel takes every count: one to four slots of a row a wave, with fewer and more tiles than
+    work-groups, bounds as above"""
+    rng = np.random.default_rng(rows)
+    bits, w = B.to_bf16(rng.standard_normal((rows, cols), np.float32))
+    w = w.reshape(rows, cols).astype(np.float64)
+    q = cai.QWeight(cai.BF16, rows, cols, bits)
+    for n in (1, 2, 3, 4, 16):
+        x = B.to_bf16(rng.standard_normal((n, cols)))[1].reshape(n, cols).astype(np.float64)
+        assert np.all(np.abs(bf16_rows(cai, q, x) - x @ w.T) <= 2.0 ** -19 * (np.abs(x) @ np.abs(w).T)), n
+    q.close()
+
+
+@pytest.mark.parametrize("rows, cols", [(32, 64), (96, 320), (5664, 72), (8224, 72), (2144, 2112), (8288, 2112), (64, 8192), (160, 264), (64, 8200)])
 def test_gated_products_over_bf16_rows(cai, rows, cols):
     """the same of gate and up rows: the bounds of both sums, then one rounding to bfloat16 (2^-8 of the value at most)"""
     rng = np.random.default_rng(rows + cols)
@@ -93,14 +107,14 @@ def test_gated_products_over_bf16_rows(cai, rows, cols):
 @pytest.mark.parametrize("cols", [320, 1024, 2048, 5632, 8192])
 @pytest.mark.parametrize("spread", [0.0, 1.5])
 def test_few_bf16_rows_are_as_near_as_the_32_bit_walk(cai, cols, spread):
-    """activations of even and of widely differing sizes: what the matrix cores make of one to sixteen rows is as close to 64 bits as the 32-bit walk over the same
+    """activations of even and of widely differing sizes: what the matrix cores make of five to sixteen rows is as close to 64 bits as the 32-bit walk over the same
     rows (relative errors of 40 rows of 2000 results, squares averaged; one chain of matrix instructions was 1.4 to 2.2 times as far off)"""
     rng = np.random.default_rng(cols)
     bits, w = B.to_bf16(rng.standard_normal((2000, cols)))
     w = w.reshape(2000, cols).astype(np.float64)
     q = cai.QWeight(cai.BF16, 2000, cols, bits)
     off = np.zeros(2)
-    for n in (1, 3, 4, 8, 8, 16):
+    for n in (5, 5, 6, 8, 16):
         x = B.to_bf16(rng.standard_normal((n, cols)) * np.exp(spread * rng.standard_normal((n, cols))))[1].reshape(n, cols).astype(np.float64)
         want = x @ w.T
         for i, got in enumerate((bf16_rows(cai, q, x), np.concatenate([q.gemv(x[k:k + 8]) for k in range(0, n, 8)]))):
