@@ -609,9 +609,9 @@ static int run_lin(const cai_qw_s* w, const AT* x, int64_t ldx, int n_tok, const
 {
   if constexpr (sizeof(AT) == 2) {
     // The 32-bit walk costs more with every row, this form hardly.  Of fewer than 8192 outputs (the walk's two-row form) one and two rows are the walk's, and up to
-    // four between 2048 and 4096 columns, where a wave has two slots a tile and the walk one panel.  us a launch, walk | here: 2048 x 5632, one row 7.85 | 9.15, two
-    // 8.7 | 9.35, three 10.8 | 9.5; 5120 x 2048 6.9 | 8.0, 7.5 | 7.9, 8.1 | 7.9; 2048 x 2048 5.2 | 5.2, 5.5 | 5.3, 6.05 | 5.4; 4096 x 4096 9.0 | 11.2, 10.2 | 11.3,
-    // 10.8 | 11.4, four 11.5 | 11.5, eight 16.9 | 12.3; 18720 x 4096, one row 35.7 | 28.6; 32768 x 2048 27.7 | 26.8
+    // four between 2048 and 4096 columns, where a wave has two slots a tile and the walk one panel.  us a launch, walk | here: 2048 x 5632, one row 7.5 | 8.9, two
+    // 8.25 | 9.1, three 10.8 | 9.3; 6200 x 2048 7.3 | 8.6, 7.95 | 8.65; 2048 x 2048 4.8 | 4.9, 5.0 | 5.0, three 6.05 | 5.0; 4096 x 4096 9.3 | 11.2, 10.55 | 11.3,
+    // 11.0 | 11.4, four 11.65 | 11.5, eight 16.9 | 12.3; 18720 x 4096, one row 35.7 | 28.6; 32768 x 2048 27.7 | 26.8
     const bool few_outputs = (int)w->rows / 4 < ctx().n_cu * 8;
     const bool walk = few_outputs && (n_tok <= 2 || (n_tok <= 4 && w->ld > 2048 && w->ld <= 4096));
     if (!walk && n_tok <= MC_ROWS && w->ld <= 256 * MC_WAVES * MC_SLOTS) return run_gemv_mc(w, x, ldx, n_tok, e);
