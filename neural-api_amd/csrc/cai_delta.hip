@@ -9,6 +9,8 @@
 
 namespace cai {
 
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+
 // ------------------------------------------------------------------------------------------
 // prompt pass 1: q and k unit vectors (q scaled), v, decay, write strength, q . k.
 // A wave owns one unit - the q and k channels of a key head, 256 channels of v, 256 decays, the write strengths - over eight
@@ -215,6 +217,17 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const DeltaDims d, floa
 // Everything before "S" is made for all chunks at once (first kernel); the second kernel walks the chunks of a sequence with a
 // 16-column slice of the state in registers.  Decays enter only as running products, never as quotients or differences of
 // logarithms, so strong decay costs no accuracy.
+//
+// The first kernel leaves a chunk's factors of one head as the walk's matrix operands, a record of 1 KB blocks [64 lanes][4 floats]
+// (fr = lane % 16, fg = lane / 16; everything past the portion's end or a width is zero):
+//     block j                 - W,    token fr, channels 16 j + 4 fg ..      (tiles of them)
+//     block tiles + j         P q,    token fr, channels 16 j + 4 fg ..
+//     block 2 tiles + j       D_16 k, tokens 4 fg .., channel 16 j + fr
+//     block 3 tiles           q D k,  token fr, writing tokens 4 fg ..
+//     block 3 tiles + 1 + c   U0,     tokens 4 fg .., value column 16 c + fr
+// so that the walk, whose chain of 128 chunks is what a prompt of 2048 tokens waits for, requests one contiguous KB an instruction
+// and puts it into a product as it comes.  Read from arrays by row instead, with the masks, decays and signs applied in the walk (18 requests
+// and 70 more vector instructions a chunk), 16 heads of 128 x 128 took 157 us for 2048 tokens; now 96 (128 work-groups).
 // ------------------------------------------------------------------------------------------
 constexpr int CHUNK = DELTA_CHUNK;
 
@@ -224,14 +237,14 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaDims d, con
   extern __shared__ float lds[];
   __shared__ float sA[CHUNK][CHUNK + 1], sQ[CHUNK][CHUNK + 1], sP[CH ? 1 : 4][CHUNK][CHUNK + 1];
   __shared__ f32x4 sT[CHUNK][CHUNK / 4];
-  __shared__ float sbeta[CHUNK], sg1[CHUNK], sdot[CHUNK];
+  __shared__ float sbeta[CHUNK], sg1[CHUNK], sdot[CHUNK], sz[CHUNK];      // sdot: q . k, later (one decay a head) the running products of the decays
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), fr = lane & 15, fg = lane >> 4;
   const int32_t* en = r.ent + 4 * chunks[2 * blockIdx.x];
   const int t0 = chunks[2 * blockIdx.x + 1], nt = min(CHUNK, en[2] - t0), h = blockIdx.y;
   const int64_t row0 = en[1] + t0;
   const int g = h / (d.heads / d.kv_heads), kw = d.kv_heads * d.dim, vw = d.heads * d.vdim, gw = d.heads * d.dim, bw = d.heads + d.kv_heads;
-  const int dp = (d.dim + 15) & ~15, DS = dp + 4;
-  float *sk = lds, *sq = lds + CHUNK * DS, *sg = lds + 2 * CHUNK * DS;       // sg: channel decays, later their running products
+  const int dp = (d.dim + 15) & ~15, DS = dp + 4, tiles = delta_tiles(d);
+  float *sk = lds, *sq = lds + CHUNK * DS, *sg = lds + 2 * CHUNK * DS;       // sg: channel decays
   for (int e = tid; e < CHUNK * dp; e += 256) {
     const int t = e / dp, c = e - t * dp;
     const bool ok = t < nt && c < d.dim;
@@ -267,24 +280,24 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaDims d, con
       if (cl == 0) { sA[t][s] = t > s ? x : 0.0f; sQ[t][s] = t > s ? y : t == s ? sdot[t] : 0.0f; }
     }
     __syncthreads();
-    // k times the decays behind it (in place of the decays), q times those up to it, the chunk's whole decay
-    for (int c = tid; c < dp; c += 256) {
-      float z = 1.0f;
-      float gr[CHUNK];
-#pragma unroll
-      for (int t = CHUNK - 1; t >= 0; t--) {
-        gr[t] = sg[t * DS + c];
-        if (t < nt && c < d.dim) b.g[(row0 + t) * gw + h * d.dim + c] = sk[t * DS + c] * z;
-        z *= gr[t];
-      }
+    // the factors of the three products, each in its place: k times the decays behind it, q and k (in place of the decays) times those up to it
+    for (int c = tid; c < 16 * tiles; c += 256) {
       float p = 1.0f;
+      if (c < dp) {
+        float z = 1.0f, k[CHUNK], gr[CHUNK];
 #pragma unroll
-      for (int t = 0; t < CHUNK; t++) {
-        p *= gr[t];
-        sg[t * DS + c] = p;
-        if (t < nt && c < d.dim) b.qt[(row0 + t) * gw + h * d.dim + c] = sq[t * DS + c] * p;
+        for (int t = CHUNK - 1; t >= 0; t--) {
+          gr[t] = sg[t * DS + c]; k[t] = sk[t * DS + c];
+          sk[t * DS + c] = k[t] * z;
+          z *= gr[t];
+        }
+#pragma unroll
+        for (int t = 0; t < CHUNK; t++) {
+          p *= gr[t];
+          sq[t * DS + c] *= p; sg[t * DS + c] = k[t] * p;
+        }
       }
-      if (c < d.dim) b.gt[(int64_t)blockIdx.x * gw + h * d.dim + c] = p;
+      b.gt[((int64_t)blockIdx.x * d.heads + h) * (16 * tiles) + c] = p;
     }
   } else {
     // K K^T and Q K^T, half of the width by each of two waves
@@ -304,19 +317,16 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaDims d, con
     for (int x = 1; x < CHUNK; x++) e *= x > s && x <= t ? sg1[x] : 1.0f;
     sA[t][s] = t > s ? e * (sP[0][t][s] + sP[2][t][s]) : 0.0f;
     sQ[t][s] = e * (sP[1][t][s] + sP[3][t][s]);
-    if (tid < nt) {
+    if (tid < CHUNK) {
       float p = 1.0f, z = 1.0f;
 #pragma unroll
       for (int x = 0; x < CHUNK; x++) { p *= x <= tid ? sg1[x] : 1.0f; z *= x > tid ? sg1[x] : 1.0f; }
-      float* o = b.gt + ((row0 + tid) * d.heads + h) * 2;
-      o[0] = p; o[1] = z;
+      sdot[tid] = p; sz[tid] = z;
+      if (tid == CHUNK - 1) b.gt[(int64_t)blockIdx.x * d.heads + h] = p;
     }
   }
   __syncthreads();
-  {
-    const int t = tid >> 4, s = tid & 15;
-    if (t < nt) b.qk[((row0 + t) * d.heads + h) * CHUNK + s] = sQ[t][s];
-  }
+  f32x4* const rec = reinterpret_cast<f32x4*>(b.rec) + ((int64_t)blockIdx.x * d.heads + h) * (64 * delta_record_blocks(d)) + lane;
   if (tid < CHUNK) {                       // column tid of T by forward substitution
     float c[CHUNK];
 #pragma unroll
@@ -328,25 +338,38 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaDims d, con
       reinterpret_cast<float*>(sT[t])[tid] = c[t];
     }
   }
-  if (!CH && tid >= 64 && tid < 64 + CHUNK) {            // running products for T [P k]
-    float p = 1.0f;
-    for (int x = 0; x <= tid - 64; x++) p *= sg1[x];
-    sdot[tid - 64] = p;
+  // the factors that do not need T, while wave 0 substitutes
+  for (int j = wave; j < 2 * tiles + 1; j += 4) {
+    f32x4 x = {0.0f, 0.0f, 0.0f, 0.0f};
+    const int ct = j < tiles ? j : j - tiles;
+    if (j == 2 * tiles) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) x[i] = sQ[fr][fg * 4 + i];
+    } else if (ct * 16 < dp) {
+      if (j < tiles) {
+        x = *reinterpret_cast<const f32x4*>(sq + fr * DS + ct * 16 + fg * 4);
+        if (!CH) x *= sdot[fr];
+      } else
+#pragma unroll
+        for (int i = 0; i < 4; i++) x[i] = CH ? sk[(fg * 4 + i) * DS + ct * 16 + fr] : sk[(fg * 4 + i) * DS + ct * 16 + fr] * sz[fg * 4 + i];
+    }
+    rec[64 * (tiles + j)] = x;
   }
   __syncthreads();
   const f32x4 tf = sT[fr][fg];
-  for (int ct = wave; ct < dp / 16; ct += 4) {           // W = T [P k]
+  for (int ct = wave; ct < tiles; ct += 4) {             // W = T [P k]: channels as rows, tokens as columns of the result
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    const int c = ct * 16 + fr;
+    if (ct * 16 < dp)
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int s = fg * 4 + i;
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(tf[i], sk[s * DS + c] * (CH ? sg[s * DS + c] : sdot[s]), acc, 0, 0, 0);
-    }
+      for (int i = 0; i < 4; i++) {
+        const int s = fg * 4 + i, c = ct * 16 + fr;
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(CH ? sg[s * DS + c] : sk[s * DS + c] * sdot[s], tf[i], acc, 0, 0, 0);
+      }
 #pragma unroll
-    for (int i = 0; i < 4; i++) if (fg * 4 + i < nt && c < d.dim) b.w[(row0 + fg * 4 + i) * gw + h * d.dim + c] = acc[i];
+    for (int i = 0; i < 4; i++) acc[i] = fr < nt ? -acc[i] : 0.0f;
+    rec[64 * ct] = acc;
   }
-  for (int ct = wave; ct * 16 < d.vdim; ct += 4) {       // U0 = T V, in place of V
+  for (int ct = wave; ct * 16 < d.vdim; ct += 4) {       // U0 = T V
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
     const int c = ct * 16 + fr;
     float x[4];
@@ -355,28 +378,35 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaDims d, con
 #pragma unroll
     for (int i = 0; i < 4; i++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(tf[i], x[i], acc, 0, 0, 0);
 #pragma unroll
-    for (int i = 0; i < 4; i++) if (fg * 4 + i < nt && c < d.vdim) b.v[(row0 + fg * 4 + i) * vw + h * d.vdim + c] = acc[i];
+    for (int i = 0; i < 4; i++) acc[i] = fg * 4 + i < nt ? acc[i] : 0.0f;
+    rec[64 * (3 * tiles + 1 + ct)] = acc;
   }
 }
 
 // The walk: one work-group per (16 value columns, head, entry).  Waves 0 .. NW - 1 hold the state - wave w the key rows of tiles
-// w TPW .. as matrix-core result registers, which are at the same time the right operand of the products with S - and wave NW makes
+// w TPW .. as matrix-core result registers, which are at the same time an operand of the products with S - and wave NW makes
 // the output: it contributes U0 to the sum of a chunk's writes and finishes the previous chunk's rows of o while the others are a
 // chunk further.  One barrier a chunk; the partial sums live in LDS for three chunks.
-template <int NW, int TPW, bool CH, bool VEC>      // VEC: the key width is a multiple of four
+// What bounds it: the chain from chunk to chunk - 8 products, their parts through LDS (a third of the time), 8 products: 1700 cycles, 130 of
+// them waiting for the other waves.  U0 as the start of a state wave's sums and U handed to wave NW took 102 us where this takes 96, factors
+// five chunks ahead 92 to 98, the read-out in front of the barrier or around it 98 to 100.
+template <int NW, int TPW, bool CH, bool WHOLE>      // WHOLE: the value width is a multiple of sixteen
 __global__ __launch_bounds__(64 * (NW + 1)) void delta_walk_kernel(const DeltaDims d, float* state, const int64_t s_elems, const StepRows r, const DeltaBuf b, const int32_t* chunk0)
 {
+  constexpr int TILES = NW * TPW;
   __shared__ f32x4 pu[3][NW + 1][64], po[3][NW][64];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), fr = lane & 15, fg = lane >> 4;
   // consecutive work-groups go to different XCDs; the column slices of a head read the same chunk data, so with heads in whole
   // eights every head stays on one XCD (and in its L2)
   const int slices = (d.vdim + 15) / 16;
   const int h = d.heads % 8 == 0 ? (blockIdx.x & 7) + 8 * ((blockIdx.x >> 3) / slices) : blockIdx.x / slices;
-  const int col = (d.heads % 8 == 0 ? (blockIdx.x >> 3) % slices : blockIdx.x % slices) * 16 + fr;
+  const int slice = d.heads % 8 == 0 ? (blockIdx.x >> 3) % slices : blockIdx.x % slices, col = slice * 16 + fr;
   const int32_t* en = r.ent + 4 * blockIdx.y;
   const int slot = en[0], row0 = en[1], n = en[2], pos0 = en[3], ch0 = chunk0[blockIdx.y];
-  const int g = h / (d.heads / d.kv_heads), kw = d.kv_heads * d.dim, vw = d.heads * d.vdim, gw = d.heads * d.dim, dvp = d.vdim_p();
+  const int vw = d.heads * d.vdim, dvp = d.vdim_p(), blocks = delta_record_blocks(d);
   const int nc = (n + CHUNK - 1) / CHUNK;
+  const f32x4* const rec = reinterpret_cast<const f32x4*>(b.rec) + ((int64_t)ch0 * d.heads + h) * (64 * blocks);
+  const int64_t step = (int64_t)d.heads * (64 * blocks);
   auto total = [&](int it) -> f32x4 {                    // a chunk's writes: U0 and every wave's part of - W S
     f32x4 x[NW];
 #pragma unroll
@@ -389,49 +419,48 @@ __global__ __launch_bounds__(64 * (NW + 1)) void delta_walk_kernel(const DeltaDi
     return x[0];
   };
   if (wave == NW) {
-    const unsigned lv = fg * 4 * vw + min(col, d.vdim - 1), lqk = fr * d.heads * CHUNK + fg * 4, lo = fg * 4 * vw + col;
     struct Out { f32x4 u0, qk; };
     auto fetch = [&](int c, Out& x) {
-      const int64_t rr = row0 + min(c, nc - 1) * CHUNK;
-      const float* vb = b.v + rr * vw + h * d.vdim;
-#pragma unroll
-      for (int i = 0; i < 4; i++) x.u0[i] = (vb + i * vw)[lv];
-      x.qk = *reinterpret_cast<const f32x4*>(b.qk + (rr * d.heads + h) * CHUNK + lqk);
+      const f32x4* p = rec + min(c, nc - 1) * step;
+      x.u0 = p[64 * (3 * TILES + 1 + slice) + lane]; x.qk = p[64 * (3 * TILES) + lane];
     };
-    f32x4 qk_last = {0.0f, 0.0f, 0.0f, 0.0f};
-    auto finish = [&](int c, int it) {                   // rows of o of chunk c (parts it)
+    f32x4 qk_last;
+    float* const ob = b.o + (int64_t)(row0 + fr) * vw + h * d.vdim + slice * 16 + fg * 4;     // token fr, columns 4 fg ..
+    auto finish = [&](int c, int it, bool last) {        // rows of o of chunk c (parts it)
       f32x4 o = po[it][0][lane];
 #pragma unroll
       for (int v = 1; v < NW; v++) o += po[it][v][lane];
       const f32x4 u = total(it);
 #pragma unroll
-      for (int i = 0; i < 4; i++) o = __builtin_amdgcn_mfma_f32_16x16x4f32(qk_last[i], u[i], o, 0, 0, 0);
-      const int nt = n - c * CHUNK;
-      if (c < 0) return;
-      float* ob = b.o + (int64_t)(row0 + c * CHUNK) * vw + h * d.vdim;
+      for (int i = 0; i < 4; i++) o = __builtin_amdgcn_mfma_f32_16x16x4f32(u[i], qk_last[i], o, 0, 0, 0);
+      float* const p = ob + (int64_t)c * CHUNK * vw;
+      if (WHOLE && !last) *reinterpret_cast<f32x4_any*>(p) = o;
+      else if (c * CHUNK + fr < n)
 #pragma unroll
-      for (int i = 0; i < 4; i++) if (fg * 4 + i < nt && col < d.vdim) (ob + i * vw)[lo] = o[i];
+        for (int i = 0; i < 4; i++) if (slice * 16 + fg * 4 + i < d.vdim) p[i] = o[i];
     };
     auto chunk = [&](int c, const Out& x, int it) {
-      const int nt = n - c * CHUNK;
-      f32x4 u;
-#pragma unroll
-      for (int i = 0; i < 4; i++) u[i] = fg * 4 + i < nt && col < d.vdim ? x.u0[i] : 0.0f;
-      pu[it][NW][lane] = u;
+      pu[it][NW][lane] = x.u0;
       __syncthreads();
-      finish(c - 1, (it + 2) % 3);
-#pragma unroll
-      for (int i = 0; i < 4; i++) qk_last[i] = fr < nt ? x.qk[i] : 0.0f;
+      finish(c - 1, (it + 2) % 3, false);
+      qk_last = x.qk;
     };
+    // (all stores of the loop are without a condition: a store that may not have happened makes every wait for a chunk's factors wait for
+    // the stores behind them too, and this wave then holds up the others: 110 us)
     Out xa, xb, xc;
-    fetch(0, xa); fetch(1, xb);
-    for (int c = 0; c < nc; c += 3) {
-      fetch(c + 2, xc); chunk(c, xa, 0);
-      fetch(c + 3, xa); chunk(c + 1, xb, 1);
-      fetch(c + 4, xb); chunk(c + 2, xc, 2);
+    fetch(0, xa); fetch(1, xb); fetch(2, xc);
+    pu[0][NW][lane] = xa.u0;
+    qk_last = xa.qk;
+    __syncthreads();
+    for (int c = 1; c < nc; c += 3) {
+      fetch(c + 2, xa); chunk(c, xb, 1);
+      if (c + 1 >= nc) break;
+      fetch(c + 3, xb); chunk(c + 1, xc, 2);
+      if (c + 2 >= nc) break;
+      fetch(c + 4, xc); chunk(c + 2, xa, 0);
     }
     __syncthreads();
-    finish((nc + 2) / 3 * 3 - 1, 2);
+    finish(nc - 1, (nc - 1) % 3, true);
     return;
   }
   float* Sg = state + slot * s_elems + (int64_t)h * d.dim * dvp;
@@ -443,93 +472,63 @@ __global__ __launch_bounds__(64 * (NW + 1)) void delta_walk_kernel(const DeltaDi
       const int c = (wave * TPW + j) * 16 + fg * 4 + i;
       S[j][i] = pos0 > 0 && c < d.dim && col < d.vdim ? Sg[(int64_t)c * dvp + col] : 0.0f;
     }
-  // A chunk's inputs are requested two chunks ahead and stay as they come until they are used: arithmetic on them here would wait
-  // for them here, and so would a request under a branch where the paths join.  A request is a scalar base of the chunk plus a lane
-  // offset that never changes; rows past the portion's end (of another entry, or of the slack behind the last row) and columns past
-  // the width are replaced by zeros at use.
-  struct In { f32x4 w[TPW], q[TPW], k[TPW], tot[TPW]; float p, all, kz[4]; };
-  bool ok4[TPW][VEC ? 1 : 4], ok1[TPW];
-  unsigned lw[TPW], lq[TPW], lk[TPW], lt[TPW];
-#pragma unroll
-  for (int j = 0; j < TPW; j++) {
-    const int c4 = (wave * TPW + j) * 16 + fg * 4, c1 = (wave * TPW + j) * 16 + fr;
-    ok1[j] = c1 < d.dim;
-#pragma unroll
-    for (int i = 0; i < (VEC ? 1 : 4); i++) ok4[j][i] = c4 + i < d.dim;
-    lt[j] = c4 < d.dim ? c4 : 0;
-    lw[j] = fr * gw + lt[j]; lq[j] = fr * (CH ? gw : kw) + lt[j];
-    lk[j] = fg * 4 * (CH ? gw : kw) + (ok1[j] ? c1 : 0);
-  }
-  const unsigned lp = fr * d.heads * 2, lz = fg * 4 * d.heads * 2 + 1;
-  auto four = [&](const float* p, unsigned c) -> f32x4 {
-    if (VEC) return *reinterpret_cast<const f32x4*>(p + c);
-    return f32x4{p[c], p[c + 1], p[c + 2], p[c + 3]};                     // (may run into the next row: replaced at use)
-  };
+  // a chunk's factors are requested two chunks ahead
+  struct In { f32x4 w[TPW], q[TPW], k[TPW], tot[CH ? TPW : 1]; };
+  const f32x4* const mine = rec + 64 * TPW * wave + lane;
+  const float* const tot = CH ? b.gt + ((int64_t)ch0 * d.heads + h) * (16 * TILES) + 16 * TPW * wave + 4 * fg : b.gt + (int64_t)ch0 * d.heads + h;
+  const int tstep = CH ? d.heads * (16 * TILES) : d.heads;
   auto fetch = [&](int c, In& x) {
     const int cc = min(c, nc - 1);
-    const int64_t rr = row0 + cc * CHUNK;
-    const float *wb = b.w + rr * gw + h * d.dim, *qb = CH ? b.qt + rr * gw + h * d.dim : b.q + rr * kw + g * d.dim;
-    const float *kb = CH ? b.g + rr * gw + h * d.dim : b.k + rr * kw + g * d.dim, *tb = b.gt + (int64_t)(ch0 + cc) * gw + h * d.dim;
-    const int ks = CH ? gw : kw;
+    const f32x4* const p = mine + cc * step;
+    const float* const t = tot + (int64_t)cc * tstep;
 #pragma unroll
-    for (int j = 0; j < TPW; j++) {
-      x.w[j] = four(wb, lw[j]); x.q[j] = four(qb, lq[j]);
+    for (int j = 0; j < TPW; j++) x.w[j] = p[64 * j];
+    if (CH)
 #pragma unroll
-      for (int i = 0; i < 4; i++) x.k[j][i] = (kb + i * ks)[lk[j]];
-      if (CH) x.tot[j] = four(tb, lt[j]);
-    }
-    if (!CH) {
-      const float* pz = b.gt + (rr * d.heads + h) * 2;
-      x.p = pz[lp]; x.all = pz[(min(CHUNK, n - cc * CHUNK) - 1) * d.heads * 2];
+      for (int j = 0; j < TPW; j++) x.tot[j] = *reinterpret_cast<const f32x4*>(t + 16 * j);
+    else x.tot[0][0] = *t;
 #pragma unroll
-      for (int i = 0; i < 4; i++) x.kz[i] = (pz + i * d.heads * 2)[lz];
-    }
+    for (int j = 0; j < TPW; j++) { x.q[j] = p[64 * (TILES + j)]; x.k[j] = p[64 * (2 * TILES + j)]; }
   };
-  auto chunk = [&](int c, const In& x, int it) {         // (a chunk past the last one changes nothing)
-    const int nt = n - c * CHUNK;
-    const bool rok = fr < nt;
-    f32x4 u[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}}, o = {0.0f, 0.0f, 0.0f, 0.0f};
+  auto chunk = [&](const In& x, int it) {
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 u[2] = {zero, zero}, o = zero;
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
-      for (int j = 0; j < TPW; j++)
-        u[(i * TPW + j) & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(rok && ok4[j][VEC ? 0 : i] ? -x.w[j][i] : 0.0f, S[j][i], u[(i * TPW + j) & 1], 0, 0, 0);
+      for (int j = 0; j < TPW; j++) u[(i * TPW + j) & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w[j][i], S[j][i], u[(i * TPW + j) & 1], 0, 0, 0);
     pu[it][wave][lane] = u[0] + u[1];
     __syncthreads();
     const f32x4 t = total(it);
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
-      for (int j = 0; j < TPW; j++) {      // the read-out with the state before the chunk, while the sums arrive
-        const float q = rok && ok4[j][VEC ? 0 : i] ? (CH ? x.q[j][i] : x.q[j][i] * x.p) : 0.0f;
-        o = __builtin_amdgcn_mfma_f32_16x16x4f32(q, S[j][i], o, 0, 0, 0);
-      }
+      for (int j = 0; j < TPW; j++)        // the read-out with the state before the chunk, columns as rows of the result, while the sums arrive
+        o = __builtin_amdgcn_mfma_f32_16x16x4f32(S[j][i], x.q[j][i], o, 0, 0, 0);
     po[it][wave][lane] = o;
 #pragma unroll
-    for (int j = 0; j < TPW; j++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) S[j][i] *= nt > 0 ? (CH ? x.tot[j][i] : x.all) : 1.0f;
+    for (int j = 0; j < TPW; j++) S[j] *= CH ? x.tot[CH ? j : 0] : f32x4{x.tot[0][0], x.tot[0][0], x.tot[0][0], x.tot[0][0]};
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
-      for (int j = 0; j < TPW; j++) {
-        const float k = fg * 4 + i < nt && ok1[j] ? (CH ? x.k[j][i] : x.k[j][i] * x.kz[i]) : 0.0f;
-        S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(k, t[i], S[j], 0, 0, 0);
-      }
+      for (int j = 0; j < TPW; j++) S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[j][i], t[i], S[j], 0, 0, 0);
   };
   // (the scheduling barriers keep a chunk's requests in front of the chunk that is worked on: they are used two chunks later)
   In xa, xb, xc;
   fetch(0, xa); fetch(1, xb);
-  for (int c = 0; c < nc; c += 3) {
+  for (int c = 0;; c += 3) {
     fetch(c + 2, xc);
     __builtin_amdgcn_sched_barrier(0);
-    chunk(c, xa, 0);
+    chunk(xa, 0);
+    if (c + 1 >= nc) break;
     fetch(c + 3, xa);
     __builtin_amdgcn_sched_barrier(0);
-    chunk(c + 1, xb, 1);
+    chunk(xb, 1);
+    if (c + 2 >= nc) break;
     fetch(c + 4, xb);
     __builtin_amdgcn_sched_barrier(0);
-    chunk(c + 2, xc, 2);
+    chunk(xc, 2);
+    if (c + 3 >= nc) break;
   }
   __syncthreads();                         // the last chunk's read-outs are there
 #pragma unroll
@@ -753,12 +752,12 @@ int delta_chunked(const DeltaDims& d, const SeqPool::StateRun& st, const StepRow
   const dim3 g1(n_chunks, d.heads), g2((d.vdim + 15) / 16 * d.heads, r.n_ent), blk(256);
   if (d.channel_decay) hipLaunchKernelGGL(delta_chunk_kernel<true>, g1, blk, lds, s, d, r, b, chunks);
   else hipLaunchKernelGGL(delta_chunk_kernel<false>, g1, blk, lds, s, d, r, b, chunks);
-#define WALK_V(NW, N, CH) do { if (d.dim % 4 == 0) hipLaunchKernelGGL((delta_walk_kernel<NW, N, CH, true>), g2, dim3(64 * (NW + 1)), 0, s, d, st.S, st.s_elems, r, b, chunk0); \
+#define WALK_C(NW, N, CH) do { if (d.vdim % 16 == 0) hipLaunchKernelGGL((delta_walk_kernel<NW, N, CH, true>), g2, dim3(64 * (NW + 1)), 0, s, d, st.S, st.s_elems, r, b, chunk0); \
                                else hipLaunchKernelGGL((delta_walk_kernel<NW, N, CH, false>), g2, dim3(64 * (NW + 1)), 0, s, d, st.S, st.s_elems, r, b, chunk0); } while (0)
-#define WALK(NW, N) do { if (d.channel_decay) WALK_V(NW, N, true); else WALK_V(NW, N, false); } while (0)
-  if (d.dim <= 64) WALK(4, 1); else if (d.dim <= 128) WALK(4, 2); else WALK(8, 2);
+#define WALK(NW, N) do { if (d.channel_decay) WALK_C(NW, N, true); else WALK_C(NW, N, false); } while (0)
+  switch (delta_tiles(d)) { case 4: WALK(4, 1); break; case 8: WALK(4, 2); break; default: WALK(8, 2); break; }
+#undef WALK_C
 #undef WALK
-#undef WALK_V
   CAI_HIP(hipGetLastError());
   return CAI_OK;
 }

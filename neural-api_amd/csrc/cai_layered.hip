@@ -252,7 +252,7 @@ struct LayeredNet {
   std::vector<NetRun> runs;
   // widths over all layers
   int wp = 0, ld_proj = 0, ld_mid = 0, ld_att = 0, ld_attl = 0, ld_q = 0, ld_ra = 0, ld_rg = 0;
-  int w_q = 0, w_k = 0, w_v = 0, w_g = 0, w_b = 0, w_za = 0, w_zg = 0, w_hd = 0, w_qt = 0, w_qk = 0, w_gt1 = 0;
+  int w_q = 0, w_k = 0, w_v = 0, w_g = 0, w_b = 0, w_za = 0, w_zg = 0, w_qt = 0, w_qk = 0; int64_t w_rec = 0, w_gt = 0;
   int ld_cat = 0, ld_ys = 0, ld_g2 = 0, ld_h2 = 0;
   size_t part_floats = 0;
   int64_t w_cb = 0, w_sx = 0, w_sb = 0, w_sdt = 0, w_sy = 0;                       // state-space scratch, elements per row (cb: per chunk)
@@ -297,7 +297,7 @@ static void drop_graphs(LayeredNet* n)
 
 static void free_rows(LayeredNet* n)
 {
-  void* p[] = {n->x, n->x0, n->proj, n->yl, n->yr, n->part, n->h, n->mid, n->att, n->attl, n->qbuf, n->ra, n->rgb, n->db.q, n->db.k, n->db.v, n->db.g, n->db.beta, n->db.o, n->db.za, n->db.zg, n->db.w, n->db.qt, n->db.qk, n->db.gt, n->cat, n->h2, n->g2, n->kept, n->inv, n->ql, n->qraw, n->qabs,
+  void* p[] = {n->x, n->x0, n->proj, n->yl, n->yr, n->part, n->h, n->mid, n->att, n->attl, n->qbuf, n->ra, n->rgb, n->db.q, n->db.k, n->db.v, n->db.g, n->db.beta, n->db.o, n->db.za, n->db.zg, n->db.rec, n->db.qt, n->db.qk, n->db.gt, n->cat, n->h2, n->g2, n->kept, n->inv, n->ql, n->qraw, n->qabs,
                n->sb.x, n->sb.B, n->sb.C, n->sb.dt, n->sb.cb, n->sb.bt, n->sb.fac, n->sb.y, n->eb.z, n->eb.wgt, n->eb.y, n->eb.ys, n->eb.sel, n->eb.order, n->eb.tiles, n->eb.n_tiles, n->eb.few, n->eb.mid, n->eb.mid_s};
   for (void* q : p) if (q) (void)hipFree(q);
   n->x = n->x0 = n->proj = n->yl = n->yr = n->part = nullptr;
@@ -321,7 +321,8 @@ static int ensure_rows(LayeredNet* n, int rows)
     CAI_HIP(hipMemsetAsync(*p, 0, bytes, ctx().stream));
     return CAI_OK;
   };
-  const size_t RS = R + DELTA_CHUNK + 1;    // the chunked walk requests whole chunks: up to 15 rows (and three values) past the last one
+  const size_t RS = R + DELTA_CHUNK + 1;    // the walk of the gated linear attention requests whole chunks: up to 15 rows (and three values) past the last one
+  const size_t chunks = R / DELTA_CHUNK + n->max_seq + 1;
   size_t part = 0;
   // (with bfloat16 activations only steps without a prompt portion take the row form)
   const int part_rows = n->act_t == ACT_T_F32 ? (int)R : std::min((int)R, ATTN_PROMPT_MIN * n->max_seq);
@@ -336,8 +337,8 @@ static int ensure_rows(LayeredNet* n, int rows)
       (rc = get((void**)&n->db.q, RS * n->w_q * 4)) || (rc = get((void**)&n->db.k, RS * n->w_k * 4)) || (rc = get((void**)&n->db.v, RS * n->w_v * 4)) ||
       (rc = get((void**)&n->db.g, RS * n->w_g * 4)) || (rc = get((void**)&n->db.beta, RS * n->w_b * 4)) || (rc = get((void**)&n->db.o, RS * n->w_v * 4)) ||
       (rc = get((void**)&n->db.za, R * n->w_za * 4)) || (rc = get((void**)&n->db.zg, R * n->w_zg * 4)) ||
-      (rc = get((void**)&n->db.w, RS * n->w_hd * 4)) || (rc = get((void**)&n->db.qt, RS * n->w_qt * 4)) || (rc = get((void**)&n->db.qk, RS * n->w_qk * 4)) ||
-      (rc = get((void**)&n->db.gt, std::max(RS * n->w_gt1, (R / DELTA_CHUNK + n->max_seq + 1) * n->w_qt + 4) * 4)) ||
+      (rc = get((void**)&n->db.rec, chunks * n->w_rec * 4)) || (rc = get((void**)&n->db.qt, RS * n->w_qt * 4)) || (rc = get((void**)&n->db.qk, RS * n->w_qk * 4)) ||
+      (rc = get((void**)&n->db.gt, n->w_gt ? (chunks * n->w_gt + 4) * 4 : 0)) ||
       (rc = get(&n->cat, R * n->ld_cat * n->es)) || (rc = get(&n->h2, R * n->ld_h2 * n->es)) || (rc = get((void**)&n->g2, R * n->ld_g2 * 4)) ||
       (rc = get((void**)&n->kept, n->has_sandwich ? (n->s.layers.size() + 1) * R * w * 4 : 0)) || (rc = get((void**)&n->inv, n->has_sandwich ? R * 4 : 0)) ||
       (rc = get(&n->ql, R * n->ld_ql * n->es)) || (rc = get((void**)&n->qraw, R * n->ld_qr * 4)) || (rc = get((void**)&n->qabs, R * n->w_qa * 4)) ||
@@ -438,8 +439,7 @@ int net_create(NetSpec&& spec, int max_tokens, int max_seq, int act_t, LayeredNe
       up(n->ld_att, pad_to(d.heads * d.vdim, LIN_PAD));
       up(n->w_q, d.kv_heads * d.dim); up(n->w_k, d.kv_heads * d.dim); up(n->w_v, d.heads * d.vdim);
       up(n->w_g, d.channel_decay ? d.heads * d.dim : d.heads); up(n->w_b, d.heads + d.kv_heads);
-      up(n->w_hd, d.heads * d.dim); up(n->w_qk, d.heads * DELTA_CHUNK);
-      if (d.channel_decay) up(n->w_qt, d.heads * d.dim); else up(n->w_gt1, 2 * d.heads);
+      up(n->w_rec, (int64_t)d.heads * delta_record_blocks(d) * 256); up(n->w_gt, d.channel_decay ? d.heads * delta_tiles(d) * 16 : d.heads);
       if (d.rank_a) { up(n->ld_ra, pad_to(d.rank_a, LIN_PAD)); up(n->w_za, d.channel_decay ? d.heads * d.dim : d.heads); }
       if (d.rank_g) { up(n->ld_rg, pad_to(d.rank_g, LIN_PAD)); up(n->w_zg, d.heads * d.vdim); }
     }
@@ -458,7 +458,7 @@ int net_create(NetSpec&& spec, int max_tokens, int max_seq, int act_t, LayeredNe
     if (y.kind == MIX_GLA) {
       const GlaDims& d = y.gla.d;
       up(n->ld_att, pad_to(d.heads * d.vdim, LIN_PAD));
-      up(n->w_v, d.heads * d.vdim); up(n->w_g, d.heads * d.dim); up(n->w_qt, d.heads * d.dim); up(n->w_qk, d.heads * DELTA_CHUNK);
+      up(n->w_v, d.heads * d.vdim); up(n->w_g, d.heads * d.dim); up(n->w_qt, d.heads * d.dim); up(n->w_qk, d.heads * DELTA_CHUNK); up(n->w_gt, d.heads * d.dim);
     }
     if (y.kind == MIX_SSD) {
       const SsdDims& d = y.ssd.d;

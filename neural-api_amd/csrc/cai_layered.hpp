@@ -219,9 +219,13 @@ struct DeltaW {
 };
 struct DeltaBuf {                          // per-row scratch of a prompt pass
   float *q, *k, *v, *g, *beta, *o, *za, *zg;
-  float *w, *qt, *qk, *gt;                 // chunked form: T [P k], P q, q D k, and the products of decays
+  float *rec;                              // chunked delta rule: a record of matrix operands per chunk and head (delta_record_blocks KB)
+  float *qt, *qk;                          // chunked gated linear attention: P q, q D k
+  float *gt;                               // both: the decays of whole chunks
 };
 constexpr int DELTA_CHUNK = 16;            // tokens per chunk
+__host__ __device__ inline int delta_tiles(const DeltaDims& d) { return d.dim <= 64 ? 4 : d.dim <= 128 ? 8 : 16; }                  // of 16 key channels, as the walk's waves share them
+__host__ __device__ inline int delta_record_blocks(const DeltaDims& d) { return 3 * delta_tiles(d) + 1 + (d.vdim + 15) / 16; }      // of [64 lanes][4] floats
 constexpr int DELTA_CHUNK_MIN = 32;        // portions from here on make a step take the chunked form
 int delta_prep(const DeltaDims& d, const DeltaIn& in, const DeltaW& w, const SeqPool::StateRun& st, const StepRows& r, const DeltaBuf& b);
 int delta_scan(const DeltaDims& d, const SeqPool::StateRun& st, const StepRows& r, const DeltaBuf& b);

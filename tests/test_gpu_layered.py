@@ -168,6 +168,20 @@ def test_mechanism_alone(cai, tmp_path, mech, i, dt):
     dec.close()
 
 
+# Numbers of chunks of 16 that leave the walk's loop over three at each of its places, last chunks whole and ragged; key widths of 4, 8 and 16
+# tiles, value widths of whole and of ragged slices
+@pytest.mark.parametrize("n", [32, 33, 47, 48, 49, 64, 81])
+@pytest.mark.parametrize("h, g, d, dv", [(8, 4, 64, 48), (2, 1, 72, 22), (2, 2, 136, 16)])
+@pytest.mark.parametrize("mech", ["delta", "channel delta"])
+def test_chunks_of_a_portion(cai, tmp_path, mech, h, g, d, dv, n):
+    mixer = B.delta(h, g, d, dv, 4)
+    m = Model(tmp_path, B.config([B.layer(mixer if mech == "delta" else (B.attn(), mixer))], width=72, vocab=67), seed=n, edit=only(mech), rank_a=9, rank_g=20)
+    tok = m.tokens(n + 5, d)
+    dec = m.open(cai, 192, 1, "f32")
+    check(feed(dec, tok, [n, 5]), m.ref(tok), "f32")
+    dec.close()
+
+
 @pytest.mark.parametrize("tokens, ff", [(129, 16400), (257, 8208), (300, 12000)])
 def test_products_on_tiles_of_256_tokens(cai, tmp_path, tokens, ff):
     """gate | up matrices whose products fill the chip with large tiles: tokens one past half a tile, one past a tile and inside a second one, rows
