@@ -9,8 +9,6 @@
 
 namespace cai {
 
-typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
-
 // ------------------------------------------------------------------------------------------
 // prompt pass 1: q and k unit vectors (q scaled), v, decay, write strength, q . k.
 // A wave owns one unit - the q and k channels of a key head, 256 channels of v, 256 decays, the write strengths - over eight

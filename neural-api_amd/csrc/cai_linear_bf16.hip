@@ -436,6 +436,51 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16(const uint16_t* __rest
       __syncthreads();
     }
   }
+  const bool whole = (e.ldy & 3) == 0 && (e.ldh & 3) == 0 && (e.ld0 & 3) == 0 && (e.ldg & 3) == 0 && (e.split & 3) == 0;
+  if constexpr (MODE == EPI_RESIDUAL && !BANK) {
+    // outputs in the outer loop: their bias and norm factors are requested once (for every token again, behind stores they might alias, they
+    // are half of the epilogue), and the stream of all the tokens before the first is changed
+    if (whole) {
+#pragma unroll
+      for (int j = 0; j < TN; j++) {
+        const int n = n0 + wn + j * 16 + fc * 4;
+        if (n >= n_rows) continue;
+        if (n + 3 >= n_rows) {
+          for (int i = 0; i < TM; i++) {
+            const int t = m0 + wm + i * 16 + fr;
+#pragma unroll
+            for (int q = 0; q < 4; q++) if (t < n_tok && n + q < n_rows) epi_as<AT, MODE>(e, n + q, t, acc[j][i][q]);
+          }
+          continue;
+        }
+        const DytFour post = dyt_four(e.post, n), next = dyt_four(e.next, n);
+        const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+        f32x4 bias = zero;
+        if (e.bias) bias = *reinterpret_cast<const f32x4_any*>(e.bias + n);
+        constexpr int P = TM * TN < 16 ? TM : 2;         // (tokens at once: with more the largest tile's sums leave their registers)
+#pragma unroll
+        for (int i0 = 0; i0 < TM; i0 += P) {
+          f32x4 x[P], x0[P];
+#pragma unroll
+          for (int i = 0; i < P; i++) {
+            const int64_t t = min(m0 + wm + (i0 + i) * 16 + fr, n_tok - 1);
+            x[i] = e.fresh ? zero : *reinterpret_cast<const f32x4*>(e.y + t * e.ldy + n);
+            x0[i] = e.add0 ? *reinterpret_cast<const f32x4*>(e.add0 + t * e.ld0 + n) : zero;
+          }
+#pragma unroll
+          for (int i = 0; i < P; i++) {
+            const int64_t t = m0 + wm + (i0 + i) * 16 + fr;
+            x[i] += dyt(e.post, post, acc[j][i0 + i] + bias);
+            if (e.add0) x[i] += x0[i];
+            if (t >= n_tok) continue;
+            *reinterpret_cast<f32x4*>(e.y + t * e.ldy + n) = x[i];
+            if (e.h) put_four<AT>(e.h, t * e.ldh + n, dyt(e.next, next, x[i]));
+          }
+        }
+      }
+      return;
+    }
+  }
 #pragma unroll
   for (int i = 0; i < TM; i++) {
     int t = m0 + wm + i * 16 + fr;
@@ -471,7 +516,6 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16(const uint16_t* __rest
       }
       continue;
     }
-    const bool whole = (e.ldy & 3) == 0 && (e.ldh & 3) == 0 && (e.ld0 & 3) == 0 && (e.ldg & 3) == 0 && (e.split & 3) == 0;
 #pragma unroll
     for (int j = 0; j < TN; j++) {
       const int n = n0 + wn + j * 16 + fc * 4;
@@ -623,16 +667,24 @@ static int run_lin(const cai_qw_s* w, const AT* x, int64_t ldx, int n_tok, const
     return CAI_OK;
   }
   auto tiles = [&](int bm, int bn) { return (int64_t)((n_tok + bm - 1) / bm) * ((w->rows + bn - 1) / bn); };
-  // 256 x 128 by sixteen waves, one work-group a CU, or 128 x 128 by eight, two a CU: whichever takes less time by rounds over the chip.  A
-  // full round takes 32 us of the one and 37 of the other (at a depth of 2048), one of at most a work-group a CU 28.  Products alone, us,
-  // 256 x 128 | 128 x 128 (by four waves, staged through registers, before): 11264 rows, 300 tokens 30.8 | 31.9 (40.7), 640: 57.1 | 35.6
-  // (46.2), 768: 59.0 | 57.1, 1024: 63.5 | 67.5, 2048: 98.6 | 110.2 (127); 32800 rows, 128 tokens 57.6 | 43.9 (45.4); 49152 rows, 100: 61.1 | 50.4.
-  // (Where 128 x 128 leaves CUs idle the halved tiles of 64 x 64 are faster: whole prompt of 511 tokens, width 512: 609, 628.)
-  if (n_tok > 64 && tiles(128, 128) >= ctx().n_cu) {
+  // Large tiles, by rounds over the chip: 256 x 256 by sixteen waves or 256 x 128 by sixteen, one work-group a CU, or 128 x 128 by eight, two a
+  // CU.  A full round takes 57, 33 and 37 us (at a depth of 2048), one of 128 x 128 with at most a work-group a CU 28.  Products alone, us,
+  // 256 x 256 | 256 x 128 | 128 x 128 by eight: 11264 rows, 1024 tokens 56 | 65 | 59, 2048: 113 | 105 | 108; 6200 rows, 1024 tokens 49 | 34 | 34, 2048: 57 | 67 | 67;
+  // without the first: 11264 rows, 300 tokens 30.8 | 31.9, 640: 57.1 | 35.6; 32800 rows, 128 tokens 57.6 | 43.9; 49152 rows, 100: 61.1 | 50.4.
+  // Where one round of 128 x 128 covers everything, sixteen waves and copies three steps ahead (a CU has one work-group): 2048 x 2048, 2048 tokens 33 | 24 (256 x 128 |
+  // here), 2048 x 5632 75 | 54, 6200 x 2048, 512 tokens 29 (64 x 64) | 21, 11264 x 2048, 256 tokens 23 | 21; up to two tiles of 64 x 64 a CU those take less
+  // (2048 rows, 1024 tokens 16 | 20; 6200 rows, 256: 15 | 18.5).
+  // What holds a tile's step up is neither the copies by themselves (128 x 128 steps alone 0.39 us, here 0.55), the fragment reads (two groups of waves with half
+  // the columns each, a quarter fewer, took the same) nor their order (a half step's read while the half before is multiplied: the same).
+  const int64_t n_cu = ctx().n_cu, small = tiles(128, 128);
+  if constexpr (sizeof(AT) == 2)
+    if (n_tok > 64 && small <= n_cu && tiles(64, 64) > 2 * n_cu) return run_gemm<AT, 128, 128, 4, 4, 4>(w, x, ldx, n_tok, e);
+  if (n_tok > 64 && small >= n_cu) {
     if constexpr (sizeof(AT) == 2) {
-      const int64_t n_cu = ctx().n_cu, large = tiles(256, 128), small = tiles(128, 128), left = small % (2 * n_cu);
-      if (32 * ((large + n_cu - 1) / n_cu) <= 37 * (small / (2 * n_cu)) + (left == 0 ? 0 : left <= n_cu && small > n_cu ? 28 : 37))
-        return run_gemm<AT, 256, 128, 4, 4, 3>(w, x, ldx, n_tok, e);
+      const int64_t left = small % (2 * n_cu), t_small = 37 * (small / (2 * n_cu)) + (left == 0 ? 0 : left <= n_cu && small > n_cu ? 28 : 37);
+      const int64_t t_large = 33 * ((tiles(256, 128) + n_cu - 1) / n_cu), t_huge = 57 * ((tiles(256, 256) + n_cu - 1) / n_cu);
+      if (t_huge < t_large && t_huge < t_small) return run_gemm<AT, 256, 256, 4, 4, 2>(w, x, ldx, n_tok, e);
+      if (t_large <= t_small) return run_gemm<AT, 256, 128, 4, 4, 3>(w, x, ldx, n_tok, e);
     }
     return run_gemm<AT, 128, 128, 2, sizeof(AT) == 2 ? 4 : 2>(w, x, ldx, n_tok, e);
   }

@@ -88,13 +88,22 @@ def test_few_rows_of_many_outputs_over_bf16_rows(cai, rows, cols):
 
 @pytest.mark.parametrize("rows, cols", [(32, 64), (96, 320), (5664, 72), (8224, 72), (2144, 2112), (8288, 2112), (64, 8192), (160, 264), (64, 8200)])
 def test_gated_products_over_bf16_rows(cai, rows, cols):
+    gated_products(cai, rows, cols, (1, 2, 3, 5, 7, 8, 9, 13, 16, 17, 33, 70))
+
+
+@pytest.mark.parametrize("rows, cols, tokens", [(2016, 264, 1100), (6208, 136, 2050)])
+def test_gated_products_on_one_round_of_large_tiles(cai, rows, cols, tokens):
+    gated_products(cai, rows, cols, (tokens,))
+
+
+def gated_products(cai, rows, cols, tokens):
     """the same of gate and up rows: the bounds of both sums, then one rounding to bfloat16 (2^-8 of the value at most)"""
     rng = np.random.default_rng(rows + cols)
     bits, w = B.to_bf16(rng.standard_normal((rows, cols)))
     w = w.reshape(rows // 32, 2, 16, cols).astype(np.float64)
     gate, up = w[:, 0].reshape(-1, cols), w[:, 1].reshape(-1, cols)
     q = cai.QWeight(cai.BF16, rows, cols, bits)
-    for n in (1, 2, 3, 5, 7, 8, 9, 13, 16, 17, 33, 70):
+    for n in tokens:
         x = B.to_bf16(rng.standard_normal((n, cols)))[1].reshape(n, cols).astype(np.float64)
         g, u = x @ gate.T, x @ up.T
         dg, du = 2.0 ** -19 * (np.abs(x) @ np.abs(gate).T), 2.0 ** -19 * (np.abs(x) @ np.abs(up).T)
@@ -200,6 +209,29 @@ def test_products_on_large_tiles_of_many_steps(cai, tmp_path, tokens, ff, width)
     m = Model(tmp_path, B.config([B.layer(B.delta(), ff=ff)], width=width, vocab=67), seed=tokens, edit=only("feed-forward"), rank_a=3, rank_g=20)
     tok = m.tokens(tokens, 1)
     dec = m.open(cai, 768, 1, "bf16")
+    check(feed(dec, tok, [tokens]), m.ref(tok), "bf16")
+    dec.close()
+
+
+@pytest.mark.parametrize("rows, cols, tokens", [(2041, 264, 1100), (4300, 72, 513), (16300, 320, 130), (6200, 328, 2050), (4104, 72, 2100)])
+def test_one_round_of_large_tiles(cai, rows, cols, tokens):
+    """Tiles of 128 x 128 by sixteen waves (one round of them that has more than two tiles of 64 x 64 a CU: the first three) and of 256 x 256 (one round instead
+    of two of 256 x 128), one to six steps of 64 deep, rows and tokens that end inside a tile.  The bound is that of test_products_over_bf16_rows."""
+    rng = np.random.default_rng(rows)
+    bits, w = B.to_bf16(rng.standard_normal((rows, cols)))
+    w = w.reshape(rows, cols).astype(np.float64); bias = rng.standard_normal(rows).astype(np.float32)
+    q = cai.QWeight(cai.BF16, rows, cols, bits, bias)
+    x = B.to_bf16(rng.standard_normal((tokens, cols)))[1].reshape(tokens, cols).astype(np.float64)
+    assert np.all(np.abs(bf16_rows(cai, q, x) - (x @ w.T + bias)) <= 2.0 ** -19 * (np.abs(x) @ np.abs(w).T + np.abs(bias)))
+    q.close()
+
+
+@pytest.mark.parametrize("width, tokens", [(2056, 1100), (4104, 2050), (2054, 1090)])
+def test_residuals_of_large_tiles(cai, tmp_path, width, tokens):
+    """the stream's update and the norms around it behind tiles of 128 x 128 by sixteen waves and of 256 x 256; a width that is no whole fours"""
+    m = Model(tmp_path, B.config([B.layer(B.delta(1, 1, 8, 8, 2), ff=72)], width=width, vocab=67), seed=width, rank_a=3, rank_g=20)
+    tok = m.tokens(tokens, 1)
+    dec = m.open(cai, 2112, 1, "bf16")
     check(feed(dec, tok, [tokens]), m.ref(tok), "bf16")
     dec.close()
 
