@@ -420,13 +420,23 @@ static int enqueue_prefill_chunk(cai_decoder_s* d, int seq, int n)
   const int32_t* toks = d->ptokpos; const int32_t* poss = d->ptokpos + d->pf_cap;
   int rc;
   if ((rc = launch_embed(d->embed, toks, n, d->px))) return rc;
+  // Between the layers of a short prompt the activations stay planes (7 launches a layer instead of 10)
+  bool planes = c.n_experts == 0;
+  for (int l = 0; planes && l < c.n_layers; l++) {
+    auto& L = d->layers[l];
+    planes = blk_short_wanted(L.w[CAI_W_Q], L.w[CAI_W_K], L.w[CAI_W_V], L.w[CAI_W_O], L.w[CAI_W_GATEUP], L.w[CAI_W_DOWN], n) && L.v[CAI_V_ATTN_NORM] && L.v[CAI_V_MLP_NORM];
+  }
+  BlkPlanes xp[2];                 // of the stream, and of what the attention and the feed-forward leave
+  if (planes && ((rc = blk_short_planes(n, dm, std::max(qw, I), xp)) || (rc = launch_blk_planes(d->layers[0].w[CAI_W_Q], d->px, d->layers[0].v[CAI_V_ATTN_NORM], n, xp[0])))) return rc;
   for (int l = 0; l < c.n_layers; l++) {
     auto& L = d->layers[l];
     const cai_qw_s* wq = L.w[CAI_W_Q]; const cai_qw_s* wk = L.w[CAI_W_K]; const cai_qw_s* wv = L.w[CAI_W_V];
     const bool all_mfma = prompt_route(wq, n) == 2 && prompt_route(wk, n) == 2 && prompt_route(wv, n) == 2;   // one pre-pass serves q, k and v
-    if (all_mfma && (rc = prefill_prep(d->px, dm, L.v[CAI_V_ATTN_NORM], c.eps, dm, n))) return rc;
+    if (!planes && all_mfma && (rc = prefill_prep(d->px, dm, L.v[CAI_V_ATTN_NORM], c.eps, dm, n))) return rc;
     const cai_qw_s* qkv3[3] = {wq, wk, wv}; const int qkv_off[3] = {0, qw, qw + kw};
-    if (all_mfma && prefill_multi_supported(qkv3, 3)) {   // one launch: the k and v projections alone leave half the chip idle
+    if (planes) {
+      if ((rc = launch_gemm_blk_short(qkv3, qkv_off, 3, xp[0], c.eps, n, d->pqkv, qkvw, nullptr, 0, BlkPlanes(), nullptr))) return rc;
+    } else if (all_mfma && prefill_multi_supported(qkv3, 3)) {   // one launch: the k and v projections alone leave half the chip idle
       if ((rc = prefill_gemm_multi(qkv3, qkv_off, 3, n, d->pqkv, qkvw))) return rc;
     } else if (all_mfma && prefill_multi_supported(qkv3, 2)) {   // attn_v of another type (a Q4_K_M file keeps some in Q6_K): q | k together
       if ((rc = prefill_gemm_multi(qkv3, qkv_off, 2, n, d->pqkv, qkvw))) return rc;
@@ -441,6 +451,15 @@ static int enqueue_prefill_chunk(cai_decoder_s* d, int seq, int n)
       if ((rc = launch_attn_step(&d->kv, l, d->pqkv + (int64_t)r0 * qkvw, qkvw, std::min(d->ppart_rows, n - r0), c.n_q_heads, c.window, 0.0f, d->theta,
                                  poss + r0, d->patt + (int64_t)r0 * qw, qw, seq, 1, d->ppart,
                                  c.qk_norm_full ? L.v[CAI_V_Q_NORM] : nullptr, c.qk_norm_full ? L.v[CAI_V_K_NORM] : nullptr, c.eps))) return rc;
+    if (planes) {
+      const cai_qw_s *wo = L.w[CAI_W_O], *wgu = L.w[CAI_W_GATEUP], *wd = L.w[CAI_W_DOWN]; const int zero = 0;
+      const float* next = l + 1 < c.n_layers ? d->layers[l + 1].v[CAI_V_ATTN_NORM] : nullptr;
+      if ((rc = launch_blk_planes(wo, d->patt, nullptr, n, xp[1]))) return rc;
+      if ((rc = launch_gemm_blk_short(&wo, &zero, 1, xp[1], -1.0f, n, d->px, dm, d->px, 0, xp[0], L.v[CAI_V_MLP_NORM]))) return rc;
+      if ((rc = launch_gemm_blk_short(&wgu, &zero, 1, xp[0], c.eps, n, nullptr, 0, nullptr, I, xp[1], nullptr))) return rc;
+      if ((rc = launch_gemm_blk_short(&wd, &zero, 1, xp[1], -1.0f, n, d->px, dm, d->px, 0, next ? xp[0] : BlkPlanes(), next))) return rc;
+      continue;
+    }
     if ((rc = linear_rows(L.w[CAI_W_O], false, d->patt, qw, nullptr, 0.0f, n, d->px, dm, d->px))) return rc;
     if (c.n_experts > 0) {
       // experts differ from token to token.  A chunk of more than 8 tokens whose banks the block prompt kernel takes is

@@ -306,6 +306,15 @@ int moe_group_max_tiles(int n_slots, int n_experts);
 int launch_moe_group(const int32_t* expert, int n_slots, int n_experts, int32_t* perm, int32_t* tile_tab);
 int launch_gemm_blk_grouped(const cai_qw_s* bank, int64_t expert_rows, const _Float16* xhi, const _Float16* xlo, const float* sinv, int x_div,
                             int n_slots, int n_experts, const int32_t* perm, const int32_t* tile_tab, float* y, int64_t y_stride);
+// Activations of a short prompt between its products (cai_prefill_blk.hip): hi / lo planes in the order of the matrix operands, scaled by a power of two a token and 32
+// columns, its reciprocal, and the sums of the 32 values' squares before the gain
+struct BlkPlanes { _Float16 *hi = nullptr, *lo = nullptr; float *scale = nullptr, *squares = nullptr; };
+bool blk_short_wanted(const cai_qw_s* wq, const cai_qw_s* wk, const cai_qw_s* wv, const cai_qw_s* wo, const cai_qw_s* wgu, const cai_qw_s* wd, int n_tok);
+int  blk_short_planes(int n_tok, int width0, int width1, BlkPlanes (&out)[2]);
+void blk_short_release();
+int  launch_blk_planes(const cai_qw_s* w, const float* x, const float* gain, int n_tok, const BlkPlanes& o);
+int  launch_gemm_blk_short(const cai_qw_s* const* ws, const int* y_off, int n_w, const BlkPlanes& x, float eps, int n_tok, float* y, int64_t y_stride, const float* residual, int half,
+                           const BlkPlanes& out, const float* gain);
 void prefill_planes(const _Float16** hi, const _Float16** lo, const float** sinv);   // what the last prefill_prep filled
 int  prompt_route(const cai_qw_s* w, int n_tok);   // 0 matrix-vector passes, 1 small-batch kernel, 2 prompt kernel
 bool nb_supported(const cai_qw_s* w);          // 2..8-token matrix-core kernel

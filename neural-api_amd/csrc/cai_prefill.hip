@@ -702,6 +702,7 @@ void prefill_release()   // cai_shutdown
   for (void* v : q) if (v) (void)hipFree(v);
   g_pws = PrefillWs();
   raw_release();
+  blk_short_release();
 }
 
 int prefill_prep(const float* x, int64_t x_stride, const float* gain, float eps, int K, int n_tok)

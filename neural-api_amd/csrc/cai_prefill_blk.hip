@@ -70,6 +70,15 @@ __device__ __forceinline__ half8_b codes8(uint32_t w0, uint32_t w1, int high, bo
   return half8_b{h0.x, h0.y, h1.x, h1.y, h2.x, h2.y, h3.x, h3.y};
 }
 
+// where token t (of 16) and column c of a block lie in it, in the order of gemm_blk_short's operands: which eight columns a lane (t, kg) holds
+// follows from how the lanes share a chunk of weights
+template <int QT> __device__ __forceinline__ int plane_place(int t, int c)
+{
+  const int g = c >> 3, kg = QT == CAI_Q8_0 ? (g >> 1) | ((g & 1) << 1) : g;
+  return kg * 128 + t * 8 + (c & 7);
+}
+typedef uint32_t uint2_b __attribute__((ext_vector_type(2)));
+
 }  // namespace
 
 // ------------------------------------------------------------------------------------------
@@ -498,6 +507,194 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 }
 
 // ------------------------------------------------------------------------------------------
+// The products of a short prompt's layers, whose activations stay planes from product to product (launch_gemm_blk_short): what finishes 32
+// outputs of a token scales them by a power of two of their largest and leaves them in the order of the matrix operands, with the sum of their
+// squares; the norm's gain is multiplied in by the writer, its root divided by at the end of the reader.  So a layer has 7 launches instead of 10, and a
+// wave requests its operands straight into registers, one contiguous KB an instruction, all of a short width at once: a width of 2048 comes in
+// one round trip, where the cut tiles above take one a chunk of 64 columns and stage them in LDS.
+//   planes: tile of 16 tokens, block of 32 columns, [64 lanes][8 halfs]; scales and squares: tile, block, [16 tokens].
+// A work-group's waves cut the width of 16 tokens x 32 rows (PAIR: 32 up rows and their 32 gate rows) and meet in LDS at the end, a result a thread.  hi and lo
+// are summed apart, every second block with its sign changed, in chains of eight blocks (FINE above).
+// What bounds it: a launch, a round trip and the requests themselves, which touch a line a row of weights: 14 a chunk (the scales one by one, eight
+// bytes of a row) took 11.2 us for the down product of the 135M shape (576 x 1536, 37 tokens), 9 a chunk 8.2; tiles of 32 tokens 10.2.  Results that
+// left as single halfs cost gate | up 1.7 us.  A layer of that prompt, kernels alone, us: q | k | v 4.8, append 2.8, attention 6.4, its planes
+// 2.3, o 4.9, gate | up with SwiGLU 6.9, down 8.2 = 36; with rows between the products 51 (four pre-passes of 4.1, products 5.2, 4.5, 5.4 and 9.4).
+// ------------------------------------------------------------------------------------------
+struct BlkShortParams {
+  const uint8_t* q[3]; const uint8_t* d[3]; const float* bias[3]; int rows[3]; int y_off[3]; int seg_end[2]; int n_seg;     // up to three matrices of one type and width
+  int cols, n_tok, n_row_groups, n_tok_tiles, half;   // half > 0: rows [0, half) are up, [half, 2 half) gate
+  BlkPlanes x; int normed; float eps;                 // (x.squares are read where the rows are normed)
+  float* y; int64_t y_stride; const float* residual;
+  BlkPlanes out; const float* gain;                   // planes of the results, times a gain (out.hi null: none)
+};
+constexpr int BS_NW = 8;
+template <int QT, bool PAIR, bool TWICE>       // TWICE: two work-groups a CU
+__global__ __launch_bounds__(64 * BS_NW) __attribute__((amdgpu_waves_per_eu(TWICE ? 4 : 2, TWICE ? 4 : 2))) void gemm_blk_short(const BlkShortParams p)
+{
+  constexpr int NW = BS_NW, RT = PAIR ? 4 : 2, P = TWICE ? (PAIR ? 1 : 2) : PAIR ? 3 : 4;      // row tiles of 16; chunks of 64 columns on their way to a wave
+  __shared__ float sums[NW][RT * 4][64];
+  __shared__ float s_sq[NW][16];
+  __shared__ __align__(16) _Float16 s_out[2][512];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 15, kg = lane >> 4;
+  const int L = blockIdx.x, rg = (L & 7) + 8 * ((L >> 3) / p.n_tok_tiles), tile = (L >> 3) % p.n_tok_tiles;     // (the token tiles of a row group share an XCD and its L2)
+  if (rg >= p.n_row_groups) return;
+  int sg = 0, rgl = rg;
+  if (p.n_seg > 1 && rg >= p.seg_end[0]) { sg = 1; rgl = rg - p.seg_end[0]; }
+  if (p.n_seg > 2 && rg >= p.seg_end[1]) { sg = 2; rgl = rg - p.seg_end[1]; }
+  const float* const bias = p.bias[sg];
+  const int rows = p.rows[sg], R0 = rgl * 32, K = p.cols, nb32 = K >> 5, n_chunks = (nb32 + 1) >> 1;
+  const int c0 = n_chunks * wave / NW, c1 = n_chunks * (wave + 1) / NW;
+  const _Float16 *const xh = p.x.hi + (int64_t)tile * nb32 * 512 + lane * 8, *const xl = p.x.lo + (int64_t)tile * nb32 * 512 + lane * 8;
+  const float* const xs = p.x.scale + (int64_t)tile * nb32 * 16 + 4 * kg;
+  // A request touches sixteen rows, a line each, so a chunk of a row is shared out over the four lanes of the row and changes hands in registers:
+  // (Q8_0) 16 bytes a lane, (Q4_0) 8; the two scales of a row, of row tile kg.
+  auto row_of = [&](int rt) { return (PAIR && rt >= 2 ? (int64_t)p.half : 0) + min(R0 + 16 * (rt & 1) + n, rows - 1); };     // rows past the end: the last one again, not written
+  const uint8_t* wq[RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; rt++) wq[rt] = p.q[sg] + row_of(rt) * (QT == CAI_Q8_0 ? K : K / 2) + (QT == CAI_Q8_0 ? 16 : 8) * kg;
+  const uint8_t* const wd = p.d[sg] + (kg & 2 ? row_of(RT == 4 ? 2 + (kg & 1) : kg & 1) : row_of(kg & 1)) * (nb32 * 2);
+  const bool odd = nb32 & 1;
+  typedef std::conditional_t<QT == CAI_Q8_0, u32x4_b, uint2_b> Quants;
+  struct Chunk { half8_b h[2], l[2]; f32x4_b sc[2]; Quants w[RT]; uint32_t d; };
+  auto fetch = [&](int c, Chunk& x) {
+#pragma unroll
+    for (int b = 0; b < 2; b++) {                       // (behind the last block of an odd number of them: that one again, not used)
+      const int kb = min(2 * c + b, nb32 - 1);
+      x.h[b] = *reinterpret_cast<const half8_b*>(xh + kb * 512); x.l[b] = *reinterpret_cast<const half8_b*>(xl + kb * 512);
+      x.sc[b] = *reinterpret_cast<const f32x4_b*>(xs + kb * 16);
+    }
+    // the last chunk of an odd number of blocks: the lanes of its second half stay on the first
+    const int back = odd && 2 * c + 1 >= nb32 && kg >= 2 ? (QT == CAI_Q8_0 ? 32 : 16) : 0;
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++) x.w[rt] = *reinterpret_cast<const Quants*>(wq[rt] + c * (QT == CAI_Q8_0 ? 64 : 32) - back);
+    if (odd) x.d = *reinterpret_cast<const uint16_t*>(wd + c * 4) | (uint32_t)*reinterpret_cast<const uint16_t*>(wd + min(2 * c + 1, nb32 - 1) * 2) << 16;
+    else x.d = *reinterpret_cast<const uint32_t*>(wd + c * 4);
+  };
+  Chunk r[P];
+#pragma unroll
+  for (int i = 0; i < P; i++) if (c0 + i < c1) fetch(c0 + i, r[i]);
+  // what finishes this thread's result - row R0 + tid % 32, token tid / 32 - is requested behind them
+  const int tl = tid >> 5, t = tile * 16 + tl, row = R0 + (tid & 31), rc = min(row, rows - 1);
+  const int64_t at_y = (int64_t)min(t, p.n_tok - 1) * p.y_stride + p.y_off[sg] + rc;
+  const float res = p.residual ? p.residual[at_y] : 0.0f, bs = bias ? bias[rc] : 0.0f, bs2 = PAIR && bias ? bias[p.half + rc] : 0.0f, gain = p.gain ? p.gain[rc] : 1.0f;
+  if (p.normed) {                                       // sums of squares: token tid % 16, a 32nd of the blocks
+    float ss = 0.0f;
+    for (int kb = tid >> 4; kb < nb32; kb += 4 * NW) ss += p.x.squares[((int64_t)tile * nb32 + kb) * 16 + n];
+    ss += __shfl_xor(ss, 16); ss += __shfl_xor(ss, 32);
+    if (kg == 0) s_sq[wave][n] = ss;
+  }
+  const f32x4_b zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4_b Y[RT], Z[RT], U[RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; rt++) Y[rt] = Z[rt] = U[rt] = zero;
+  auto use = [&](const Chunk& x, bool half) {
+    uint32_t d[4];                                      // of each row tile, in all lanes of a row
+    {
+      const uint2_b a = __builtin_amdgcn_permlane16_swap(x.d, x.d, false, false);         // tiles 0 0 2 2, 1 1 3 3
+      const uint2_b e = __builtin_amdgcn_permlane32_swap(a.x, a.x, false, false), o = __builtin_amdgcn_permlane32_swap(a.y, a.y, false, false);
+      d[0] = e.x; d[2] = e.y; d[1] = o.x; d[3] = o.y;
+    }
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++) {
+      uint32_t w0[2], w1[2];                            // a block's eight codes of this lane
+      if constexpr (QT == CAI_Q8_0) {
+        // lanes kg 0, 1 asked for block 0, kg 2, 3 for block 1: the halves change places, and each block is in all four
+        const uint2_b xz = __builtin_amdgcn_permlane32_swap(x.w[rt].x, x.w[rt].z, false, false), yw = __builtin_amdgcn_permlane32_swap(x.w[rt].y, x.w[rt].w, false, false);
+        w0[0] = xz.x; w1[0] = yw.x; w0[1] = xz.y; w1[1] = yw.y;
+      } else {
+        const uint2_b xx = __builtin_amdgcn_permlane32_swap(x.w[rt].x, x.w[rt].x, false, false), yy = __builtin_amdgcn_permlane32_swap(x.w[rt].y, x.w[rt].y, false, false);
+        const int sh = kg & 2 ? 4 : 0;
+        w0[0] = xx.x >> sh; w1[0] = yy.x >> sh; w0[1] = xx.y >> sh; w1[1] = yy.y >> sh;
+      }
+#pragma unroll
+      for (int b = 0; b < 2; b++) {
+        if (b && half) break;
+        const half8_b W = codes8<QT>(w0[b], w1[b], 0, b);
+        const float dh = __half2float(__ushort_as_half((unsigned short)(b ? d[rt] >> 16 : d[rt] & 0xffffu))), dv = b ? -dh : dh;
+        const f32x4_b C = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.h[b], W, zero, 0, 0, 0), D = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.l[b], W, zero, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; i++) { const float f = dv * x.sc[b][i]; Y[rt][i] = fmaf(f, C[i], Y[rt][i]); U[rt][i] = fmaf(f, D[i], U[rt][i]); }
+      }
+    }
+  };
+  for (int c = c0; c < c1; c += P) {
+#pragma unroll
+    for (int i = 0; i < P; i++) {
+      if (c + i >= c1) break;
+      use(r[i], 2 * (c + i) + 1 >= nb32);
+      if (c + i + P < c1) fetch(c + i + P, r[i]);
+      if (((c + i - c0) & 3) == 3)
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++) { Z[rt] += Y[rt]; Y[rt] = zero; }
+    }
+  }
+#pragma unroll
+  for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) sums[wave][rt * 4 + i][lane] = Z[rt][i] + (Y[rt][i] + U[rt][i]);
+  __syncthreads();
+  // lane (n, kg) of a sum: row n of the tile, tokens 4 kg + i
+  const int from = (tl >> 2) * 16 + (tid & 15), v = ((tid >> 4) & 1) * 4 + (tl & 3);
+  float y = 0.0f, gate = 0.0f, inv = 1.0f;
+#pragma unroll
+  for (int w = 0; w < NW; w++) { y += sums[w][v][from]; if (PAIR) gate += sums[w][PAIR ? 8 + v : 0][from]; }
+  if (p.normed) {
+    float ss = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; w++) ss += s_sq[w][tl];
+    inv = 1.0f / sqrtf(ss / (float)K + p.eps);
+  }
+  y = y * inv + bs;
+  if constexpr (PAIR) y = silu_mul(y, gate * inv + bs2);
+  else {
+    y += res;
+    if (t < p.n_tok && row < rows) p.y[at_y] = y;
+  }
+  if (!p.out.hi) return;
+  // (rows in whole blocks of 32: the lanes of a half-wave are one of them)
+  const float x = y * gain;
+  float m = finite_abs(x), ss = y * y;
+#define BS_DPP(z, ctrl) __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, (z)), (ctrl), 0xf, 0xf, false))
+  m = fmaxf(m, BS_DPP(m, 0xb1)); m = fmaxf(m, BS_DPP(m, 0x4e)); m = fmaxf(m, BS_DPP(m, 0x141)); m = fmaxf(m, BS_DPP(m, 0x140));
+  ss += BS_DPP(ss, 0xb1); ss += BS_DPP(ss, 0x4e); ss += BS_DPP(ss, 0x141); ss += BS_DPP(ss, 0x140);
+#undef BS_DPP
+  m = fmaxf(m, __shfl_xor(m, 16)); ss += __shfl_xor(ss, 16);
+  const int e = plane_exponent(m);
+  _Float16 h, l; split_plane(x * ldexpf(1.0f, e), h, l);
+  // (the work-group's results are one block of the planes: it leaves as whole lines; tokens past the end are its padding)
+  const int at = plane_place<QT>(tl, tid & 31);
+  s_out[0][at] = h; s_out[1][at] = l;
+  const int64_t blk = (int64_t)tile * (rows >> 5) + (R0 >> 5);
+  if ((tid & 31) == 0) { p.out.scale[blk * 16 + tl] = ldexpf(1.0f, -e); p.out.squares[blk * 16 + tl] = ss; }
+  __syncthreads();
+  if (wave < 2) reinterpret_cast<u32x4_b*>((wave ? p.out.lo : p.out.hi) + blk * 512)[lane] = reinterpret_cast<const u32x4_b*>(s_out[wave])[lane];
+}
+
+// Float rows times a gain (or as they are) as such planes, with their sums of squares: the stream in front of the first layer, and what the attention leaves.  Eight
+// lanes a block.
+template <int QT>
+__global__ __launch_bounds__(256) void blk_planes_kernel(const float* __restrict__ x, const float* __restrict__ gain, int K, int n4, BlkPlanes o)
+{
+  const int id = blockIdx.x * 256 + threadIdx.x, t = blockIdx.y;
+  if (id >= n4) return;                    // (whole blocks: K is a multiple of 32)
+  const f32x4_b v = *reinterpret_cast<const f32x4_b*>(x + (int64_t)t * K + 4 * id), one = {1.0f, 1.0f, 1.0f, 1.0f}, g = gain ? *reinterpret_cast<const f32x4_b*>(gain + 4 * id) : one;
+  float m = 0.0f, ss = 0.0f, u[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) { u[i] = v[i] * g[i]; m = fmaxf(m, finite_abs(u[i])); ss = fmaf(v[i], v[i], ss); }
+#pragma unroll
+  for (int d = 4; d; d >>= 1) { m = fmaxf(m, __shfl_xor(m, d)); ss += __shfl_xor(ss, d); }
+  const int e = plane_exponent(m);
+  const float s = ldexpf(1.0f, e);
+  typedef _Float16 half4_b __attribute__((ext_vector_type(4)));
+  half4_b h, l;
+#pragma unroll
+  for (int i = 0; i < 4; i++) { _Float16 a, b; split_plane(u[i] * s, a, b); h[i] = a; l[i] = b; }
+  const int64_t blk = (int64_t)(t >> 4) * (K >> 5) + (id >> 3), at = blk * 512 + plane_place<QT>(t & 15, 4 * (id & 7));
+  *reinterpret_cast<half4_b*>(o.hi + at) = h; *reinterpret_cast<half4_b*>(o.lo + at) = l;
+  if ((id & 7) == 0) { o.scale[blk * 16 + (t & 15)] = ldexpf(1.0f, -e); o.squares[blk * 16 + (t & 15)] = ss; }
+}
+
+// ------------------------------------------------------------------------------------------
 // Grouping of a prompt's (token, rank) slots by expert: perm lists the slots expert by expert, tile_tab cuts each expert's
 // run into token tiles of at most `tile` slots.  One work-group; the order of the slots inside an expert's run depends on
 // the arrival of LDS atomics, which does not matter: every result row is computed from its own activation row only.
@@ -772,6 +969,81 @@ int launch_gemm_blk_multi(const cai_qw_s* const* ws, const int* y_off, int n_w, 
   p.x_div = 1; p.expert_rows = 0; p.post = 1.0f; p.n_seg = n_w;
   for (int i = 1; i < n_w; i++) { p.q2[i - 1] = ws[i]->data; p.d2[i - 1] = ws[i]->aux; p.bias2[i - 1] = ws[i]->bias; p.rows2[i - 1] = (int)ws[i]->rows; p.y_off2[i - 1] = y_off[i] - y_off[0]; }
   return launch_blk(w, p, 0);
+}
+
+// Whether the products of a layer go through gemm_blk_short: all of them of one type, in whole blocks of 32 rows where their results become planes, and each
+// of at most two work-groups of 16 tokens x 32 rows a CU.  Beyond that the tiles that share their operands are faster than the launches they
+// need.  Prompts, us, one product after the other | this way: six layers of 2048 / ffn 5632 in Q8_0, 24 tokens (352 work-groups of gate | up) 574 | 550, 64 tokens (704)
+// 684 | 649 .. 728; eight of 1024 / 4096, 64 tokens (512) 610 | 577, 100 (896) 693 | 701; four of 4096 / 14336, 24 tokens (896) 768 | 809; twelve of
+// 576 / 1536, 37 tokens (144) 576 | 525 (Q4_0 653 | 512), 128 (384) 661 | 603.  Up to one work-group a CU registers for three or four chunks a wave, past that for two work-groups:
+// 1024 / 4096, 64 tokens 591 | 577, 24 tokens 501 | 515.
+bool blk_short_wanted(const cai_qw_s* wq, const cai_qw_s* wk, const cai_qw_s* wv, const cai_qw_s* wo, const cai_qw_s* wgu, const cai_qw_s* wd, int n_tok)
+{
+  const cai_qw_s* ws[6] = {wq, wk, wv, wo, wgu, wd};
+  for (const cai_qw_s* w : ws)
+    if (!w || !gemm_blk_supported(w) || w->qtype != wq->qtype || prompt_route(w, n_tok) != 2) return false;
+  if (wo->rows % 32 || wgu->rows % 64 || wd->rows != wo->rows || wd->cols * 2 != wgu->rows || wq->cols != wo->rows || wk->cols != wq->cols || wv->cols != wq->cols || wgu->cols != wo->rows || wo->cols != wq->rows) return false;
+  const int64_t tiles = (n_tok + 15) / 16, most = 2 * ctx().n_cu;
+  return ((wq->rows + 31) / 32 + (wk->rows + 31) / 32 + (wv->rows + 31) / 32) * tiles <= most && wo->rows / 32 * tiles <= most && wd->cols / 32 * tiles <= most;
+}
+
+// y[t][y_off[i] + r] = (W_i x[t])[r] (+ bias_i) (+ residual), or with half > 0 (one matrix of 2 half rows) up * silu(gate), which only out receives; eps >= 0: x is the
+// stream, to be normed; out: planes of the results times a gain, for the next product
+int launch_gemm_blk_short(const cai_qw_s* const* ws, const int* y_off, int n_w, const BlkPlanes& x, float eps, int n_tok, float* y, int64_t y_stride, const float* residual, int half,
+                          const BlkPlanes& out, const float* gain)
+{
+  const cai_qw_s* w = ws[0];
+  if (!gemm_blk_multi_supported(ws, n_w) || (half && (n_w != 1 || !out.hi || w->rows != 2 * (int64_t)half || half % 32)) || (out.hi && (n_w != 1 || w->rows % 32)))
+    return set_error(CAI_ERR_UNSUPPORTED, "short prompt: %d matrices of %lld rows", n_w, (long long)w->rows);
+  BlkShortParams p{};
+  p.cols = (int)w->cols; p.n_tok = n_tok; p.n_tok_tiles = (n_tok + 15) / 16; p.half = half; p.x = x; p.normed = eps >= 0.0f; p.eps = eps;
+  p.y = y; p.y_stride = y_stride; p.residual = residual; p.out = out; p.gain = gain; p.n_seg = n_w;
+  for (int i = 0; i < n_w; i++) { p.q[i] = ws[i]->data; p.d[i] = ws[i]->aux; p.bias[i] = ws[i]->bias; p.rows[i] = half ? half : (int)ws[i]->rows; p.y_off[i] = y_off[i]; }
+  for (int i = 0; i < n_w; i++) { if (i) p.seg_end[i - 1] = p.n_row_groups; p.n_row_groups += (p.rows[i] + 31) / 32; }
+  const dim3 grid(8 * p.n_tok_tiles * ((p.n_row_groups + 7) / 8)), blk(64 * BS_NW);
+  const bool twice = p.n_row_groups * p.n_tok_tiles > ctx().n_cu;
+#define SHORT_T(QT, PAIR) do { if (twice) hipLaunchKernelGGL((gemm_blk_short<QT, PAIR, true>), grid, blk, 0, ctx().stream, p); \
+                               else hipLaunchKernelGGL((gemm_blk_short<QT, PAIR, false>), grid, blk, 0, ctx().stream, p); } while (0)
+#define SHORT(QT) do { if (half) SHORT_T(QT, true); else SHORT_T(QT, false); } while (0)
+  if (w->qtype == CAI_Q8_0) SHORT(CAI_Q8_0); else SHORT(CAI_Q4_0);
+#undef SHORT
+#undef SHORT_T
+  return CAI_OK;
+}
+int launch_blk_planes(const cai_qw_s* w, const float* x, const float* gain, int n_tok, const BlkPlanes& o)      // for products with w
+{
+  const int K = (int)w->cols;
+  const dim3 grid((K / 4 + 255) / 256, n_tok);
+  if (w->qtype == CAI_Q8_0) hipLaunchKernelGGL(blk_planes_kernel<CAI_Q8_0>, grid, dim3(256), 0, ctx().stream, x, gain, K, K / 4, o);
+  else hipLaunchKernelGGL(blk_planes_kernel<CAI_Q4_0>, grid, dim3(256), 0, ctx().stream, x, gain, K, K / 4, o);
+  return CAI_OK;
+}
+
+// Two sets of planes, of whole tiles of 16 tokens; grown, never inside a capture (prompts are not captured)
+struct ShortWs { BlkPlanes p[2]; size_t cap[2] = {0, 0}; };
+static ShortWs g_short;
+void blk_short_release()
+{
+  for (BlkPlanes& b : g_short.p) { void* q[] = {b.hi, b.lo, b.scale, b.squares}; for (void* v : q) if (v) (void)hipFree(v); }
+  g_short = ShortWs();
+}
+int blk_short_planes(int n_tok, int width0, int width1, BlkPlanes (&out)[2])
+{
+  const size_t tok = (size_t)(n_tok + 15) / 16 * 16, need[2] = {tok * width0, tok * width1};
+  for (int i = 0; i < 2; i++) {
+    if (need[i] > g_short.cap[i]) {
+      CAI_HIP(hipStreamSynchronize(ctx().stream));
+      BlkPlanes& b = g_short.p[i];
+      void* q[] = {b.hi, b.lo, b.scale, b.squares};
+      for (void* v : q) if (v) (void)hipFree(v);
+      b = BlkPlanes(); g_short.cap[i] = 0;
+      const size_t n = std::max(need[i], (size_t)128 * (i ? width1 : width0));
+      CAI_HIP(hipMalloc((void**)&b.hi, n * 2)); CAI_HIP(hipMalloc((void**)&b.lo, n * 2)); CAI_HIP(hipMalloc((void**)&b.scale, n / 8)); CAI_HIP(hipMalloc((void**)&b.squares, n / 8));
+      g_short.cap[i] = n;
+    }
+    out[i] = g_short.p[i];
+  }
+  return CAI_OK;
 }
 
 bool gemm_raw_supported(const cai_qw_s* w)

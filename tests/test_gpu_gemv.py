@@ -484,6 +484,36 @@ def test_prompt_of_a_decoder_on_wide_tiles(qt):
     dec.close()
 
 
+# one block of width and of ffn, odd numbers of blocks, k and v rows that are no whole 32, tiles of 16 tokens (whole, one token over), one work-group a CU
+# (the last but one refills its rings of four chunks a wave), two (the last two: gate | up alone, all but the ends, rings refilled)
+@pytest.mark.parametrize("qt", [O.Q8_0, O.Q4_0])
+@pytest.mark.parametrize("d,ffn,hq,hkv,hd,T", [(32, 32, 1, 1, 32, 9), (64, 96, 2, 1, 32, 17), (96, 160, 6, 3, 16, 16), (96, 1120, 6, 3, 16, 33), (1056, 2144, 8, 2, 64, 12), (1600, 320, 8, 2, 64, 9),
+                                             (576, 1536, 9, 3, 64, 90), (1088, 1120, 9, 3, 128, 125)])
+def test_short_prompts_whose_activations_stay_planes(qt, d, ffn, hq, hkv, hd, T):
+    """A prompt equals its tokens one by one, with gains and biases everywhere.  Both sides are 32-bit sums over activations of 22 bits: 4e-7 from 64 bits a layer
+    (2e-6 of the largest logit where a layer's rounding is carried on), so 1e-5 apart at most."""
+    from helpers.device import dev, rel_err
+    from helpers.model_build import synthetic_spec
+    cai = dev()
+    cfg = dict(n_layers=3, d_model=d, n_q_heads=hq, n_kv_heads=hkv, head_dim=hd, ffn=ffn, vocab=300, max_ctx=128, eps=1e-5, rope_theta=1e4)
+    spec = synthetic_spec(cfg, qt, head_qtype=O.Q8_0, seed=d + T, std=0.05, qkv_bias=True)
+    rng = np.random.default_rng(T)
+    for key in spec["vecs"]:
+        spec["vecs"][key] = (1.0 + 0.3 * rng.standard_normal(spec["vecs"][key].size)).astype(np.float32)
+    for l in range(cfg["n_layers"]):
+        for slot, n in ((O.W_O, d), (O.W_GATEUP, 2 * ffn), (O.W_DOWN, d)):
+            spec["tensors"][(l, slot)]["bias"] = (0.1 * rng.standard_normal(n)).astype(np.float32)
+    dec = cai.Decoder(spec, max_batch=2)
+    tok = rng.integers(0, 300, T).astype(np.int32)
+    _, got = dec.prefill(tok)
+    for p_, t in enumerate(tok):
+        _, want = dec.step_window([t], p_, seq=1)
+    assert rel_err(got, want[0]) < 1e-5
+    after = dec.step(np.array([7, 7], np.int32), np.array([T, T], np.int32))[1]      # (from the cached rows of either)
+    assert rel_err(after[0], after[1]) < 1e-5
+    dec.close()
+
+
 @pytest.mark.parametrize("qt,ffn,T", [(O.Q8_0, 352, 100), (O.Q4_0, 64, 40), (O.Q8_0, 320, 150)])
 def test_prompt_of_a_mixture_on_tiles_of_64_slots(qt, ffn, T):
     """banks of four experts, two a token: runs of about T / 2 slots in tiles of 64 (full, half empty, a remainder), widths of an odd and an
