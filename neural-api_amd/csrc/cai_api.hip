@@ -77,10 +77,18 @@ int ensure_host_stage(size_t need)
 // few words of the arg-max.  Here kernels write pieces into pinned memory behind the step, with an event after each, and the host copies
 // piece i on while i + 1 crosses.
 // ------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void words_copy_kernel(const uint32_t* src, uint32_t* dst, size_t words)
+// A launch copies up to WORDS_SEGS runs of words, 16 KB a work-group: the arg-max leaves with the logits (by itself it was another launch, 2.6 to 3.9 us
+// of kernel time at the end of every call).
+constexpr int WORDS_SEGS = 4;
+struct WordsCopy { const uint32_t* src[WORDS_SEGS]; uint32_t* dst[WORDS_SEGS]; size_t words[WORDS_SEGS]; unsigned end[WORDS_SEGS]; };      // end: first work-group behind a run's
+__global__ __launch_bounds__(256) void words_copy_kernel(const WordsCopy c)
 {
   typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-  const size_t i = (size_t)blockIdx.x * 4096 + threadIdx.x * 4;   // 16 KB a work-group
+  const uint32_t* src = c.src[0]; uint32_t* dst = c.dst[0]; size_t words = c.words[0]; unsigned first = 0;
+#pragma unroll
+  for (int s = 1; s < WORDS_SEGS; s++)
+    if (blockIdx.x >= c.end[s - 1]) { src = c.src[s]; dst = c.dst[s]; words = c.words[s]; first = c.end[s - 1]; }
+  const size_t i = (size_t)(blockIdx.x - first) * 4096 + threadIdx.x * 4;
   if ((((uintptr_t)src | (uintptr_t)dst) & 15) == 0) {
     u4 v[4];
 #pragma unroll
@@ -93,14 +101,28 @@ __global__ __launch_bounds__(256) void words_copy_kernel(const uint32_t* src, ui
     }
   } else {
     for (int k = 0; k < 16; k++) {
-      const size_t j = (size_t)blockIdx.x * 4096 + k * 256 + threadIdx.x;
+      const size_t j = (size_t)(blockIdx.x - first) * 4096 + k * 256 + threadIdx.x;
       if (j < words) dst[j] = src[j];
     }
   }
 }
+static void words_copy_add(WordsCopy& c, int& n, const void* src, void* dst, size_t words)
+{
+  c.src[n] = (const uint32_t*)src; c.dst[n] = (uint32_t*)dst; c.words[n] = words;
+  const unsigned end = (n ? c.end[n - 1] : 0) + (unsigned)((words + 4095) / 4096);
+  for (int s = n; s < WORDS_SEGS; s++) c.end[s] = end;
+  n++;
+}
+static void words_copy_go(WordsCopy& c, int& n)
+{
+  if (n) hipLaunchKernelGGL(words_copy_kernel, dim3(c.end[n - 1]), dim3(256), 0, g_ctx.stream, c);
+  c = WordsCopy(); n = 0;
+}
 void launch_words_copy(const void* src, void* dst, int words)
 {
-  hipLaunchKernelGGL(words_copy_kernel, dim3((words + 4095) / 4096), dim3(256), 0, g_ctx.stream, (const uint32_t*)src, (uint32_t*)dst, (size_t)words);
+  WordsCopy c{}; int n = 0;
+  words_copy_add(c, n, src, dst, (size_t)words);
+  words_copy_go(c, n);
 }
 
 int fetch_to_host(const HostCopy* c, int n)
@@ -124,16 +146,20 @@ int fetch_to_host(const HostCopy* c, int n)
   std::vector<Part> parts;
   char* h = (char*)g_ctx.h_stage;
   size_t open = 0;        // bytes behind the last event
-  int ev = 0;
+  int ev = 0, n_run = 0;
+  WordsCopy run{};
   for (int k = 0; k < n; k++) {
     for (size_t b = 0; b < c[k].bytes;) {
       const size_t m = std::min(c[k].bytes - b, piece - open);
-      hipLaunchKernelGGL(words_copy_kernel, dim3((unsigned)((m / 4 + 4095) / 4096)), dim3(256), 0, st, (const uint32_t*)((const char*)c[k].src + b), (uint32_t*)h, m / 4);
+      words_copy_add(run, n_run, (const char*)c[k].src + b, h, m / 4);
       parts.push_back({(char*)c[k].dst + b, h, m, ev});
       b += m; h += pad(m); open += pad(m);
-      if (open >= piece && ev + 1 < N_EV) { CAI_HIP(hipEventRecord(g_ctx.piece_ev[ev++], st)); open = 0; }
+      const bool full = open >= piece && ev + 1 < N_EV;
+      if (full || n_run == WORDS_SEGS) words_copy_go(run, n_run);
+      if (full) { CAI_HIP(hipEventRecord(g_ctx.piece_ev[ev++], st)); open = 0; }
     }
   }
+  words_copy_go(run, n_run);
   CAI_HIP(hipGetLastError());
   int seen = 0;           // events waited for
   for (const Part& p : parts) {
