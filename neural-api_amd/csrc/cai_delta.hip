@@ -12,11 +12,13 @@ namespace cai {
 // ------------------------------------------------------------------------------------------
 // prompt pass 1: q and k unit vectors (q scaled), v, decay, write strength, q . k.
 // A wave owns one unit - the q and k channels of a key head, 256 channels of v, 256 decays, the write strengths - over eight
-// consecutive rows; the convolution slides over them, so each input is fetched once (TAPS = 4; other lengths look back per row).
+// consecutive rows; the convolution slides over them, so each input is fetched once (TAPS = 4; other lengths look back per row).  Where the eight rows
+// are of one portion, all of them are requested before the first is convolved: row by row it was eight round trips (2048 rows of 8 + 16 heads of 128:
+// 29 us, now 22).
 // ------------------------------------------------------------------------------------------
 constexpr int PREP_ROWS = 8;
 
-template <int TAPS>
+template <int TAPS, int ND>                // ND: runs of 64 channels of a key head
 __global__ __launch_bounds__(256) void delta_prep_kernel(const DeltaDims d, const DeltaIn in, const DeltaW w, const float* hist, const int64_t h_elems, const StepRows r, const DeltaBuf b)
 {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -25,10 +27,48 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(const DeltaDims d, cons
   const int gw = d.channel_decay ? d.heads * d.dim : d.heads;
   const int nv = (vw + 255) / 256, ng = (gw + 255) / 256;
   int unit = blockIdx.y * 4 + wave;
+  const bool one = TAPS && r1 - r0 == PREP_ROWS && r.first[r0] == r.first[r1 - 1];
   if (unit < d.kv_heads) {
     const int g = unit, c0 = g * d.dim;
     const float qs = rsqrtf((float)d.dim);
     ConvWindow<TAPS ? TAPS : 2> wq, wk;
+    // unit vectors and their product from a row's convolved channels
+    auto finish = [&](int row, const float (&q)[4], const float (&k)[4]) {
+      float sq = 0.0f, sk = 0.0f, dot = 0.0f;
+#pragma unroll
+      for (int i = 0; i < ND; i++) { sq = fmaf(q[i], q[i], sq); sk = fmaf(k[i], k[i], sk); dot = fmaf(q[i], k[i], dot); }
+      const float nq = qs / sqrtf(wave_total(sq) + 1e-6f), nk = 1.0f / sqrtf(wave_total(sk) + 1e-6f);
+      dot = wave_total(dot) * nq * nk;
+#pragma unroll
+      for (int i = 0; i < ND; i++) {
+        const int c = lane + 64 * i;
+        if (c < d.dim) { b.q[(int64_t)row * kw + c0 + c] = q[i] * nq; b.k[(int64_t)row * kw + c0 + c] = k[i] * nk; }
+      }
+      if (lane == 0) b.beta[(int64_t)row * bw + d.heads + g] = dot;
+    };
+    if constexpr (TAPS != 0) {
+      if (one) {
+        float qi[PREP_ROWS][ND], ki[PREP_ROWS][ND];
+        const float* const p0 = in.proj + r0 * in.ldp + c0;
+#pragma unroll
+        for (int u = 0; u < PREP_ROWS; u++)
+#pragma unroll
+          for (int i = 0; i < ND; i++) { const int c = min(lane + 64 * i, d.dim - 1); qi[u][i] = p0[u * in.ldp + in.oq + c]; ki[u][i] = p0[u * in.ldp + in.ok + c]; }
+        const int pos = r.pos[r0], back = r0 - r.first[r0];
+        const float* const ring = hist + r.slot[r0] * h_elems;
+        wq.taps(w.cq, c0, lane, d.dim); wk.taps(w.ck, c0, lane, d.dim);
+        wq.history(in.proj + r0 * in.ldp + in.oq, in.ldp, back, pos, ring, C, 0, c0, lane, d.dim);
+        wk.history(in.proj + r0 * in.ldp + in.ok, in.ldp, back, pos, ring, C, kw, c0, lane, d.dim);
+#pragma unroll
+        for (int u = 0; u < PREP_ROWS; u++) {
+          float q[4], k[4];
+#pragma unroll
+          for (int i = 0; i < ND; i++) { const bool in_head = lane + 64 * i < d.dim; q[i] = wq.step(i, in_head ? qi[u][i] : 0.0f); k[i] = wk.step(i, in_head ? ki[u][i] : 0.0f); }
+          finish(r0 + u, q, k);
+        }
+        return;
+      }
+    }
     if (TAPS) { wq.taps(w.cq, c0, lane, d.dim); wk.taps(w.ck, c0, lane, d.dim); }
     for (int row = r0; row < r1; row++) {
       const int pos = r.pos[row], back = row - r.first[row];
@@ -38,28 +78,19 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(const DeltaDims d, cons
         wq.history(p + in.oq, in.ldp, back, pos, ring, C, 0, c0, lane, d.dim);
         wk.history(p + in.ok, in.ldp, back, pos, ring, C, kw, c0, lane, d.dim);
       }
-      float q[4], k[4], sq = 0.0f, sk = 0.0f, dot = 0.0f;
+      float q[4], k[4];
 #pragma unroll
-      for (int i = 0; i < 4; i++) { const int c = lane + 64 * i; q[i] = c < d.dim ? p[in.oq + c0 + c] : 0.0f; k[i] = c < d.dim ? p[in.ok + c0 + c] : 0.0f; }
+      for (int i = 0; i < ND; i++) { const int c = lane + 64 * i; q[i] = c < d.dim ? p[in.oq + c0 + c] : 0.0f; k[i] = c < d.dim ? p[in.ok + c0 + c] : 0.0f; }
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
+      for (int i = 0; i < ND; i++) {
         const int c = lane + 64 * i;
-        if (i * 64 >= d.dim) continue;
         if (TAPS) { q[i] = wq.step(i, q[i]); k[i] = wk.step(i, k[i]); }
         else if (c < d.dim) {
           q[i] = conv_silu(p + in.oq, in.ldp, back, pos, ring, C, 0, w.cq, d.taps, c0 + c);
           k[i] = conv_silu(p + in.ok, in.ldp, back, pos, ring, C, kw, w.ck, d.taps, c0 + c);
         }
-        sq = fmaf(q[i], q[i], sq); sk = fmaf(k[i], k[i], sk); dot = fmaf(q[i], k[i], dot);
       }
-      const float nq = qs / sqrtf(wave_total(sq) + 1e-6f), nk = 1.0f / sqrtf(wave_total(sk) + 1e-6f);
-      dot = wave_total(dot) * nq * nk;
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int c = lane + 64 * i;
-        if (c < d.dim) { b.q[(int64_t)row * kw + c0 + c] = q[i] * nq; b.k[(int64_t)row * kw + c0 + c] = k[i] * nk; }
-      }
-      if (lane == 0) b.beta[(int64_t)row * bw + d.heads + g] = dot;
+      finish(row, q, k);
     }
     return;
   }
@@ -67,6 +98,28 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(const DeltaDims d, cons
   if (unit < nv) {
     const int c0 = unit * 256, n = min(256, vw - c0);
     ConvWindow<TAPS ? TAPS : 2> wv;
+    if constexpr (TAPS != 0) {
+      if (one) {
+        float vi[PREP_ROWS][4];
+        const float* const p0 = in.proj + r0 * in.ldp + in.ov;
+#pragma unroll
+        for (int u = 0; u < PREP_ROWS; u++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) vi[u][i] = p0[u * in.ldp + c0 + min(lane + 64 * i, n - 1)];
+        const int pos = r.pos[r0], back = r0 - r.first[r0];
+        wv.taps(w.cv, c0, lane, n);
+        wv.history(p0, in.ldp, back, pos, hist + r.slot[r0] * h_elems, C, 2 * kw, c0, lane, n);
+#pragma unroll
+        for (int u = 0; u < PREP_ROWS; u++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const int c = lane + 64 * i;
+            const float v = wv.step(i, c < n ? vi[u][i] : 0.0f);
+            if (c < n) b.v[(int64_t)(r0 + u) * vw + c0 + c] = v;
+          }
+        return;
+      }
+    }
     if (TAPS) wv.taps(w.cv, c0, lane, n);
     for (int row = r0; row < r1; row++) {
       const int pos = r.pos[row], back = row - r.first[row];
@@ -541,28 +594,40 @@ __global__ __launch_bounds__(64 * (NW + 1)) void delta_walk_kernel(const DeltaDi
 // ------------------------------------------------------------------------------------------
 // prompt pass 3: per row and head RMS norm, gain, gate; then the row's raw inputs into the ring if the portion's last taps reach it
 // ------------------------------------------------------------------------------------------
-template <typename AT>
+template <typename AT, int NV>             // NV: runs of 64 columns of a head
 __global__ __launch_bounds__(256) void delta_finish_kernel(const DeltaDims d, const DeltaIn in, const DeltaW w, float* hist, const int64_t h_elems, const StepRows r, const DeltaBuf b, AT* out, const int64_t ldo)
 {
   const int row = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int vw = d.heads * d.vdim;
   const float* p = in.proj + row * in.ldp;
   const float* gate = d.rank_g ? b.zg + (int64_t)row * vw : p + in.og;
-  for (int h = wave; h < d.heads; h += 4) {
-    float o[4], s = 0.0f;
+  // four heads of a wave requested together (heads past the last one: that again, not written)
+  constexpr int AT_ONCE = 4;
+  for (int h0 = wave; h0 < d.heads; h0 += 4 * AT_ONCE) {
+    float o[AT_ONCE][NV], z[AT_ONCE][NV], gain[NV];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int c = lane + 64 * i;
-      o[i] = c < d.vdim ? b.o[(int64_t)row * vw + h * d.vdim + c] : 0.0f;
-      s = fmaf(o[i], o[i], s);
-    }
-    const float inv = 1.0f / sqrtf(wave_total(s) / (float)d.vdim + d.eps);
+    for (int k = 0; k < AT_ONCE; k++)
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int c = lane + 64 * i;
-      if (c < d.vdim) {
-        const float z = gate[h * d.vdim + c], sg = sigmoid_f(z);
-        out[row * ldo + h * d.vdim + c] = (AT)(o[i] * inv * w.norm[c] * (d.sigmoid_gate ? sg : z * sg));
+      for (int i = 0; i < NV; i++) {
+        const int at = min(h0 + 4 * k, d.heads - 1) * d.vdim + min(lane + 64 * i, d.vdim - 1);
+        o[k][i] = b.o[(int64_t)row * vw + at]; z[k][i] = gate[at];
+      }
+#pragma unroll
+    for (int i = 0; i < NV; i++) gain[i] = w.norm[min(lane + 64 * i, d.vdim - 1)];
+#pragma unroll
+    for (int k = 0; k < AT_ONCE; k++) {
+      const int h = h0 + 4 * k;
+      if (h >= d.heads) break;
+      float s = 0.0f;
+#pragma unroll
+      for (int i = 0; i < NV; i++) if (lane + 64 * i < d.vdim) s = fmaf(o[k][i], o[k][i], s);
+      const float inv = 1.0f / sqrtf(wave_total(s) / (float)d.vdim + d.eps);
+#pragma unroll
+      for (int i = 0; i < NV; i++) {
+        const int c = lane + 64 * i;
+        if (c >= d.vdim) continue;
+        const float sg = sigmoid_f(z[k][i]);
+        out[row * ldo + h * d.vdim + c] = (AT)(o[k][i] * inv * gain[i] * (d.sigmoid_gate ? sg : z[k][i] * sg));
       }
     }
   }
@@ -725,8 +790,11 @@ int delta_prep(const DeltaDims& d, const DeltaIn& in, const DeltaW& w, const Seq
   const int gw = d.channel_decay ? d.heads * d.dim : d.heads;
   const int units = d.kv_heads + (d.heads * d.vdim + 255) / 256 + (gw + 255) / 256 + 1;
   const dim3 grid((r.n_rows + PREP_ROWS - 1) / PREP_ROWS, (units + 3) / 4);
-  if (d.taps == 4) hipLaunchKernelGGL(delta_prep_kernel<4>, grid, dim3(256), 0, ctx().stream, d, in, w, st.hist, st.h_elems, r, b);
-  else hipLaunchKernelGGL(delta_prep_kernel<0>, grid, dim3(256), 0, ctx().stream, d, in, w, st.hist, st.h_elems, r, b);
+#define PREP(TAPS, ND) hipLaunchKernelGGL((delta_prep_kernel<TAPS, ND>), grid, dim3(256), 0, ctx().stream, d, in, w, st.hist, st.h_elems, r, b)
+#define PREP_N(TAPS) do { if (d.dim <= 64) PREP(TAPS, 1); else if (d.dim <= 128) PREP(TAPS, 2); else PREP(TAPS, 4); } while (0)
+  if (d.taps == 4) PREP_N(4); else PREP_N(0);
+#undef PREP_N
+#undef PREP
   CAI_HIP(hipGetLastError());
   return CAI_OK;
 }
@@ -762,8 +830,11 @@ int delta_chunked(const DeltaDims& d, const SeqPool::StateRun& st, const StepRow
 
 int delta_finish(const DeltaDims& d, const DeltaIn& in, const DeltaW& w, const SeqPool::StateRun& st, const StepRows& r, const DeltaBuf& b, int act_t, void* out, int64_t ldo)
 {
-  if (act_t == ACT_T_BF16) hipLaunchKernelGGL(delta_finish_kernel<bf16_t>, dim3(r.n_rows), dim3(256), 0, ctx().stream, d, in, w, st.hist, st.h_elems, r, b, (bf16_t*)out, ldo);
-  else hipLaunchKernelGGL(delta_finish_kernel<float>, dim3(r.n_rows), dim3(256), 0, ctx().stream, d, in, w, st.hist, st.h_elems, r, b, (float*)out, ldo);
+#define FINISH(AT, NV) hipLaunchKernelGGL((delta_finish_kernel<AT, NV>), dim3(r.n_rows), dim3(256), 0, ctx().stream, d, in, w, st.hist, st.h_elems, r, b, (AT*)out, ldo)
+#define FINISH_N(AT) do { if (d.vdim <= 64) FINISH(AT, 1); else if (d.vdim <= 128) FINISH(AT, 2); else FINISH(AT, 4); } while (0)
+  if (act_t == ACT_T_BF16) FINISH_N(bf16_t); else FINISH_N(float);
+#undef FINISH_N
+#undef FINISH
   CAI_HIP(hipGetLastError());
   return CAI_OK;
 }

@@ -13,10 +13,10 @@ __device__ __forceinline__ float wave_total(float v)   // the sum in every lane
   v = wave_sum(v);
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
-__device__ __forceinline__ float sigmoid_f(float z)
+__device__ __forceinline__ float sigmoid_f(float z)    // (one exponential and one division whatever the lanes' signs)
 {
-  if (z >= 0.0f) return 1.0f / (1.0f + expf(-z));
-  const float s = expf(z); return s / (1.0f + s);
+  const float e = expf(-fabsf(z));
+  return (z >= 0.0f ? 1.0f : e) / (1.0f + e);
 }
 __device__ __forceinline__ float softplus_f(float z) { return fmaxf(z, 0.0f) + log1pf(expf(-fabsf(z))); }
 template <int CTRL> __device__ __forceinline__ float dpp_add(float v)

@@ -185,9 +185,9 @@ def test_mechanism_alone(cai, tmp_path, mech, i, dt):
 def test_chunks_of_a_portion(cai, tmp_path, mech, h, g, d, dv, n):
     mixer = B.delta(h, g, d, dv, 4)
     m = Model(tmp_path, B.config([B.layer(mixer if mech == "delta" else (B.attn(), mixer))], width=72, vocab=67), seed=n, edit=only(mech), rank_a=9, rank_g=20)
-    tok = m.tokens(n + 5, d)
+    tok = m.tokens(n + 13, d)              # (the second portion: eight rows together behind what the ring holds, and five one by one)
     dec = m.open(cai, 192, 1, "f32")
-    check(feed(dec, tok, [n, 5]), m.ref(tok), "f32")
+    check(feed(dec, tok, [n, 13]), m.ref(tok), "f32")
     dec.close()
 
 
