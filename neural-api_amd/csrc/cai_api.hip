@@ -5,6 +5,8 @@
 #include <string.h>
 #include <mutex>
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 
 namespace cai {
 
@@ -66,7 +68,7 @@ int ensure_host_stage(size_t need)
   CAI_HIP(hipStreamSynchronize(g_ctx.stream));
   if (g_ctx.h_stage) { (void)hipHostFree(g_ctx.h_stage); g_ctx.h_stage = nullptr; g_ctx.h_stage_cap = 0; }
   const size_t want = need < (1u << 20) ? (1u << 20) : need;
-  CAI_HIP(hipHostMalloc(&g_ctx.h_stage, want, hipHostMallocDefault));
+  CAI_HIP(hipHostMalloc(&g_ctx.h_stage, want, hipHostMallocCoherent));
   g_ctx.h_stage_cap = want;
   return CAI_OK;
 }
@@ -74,37 +76,58 @@ int ensure_host_stage(size_t need)
 // ------------------------------------------------------------------------------------------
 // Results on their way to the caller's memory, which is pageable: hipMemcpyAsync into it waits for the stream, copies at most a MB at a time
 // into pinned memory of the runtime's, waits, and copies on, so that PCIe and the host's copy never overlap, and does all of it again for the
-// few words of the arg-max.  Here kernels write pieces into pinned memory behind the step, with an event after each, and the host copies
+// few words of the arg-max.  Here kernels write pieces into pinned memory behind the step, with a signal after each, and the host copies
 // piece i on while i + 1 crosses.
 // ------------------------------------------------------------------------------------------
+HostSignal host_signal_next(int k)
+{
+  if (k == 0) g_ctx.signals++;
+  return HostSignal{g_ctx.h_flags + 16 * k, g_ctx.d_arrive, g_ctx.signals};
+}
+int host_signal_wait(const HostSignal& s)
+{
+  volatile const uint32_t* const flag = s.flag;
+  const auto t0 = std::chrono::steady_clock::now();
+  for (int i = 1; *flag != s.value; i++) {
+    __builtin_ia32_pause();
+    if ((i & 255) || std::chrono::steady_clock::now() - t0 < std::chrono::milliseconds(50)) continue;
+    CAI_HIP(hipStreamSynchronize(g_ctx.stream));
+    if (*flag != s.value) return set_error(CAI_ERR_HIP, "the stream ended without the signal of its last launch");
+  }
+  std::atomic_thread_fence(std::memory_order_acquire);
+  return CAI_OK;
+}
+__global__ void host_signal_kernel(const HostSignal s) { host_signal(s, 1); }
+void launch_host_signal(const HostSignal& s) { hipLaunchKernelGGL(host_signal_kernel, dim3(1), dim3(64), 0, g_ctx.stream, s); }
+
 // A launch copies up to WORDS_SEGS runs of words, 16 KB a work-group: the arg-max leaves with the logits (by itself it was another launch, 2.6 to 3.9 us
 // of kernel time at the end of every call).
 constexpr int WORDS_SEGS = 4;
-struct WordsCopy { const uint32_t* src[WORDS_SEGS]; uint32_t* dst[WORDS_SEGS]; size_t words[WORDS_SEGS]; unsigned end[WORDS_SEGS]; };      // end: first work-group behind a run's
+struct WordsCopy { const uint32_t* src[WORDS_SEGS]; uint32_t* dst[WORDS_SEGS]; size_t words[WORDS_SEGS]; unsigned end[WORDS_SEGS]; HostSignal done; };      // end: first work-group behind a run's
 __global__ __launch_bounds__(256) void words_copy_kernel(const WordsCopy c)
 {
-  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
   const uint32_t* src = c.src[0]; uint32_t* dst = c.dst[0]; size_t words = c.words[0]; unsigned first = 0;
 #pragma unroll
   for (int s = 1; s < WORDS_SEGS; s++)
     if (blockIdx.x >= c.end[s - 1]) { src = c.src[s]; dst = c.dst[s]; words = c.words[s]; first = c.end[s - 1]; }
-  const size_t i = (size_t)(blockIdx.x - first) * 4096 + threadIdx.x * 4;
-  if ((((uintptr_t)src | (uintptr_t)dst) & 15) == 0) {
-    u4 v[4];
+  const size_t base = (size_t)(blockIdx.x - first) * 4096;
+  if ((((uintptr_t)src | (uintptr_t)dst) & 7) == 0) {
+    uint64_t v[8];
 #pragma unroll
-    for (int k = 0; k < 4; k++) if (i + k * 1024 + 4 <= words) v[k] = *reinterpret_cast<const u4*>(src + i + k * 1024);
+    for (int k = 0; k < 8; k++) { const size_t j = base + 512 * k + 2 * threadIdx.x; if (j + 2 <= words) v[k] = *reinterpret_cast<const uint64_t*>(src + j); }
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-      const size_t j = i + k * 1024;
-      if (j + 4 <= words) *reinterpret_cast<u4*>(dst + j) = v[k];
-      else for (size_t t = j; t < words; t++) dst[t] = src[t];
+    for (int k = 0; k < 8; k++) {
+      const size_t j = base + 512 * k + 2 * threadIdx.x;
+      if (j + 2 <= words) host_store(reinterpret_cast<uint64_t*>(dst + j), v[k]);
+      else if (j < words) host_store(dst + j, src[j]);
     }
   } else {
     for (int k = 0; k < 16; k++) {
-      const size_t j = (size_t)(blockIdx.x - first) * 4096 + k * 256 + threadIdx.x;
-      if (j < words) dst[j] = src[j];
+      const size_t j = base + k * 256 + threadIdx.x;
+      if (j < words) host_store(dst + j, src[j]);
     }
   }
+  host_signal(c.done, gridDim.x);
 }
 static void words_copy_add(WordsCopy& c, int& n, const void* src, void* dst, size_t words)
 {
@@ -113,8 +136,9 @@ static void words_copy_add(WordsCopy& c, int& n, const void* src, void* dst, siz
   for (int s = n; s < WORDS_SEGS; s++) c.end[s] = end;
   n++;
 }
-static void words_copy_go(WordsCopy& c, int& n)
+static void words_copy_go(WordsCopy& c, int& n, const HostSignal& done = HostSignal())
 {
+  c.done = done;
   if (n) hipLaunchKernelGGL(words_copy_kernel, dim3(c.end[n - 1]), dim3(256), 0, g_ctx.stream, c);
   c = WordsCopy(); n = 0;
 }
@@ -129,45 +153,42 @@ int fetch_to_host(const HostCopy* c, int n)
 {
   // staged up to 8 MB (eight rows of 152k logits are 4.9), as up to eight pieces; more (a prompt whose every row was asked for) as the runtime does it
   constexpr size_t MOST = 8u << 20, ONE_PIECE = 1u << 20;
-  constexpr int N_EV = (int)(sizeof(g_ctx.piece_ev) / sizeof(g_ctx.piece_ev[0]));
   auto pad = [](size_t b) { return (b + 15) / 16 * 16; };
   size_t total = 0;
   for (int k = 0; k < n; k++) total += pad(c[k].bytes);
   const hipStream_t st = g_ctx.stream;
-  if (total > MOST) {
+  if (total > MOST || total == 0) {
     for (int k = 0; k < n; k++) if (c[k].bytes) CAI_HIP(hipMemcpyAsync(c[k].dst, c[k].src, c[k].bytes, hipMemcpyDeviceToHost, st));
     CAI_HIP(hipStreamSynchronize(st));
     return CAI_OK;
   }
   int rc = ensure_host_stage(total); if (rc) return rc;
   // (eight rows of 152064: 311 us of a 3367 us step through the runtime, 187 in eight pieces, 220 to 250 in three to five; one row: 33 whole, 38 in three)
-  const size_t piece = total <= ONE_PIECE ? std::max<size_t>(total, 16) : pad(total / N_EV);
-  struct Part { char* dst; const char* src; size_t bytes; int ev; };
+  const size_t piece = total <= ONE_PIECE ? std::max<size_t>(total, 16) : pad(total / HOST_SIGNALS);
+  struct Part { char* dst; const char* src; size_t bytes; int piece; };
   std::vector<Part> parts;
+  HostSignal done[HOST_SIGNALS];
   char* h = (char*)g_ctx.h_stage;
-  size_t open = 0;        // bytes behind the last event
-  int ev = 0, n_run = 0;
+  size_t open = 0, left = total;        // bytes of the piece in hand, bytes without a launch
+  int at = 0, n_run = 0;
   WordsCopy run{};
   for (int k = 0; k < n; k++) {
     for (size_t b = 0; b < c[k].bytes;) {
-      const size_t m = std::min(c[k].bytes - b, piece - open);
+      const bool last = at + 1 == HOST_SIGNALS;
+      const size_t m = last ? c[k].bytes - b : std::min(c[k].bytes - b, piece - open);
       words_copy_add(run, n_run, (const char*)c[k].src + b, h, m / 4);
-      parts.push_back({(char*)c[k].dst + b, h, m, ev});
-      b += m; h += pad(m); open += pad(m);
-      const bool full = open >= piece && ev + 1 < N_EV;
-      if (full || n_run == WORDS_SEGS) words_copy_go(run, n_run);
-      if (full) { CAI_HIP(hipEventRecord(g_ctx.piece_ev[ev++], st)); open = 0; }
+      parts.push_back({(char*)c[k].dst + b, h, m, at});
+      b += m; h += pad(m); open += pad(m); left -= std::min(left, pad(m));
+      if (left == 0 || (!last && open >= piece)) { done[at] = host_signal_next(at); words_copy_go(run, n_run, done[at]); at++; open = 0; }
+      else if (n_run == WORDS_SEGS) words_copy_go(run, n_run);
     }
   }
-  words_copy_go(run, n_run);
   CAI_HIP(hipGetLastError());
-  int seen = 0;           // events waited for
+  int seen = -1;          // the last piece that is there
   for (const Part& p : parts) {
-    if (p.ev < ev) { for (; seen <= p.ev; seen++) CAI_HIP(hipEventSynchronize(g_ctx.piece_ev[seen])); }
-    else if (seen <= ev) { CAI_HIP(hipStreamSynchronize(st)); seen = ev + 1; }
+    if (p.piece > seen) { rc = host_signal_wait(done[p.piece]); if (rc) return rc; seen = p.piece; }
     memcpy(p.dst, p.src, p.bytes);
   }
-  if (seen <= ev) CAI_HIP(hipStreamSynchronize(st));
   return CAI_OK;
 }
 
@@ -210,7 +231,9 @@ extern "C" int cai_init(int device_ordinal)
   CAI_HIP(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
   CAI_HIP(hipEventCreate(&c.ev0));
   CAI_HIP(hipEventCreate(&c.ev1));
-  for (hipEvent_t& e : c.piece_ev) CAI_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  CAI_HIP(hipMalloc(&c.d_arrive, 64)); CAI_HIP(hipMemset(c.d_arrive, 0, 64));
+  CAI_HIP(hipHostMalloc(&c.h_flags, HOST_SIGNALS * 64, hipHostMallocCoherent));
+  memset(c.h_flags, 0, HOST_SIGNALS * 64);
   CAI_HIP(hipMalloc(&c.d_small, 1024 * sizeof(int32_t)));
   CAI_HIP(hipHostMalloc(&c.h_small, 1024 * sizeof(int32_t), hipHostMallocDefault));
   { const int rc = noalloc_setup(device_ordinal); if (rc) return rc; }
@@ -233,7 +256,8 @@ extern "C" int cai_shutdown(void)
   if (c.h_stage) (void)hipHostFree(c.h_stage);
   if (c.tl.buf) (void)hipFree(c.tl.buf);
   (void)hipEventDestroy(c.ev0); (void)hipEventDestroy(c.ev1);
-  for (hipEvent_t e : c.piece_ev) if (e) (void)hipEventDestroy(e);
+  if (c.d_arrive) (void)hipFree(c.d_arrive);
+  if (c.h_flags) (void)hipHostFree(c.h_flags);
   (void)hipStreamDestroy(c.stream);
   c = Context();
   return CAI_OK;

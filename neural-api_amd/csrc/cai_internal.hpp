@@ -26,7 +26,7 @@ struct Context {
   void*  h_stage = nullptr; size_t h_stage_cap = 0;      // pinned host memory of calls that wait for their results (kernels read and write it in place)
   int32_t* d_small = nullptr;            // 1024 ints of device scratch for small arguments/results
   int32_t* h_small = nullptr;            // 1024 ints of pinned host memory paired with d_small
-  hipEvent_t  piece_ev[8] = {};          // pieces of a result on their way to the host (fetch_to_host)
+  uint32_t* h_flags = nullptr; unsigned* d_arrive = nullptr; uint32_t signals = 0;      // HostSignal
   // Step timeline (measurement aid, cai_decoder_timeline): while armed, every instrumented launch gets a record of eight
   // wall-clock stamps per work-group (0 entry .. 7 exit, the ones between are the kernel's own) and a descriptor (class,
   // work-groups, offset)
@@ -71,7 +71,31 @@ int  set_error(int code, const char* fmt, ...);
 int  hip_fail(hipError_t e, const char* what, const char* file, int line);
 int  ensure_stage(void** p, size_t* cap, size_t need);
 int  ensure_host_stage(size_t need);   // grows ctx().h_stage; only for calls that do not return before the stream is done with it
-// A call's results: `bytes` (whole words) at the device address src for the caller's memory dst.  fetch_to_host waits for the stream.
+// What a call's last launch writes into pinned memory when its results there, and what the launches before it wrote, can be read: the host sees it 5 us before the
+// end of the stream (a launch and hipStreamSynchronize 10.9 us, a launch and this 5.6).  The last work-group to arrive writes it; the arrivals wrap to
+// zero.  A wait of more than 50 ms goes on in hipStreamSynchronize, which also returns an error of the launches.
+constexpr int HOST_SIGNALS = 8;            // of one call
+struct HostSignal { uint32_t* flag = nullptr; unsigned* arrive = nullptr; uint32_t value = 0; };      // flag null: none
+HostSignal host_signal_next(int k = 0);    // the k-th of this call
+int  host_signal_wait(const HostSignal& s);
+void launch_host_signal(const HostSignal& s);      // as a launch of its own
+// A result in coherent pinned memory: a store of system scope, which no cache keeps and which is acknowledged when it is there.
+template <typename T> __device__ __forceinline__ void host_store(T* p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
+// By every thread, at the end of a kernel that leaves its results with host_store: they are acknowledged (vmcnt(0)) before the work-group arrives, so
+// there is nothing to write back.  (With ordinary stores and a fence of system scope the last of the candidates' launches took 9.5 us instead of 5.8;
+// with ordinary stores and no fence the host read what had been there before.)
+__device__ __forceinline__ void host_signal(const HostSignal& s, unsigned work_groups)
+{
+  if (!s.flag) return;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  if (work_groups > 1 && __builtin_amdgcn_atomic_inc32(s.arrive, work_groups - 1, __ATOMIC_RELAXED, "agent") != work_groups - 1) return;
+  __hip_atomic_store(s.flag, s.value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// A call's results: `bytes` (whole words) at the device address src for the caller's memory dst.  fetch_to_host waits for them, and with them for
+// everything the stream held before.
 struct HostCopy { void* dst; const void* src; size_t bytes; };
 int  fetch_to_host(const HostCopy* c, int n);
 void launch_words_copy(const void* src, void* dst, int words);   // a few words between device and pinned memory, either way, as a launch of the stream (or node of a graph)

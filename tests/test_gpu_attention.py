@@ -540,3 +540,28 @@ def test_device_rows_are_used_in_place_or_copied(kvt, hq, hkv, dk, ctx, sinks, r
             np.testing.assert_array_equal(y.cpu().numpy(), want, err_msg=f"row {pos} shift {shift} over {over}")
             if not over:
                 np.testing.assert_array_equal(x.cpu().numpy(), rows[pos])
+
+
+@pytest.mark.parametrize("hq,hkv,dk,n", [(2, 1, 4, 3), (9, 3, 64, 40), (40, 8, 128, 40)])
+def test_rows_left_on_the_device_or_in_pinned_memory_are_there_when_the_call_returns(hq, hkv, dk, n):
+    """The call waits for a signal behind the kernels where the row stays on this card, and for the end of the stream elsewhere: each row is that of the call
+    that copies it to the host, bit for bit, read by another stream at once, and the next call's does not reach it."""
+    import torch
+    from helpers.device import dev
+    cai = dev()
+    g = np.random.default_rng(dk)
+    rows = g.standard_normal((n, (hq + 2 * hkv) * dk)).astype(np.float32)
+    a, b, c = (cai.KVCache(1, hkv, dk, 256, cai.KV_I8) for _ in range(3))
+    x = torch.from_numpy(rows).cuda()
+    y = torch.zeros((n, hq * dk), device="cuda")
+    z = torch.zeros((n, hq * dk), pin_memory=True)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    for p in range(n):
+        want = a.attn_decode(0, rows[p], hq)
+        cai.check(cai.load().cai_attn_decode(b.h, 0, x[p].data_ptr(), hq, 0, 0.0, y[p].data_ptr(), cai.X_DEVICE | cai.Y_DEVICE))
+        with torch.cuda.stream(side):
+            got = y[p] * 1.0
+        assert np.array_equal(got.cpu().numpy(), want), p
+        cai.check(cai.load().cai_attn_decode(c.h, 0, x[p].data_ptr(), hq, 0, 0.0, z[p].data_ptr(), cai.X_DEVICE | cai.Y_DEVICE))
+        assert np.array_equal(z[p].numpy(), want), p
