@@ -1410,9 +1410,13 @@ __global__ __launch_bounds__(256) void kv_append_rows_i8_kernel(const AttnParams
 
 // ------------------------------------------------------------------------------------------
 // Prompt ingestion on the matrix cores: every prompt token attends over the cached rows up to its own position.
-// Work-group = (KV head, four query heads of its group, 32 consecutive tokens); wave w takes head h0 + w.  Heads are HD = 128 or 64 wide.  K and V
-// tiles of 32 cached rows are staged in LDS (V transposed) and shared by the four waves.  Per tile and wave:
-//   S^T[row][token] = K . q^T   on v_mfma_f32_32x32x8_f16: the result lane holds ONE token column, so the running
+//
+// prompt_rows_kernel: the rotated K and the V of the chunk's tokens into the cache, and what the products read: q and the cached rows of the layer's
+// range as planes of halfs (a float or dequantised row two of them, hi + lo), the rows in the order of the matrix operands, so that a wave takes
+// an operand of a tile of 32 rows with one request of a whole KB.
+// attn_prompt_kernel: a work-group = (query head, 32 consecutive tokens); its four waves take every fourth tile of the tokens' range, each with sums of
+// its own, and fold them through LDS at the end.  Per tile and wave:
+//   S^T[row][token] = K . q^T   on v_mfma_f32_32x32x16_f16: the result lane holds ONE token column, so the running
 //                               maximum, the normaliser and the rescaling of the output are per-lane scalars, and the
 //                               result registers of k-step s are exactly the B operand of step s of the next product;
 //   O^T[dim][token] += V^T . P^T   with P split hi + lo into two f16 (22 bits), like q; a float cache is split too.
@@ -1421,41 +1425,56 @@ __global__ __launch_bounds__(256) void kv_append_rows_i8_kernel(const AttnParams
 // two first: q per token and head, the rows of a float cache each (int8 codes are exact halfs; their scales count as the row's), the weights
 // times the value rows' scales per token and tile, whose sums are then added to O as floats; over a half cache only q and, by 2^14, the
 // weights.  9 / 3 heads, float cache, six layers of a 511-token prompt: 593 us without, 630; values of 1e-5 were 7e-5 off and such past 65504 NaN.
+// What bounds it: a CU takes in 85 KB/us, an operand pair of a tile of a float cache is 32 KB for 1536 cycles of products.
+// Before, four heads of a group shared tiles that every work-group converted itself, V transposed by two-byte stores, one wave a SIMD and three of
+// four without a head where a KV head has one.  511 tokens of 28 / 4 heads, float rows: 39.5 us and 11.7 for adding two pieces, 18.7 now (6.6 without any tile,
+// 11.3 with one a wave); 255 of 16 / 16: 20.5 + 5.3, 10.2; rows and planes 8.3, 8.5.  512 behind 4096 cached rows, three layers, whole prompt:
+// 28 / 4 heads 1088, 646; 16 / 16 1759, 542; 9 / 3 of 64 478, 326.
 // ------------------------------------------------------------------------------------------
 typedef float pf16_t __attribute__((ext_vector_type(16)));
 
 struct PromptParams {
-  const float* qkv; int64_t qkv_stride;      // rows [Q | K | V], K and V already appended to the cache
+  const float* qkv; int64_t qkv_stride;      // rows [Q | K | V]
   _Float16* qhi; _Float16* qlo;              // [token][q_heads * HD] rotated q, hi + lo
-  const void* kc; const void* vc;            // this sequence's layer plane: [kv_head][max_ctx][HD]
+  _Float16* planes;                          // [kv_head][n_tiles] tiles of 32 cached rows: PromptShape::TILE halfs
+  float* rsc;                                // PromptShape::ROWS: [kv_head][n_tiles][K 32 | V 32] what a row's planes are to be multiplied by
+  void* kc; void* vc;                        // this sequence's layer plane: [kv_head][max_ctx][HD]
   const float* ksc; const float* vsc;        // int8 cache: row scales of the same plane, [kv_head][max_ctx]
-  int q_heads, kv_heads, max_ctx, n_tok, window;
+  int q_heads, kv_heads, max_ctx, n_tok, n_tiles, window;
   float softcap, inv_sqrt;
-  const float* theta; const int32_t* pos;
+  const float* theta; int pos0;              // token t: position pos0 + t of the sequence
   float* out; int64_t out_stride;
   float* part;                               // [token][q_head][K split][HD + 2]: unnormalised sums, maximum, normaliser
   float* qsc;                                // HD = 64: [token][q_head] what the head's planes are to be multiplied by
 };
 
-constexpr int PA_KT_MIN = 2;     // K tiles (of 32 cached rows) a split takes at least
+template <typename KV_T, int HD> struct PromptShape {
+  static constexpr bool I8 = sizeof(KV_T) == 1;          // int8 rows: HD = 128: dequantised (code * row scale)
+  static constexpr bool SC = HD == 64;                   // every operand holds what a float holds, whatever its size: see the comment above
+  static constexpr bool ROWS = SC && sizeof(KV_T) != 2;  // row scales
+  static constexpr int NP = (SC ? sizeof(KV_T) == 4 : sizeof(KV_T) != 2) ? 2 : 1;      // planes of K and V
+  static constexpr int PLANE = 32 * HD, TILE = 2 * NP * PLANE;      // halfs: K's planes [step of 16 dims][lane][8], V's [step of 16 rows][32 dims][lane][8]
+};
+
+constexpr int PA_KT_MIN = 8;     // K tiles (of 32 cached rows) a split takes at least: two a wave
 constexpr int PA_KS_MAX = 8;     // splits of a token tile's K range at most
-// K tiles a token tile walks and the number of work-groups (blockIdx.z) they are cut over: long ranges are split so that a
-// short prompt (few token tiles, a causal triangle of work) still fills the chip; the merge kernel adds the pieces.
+// K tiles a token tile walks and the number of work-groups (blockIdx.z) they are cut over: a short prompt behind many rows
+// (few token tiles) still fills the chip; the merge kernel adds the pieces.
 __device__ __forceinline__ void prompt_k_range(const PromptParams& p, int t0, int n_ks, int& jt0, int& jt1, int& splits)
 {
-  const int pos_first = p.pos[t0], pos_last = p.pos[min(t0 + 31, p.n_tok - 1)];
+  const int pos_first = p.pos0 + t0, pos_last = p.pos0 + min(t0 + 31, p.n_tok - 1);
   const int j_lo = (p.window > 0 && pos_first + 1 > p.window) ? pos_first + 1 - p.window : 0;
   jt0 = j_lo >> 5; jt1 = pos_last >> 5;
   splits = max(1, min(n_ks, (jt1 - jt0 + 1) / PA_KT_MIN));
 }
 
-// rotated q (neural/neural.cl:1517-1542) as two f16 planes
+// rotated q of token t (neural/neural.cl:1517-1542) as two f16 planes
 template <int HD>
-__device__ __forceinline__ void prompt_q_row(const PromptParams& p)
+__device__ __forceinline__ void prompt_q_row(const PromptParams& p, const int t)
 {
-  const int t = blockIdx.x, qw = p.q_heads * HD;
+  const int qw = p.q_heads * HD;
   const float* row = p.qkv + (int64_t)t * p.qkv_stride;
-  const int pos = p.pos[t];
+  const int pos = p.pos0 + t;
   for (int e = threadIdx.x; e < (qw >> 1); e += 256) {
     const int d = (2 * e) & (HD - 1);
     float x0 = row[2 * e], x1 = row[2 * e + 1];
@@ -1477,37 +1496,134 @@ __device__ __forceinline__ void prompt_q_row(const PromptParams& p)
     p.qlo[(int64_t)t * qw + 2 * e] = l0; p.qlo[(int64_t)t * qw + 2 * e + 1] = l1;
   }
 }
-template <int HD>
-__global__ __launch_bounds__(256) void prompt_q_kernel(const PromptParams p) { prompt_q_row<HD>(p); }
-// one launch per chunk for both: the token's K and V rows into the cache, its rotated q into the planes
-template <typename KV_T, int HD>
-__global__ __launch_bounds__(256) void prompt_rows_kernel(const AttnParams p, const PromptParams pp) { kv_append_row<KV_T>(p); prompt_q_row<HD>(pp); }
 
-constexpr int PA_LDV = 36;     // halfs per staged V^T row (32 cached rows + pad)
-
+// Work-groups 0 .. n_tiles * kv_heads - 1: 32 cached rows of a KV head each, those of the chunk from its K and V (an int8 cache has them already);
+// the others: a token's q.
 template <typename KV_T, int HD>
-__global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
+__global__ __launch_bounds__(256) void prompt_rows_kernel(const PromptParams p)
 {
-  constexpr bool I8P = sizeof(KV_T) == 1;         // int8 rows: HD = 128: dequantised (code * row scale) while they are staged
-  constexpr bool SC = HD == 64;                   // every operand holds what a float holds, whatever its size: see the comment above
-  constexpr bool F32 = SC ? sizeof(KV_T) == 4 : sizeof(KV_T) != 2;         // ... and, like a float cache, split hi + lo
-  constexpr bool ROWS = SC && sizeof(KV_T) != 2;  // row scales
-  constexpr int NP = F32 ? 2 : 1;                 // planes of K and V
-  constexpr int PA_LDK = HD + 8;                  // halfs per staged K row (rows stay 16-byte aligned for the 8-half operand reads)
-  constexpr int E = HD / 8;                       // elements of a row that a thread stages
-  __shared__ __align__(16) _Float16 sK[NP][32 * PA_LDK];
-  __shared__ __align__(16) _Float16 sV[NP][HD * PA_LDV];
-  __shared__ __align__(16) float sKS[ROWS ? 32 : 4], sVS[ROWS ? 32 : 4];      // of each cached row: what its staged K and V are to be multiplied by
-  const int G = p.q_heads / p.kv_heads, quads = (G + 3) >> 2;
-  const int g = blockIdx.y / quads, h0 = (blockIdx.y % quads) * 4;
-  const int t0 = blockIdx.x * 32;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, n = lane & 31, kg = lane >> 5;
-  const int hq = h0 + wave;                       // head within the group
-  const bool head_on = hq < G;
-  const int head = g * G + (head_on ? hq : 0);
+  using S = PromptShape<KV_T, HD>;
+  constexpr int E = HD / 8, DT = HD / 32, LDF = HD + 4;
+  __shared__ __align__(16) float sv[32 * LDF];
+  const int tiles = p.n_tiles * p.kv_heads, tid = threadIdx.x;
+  if ((int)blockIdx.x >= tiles) { prompt_q_row<HD>(p, blockIdx.x - tiles); return; }
+  const int g = blockIdx.x % p.kv_heads, jt = blockIdx.x / p.kv_heads;
+  const int pos0 = p.pos0, last = pos0 + p.n_tok - 1;
+  const int lo = p.window > 0 && pos0 + 1 > p.window ? pos0 + 1 - p.window : 0;
+  if (32 * jt > last || jt < (lo >> 5)) return;                    // (whole work-groups)
+  const int r = tid >> 3, d0 = (tid & 7) * E, j = 32 * jt + r;     // E consecutive elements of a cached row
+  const bool live = j <= last;
+  const int64_t at = ((int64_t)g * p.max_ctx + min(j, last)) * HD + d0;
+  float k[E], v[E], ks = 1.0f, vs = 1.0f;
+  if constexpr (S::I8) {
+    const int8_t *kq = reinterpret_cast<const int8_t*>(p.kc) + at, *vq = reinterpret_cast<const int8_t*>(p.vc) + at;
+    ks = p.ksc[(int64_t)g * p.max_ctx + min(j, last)]; vs = p.vsc[(int64_t)g * p.max_ctx + min(j, last)];
+#pragma unroll
+    for (int i = 0; i < E; i += 4) {
+      const int a = *reinterpret_cast<const int*>(kq + i), b = *reinterpret_cast<const int*>(vq + i);
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        k[i + u] = (float)((a << (24 - 8 * u)) >> 24) * (S::ROWS ? 1.0f : ks);      // (codes are exact halfs)
+        v[i + u] = (float)((b << (24 - 8 * u)) >> 24) * (S::ROWS ? 1.0f : vs);
+      }
+    }
+  } else {
+    KV_T ko[E], vo[E];
+    if (live && j >= pos0) {
+      const float *kr = p.qkv + (int64_t)(j - pos0) * p.qkv_stride + (int64_t)p.q_heads * HD + g * HD + d0, *vr = kr + p.kv_heads * HD;
+      KV_T *kd = reinterpret_cast<KV_T*>(p.kc) + at, *vd = reinterpret_cast<KV_T*>(p.vc) + at;
+#pragma unroll
+      for (int i = 0; i < E; i += 4) { *reinterpret_cast<float4*>(k + i) = *reinterpret_cast<const float4*>(kr + i); *reinterpret_cast<float4*>(v + i) = *reinterpret_cast<const float4*>(vr + i); }
+      if (p.theta)
+#pragma unroll
+        for (int i = 0; i < E; i += 2) {
+          float sn, cs; sincosf((float)j * p.theta[(d0 + i) >> 1], &sn, &cs);
+          const float y0 = cs * k[i] - sn * k[i + 1], y1 = sn * k[i] + cs * k[i + 1];
+          k[i] = y0; k[i + 1] = y1;
+        }
+#pragma unroll
+      for (int i = 0; i < E; i++) { ko[i] = kv_from_float<KV_T>(k[i]); vo[i] = kv_from_float<KV_T>(v[i]); k[i] = kv_to_float(ko[i]); v[i] = kv_to_float(vo[i]); }
+#pragma unroll
+      for (int i = 0; i < E * (int)sizeof(KV_T) / 16; i++) { reinterpret_cast<uint4*>(kd)[i] = reinterpret_cast<const uint4*>(ko)[i]; reinterpret_cast<uint4*>(vd)[i] = reinterpret_cast<const uint4*>(vo)[i]; }
+    } else {
+#pragma unroll
+      for (int i = 0; i < E * (int)sizeof(KV_T) / 16; i++) {
+        reinterpret_cast<uint4*>(ko)[i] = reinterpret_cast<const uint4*>(reinterpret_cast<const KV_T*>(p.kc) + at)[i];
+        reinterpret_cast<uint4*>(vo)[i] = reinterpret_cast<const uint4*>(reinterpret_cast<const KV_T*>(p.vc) + at)[i];
+      }
+#pragma unroll
+      for (int i = 0; i < E; i++) { k[i] = kv_to_float(ko[i]); v[i] = kv_to_float(vo[i]); }
+    }
+  }
+  if (!live) {                                // rows behind the last one hold what an earlier sequence left: not multiplied, not even by zero
+#pragma unroll
+    for (int i = 0; i < E; i++) k[i] = v[i] = 0.0f;
+    ks = vs = 0.0f;
+  }
+  if constexpr (S::ROWS) {                    // (the eight threads of a row are neighbours)
+    if (!S::I8) {
+      float mk = 0.0f, mv = 0.0f;
+#pragma unroll
+      for (int i = 0; i < E; i++) { mk = fmaxf(mk, finite_abs(k[i])); mv = fmaxf(mv, finite_abs(v[i])); }
+#pragma unroll
+      for (int off = 1; off < 8; off <<= 1) { mk = fmaxf(mk, __shfl_xor(mk, off)); mv = fmaxf(mv, __shfl_xor(mv, off)); }
+      const int ek = plane_exponent(mk), ev = plane_exponent(mv);
+#pragma unroll
+      for (int i = 0; i < E; i++) { k[i] = ldexpf(k[i], ek); v[i] = ldexpf(v[i], ev); }
+      ks = ldexpf(1.0f, -ek); vs = ldexpf(1.0f, -ev);
+    }
+    if ((tid & 7) == 0) { float* s = p.rsc + ((int64_t)g * p.n_tiles + jt) * 64 + r; s[0] = ks; s[32] = vs; }
+  }
+  auto split = [](float x, _Float16& h, _Float16& l) { if (S::SC) split_plane(x, h, l); else split_f16(x, h, l); };
+  _Float16* tile = p.planes + ((int64_t)g * p.n_tiles + jt) * S::TILE;
+#pragma unroll
+  for (int i8 = 0; i8 < E; i8 += 8) {         // dims d0 + i8 .. + 7: step d / 16, lane half (d / 8) % 2, row r
+    ph8_t h, l;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      if (S::NP == 2) { _Float16 a, b; split(k[i8 + i], a, b); h[i] = a; l[i] = b; }
+      else h[i] = (_Float16)k[i8 + i];
+    }
+    const int d = d0 + i8, o = ((d >> 4) * 64 + ((d >> 3) & 1) * 32 + r) * 8;
+    *reinterpret_cast<ph8_t*>(tile + o) = h;
+    if (S::NP == 2) *reinterpret_cast<ph8_t*>(tile + S::PLANE + o) = l;
+  }
+#pragma unroll
+  for (int i = 0; i < E; i += 4) *reinterpret_cast<float4*>(&sv[r * LDF + d0 + i]) = *reinterpret_cast<const float4*>(v + i);
+  __syncthreads();
+  tile += S::NP * S::PLANE;
+  for (int f = tid; f < 2 * DT * 64; f += 256) {      // lane (n, kg) of step s2, dims 32 dt + n: the rows that the weights' registers hold (below)
+    const int lane = f & 63, dt = (f >> 6) % DT, s2 = (f >> 6) / DT, n = lane & 31, kg = lane >> 5;
+    ph8_t h, l;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const float x = sv[(16 * s2 + 8 * (i >> 2) + 4 * kg + (i & 3)) * LDF + 32 * dt + n];
+      if (S::NP == 2) { _Float16 a, b; split(x, a, b); h[i] = a; l[i] = b; }
+      else h[i] = (_Float16)x;
+    }
+    *reinterpret_cast<ph8_t*>(tile + 8 * f) = h;
+    if (S::NP == 2) *reinterpret_cast<ph8_t*>(tile + S::PLANE + 8 * f) = l;
+  }
+}
+
+constexpr int PA_LDO = 33;     // floats per output dimension in LDS (32 tokens + 1)
+
+template <typename KV_T, int HD>
+__global__ __launch_bounds__(256, 2) void attn_prompt_kernel(const PromptParams p)
+{
+  using S = PromptShape<KV_T, HD>;
+  constexpr bool SC = S::SC, ROWS = S::ROWS;
+  constexpr int NP = S::NP, STEPS = HD / 16, DT = HD / 32, LDQ = HD + 8;      // (LDQ: rows stay 16-byte aligned for the 8-half operand reads)
+  constexpr int Q_B = 2 * 32 * LDQ * 2, O_B = 4 * HD * PA_LDO * 4;
+  __shared__ __align__(16) unsigned char lds[Q_B > O_B ? Q_B : O_B];          // q's planes [2][32][LDQ] halfs; then the waves' sums [4][HD][PA_LDO]
+  __shared__ float sM[4][32], sL[4][32];
+  _Float16* sQ = reinterpret_cast<_Float16*>(lds);
+  float* sO = reinterpret_cast<float*>(lds);
+  const int head = blockIdx.x, g = head / (p.q_heads / p.kv_heads);
+  const int t0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * 32;                 // the longest ranges first
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, n = lane & 31, kg = lane >> 5;
   const int tok = t0 + n;
-  const bool tok_on = tok < p.n_tok;
-  const int pos_n = tok_on ? p.pos[tok] : -1;
+  const int pos_n = tok < p.n_tok ? p.pos0 + tok : -1;
   const int jstart_n = (p.window > 0 && pos_n + 1 > p.window) ? pos_n + 1 - p.window : 0;
   // the tile's range of cached rows (tokens are consecutive positions of one sequence) and this work-group's share of it
   int jt_first, jt_last, splits;
@@ -1519,166 +1635,82 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
     const int a = jt_first + ks * per;
     jt_last = min(jt_last, a + per - 1); jt_first = a;
   }
-  const KV_T* kc = reinterpret_cast<const KV_T*>(p.kc) + (int64_t)g * p.max_ctx * HD;
-  const KV_T* vc = reinterpret_cast<const KV_T*>(p.vc) + (int64_t)g * p.max_ctx * HD;
-
-  // this lane's q fragments: token n, dims 16 s + 8 kg .. + 7 of the wave's head
-  ph8_t qh[HD / 16], ql[HD / 16];
-  {
-    const int64_t qo = (int64_t)min(tok, p.n_tok - 1) * (p.q_heads * HD) + head * HD + 8 * kg;
+  // The operands of the wave's next tile are requested as soon as the registers of the current one are free: K's run behind the weights and the second
+  // product, V's behind the next tile's first product.
+  const _Float16* planes = p.planes + (int64_t)g * p.n_tiles * S::TILE + 8 * lane;
+  const float* scales = ROWS ? p.rsc + (int64_t)g * p.n_tiles * 64 + 4 * kg : nullptr;
+  ph8_t K[NP][STEPS], V[NP][2 * DT];
+  float4 rk[ROWS ? 4 : 1], rv[ROWS ? 4 : 1];
+  auto load_k = [&](int jt) __attribute__((always_inline)) {
+    if (jt > jt_last) return;
 #pragma unroll
-    for (int s = 0; s < HD / 16; s++) {
-      qh[s] = *reinterpret_cast<const ph8_t*>(p.qhi + qo + 16 * s);
-      ql[s] = *reinterpret_cast<const ph8_t*>(p.qlo + qo + 16 * s);
-    }
+    for (int s = 0; s < STEPS; s++)
+#pragma unroll
+      for (int q = 0; q < NP; q++) K[q][s] = *reinterpret_cast<const ph8_t*>(planes + (int64_t)jt * S::TILE + q * S::PLANE + 512 * s);
+    if constexpr (ROWS)
+#pragma unroll
+      for (int i = 0; i < 4; i++) rk[i] = *reinterpret_cast<const float4*>(scales + (int64_t)jt * 64 + 8 * i);
+  };
+  auto load_v = [&](int jt) __attribute__((always_inline)) {
+    if (jt > jt_last) return;
+#pragma unroll
+    for (int s = 0; s < 2 * DT; s++)
+#pragma unroll
+      for (int q = 0; q < NP; q++) V[q][s] = *reinterpret_cast<const ph8_t*>(planes + (int64_t)jt * S::TILE + (NP + q) * S::PLANE + 512 * s);
+    if constexpr (ROWS)
+#pragma unroll
+      for (int i = 0; i < 4; i++) rv[i] = *reinterpret_cast<const float4*>(scales + (int64_t)jt * 64 + 32 + 8 * i);
+  };
+  constexpr int QN = 2 * 32 * (HD / 8) / 256;
+  ph8_t qr[QN];
+#pragma unroll
+  for (int i = 0; i < QN; i++) {
+    const int u = tid + 256 * i, q = u / (32 * (HD / 8)), r = u / (HD / 8) % 32, c = u % (HD / 8);
+    qr[i] = *reinterpret_cast<const ph8_t*>((q ? p.qlo : p.qhi) + (int64_t)min(t0 + r, p.n_tok - 1) * (p.q_heads * HD) + head * HD + 8 * c);
+  }
+  load_k(jt_first + wave);
+#pragma unroll
+  for (int i = 0; i < QN; i++) {
+    const int u = tid + 256 * i, r = u / (HD / 8) % 64, c = u % (HD / 8);
+    *reinterpret_cast<ph8_t*>(sQ + r * LDQ + 8 * c) = qr[i];
   }
   const float qs = SC ? p.qsc[(int64_t)min(tok, p.n_tok - 1) * p.q_heads + head] * p.inv_sqrt : p.inv_sqrt;
-  const int last = p.pos[p.n_tok - 1];            // rows behind it hold what an earlier sequence left: not multiplied, not even by zero
-  pf16_t O[HD / 32];
+  load_v(jt_first + wave);
+  pf16_t O[DT];
 #pragma unroll
-  for (int dt = 0; dt < HD / 32; dt++)
+  for (int dt = 0; dt < DT; dt++)
 #pragma unroll
     for (int v = 0; v < 16; v++) O[dt][v] = 0.0f;
   float m_run = -1e30f, l_run = 0.0f;
+  __syncthreads();
 
-  const int srow = tid >> 3, sdim = (tid & 7) * E;          // staging: E consecutive elements of one cached row
-  // The rows of the NEXT tile are requested before the products of the current one and converted into LDS after them: the
-  // memory round trip runs behind the matrix-core work instead of in front of it.  Requests are unconditional (rows past the
-  // live range are clamped and masked below).
-  struct RawTile { uint4 k[sizeof(KV_T) == 4 ? E / 4 : 2], v[sizeof(KV_T) == 4 ? E / 4 : 2]; float ks, vs; };   // (int8: one uint4 each is used)
-  auto fetch = [&](int jt, RawTile& r) {
-    const int j = min(jt * 32 + srow, p.max_ctx - 1);
-    if (I8P) {
-      if constexpr (E == 16) {
-        r.k[0] = *reinterpret_cast<const uint4*>(reinterpret_cast<const int8_t*>(kc) + (int64_t)j * HD + sdim);
-        r.v[0] = *reinterpret_cast<const uint4*>(reinterpret_cast<const int8_t*>(vc) + (int64_t)j * HD + sdim);
-      } else {
-        const uint2 a = *reinterpret_cast<const uint2*>(reinterpret_cast<const int8_t*>(kc) + (int64_t)j * HD + sdim), b = *reinterpret_cast<const uint2*>(reinterpret_cast<const int8_t*>(vc) + (int64_t)j * HD + sdim);
-        r.k[0] = make_uint4(a.x, a.y, 0u, 0u); r.v[0] = make_uint4(b.x, b.y, 0u, 0u);
-      }
-      r.ks = p.ksc[(int64_t)g * p.max_ctx + j]; r.vs = p.vsc[(int64_t)g * p.max_ctx + j];
-    } else if (sizeof(KV_T) == 4) {
-#pragma unroll
-      for (int c4 = 0; c4 < E / 4; c4++) {
-        r.k[c4] = *reinterpret_cast<const uint4*>(reinterpret_cast<const float*>(kc) + (int64_t)j * HD + sdim + 4 * c4);
-        r.v[c4] = *reinterpret_cast<const uint4*>(reinterpret_cast<const float*>(vc) + (int64_t)j * HD + sdim + 4 * c4);
-      }
-    } else {
-#pragma unroll
-      for (int c8 = 0; c8 < E / 8; c8++) {
-        r.k[c8] = *reinterpret_cast<const uint4*>(reinterpret_cast<const __half*>(kc) + (int64_t)j * HD + sdim + 8 * c8);
-        r.v[c8] = *reinterpret_cast<const uint4*>(reinterpret_cast<const __half*>(vc) + (int64_t)j * HD + sdim + 8 * c8);
-      }
-    }
-  };
-  RawTile raw;
-  fetch(jt_first, raw);
-  for (int jt = jt_first; jt <= jt_last; jt++) {
-    __syncthreads();                                        // the previous tile has been consumed
-    {
-      float kv[E], vv[E];
-      if (jt * 32 + srow > last) {
-#pragma unroll
-        for (int i = 0; i < (int)(sizeof(raw.v) / sizeof(uint4)); i++) raw.v[i] = make_uint4(0u, 0u, 0u, 0u);
-        raw.vs = 0.0f;
-      }
-      if (I8P) {
-        const uint4 a = raw.k[0], b = raw.v[0];
-        const float ks = ROWS ? 1.0f : raw.ks, vs = ROWS ? 1.0f : raw.vs;     // (codes are exact halfs)
-        if (ROWS && (tid & 7) == 0) { sKS[srow] = raw.ks; sVS[srow] = raw.vs; }
-        const int aw[4] = {(int)a.x, (int)a.y, (int)a.z, (int)a.w}, bw[4] = {(int)b.x, (int)b.y, (int)b.z, (int)b.w};
-#pragma unroll
-        for (int i = 0; i < E / 4; i++) {
-          kv[4 * i] = (float)((aw[i] << 24) >> 24) * ks; kv[4 * i + 1] = (float)((aw[i] << 16) >> 24) * ks;
-          kv[4 * i + 2] = (float)((aw[i] << 8) >> 24) * ks; kv[4 * i + 3] = (float)(aw[i] >> 24) * ks;
-          vv[4 * i] = (float)((bw[i] << 24) >> 24) * vs; vv[4 * i + 1] = (float)((bw[i] << 16) >> 24) * vs;
-          vv[4 * i + 2] = (float)((bw[i] << 8) >> 24) * vs; vv[4 * i + 3] = (float)(bw[i] >> 24) * vs;
-        }
-      } else if (sizeof(KV_T) == 4) {
-#pragma unroll
-        for (int c4 = 0; c4 < E / 4; c4++) {
-          const uint4 a = raw.k[c4], b = raw.v[c4];
-          kv[4 * c4] = __builtin_bit_cast(float, a.x); kv[4 * c4 + 1] = __builtin_bit_cast(float, a.y); kv[4 * c4 + 2] = __builtin_bit_cast(float, a.z); kv[4 * c4 + 3] = __builtin_bit_cast(float, a.w);
-          vv[4 * c4] = __builtin_bit_cast(float, b.x); vv[4 * c4 + 1] = __builtin_bit_cast(float, b.y); vv[4 * c4 + 2] = __builtin_bit_cast(float, b.z); vv[4 * c4 + 3] = __builtin_bit_cast(float, b.w);
-        }
-        if constexpr (ROWS) {                             // (the eight threads of a row are neighbours)
-          float mk = 0.0f, mv = 0.0f;
-#pragma unroll
-          for (int i = 0; i < E; i++) { mk = fmaxf(mk, finite_abs(kv[i])); mv = fmaxf(mv, finite_abs(vv[i])); }
-#pragma unroll
-          for (int off = 1; off < 8; off <<= 1) { mk = fmaxf(mk, __shfl_xor(mk, off)); mv = fmaxf(mv, __shfl_xor(mv, off)); }
-          const int ek = plane_exponent(mk), ev = plane_exponent(mv);
-#pragma unroll
-          for (int i = 0; i < E; i++) { kv[i] = ldexpf(kv[i], ek); vv[i] = ldexpf(vv[i], ev); }
-          if ((tid & 7) == 0) { sKS[srow] = ldexpf(1.0f, -ek); sVS[srow] = ldexpf(1.0f, -ev); }
-        }
-      }
-      if constexpr (sizeof(KV_T) == 2) {                  // a half cache goes in as it is
-#pragma unroll
-        for (int c8 = 0; c8 < E / 8; c8++) {
-          const uint4 a = raw.k[c8], b = raw.v[c8];
-          *reinterpret_cast<uint2*>(&sK[0][srow * PA_LDK + sdim + 8 * c8]) = make_uint2(a.x, a.y);
-          *reinterpret_cast<uint2*>(&sK[0][srow * PA_LDK + sdim + 8 * c8 + 4]) = make_uint2(a.z, a.w);
-          const uint32_t bw[4] = {b.x, b.y, b.z, b.w};
-#pragma unroll
-          for (int i = 0; i < 4; i++) {
-            sV[0][(sdim + 8 * c8 + 2 * i) * PA_LDV + srow] = __builtin_bit_cast(_Float16, (unsigned short)(bw[i] & 0xffffu));
-            sV[0][(sdim + 8 * c8 + 2 * i + 1) * PA_LDV + srow] = __builtin_bit_cast(_Float16, (unsigned short)(bw[i] >> 16));
-          }
-        }
-      } else {
-#pragma unroll
-      for (int i4 = 0; i4 < E / 4; i4++) {                    // K rows stay row-major: 8-byte stores
-        ph4_t kh, kl;
-#pragma unroll
-        for (int i = 0; i < 4; i++) { _Float16 a, b; if (SC) split_plane(kv[4 * i4 + i], a, b); else split_f16(kv[4 * i4 + i], a, b); kh[i] = a; kl[i] = b; }
-        *reinterpret_cast<ph4_t*>(&sK[0][srow * PA_LDK + sdim + 4 * i4]) = kh;
-        if (F32) *reinterpret_cast<ph4_t*>(&sK[NP - 1][srow * PA_LDK + sdim + 4 * i4]) = kl;
-      }
-#pragma unroll
-      for (int i = 0; i < E; i++) {                       // V goes in transposed
-        _Float16 vh, vl;
-        if (SC) split_plane(vv[i], vh, vl); else split_f16(vv[i], vh, vl);
-        sV[0][(sdim + i) * PA_LDV + srow] = vh;
-        if (F32) sV[NP - 1][(sdim + i) * PA_LDV + srow] = vl;
-      }
-      }
-    }
-    fetch(jt + 1, raw);                                     // in flight during the products below
-    __syncthreads();
-    if (!head_on) continue;                                 // (an idle wave still stages and meets the barriers)
-
+  for (int jt = jt_first + wave; jt <= jt_last; jt += 4) {
     // ---- S^T = K . q^T ----
     pf16_t C;
 #pragma unroll
     for (int v = 0; v < 16; v++) C[v] = 0.0f;
 #pragma unroll
-    for (int s = 0; s < HD / 16; s++) {
-      const ph8_t a = *reinterpret_cast<const ph8_t*>(&sK[0][n * PA_LDK + 16 * s + 8 * kg]);
-      C = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qh[s], C, 0, 0, 0);
-      C = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, ql[s], C, 0, 0, 0);
-      if (F32) {
-        const ph8_t al = *reinterpret_cast<const ph8_t*>(&sK[NP - 1][n * PA_LDK + 16 * s + 8 * kg]);
-        C = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, qh[s], C, 0, 0, 0);
-      }
+    for (int s = 0; s < STEPS; s++) {
+      const ph8_t qh = *reinterpret_cast<const ph8_t*>(sQ + n * LDQ + 16 * s + 8 * kg), ql = *reinterpret_cast<const ph8_t*>(sQ + (32 + n) * LDQ + 16 * s + 8 * kg);
+      C = __builtin_amdgcn_mfma_f32_32x32x16_f16(K[0][s], qh, C, 0, 0, 0);
+      C = __builtin_amdgcn_mfma_f32_32x32x16_f16(K[0][s], ql, C, 0, 0, 0);
+      if (NP == 2) C = __builtin_amdgcn_mfma_f32_32x32x16_f16(K[NP - 1][s], qh, C, 0, 0, 0);
     }
     // ---- this token's column: mask, running maximum, weights ----
     float tmax = -1e30f;
     bool ok[16];
-    float4 rs[ROWS ? 4 : 1];
-    if constexpr (ROWS)
-#pragma unroll
-      for (int i = 0; i < 4; i++) rs[i] = *reinterpret_cast<const float4*>(&sKS[8 * i + 4 * kg]);
-    auto row_scale = [&](int v) { const float4 r = rs[ROWS ? v >> 2 : 0]; return (v & 3) == 0 ? r.x : (v & 3) == 1 ? r.y : (v & 3) == 2 ? r.z : r.w; };
+    auto of_row = [](const float4* r, int v) { const float4 x = r[ROWS ? v >> 2 : 0]; return (v & 3) == 0 ? x.x : (v & 3) == 1 ? x.y : (v & 3) == 2 ? x.z : x.w; };
 #pragma unroll
     for (int v = 0; v < 16; v++) {
       const int krow = jt * 32 + 8 * (v >> 2) + 4 * kg + (v & 3);
-      float sc = C[v] * (ROWS ? row_scale(v) * qs : qs);
+      float sc = C[v] * (ROWS ? of_row(rk, v) * qs : qs);
       if (p.softcap > 0.0f) sc = p.softcap * tanhf(sc / p.softcap);
       ok[v] = krow <= pos_n && krow >= jstart_n;
       C[v] = sc;
       if (ok[v]) tmax = fmaxf(tmax, sc);
     }
+    __builtin_amdgcn_sched_barrier(0);        // (moved up, the requests would take registers of their own)
+    load_k(jt + 4);
     tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
     const float m_new = fmaxf(m_run, tmax), corr = expf(m_run - m_new);
     float psum = 0.0f;
@@ -1688,32 +1720,30 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
     l_run = l_run * corr + psum; m_run = m_new;
     if (__builtin_amdgcn_ballot_w64(corr != 1.0f)) {      // (after the first tiles a new maximum is rare: the whole wave skips the rescaling)
 #pragma unroll
-      for (int dt = 0; dt < HD / 32; dt++)
+      for (int dt = 0; dt < DT; dt++)
 #pragma unroll
         for (int v = 0; v < 16; v++) O[dt][v] *= corr;
     }
     // row scales: the weights take them, and a power of two per token and tile brings the largest to 2^13
     float back = 1.0f;
-    pf16_t T[ROWS ? HD / 32 : 1];
+    pf16_t T[ROWS ? DT : 1];
     if constexpr (ROWS) {
       float wmax = 0.0f;
 #pragma unroll
-      for (int i = 0; i < 4; i++) rs[i] = *reinterpret_cast<const float4*>(&sVS[8 * i + 4 * kg]);
-#pragma unroll
-      for (int v = 0; v < 16; v++) { C[v] = ok[v] ? C[v] * row_scale(v) : 0.0f; wmax = fmaxf(wmax, finite_abs(C[v])); }
+      for (int v = 0; v < 16; v++) { C[v] = ok[v] ? C[v] * of_row(rv, v) : 0.0f; wmax = fmaxf(wmax, finite_abs(C[v])); }
       wmax = fmaxf(wmax, __shfl_xor(wmax, 32, 64));
       const int e = plane_exponent(wmax);
       back = ldexpf(1.0f, -e);
 #pragma unroll
       for (int v = 0; v < 16; v++) C[v] = ldexpf(C[v], e);
 #pragma unroll
-      for (int dt = 0; dt < HD / 32; dt++)
+      for (int dt = 0; dt < DT; dt++)
 #pragma unroll
         for (int v = 0; v < 16; v++) T[dt][v] = 0.0f;
     }
     // ---- O^T += V^T . P^T ----
     // The score registers 8 s2 .. 8 s2 + 7 of a lane are cached rows 16 s2 + 4 kg + (0..3) and 16 s2 + 8 + 4 kg + (0..3): taken as
-    // the eight k of a 16-deep step, with the value operand read as the same two groups of four rows (the order of the
+    // the eight k of a 16-deep step, with the value operand holding the same two groups of four rows (the order of the
     // rows inside a step is free as long as both operands agree).
 #pragma unroll
     for (int s2 = 0; s2 < 2; s2++) {
@@ -1721,48 +1751,56 @@ __global__ __launch_bounds__(256) void attn_prompt_kernel(const PromptParams p)
 #pragma unroll
       for (int i = 0; i < 8; i++) { _Float16 hv, lv; split_f16(C[8 * s2 + i], hv, lv); ph[i] = hv; pl[i] = lv; }
 #pragma unroll
-      for (int dt = 0; dt < HD / 32; dt++) {
-        const ph4_t a0 = *reinterpret_cast<const ph4_t*>(&sV[0][(32 * dt + n) * PA_LDV + 16 * s2 + 4 * kg]);
-        const ph4_t a1 = *reinterpret_cast<const ph4_t*>(&sV[0][(32 * dt + n) * PA_LDV + 16 * s2 + 8 + 4 * kg]);
-        const ph8_t a = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
-        pf16_t& S = ROWS ? T[ROWS ? dt : 0] : O[dt];
-        S = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, ph, S, 0, 0, 0);
-        S = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pl, S, 0, 0, 0);
-        if (F32) {
-          const ph4_t b0 = *reinterpret_cast<const ph4_t*>(&sV[NP - 1][(32 * dt + n) * PA_LDV + 16 * s2 + 4 * kg]);
-          const ph4_t b1 = *reinterpret_cast<const ph4_t*>(&sV[NP - 1][(32 * dt + n) * PA_LDV + 16 * s2 + 8 + 4 * kg]);
-          const ph8_t al = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
-          S = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, ph, S, 0, 0, 0);
-        }
+      for (int dt = 0; dt < DT; dt++) {
+        pf16_t& A = ROWS ? T[ROWS ? dt : 0] : O[dt];
+        A = __builtin_amdgcn_mfma_f32_32x32x16_f16(V[0][s2 * DT + dt], ph, A, 0, 0, 0);
+        A = __builtin_amdgcn_mfma_f32_32x32x16_f16(V[0][s2 * DT + dt], pl, A, 0, 0, 0);
+        if (NP == 2) A = __builtin_amdgcn_mfma_f32_32x32x16_f16(V[NP - 1][s2 * DT + dt], ph, A, 0, 0, 0);
       }
     }
+    __builtin_amdgcn_sched_barrier(0);
+    load_v(jt + 4);
     if constexpr (ROWS)
 #pragma unroll
-      for (int dt = 0; dt < HD / 32; dt++)
+      for (int dt = 0; dt < DT; dt++)
 #pragma unroll
         for (int v = 0; v < 16; v++) O[dt][v] = fmaf(T[dt][v], back, O[dt][v]);
   }
-  if (!head_on || !tok_on) return;
-  if (splits > 1) {        // this piece's unnormalised sums, maximum and normaliser; prompt_merge_kernel adds the pieces
-    float* pt = p.part + (((int64_t)tok * p.q_heads + head) * gridDim.z + ks) * (HD + 2);
+
+  // ---- the waves' sums, in wave order ----
+  if (kg == 0) { sM[wave][n] = m_run; sL[wave][n] = l_run; }
+  __syncthreads();                                // (and q has been read)
+  {
+    const float M = fmaxf(fmaxf(sM[0][n], sM[1][n]), fmaxf(sM[2][n], sM[3][n])), c = expf(m_run - M);
 #pragma unroll
-    for (int dt = 0; dt < HD / 32; dt++)
+    for (int dt = 0; dt < DT; dt++)
 #pragma unroll
-      for (int g4 = 0; g4 < 4; g4++) {
-        float* q4 = pt + 32 * dt + 8 * g4 + 4 * kg;       // (records of HD + 2 floats: 8-byte aligned only)
-        q4[0] = O[dt][4 * g4]; q4[1] = O[dt][4 * g4 + 1]; q4[2] = O[dt][4 * g4 + 2]; q4[3] = O[dt][4 * g4 + 3];
-      }
-    if (kg == 0) { pt[HD] = m_run; pt[HD + 1] = l_run; }
-    return;
+      for (int v = 0; v < 16; v++) sO[(wave * HD + 32 * dt + 8 * (v >> 2) + 4 * kg + (v & 3)) * PA_LDO + n] = l_run > 0.0f ? O[dt][v] * c : 0.0f;      // (no row of this wave: nothing)
   }
-  const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
-  float* dst = p.out + (int64_t)tok * p.out_stride + head * HD;
+  __syncthreads();
+  const int r = tid >> 3, t = t0 + r;
+  if (t >= p.n_tok) return;
+  const float M = fmaxf(fmaxf(sM[0][r], sM[1][r]), fmaxf(sM[2][r], sM[3][r]));
+  float L = 0.0f;
 #pragma unroll
-  for (int dt = 0; dt < HD / 32; dt++)
+  for (int w = 0; w < 4; w++) if (sL[w][r] > 0.0f) L = fmaf(sL[w][r], expf(sM[w][r] - M), L);
+  const float inv = splits > 1 ? 1.0f : L > 0.0f ? 1.0f / L : 0.0f;           // a piece leaves unnormalised sums, maximum and normaliser; prompt_merge_kernel adds the pieces
+  float* dst = splits > 1 ? p.part + (((int64_t)t * p.q_heads + head) * gridDim.z + ks) * (HD + 2) : p.out + (int64_t)t * p.out_stride + head * HD;
 #pragma unroll
-    for (int g4 = 0; g4 < 4; g4++)
-      *reinterpret_cast<float4*>(dst + 32 * dt + 8 * g4 + 4 * kg) =
-          make_float4(O[dt][4 * g4] * inv, O[dt][4 * g4 + 1] * inv, O[dt][4 * g4 + 2] * inv, O[dt][4 * g4 + 3] * inv);
+  for (int i = 0; i < HD / 32; i++) {
+    const int d = 32 * i + 4 * (tid & 7);
+    float a[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      a[u] = 0.0f;
+#pragma unroll
+      for (int w = 0; w < 4; w++) a[u] += sO[(w * HD + d + u) * PA_LDO + r];
+      a[u] *= inv;
+    }
+    if (splits > 1) { *reinterpret_cast<float2*>(dst + d) = make_float2(a[0], a[1]); *reinterpret_cast<float2*>(dst + d + 2) = make_float2(a[2], a[3]); }      // (records of HD + 2 floats: 8-byte aligned only)
+    else *reinterpret_cast<float4*>(dst + d) = make_float4(a[0], a[1], a[2], a[3]);
+  }
+  if (splits > 1 && (tid & 7) == 0) { dst[HD] = M; dst[HD + 1] = L; }
 }
 
 // out[token][head] = sum of the K splits of a token tile, folded with a running maximum in split order (a tile walked by one
@@ -1838,65 +1876,61 @@ int launch_attn_step(cai_kv_s* kv, int layer, float* qkv, int64_t qkv_stride, in
     if (!prompt_rows && !grouped) { p.qn_gain = qn_gain; p.kn_gain = kn_gain; p.qk_eps = qk_eps; }
     else if ((rc = launch_rmsnorm_pair(qkv, qn_gain, qw, kn_gain, kw, n_seq, qk_eps, qkv_stride))) return rc;
   }
-  // prompts over a 128- or 64-wide cache: matrix-core kernel, 32 tokens x 4 heads per work-group
+  // prompts over a 128- or 64-wide cache: matrix-core kernel, 32 tokens of a head per work-group
   const bool flash = prompt_rows == 1 && attn_prompt_is_flash(kv, n_seq);
-  const bool rows_fused = flash && kv->dtype != CAI_KV_I8;     // the append and the q planes share a launch (below)
   if (prompt_rows && kv->dtype == CAI_KV_I8) {
     if (p.hd <= 32) hipLaunchKernelGGL(kv_append_rows_i8_kernel<1>, dim3(n_seq), dim3(256), 0, c.stream, p);
     else if (p.hd <= 64) hipLaunchKernelGGL(kv_append_rows_i8_kernel<2>, dim3(n_seq), dim3(256), 0, c.stream, p);
     else hipLaunchKernelGGL(kv_append_rows_i8_kernel<4>, dim3(n_seq), dim3(256), 0, c.stream, p);
-  } else if (prompt_rows && !rows_fused) {
+  } else if (prompt_rows && !flash) {        // (prompt_rows_kernel appends by itself)
     if (kv->dtype == CAI_KV_F16) hipLaunchKernelGGL(kv_append_rows_kernel<__half>, dim3(n_seq), dim3(256), 0, c.stream, p);
     else hipLaunchKernelGGL(kv_append_rows_kernel<float>, dim3(n_seq), dim3(256), 0, c.stream, p);
   }
   if (flash) {
-    const size_t need = (size_t)n_seq * q_heads * p.hd;
+    if (kv->prompt_end < n_seq || kv->prompt_end > kv->max_ctx) return set_error(CAI_ERR_STATE, "attention: a prompt of %d rows ends at row %d of %d", n_seq, kv->prompt_end, kv->max_ctx);
+    const int tok_tiles = (n_seq + 31) / 32, n_tiles = (kv->prompt_end + 31) / 32;
+    // K splits per token tile: a work-group takes a CU's half, so the range is cut where that shortens (rounds of work-groups) / splits by a fifth or more, and
+    // never to less than two tiles a wave.  Three layers of the 28 / 4 heads shape, whole prompts: 16 tokens behind 4096 rows 387 us uncut, 249 in eight; 300 behind 7000
+    // 855, 699 in three; 64 behind 2000 325, 277; a single tile a wave (a limit of four tiles a work-group) changes nothing at 28 / 4.
+    int n_ks = 1;
+    auto rounds = [&](int k) { return (tok_tiles * q_heads * k + 2 * c.n_cu - 1) / (2 * c.n_cu) / (double)k; };
+    for (int k = 2; k <= std::min(PA_KS_MAX, n_tiles / PA_KT_MIN); k++) if (rounds(k) <= 0.8 * rounds(n_ks)) n_ks = k;
+    // One piece of memory: q's planes, their scales, the cached rows' planes (as large as the rows are as floats or halfs, of one layer and
+    // sequence) and scales, the pieces' sums.  Tiles are counted up to a power of two, so that the chunks of a long prompt find it large enough.
+    const int np = p.hd == 64 ? (kv->dtype == CAI_KV_F32 ? 2 : 1) : (kv->dtype == CAI_KV_F16 ? 1 : 2);
+    int most = 16; while (most < n_tiles) most *= 2;
+    most = std::min(most, (kv->max_ctx + 31) / 32);
+    const size_t q_b = (size_t)n_seq * q_heads * p.hd * 2, s_b = ((size_t)n_seq * q_heads * 4 + 255) / 256 * 256;
+    const size_t t_b = (size_t)most * kv->kv_heads * (4 * np * 32 * p.hd), r_b = (size_t)most * kv->kv_heads * 256;
+    const size_t need = 2 * q_b + s_b + t_b + r_b + (n_ks > 1 ? (size_t)n_seq * q_heads * n_ks * (p.hd + 2) * 4 : 0);
     if (need > kv->pq_cap) {
       CAI_HIP(hipStreamSynchronize(c.stream));
-      if (kv->pq_hi) (void)hipFree(kv->pq_hi);
-      if (kv->pq_lo) (void)hipFree(kv->pq_lo);
-      kv->pq_hi = kv->pq_lo = nullptr; kv->pq_cap = 0;
-      CAI_HIP(hipMalloc(&kv->pq_hi, need * 2));
-      CAI_HIP(hipMalloc(&kv->pq_lo, need * 2 + need / p.hd * 4));
+      if (kv->pq) (void)hipFree(kv->pq);
+      kv->pq = nullptr; kv->pq_cap = 0;
+      CAI_HIP(hipMalloc(&kv->pq, need));
       kv->pq_cap = need;
     }
     PromptParams pp{};
-    pp.qkv = qkv; pp.qkv_stride = qkv_stride; pp.qhi = (_Float16*)kv->pq_hi; pp.qlo = (_Float16*)kv->pq_lo;
-    pp.qsc = (float*)(pp.qlo + kv->pq_cap);
+    char* ws = (char*)kv->pq;
+    pp.qkv = qkv; pp.qkv_stride = qkv_stride; pp.qhi = (_Float16*)ws; pp.qlo = (_Float16*)(ws + q_b);
+    pp.qsc = (float*)(ws + 2 * q_b); pp.planes = (_Float16*)(ws + 2 * q_b + s_b); pp.rsc = (float*)(ws + 2 * q_b + s_b + t_b); pp.part = (float*)(ws + 2 * q_b + s_b + t_b + r_b);
     const size_t plane = ((size_t)seq0 * kv->seq_elems() + (size_t)layer * kv->layer_elems()) * kv->elem();
-    pp.kc = (const char*)kv->k + plane; pp.vc = (const char*)kv->v + plane;
+    pp.kc = (char*)kv->k + plane; pp.vc = (char*)kv->v + plane;
     if (kv->dtype == CAI_KV_I8) {
       const size_t rows0 = (size_t)seq0 * kv->seq_rows() + (size_t)layer * kv->layer_rows();
       pp.ksc = kv->ks + rows0; pp.vsc = kv->vs + rows0;
     }
-    pp.q_heads = q_heads; pp.kv_heads = kv->kv_heads; pp.max_ctx = kv->max_ctx; pp.n_tok = n_seq; pp.window = window;
-    pp.softcap = softcap; pp.inv_sqrt = p.inv_sqrt; pp.theta = theta; pp.pos = pos_dev; pp.out = out; pp.out_stride = out_stride;
-    const int G = q_heads / kv->kv_heads;
-    const int wgs = ((n_seq + 31) / 32) * kv->kv_heads * ((G + 3) / 4);
-    // K splits per token tile: as many as keep the launch at one work-group per CU (a tile with few K tiles takes fewer).
-    // Measured on 511 tokens of the 7B shape (128 work-groups unsplit): 67 us -> 38.7 + 11.2 us (merge) with two splits,
-    // 50.8 + 11.6 with three; on 512-token chunks of the 32B shape (256 work-groups) splitting loses (365 -> 373 + 16 us).
-    const int n_ks = std::max(1, std::min(PA_KS_MAX, c.n_cu / wgs));
-    if (n_ks > 1) {
-      const size_t pneed = (size_t)n_seq * q_heads * n_ks * (p.hd + 2);
-      if (pneed > kv->pq_part_cap) {
-        CAI_HIP(hipStreamSynchronize(c.stream));
-        if (kv->pq_part) (void)hipFree(kv->pq_part);
-        kv->pq_part = nullptr; kv->pq_part_cap = 0;
-        CAI_HIP(hipMalloc((void**)&kv->pq_part, pneed * 4));
-        kv->pq_part_cap = pneed;
-      }
-    }
-    pp.part = kv->pq_part;
-    const dim3 grid((n_seq + 31) / 32, kv->kv_heads * ((G + 3) / 4), n_ks);
+    pp.q_heads = q_heads; pp.kv_heads = kv->kv_heads; pp.max_ctx = kv->max_ctx; pp.n_tok = n_seq; pp.n_tiles = n_tiles; pp.window = window;
+    pp.softcap = softcap; pp.inv_sqrt = p.inv_sqrt; pp.theta = theta; pp.pos0 = kv->prompt_end - n_seq; pp.out = out; pp.out_stride = out_stride;
+    const dim3 rows(n_tiles * kv->kv_heads + n_seq), grid(q_heads, tok_tiles, n_ks);
     auto go = [&](auto hd_) {
       constexpr int HD = hd_;
-      if (!rows_fused) hipLaunchKernelGGL(prompt_q_kernel<HD>, dim3(n_seq), dim3(256), 0, c.stream, pp);
-      else if (kv->dtype == CAI_KV_F16) hipLaunchKernelGGL((prompt_rows_kernel<__half, HD>), dim3(n_seq), dim3(256), 0, c.stream, p, pp);
-      else hipLaunchKernelGGL((prompt_rows_kernel<float, HD>), dim3(n_seq), dim3(256), 0, c.stream, p, pp);
-      if (kv->dtype == CAI_KV_F16) hipLaunchKernelGGL((attn_prompt_kernel<__half, HD>), grid, dim3(256), 0, c.stream, pp);
-      else if (kv->dtype == CAI_KV_I8) hipLaunchKernelGGL((attn_prompt_kernel<int8_t, HD>), grid, dim3(256), 0, c.stream, pp);
-      else hipLaunchKernelGGL((attn_prompt_kernel<float, HD>), grid, dim3(256), 0, c.stream, pp);
+      auto both = [&](auto kv_) {
+        using KV_T = decltype(kv_);
+        hipLaunchKernelGGL((prompt_rows_kernel<KV_T, HD>), rows, dim3(256), 0, c.stream, pp);
+        hipLaunchKernelGGL((attn_prompt_kernel<KV_T, HD>), grid, dim3(256), 0, c.stream, pp);
+      };
+      if (kv->dtype == CAI_KV_F16) both(__half()); else if (kv->dtype == CAI_KV_I8) both(int8_t()); else both(float());
       if (n_ks > 1) hipLaunchKernelGGL(prompt_merge_kernel<HD>, dim3(n_seq, (q_heads + 3) / 4), dim3(512), 0, c.stream, pp, n_ks);
     };
     if (p.hd == 64) go(std::integral_constant<int, 64>()); else go(std::integral_constant<int, 128>());
@@ -2006,10 +2040,8 @@ void kv_free(cai_kv_s* kv)
   if (kv->ks) (void)hipFree(kv->ks);
   if (kv->vs) (void)hipFree(kv->vs);
   kv->ks = kv->vs = nullptr;
-  if (kv->pq_hi) (void)hipFree(kv->pq_hi);
-  if (kv->pq_lo) (void)hipFree(kv->pq_lo);
-  if (kv->pq_part) (void)hipFree(kv->pq_part);
-  kv->pq_hi = kv->pq_lo = nullptr; kv->pq_cap = 0; kv->pq_part = nullptr; kv->pq_part_cap = 0;
+  if (kv->pq) (void)hipFree(kv->pq);
+  kv->pq = nullptr; kv->pq_cap = 0;
   if (kv->part) (void)hipFree(kv->part);
   if (kv->d_len) (void)hipFree(kv->d_len);
   if (kv->merge_cnt) (void)hipFree(kv->merge_cnt);

@@ -1093,7 +1093,7 @@ extern "C" int cai_decoder_prefill(cai_decoder_t d, int seq, const int32_t* toke
       for (int i = 0; i < m; i++) { tp[i] = tokens[t0 + i]; tp[d->pf_cap + i] = pos0 + t0 + i; }
       CAI_HIP(hipMemcpyAsync(d->ptokpos, tp.data(), tp.size() * sizeof(int32_t), hipMemcpyHostToDevice, cx.stream));
       CAI_HIP(hipStreamSynchronize(cx.stream));
-      d->kv.geo_rows = kv_bucket_rows(&d->kv, pos0 + t0 + m);
+      d->kv.geo_rows = kv_bucket_rows(&d->kv, pos0 + t0 + m); d->kv.prompt_end = pos0 + t0 + m;
       if ((rc = ensure_ppart(d, pos0 + t0 + m, m))) return rc;
       if ((rc = enqueue_prefill_chunk(d, seq, m))) return rc;
       CAI_HIP(hipGetLastError());

@@ -446,6 +446,26 @@ def test_prompt_attention_of_64_wide_heads_on_matrix_cores(kv, window, hq, hkv):
     dec.close()
 
 
+@pytest.mark.parametrize("kv,window,hq,hkv", [("f32", 0, 7, 1), ("f16", 0, 3, 3), ("i8", 0, 4, 2), ("f32", 300, 4, 4), ("f16", 70, 5, 1)])
+@pytest.mark.parametrize("before,n", [(0, 8), (0, 31), (0, 33), (31, 34), (256, 129), (610, 20), (1210, 70)])
+def test_prompt_attention_of_128_wide_heads_behind_cached_rows(kv, window, hq, hkv, before, n):
+    """One token tile and a row more or less, fewer tiles than waves, ranges that start inside a tile, pieces of a range that are added afterwards
+    (20 tokens behind 610 rows): equal to the same rows in pieces of seven, which go to the per-row kernels.  Cached elements on the edge between two halfs
+    (2^-11) or codes may land one apart."""
+    from helpers.device import dev, rel_err
+    cai = dev()
+    cfg = dict(n_layers=2, d_model=256, n_q_heads=hq, n_kv_heads=hkv, head_dim=128, ffn=256, vocab=300, max_ctx=1300, eps=1e-5, rope_theta=1e4, window=window)
+    dec = cai.Decoder(synthetic_spec(cfg, O.Q8_0, head_qtype=O.Q8_0, seed=hq, std=0.05, qkv_bias=True), max_batch=2, kv_dtype={"f32": cai.KV_F32, "f16": cai.KV_F16, "i8": cai.KV_I8}[kv])
+    toks = np.random.default_rng(before + n).integers(0, 300, before + n).astype(np.int32)
+    for p in range(0, before + n, 7):
+        _, want = dec.prefill(toks[p:p + 7], p, seq=0)
+    if before:
+        dec.prefill(toks[:before], 0, seq=1)
+    _, got = dec.prefill(toks[before:], before, seq=1)
+    assert rel_err(got, want) < {"f32": 2e-5, "f16": 1e-3, "i8": 5e-3}[kv]
+    dec.close()
+
+
 @pytest.mark.parametrize("kv,gain,std_qk,std_v,std_o", [("f32", 1e-4, 600.0, 0.05, 60.0), ("f32", 2e4, 5e-6, 0.4, 1e-5), ("i8", 2e4, 5e-6, 0.4, 1e-5), ("f16", 1e-4, 600.0, 600.0, 6e-3)])
 def test_prompt_attention_of_64_wide_heads_at_any_size_of_its_values(kv, gain, std_qk, std_v, std_o):
     """values of 1e-5 and of 1e5, the latter past the largest half, with scores of ordinary size; the attention's output outweighs the stream.
