@@ -36,6 +36,7 @@ struct WideParams {
   // The first n_whole tiles are one work-group each; the width of the others is cut into n_splits slices, which leave their sums in
   // part[tile - n_whole][slice][token of the tile][row of the tile]
   int n_whole, n_splits; float* part;
+  int sum_wide;                              // gemm_wide_sum: four rows of a result lie on 16 bytes, and so do their bias and residual
 };
 
 __device__ __forceinline__ void wide_store(const WideParams& p, const float* bias, int64_t o, int row, float v)
@@ -72,7 +73,7 @@ __device__ __forceinline__ half2_w pk_codes(uint32_t v, uint32_t sel, half2_w s2
 // whose arrival the compiler would wait for, and the waits count the copies.  The copies are what costs most beside the MFMAs: with 128
 // rows a work-group needs 32 KB of activations for half the products, 37888 x 3584 x 2048 tokens took 1370 us instead of 1213
 // (useful 398 and 458 TFLOP/s; a library product of 4096 f16 rows, the same MFMAs, takes 874 us).  x 511 tokens, by launch: 286 us beside 7.6 for the
-// planes and 9.6 for the sums of cut tiles, the kernel of narrow tiles 369; 3584 x 18944 143 + 24 + 8.5 us, 229 + 24.
+// planes and 8.3 for the sums of cut tiles, the kernel of narrow tiles 369; 3584 x 18944 143 + 24 + 8.5 us, 229 + 24.
 template <int QT, int TT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_wide_pf(const WideParams p)
 {
@@ -299,39 +300,70 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
 }
 
-// the slices of a cut tile, added in order, and its results: a work-group takes eight tokens, a thread one row of the tile
+// The slices of a cut tile, added in order, and its results: a work-group takes eight tokens, a thread four rows of two of them (four up rows and
+// their gate rows of one).  What it reads was written on other XCDs, so it is bound by those round trips: eight slices are requested at once, and what is
+// added to the sums in front of them (one slice after another: 3584 rows x 511 tokens in four slices 12.0 us, 8.3 so).
 template <int BN>
 __global__ __launch_bounds__(256) void gemm_wide_sum(const WideParams p)
 {
-  constexpr int BM = 256;
-  const int ci = blockIdx.x, r = threadIdx.x;
+  constexpr int BM = 256, AT_ONCE = 8;
+  const int ci = blockIdx.x, tid = threadIdx.x;
   int rg, ttile; wide_tile(p, p.n_whole + ci, rg, ttile);
   const float* bias = p.bias; int rows = p.rows, yo = 0, rgl = rg;
   if (p.n_seg > 1 && rg >= p.seg_end[0]) { bias = p.bias2[0]; yo = p.y_off2[0]; rgl = rg - p.seg_end[0]; rows = p.rows2[0]; }
   if (p.n_seg > 2 && rg >= p.seg_end[1]) { bias = p.bias2[1]; yo = p.y_off2[1]; rgl = rg - p.seg_end[1]; rows = p.rows2[1]; }
-  const int half = p.swiglu_half, row = half ? rgl * (BM / 2) + (r & 127) : rgl * BM + r, t0 = blockIdx.y * 8;
-  const float* src = p.part + (int64_t)ci * p.n_splits * (BN * BM) + r;
-  float v[8];
+  const int half = p.swiglu_half, r = half ? 4 * (tid & 31) : 4 * (tid & 63), row = half ? rgl * (BM / 2) + r : rgl * BM + r;
+  int tl[2], last = p.n_tok - 1 - ttile * BN;                        // tokens of the tile
+  tl[0] = blockIdx.y * 8 + (half ? tid >> 5 : tid >> 6); tl[1] = tl[0] + (half ? 0 : 4);
+  float si[2]; float4 extra[2];
+  const bool wide = p.sum_wide && row < (half ? half : rows);
 #pragma unroll
-  for (int k = 0; k < 8; k++) v[k] = 0.0f;
-  for (int s = 0; s < p.n_splits; s++)
+  for (int u = 0; u < 2; u++) {
+    const int t = ttile * BN + min(tl[u], last);
+    si[u] = p.sinv[t];
+    extra[u] = wide && p.residual ? *reinterpret_cast<const float4*>(p.residual + (int64_t)t * p.y_stride + yo + row) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  }
+  const float* src = p.part + (int64_t)ci * p.n_splits * (BN * BM);
+  const float* at[2] = {src + min(tl[0], last) * BM + r, src + min(tl[1], last) * BM + r + (half ? BM / 2 : 0)};
+  float4 v[2] = {make_float4(0.0f, 0.0f, 0.0f, 0.0f), make_float4(0.0f, 0.0f, 0.0f, 0.0f)};
+  for (int s = 0; s < p.n_splits; s += AT_ONCE) {
+    float4 a[AT_ONCE][2];
 #pragma unroll
-    for (int k = 0; k < 8; k++) v[k] += src[(int64_t)s * (BN * BM) + min(t0 + k, p.n_tok - 1 - ttile * BN) * BM];
-  __shared__ float gate[8][128];
-  if (half) {
-    if (r >= 128)
+    for (int k = 0; k < AT_ONCE; k++)
+      if (k < 4 || s + 4 < p.n_splits)                               // (uniform)
 #pragma unroll
-      for (int k = 0; k < 8; k++) gate[k][r - 128] = v[k];
-    __syncthreads();
-    if (r >= 128) return;
+        for (int u = 0; u < 2; u++) a[k][u] = *reinterpret_cast<const float4*>(at[u] + (int64_t)min(s + k, p.n_splits - 1) * (BN * BM));
+#pragma unroll
+    for (int k = 0; k < AT_ONCE; k++)
+      if (s + k < p.n_splits)
+#pragma unroll
+        for (int u = 0; u < 2; u++) { v[u].x += a[k][u].x; v[u].y += a[k][u].y; v[u].z += a[k][u].z; v[u].w += a[k][u].w; }
   }
 #pragma unroll
-  for (int k = 0; k < 8; k++) {
-    const int t = ttile * BN + t0 + k;
-    if (t >= p.n_tok) break;
-    const float si = p.sinv[t];
-    if (half) { if (row < half) wide_store_pair(p, bias, (int64_t)t * p.y_stride + row, row, v[k] * si, gate[k][r] * si); }
-    else if (row < rows) wide_store(p, bias, (int64_t)t * p.y_stride + yo + row, row, v[k] * si);
+  for (int u = 0; u < 2; u++) { v[u].x *= si[u]; v[u].y *= si[u]; v[u].z *= si[u]; v[u].w *= si[u]; }
+  if (half) {
+    const int t = ttile * BN + tl[0];
+    if (t >= p.n_tok) return;
+    const float up[4] = {v[0].x, v[0].y, v[0].z, v[0].w}, gate[4] = {v[1].x, v[1].y, v[1].z, v[1].w};
+#pragma unroll
+    for (int i = 0; i < 4; i++) if (row + i < half) wide_store_pair(p, bias, (int64_t)t * p.y_stride + row + i, row + i, up[i], gate[i]);
+    return;
+  }
+#pragma unroll
+  for (int u = 0; u < 2; u++) {
+    const int t = ttile * BN + tl[u];
+    if (t >= p.n_tok) continue;
+    const int64_t o = (int64_t)t * p.y_stride + yo + row;
+    if (wide) {
+      float4 b = bias ? *reinterpret_cast<const float4*>(bias + row) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      if (bias) { v[u].x += b.x; v[u].y += b.y; v[u].z += b.z; v[u].w += b.w; }
+      if (p.residual) { v[u].x += extra[u].x; v[u].y += extra[u].y; v[u].z += extra[u].z; v[u].w += extra[u].w; }
+      *reinterpret_cast<float4*>(p.y + o) = v[u];
+    } else {
+      const float w[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+      for (int i = 0; i < 4; i++) if (row + i < rows) wide_store(p, bias, o + i, row + i, w[i]);
+    }
   }
 }
 
@@ -415,6 +447,9 @@ int launch_gemm_wide(const cai_qw_s* const* ws, const int* y_off, int n_w, const
     if (n_cut * p.n_splits > slots) return set_error(CAI_ERR_INVALID, "prompt gemm: %d tiles cut into %d slices for %d work-groups", n_cut, p.n_splits, slots);
     const int rc = wide_reserve(); if (rc) return rc;
     p.part = g_wide_part;
+    uintptr_t low = (uintptr_t)p.y | (uintptr_t)residual | (uintptr_t)(y_stride * 4);
+    for (int i = 0; i < n_w; i++) low |= (uintptr_t)ws[i]->bias | (uintptr_t)(ws[i]->rows * 4) | (uintptr_t)(i ? p.y_off2[i - 1] : 0) * 4;
+    p.sum_wide = !swiglu_half && (low & 15) == 0;
   }
   const bool q5 = ws[0]->qtype == CAI_Q5_K;
   const int rc = BN == 128 ? (q5 ? go_wide<CAI_Q5_K, 2>(p) : go_wide<CAI_Q4_K, 2>(p)) : (q5 ? go_wide<CAI_Q5_K, 1>(p) : go_wide<CAI_Q4_K, 1>(p));
