@@ -641,9 +641,14 @@ __global__ __launch_bounds__(256) void delta_finish_kernel(const DeltaDims d, co
 
 // ------------------------------------------------------------------------------------------
 // decode: one token of each entry, one work-group per (head, row): low-rank seconds, convolutions, unit norms, decay, the state
-// update, output norm and gate.  The state is requested first and sits in registers while the rest is made.
+// update, output norm and gate.
+// What bounds it: round trips (a state of 64 KB is 1 us of a CU).  Everything is requested before the first value is used, in the order of its use - what lies at
+// known places, then what needs the row's slot and position, the state last - and without a condition that would make a wait count the state's
+// requests too.  (Taps and low-rank rows requested as they came to their use: four rows of 16 heads 9.6 us, 8.2 so.)
+// TAPS: of the convolutions (0: any number, requested one after another, and heads of more than 128 channels, whose four a lane take too many registers).
 // ------------------------------------------------------------------------------------------
-template <typename AT, int RPT>
+constexpr int SINGLE_LOW = 2, SINGLE_QUADS = 13 * 16;      // low-rank rows a quad has requested ahead; quads of waves 3 .. 15
+template <typename AT, int RPT, int TAPS>
 __global__ __launch_bounds__(1024) void delta_single_kernel(const DeltaDims d, const DeltaIn in, const DeltaW w, const uint16_t* a2, const int lda2, const uint16_t* g2, const int ldg2,
                                                             float* state, const int64_t s_elems, float* hist, const int64_t h_elems, const StepRows r, AT* out, const int64_t ldo, const int ct_log)
 {
@@ -659,82 +664,153 @@ __global__ __launch_bounds__(1024) void delta_single_kernel(const DeltaDims d, c
   const int CT = 1 << ct_log, CP = CT * 4, RG = 1024 >> ct_log, ct = tid & (CT - 1), rg = tid >> ct_log;
   const int dvp = d.vdim_p();
   float* Sg = state + slot * s_elems + (int64_t)h * d.dim * dvp;
-  f32x4 S[RPT];
-  auto load_state = [&](int c0) {
-#pragma unroll
-    for (int j = 0; j < RPT; j++) {
-      const int rr = rg + j * RG;
-      S[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      if (pos > 0 && rr < d.dim && c0 + ct * 4 < dvp) S[j] = *reinterpret_cast<const f32x4*>(Sg + (unsigned)(rr * dvp + c0 + ct * 4));
-    }
-  };
-  load_state(0);
   const float* p = in.proj + row * in.ldp;
   float* ring = hist + slot * h_elems;
   float* ring_now = ring + (int64_t)(pos % d.taps) * C;
-  for (int i = tid; i < d.rank_a; i += 1024) sra[i] = p[in.oa + i];
-  for (int i = tid; i < d.rank_g; i += 1024) srg[i] = p[in.og + i];
-  if (d.rank_a || d.rank_g) __syncthreads();
-  if (wave < 2) {                                        // q (wave 0) and k (wave 1): convolution and unit norm
-    const int oc = wave ? in.ok : in.oq, hc = wave ? kw : 0;
-    const float* cw = wave ? w.ck : w.cq;
-    float v[4], s = 0.0f;
+  const float ra = tid < d.rank_a ? p[in.oa + tid] : 0.0f, rgv = tid < d.rank_g ? p[in.og + tid] : 0.0f;      // (ranks of at most 512)
+  const float beta_z = p[in.ob + h];
+
+  // q (wave 0), k (wave 1) and v (wave 2): channels lane + 64 i of the head; the other waves: low-rank rows of decay and gate, four lanes a row
+  const int oc = wave == 0 ? in.oq : wave == 1 ? in.ok : in.ov, hc = wave == 0 ? 0 : wave == 1 ? kw : 2 * kw, n_ch = wave == 2 ? d.vdim : d.dim, c0h = wave == 2 ? h * d.vdim : g * d.dim;
+  const float* const cw = wave == 0 ? w.cq : wave == 1 ? w.ck : w.cv;
+  constexpr int T = TAPS ? TAPS : 2, NC = TAPS ? 2 : 4;
+  float x[NC], taps[NC][T], past[NC][T - 1], gain[NC];
+  const int nd = d.channel_decay ? d.dim : 1, quad = (tid - 192) >> 2, ql = tid & 3;
+  const bool ahead = d.rank_a && d.rank_g && d.rank_a <= 128 && d.rank_g <= 128 && nd + d.vdim <= SINGLE_LOW * SINGLE_QUADS;
+  u32x4 low_m[SINGLE_LOW][4]; float low_b[SINGLE_LOW];
+  if (wave < 3) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int c = lane + 64 * i, ch = g * d.dim + c;
-      v[i] = c < d.dim ? conv_silu(p + oc, in.ldp, 0, pos, ring, C, hc, cw, d.taps, ch) : 0.0f;
+    for (int i = 0; i < NC; i++) {
+      const int c = c0h + min(lane + 64 * i, n_ch - 1);
+      x[i] = p[oc + c];
+      if constexpr (TAPS != 0)
+#pragma unroll
+        for (int k = 0; k < T; k++) taps[i][k] = cw[c * T + k];
+      gain[i] = w.norm[min(lane + 64 * i, d.vdim - 1)];
+    }
+  } else if (ahead) {
+#pragma unroll
+    for (int u = 0; u < SINGLE_LOW; u++) {
+      const int i = min(quad + u * SINGLE_QUADS, nd + d.vdim - 1);
+      const uint16_t* m = i < nd ? a2 + (int64_t)(h * nd + i) * lda2 : g2 + (int64_t)(h * d.vdim + i - nd) * ldg2;
+      const int ld = i < nd ? lda2 : ldg2;
+#pragma unroll
+      for (int k = 0; k < 4; k++) low_m[u][k] = *reinterpret_cast<const u32x4*>(m + (ql * 8 + 32 * k < ld ? ql * 8 + 32 * k : 0));
+      low_b[u] = w.dt_bias[h * nd + min(i, nd - 1)];
+    }
+  }
+  const float rate = w.rate[h];
+  asm volatile("" ::: "memory");
+  if (TAPS != 0 && wave < 3)
+#pragma unroll
+    for (int i = 0; i < NC; i++)
+#pragma unroll
+      for (int j = 1; j < T; j++) past[i][j - 1] = ring[(int64_t)((pos + T - j) % T) * C + hc + c0h + min(lane + 64 * i, n_ch - 1)];
+  asm volatile("" ::: "memory");
+  f32x4 S[RPT];
+  auto load_state = [&](int c0) {
+#pragma unroll
+    for (int j = 0; j < RPT; j++) S[j] = *reinterpret_cast<const f32x4*>(Sg + (unsigned)(min(rg + j * RG, d.dim - 1) * dvp + min(c0 + ct * 4, dvp - 4)));
+  };
+  auto keep_state = [&](int c0) {                        // what this thread holds of a state that there is
+#pragma unroll
+    for (int j = 0; j < RPT; j++)
+      if (!(pos > 0 && rg + j * RG < d.dim && c0 + ct * 4 < dvp)) S[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  };
+  load_state(0);
+  asm volatile("" ::: "memory");
+  if (tid < d.rank_a) sra[tid] = ra;
+  if (tid < d.rank_g) srg[tid] = rgv;
+  if (d.rank_a || d.rank_g) {                            // (waits for LDS only: the other requests stay on their way)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  }
+  if (wave < 3) {
+    float v[NC], s = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NC; i++) {
+      const int c = lane + 64 * i;
+      v[i] = 0.0f;
+      if (c >= n_ch) continue;
+      if constexpr (TAPS != 0) {
+        float t = fmaf(taps[i][T - 1], x[i], 0.0f);
+#pragma unroll
+        for (int j = 1; j < T; j++) t = fmaf(taps[i][T - 1 - j], j <= pos ? past[i][j - 1] : 0.0f, t);
+        v[i] = t * sigmoid_f(t);
+      } else v[i] = conv_silu(p + oc, in.ldp, 0, pos, ring, C, hc, cw, d.taps, c0h + c);
       s = fmaf(v[i], v[i], s);
     }
-    const float nrm = (wave ? 1.0f : rsqrtf((float)d.dim)) / sqrtf(wave_total(s) + 1e-6f);
-    float* dst = wave ? sk : sq;
+    if (wave < 2) {                                      // unit norm
+      const float nrm = (wave ? 1.0f : rsqrtf((float)d.dim)) / sqrtf(wave_total(s) + 1e-6f);
+      float* dst = wave ? sk : sq;
 #pragma unroll
-    for (int i = 0; i < 4; i++) dst[lane + 64 * i] = v[i] * nrm;
-    if (h % hg == 0) for (int c = lane; c < d.dim; c += 64) ring_now[hc + g * d.dim + c] = p[oc + g * d.dim + c];
-  } else if (wave < 4) {                                 // v
-    for (int c = tid - 128; c < d.vdim; c += 128) {
-      const int ch = h * d.vdim + c;
-      sv[c] = conv_silu(p + in.ov, in.ldp, 0, pos, ring, C, 2 * kw, w.cv, d.taps, ch);
-      ring_now[2 * kw + ch] = p[in.ov + ch];
-    }
-  } else {                                               // decay and gate, four lanes to a low-rank row
-    const int quad = (tid - 256) >> 2, ql = tid & 3, nd = d.channel_decay ? d.dim : 1, rate_i = h;
+      for (int i = 0; i < NC; i++) dst[lane + 64 * i] = v[i] * nrm;
+    } else
+#pragma unroll
+      for (int i = 0; i < NC; i++) if (lane + 64 * i < n_ch) sv[lane + 64 * i] = v[i];
+    if (wave == 2 || h % hg == 0)
+#pragma unroll
+      for (int i = 0; i < NC; i++) if (lane + 64 * i < n_ch) ring_now[hc + c0h + lane + 64 * i] = x[i];
+  } else {                                               // decay and gate
+    auto part = [&](float s, const u32x4 u, const float* v, int rank, int i) {      // (columns beyond the rank are zero in the matrix, the vector is guarded)
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        if (i + 2 * j < rank) s = fmaf(bf16_lo(u[j]), v[i + 2 * j], s);
+        if (i + 2 * j + 1 < rank) s = fmaf(bf16_hi(u[j]), v[i + 2 * j + 1], s);
+      }
+      return s;
+    };
+    auto quad_sum = [](float s) { s += __shfl_xor(s, 1); return s + __shfl_xor(s, 2); };
     auto low = [&](const uint16_t* m, int ld, const float* v, int rank, int rw) {
       float s = 0.0f;
       const uint16_t* mr = m + (int64_t)rw * ld;
-      for (int i = ql * 8; i < rank; i += 32) {          // (columns beyond the rank are zero in the matrix, the vector is guarded)
-        const u32x4 u = *reinterpret_cast<const u32x4*>(mr + i);
+      for (int i = ql * 8; i < rank; i += 32) s = part(s, *reinterpret_cast<const u32x4*>(mr + i), v, rank, i);
+      return quad_sum(s);
+    };
+    auto put = [&](int i, float z) {
+      if (ql != 0) return;
+      if (i < nd) sg[i] = expf(rate * softplus_f(z));
+      else { const float s = sigmoid_f(z); sgate[i - nd] = d.sigmoid_gate ? s : z * s; }
+    };
+    if (ahead) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-          if (i + 2 * j < rank) s = fmaf(bf16_lo(u[j]), v[i + 2 * j], s);
-          if (i + 2 * j + 1 < rank) s = fmaf(bf16_hi(u[j]), v[i + 2 * j + 1], s);
+      for (int u = 0; u < SINGLE_LOW; u++) {
+        const int i = quad + u * SINGLE_QUADS;
+        if (i >= nd + d.vdim) break;                     // (whole quads)
+        const bool decay = i < nd;
+        const float* v = decay ? sra : srg;
+        const int rank = decay ? d.rank_a : d.rank_g;
+        float s = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 4; k++) s = part(s, low_m[u][k], v, rank, ql * 8 + 32 * k);
+        s = quad_sum(s);
+        put(i, decay ? s + low_b[u] : s);
+      }
+    } else
+      for (int i = quad; i < nd + d.vdim; i += SINGLE_QUADS) {
+        if (i < nd) {
+          const int c = h * nd + i;
+          put(i, (d.rank_a ? low(a2, lda2, sra, d.rank_a, c) : p[in.oa + c]) + w.dt_bias[c]);
+        } else {
+          const int c = h * d.vdim + i - nd;
+          put(i, d.rank_g ? low(g2, ldg2, srg, d.rank_g, c) : p[in.og + c]);
         }
       }
-      s += __shfl_xor(s, 1); s += __shfl_xor(s, 2);
-      return s;
-    };
-    for (int i = quad; i < nd + d.vdim; i += 192) {
-      if (i < nd) {
-        const int c = h * nd + i;
-        const float z = (d.rank_a ? low(a2, lda2, sra, d.rank_a, c) : p[in.oa + c]) + w.dt_bias[c];
-        if (ql == 0) sg[i] = expf(w.rate[rate_i] * softplus_f(z));
-      } else {
-        const int c = h * d.vdim + i - nd;
-        const float z = d.rank_g ? low(g2, ldg2, srg, d.rank_g, c) : p[in.og + c];
-        if (ql == 0) { const float s = sigmoid_f(z); sgate[i - nd] = d.sigmoid_gate ? s : z * s; }
-      }
-    }
   }
   __syncthreads();
   if (wave == 0) {
     float s = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 4; i++) s = fmaf(sq[lane + 64 * i], sk[lane + 64 * i], s);
+    for (int i = 0; i < NC; i++) s = fmaf(sq[lane + 64 * i], sk[lane + 64 * i], s);
     s = wave_total(s);
     if (lane == 0) sc[0] = s;
   }
-  const float beta = sigmoid_f(p[in.ob + h]);
+  const float beta = sigmoid_f(beta_z);
   for (int c0 = 0; c0 < d.vdim; c0 += CP) {
     if (c0) load_state(c0);
+    keep_state(c0);
     f32x4 ks = {0.0f, 0.0f, 0.0f, 0.0f}, qd = ks;
 #pragma unroll
     for (int j = 0; j < RPT; j++) {
@@ -773,14 +849,14 @@ __global__ __launch_bounds__(1024) void delta_single_kernel(const DeltaDims d, c
   }
   __syncthreads();
   if (wave == 0) {
-    float o[4], s = 0.0f;
+    float o[NC], s = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 4; i++) { const int c = lane + 64 * i; o[i] = c < d.vdim ? so[c] : 0.0f; s = fmaf(o[i], o[i], s); }
+    for (int i = 0; i < NC; i++) { const int c = lane + 64 * i; o[i] = c < d.vdim ? so[c] : 0.0f; s = fmaf(o[i], o[i], s); }
     const float inv = 1.0f / sqrtf(wave_total(s) / (float)d.vdim + d.eps);
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < NC; i++) {
       const int c = lane + 64 * i;
-      if (c < d.vdim) out[row * ldo + h * d.vdim + c] = (AT)(o[i] * inv * w.norm[c] * sgate[c]);
+      if (c < d.vdim) out[row * ldo + h * d.vdim + c] = (AT)(o[i] * inv * gain[i] * sgate[c]);
     }
   }
 }
@@ -846,8 +922,9 @@ int delta_single(const DeltaDims& d, const DeltaIn& in, const DeltaW& w, const S
   const uint16_t* a2 = w.a2 ? (const uint16_t*)w.a2->data : nullptr; const uint16_t* g2 = w.g2 ? (const uint16_t*)w.g2->data : nullptr;
   const int la = w.a2 ? (int)w.a2->ld : 0, lg = w.g2 ? (int)w.g2->ld : 0;
   auto s = ctx().stream;
-#define SINGLE(AT, N) hipLaunchKernelGGL((delta_single_kernel<AT, N>), grid, blk, 0, s, d, in, w, a2, la, g2, lg, st.S, st.s_elems, st.hist, st.h_elems, r, (AT*)out, ldo, ct_log)
-#define SINGLE_N(AT) do { if (rpt <= 2) SINGLE(AT, 2); else if (rpt <= 4) SINGLE(AT, 4); else SINGLE(AT, 8); } while (0)
+#define SINGLE(AT, N, TAPS) hipLaunchKernelGGL((delta_single_kernel<AT, N, TAPS>), grid, blk, 0, s, d, in, w, a2, la, g2, lg, st.S, st.s_elems, st.hist, st.h_elems, r, (AT*)out, ldo, ct_log)
+  const bool ahead = d.taps == 4 && d.dim <= 128 && d.vdim <= 128;      // (four rows of the state a thread at most then)
+#define SINGLE_N(AT) do { if (ahead && rpt <= 2) SINGLE(AT, 2, 4); else if (ahead) SINGLE(AT, 4, 4); else if (rpt <= 2) SINGLE(AT, 2, 0); else if (rpt <= 4) SINGLE(AT, 4, 0); else SINGLE(AT, 8, 0); } while (0)
   if (act_t == ACT_T_BF16) SINGLE_N(bf16_t); else SINGLE_N(float);
 #undef SINGLE_N
 #undef SINGLE

@@ -177,6 +177,23 @@ def test_mechanism_alone(cai, tmp_path, mech, i, dt):
     dec.close()
 
 
+# Heads at the edges of what a lane and a quad have requested ahead: one and two channels a lane, low-rank rows of one piece, of all four, and of one more; more
+# rows than quads have places for (128 channels and 128 gates are 256 of 416)
+@pytest.mark.parametrize("h, g, d, dv, ra, rg", [(4, 2, 64, 64, 7, 11), (2, 1, 128, 128, 128, 127), (2, 2, 128, 128, 129, 33), (3, 1, 65, 70, 32, 128), (2, 1, 20, 126, 40, 8), (2, 1, 128, 130, 16, 16)])
+@pytest.mark.parametrize("mech", ["delta", "channel delta"])
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+def test_single_tokens(cai, tmp_path, mech, h, g, d, dv, ra, rg, dt):
+    """tokens one by one from the first on, where the convolutions reach in front of the text and the state is what an earlier sequence left"""
+    mixer = B.delta(h, g, d, dv, 4)
+    m = Model(tmp_path, B.config([B.layer(mixer if mech == "delta" else (B.attn(), mixer))], width=72, vocab=67), seed=d, edit=only(mech), rank_a=ra, rank_g=rg)
+    tok = m.tokens(24, dv)
+    dec = m.open(cai, 64, 1, dt)
+    feed(dec, m.tokens(9, 1), [9])
+    dec.reset()
+    check(feed(dec, tok, [1] * 7 + [9] + [1] * 8), m.ref(tok), dt)
+    dec.close()
+
+
 # Numbers of chunks of 16 that leave the walk's loop over three at each of its places, last chunks whole and ragged; key widths of 4, 8 and 16
 # tiles, value widths of whole and of ragged slices
 @pytest.mark.parametrize("n", [32, 33, 47, 48, 49, 64, 81])
