@@ -113,7 +113,38 @@ struct AttnParams {
   const float* qn_gain; const float* kn_gain; float qk_eps;   // full-width RMSNorm of q and of k applied while they are read (null: rows are used as they are)
   unsigned* merge_cnt;         // decode steps: arrival counters [seq][head]; the work-group that completes the last slice merges (null: a merge launch follows)
   unsigned long long* timeline; // stamps of this launch's work-groups (null: none)
+  BlkPlanes planes; bool planes_q8; // prompts: the results leave as planes (planes.hi null: as rows)
 };
+
+typedef _Float16 ph4_t __attribute__((ext_vector_type(4)));
+typedef _Float16 ph8_t __attribute__((ext_vector_type(8)));
+
+// A result of row t, column c of w, whose neighbours of a block of 32 columns are in the neighbouring lanes
+__device__ __forceinline__ void out_plane(const BlkPlanes& o, bool q8_0, int t, int c, int w, float y)
+{
+  float m = finite_abs(y);
+#pragma unroll
+  for (int k = 1; k < 32; k <<= 1) m = fmaxf(m, __shfl_xor(m, k));
+  const int e = plane_exponent(m);
+  _Float16 h, l; split_plane(y * ldexpf(1.0f, e), h, l);
+  const int64_t blk = (int64_t)(t >> 4) * (w >> 5) + (c >> 5), at = blk * 512 + plane_place(q8_0, t & 15, c & 31);
+  o.hi[at] = h; o.lo[at] = l;
+  if ((c & 31) == 0) o.scale[blk * 16 + (t & 15)] = ldexpf(1.0f, -e);
+}
+// Four of them, c .. c + 3: eight neighbouring lanes hold a block
+__device__ __forceinline__ void out_plane4(const BlkPlanes& o, bool q8_0, int t, int c, int w, const float (&y)[4])
+{
+  float m = fmaxf(fmaxf(finite_abs(y[0]), finite_abs(y[1])), fmaxf(finite_abs(y[2]), finite_abs(y[3])));
+#pragma unroll
+  for (int k = 1; k < 8; k <<= 1) m = fmaxf(m, __shfl_xor(m, k));
+  const int e = plane_exponent(m);
+  ph4_t h, l;
+#pragma unroll
+  for (int i = 0; i < 4; i++) { _Float16 a, b; split_plane(y[i] * ldexpf(1.0f, e), a, b); h[i] = a; l[i] = b; }
+  const int64_t blk = (int64_t)(t >> 4) * (w >> 5) + (c >> 5), at = blk * 512 + plane_place(q8_0, t & 15, c & 31);
+  *reinterpret_cast<ph4_t*>(o.hi + at) = h; *reinterpret_cast<ph4_t*>(o.lo + at) = l;
+  if ((c & 31) == 0) o.scale[blk * 16 + (t & 15)] = ldexpf(1.0f, -e);
+}
 
 // ---- merge of the split partials inside the split kernels ----
 // The slices of a head (or of a KV head's group of heads) finish in any order on any XCD.  Each work-group writes its partial
@@ -538,8 +569,6 @@ __global__ __launch_bounds__(256) void attn_group_kernel(const int32_t* hpos, co
 //                                     that one byte permute per word pair builds the operand of the even and of the odd dims.
 //      Every wave keeps its own maximum and sum per head; the four waves meet once, in LDS, and the slice partial has the
 //      same form as above.  Same contract and tolerance as the VALU kernels (1e-5 against the oracle). ----
-typedef _Float16 ph4_t __attribute__((ext_vector_type(4)));
-typedef _Float16 ph8_t __attribute__((ext_vector_type(8)));
 constexpr int GM_LD = 136;                         // halfs per staged row (128 + pad: 16-byte aligned, 4 rows apart = 16 banks apart)
 constexpr int GM_FIXED = 2 * 16 * GM_LD * 2 + 512 + 1024;  // q hi | q lo | new K,V row | per-wave maximum and sum
 constexpr int gm_lds_bytes(int tpw, int nw) { return GM_FIXED + nw * tpw * 16 * GM_LD * 2; }
@@ -871,7 +900,7 @@ __global__ __launch_bounds__(64 * NW) void attn_group_mfma_kernel(const int32_t*
 // ---- merge of the split partials: one work-group per query head.  Four quarter-groups of head_dim threads each take every
 //      fourth slice (all their loads go out together: one round trip for up to 32 slices per quarter), fold them with a running
 //      maximum, and meet in LDS. ----
-template <int MR>      // slices per quarter and round trip: 12, or 32 for long caches (130k rows = 508 slices: 4 dependent rounds instead of 11)
+template <int MR, bool PLANES>      // slices per quarter and round trip: 12, or 32 for long caches (130k rows = 508 slices: 4 dependent rounds instead of 11)
 __global__ __launch_bounds__(512) void attn_merge_kernel(const int32_t* hpos, const float* hpart, float* hout, const long long hout_stride,
                                                          const int hheads, const int hgeo, const int hsl, const AttnParams p)
 {
@@ -928,7 +957,9 @@ __global__ __launch_bounds__(512) void attn_merge_kernel(const int32_t* hpos, co
       const float e = qL[k] > 0.0f ? expf(qM[k] - Mx) : 0.0f;
       At = fmaf(qA[k][d], e, At); Lt = fmaf(qL[k], e, Lt);
     }
-    hout[(int64_t)seq * hout_stride + qh * hd + d] = Lt > 0.0f ? At * (1.0f / Lt) : 0.0f;
+    const float y = Lt > 0.0f ? At * (1.0f / Lt) : 0.0f;
+    if (PLANES) out_plane(p.planes, p.planes_q8, seq, qh * hd + d, h_q_heads * hd, y);
+    else hout[(int64_t)seq * hout_stride + qh * hd + d] = y;
   }
 }
 
@@ -950,10 +981,13 @@ __global__ __launch_bounds__(512) void attn_merge_kernel(const int32_t* hpos, co
 // 32 lanes a row, sums of five steps and two scalar reads, 64 rows cost 1.5 us (0.5 here); sine and cosine are worked out once a wave
 // and not once a group, the exponentials of the meeting once a lane.  More waves (8, 16 a work-group) took longer to start and to meet
 // (100 half rows of 128: 5.5 us with four, 6.3, 9.6; 200: 7.2, 7.2, 9.6).  NCH: chunks of 64 rows on their way at once.
-template <int VW, int NV, typename KV_T, int NCH, bool QN>
+// MODE: a step's rows as they are, with the norms of whole q and k rows, or a prompt's rows whose results leave as planes.
+enum { HEAD_PLAIN, HEAD_NORMED, HEAD_PLANES };
+template <int VW, int NV, typename KV_T, int NCH, int MODE>
 __global__ __launch_bounds__(256) void attn_split_head_kernel(const int32_t* hpos, const float* hqkv, const void* hk, const void* hv, const int hqkv_stride,
                                                                   const int hheads, const int hgeo, const int hsl, const int hmax_ctx, const int hseq_planes, const AttnParams p)
 {
+  constexpr bool QN = MODE == HEAD_NORMED;
   constexpr int DS = VW * NV, NG = 16;         // groups of 16 lanes, four waves: row j of the slice belongs to group j % NG
   const unsigned long long tl0 = timeline_now();
   const int q_heads = hheads & 0xffff, kv_heads = hheads >> 16, n_splits = hgeo & 0xffff, hd = hgeo >> 16;
@@ -1206,7 +1240,9 @@ __global__ __launch_bounds__(256) void attn_split_head_kernel(const int32_t* hpo
     const float Ls = (Lp[0] + Lp[1]) + (Lp[2] + Lp[3]), A = (Ap[0] + Ap[1]) + (Ap[2] + Ap[3]);
     const int qh = g * G + h;
     if (tid < hd && n_active == 1) {
-      p.out[(int64_t)seq * p.out_stride + qh * hd + d] = Ls > 0.0f ? A * (1.0f / Ls) : 0.0f;
+      const float y = Ls > 0.0f ? A * (1.0f / Ls) : 0.0f;
+      if (MODE == HEAD_PLANES) out_plane(p.planes, p.planes_q8, seq, qh * hd + d, q_heads * hd, y);
+      else p.out[(int64_t)seq * p.out_stride + qh * hd + d] = y;
     } else if (tid < hd) {
       float* pt = p.part + (((int64_t)seq * p.q_heads + qh) * p.n_splits + split) * (hd + 2);
       if (p.merge_cnt) { part_store(pt + d, A); if (d == 0) { part_store(pt + hd, M); part_store(pt + hd + 1, Ls); } }
@@ -1240,9 +1276,13 @@ static int launch_split_head(const AttnParams& p0, int n_seq, hipStream_t st)
     constexpr int VW = decltype(vw)::value, NV = decltype(nv)::value;
     // a slice of up to 64 rows is one chunk; longer ones have 128 rows on their way (256: 0.1 us less at 200 rows, 0.5 more at 100)
     constexpr int LONG = 2;
-    if (p.split_len <= 64) { if (p.qn_gain) put(attn_split_head_kernel<VW, NV, KV_T, 1, true>); else put(attn_split_head_kernel<VW, NV, KV_T, 1, false>); }
-    else if (p.qn_gain) put(attn_split_head_kernel<VW, NV, KV_T, LONG, true>);
-    else put(attn_split_head_kernel<VW, NV, KV_T, LONG, false>);
+    auto of = [&](auto mode) {
+      constexpr int MODE = decltype(mode)::value;
+      if (p.split_len <= 64) put(attn_split_head_kernel<VW, NV, KV_T, 1, MODE>); else put(attn_split_head_kernel<VW, NV, KV_T, LONG, MODE>);
+    };
+    if (p.qn_gain) of(std::integral_constant<int, HEAD_NORMED>());
+    else if (p.planes.hi) of(std::integral_constant<int, HEAD_PLANES>());
+    else of(std::integral_constant<int, HEAD_PLAIN>());
   };
   using std::integral_constant;
   if (p.hd > 64) go(integral_constant<int, 4>(), integral_constant<int, 2>());       // (widths past 64 are whole fours, all are even)
@@ -1446,6 +1486,7 @@ struct PromptParams {
   float* out; int64_t out_stride;
   float* part;                               // [token][q_head][K split][HD + 2]: unnormalised sums, maximum, normaliser
   float* qsc;                                // HD = 64: [token][q_head] what the head's planes are to be multiplied by
+  BlkPlanes planes_out; bool planes_q8;      // the results leave as planes of the next product (planes_out.hi null: as rows)
 };
 
 template <typename KV_T, int HD> struct PromptShape {
@@ -1798,6 +1839,7 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(const PromptParams 
       a[u] *= inv;
     }
     if (splits > 1) { *reinterpret_cast<float2*>(dst + d) = make_float2(a[0], a[1]); *reinterpret_cast<float2*>(dst + d + 2) = make_float2(a[2], a[3]); }      // (records of HD + 2 floats: 8-byte aligned only)
+    else if (p.planes_out.hi) out_plane4(p.planes_out, p.planes_q8, t, head * HD + d, p.q_heads * HD, a);
     else *reinterpret_cast<float4*>(dst + d) = make_float4(a[0], a[1], a[2], a[3]);
   }
   if (splits > 1 && (tid & 7) == 0) { dst[HD] = M; dst[HD + 1] = L; }
@@ -1824,7 +1866,9 @@ __global__ __launch_bounds__(512) void prompt_merge_kernel(const PromptParams p,
       A = A * c0 + as[s] * c1; L = L * c0 + ls[s] * c1; M = mn;
     }
   }
-  p.out[(int64_t)tok * p.out_stride + head * HD + d] = L > 0.0f ? A * (1.0f / L) : 0.0f;
+  const float y = L > 0.0f ? A * (1.0f / L) : 0.0f;
+  if (p.planes_out.hi) out_plane(p.planes_out, p.planes_q8, tok, head * HD + d, p.q_heads * HD, y);
+  else p.out[(int64_t)tok * p.out_stride + head * HD + d] = y;
 }
 
 // Whether n prompt rows of this cache go to the matrix-core prompt kernel (it needs no per-slice partial results).
@@ -1837,9 +1881,18 @@ bool attn_prompt_is_flash(const cai_kv_s* kv, int n)
   return flash_on && kv->evict_cap == 0 && ((kv->head_dim == 128 && n >= 8) || (kv->head_dim == 64 && n >= 256));
 }
 
+bool attn_rows_for_product(const cai_kv_s* kv, int seq, int layer, int n, const float* theta, const int32_t* pos, KvRows& out)
+{
+  if (kv->dtype == CAI_KV_I8 || kv->evict_cap > 0 || (kv->head_dim & 1) || attn_prompt_is_flash(kv, n)) return false;      // (those take them by themselves, or quantise whole rows)
+  const size_t at = ((size_t)seq * kv->seq_elems() + (size_t)layer * kv->layer_elems()) * kv->elem();
+  out.k = (char*)kv->k + at; out.v = (char*)kv->v + at; out.half = kv->dtype == CAI_KV_F16; out.head_dim = kv->head_dim; out.max_ctx = kv->max_ctx;
+  out.theta = theta; out.pos = pos;
+  return true;
+}
+
 int launch_attn_step(cai_kv_s* kv, int layer, float* qkv, int64_t qkv_stride, int n_seq, int q_heads, int window,
                      float softcap, const float* theta, const int32_t* pos_dev, float* out, int64_t out_stride, int seq0,
-                     int prompt_rows, float* prompt_part, const float* qn_gain, const float* kn_gain, float qk_eps)
+                     int prompt_rows, float* prompt_part, const float* qn_gain, const float* kn_gain, float qk_eps, AttnOnPlanes* on_planes)
 {
   Context& c = ctx();
   if (layer < 0 || layer >= kv->n_layers) return set_error(CAI_ERR_INVALID, "attention: layer %d of %d", layer, kv->n_layers);
@@ -1878,7 +1931,9 @@ int launch_attn_step(cai_kv_s* kv, int layer, float* qkv, int64_t qkv_stride, in
   }
   // prompts over a 128- or 64-wide cache: matrix-core kernel, 32 tokens of a head per work-group
   const bool flash = prompt_rows == 1 && attn_prompt_is_flash(kv, n_seq);
-  if (prompt_rows && kv->dtype == CAI_KV_I8) {
+  if (on_planes && on_planes->planes.hi && (flash || (!grouped && p.hd % 32 == 0))) { p.planes = on_planes->planes; p.planes_q8 = on_planes->q8_0; on_planes->planes_done = true; }
+  if (on_planes && on_planes->appended) {}      // (by the product that made them)
+  else if (prompt_rows && kv->dtype == CAI_KV_I8) {
     if (p.hd <= 32) hipLaunchKernelGGL(kv_append_rows_i8_kernel<1>, dim3(n_seq), dim3(256), 0, c.stream, p);
     else if (p.hd <= 64) hipLaunchKernelGGL(kv_append_rows_i8_kernel<2>, dim3(n_seq), dim3(256), 0, c.stream, p);
     else hipLaunchKernelGGL(kv_append_rows_i8_kernel<4>, dim3(n_seq), dim3(256), 0, c.stream, p);
@@ -1921,7 +1976,7 @@ int launch_attn_step(cai_kv_s* kv, int layer, float* qkv, int64_t qkv_stride, in
       pp.ksc = kv->ks + rows0; pp.vsc = kv->vs + rows0;
     }
     pp.q_heads = q_heads; pp.kv_heads = kv->kv_heads; pp.max_ctx = kv->max_ctx; pp.n_tok = n_seq; pp.n_tiles = n_tiles; pp.window = window;
-    pp.softcap = softcap; pp.inv_sqrt = p.inv_sqrt; pp.theta = theta; pp.pos0 = kv->prompt_end - n_seq; pp.out = out; pp.out_stride = out_stride;
+    pp.softcap = softcap; pp.inv_sqrt = p.inv_sqrt; pp.theta = theta; pp.pos0 = kv->prompt_end - n_seq; pp.planes_out = p.planes; pp.planes_q8 = p.planes_q8; pp.out = out; pp.out_stride = out_stride;
     const dim3 rows(n_tiles * kv->kv_heads + n_seq), grid(q_heads, tok_tiles, n_ks);
     auto go = [&](auto hd_) {
       constexpr int HD = hd_;
@@ -1947,12 +2002,13 @@ int launch_attn_step(cai_kv_s* kv, int layer, float* qkv, int64_t qkv_stride, in
   if (rc) return rc;
   if (p.n_splits > 1 && !p.merge_cnt)
   {
-    if (p.n_splits > 96)
-      hipLaunchKernelGGL(attn_merge_kernel<32>, dim3(q_heads, n_seq), dim3(512), 0, c.stream, p.pos, (const float*)p.part, p.out, (long long)p.out_stride,
+    auto merge = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(q_heads, n_seq), dim3(512), 0, c.stream, p.pos, (const float*)p.part, p.out, (long long)p.out_stride,
                          p.q_heads | p.kv_heads << 16, p.n_splits | p.hd << 16, p.split_len, p);
-    else
-      hipLaunchKernelGGL(attn_merge_kernel<12>, dim3(q_heads, n_seq), dim3(512), 0, c.stream, p.pos, (const float*)p.part, p.out, (long long)p.out_stride,
-                         p.q_heads | p.kv_heads << 16, p.n_splits | p.hd << 16, p.split_len, p);
+    };
+    if (p.planes.hi) { if (p.n_splits > 96) merge(attn_merge_kernel<32, true>); else merge(attn_merge_kernel<12, true>); }
+    else if (p.n_splits > 96) merge(attn_merge_kernel<32, false>);
+    else merge(attn_merge_kernel<12, false>);
   }
   return CAI_OK;
 }

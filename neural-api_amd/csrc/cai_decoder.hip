@@ -420,7 +420,7 @@ static int enqueue_prefill_chunk(cai_decoder_s* d, int seq, int n)
   const int32_t* toks = d->ptokpos; const int32_t* poss = d->ptokpos + d->pf_cap;
   int rc;
   if ((rc = launch_embed(d->embed, toks, n, d->px))) return rc;
-  // Between the layers of a short prompt the activations stay planes (7 launches a layer instead of 10)
+  // Between the layers of a short prompt the activations stay planes (5 launches a layer instead of 10)
   bool planes = c.n_experts == 0;
   for (int l = 0; planes && l < c.n_layers; l++) {
     auto& L = d->layers[l];
@@ -434,8 +434,12 @@ static int enqueue_prefill_chunk(cai_decoder_s* d, int seq, int n)
     const bool all_mfma = prompt_route(wq, n) == 2 && prompt_route(wk, n) == 2 && prompt_route(wv, n) == 2;   // one pre-pass serves q, k and v
     if (!planes && all_mfma && (rc = prefill_prep(d->px, dm, L.v[CAI_V_ATTN_NORM], c.eps, dm, n))) return rc;
     const cai_qw_s* qkv3[3] = {wq, wk, wv}; const int qkv_off[3] = {0, qw, qw + kw};
+    AttnOnPlanes on;
     if (planes) {
-      if ((rc = launch_gemm_blk_short(qkv3, qkv_off, 3, xp[0], c.eps, n, d->pqkv, qkvw, nullptr, 0, BlkPlanes(), nullptr))) return rc;
+      KvRows kvr;
+      on.appended = !c.qk_norm_full && attn_rows_for_product(&d->kv, seq, l, n, d->theta, poss, kvr);
+      if ((rc = launch_gemm_blk_short(qkv3, qkv_off, 3, xp[0], c.eps, n, d->pqkv, qkvw, nullptr, 0, BlkPlanes(), nullptr, kvr))) return rc;
+      if (d->ppart_rows >= n) { on.planes = xp[1]; on.q8_0 = L.w[CAI_W_O]->qtype == CAI_Q8_0; }
     } else if (all_mfma && prefill_multi_supported(qkv3, 3)) {   // one launch: the k and v projections alone leave half the chip idle
       if ((rc = prefill_gemm_multi(qkv3, qkv_off, 3, n, d->pqkv, qkvw))) return rc;
     } else if (all_mfma && prefill_multi_supported(qkv3, 2)) {   // attn_v of another type (a Q4_K_M file keeps some in Q6_K): q | k together
@@ -450,11 +454,11 @@ static int enqueue_prefill_chunk(cai_decoder_s* d, int seq, int n)
     for (int r0 = 0; r0 < n; r0 += d->ppart_rows)
       if ((rc = launch_attn_step(&d->kv, l, d->pqkv + (int64_t)r0 * qkvw, qkvw, std::min(d->ppart_rows, n - r0), c.n_q_heads, c.window, 0.0f, d->theta,
                                  poss + r0, d->patt + (int64_t)r0 * qw, qw, seq, 1, d->ppart,
-                                 c.qk_norm_full ? L.v[CAI_V_Q_NORM] : nullptr, c.qk_norm_full ? L.v[CAI_V_K_NORM] : nullptr, c.eps))) return rc;
+                                 c.qk_norm_full ? L.v[CAI_V_Q_NORM] : nullptr, c.qk_norm_full ? L.v[CAI_V_K_NORM] : nullptr, c.eps, planes ? &on : nullptr))) return rc;
     if (planes) {
       const cai_qw_s *wo = L.w[CAI_W_O], *wgu = L.w[CAI_W_GATEUP], *wd = L.w[CAI_W_DOWN]; const int zero = 0;
       const float* next = l + 1 < c.n_layers ? d->layers[l + 1].v[CAI_V_ATTN_NORM] : nullptr;
-      if ((rc = launch_blk_planes(wo, d->patt, nullptr, n, xp[1]))) return rc;
+      if (!on.planes_done && (rc = launch_blk_planes(wo, d->patt, nullptr, n, xp[1]))) return rc;
       if ((rc = launch_gemm_blk_short(&wo, &zero, 1, xp[1], -1.0f, n, d->px, dm, d->px, 0, xp[0], L.v[CAI_V_MLP_NORM]))) return rc;
       if ((rc = launch_gemm_blk_short(&wgu, &zero, 1, xp[0], c.eps, n, nullptr, 0, nullptr, I, xp[1], nullptr))) return rc;
       if ((rc = launch_gemm_blk_short(&wd, &zero, 1, xp[1], -1.0f, n, d->px, dm, d->px, 0, next ? xp[0] : BlkPlanes(), next))) return rc;

@@ -291,10 +291,24 @@ int launch_split_q6k(const uint8_t* raw, int64_t n_blocks, uint8_t* rec, uint8_t
 // hold n_seq * q_heads * n_splits * (head_dim + 2) floats.  1 = a prompt chunk (eight rows or more of a 128-wide cache, 256 of a 64-wide one, go to the
 // matrix-core kernel, which may grow its operand planes); 2 = a window step inside a captured graph (decode kernels only,
 // nothing is allocated).
+// Activations as the operands of gemm_blk_short: tiles of 16 tokens, blocks of 32 columns (cai_prefill_blk.hip)
+struct BlkPlanes { _Float16 *hi = nullptr, *lo = nullptr; float *scale = nullptr, *squares = nullptr; };
+// where token t (of 16) and column c of a block lie in it: which eight columns a lane (t, kg) holds follows from how the lanes share a chunk of weights
+__device__ __forceinline__ int plane_place(bool q8_0, int t, int c)
+{
+  const int g = c >> 3, kg = q8_0 ? (g >> 1) | ((g & 1) << 1) : g;
+  return kg * 128 + t * 8 + (c & 7);
+}
+// Where the rows of K (rotated) and V of a prompt's tokens go: a layer of a sequence, [kv_head][max_ctx][head_dim] of floats or halfs
+struct KvRows { void *k = nullptr, *v = nullptr; int half = 0, head_dim = 1, max_ctx = 0; const float* theta = nullptr; const int32_t* pos = nullptr; };
+// A prompt's attention between products on planes: whether the rows are in the cache already; planes of the result, which planes_done says were left
+// instead of the rows
+struct AttnOnPlanes { bool appended = false; BlkPlanes planes; bool q8_0 = true, planes_done = false; };
+bool attn_rows_for_product(const cai_kv_s* kv, int seq, int layer, int n, const float* theta, const int32_t* pos, KvRows& out);   // whether a product may append them (see launch_attn_step)
 int launch_attn_step(cai_kv_s* kv, int layer, float* qkv, int64_t qkv_stride, int n_seq, int q_heads, int window,
                      float softcap, const float* theta, const int32_t* pos_dev, float* out, int64_t out_stride, int seq0,
                      int prompt_rows = 0, float* prompt_part = nullptr,
-                     const float* qn_gain = nullptr, const float* kn_gain = nullptr, float qk_eps = 0.0f);   // full-width q / k RMSNorm done on the way (null: none)
+                     const float* qn_gain = nullptr, const float* kn_gain = nullptr, float qk_eps = 0.0f, AttnOnPlanes* on_planes = nullptr);   // full-width q / k RMSNorm done on the way (null: none)
 int kv_alloc(cai_kv_s* kv, int n_seq, int n_layers, int kv_heads, int head_dim, int max_ctx, int dtype, bool positions = false);
 void kv_free(cai_kv_s* kv);
 int kv_set_eviction(cai_kv_s* kv, int sinks, int recent);
@@ -332,13 +346,12 @@ int launch_gemm_blk_grouped(const cai_qw_s* bank, int64_t expert_rows, const _Fl
                             int n_slots, int n_experts, const int32_t* perm, const int32_t* tile_tab, float* y, int64_t y_stride);
 // Activations of a short prompt between its products (cai_prefill_blk.hip): hi / lo planes in the order of the matrix operands, scaled by a power of two a token and 32
 // columns, its reciprocal, and the sums of the 32 values' squares before the gain
-struct BlkPlanes { _Float16 *hi = nullptr, *lo = nullptr; float *scale = nullptr, *squares = nullptr; };
 bool blk_short_wanted(const cai_qw_s* wq, const cai_qw_s* wk, const cai_qw_s* wv, const cai_qw_s* wo, const cai_qw_s* wgu, const cai_qw_s* wd, int n_tok);
 int  blk_short_planes(int n_tok, int width0, int width1, BlkPlanes (&out)[2]);
 void blk_short_release();
 int  launch_blk_planes(const cai_qw_s* w, const float* x, const float* gain, int n_tok, const BlkPlanes& o);
 int  launch_gemm_blk_short(const cai_qw_s* const* ws, const int* y_off, int n_w, const BlkPlanes& x, float eps, int n_tok, float* y, int64_t y_stride, const float* residual, int half,
-                           const BlkPlanes& out, const float* gain);
+                           const BlkPlanes& out, const float* gain, const KvRows& kv = KvRows());
 void prefill_planes(const _Float16** hi, const _Float16** lo, const float** sinv);   // what the last prefill_prep filled
 int  prompt_route(const cai_qw_s* w, int n_tok);   // 0 matrix-vector passes, 1 small-batch kernel, 2 prompt kernel
 bool nb_supported(const cai_qw_s* w);          // 2..8-token matrix-core kernel

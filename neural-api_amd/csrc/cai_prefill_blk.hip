@@ -70,13 +70,6 @@ __device__ __forceinline__ half8_b codes8(uint32_t w0, uint32_t w1, int high, bo
   return half8_b{h0.x, h0.y, h1.x, h1.y, h2.x, h2.y, h3.x, h3.y};
 }
 
-// where token t (of 16) and column c of a block lie in it, in the order of gemm_blk_short's operands: which eight columns a lane (t, kg) holds
-// follows from how the lanes share a chunk of weights
-template <int QT> __device__ __forceinline__ int plane_place(int t, int c)
-{
-  const int g = c >> 3, kg = QT == CAI_Q8_0 ? (g >> 1) | ((g & 1) << 1) : g;
-  return kg * 128 + t * 8 + (c & 7);
-}
 typedef uint32_t uint2_b __attribute__((ext_vector_type(2)));
 
 }  // namespace
@@ -509,7 +502,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 // ------------------------------------------------------------------------------------------
 // The products of a short prompt's layers, whose activations stay planes from product to product (launch_gemm_blk_short): what finishes 32
 // outputs of a token scales them by a power of two of their largest and leaves them in the order of the matrix operands, with the sum of their
-// squares; the norm's gain is multiplied in by the writer, its root divided by at the end of the reader.  So a layer has 7 launches instead of 10, and a
+// squares; the norm's gain is multiplied in by the writer, its root divided by at the end of the reader.  So a layer has 5 launches instead of 10 - the rotated
+// K and the V go into the cache from the product that makes them, and the attention leaves planes too - and a
 // wave requests its operands straight into registers, one contiguous KB an instruction, all of a short width at once: a width of 2048 comes in
 // one round trip, where the cut tiles above take one a chunk of 64 columns and stage them in LDS.
 //   planes: tile of 16 tokens, block of 32 columns, [64 lanes][8 halfs]; scales and squares: tile, block, [16 tokens].
@@ -517,8 +511,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 // are summed apart, every second block with its sign changed, in chains of eight blocks (FINE above).
 // What bounds it: a launch, a round trip and the requests themselves, which touch a line a row of weights: 14 a chunk (the scales one by one, eight
 // bytes of a row) took 11.2 us for the down product of the 135M shape (576 x 1536, 37 tokens), 9 a chunk 8.2; tiles of 32 tokens 10.2.  Results that
-// left as single halfs cost gate | up 1.7 us.  A layer of that prompt, kernels alone, us: q | k | v 4.8, append 2.8, attention 6.4, its planes
-// 2.3, o 4.9, gate | up with SwiGLU 6.9, down 8.2 = 36; with rows between the products 51 (four pre-passes of 4.1, products 5.2, 4.5, 5.4 and 9.4).
+// left as single halfs cost gate | up 1.7 us.  A layer of that prompt, kernels alone, us: q | k | v 5.4, attention 6.5, o 4.8, gate | up with
+// SwiGLU 6.8, down 8.0 = 32; with launches of their own for the append (2.8) and the attention's planes (2.3) 36 and 1201 -> 1080 a prompt; with rows between
+// the products 51 (four pre-passes of 4.1, products 5.2, 4.5, 5.4 and 9.4).
 // ------------------------------------------------------------------------------------------
 struct BlkShortParams {
   const uint8_t* q[3]; const uint8_t* d[3]; const float* bias[3]; int rows[3]; int y_off[3]; int seg_end[2]; int n_seg;     // up to three matrices of one type and width
@@ -526,9 +521,10 @@ struct BlkShortParams {
   BlkPlanes x; int normed; float eps;                 // (x.squares are read where the rows are normed)
   float* y; int64_t y_stride; const float* residual;
   BlkPlanes out; const float* gain;                   // planes of the results, times a gain (out.hi null: none)
+  KvRows kv;                                          // the second and third matrix are K and V: their results go into the cache (kv.k null: to y)
 };
 constexpr int BS_NW = 8;
-template <int QT, bool PAIR, bool TWICE>       // TWICE: two work-groups a CU
+template <int QT, bool PAIR, bool TWICE, bool KV>       // TWICE: two work-groups a CU; KV: results of the second and third matrix go into the cache (a form of its own: 2 % of the others' time)
 __global__ __launch_bounds__(64 * BS_NW) __attribute__((amdgpu_waves_per_eu(TWICE ? 4 : 2, TWICE ? 4 : 2))) void gemm_blk_short(const BlkShortParams p)
 {
   constexpr int NW = BS_NW, RT = PAIR ? 4 : 2, P = TWICE ? (PAIR ? 1 : 2) : PAIR ? 3 : 4;      // row tiles of 16; chunks of 64 columns on their way to a wave
@@ -577,6 +573,10 @@ __global__ __launch_bounds__(64 * BS_NW) __attribute__((amdgpu_waves_per_eu(TWIC
   const int tl = tid >> 5, t = tile * 16 + tl, row = R0 + (tid & 31), rc = min(row, rows - 1);
   const int64_t at_y = (int64_t)min(t, p.n_tok - 1) * p.y_stride + p.y_off[sg] + rc;
   const float res = p.residual ? p.residual[at_y] : 0.0f, bs = bias ? bias[rc] : 0.0f, bs2 = PAIR && bias ? bias[p.half + rc] : 0.0f, gain = p.gain ? p.gain[rc] : 1.0f;
+  const int hd = KV ? p.kv.head_dim : 1, pos = KV ? p.kv.pos[min(t, p.n_tok - 1)] : 0;
+  float sn = 0.0f, cs = 1.0f;
+  auto rotation = [&]() { if (KV && sg == 1 && p.kv.theta) sincosf((float)pos * p.kv.theta[(rc % hd) >> 1], &sn, &cs); };
+  if (!TWICE) rotation();                               // (behind the requests, in front of what they bring; two work-groups a CU lack the registers)
   if (p.normed) {                                       // sums of squares: token tid % 16, a 32nd of the blocks
     float ss = 0.0f;
     for (int kb = tid >> 4; kb < nb32; kb += 4 * NW) ss += p.x.squares[((int64_t)tile * nb32 + kb) * 16 + n];
@@ -648,6 +648,15 @@ __global__ __launch_bounds__(64 * BS_NW) __attribute__((amdgpu_waves_per_eu(TWIC
   if constexpr (PAIR) y = silu_mul(y, gate * inv + bs2);
   else {
     y += res;
+    if (KV && sg > 0) {                                 // two neighbouring lanes hold a pair of K
+      if (TWICE) rotation();
+      const float mate = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, y), 0xb1, 0xf, 0xf, false));
+      if (sg == 1 && p.kv.theta) y = row & 1 ? sn * mate + cs * y : cs * y - sn * mate;
+      const int64_t o = ((int64_t)(rc / hd) * p.kv.max_ctx + pos) * hd + rc % hd;
+      void* const c = sg == 1 ? p.kv.k : p.kv.v;
+      if (t < p.n_tok && row < rows) { if (p.kv.half) reinterpret_cast<__half*>(c)[o] = __float2half_rn(y); else reinterpret_cast<float*>(c)[o] = y; }
+      return;
+    }
     if (t < p.n_tok && row < rows) p.y[at_y] = y;
   }
   if (!p.out.hi) return;
@@ -662,7 +671,7 @@ __global__ __launch_bounds__(64 * BS_NW) __attribute__((amdgpu_waves_per_eu(TWIC
   const int e = plane_exponent(m);
   _Float16 h, l; split_plane(x * ldexpf(1.0f, e), h, l);
   // (the work-group's results are one block of the planes: it leaves as whole lines; tokens past the end are its padding)
-  const int at = plane_place<QT>(tl, tid & 31);
+  const int at = plane_place(QT == CAI_Q8_0, tl, tid & 31);
   s_out[0][at] = h; s_out[1][at] = l;
   const int64_t blk = (int64_t)tile * (rows >> 5) + (R0 >> 5);
   if ((tid & 31) == 0) { p.out.scale[blk * 16 + tl] = ldexpf(1.0f, -e); p.out.squares[blk * 16 + tl] = ss; }
@@ -689,7 +698,7 @@ __global__ __launch_bounds__(256) void blk_planes_kernel(const float* __restrict
   half4_b h, l;
 #pragma unroll
   for (int i = 0; i < 4; i++) { _Float16 a, b; split_plane(u[i] * s, a, b); h[i] = a; l[i] = b; }
-  const int64_t blk = (int64_t)(t >> 4) * (K >> 5) + (id >> 3), at = blk * 512 + plane_place<QT>(t & 15, 4 * (id & 7));
+  const int64_t blk = (int64_t)(t >> 4) * (K >> 5) + (id >> 3), at = blk * 512 + plane_place(QT == CAI_Q8_0, t & 15, 4 * (id & 7));
   *reinterpret_cast<half4_b*>(o.hi + at) = h; *reinterpret_cast<half4_b*>(o.lo + at) = l;
   if ((id & 7) == 0) { o.scale[blk * 16 + (t & 15)] = ldexpf(1.0f, -e); o.squares[blk * 16 + (t & 15)] = ss; }
 }
@@ -990,21 +999,21 @@ bool blk_short_wanted(const cai_qw_s* wq, const cai_qw_s* wk, const cai_qw_s* wv
 // y[t][y_off[i] + r] = (W_i x[t])[r] (+ bias_i) (+ residual), or with half > 0 (one matrix of 2 half rows) up * silu(gate), which only out receives; eps >= 0: x is the
 // stream, to be normed; out: planes of the results times a gain, for the next product
 int launch_gemm_blk_short(const cai_qw_s* const* ws, const int* y_off, int n_w, const BlkPlanes& x, float eps, int n_tok, float* y, int64_t y_stride, const float* residual, int half,
-                          const BlkPlanes& out, const float* gain)
+                          const BlkPlanes& out, const float* gain, const KvRows& kv)
 {
   const cai_qw_s* w = ws[0];
   if (!gemm_blk_multi_supported(ws, n_w) || (half && (n_w != 1 || !out.hi || w->rows != 2 * (int64_t)half || half % 32)) || (out.hi && (n_w != 1 || w->rows % 32)))
     return set_error(CAI_ERR_UNSUPPORTED, "short prompt: %d matrices of %lld rows", n_w, (long long)w->rows);
   BlkShortParams p{};
   p.cols = (int)w->cols; p.n_tok = n_tok; p.n_tok_tiles = (n_tok + 15) / 16; p.half = half; p.x = x; p.normed = eps >= 0.0f; p.eps = eps;
-  p.y = y; p.y_stride = y_stride; p.residual = residual; p.out = out; p.gain = gain; p.n_seg = n_w;
+  p.y = y; p.y_stride = y_stride; p.residual = residual; p.out = out; p.gain = gain; p.n_seg = n_w; p.kv = kv;
   for (int i = 0; i < n_w; i++) { p.q[i] = ws[i]->data; p.d[i] = ws[i]->aux; p.bias[i] = ws[i]->bias; p.rows[i] = half ? half : (int)ws[i]->rows; p.y_off[i] = y_off[i]; }
   for (int i = 0; i < n_w; i++) { if (i) p.seg_end[i - 1] = p.n_row_groups; p.n_row_groups += (p.rows[i] + 31) / 32; }
   const dim3 grid(8 * p.n_tok_tiles * ((p.n_row_groups + 7) / 8)), blk(64 * BS_NW);
   const bool twice = p.n_row_groups * p.n_tok_tiles > ctx().n_cu;
-#define SHORT_T(QT, PAIR) do { if (twice) hipLaunchKernelGGL((gemm_blk_short<QT, PAIR, true>), grid, blk, 0, ctx().stream, p); \
-                               else hipLaunchKernelGGL((gemm_blk_short<QT, PAIR, false>), grid, blk, 0, ctx().stream, p); } while (0)
-#define SHORT(QT) do { if (half) SHORT_T(QT, true); else SHORT_T(QT, false); } while (0)
+#define SHORT_T(QT, PAIR, KV) do { if (twice) hipLaunchKernelGGL((gemm_blk_short<QT, PAIR, true, KV>), grid, blk, 0, ctx().stream, p); \
+                                   else hipLaunchKernelGGL((gemm_blk_short<QT, PAIR, false, KV>), grid, blk, 0, ctx().stream, p); } while (0)
+#define SHORT(QT) do { if (half) SHORT_T(QT, true, false); else if (kv.k) SHORT_T(QT, false, true); else SHORT_T(QT, false, false); } while (0)
   if (w->qtype == CAI_Q8_0) SHORT(CAI_Q8_0); else SHORT(CAI_Q4_0);
 #undef SHORT
 #undef SHORT_T

@@ -514,6 +514,37 @@ def test_short_prompts_whose_activations_stay_planes(qt, d, ffn, hq, hkv, hd, T)
     dec.close()
 
 
+# heads whose results become planes in the attention (64, 32, 128 on the matrix cores) and not (16, 48); rows appended by the product (float, half) and not (int8, a rolling cache);
+# one slice, slices that a merge adds, a window that leaves out the first of them; a prompt behind cached rows
+@pytest.mark.parametrize("qt", [O.Q8_0, O.Q4_0])
+@pytest.mark.parametrize("hq,hkv,hd", [(3, 1, 64), (4, 2, 32), (6, 6, 16), (2, 1, 48), (3, 1, 128)])
+@pytest.mark.parametrize("kv,ctx,window,rolling", [("f32", 40, 0, 0), ("f16", 96, 20, 0), ("f16", 700, 0, 0), ("f32", 2000, 50, 0), ("i8", 96, 0, 0), ("f32", 200, 0, 90)])
+def test_short_prompts_append_their_rows_and_leave_planes(qt, hq, hkv, hd, kv, ctx, window, rolling):
+    """Two portions of a prompt equal its tokens one by one, and so does a step from the rows they left (a half on the edge between two may land one
+    apart, 2^-11 of a cached element, a code of an int8 cache too)"""
+    from helpers.device import dev, rel_err
+    from helpers.model_build import synthetic_spec
+    cai = dev()
+    cfg = dict(n_layers=2, d_model=96, n_q_heads=hq, n_kv_heads=hkv, head_dim=hd, ffn=160, vocab=300, max_ctx=ctx, eps=1e-5, rope_theta=1e4, window=window)
+    spec = synthetic_spec(cfg, qt, head_qtype=O.Q8_0, seed=hd, std=0.05, qkv_bias=True)
+    dec = cai.Decoder(spec, max_batch=2, kv_dtype={"f32": cai.KV_F32, "f16": cai.KV_F16, "i8": cai.KV_I8}[kv])
+    if rolling:
+        dec.set_eviction(8, rolling - 8)
+    tok = np.random.default_rng(ctx).integers(0, 300, 39).astype(np.int32)
+    tol = {"f32": 1e-5, "f16": 1e-3, "i8": 5e-3}[kv]
+    for p_, t in enumerate(tok[:38]):
+        _, want = dec.step_window([t], p_, seq=1)
+        if p_ == 20:
+            first = want[0].copy()
+    _, got = dec.prefill(tok[:21])
+    assert rel_err(got, first) < tol
+    _, got = dec.prefill(tok[21:38], 21)
+    assert rel_err(got, want[0]) < tol
+    after = dec.step(np.array([tok[38]] * 2, np.int32), np.array([38, 38], np.int32))[1]
+    assert rel_err(after[0], after[1]) < tol
+    dec.close()
+
+
 @pytest.mark.parametrize("qt,ffn,T", [(O.Q8_0, 352, 100), (O.Q4_0, 64, 40), (O.Q8_0, 320, 150)])
 def test_prompt_of_a_mixture_on_tiles_of_64_slots(qt, ffn, T):
     """banks of four experts, two a token: runs of about T / 2 slots in tiles of 64 (full, half empty, a remainder), widths of an odd and an
