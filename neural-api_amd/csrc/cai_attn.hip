@@ -113,8 +113,8 @@ struct AttnParams {
   const float* qn_gain; const float* kn_gain; float qk_eps;   // full-width RMSNorm of q and of k applied while they are read (null: rows are used as they are)
   unsigned* merge_cnt;         // decode steps: arrival counters [seq][head]; the work-group that completes the last slice merges (null: a merge launch follows)
   unsigned long long* timeline; // stamps of this launch's work-groups (null: none)
-  BlkPlanes planes; bool planes_q8; // prompts: the results leave as planes (planes.hi null: as rows)
 };
+struct PlanesParams : AttnParams { BlkPlanes planes; bool planes_q8 = true; };      // a prompt's rows whose results leave as planes (planes.hi null: as rows)
 
 typedef _Float16 ph4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 ph8_t __attribute__((ext_vector_type(8)));
@@ -902,7 +902,7 @@ __global__ __launch_bounds__(64 * NW) void attn_group_mfma_kernel(const int32_t*
 //      maximum, and meet in LDS. ----
 template <int MR, bool PLANES>      // slices per quarter and round trip: 12, or 32 for long caches (130k rows = 508 slices: 4 dependent rounds instead of 11)
 __global__ __launch_bounds__(512) void attn_merge_kernel(const int32_t* hpos, const float* hpart, float* hout, const long long hout_stride,
-                                                         const int hheads, const int hgeo, const int hsl, const AttnParams p)
+                                                         const int hheads, const int hgeo, const int hsl, const std::conditional_t<PLANES, PlanesParams, AttnParams> p)
 {
   const int h_q_heads = hheads & 0xffff, h_n_splits = hgeo & 0xffff, h_hd = hgeo >> 16;     // (preloaded leading arguments, as in the split kernels)
   const int qh = blockIdx.x, seq = blockIdx.y;
@@ -958,7 +958,7 @@ __global__ __launch_bounds__(512) void attn_merge_kernel(const int32_t* hpos, co
       At = fmaf(qA[k][d], e, At); Lt = fmaf(qL[k], e, Lt);
     }
     const float y = Lt > 0.0f ? At * (1.0f / Lt) : 0.0f;
-    if (PLANES) out_plane(p.planes, p.planes_q8, seq, qh * hd + d, h_q_heads * hd, y);
+    if constexpr (PLANES) out_plane(p.planes, p.planes_q8, seq, qh * hd + d, h_q_heads * hd, y);
     else hout[(int64_t)seq * hout_stride + qh * hd + d] = y;
   }
 }
@@ -982,10 +982,13 @@ __global__ __launch_bounds__(512) void attn_merge_kernel(const int32_t* hpos, co
 // and not once a group, the exponentials of the meeting once a lane.  More waves (8, 16 a work-group) took longer to start and to meet
 // (100 half rows of 128: 5.5 us with four, 6.3, 9.6; 200: 7.2, 7.2, 9.6).  NCH: chunks of 64 rows on their way at once.
 // MODE: a step's rows as they are, with the norms of whole q and k rows, or a prompt's rows whose results leave as planes.
-enum { HEAD_PLAIN, HEAD_NORMED, HEAD_PLANES };
+constexpr int HEAD_PLAIN = 0, HEAD_NORMED = 1, HEAD_PLANES = 2;
+// (a trait, and no enumerator in the kernel's signature: an enumeration without a name is numbered differently for host and device, and so is the kernel's)
+template <int MODE> struct HeadParams { using type = AttnParams; };
+template <> struct HeadParams<HEAD_PLANES> { using type = PlanesParams; };
 template <int VW, int NV, typename KV_T, int NCH, int MODE>
 __global__ __launch_bounds__(256) void attn_split_head_kernel(const int32_t* hpos, const float* hqkv, const void* hk, const void* hv, const int hqkv_stride,
-                                                                  const int hheads, const int hgeo, const int hsl, const int hmax_ctx, const int hseq_planes, const AttnParams p)
+                                                                  const int hheads, const int hgeo, const int hsl, const int hmax_ctx, const int hseq_planes, const typename HeadParams<MODE>::type p)
 {
   constexpr bool QN = MODE == HEAD_NORMED;
   constexpr int DS = VW * NV, NG = 16;         // groups of 16 lanes, four waves: row j of the slice belongs to group j % NG
@@ -1241,7 +1244,7 @@ __global__ __launch_bounds__(256) void attn_split_head_kernel(const int32_t* hpo
     const int qh = g * G + h;
     if (tid < hd && n_active == 1) {
       const float y = Ls > 0.0f ? A * (1.0f / Ls) : 0.0f;
-      if (MODE == HEAD_PLANES) out_plane(p.planes, p.planes_q8, seq, qh * hd + d, q_heads * hd, y);
+      if constexpr (MODE == HEAD_PLANES) out_plane(p.planes, p.planes_q8, seq, qh * hd + d, q_heads * hd, y);
       else p.out[(int64_t)seq * p.out_stride + qh * hd + d] = y;
     } else if (tid < hd) {
       float* pt = p.part + (((int64_t)seq * p.q_heads + qh) * p.n_splits + split) * (hd + 2);
@@ -1254,9 +1257,9 @@ __global__ __launch_bounds__(256) void attn_split_head_kernel(const int32_t* hpo
 }
 
 template <typename KV_T>
-static int launch_split_head(const AttnParams& p0, int n_seq, hipStream_t st)
+static int launch_split_head(const PlanesParams& p0, int n_seq, hipStream_t st)
 {
-  AttnParams p = p0;
+  PlanesParams p = p0;
   const int G = p.q_heads / p.kv_heads;
   const int items = p.n_splits * p.kv_heads;
   const dim3 grid(8 * G * ((items + 7) / 8), n_seq);
@@ -1269,8 +1272,8 @@ static int launch_split_head(const AttnParams& p0, int n_seq, hipStream_t st)
   const int64_t at = (p.seq0 * p.seq_elems + p.layer_off) * (int64_t)sizeof(KV_T);
   const void* hk = (const char*)p.kc + at; const void* hv = (const char*)p.vc + at;
   p.scale_row0 = p.seq0 * p.seq_rows + p.layer_row_off;
-  auto put = [&](auto kern) {
-    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, p.pos, (const float*)p.qkv, hk, hv, (int)qkv_stride, hheads, hgeo, hsl, p.max_ctx, (int)seq_planes, p);
+  auto put = [&](auto kern, const auto& params) {
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, p.pos, (const float*)p.qkv, hk, hv, (int)qkv_stride, hheads, hgeo, hsl, p.max_ctx, (int)seq_planes, params);
   };
   auto go = [&](auto vw, auto nv) {
     constexpr int VW = decltype(vw)::value, NV = decltype(nv)::value;
@@ -1278,7 +1281,8 @@ static int launch_split_head(const AttnParams& p0, int n_seq, hipStream_t st)
     constexpr int LONG = 2;
     auto of = [&](auto mode) {
       constexpr int MODE = decltype(mode)::value;
-      if (p.split_len <= 64) put(attn_split_head_kernel<VW, NV, KV_T, 1, MODE>); else put(attn_split_head_kernel<VW, NV, KV_T, LONG, MODE>);
+      const typename HeadParams<MODE>::type& q = p;
+      if (p.split_len <= 64) put(attn_split_head_kernel<VW, NV, KV_T, 1, MODE>, q); else put(attn_split_head_kernel<VW, NV, KV_T, LONG, MODE>, q);
     };
     if (p.qn_gain) of(std::integral_constant<int, HEAD_NORMED>());
     else if (p.planes.hi) of(std::integral_constant<int, HEAD_PLANES>());
@@ -1899,7 +1903,7 @@ int launch_attn_step(cai_kv_s* kv, int layer, float* qkv, int64_t qkv_stride, in
   if (n_seq < 1 || seq0 < 0 || seq0 + (prompt_rows ? 1 : n_seq) > kv->n_seq) return set_error(CAI_ERR_INVALID, "attention: %d sequences, cache holds %d", n_seq, kv->n_seq);
   if (q_heads % kv->kv_heads) return set_error(CAI_ERR_INVALID, "attention: %d query heads not a multiple of %d KV heads", q_heads, kv->kv_heads);
   if (q_heads > kv->part_q_heads) return set_error(CAI_ERR_INVALID, "attention: %d query heads exceed the cache's scratch (%d)", q_heads, kv->part_q_heads);
-  AttnParams p{};
+  PlanesParams p{};
   p.qkv = qkv; p.qkv_stride = qkv_stride; p.kc = kv->k; p.vc = kv->v;
   p.seq_elems = kv->seq_elems(); p.layer_off = (int64_t)layer * kv->layer_elems();
   p.q_heads = q_heads; p.kv_heads = kv->kv_heads; p.hd = kv->head_dim; p.max_ctx = kv->max_ctx;
@@ -2002,13 +2006,14 @@ int launch_attn_step(cai_kv_s* kv, int layer, float* qkv, int64_t qkv_stride, in
   if (rc) return rc;
   if (p.n_splits > 1 && !p.merge_cnt)
   {
-    auto merge = [&](auto kern) {
+    auto merge = [&](auto kern, const auto& params) {
       hipLaunchKernelGGL(kern, dim3(q_heads, n_seq), dim3(512), 0, c.stream, p.pos, (const float*)p.part, p.out, (long long)p.out_stride,
-                         p.q_heads | p.kv_heads << 16, p.n_splits | p.hd << 16, p.split_len, p);
+                         p.q_heads | p.kv_heads << 16, p.n_splits | p.hd << 16, p.split_len, params);
     };
-    if (p.planes.hi) { if (p.n_splits > 96) merge(attn_merge_kernel<32, true>); else merge(attn_merge_kernel<12, true>); }
-    else if (p.n_splits > 96) merge(attn_merge_kernel<32, false>);
-    else merge(attn_merge_kernel<12, false>);
+    const AttnParams& rows = p;
+    if (p.planes.hi) { if (p.n_splits > 96) merge(attn_merge_kernel<32, true>, p); else merge(attn_merge_kernel<12, true>, p); }
+    else if (p.n_splits > 96) merge(attn_merge_kernel<32, false>, rows);
+    else merge(attn_merge_kernel<12, false>, rows);
   }
   return CAI_OK;
 }
