@@ -378,8 +378,9 @@ static int linear_rows(const cai_qw_s* w, bool prepped, const float* x, int64_t 
 
 // Expert half of a block for a whole prompt chunk in px (n tokens), in place (neural/neuralpretrained.pas:15331-15388):
 // router logits -> soft-max / top-k for every token -> the n * top_k slots grouped by expert -> gate|up over the bank in one
-// launch -> SwiGLU -> down over the bank in one launch -> gate-weighted mixture added to each row.
-static int moe_ffn_prompt(cai_decoder_s* d, const cai_decoder_s::Layer& L, int n)
+// launch -> SwiGLU -> down over the bank in one launch -> gate-weighted mixture added to each row, which becomes planes for the next block's q, k and v
+// where it gives its gain.
+static int moe_ffn_prompt(cai_decoder_s* d, const cai_decoder_s::Layer& L, int n, const float* next_gain)
 {
   const cai_decoder_config& c = d->cfg;
   const int dm = c.d_model, I = c.ffn, E = c.n_experts, K = c.top_k, slots = n * K;
@@ -397,7 +398,7 @@ static int moe_ffn_prompt(cai_decoder_s* d, const cai_decoder_s::Layer& L, int n
   if ((rc = prefill_prep_swiglu(d->pm_gu, 2 * I, I, slots))) return rc;   // SwiGLU inside the pre-pass of the down projection
   prefill_planes(&hi, &lo, &sinv);
   if ((rc = launch_gemm_blk_grouped(L.w[CAI_W_DOWN], dm, hi, lo, sinv, 1, slots, E, d->pm_perm, d->pm_tiles, d->pm_part, dm))) return rc;
-  return launch_moe_combine(d->px, d->pm_part, d->pm_gate, K, dm, n);
+  return next_gain ? prefill_prep_mixture(d->px, d->pm_part, d->pm_gate, K, next_gain, c.eps, dm, n) : launch_moe_combine(d->px, d->pm_part, d->pm_gate, K, dm, n);
 }
 
 static int linear_rows(const cai_qw_s* w, bool prepped, const float* x, int64_t x_stride, const float* gain, float eps, int n,
@@ -413,6 +414,7 @@ static int linear_rows(const cai_qw_s* w, bool prepped, const float* x, int64_t 
   return prefill_linear(w, x, x_stride, gain, eps, n, y, y_stride, residual);
 }
 
+static bool qkv_on_planes(const cai_decoder_s::Layer& L, int n) { return prompt_route(L.w[CAI_W_Q], n) == 2 && prompt_route(L.w[CAI_W_K], n) == 2 && prompt_route(L.w[CAI_W_V], n) == 2; }
 static int enqueue_prefill_chunk(cai_decoder_s* d, int seq, int n)
 {
   const cai_decoder_config& c = d->cfg;
@@ -426,13 +428,15 @@ static int enqueue_prefill_chunk(cai_decoder_s* d, int seq, int n)
     auto& L = d->layers[l];
     planes = blk_short_wanted(L.w[CAI_W_Q], L.w[CAI_W_K], L.w[CAI_W_V], L.w[CAI_W_O], L.w[CAI_W_GATEUP], L.w[CAI_W_DOWN], n) && L.v[CAI_V_ATTN_NORM] && L.v[CAI_V_MLP_NORM];
   }
+  bool prepped = false;            // the stream is planes already, normed for this layer's q, k and v
   BlkPlanes xp[2];                 // of the stream, and of what the attention and the feed-forward leave
   if (planes && ((rc = blk_short_planes(n, dm, std::max(qw, I), xp)) || (rc = launch_blk_planes(d->layers[0].w[CAI_W_Q], d->px, d->layers[0].v[CAI_V_ATTN_NORM], n, xp[0])))) return rc;
   for (int l = 0; l < c.n_layers; l++) {
     auto& L = d->layers[l];
     const cai_qw_s* wq = L.w[CAI_W_Q]; const cai_qw_s* wk = L.w[CAI_W_K]; const cai_qw_s* wv = L.w[CAI_W_V];
-    const bool all_mfma = prompt_route(wq, n) == 2 && prompt_route(wk, n) == 2 && prompt_route(wv, n) == 2;   // one pre-pass serves q, k and v
-    if (!planes && all_mfma && (rc = prefill_prep(d->px, dm, L.v[CAI_V_ATTN_NORM], c.eps, dm, n))) return rc;
+    const bool all_mfma = qkv_on_planes(L, n);   // one pre-pass serves q, k and v
+    const bool have = prepped; prepped = false;
+    if (!planes && all_mfma && !have && (rc = prefill_prep(d->px, dm, L.v[CAI_V_ATTN_NORM], c.eps, dm, n))) return rc;
     const cai_qw_s* qkv3[3] = {wq, wk, wv}; const int qkv_off[3] = {0, qw, qw + kw};
     AttnOnPlanes on;
     if (planes) {
@@ -471,7 +475,9 @@ static int enqueue_prefill_chunk(cai_decoder_s* d, int seq, int n)
       // rows (one router / top-k launch per group, the gathered products per token)
       if (n > 8 && d->pm_gu && gemm_blk_supported(L.w[CAI_W_GATEUP]) && gemm_blk_supported(L.w[CAI_W_DOWN]) &&
           (int64_t)n * c.top_k * I < ((int64_t)1 << 31)) {   // (an activation row of the grouped products lies at a 32-bit byte offset)
-        if ((rc = moe_ffn_prompt(d, L, n))) return rc;
+        const auto* N = l + 1 < c.n_layers ? &d->layers[l + 1] : nullptr;
+        prepped = N && N->v[CAI_V_ATTN_NORM] && prefill_prep_mixture_supported(dm) && qkv_on_planes(*N, n);
+        if ((rc = moe_ffn_prompt(d, L, n, prepped ? N->v[CAI_V_ATTN_NORM] : nullptr))) return rc;
         continue;
       }
       const int grp = 8;

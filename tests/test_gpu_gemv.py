@@ -545,6 +545,24 @@ def test_short_prompts_append_their_rows_and_leave_planes(qt, hq, hkv, hd, kv, c
     dec.close()
 
 
+# rows that fill a part of the work-group, one, two and four pieces a thread, and rows past what it holds; one expert, and more than are requested at once
+@pytest.mark.parametrize("d,experts,top", [(96, 4, 1), (1056, 12, 9), (2080, 3, 2), (4128, 2, 2)])
+def test_prompt_of_a_mixture_whose_rows_become_planes(d, experts, top):
+    """The experts' rows are added where the next layer's planes are made: a prompt equals its tokens one by one (32-bit sums over activations of 22 bits, 1e-5
+    apart at most where a layer's rounding is carried on)"""
+    from helpers.device import dev, rel_err
+    from helpers.model_build import synthetic_spec
+    cai = dev()
+    cfg = dict(n_layers=3, d_model=d, n_q_heads=2, n_kv_heads=1, head_dim=32, ffn=64, vocab=300, max_ctx=64, eps=1e-5, rope_theta=1e4, n_experts=experts, top_k=top, norm_topk=1)
+    dec = cai.Decoder(synthetic_spec(cfg, O.Q8_0, head_qtype=O.Q8_0, seed=d, std=0.05), max_batch=2)
+    tok = np.random.default_rng(d).integers(0, 300, 33).astype(np.int32)
+    _, got = dec.prefill(tok)
+    for p_, t in enumerate(tok):
+        _, want = dec.step_window([t], p_, seq=1)
+    assert rel_err(got, want[0]) < 1e-5
+    dec.close()
+
+
 @pytest.mark.parametrize("qt,ffn,T", [(O.Q8_0, 352, 100), (O.Q4_0, 64, 40), (O.Q8_0, 320, 150)])
 def test_prompt_of_a_mixture_on_tiles_of_64_slots(qt, ffn, T):
     """banks of four experts, two a token: runs of about T / 2 slots in tiles of 64 (full, half empty, a remainder), widths of an odd and an
