@@ -392,7 +392,7 @@ def test_streaming_eviction_session_runs_past_max_ctx():
 
 @pytest.mark.parametrize("kv,window", [("f32", 0), ("f16", 0), ("f32", 40), ("f16", 70), ("i8", 0), ("i8", 50)])
 def test_prompt_attention_on_matrix_cores_equals_steps(kv, window):
-    """Prompt ingestion over a 128-wide cache runs the matrix-core attention kernel (32 tokens x 4 heads per
+    """Prompt ingestion over a 128-wide cache runs the matrix-core attention kernel (32 tokens of a head per
     work-group): the last token's logits equal token-at-a-time ingestion for fp32, fp16 and int8 caches, under a sliding
     window, for prompt lengths that are not multiples of the tile and for a continuation from position > 0."""
     from helpers.device import dev, rel_err
