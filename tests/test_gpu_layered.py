@@ -208,6 +208,29 @@ def test_chunks_of_a_portion(cai, tmp_path, mech, h, g, d, dv, n):
     dec.close()
 
 
+def test_dynamic_tanh_is_as_near_as_the_library_s(cai, tmp_path):
+    """The identity as vocabulary matrix and a layer that adds a constant a channel: the logits are the final norm of known 32-bit values.  tanhf is 2.43 * 2^-24 of its
+    value from 64 bits at most below 1, and 1.25 * 2^-24 from there on (measured); what takes its place may not be further off.  Half of the arguments lie
+    around 1, where forms of a tanh meet."""
+    n, rng = 1024, np.random.default_rng(5)
+
+    def edit(w):
+        w["l0.mix.o"] = w["l0.mix.o"] * 0
+        w["l0.norm1b.b"] = np.exp(rng.uniform(np.log(2.0 ** -22), np.log(2.0 ** -7), n))
+        w["embed"] = np.exp(rng.uniform(np.log(0.02), np.log(9.5), (n, n))) * rng.choice([-1, 1], (n, n))
+        w["embed"][::2] = 1.0 + rng.integers(-5, 3, (n // 2, n)) / 256.0
+        w["head"], w["final.norm"], w["final.norm.b"], w["final.norm.alpha"] = np.eye(n), np.ones(n), np.zeros(n), np.asarray(1.0)
+
+    m = Model(tmp_path, B.config([B.layer(B.delta(1, 1, 8, 8, 2), ff=None)], width=n, vocab=n), edit=edit)
+    dec = m.open(cai, 1024, 1, "f32")
+    got = feed(dec, list(range(n)), [n]).astype(np.float64)
+    dec.close()
+    x = (m.w["embed"].astype(np.float32) + m.w["l0.norm1b.b"].astype(np.float32)).astype(np.float64)
+    want = np.tanh(x)
+    off = np.abs(got - want) / np.abs(want) * 2.0 ** 24
+    assert off[np.abs(x) < 1].max() < 2.45 and off[np.abs(x) >= 1].max() < 1.27, (off[np.abs(x) < 1].max(), off[np.abs(x) >= 1].max())
+
+
 @pytest.mark.parametrize("tokens, ff", [(129, 16400), (257, 8208), (300, 12000)])
 def test_products_on_tiles_of_256_tokens(cai, tmp_path, tokens, ff):
     """gate | up matrices whose products fill the chip with large tiles: tokens one past half a tile, one past a tile and inside a second one, rows
