@@ -1812,7 +1812,8 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(const PromptParams 
         for (int v = 0; v < 16; v++) O[dt][v] = fmaf(T[dt][v], back, O[dt][v]);
   }
 
-  // ---- the waves' sums, in wave order ----
+  // ---- the waves' sums, in wave order: a wave without a row of the token (a normaliser of exactly 0) leaves nothing, one that met a score that is not a number or
+  // infinite (a normaliser that is not a number) makes the token's result that too ----
   if (kg == 0) { sM[wave][n] = m_run; sL[wave][n] = l_run; }
   __syncthreads();                                // (and q has been read)
   {
@@ -1820,7 +1821,7 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(const PromptParams 
 #pragma unroll
     for (int dt = 0; dt < DT; dt++)
 #pragma unroll
-      for (int v = 0; v < 16; v++) sO[(wave * HD + 32 * dt + 8 * (v >> 2) + 4 * kg + (v & 3)) * PA_LDO + n] = l_run > 0.0f ? O[dt][v] * c : 0.0f;      // (no row of this wave: nothing)
+      for (int v = 0; v < 16; v++) sO[(wave * HD + 32 * dt + 8 * (v >> 2) + 4 * kg + (v & 3)) * PA_LDO + n] = l_run == 0.0f ? 0.0f : O[dt][v] * c;
   }
   __syncthreads();
   const int r = tid >> 3, t = t0 + r;
@@ -1828,8 +1829,8 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(const PromptParams 
   const float M = fmaxf(fmaxf(sM[0][r], sM[1][r]), fmaxf(sM[2][r], sM[3][r]));
   float L = 0.0f;
 #pragma unroll
-  for (int w = 0; w < 4; w++) if (sL[w][r] > 0.0f) L = fmaf(sL[w][r], expf(sM[w][r] - M), L);
-  const float inv = splits > 1 ? 1.0f : L > 0.0f ? 1.0f / L : 0.0f;           // a piece leaves unnormalised sums, maximum and normaliser; prompt_merge_kernel adds the pieces
+  for (int w = 0; w < 4; w++) if (sL[w][r] != 0.0f) L = fmaf(sL[w][r], expf(sM[w][r] - M), L);
+  const float inv = splits > 1 ? 1.0f : L == 0.0f ? 0.0f : 1.0f / L;          // a piece leaves unnormalised sums, maximum and normaliser; prompt_merge_kernel adds the pieces
   float* dst = splits > 1 ? p.part + (((int64_t)t * p.q_heads + head) * gridDim.z + ks) * (HD + 2) : p.out + (int64_t)t * p.out_stride + head * HD;
 #pragma unroll
   for (int i = 0; i < HD / 32; i++) {
@@ -1865,12 +1866,12 @@ __global__ __launch_bounds__(512) void prompt_merge_kernel(const PromptParams p,
   for (int s = 0; s < PA_KS_MAX; s++) { const int sc = min(s, splits - 1); ms[s] = pt[sc * (HD + 2) + HD]; ls[s] = pt[sc * (HD + 2) + HD + 1]; as[s] = pt[sc * (HD + 2) + d]; }
 #pragma unroll
   for (int s = 0; s < PA_KS_MAX; s++) {
-    if (s < splits && ls[s] > 0.0f) {
+    if (s < splits && ls[s] != 0.0f) {      // (a piece that is not a number stays one)
       const float mn = fmaxf(M, ms[s]), c0 = expf(M - mn), c1 = expf(ms[s] - mn);
       A = A * c0 + as[s] * c1; L = L * c0 + ls[s] * c1; M = mn;
     }
   }
-  const float y = L > 0.0f ? A * (1.0f / L) : 0.0f;
+  const float y = L == 0.0f ? 0.0f : A * (1.0f / L);
   if (p.planes_out.hi) out_plane(p.planes_out, p.planes_q8, tok, head * HD + d, p.q_heads * HD, y);
   else p.out[(int64_t)tok * p.out_stride + head * HD + d] = y;
 }

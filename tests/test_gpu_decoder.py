@@ -520,6 +520,30 @@ def test_prompt_attention_leaves_alone_what_an_earlier_sequence_left(kv, hd):
     dec.close()
 
 
+@pytest.mark.parametrize("kv", ["f32", "f16"])
+@pytest.mark.parametrize("hd,before,n,at", [(128, 0, 70, 20), (128, 0, 100, 40), (64, 0, 257, 200), (128, 610, 20, 300), (64, 1000, 256, 500)])
+def test_prompt_attention_shows_a_cached_row_that_is_not_a_number(kv, hd, before, n, at):
+    """one row of NaN keys and values in a tile that is not the last token's, so that one wave of four (or one piece of several, the last two) meets it: the
+    last token's logits are not numbers either, and are again where the row is outside the window"""
+    from helpers.device import dev
+    cai = dev()
+    for window, shown in ((0, True), (32, False)):
+        cfg = dict(n_layers=1, d_model=256, n_q_heads=4, n_kv_heads=2, head_dim=hd, ffn=256, vocab=300, max_ctx=1300, eps=1e-5, rope_theta=1e4, window=window)
+        spec = synthetic_spec(cfg, O.Q8_0, head_qtype=O.Q8_0, seed=3, std=0.05)
+        t = spec["tensors"][(-1, O.W_EMBED)]
+        raw = t["raw"].reshape(300, -1)
+        raw[299, 0:2] = np.array([np.inf], np.float16).view(np.uint8)       # token 299: the scale of its first block
+        t["raw"] = raw.reshape(-1)
+        dec = cai.Decoder(spec, kv_dtype={"f32": cai.KV_F32, "f16": cai.KV_F16}[kv])
+        toks = np.random.default_rng(hd + n).integers(0, 299, before + n).astype(np.int32)
+        toks[at] = 299
+        if before:
+            dec.prefill(toks[:before])
+        _, got = dec.prefill(toks[before:], before)
+        assert not np.isfinite(got).any() if shown else np.isfinite(got).all()
+        dec.close()
+
+
 @pytest.mark.parametrize("name", ["qwen7b_like_q4k", "olmoe_like_q8"])
 def test_per_class_timing_leaves_the_session_as_it_found_it(name):
     """cai_decoder_profile (a measurement aid without a counterpart in the reference) replays whole steps and steps without one
