@@ -149,7 +149,8 @@ __global__ __launch_bounds__(NT) void xprep_regs_kernel(const float* x, int64_t 
       const int j = 4 * ((int)threadIdx.x + e * NT);
 #pragma unroll
       for (int i = 0; i < 4; i++) v[e][i] += acc[e][i];
-      if (j < K) *reinterpret_cast<f32x4_any*>(mix.x + (int64_t)t * x_stride + j) = v[e];
+      // (past the end: the last values before or after their thread wrote them back, so not even for the maximum)
+      if (j < K) *reinterpret_cast<f32x4_any*>(mix.x + (int64_t)t * x_stride + j) = v[e]; else v[e] = f32x4_any{0.0f, 0.0f, 0.0f, 0.0f};
     }
   }
   if (!SWIGLU && gain) {
