@@ -219,9 +219,11 @@ static void xprep_launch(const float* x, int64_t x_stride, const float* gain, fl
   if (K <= 1024) hipLaunchKernelGGL((xprep_regs_kernel<SRC, 256, 1>), dim3(n_tok), dim3(256), 0, st, x, x_stride, gain, eps, K, hi, lo, sinv, sxhi, sxlo, mix);
   else if (K <= 2048) hipLaunchKernelGGL((xprep_regs_kernel<SRC, 256, 2>), dim3(n_tok), dim3(256), 0, st, x, x_stride, gain, eps, K, hi, lo, sinv, sxhi, sxlo, mix);
   else if (K <= 4096) hipLaunchKernelGGL((xprep_regs_kernel<SRC, 256, 4>), dim3(n_tok), dim3(256), 0, st, x, x_stride, gain, eps, K, hi, lo, sinv, sxhi, sxlo, mix);
-  else if (K <= 8192) hipLaunchKernelGGL((xprep_regs_kernel<SRC, 1024, 2>), dim3(n_tok), dim3(1024), 0, st, x, x_stride, gain, eps, K, hi, lo, sinv, sxhi, sxlo, mix);
-  else if (K <= 24 * 1024) hipLaunchKernelGGL((xprep_regs_kernel<SRC, 1024, 6>), dim3(n_tok), dim3(1024), 0, st, x, x_stride, gain, eps, K, hi, lo, sinv, sxhi, sxlo, mix);
-  else if constexpr (SRC != PREP_MIXTURE) hipLaunchKernelGGL((xprep_kernel<SRC == PREP_SWIGLU, 1024>), dim3(n_tok), dim3(1024), 0, st, x, x_stride, gain, eps, K, hi, lo, sinv, sxhi, sxlo);
+  else if constexpr (SRC != PREP_MIXTURE) {      // (prefill_prep_mixture takes no wider rows)
+    if (K <= 8192) hipLaunchKernelGGL((xprep_regs_kernel<SRC, 1024, 2>), dim3(n_tok), dim3(1024), 0, st, x, x_stride, gain, eps, K, hi, lo, sinv, sxhi, sxlo, mix);
+    else if (K <= 24 * 1024) hipLaunchKernelGGL((xprep_regs_kernel<SRC, 1024, 6>), dim3(n_tok), dim3(1024), 0, st, x, x_stride, gain, eps, K, hi, lo, sinv, sxhi, sxlo, mix);
+    else hipLaunchKernelGGL((xprep_kernel<SRC == PREP_SWIGLU, 1024>), dim3(n_tok), dim3(1024), 0, st, x, x_stride, gain, eps, K, hi, lo, sinv, sxhi, sxlo);
+  }
 }
 
 struct GemmParams {
@@ -758,6 +760,7 @@ int prefill_prep_swiglu(const float* gu, int64_t gu_stride, int half, int n_tok)
 bool prefill_prep_mixture_supported(int K) { return K <= 4096 && K % 32 == 0; }
 int prefill_prep_mixture(float* x, const float* part, const float* gate, int k, const float* gain, float eps, int K, int n_tok)
 {
+  if (!prefill_prep_mixture_supported(K)) return set_error(CAI_ERR_UNSUPPORTED, "prompt: a mixture's rows of %d values are not added where the planes are made", K);
   int rc;
   if ((rc = prefill_reserve(n_tok, K))) return rc;
   xprep_launch<PREP_MIXTURE>(x, K, gain, eps, K, n_tok, g_pws.hi, g_pws.lo, g_pws.sinv, g_pws.sxhi, g_pws.sxlo, Mixture{x, part, gate, k});
