@@ -2397,20 +2397,23 @@ extern "C" int cai_attn_decode(cai_kv_t kv, int layer, const float* qkv, int q_h
     CAI_HIP(hipMemcpyAsync(kv->d_len, c.h_small, sizeof(int32_t), hipMemcpyHostToDevice, c.stream));
   }
   kv->geo_rows = kv_bucket_rows(kv, len + 1);
+  (void)hipGetLastError();      // what an earlier call of this thread left is no error of these launches
   rc = launch_attn_step(kv, layer, d_qkv, 0, 1, q_heads, window, softcap, nullptr, d_pos, d_out, 0, 0, 0, nullptr);
   if (rc) return rc;
+  CAI_HIP(hipGetLastError());
   if (flags & CAI_Y_DEVICE) {
     // The signal behind the row says that launches can read it: memory of this card.  A row anywhere else (pinned, managed, a peer's) is there for the host
     // when the stream has ended.  40 / 8 heads x 128 behind 8191 int8 rows: 23.9 us with hipStreamSynchronize, 20.4 with the signal (the question
     // about the address is asked while the kernels run).
     hipPointerAttribute_t at{};
-    const bool here = hipPointerGetAttributes(&at, out) == hipSuccess && at.type == hipMemoryTypeDevice && at.device == c.device;
-    if (here) {
+    const bool known = hipPointerGetAttributes(&at, out) == hipSuccess;
+    if (!known) (void)hipGetLastError();      // (the question's)
+    if (known && at.type == hipMemoryTypeDevice && at.device == c.device) {
       const HostSignal done = host_signal_next();
       launch_host_signal(done);
       CAI_HIP(hipGetLastError());
       rc = host_signal_wait(done); if (rc) return rc;
-    } else { (void)hipGetLastError(); CAI_HIP(hipStreamSynchronize(c.stream)); }
+    } else CAI_HIP(hipStreamSynchronize(c.stream));
   } else {
     const HostCopy res = {out, d_out, out_b};
     rc = fetch_to_host(&res, 1); if (rc) return rc;

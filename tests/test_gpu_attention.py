@@ -565,3 +565,21 @@ def test_rows_left_on_the_device_or_in_pinned_memory_are_there_when_the_call_ret
         assert np.array_equal(got.cpu().numpy(), want), p
         cai.check(cai.load().cai_attn_decode(c.h, 0, x[p].data_ptr(), hq, 0, 0.0, z[p].data_ptr(), cai.X_DEVICE | cai.Y_DEVICE))
         assert np.array_equal(z[p].numpy(), want), p
+
+
+@pytest.mark.parametrize("where", ["device", "pinned", "host"])
+def test_an_error_that_another_call_left_is_not_this_call_s(where):
+    """the runtime keeps an error of a thread until someone reads it: a host program's own failing call in front does not make a row of attention fail"""
+    import torch
+    from helpers.device import dev
+    cai = dev()
+    g = np.random.default_rng(1)
+    a, b = cai.KVCache(1, 2, 64, 64, cai.KV_F32), cai.KVCache(1, 2, 64, 64, cai.KV_F32)
+    x, y = g.standard_normal(8 * 64).astype(np.float32), torch.zeros(4 * 64)
+    want = a.attn_decode(0, x, 4)
+    if where != "host":
+        y = y.cuda() if where == "device" else y.pin_memory()
+    torch.cuda.synchronize()
+    assert cai.load().hipGetDevice(None) != 0        # (a null pointer, refused on the host)
+    cai.check(cai.load().cai_attn_decode(b.h, 0, x.ctypes.data, 4, 0, 0.0, y.data_ptr(), 0 if where == "host" else cai.Y_DEVICE))
+    assert np.array_equal(y.cpu().numpy(), want)
