@@ -86,6 +86,7 @@ HostSignal host_signal_next(int k)
 }
 int host_signal_wait(const HostSignal& s)
 {
+  if (s.flag == g_ctx.h_flags) CAI_HIP(hipEventRecord(g_ctx.behind, g_ctx.stream));      // (a call waits for its first signal first, when all its launches are out)
   volatile const uint32_t* const flag = s.flag;
   const auto t0 = std::chrono::steady_clock::now();
   for (int i = 1; *flag != s.value; i++) {
@@ -231,6 +232,7 @@ extern "C" int cai_init(int device_ordinal)
   CAI_HIP(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
   CAI_HIP(hipEventCreate(&c.ev0));
   CAI_HIP(hipEventCreate(&c.ev1));
+  CAI_HIP(hipEventCreateWithFlags(&c.behind, hipEventDisableTiming));
   CAI_HIP(hipMalloc(&c.d_arrive, 64)); CAI_HIP(hipMemset(c.d_arrive, 0, 64));
   CAI_HIP(hipHostMalloc(&c.h_flags, HOST_SIGNALS * 64, hipHostMallocCoherent));
   memset(c.h_flags, 0, HOST_SIGNALS * 64);
@@ -256,6 +258,7 @@ extern "C" int cai_shutdown(void)
   if (c.h_stage) (void)hipHostFree(c.h_stage);
   if (c.tl.buf) (void)hipFree(c.tl.buf);
   (void)hipEventDestroy(c.ev0); (void)hipEventDestroy(c.ev1);
+  if (c.behind) (void)hipEventDestroy(c.behind);
   if (c.d_arrive) (void)hipFree(c.d_arrive);
   if (c.h_flags) (void)hipHostFree(c.h_flags);
   (void)hipStreamDestroy(c.stream);

@@ -26,7 +26,7 @@ struct Context {
   void*  h_stage = nullptr; size_t h_stage_cap = 0;      // pinned host memory of calls that wait for their results (kernels read and write it in place)
   int32_t* d_small = nullptr;            // 1024 ints of device scratch for small arguments/results
   int32_t* h_small = nullptr;            // 1024 ints of pinned host memory paired with d_small
-  uint32_t* h_flags = nullptr; unsigned* d_arrive = nullptr; uint32_t signals = 0;      // HostSignal
+  uint32_t* h_flags = nullptr; unsigned* d_arrive = nullptr; uint32_t signals = 0; hipEvent_t behind = nullptr;      // HostSignal
   // Step timeline (measurement aid, cai_decoder_timeline): while armed, every instrumented launch gets a record of eight
   // wall-clock stamps per work-group (0 entry .. 7 exit, the ones between are the kernel's own) and a descriptor (class,
   // work-groups, offset)
@@ -74,6 +74,9 @@ int  ensure_host_stage(size_t need);   // grows ctx().h_stage; only for calls th
 // What a call's last launch writes into pinned memory when its results there, and what the launches before it wrote, can be read: the host sees it 5 us before the
 // end of the stream (a launch and hipStreamSynchronize 10.9 us, a launch and this 5.6).  The last work-group to arrive writes it; the arrivals wrap to
 // zero.  A wait of more than 50 ms goes on in hipStreamSynchronize, which also returns an error of the launches.
+// An event goes out behind the last launch, while it runs: without one the runtime asks for the stream's end when the host program next
+// synchronises the device, later and at more cost.  us, 40 / 8 heads behind 8191 int8 rows, call after call | one call and hipDeviceSynchronize: hipStreamSynchronize in
+// the call 24.1 | 27.1, the flag alone 20.9 | 32, flag and event 22.1 | 25.6; candidates of 152064 45.6 | 48.6, 44.0 | 55, 45.2 | 47.3; a step of the 135M shape 583 | 586, 575 | 595, 575 | 584.
 constexpr int HOST_SIGNALS = 8;            // of one call
 struct HostSignal { uint32_t* flag = nullptr; unsigned* arrive = nullptr; uint32_t value = 0; };      // flag null: none
 HostSignal host_signal_next(int k = 0);    // the k-th of this call
