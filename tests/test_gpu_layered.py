@@ -91,8 +91,10 @@ def test_gated_products_over_bf16_rows(cai, rows, cols):
     gated_products(cai, rows, cols, (1, 2, 3, 5, 7, 8, 9, 13, 16, 17, 33, 70))
 
 
-@pytest.mark.parametrize("rows, cols, tokens", [(2016, 264, 1100), (6208, 136, 2050)])
+@pytest.mark.parametrize("rows, cols, tokens", [(2016, 264, 1100), (6208, 136, 2050), (2016, 264, 2000), (6208, 136, 2310)])
 def test_gated_products_on_one_round_of_large_tiles(cai, rows, cols, tokens):
+    """tiles of 128 x 128 by sixteen waves and of 256 x 256 (the last two), and what smaller numbers of tokens take"""
+    assert cai.load().cai_bf16_tiles(rows, cols, tokens) == {1100: 1, 2050: 4, 2000: 2, 2310: 5}[tokens]
     gated_products(cai, rows, cols, (tokens,))
 
 
@@ -253,10 +255,13 @@ def test_products_on_large_tiles_of_many_steps(cai, tmp_path, tokens, ff, width)
     dec.close()
 
 
-@pytest.mark.parametrize("rows, cols, tokens", [(2041, 264, 1100), (4300, 72, 513), (16300, 320, 130), (6200, 328, 2050), (4104, 72, 2100)])
-def test_one_round_of_large_tiles(cai, rows, cols, tokens):
-    """Tiles of 128 x 128 by sixteen waves (one round of them that has more than two tiles of 64 x 64 a CU: the first three) and of 256 x 256 (one round instead
-    of two of 256 x 128), one to six steps of 64 deep, rows and tokens that end inside a tile.  The bound is that of test_products_over_bf16_rows."""
+@pytest.mark.parametrize("rows, cols, tokens, tiles", [(2041, 264, 1100, 1), (4300, 72, 513, 1), (16300, 320, 130, 4), (6200, 328, 2050, 4), (4104, 72, 2100, 3),
+                                                      (2041, 264, 2000, 2), (4300, 72, 890, 2), (16300, 320, 193, 2), (16300, 1096, 130, 2), (6200, 328, 2310, 5), (4104, 72, 3810, 5), (4104, 776, 2050, 5)])
+def test_one_round_of_large_tiles(cai, rows, cols, tokens, tiles):
+    """Tiles of 128 x 128 by sixteen waves (2: one round of them) and of 256 x 256 (5: one round instead of two of smaller ones), one to eighteen steps of 64 deep, rows and
+    tokens that end inside a tile; and what sizes a little below them take (1: 64 x 64, 3: 128 x 128 by eight waves, 4: 256 x 128).  The bound is that of
+    test_products_over_bf16_rows."""
+    assert cai.load().cai_bf16_tiles(rows, cols, tokens) == tiles
     rng = np.random.default_rng(rows)
     bits, w = B.to_bf16(rng.standard_normal((rows, cols)))
     w = w.reshape(rows, cols).astype(np.float64); bias = rng.standard_normal(rows).astype(np.float32)
@@ -266,10 +271,13 @@ def test_one_round_of_large_tiles(cai, rows, cols, tokens):
     q.close()
 
 
-@pytest.mark.parametrize("width, tokens", [(2056, 1100), (4104, 2050), (2054, 1090)])
-def test_residuals_of_large_tiles(cai, tmp_path, width, tokens):
-    """the stream's update and the norms around it behind tiles of 128 x 128 by sixteen waves and of 256 x 256; a width that is no whole fours"""
-    m = Model(tmp_path, B.config([B.layer(B.delta(1, 1, 8, 8, 2), ff=72)], width=width, vocab=67), seed=width, rank_a=3, rank_g=20)
+@pytest.mark.parametrize("width, tokens, ff", [(2056, 1100, 72), (4104, 2050, 72), (2054, 1090, 72), (2056, 1100, 1032), (4104, 2050, 776), (2054, 1090, 1032)])
+def test_residuals_of_large_tiles(cai, tmp_path, width, tokens, ff):
+    """the stream's update and the norms around it behind tiles of 128 x 128 by sixteen waves and of 256 x 256 (ff of 1032 and of 776, depths at which they are taken), and behind
+    the tiles of shallow products; a width that is no whole fours"""
+    if ff > 72:
+        assert cai.load().cai_bf16_tiles(width, ff, tokens) == (5 if ff == 776 else 2)
+    m = Model(tmp_path, B.config([B.layer(B.delta(1, 1, 8, 8, 2), ff=ff)], width=width, vocab=67), seed=width, rank_a=3, rank_g=20)
     tok = m.tokens(tokens, 1)
     dec = m.open(cai, 2112, 1, "bf16")
     check(feed(dec, tok, [tokens]), m.ref(tok), "bf16")
