@@ -282,16 +282,20 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const DeltaDims d, floa
 // ------------------------------------------------------------------------------------------
 constexpr int CHUNK = DELTA_CHUNK;
 
+// The chunks of a launch and their records: all of a step as listed, or (chunks null) of every entry those from `first` on, `most` records each
+struct DeltaPass { const int32_t *chunks, *chunk0; int first, most; };
+
 template <bool CH>
-__global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaDims d, const StepRows r, const DeltaBuf b, const int32_t* chunks)
+__global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaDims d, const StepRows r, const DeltaBuf b, const DeltaPass p)
 {
   extern __shared__ float lds[];
   __shared__ float sA[CHUNK][CHUNK + 1], sQ[CHUNK][CHUNK + 1], sP[CH ? 1 : 4][CHUNK][CHUNK + 1];
   __shared__ f32x4 sT[CHUNK][CHUNK / 4];
   __shared__ float sbeta[CHUNK], sg1[CHUNK], sdot[CHUNK], sz[CHUNK];      // sdot: q . k, later (one decay a head) the running products of the decays
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), fr = lane & 15, fg = lane >> 4;
-  const int32_t* en = r.ent + 4 * chunks[2 * blockIdx.x];
-  const int t0 = chunks[2 * blockIdx.x + 1], nt = min(CHUNK, en[2] - t0), h = blockIdx.y;
+  const int32_t* en = r.ent + 4 * (p.chunks ? p.chunks[2 * blockIdx.x] : (int)blockIdx.x / p.most);
+  const int t0 = p.chunks ? p.chunks[2 * blockIdx.x + 1] : (p.first + (int)blockIdx.x % p.most) * CHUNK, nt = min(CHUNK, en[2] - t0), h = blockIdx.y;
+  if (nt <= 0) return;                     // (whole work-groups: an entry that ends before the pass does)
   const int64_t row0 = en[1] + t0;
   const int g = h / (d.heads / d.kv_heads), kw = d.kv_heads * d.dim, vw = d.heads * d.vdim, gw = d.heads * d.dim, bw = d.heads + d.kv_heads;
   const int dp = (d.dim + 15) & ~15, DS = dp + 4, tiles = delta_tiles(d);
@@ -442,7 +446,7 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaDims d, con
 // them waiting for the other waves.  U0 as the start of a state wave's sums and U handed to wave NW took 102 us where this takes 96, factors
 // five chunks ahead 92 to 98, the read-out in front of the barrier or around it 98 to 100.
 template <int NW, int TPW, bool CH, bool WHOLE>      // WHOLE: the value width is a multiple of sixteen
-__global__ __launch_bounds__(64 * (NW + 1)) void delta_walk_kernel(const DeltaDims d, float* state, const int64_t s_elems, const StepRows r, const DeltaBuf b, const int32_t* chunk0)
+__global__ __launch_bounds__(64 * (NW + 1)) void delta_walk_kernel(const DeltaDims d, float* state, const int64_t s_elems, const StepRows r, const DeltaBuf b, const DeltaPass p)
 {
   constexpr int TILES = NW * TPW;
   __shared__ f32x4 pu[3][NW + 1][64], po[3][NW][64];
@@ -453,7 +457,8 @@ __global__ __launch_bounds__(64 * (NW + 1)) void delta_walk_kernel(const DeltaDi
   const int h = d.heads % 8 == 0 ? (blockIdx.x & 7) + 8 * ((blockIdx.x >> 3) / slices) : blockIdx.x / slices;
   const int slice = d.heads % 8 == 0 ? (blockIdx.x >> 3) % slices : blockIdx.x % slices, col = slice * 16 + fr;
   const int32_t* en = r.ent + 4 * blockIdx.y;
-  const int slot = en[0], row0 = en[1], n = en[2], pos0 = en[3], ch0 = chunk0[blockIdx.y];
+  const int skip = p.first * CHUNK, slot = en[0], row0 = en[1] + skip, n = min(en[2] - skip, p.most * CHUNK), pos0 = en[3] + skip, ch0 = p.chunks ? p.chunk0[blockIdx.y] : (int)blockIdx.y * p.most;
+  if (n <= 0) return;
   const int vw = d.heads * d.vdim, dvp = d.vdim_p(), blocks = delta_record_blocks(d);
   const int nc = (n + CHUNK - 1) / CHUNK;
   const f32x4* const rec = reinterpret_cast<const f32x4*>(b.rec) + ((int64_t)ch0 * d.heads + h) * (64 * blocks);
@@ -887,20 +892,34 @@ int delta_scan(const DeltaDims& d, const SeqPool::StateRun& st, const StepRows& 
   return CAI_OK;
 }
 
-int delta_chunked(const DeltaDims& d, const SeqPool::StateRun& st, const StepRows& r, const DeltaBuf& b, const int32_t* chunks, int n_chunks, const int32_t* chunk0)
+static int delta_pass(const DeltaDims& d, const SeqPool::StateRun& st, const StepRows& r, const DeltaBuf& b, const DeltaPass& p, int n_chunks)
 {
   auto s = ctx().stream;
   const size_t lds = (size_t)(d.channel_decay ? 3 : 2) * CHUNK * (((d.dim + 15) & ~15) + 4) * 4;
   const dim3 g1(n_chunks, d.heads), g2((d.vdim + 15) / 16 * d.heads, r.n_ent), blk(256);
-  if (d.channel_decay) hipLaunchKernelGGL(delta_chunk_kernel<true>, g1, blk, lds, s, d, r, b, chunks);
-  else hipLaunchKernelGGL(delta_chunk_kernel<false>, g1, blk, lds, s, d, r, b, chunks);
-#define WALK_C(NW, N, CH) do { if (d.vdim % 16 == 0) hipLaunchKernelGGL((delta_walk_kernel<NW, N, CH, true>), g2, dim3(64 * (NW + 1)), 0, s, d, st.S, st.s_elems, r, b, chunk0); \
-                               else hipLaunchKernelGGL((delta_walk_kernel<NW, N, CH, false>), g2, dim3(64 * (NW + 1)), 0, s, d, st.S, st.s_elems, r, b, chunk0); } while (0)
+  if (d.channel_decay) hipLaunchKernelGGL(delta_chunk_kernel<true>, g1, blk, lds, s, d, r, b, p);
+  else hipLaunchKernelGGL(delta_chunk_kernel<false>, g1, blk, lds, s, d, r, b, p);
+#define WALK_C(NW, N, CH) do { if (d.vdim % 16 == 0) hipLaunchKernelGGL((delta_walk_kernel<NW, N, CH, true>), g2, dim3(64 * (NW + 1)), 0, s, d, st.S, st.s_elems, r, b, p); \
+                               else hipLaunchKernelGGL((delta_walk_kernel<NW, N, CH, false>), g2, dim3(64 * (NW + 1)), 0, s, d, st.S, st.s_elems, r, b, p); } while (0)
 #define WALK(NW, N) do { if (d.channel_decay) WALK_C(NW, N, true); else WALK_C(NW, N, false); } while (0)
   switch (delta_tiles(d)) { case 4: WALK(4, 1); break; case 8: WALK(4, 2); break; default: WALK(8, 2); break; }
 #undef WALK_C
 #undef WALK
   CAI_HIP(hipGetLastError());
+  return CAI_OK;
+}
+
+int delta_chunked(const DeltaDims& d, const SeqPool::StateRun& st, const StepRows& r, const DeltaBuf& b, const int32_t* chunks, int n_chunks, const int32_t* chunk0, int longest)
+{
+  const int64_t room = b.rec_floats / ((int64_t)d.heads * delta_record_blocks(d) * 256);      // chunks whose records b.rec holds: one of every entry at least
+  if (n_chunks <= room) return delta_pass(d, st, r, b, DeltaPass{chunks, chunk0, 0, n_chunks}, n_chunks);
+  if (room < r.n_ent) return set_error(CAI_ERR_STATE, "delta rule: records of %lld chunks for %d sequences", (long long)room, r.n_ent);
+  // passes over time, all entries together: they walk side by side as in one pass
+  const int most = (int)(room / r.n_ent);
+  for (int first = 0; first < longest; first += most) {
+    const int rc = delta_pass(d, st, r, b, DeltaPass{nullptr, nullptr, first, most}, r.n_ent * most);
+    if (rc) return rc;
+  }
   return CAI_OK;
 }
 

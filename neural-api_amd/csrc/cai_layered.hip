@@ -336,6 +336,8 @@ static int ensure_rows(LayeredNet* n, int rows)
   };
   const size_t RS = R + DELTA_CHUNK + 1;    // the walk of the gated linear attention requests whole chunks: up to 15 rows (and three values) past the last one
   const size_t chunks = R / DELTA_CHUNK + n->max_seq + 1;
+  const size_t rec = std::min(chunks * n->w_rec * 4, std::max(DELTA_REC_BYTES, (size_t)n->max_seq * n->w_rec * 4));
+  n->db.rec_floats = (int64_t)(rec / 4);
   size_t part = 0;
   // (with bfloat16 activations only steps without a prompt portion take the row form)
   const int part_rows = n->act_t == ACT_T_F32 ? (int)R : std::min((int)R, ATTN_PROMPT_MIN * n->max_seq);
@@ -350,7 +352,7 @@ static int ensure_rows(LayeredNet* n, int rows)
       (rc = get((void**)&n->db.q, RS * n->w_q * 4)) || (rc = get((void**)&n->db.k, RS * n->w_k * 4)) || (rc = get((void**)&n->db.v, RS * n->w_v * 4)) ||
       (rc = get((void**)&n->db.g, RS * n->w_g * 4)) || (rc = get((void**)&n->db.beta, RS * n->w_b * 4)) || (rc = get((void**)&n->db.o, RS * n->w_v * 4)) ||
       (rc = get((void**)&n->db.za, R * n->w_za * 4)) || (rc = get((void**)&n->db.zg, R * n->w_zg * 4)) ||
-      (rc = get((void**)&n->db.rec, chunks * n->w_rec * 4)) || (rc = get((void**)&n->db.qt, RS * n->w_qt * 4)) || (rc = get((void**)&n->db.qk, RS * n->w_qk * 4)) ||
+      (rc = get((void**)&n->db.rec, rec)) || (rc = get((void**)&n->db.qt, RS * n->w_qt * 4)) || (rc = get((void**)&n->db.qk, RS * n->w_qk * 4)) ||
       (rc = get((void**)&n->db.gt, n->w_gt ? (chunks * n->w_gt + 4) * 4 : 0)) ||
       (rc = get(&n->cat, R * n->ld_cat * n->es)) || (rc = get(&n->h2, R * n->ld_h2 * n->es)) || (rc = get((void**)&n->g2, R * n->ld_g2 * 4)) ||
       (rc = get((void**)&n->kept, n->has_sandwich ? (n->s.layers.size() + 1) * R * w * 4 : 0)) || (rc = get((void**)&n->inv, n->has_sandwich ? R * 4 : 0)) ||
@@ -522,7 +524,7 @@ static_assert(ATTN_TILE == SSD_CHUNK, "one list of tiles serves the prompt atten
 // the first row of every such entry there, their tiles, and the rows of the other entries.
 struct StepLists {
   const int32_t *tiles = nullptr, *tile0 = nullptr; int n_tiles = 0; bool tall = false;
-  const int32_t* chunks = nullptr; int n_chunks = 0; const int32_t* chunk0 = nullptr; bool chunked = false;
+  const int32_t* chunks = nullptr; int n_chunks = 0; const int32_t* chunk0 = nullptr; int longest = 0; bool chunked = false;
   const int32_t *pages = nullptr, *row0 = nullptr, *wide = nullptr, *short_rows = nullptr; int n_pages = 0, n_wide = 0, n_short = 0;
 };
 
@@ -756,7 +758,7 @@ static int enqueue_net(LayeredNet* n, const StepRows& r, bool single, const Step
           if ((rc = launch_pack_rows(n->proj, n->ld_proj, D.og, D.d.rank_g, R, at, n->rgb, n->ld_rg)) || (rc = launch_lin(D.w.g2, at, n->rgb, n->ld_rg, R, e))) return rc;
         }
         if ((rc = delta_prep(D.d, din, D.w, ds, r, n->db)) ||
-            (rc = lists.chunked ? delta_chunked(D.d, ds, r, n->db, lists.chunks, lists.n_chunks, lists.chunk0) : delta_scan(D.d, ds, r, n->db)) ||
+            (rc = lists.chunked ? delta_chunked(D.d, ds, r, n->db, lists.chunks, lists.n_chunks, lists.chunk0, lists.longest) : delta_scan(D.d, ds, r, n->db)) ||
             (rc = delta_finish(D.d, din, D.w, ds, r, n->db, at, n->att, n->ld_att))) return rc;
       }
     }
@@ -878,8 +880,9 @@ int net_step(LayeredNet* n, int n_ent, const int32_t* seq, const int32_t* count,
     // rows, entries, tiles of the prompt attention kernel, wanted rows
     std::vector<int32_t> tiles, tile0, chunks, chunk0, pages, row0, wide, short_rows;
     bool tall = false, chunked = false;
-    int end = 0;
+    int end = 0, longest = 0;
     for (int e = 0; e < n_ent; e++) {
+      longest = std::max(longest, (count[e] + DELTA_CHUNK - 1) / DELTA_CHUNK);
       end = std::max(end, n->pool.seq[seq[e]].len + count[e]);
       tall = tall || count[e] >= ATTN_PROMPT_MIN; chunked = chunked || count[e] >= DELTA_CHUNK_MIN;
       chunk0.push_back((int)chunks.size() / 2); tile0.push_back((int)tiles.size() / 2);
@@ -921,7 +924,7 @@ int net_step(LayeredNet* n, int n_ent, const int32_t* seq, const int32_t* count,
     auto next = [&](const std::vector<int32_t>& v) { const int32_t* p = at; at += v.size(); return p; };
     StepLists lists;
     lists.tiles = next(tiles); lists.n_tiles = (int)tiles.size() / 2; lists.tile0 = next(tile0); lists.tall = tall;
-    lists.chunks = next(chunks); lists.n_chunks = (int)chunks.size() / 2; lists.chunk0 = next(chunk0); lists.chunked = chunked;
+    lists.chunks = next(chunks); lists.n_chunks = (int)chunks.size() / 2; lists.chunk0 = next(chunk0); lists.longest = longest; lists.chunked = chunked;
     lists.pages = next(pages); lists.n_pages = (int)pages.size() / 2; lists.row0 = next(row0);
     lists.wide = next(wide); lists.n_wide = (int)wide.size() / 2; lists.short_rows = next(short_rows); lists.n_short = (int)short_rows.size();
     if ((rc = enqueue_net(n, r, false, lists, next(wrows), W))) return rc;

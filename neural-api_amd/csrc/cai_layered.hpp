@@ -236,17 +236,20 @@ struct DeltaW {
 };
 struct DeltaBuf {                          // per-row scratch of a prompt pass
   float *q, *k, *v, *g, *beta, *o, *za, *zg;
-  float *rec;                              // chunked delta rule: a record of matrix operands per chunk and head (delta_record_blocks KB)
+  float *rec; int64_t rec_floats;          // chunked delta rule: a record of matrix operands per chunk and head (delta_record_blocks KB), as many as DELTA_REC_BYTES hold
   float *qt, *qk;                          // chunked gated linear attention: P q, q D k
   float *gt;                               // both: the decays of whole chunks
 };
 constexpr int DELTA_CHUNK = 16;            // tokens per chunk
 __host__ __device__ inline int delta_tiles(const DeltaDims& d) { return d.dim <= 64 ? 4 : d.dim <= 128 ? 8 : 16; }                  // of 16 key channels, as the walk's waves share them
 __host__ __device__ inline int delta_record_blocks(const DeltaDims& d) { return 3 * delta_tiles(d) + 1 + (d.vdim + 15) / 16; }      // of [64 lanes][4] floats
+// Records of a step that lie side by side: 16000 tokens of 16 heads of 128 x 128 (33 KB a chunk and head; a step of 131072 rows of 32 such heads would need 8.9 GB).  A longer step
+// makes and walks them in passes, whose first chunk takes up the state where the last pass left it.
+constexpr size_t DELTA_REC_BYTES = (size_t)512 << 20;
 constexpr int DELTA_CHUNK_MIN = 32;        // portions from here on make a step take the chunked form
 int delta_prep(const DeltaDims& d, const DeltaIn& in, const DeltaW& w, const SeqPool::StateRun& st, const StepRows& r, const DeltaBuf& b);
 int delta_scan(const DeltaDims& d, const SeqPool::StateRun& st, const StepRows& r, const DeltaBuf& b);
-int delta_chunked(const DeltaDims& d, const SeqPool::StateRun& st, const StepRows& r, const DeltaBuf& b, const int32_t* chunks, int n_chunks, const int32_t* chunk0);   // chunks: entry, first row in it; chunk0: first chunk of each entry
+int delta_chunked(const DeltaDims& d, const SeqPool::StateRun& st, const StepRows& r, const DeltaBuf& b, const int32_t* chunks, int n_chunks, const int32_t* chunk0, int longest);   // chunks: entry, first row in it; chunk0: first chunk of each entry; longest: chunks of the longest
 int delta_finish(const DeltaDims& d, const DeltaIn& in, const DeltaW& w, const SeqPool::StateRun& st, const StepRows& r, const DeltaBuf& b, int act_t, void* out, int64_t ldo);
 int delta_single(const DeltaDims& d, const DeltaIn& in, const DeltaW& w, const SeqPool::StateRun& st, const StepRows& r, int act_t, void* out, int64_t ldo);
 

@@ -233,6 +233,37 @@ def test_dynamic_tanh_is_as_near_as_the_library_s(cai, tmp_path):
     assert off[np.abs(x) < 1].max() < 2.45 and off[np.abs(x) >= 1].max() < 1.27, (off[np.abs(x) < 1].max(), off[np.abs(x) >= 1].max())
 
 
+@pytest.mark.parametrize("counts", [(30001,), (20000, 6400, 40, 1), (585 * 16, 17)])
+@pytest.mark.parametrize("mech", ["delta", "channel delta"])
+def test_long_steps_walk_their_records_in_passes(cai, tmp_path, mech, counts):
+    """Records of 64 heads are 896 KB a chunk, so 585 chunks lie side by side: steps of three passes, of passes that an entry ends before, in or at the end of, and of one chunk more than
+    a pass holds.  The sequences are those of portions that are one pass each, from the same chunks (32-bit products by other tiles are the only difference), and what a
+    step of 30001 rows takes on the device is less than its records alone would be (1.72 GB)."""
+    import torch
+    mixer = B.delta(64, 64, 8, 8, 4)
+    m = Model(tmp_path, B.config([B.layer(mixer if mech == "delta" else (B.attn(), mixer))], width=72, vocab=67), seed=len(counts), edit=only(mech), rank_a=9, rank_g=20)
+    toks = [m.tokens(n, n) for n in counts]
+    rows = [sorted({n // 2, max(n - 2, 0), n - 1}) for n in counts]
+    want = []
+    dec = m.open(cai, sum(-(-n // 64) + 1 for n in counts) * 64, len(counts), "f32")
+    for e, (t, w) in enumerate(zip(toks, rows)):
+        for i in range(0, len(t), 4096):
+            here = [k - i for k in w if i <= k < i + 4096]
+            got = dec.step_batch([(e, t[i:i + 4096], here)])[1]
+            want += list(got) if here else []
+    dec.close()
+    dec = m.open(cai, sum(-(-n // 64) + 1 for n in counts) * 64, len(counts), "f32")
+    before = torch.cuda.mem_get_info()[0]
+    got = dec.step_batch([(e, t, w) for e, (t, w) in enumerate(zip(toks, rows))])[1]
+    taken = before - torch.cuda.mem_get_info()[0]
+    assert err(np.asarray(got, np.float64), np.asarray(want, np.float64)) < 1e-5
+    after = dec.step_batch([(e, [5], [0]) for e in range(len(counts))])[1]      # (from the states they left)
+    dec.close()
+    assert np.isfinite(after).all()
+    if counts == (30001,) and mech == "delta":
+        assert taken < 1.6e9, taken
+
+
 @pytest.mark.parametrize("tokens, ff", [(129, 16400), (257, 8208), (300, 12000)])
 def test_products_on_tiles_of_256_tokens(cai, tmp_path, tokens, ff):
     """gate | up matrices whose products fill the chip with large tiles: tokens one past half a tile, one past a tile and inside a second one, rows
