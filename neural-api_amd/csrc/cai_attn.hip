@@ -1480,11 +1480,13 @@ typedef float pf16_t __attribute__((ext_vector_type(16)));
 struct PromptParams {
   const float* qkv; int64_t qkv_stride;      // rows [Q | K | V]
   _Float16* qhi; _Float16* qlo;              // [token][q_heads * HD] rotated q, hi + lo
-  _Float16* planes;                          // [kv_head][n_tiles] tiles of 32 cached rows: PromptShape::TILE halfs
-  float* rsc;                                // PromptShape::ROWS: [kv_head][n_tiles][K 32 | V 32] what a row's planes are to be multiplied by
+  int head0, heads;                          // the launch's KV heads
+  int tile0, n_tiles;                        // the tiles of 32 cached rows that the chunk's tokens see
+  _Float16* planes;                          // [head0 + ..][tile0 + ..] PromptShape::TILE halfs
+  float* rsc;                                // PromptShape::ROWS: likewise [K 32 | V 32] what a row's planes are to be multiplied by
   void* kc; void* vc;                        // this sequence's layer plane: [kv_head][max_ctx][HD]
   const float* ksc; const float* vsc;        // int8 cache: row scales of the same plane, [kv_head][max_ctx]
-  int q_heads, kv_heads, max_ctx, n_tok, n_tiles, window;
+  int q_heads, kv_heads, max_ctx, n_tok, window;
   float softcap, inv_sqrt;
   const float* theta; int pos0;              // token t: position pos0 + t of the sequence
   float* out; int64_t out_stride;
@@ -1542,20 +1544,19 @@ __device__ __forceinline__ void prompt_q_row(const PromptParams& p, const int t)
   }
 }
 
-// Work-groups 0 .. n_tiles * kv_heads - 1: 32 cached rows of a KV head each, those of the chunk from its K and V (an int8 cache has them already);
-// the others: a token's q.
+// Work-groups 0 .. n_tiles * heads - 1: 32 cached rows of a KV head each, those of the chunk from its K and V (an int8 cache has them already);
+// the others (with the first heads): a token's q.
 template <typename KV_T, int HD>
 __global__ __launch_bounds__(256) void prompt_rows_kernel(const PromptParams p)
 {
   using S = PromptShape<KV_T, HD>;
   constexpr int E = HD / 8, DT = HD / 32, LDF = HD + 4;
   __shared__ __align__(16) float sv[32 * LDF];
-  const int tiles = p.n_tiles * p.kv_heads, tid = threadIdx.x;
+  const int tiles = p.n_tiles * p.heads, tid = threadIdx.x;
   if ((int)blockIdx.x >= tiles) { prompt_q_row<HD>(p, blockIdx.x - tiles); return; }
-  const int g = blockIdx.x % p.kv_heads, jt = blockIdx.x / p.kv_heads;
+  const int g = p.head0 + blockIdx.x % p.heads, jt = p.tile0 + blockIdx.x / p.heads;
+  const int64_t place = (int64_t)(blockIdx.x % p.heads) * p.n_tiles + blockIdx.x / p.heads;
   const int pos0 = p.pos0, last = pos0 + p.n_tok - 1;
-  const int lo = p.window > 0 && pos0 + 1 > p.window ? pos0 + 1 - p.window : 0;
-  if (32 * jt > last || jt < (lo >> 5)) return;                    // (whole work-groups)
   const int r = tid >> 3, d0 = (tid & 7) * E, j = 32 * jt + r;     // E consecutive elements of a cached row
   const bool live = j <= last;
   const int64_t at = ((int64_t)g * p.max_ctx + min(j, last)) * HD + d0;
@@ -1617,10 +1618,10 @@ __global__ __launch_bounds__(256) void prompt_rows_kernel(const PromptParams p)
       for (int i = 0; i < E; i++) { k[i] = ldexpf(k[i], ek); v[i] = ldexpf(v[i], ev); }
       ks = ldexpf(1.0f, -ek); vs = ldexpf(1.0f, -ev);
     }
-    if ((tid & 7) == 0) { float* s = p.rsc + ((int64_t)g * p.n_tiles + jt) * 64 + r; s[0] = ks; s[32] = vs; }
+    if ((tid & 7) == 0) { float* s = p.rsc + place * 64 + r; s[0] = ks; s[32] = vs; }
   }
   auto split = [](float x, _Float16& h, _Float16& l) { if (S::SC) split_plane(x, h, l); else split_f16(x, h, l); };
-  _Float16* tile = p.planes + ((int64_t)g * p.n_tiles + jt) * S::TILE;
+  _Float16* tile = p.planes + place * S::TILE;
 #pragma unroll
   for (int i8 = 0; i8 < E; i8 += 8) {         // dims d0 + i8 .. + 7: step d / 16, lane half (d / 8) % 2, row r
     ph8_t h, l;
@@ -1664,7 +1665,7 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(const PromptParams 
   __shared__ float sM[4][32], sL[4][32];
   _Float16* sQ = reinterpret_cast<_Float16*>(lds);
   float* sO = reinterpret_cast<float*>(lds);
-  const int head = blockIdx.x, g = head / (p.q_heads / p.kv_heads);
+  const int G = p.q_heads / p.kv_heads, head = p.head0 * G + blockIdx.x, g = blockIdx.x / G;      // (g: of the launch's)
   const int t0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * 32;                 // the longest ranges first
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, n = lane & 31, kg = lane >> 5;
   const int tok = t0 + n;
@@ -1682,8 +1683,8 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(const PromptParams 
   }
   // The operands of the wave's next tile are requested as soon as the registers of the current one are free: K's run behind the weights and the second
   // product, V's behind the next tile's first product.
-  const _Float16* planes = p.planes + (int64_t)g * p.n_tiles * S::TILE + 8 * lane;
-  const float* scales = ROWS ? p.rsc + (int64_t)g * p.n_tiles * 64 + 4 * kg : nullptr;
+  const _Float16* planes = p.planes + ((int64_t)g * p.n_tiles - p.tile0) * S::TILE + 8 * lane;
+  const float* scales = ROWS ? p.rsc + ((int64_t)g * p.n_tiles - p.tile0) * 64 + 4 * kg : nullptr;
   ph8_t K[NP][STEPS], V[NP][2 * DT];
   float4 rk[ROWS ? 4 : 1], rv[ROWS ? 4 : 1];
   auto load_k = [&](int jt) __attribute__((always_inline)) {
@@ -1948,20 +1949,24 @@ int launch_attn_step(cai_kv_s* kv, int layer, float* qkv, int64_t qkv_stride, in
   }
   if (flash) {
     if (kv->prompt_end < n_seq || kv->prompt_end > kv->max_ctx) return set_error(CAI_ERR_STATE, "attention: a prompt of %d rows ends at row %d of %d", n_seq, kv->prompt_end, kv->max_ctx);
-    const int tok_tiles = (n_seq + 31) / 32, n_tiles = (kv->prompt_end + 31) / 32;
+    const int pos0 = kv->prompt_end - n_seq, tok_tiles = (n_seq + 31) / 32;
+    const int tile0 = window > 0 && pos0 + 1 > window ? (pos0 + 1 - window) / 32 : 0, n_tiles = (kv->prompt_end + 31) / 32 - tile0;      // a window's rows, not the cache's
     // K splits per token tile: a work-group takes a CU's half, so the range is cut where that shortens (rounds of work-groups) / splits by a fifth or more, and
     // never to less than two tiles a wave.  Three layers of the 28 / 4 heads shape, whole prompts: 16 tokens behind 4096 rows 387 us uncut, 249 in eight; 300 behind 7000
     // 855, 699 in three; 64 behind 2000 325, 277; a single tile a wave (a limit of four tiles a work-group) changes nothing at 28 / 4.
     int n_ks = 1;
     auto rounds = [&](int k) { return (tok_tiles * q_heads * k + 2 * c.n_cu - 1) / (2 * c.n_cu) / (double)k; };
     for (int k = 2; k <= std::min(PA_KS_MAX, n_tiles / PA_KT_MIN); k++) if (rounds(k) <= 0.8 * rounds(n_ks)) n_ks = k;
-    // One piece of memory: q's planes, their scales, the cached rows' planes (as large as the rows are as floats or halfs, of one layer and
-    // sequence) and scales, the pieces' sums.  Tiles are counted up to a power of two, so that the chunks of a long prompt find it large enough.
+    // One piece of memory: q's planes, their scales, the cached rows' planes (as large as the rows are as floats or halfs) and scales, the pieces' sums.  Tiles are counted up to a
+    // power of two, so that the chunks of a long prompt find it large enough.  The planes hold the rows of one layer and sequence, of as many KV heads at a time as 512 MB take
+    // (eight of 128 behind 65536 float or int8 rows), so that a cache that leaves little room beside it can be filled.
     const int np = p.hd == 64 ? (kv->dtype == CAI_KV_F32 ? 2 : 1) : (kv->dtype == CAI_KV_F16 ? 1 : 2);
     int most = 16; while (most < n_tiles) most *= 2;
     most = std::min(most, (kv->max_ctx + 31) / 32);
     const size_t q_b = (size_t)n_seq * q_heads * p.hd * 2, s_b = ((size_t)n_seq * q_heads * 4 + 255) / 256 * 256;
-    const size_t t_b = (size_t)most * kv->kv_heads * (4 * np * 32 * p.hd), r_b = (size_t)most * kv->kv_heads * 256;
+    const size_t head_b = (size_t)most * (4 * np * 32 * p.hd);
+    const int at_once = (int)std::min<size_t>(kv->kv_heads, std::max<size_t>(1, ((size_t)512 << 20) / head_b)), turns = (kv->kv_heads + at_once - 1) / at_once, heads = (kv->kv_heads + turns - 1) / turns;
+    const size_t t_b = heads * head_b, r_b = (size_t)most * heads * 256;
     const size_t need = 2 * q_b + s_b + t_b + r_b + (n_ks > 1 ? (size_t)n_seq * q_heads * n_ks * (p.hd + 2) * 4 : 0);
     if (need > kv->pq_cap) {
       CAI_HIP(hipStreamSynchronize(c.stream));
@@ -1980,15 +1985,18 @@ int launch_attn_step(cai_kv_s* kv, int layer, float* qkv, int64_t qkv_stride, in
       const size_t rows0 = (size_t)seq0 * kv->seq_rows() + (size_t)layer * kv->layer_rows();
       pp.ksc = kv->ks + rows0; pp.vsc = kv->vs + rows0;
     }
-    pp.q_heads = q_heads; pp.kv_heads = kv->kv_heads; pp.max_ctx = kv->max_ctx; pp.n_tok = n_seq; pp.n_tiles = n_tiles; pp.window = window;
-    pp.softcap = softcap; pp.inv_sqrt = p.inv_sqrt; pp.theta = theta; pp.pos0 = kv->prompt_end - n_seq; pp.planes_out = p.planes; pp.planes_q8 = p.planes_q8; pp.out = out; pp.out_stride = out_stride;
-    const dim3 rows(n_tiles * kv->kv_heads + n_seq), grid(q_heads, tok_tiles, n_ks);
+    pp.q_heads = q_heads; pp.kv_heads = kv->kv_heads; pp.max_ctx = kv->max_ctx; pp.n_tok = n_seq; pp.tile0 = tile0; pp.n_tiles = n_tiles; pp.window = window;
+    pp.softcap = softcap; pp.inv_sqrt = p.inv_sqrt; pp.theta = theta; pp.pos0 = pos0; pp.planes_out = p.planes; pp.planes_q8 = p.planes_q8; pp.out = out; pp.out_stride = out_stride;
+    const int G = q_heads / kv->kv_heads;
     auto go = [&](auto hd_) {
       constexpr int HD = hd_;
       auto both = [&](auto kv_) {
         using KV_T = decltype(kv_);
-        hipLaunchKernelGGL((prompt_rows_kernel<KV_T, HD>), rows, dim3(256), 0, c.stream, pp);
-        hipLaunchKernelGGL((attn_prompt_kernel<KV_T, HD>), grid, dim3(256), 0, c.stream, pp);
+        for (pp.head0 = 0; pp.head0 < kv->kv_heads; pp.head0 += heads) {
+          pp.heads = std::min(heads, kv->kv_heads - pp.head0);
+          hipLaunchKernelGGL((prompt_rows_kernel<KV_T, HD>), dim3(n_tiles * pp.heads + (pp.head0 ? 0 : n_seq)), dim3(256), 0, c.stream, pp);
+          hipLaunchKernelGGL((attn_prompt_kernel<KV_T, HD>), dim3(pp.heads * G, tok_tiles, n_ks), dim3(256), 0, c.stream, pp);
+        }
       };
       if (kv->dtype == CAI_KV_F16) both(__half()); else if (kv->dtype == CAI_KV_I8) both(int8_t()); else both(float());
       if (n_ks > 1) hipLaunchKernelGGL(prompt_merge_kernel<HD>, dim3(n_seq, (q_heads + 3) / 4), dim3(512), 0, c.stream, pp, n_ks);

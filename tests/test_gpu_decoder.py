@@ -544,6 +544,30 @@ def test_prompt_attention_shows_a_cached_row_that_is_not_a_number(kv, hd, before
         dec.close()
 
 
+@pytest.mark.parametrize("kv,hkv,hd,window", [("f32", 17, 128, 0), ("i8", 20, 128, 0), ("f32", 33, 64, 0), ("f32", 17, 128, 300)])
+def test_prompt_attention_behind_many_rows_takes_little_room(kv, hkv, hd, window):
+    """The planes of 34304 rows of so many KV heads are more than 512 MB: they are made and walked for a part of the heads at a time, and under a window for its rows alone.  A
+    continuation equals the same tokens through the per-row kernels, and what the prompts took beside the cache is bounded."""
+    import torch
+    from helpers.device import dev, rel_err
+    cai = dev()
+    n, more = 34304, 260
+    cfg = dict(n_layers=1, d_model=64, n_q_heads=hkv, n_kv_heads=hkv, head_dim=hd, ffn=64, vocab=300, max_ctx=n + 512, eps=1e-5, rope_theta=1e6, window=window)
+    dec = cai.Decoder(synthetic_spec(cfg, O.Q8_0, head_qtype=O.Q8_0, seed=hkv, std=0.05), max_batch=1, kv_dtype={"f32": cai.KV_F32, "i8": cai.KV_I8}[kv])
+    toks = np.random.default_rng(hd).integers(0, 300, n + more).astype(np.int32)
+    dec.prefill(toks[:512])                         # (what does not depend on the rows is there)
+    before = torch.cuda.mem_get_info()[0]
+    dec.prefill(toks[512:n], 512)
+    _, got = dec.prefill(toks[n:], n)
+    taken = before - torch.cuda.mem_get_info()[0]
+    dec.truncate(n, 0)
+    for p in range(n, n + more, 7 if hd == 128 else 130):
+        _, want = dec.prefill(toks[p:min(p + (7 if hd == 128 else 130), n + more)], p)
+    assert rel_err(got, want) < {"f32": 2e-5, "i8": 5e-3}[kv]
+    assert taken < (64 if window else 450) * 2 ** 20, taken
+    dec.close()
+
+
 @pytest.mark.parametrize("name", ["qwen7b_like_q4k", "olmoe_like_q8"])
 def test_per_class_timing_leaves_the_session_as_it_found_it(name):
     """cai_decoder_profile (a measurement aid without a counterpart in the reference) replays whole steps and steps without one
