@@ -264,10 +264,11 @@ def test_long_steps_walk_their_records_in_passes(cai, tmp_path, mech, counts):
         assert taken < 1.6e9, taken
 
 
-@pytest.mark.parametrize("tokens, ff", [(129, 16400), (257, 8208), (300, 12000)])
+@pytest.mark.parametrize("tokens, ff", [(129, 16400), (257, 8208), (300, 12000), (129, 16000), (257, 8000), (300, 8100)])
 def test_products_on_tiles_of_256_tokens(cai, tmp_path, tokens, ff):
-    """gate | up matrices whose products fill the chip with large tiles: tokens one past half a tile, one past a tile and inside a second one, rows
-    that end inside a tile; one and a half steps of depth"""
+    """gate | up matrices whose products fill the chip with large tiles, of 256 x 128 (the last three) and of 128 x 128: tokens one past half a tile, one past a tile and inside a second
+    one, rows that end inside a tile; one and a half steps of depth"""
+    assert cai.load().cai_bf16_tiles(2 * ff, 72, tokens) == (4 if ff in (16000, 8000, 8100) else 3)
     m = Model(tmp_path, B.config([B.layer(B.delta(), ff=ff)], width=72, vocab=67), seed=tokens, edit=only("feed-forward"), rank_a=3, rank_g=20)
     tok = m.tokens(tokens, 1)
     dec = m.open(cai, 320, 1, "bf16")
@@ -275,10 +276,11 @@ def test_products_on_tiles_of_256_tokens(cai, tmp_path, tokens, ff):
     dec.close()
 
 
-@pytest.mark.parametrize("tokens, ff, width", [(300, 12000, 448), (700, 12000, 320), (129, 16400, 448), (600, 5632, 320)])
+@pytest.mark.parametrize("tokens, ff, width", [(300, 12000, 448), (700, 12000, 320), (129, 16400, 448), (600, 5632, 320), (300, 8100, 448)])
 def test_products_on_large_tiles_of_many_steps(cai, tmp_path, tokens, ff, width):
     """the same products seven and five steps of 64 deep, so that every slot of the tiles' rings is filled again and the last fill lies in another
-    slot than the first: tiles of 256 x 128 (12000) and of 128 x 128 (the others)"""
+    slot than the first: tiles of 256 x 128 (the second and the last) and of 128 x 128 (the others)"""
+    assert cai.load().cai_bf16_tiles(2 * ff, width, tokens) == (4 if (tokens, ff) in ((700, 12000), (300, 8100)) else 3)
     m = Model(tmp_path, B.config([B.layer(B.delta(), ff=ff)], width=width, vocab=67), seed=tokens, edit=only("feed-forward"), rank_a=3, rank_g=20)
     tok = m.tokens(tokens, 1)
     dec = m.open(cai, 768, 1, "bf16")
