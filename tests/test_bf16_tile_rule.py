@@ -6,7 +6,7 @@ from helpers.device import cai
 T32, T64, T128_16, T128_8, T256_128, T256 = range(6)
 
 
-@pytest.mark.parametrize("rows,cols,n_tok,want", [
+@pytest.mark.parametrize("rows,cols,n_tok,want,gated", [(*c, 0) for c in [
     # small tiles
     (2048, 2048, 32, T32), (512, 64, 2048, T64), (512, 64, 1900, T32), (18720, 256, 64, T64), (2048, 2048, 1024, T64),
     # one round of 128 x 128 against up to three tiles of 64 x 64 a CU, by depth
@@ -15,6 +15,8 @@ T32, T64, T128_16, T128_8, T256_128, T256 = range(6)
     # one round of 256 x 256 against two of 256 x 128, by depth and by how full the second is
     (6200, 256, 1536, T128_8), (6200, 768, 1536, T128_8), (6200, 769, 1536, T256), (6200, 2048, 1536, T256), (11264, 256, 700, T128_8), (8192, 256, 1792, T256_128), (8192, 256, 1793, T256),
     # by rounds otherwise
-    (11264, 2048, 300, T256_128), (11264, 2048, 640, T128_8), (32800, 2048, 128, T128_8), (11264, 2048, 2048, T256_128), (11264, 2048, 1024, T256)])
-def test_which_tiles_a_product_takes(rows, cols, n_tok, want):
-    assert cai.load().cai_bf16_tiles(rows, cols, n_tok) == want
+    (11264, 2048, 300, T256_128), (11264, 2048, 640, T128_8), (32800, 2048, 128, T128_8), (11264, 2048, 2048, T256_128), (11264, 2048, 1024, T256)]] + [
+    # gated products: 256 x 256 at every depth
+    (6208, 256, 1536, T256, 1), (12800, 256, 900, T256, 1), (3072, 256, 700, T64, 1), (4096, 256, 770, T128_16, 1), (6208, 256, 1280, T256_128, 1)])
+def test_which_tiles_a_product_takes(rows, cols, n_tok, want, gated):
+    assert cai.load().cai_bf16_tiles(rows, cols, n_tok, gated) == want
