@@ -650,19 +650,21 @@ static int run_gemv_mc(const cai_qw_s* w, const bf16_t* x, int64_t ldx, int n_to
 
 // The tiles (tokens x outputs, waves) of a product over `depth` bfloat16 columns of more rows than the walks take.
 // Large tiles, by rounds over the chip: 256 x 256 by sixteen waves or 256 x 128 by sixteen, one work-group a CU, or 128 x 128 by eight, two a
-// CU.  A full round takes 57, 33 and 37 us (at a depth of 2048), one of 128 x 128 with at most a work-group a CU 28.  Products alone, us,
+// CU.  A full round takes 57, 32 and 37 us (at a depth of 2048), one of 128 x 128 with at most a work-group a CU 28.  Products alone, us,
 // 256 x 256 | 256 x 128 | 128 x 128 by eight: 11264 rows, 1024 tokens 56 | 65 | 59, 2048: 113 | 105 | 108; 6200 rows, 1024 tokens 49 | 34 | 34, 2048: 57 | 67 | 67;
 // without the first: 11264 rows, 300 tokens 30.8 | 31.9, 640: 57.1 | 35.6; 32800 rows, 128 tokens 57.6 | 43.9; 49152 rows, 100: 61.1 | 50.4.
-// At a depth of up to 768 the start and the end of a tile of 256 x 256 are half of it or more, and where the second round of the others is less than three quarters full
-// they take less: 6200 rows, 1536 tokens, 256 x 256 | 256 x 128 | 128 x 128 at a depth of 256 20.0 | 18.3 | 16.5, 512: 25.1 | 23.8 | 20.8, 768: 30.4 | 30.0 | 26.8, 2048: 56.9 | 62.3 | 55.1.
-// Gated products write a quarter as much: there 256 x 256 is ahead at every depth (12800 rows, 900 tokens, depth 256 13.4 | 15.0 | 14.4).
+// One round of 256 x 256 wants more than three fifths of the CUs (11264 rows over 256 columns, 700 tokens, 132 tiles: 23.6 | 18.8), and up to a depth of 512, where its start
+// and end are half of it, a second round of the others that is three quarters full (11264 rows over 256, 900 tokens, not so: 25.1 | 22.5) or a gated product, which writes a quarter as much
+// (12800 rows over 256, 900 tokens 13.4 | 15.0).
 // Where one round of 128 x 128 covers everything, sixteen waves and copies three steps ahead (a CU has one work-group): 2048 x 2048, 2048 tokens 33 | 24 (256 x 128 |
 // here), 2048 x 5632 75 | 54, 6200 x 2048, 512 tokens 29 (64 x 64) | 21, 11264 x 2048, 256 tokens 23 | 21; up to two tiles of 64 x 64 a CU those take less
 // (2048 rows, 1024 tokens 16 | 20; 6200 rows, 256: 15 | 18.5), and a little past that: a CU holds three of them at once, so up to three a CU are one round.  64 x 64 | 128 x 128,
 // 3072 rows, 700 tokens (2.06 a CU), depth 256 5.7 | 8.1, 512: 7.5 | 8.6, 1024: 11.8 | 12.3, 2048: 19.6 | 20.6, 4096: 34.5 | 35.5, 6400: 52.9 | 50.6; 4096 rows, 700 tokens (2.75 a CU) 6.2 | 7.6, 8.6 | 9.2, 12.8 |
-// 13.4, 1536: 18.1 | 17.4, 2048: 22.4 | 21.6.  Over 3532 sizes, plain and gated, of eight depths from 256 to 6400 the rule takes
-// 0.954 to 0.978 times what 256 x 128, 128 x 128 by eight and the small tiles alone take, never more than 1.001 times but once (12800 gated rows, 130 tokens 19.2 -> 20.0); by the
-// times of a depth of 2048 whatever the depth is, up to 1.41.
+// 13.4, 1536: 18.1 | 17.4, 2048: 22.4 | 21.6.  (The weights are what a first pass waits for: from HBM instead of a cache 128 x 128 is 0.8 to 0.95 times 64 x 64 from two a CU and a depth of 768
+// on, but a small model's stay in the cache.)
+// Against 256 x 128, 128 x 128 by eight and the small tiles alone, over 2889 sizes of eight depths from 256 to 5632, plain and gated, weights in the 256 MB cache, and 2512 with them in HBM:
+// 0.945 to 0.990 times on average of a depth, never more than 1.01 times but for six sizes (1.015 to 1.056); by the times of a depth of 2048 whatever the depth is, up to 1.26 (1.41 with
+// the weights in L2).
 // What holds a tile's step up is neither the copies by themselves (128 x 128 steps alone 0.39 us, here 0.55), the fragment reads (two groups of waves with half
 // the columns each, a quarter fewer, took the same) nor their order (a half step's read while the half before is multiplied: the same).
 // Small tiles: a step is a hundred nanoseconds of work and a round trip to memory is a microsecond, so copies go out several steps ahead, as
@@ -673,12 +675,12 @@ enum { TILES_32, TILES_64, TILES_128_16, TILES_128_8, TILES_256_128, TILES_256 }
 static int lin_tiles(int64_t n_rows, int64_t depth, int n_tok, bool gated, int64_t n_cu)
 {
   auto tiles = [&](int bm, int bn) { return (int64_t)((n_tok + bm - 1) / bm) * ((n_rows + bn - 1) / bn); };
-  const int64_t small = tiles(128, 128), large = tiles(256, 128);
+  const int64_t small = tiles(128, 128), large = tiles(256, 128), huge = tiles(256, 256);
   if (n_tok > 64 && small <= n_cu && 4 * tiles(64, 64) > (depth > 4096 ? 8 : depth > 1024 ? 9 : 12) * n_cu) return TILES_128_16;
   if (n_tok > 64 && small >= n_cu) {
     const int64_t left = small % (2 * n_cu), t_small = 37 * (small / (2 * n_cu)) + (left == 0 ? 0 : left <= n_cu && small > n_cu ? 28 : 37);
-    const int64_t t_large = 33 * ((large + n_cu - 1) / n_cu), t_huge = 57 * ((tiles(256, 256) + n_cu - 1) / n_cu);
-    if (t_huge < t_large && t_huge < t_small && (depth > 768 || gated || 4 * large > 7 * n_cu)) return TILES_256;
+    const int64_t t_large = 32 * ((large + n_cu - 1) / n_cu), t_huge = 57 * ((huge + n_cu - 1) / n_cu);
+    if (t_huge < t_large && t_huge < t_small && 5 * huge > 3 * n_cu && (depth > 512 || gated || 4 * large > 7 * n_cu)) return TILES_256;
     return t_large <= t_small ? TILES_256_128 : TILES_128_8;
   }
   return n_tok > 32 && tiles(64, 64) >= n_cu ? TILES_64 : TILES_32;

@@ -266,9 +266,9 @@ def test_long_steps_walk_their_records_in_passes(cai, tmp_path, mech, counts):
 
 @pytest.mark.parametrize("tokens, ff", [(129, 16400), (257, 8208), (300, 12000), (129, 16000), (257, 8000), (300, 8100)])
 def test_products_on_tiles_of_256_tokens(cai, tmp_path, tokens, ff):
-    """gate | up matrices whose products fill the chip with large tiles, of 256 x 128 (the last three), 128 x 128 (the second) and 256 x 256: tokens one past half a tile, one past a tile and inside a second
+    """gate | up matrices whose products fill the chip with large tiles, of 256 x 128 (the first and the last three), 128 x 128 (the second) and 256 x 256: tokens one past half a tile, one past a tile and inside a second
     one, rows that end inside a tile; one and a half steps of depth"""
-    assert cai.load().cai_bf16_tiles(2 * ff, 72, tokens, 1) == {16400: 5, 8208: 3, 12000: 5}.get(ff, 4)
+    assert cai.load().cai_bf16_tiles(2 * ff, 72, tokens, 1) == {8208: 3, 12000: 5}.get(ff, 4)
     m = Model(tmp_path, B.config([B.layer(B.delta(), ff=ff)], width=72, vocab=67), seed=tokens, edit=only("feed-forward"), rank_a=3, rank_g=20)
     tok = m.tokens(tokens, 1)
     dec = m.open(cai, 320, 1, "bf16")
@@ -279,8 +279,8 @@ def test_products_on_tiles_of_256_tokens(cai, tmp_path, tokens, ff):
 @pytest.mark.parametrize("tokens, ff, width", [(300, 12000, 448), (700, 12000, 320), (129, 16400, 448), (600, 5632, 320), (300, 8100, 448)])
 def test_products_on_large_tiles_of_many_steps(cai, tmp_path, tokens, ff, width):
     """the same products seven and five steps of 64 deep, so that every slot of the tiles' rings is filled again and the last fill lies in another
-    slot than the first: tiles of 256 x 128 (the second and the last), 128 x 128 (the fourth) and 256 x 256"""
-    assert cai.load().cai_bf16_tiles(2 * ff, width, tokens, 1) == {(700, 12000): 4, (300, 8100): 4, (600, 5632): 3}.get((tokens, ff), 5)
+    slot than the first: tiles of 256 x 256 (the first), 128 x 128 (the fourth) and 256 x 128"""
+    assert cai.load().cai_bf16_tiles(2 * ff, width, tokens, 1) == {(300, 12000): 5, (600, 5632): 3}.get((tokens, ff), 4)
     m = Model(tmp_path, B.config([B.layer(B.delta(), ff=ff)], width=width, vocab=67), seed=tokens, edit=only("feed-forward"), rank_a=3, rank_g=20)
     tok = m.tokens(tokens, 1)
     dec = m.open(cai, 768, 1, "bf16")
@@ -288,11 +288,11 @@ def test_products_on_large_tiles_of_many_steps(cai, tmp_path, tokens, ff, width)
     dec.close()
 
 
-@pytest.mark.parametrize("rows, cols, tokens, tiles", [(2041, 264, 1100, 1), (4300, 72, 513, 1), (16300, 320, 130, 4), (6200, 328, 2050, 4), (4104, 72, 2100, 3),
-                                                      (2041, 264, 2000, 2), (4300, 72, 890, 2), (16300, 320, 193, 2), (16300, 1096, 130, 2), (6200, 328, 2310, 5), (4104, 72, 3810, 5), (4104, 776, 2050, 5)])
+@pytest.mark.parametrize("rows, cols, tokens, tiles", [(2041, 264, 1100, 1), (4300, 72, 513, 1), (16300, 320, 130, 4), (6200, 328, 2050, 4), (4104, 72, 2100, 4),
+                                                      (2041, 264, 2000, 2), (4300, 72, 890, 2), (16300, 320, 193, 2), (16300, 1096, 130, 2), (6200, 328, 2310, 5), (4104, 72, 3810, 5), (4104, 776, 2310, 5)])
 def test_one_round_of_large_tiles(cai, rows, cols, tokens, tiles):
     """Tiles of 128 x 128 by sixteen waves (2: one round of them) and of 256 x 256 (5: one round instead of two of smaller ones), one to eighteen steps of 64 deep, rows and
-    tokens that end inside a tile; and what sizes a little below them take (1: 64 x 64, 3: 128 x 128 by eight waves, 4: 256 x 128).  The bound is that of
+    tokens that end inside a tile; and what sizes a little below them take (1: 64 x 64, 4: 256 x 128).  The bound is that of
     test_products_over_bf16_rows."""
     assert cai.load().cai_bf16_tiles(rows, cols, tokens, 0) == tiles
     rng = np.random.default_rng(rows)
@@ -304,7 +304,7 @@ def test_one_round_of_large_tiles(cai, rows, cols, tokens, tiles):
     q.close()
 
 
-@pytest.mark.parametrize("width, tokens, ff", [(2056, 1100, 72), (4104, 2050, 72), (2054, 1090, 72), (2056, 1100, 1032), (4104, 2050, 776), (2054, 1090, 1032)])
+@pytest.mark.parametrize("width, tokens, ff", [(2056, 1100, 72), (4104, 2050, 72), (2054, 1090, 72), (2056, 1100, 1032), (4104, 2310, 776), (2054, 1090, 1032)])
 def test_residuals_of_large_tiles(cai, tmp_path, width, tokens, ff):
     """the stream's update and the norms around it behind tiles of 128 x 128 by sixteen waves and of 256 x 256 (ff of 1032 and of 776, depths at which they are taken), and behind
     the tiles of shallow products; a width that is no whole fours"""
@@ -312,7 +312,7 @@ def test_residuals_of_large_tiles(cai, tmp_path, width, tokens, ff):
         assert cai.load().cai_bf16_tiles(width, ff, tokens, 0) == (5 if ff == 776 else 2)
     m = Model(tmp_path, B.config([B.layer(B.delta(1, 1, 8, 8, 2), ff=ff)], width=width, vocab=67), seed=width, rank_a=3, rank_g=20)
     tok = m.tokens(tokens, 1)
-    dec = m.open(cai, 2112, 1, "bf16")
+    dec = m.open(cai, 2368, 1, "bf16")
     check(feed(dec, tok, [tokens]), m.ref(tok), "bf16")
     dec.close()
 
