@@ -2411,7 +2411,7 @@ extern "C" int cai_attn_decode(cai_kv_t kv, int layer, const float* qkv, int q_h
   CAI_HIP(hipGetLastError());
   if (flags & CAI_Y_DEVICE) {
     // The signal behind the row says that launches can read it: memory of this card.  A row anywhere else (pinned, managed, a peer's) is there for the host
-    // when the stream has ended.  40 / 8 heads x 128 behind 8191 int8 rows: 23.9 us with hipStreamSynchronize, 20.4 with the signal (the question
+    // when the stream has ended.  40 / 8 heads x 128 behind 8191 int8 rows: 24.1 us with hipStreamSynchronize, 22.1 with the signal (the question
     // about the address is asked while the kernels run).
     hipPointerAttribute_t at{};
     const bool known = hipPointerGetAttributes(&at, out) == hipSuccess;

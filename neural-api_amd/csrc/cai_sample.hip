@@ -336,7 +336,7 @@ int run_candidates(const float* logits_dev, int n, const int32_t* hist_ids, cons
     p.hist_ids = (const int32_t*)c.stage_in; p.hist_counts = p.hist_ids + hist; p.n_hist = n_hist;
   }
   const dim3 grid(p.n_slices), block(SL_T);
-  p.done = host_signal_next();       // (40 of 152064 behind a history of 512: 44.5 us with hipStreamSynchronize, 42.1 so)
+  p.done = host_signal_next();       // (40 of 152064 behind a history of 512, call after call 45.6 us with hipStreamSynchronize, 45.2 so; one call and a synchronisation 48.6, 47.3)
   hipLaunchKernelGGL(candidates_stats_kernel, grid, block, 0, c.stream, p);
   if (p.penalty) hipLaunchKernelGGL(candidates_penalty_kernel, grid, block, 0, c.stream, p);
   hipLaunchKernelGGL(candidates_value_kernel, grid, block, 0, c.stream, p);
