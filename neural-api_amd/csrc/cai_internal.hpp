@@ -76,7 +76,9 @@ int  ensure_host_stage(size_t need);   // grows ctx().h_stage; only for calls th
 // zero.  A wait of more than 50 ms goes on in hipStreamSynchronize, which also returns an error of the launches.
 // An event goes out behind the last launch, while it runs: without one the runtime asks for the stream's end when the host program next
 // synchronises the device, later and at more cost.  us, 40 / 8 heads behind 8191 int8 rows, call after call | one call and hipDeviceSynchronize: hipStreamSynchronize in
-// the call 24.1 | 27.1, the flag alone 20.9 | 32, flag and event 22.1 | 25.6; candidates of 152064 45.6 | 48.6, 44.0 | 55, 45.2 | 47.3; a step of the 135M shape 583 | 586, 575 | 595, 575 | 584.
+// the call 24.1 | 27.1, the flag alone 20.9 | 32, flag and event 22.1 | 25.6; a step of the 135M shape 583 | 586, 575 | 595, 575 | 584.
+// (The samplers' candidates leave in single words from many work-groups and wait for the end of the stream: with host_store and the flag 300 of 50000 took 69 us instead of 54, 905 of
+// 188977 68 instead of 59, 40 of 152064 the same.)
 constexpr int HOST_SIGNALS = 8;            // of one call
 struct HostSignal { uint32_t* flag = nullptr; unsigned* arrive = nullptr; uint32_t value = 0; };      // flag null: none
 HostSignal host_signal_next(int k = 0);    // the k-th of this call
@@ -85,7 +87,7 @@ void launch_host_signal(const HostSignal& s);      // as a launch of its own
 // A result in coherent pinned memory: a store of system scope, which no cache keeps and which is acknowledged when it is there.
 template <typename T> __device__ __forceinline__ void host_store(T* p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
 // By every thread, at the end of a kernel that leaves its results with host_store: they are acknowledged (vmcnt(0)) before the work-group arrives, so
-// there is nothing to write back.  (With ordinary stores and a fence of system scope the last of the candidates' launches took 9.5 us instead of 5.8;
+// there is nothing to write back.  (With ordinary stores and a fence of system scope a launch took 9.5 us instead of 5.8;
 // with ordinary stores and no fence the host read what had been there before.)
 __device__ __forceinline__ void host_signal(const HostSignal& s, unsigned work_groups)
 {

@@ -102,7 +102,6 @@ struct SampleParams {
   int* bins;                         // [4096] values per leading 12 bits
   float *st_max, *st_sum, *st_tot, *st_pmax, *st_sum2; int* st_cnt;   // [256] per slice
   int32_t* tok_out; float* p_out;    // host memory
-  HostSignal done;                   // of the last launch
 };
 
 // the same clamps as the host row soft-max (a NaN counts as far below the maximum)
@@ -297,9 +296,8 @@ __global__ __launch_bounds__(SMP_T) void candidates_rank_kernel(const SamplePara
     int rank = 0;
     for (int j = tid & 7; j < total; j += 8) { const uint32_t w = __float_as_uint(cp[j]); rank += w > u || (w == u && ct[j] < t); }
     rank += __shfl_xor(rank, 1); rank += __shfl_xor(rank, 2); rank += __shfl_xor(rank, 4);
-    if ((tid & 7) == 0 && rank < m) { host_store(p.tok_out + rank, t); host_store(p.p_out + rank, v); }
+    if ((tid & 7) == 0 && rank < m) { p.tok_out[rank] = t; p.p_out[rank] = v; }
   }
-  host_signal(p.done, gridDim.x);
 }
 
 // host arrays in, host arrays out; the row itself is a device pointer
@@ -336,14 +334,13 @@ int run_candidates(const float* logits_dev, int n, const int32_t* hist_ids, cons
     p.hist_ids = (const int32_t*)c.stage_in; p.hist_counts = p.hist_ids + hist; p.n_hist = n_hist;
   }
   const dim3 grid(p.n_slices), block(SL_T);
-  p.done = host_signal_next();       // (40 of 152064 behind a history of 512, call after call 45.6 us with hipStreamSynchronize, 45.2 so; one call and a synchronisation 48.6, 47.3)
   hipLaunchKernelGGL(candidates_stats_kernel, grid, block, 0, c.stream, p);
   if (p.penalty) hipLaunchKernelGGL(candidates_penalty_kernel, grid, block, 0, c.stream, p);
   hipLaunchKernelGGL(candidates_value_kernel, grid, block, 0, c.stream, p);
   hipLaunchKernelGGL(candidates_reach_kernel, grid, block, 0, c.stream, p);
   hipLaunchKernelGGL(candidates_rank_kernel, dim3(m > 32 ? RANK_WG : 1), dim3(SMP_T), 0, c.stream, p);
   CAI_HIP(hipGetLastError());
-  if ((rc = host_signal_wait(p.done))) return rc;
+  CAI_HIP(hipStreamSynchronize(c.stream));
   memcpy(tokens_out, h, (size_t)m * 4);
   memcpy(probs_out, h + SMP_MAX_M, (size_t)m * 4);
   if (count_out) *count_out = m;
