@@ -75,7 +75,8 @@ typedef uint32_t uint2_b __attribute__((ext_vector_type(2)));
 }  // namespace
 
 // ------------------------------------------------------------------------------------------
-// Large tiles.  Eight waves, 256 weight rows x TT * 32 tokens.  Chunks of 64 columns - token planes, quants, scales, all copied along
+// Large tiles.  NW waves, 32 NW weight rows x TT * 32 tokens: eight, or four in half the LDS, so that a CU holds two work-groups which wait, start and
+// end independently of each other.  Chunks of 64 columns - token planes, quants, scales, all copied along
 // the rows from memory into LDS - are requested DEPTH - 1 chunks ahead of the one that is multiplied; the waves meet once a chunk.
 // A wave holds 64 rows x 16 TT tokens: what it reads of a chunk from LDS (activations of its tokens, quants of its rows) takes less
 // time than its products, which 32 rows x all tokens does not.  A tile of at most 32 tokens (an expert's run, a short prompt) is
@@ -85,15 +86,16 @@ typedef uint32_t uint2_b __attribute__((ext_vector_type(2)));
 // and no codes 1.1).  Operands requested one block ahead, and folds issued between the next block's products, changed nothing.
 // 37888 x 3584 Q8_0, 2048 tokens: 1721 us in tiles of 256 x 64 that staged through registers -> 1273 (TT = 4); 3584 x 18944: 1358 -> 718.
 // Gate | up and down of 64 experts (2048 x 2048, 2048 x 1024), 2040 slots: 199 us a layer -> 149 (82 to read the banks once): with tiles
-// of 64 slots instead of 32 an expert's rows come from memory once.  Two work-groups a CU (two slots of LDS each) take the same time.
+// of 64 slots instead of 32 an expert's rows come from memory once.
 // ------------------------------------------------------------------------------------------
-template <int QT, int TT, bool ODD>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_blk_tile(const BlkGemmParams p)
+constexpr int blk_depth(int TT, int NW) { return TT == 2 && NW == 8 ? 4 : 3; }      // chunks in LDS
+template <int QT, int TT, bool ODD, int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_blk_tile(const BlkGemmParams p)
 {
   extern __shared__ __align__(16) unsigned char bl_smem[];
-  constexpr int NTOK = TT * 32, DEPTH = TT == 2 ? 4 : 3, WROW = QT == CAI_Q8_0 ? 64 : 32;
-  constexpr int PLANE = NTOK * 128, XB = 2 * PLANE, WB = 256 * WROW, SLOT = XB + WB + (ODD ? 2048 : 1024);
-  constexpr int XC = NTOK / 64, WC = WB / 8192, COPIES = 2 * XC + WC + (ODD ? 2 : 1);      // a wave's copies of a chunk
+  constexpr int NTOK = TT * 32, ROWS = 32 * NW, DEPTH = blk_depth(TT, NW), WROW = QT == CAI_Q8_0 ? 64 : 32;
+  constexpr int PLANE = NTOK * 128, XB = 2 * PLANE, WB = ROWS * WROW, DB = ROWS * 4, SLOT = XB + WB + (ODD ? 2 : 1) * DB;
+  constexpr int XC = NTOK / (8 * NW), WC = WROW / 32, COPIES = 2 * XC + WC + (ODD ? 2 : 1);      // a wave's copies of a chunk
   __shared__ int s_yrow[NTOK];
   __shared__ float s_sinv[NTOK];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -110,12 +112,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     if (rg >= p.n_row_groups) return;
     first = ttile * NTOK; n_here = min(NTOK, p.n_tok - first);
   }
-  const bool one = TT == 2 && n_here <= 32;              // half a tile: the other half is neither staged (by waves 4 .. 7) nor multiplied
-  const bool x_on = !(one && wave >= 4);
+  const bool one = TT == 2 && n_here <= 32;              // half a tile: the other half is neither staged nor multiplied
+  const int x_n = !one ? XC : 8 * wave < 32 ? 1 : 0;     // of a wave's XC copies of token rows (8 (NW i + wave) and on) those that are made
+  static_assert(XC == 1 || 8 * NW >= 32, "of half a tile a wave has one copy at most");
   const uint8_t* qbase = p.q; const uint8_t* dbase = p.d; const float* bias = p.bias; int rows = p.rows, yo = 0, rgl = rg;   // this work-group's matrix (uniform)
   if (p.n_seg > 1 && rg >= p.seg_end[0]) { qbase = p.q2[0]; dbase = p.d2[0]; bias = p.bias2[0]; rows = p.rows2[0]; yo = p.y_off2[0]; rgl = rg - p.seg_end[0]; }
   if (p.n_seg > 2 && rg >= p.seg_end[1]) { qbase = p.q2[1]; dbase = p.d2[1]; bias = p.bias2[1]; rows = p.rows2[1]; yo = p.y_off2[1]; rgl = rg - p.seg_end[1]; }
-  const int R0 = rgl * 256, K = p.cols, nb32 = K >> 5, n_chunks = (nb32 + 1) >> 1;
+  const int R0 = rgl * ROWS, K = p.cols, nb32 = K >> 5, n_chunks = (nb32 + 1) >> 1;
   const int64_t bank_row = (int64_t)expert * p.expert_rows;
   auto x_row = [&](int m) { const int t = first + min(m, n_here - 1); return p.perm ? p.perm[t] / p.x_div : t; };   // rows past the end repeat the last token; their results are not written
   if (threadIdx.x < NTOK) {
@@ -126,7 +129,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   uint32_t xo[XC], wo[WC], xcut = 0, wcut = 0;
 #pragma unroll
   for (int i = 0; i < XC; i++) {
-    const int t = 8 * (8 * i + wave) + (lane >> 3);
+    const int t = 8 * (NW * i + wave) + (lane >> 3);
     const uint32_t piece = (uint32_t)((lane & 7) ^ ((t >> 1) & 7));
     xo[i] = (uint32_t)x_row(t) * (uint32_t)K * 2u + 16u * piece;
     if (ODD && piece >= 4) xcut |= 1u << i;
@@ -135,15 +138,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
   for (int i = 0; i < WC; i++) {
     if constexpr (QT == CAI_Q8_0) {
-      const int t = 16 * (8 * i + wave) + (lane >> 2); const uint32_t piece = (uint32_t)((lane & 3) ^ ((t >> 2) & 3));
+      const int t = 16 * (NW * i + wave) + (lane >> 2); const uint32_t piece = (uint32_t)((lane & 3) ^ ((t >> 2) & 3));
       wo[i] = (uint32_t)min(t, rlast) * (uint32_t)K + 16u * piece; if (ODD && piece >= 2) wcut |= 1u << i;
     }
     else {
-      const int t = 32 * (8 * i + wave) + (lane >> 1); const uint32_t piece = (uint32_t)((lane & 1) ^ ((t >> 3) & 1));
+      const int t = 32 * (NW * i + wave) + (lane >> 1); const uint32_t piece = (uint32_t)((lane & 1) ^ ((t >> 3) & 1));
       wo[i] = (uint32_t)min(t, rlast) * (uint32_t)(K / 2) + 16u * piece; if (ODD && piece) wcut |= 1u << i;
     }
   }
-  const uint32_t dof = (uint32_t)min(64 * (wave & 3) + lane, rlast) * (uint32_t)(nb32 * 2);     // (waves 4 .. 7 repeat 0 .. 3: every wave counts the same copies)
+  const uint32_t dof = (uint32_t)min(64 * (wave & (NW / 2 - 1)) + lane, rlast) * (uint32_t)(nb32 * 2);     // (the upper half of the waves repeats the lower: every wave counts the same copies)
   const uint8_t* const qb = qbase + (bank_row + R0) * (int64_t)nb32 * (WROW / 2);
   const uint8_t* const db = dbase + (bank_row + R0) * (int64_t)nb32 * 2;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)bl_smem;
@@ -152,19 +155,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const bool half = ODD && c == n_chunks - 1;        // one block is left: the chunk's second half repeats the first and is not used
     const char* const xh = reinterpret_cast<const char*>(p.xhi) + (int64_t)c * 128;
     const char* const xl = reinterpret_cast<const char*>(p.xlo) + (int64_t)c * 128;
-    if (x_on)
 #pragma unroll
-      for (int i = 0; i < XC; i++) {
+    for (int i = 0; i < XC; i++)
+      if (i < x_n) {
         const uint32_t o = xo[i] - (half && (xcut >> i & 1) ? 64u : 0u);
-        copy16_to_lds(dst + 1024 * (8 * i + wave), o, xh);
-        copy16_to_lds(dst + PLANE + 1024 * (8 * i + wave), o, xl);
+        copy16_to_lds(dst + 1024 * (NW * i + wave), o, xh);
+        copy16_to_lds(dst + PLANE + 1024 * (NW * i + wave), o, xl);
       }
 #pragma unroll
-    for (int i = 0; i < WC; i++) copy16_to_lds(dst + XB + 1024 * (8 * i + wave), wo[i] - (half && (wcut >> i & 1) ? WROW / 2u : 0u), qb + (int64_t)c * WROW);
+    for (int i = 0; i < WC; i++) copy16_to_lds(dst + XB + 1024 * (NW * i + wave), wo[i] - (half && (wcut >> i & 1) ? WROW / 2u : 0u), qb + (int64_t)c * WROW);
     if constexpr (ODD) {
-      copy2_to_lds(dst + XB + WB + 256 * (wave & 3), dof, db + (int64_t)c * 4);
-      copy2_to_lds(dst + XB + WB + 1024 + 256 * (wave & 3), dof, db + (int64_t)c * 4 + (half ? 0 : 2));
-    } else copy4_to_lds(dst + XB + WB + 256 * (wave & 3), dof, db + (int64_t)c * 4);
+      copy2_to_lds(dst + XB + WB + 256 * (wave & (NW / 2 - 1)), dof, db + (int64_t)c * 4);
+      copy2_to_lds(dst + XB + WB + DB + 256 * (wave & (NW / 2 - 1)), dof, db + (int64_t)c * 4 + (half ? 0 : 2));
+    } else copy4_to_lds(dst + XB + WB + 256 * (wave & (NW / 2 - 1)), dof, db + (int64_t)c * 4);
   };
 
   const float16_b zero16 = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
@@ -191,7 +194,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
       for (int rt = 0; rt < RW; rt++) {
         dw[rt] = *reinterpret_cast<const uint32_t*>(s0 + XB + WB + 4 * (32 * (r0 + rt) + n));
-        if constexpr (ODD) dw[rt] |= *reinterpret_cast<const uint32_t*>(s0 + XB + WB + 1024 + 4 * (32 * (r0 + rt) + n)) << 16;
+        if constexpr (ODD) dw[rt] |= *reinterpret_cast<const uint32_t*>(s0 + XB + WB + DB + 4 * (32 * (r0 + rt) + n)) << 16;
       }
 #pragma unroll
       for (int b = 0; b < 2; b++) {
@@ -238,7 +241,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     int slot = 0;
     for (int c = 0; c < n_chunks; c++) {
       const int left = n_chunks - 1 - c;               // chunks behind this one
-      if (left >= DEPTH - 2) { if (x_on) wait_copies<(DEPTH - 2) * COPIES>(); else wait_copies<(DEPTH - 2) * (COPIES - 2 * XC)>(); }
+      if (left >= DEPTH - 2) { if (x_n == XC) wait_copies<(DEPTH - 2) * COPIES>(); else wait_copies<(DEPTH - 2) * (COPIES - 2)>(); }
       else wait_copies<0>();
       __builtin_amdgcn_s_waitcnt(0xC07F);              // lgkmcnt(0): this wave's reads of the slot that is filled next (and the row tables, the first time)
       __builtin_amdgcn_s_barrier();
@@ -281,7 +284,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   if constexpr (TT == 2) {
     if (one) { body(std::integral_constant<int, 1>(), std::integral_constant<int, 1>(), wave, 0); return; }
   }
-  body(std::integral_constant<int, 2>(), std::integral_constant<int, TT / 2>(), 2 * (wave & 3), TT / 2 * (wave >> 2));
+  body(std::integral_constant<int, 2>(), std::integral_constant<int, TT / 2>(), 2 * (wave & (NW / 2 - 1)), TT / 2 * (wave / (NW / 2)));
 }
 
 // ------------------------------------------------------------------------------------------
@@ -769,9 +772,9 @@ int launch_blk(const BlkGemmParams& p0, int n_tiles_grouped)
 {
   BlkGemmParams p = p0;
   constexpr size_t WROW = QT == CAI_Q8_0 ? 64 : 32;                                    // quant bytes of a row's chunk
-  auto tile = [&](auto tt_, int n_tiles) {
-    constexpr int TT = tt_;
-    return launch_lds<gemm_blk_tile<QT, TT, ODD>>(blk_grid(p, 256, n_tiles), 512, (TT == 2 ? 4 : 3) * (TT * 8192 + 256 * WROW + (ODD ? 2048 : 1024)), p);
+  auto tile = [&](auto tt_, auto nw_, int n_tiles) {
+    constexpr int TT = tt_, NW = nw_;
+    return launch_lds<gemm_blk_tile<QT, TT, ODD, NW>>(blk_grid(p, 32 * NW, n_tiles), 64 * NW, blk_depth(TT, NW) * (TT * 8192 + 32 * NW * (WROW + (ODD ? 8 : 4))), p);
   };
   auto cut = [&](auto rt_, auto nw_) {
     constexpr int RT = rt_, NW = nw_;
@@ -780,8 +783,12 @@ int launch_blk(const BlkGemmParams& p0, int n_tiles_grouped)
     return launch_lds<gemm_blk_cut<QT, RT, NW, ODD>>(grid, 64 * NW, lds, p);
   };
   typedef std::integral_constant<int, 1> One; typedef std::integral_constant<int, 2> Two; typedef std::integral_constant<int, 3> Three;
-  typedef std::integral_constant<int, 4> Four; typedef std::integral_constant<int, 7> Seven;
-  if (p.tile_tab) return tile(Two(), n_tiles_grouped);
+  typedef std::integral_constant<int, 4> Four; typedef std::integral_constant<int, 7> Seven; typedef std::integral_constant<int, 8> Eight;
+  // An expert's runs: 128 x 64, two work-groups a CU, us as 256 x 64 : 128 x 64: 255 tokens to 64 experts of which few are chosen (45 tiles of 64 slots), gate | up
+  // of 2048 x 2048 88 : 82, down of 2048 x 1024 52 : 47; whole prompts, four layers of width 2048, 32 experts of 1024: 17 tokens 540 : 480, 100 tokens 641 : 580,
+  // 700 1906 : 1767, 2048 4818 : 4433; eight of 1536 at width 4096, 2048 tokens 6120 : 5640; Q4_0, 255 tokens 764 : 748, eight of 2048 at 3072, 1024 tokens 2775 : 2565.
+  // (Two chunks in LDS and three work-groups a CU: the same to 4 % slower; 256 x 64 with two chunks and two work-groups 2 to 3 % slower than with one.)
+  if (p.tile_tab) return tile(Two(), Four(), n_tiles_grouped);
   // A form's time is its rounds over the chip times what a round takes, in ns a column (Q8_0; with a full chip): cut tiles of 32 rows
   // 3.0, of 64 rows 4.6 (one work-group a CU) or 9.0 (three waves, two work-groups a CU: better from the second round on, 6144 x 2048
   // and 255 tokens 34.2 us against 35.5), tiles of 256 x 64 18 (13 if half empty), of 256 x 128 27.  At the lines, with the pre-pass:
@@ -797,11 +804,16 @@ int launch_blk(const BlkGemmParams& p0, int n_tiles_grouped)
   auto rounds = [](int64_t wgs, int n) { return (double)((wgs + n - 1) / n); };
   if (groups(32) * tok32 <= n_cu) return cut(One(), Seven());
   if (groups(64) * tok32 <= n_cu) return cut(Two(), Four());
+  // 128 x 64 of four waves takes 0.6 of the time of 256 x 64 while a CU has one of them (two: all of it), so where they fill the chip once and cut tiles
+  // go into a second round by more than half: with the pre-pass, cut : 128 x 64
+  //   2048 x 2048, 1024 tokens 49.5 : 38.5   4096 x 4096, 511: 75.3 : 62.2   14336 x 4096, 100: 64.1 : 57.2   4096 x 14336, 511: 253 : 190
+  //   (6144 x 2048, 255, a round and a half: 33.0 : 34.6)
+  if (groups(64) * tok32 > 3 * n_cu && groups(128) * ((p.n_tok + 63) / 64) <= n_cu) return tile(Two(), Four(), (p.n_tok + 63) / 64);
   const double c64 = 9.0 * rounds(groups(64) * tok32, 2 * n_cu);
   const double t64 = (p.n_tok <= 32 ? 13.0 : 18.0) * rounds(groups(256) * ((p.n_tok + 63) / 64), n_cu);
   const double t128 = 27.0 * rounds(groups(256) * ((p.n_tok + 127) / 128), n_cu);
   if (c64 <= t64 && c64 <= t128) return cut(Two(), Three());
-  return t128 <= t64 ? tile(Four(), (p.n_tok + 127) / 128) : tile(Two(), (p.n_tok + 63) / 64);
+  return t128 <= t64 ? tile(Four(), Eight(), (p.n_tok + 127) / 128) : tile(Two(), Eight(), (p.n_tok + 63) / 64);
 }
 
 int launch_blk(const cai_qw_s* w, const BlkGemmParams& p0, int n_tiles_grouped)

@@ -599,6 +599,23 @@ def test_large_block_tiles_of_many_chunks(qt, rows, cols, T):
     w.close()
 
 
+@pytest.mark.parametrize("qt", [O.Q8_0, O.Q4_0])
+@pytest.mark.parametrize("rows,cols,T", [(16380, 544, 97), (10600, 576, 140), (10600, 544, 150)])
+def test_block_tiles_of_128_rows(qt, rows, cols, T):
+    """tiles of 128 rows x 64 tokens, one a CU: a last tile of 33, 12 and 22 tokens, rows that are no whole tile, an odd and an even number of blocks"""
+    from helpers.device import dev, rel_err
+    cai = dev()
+    rng = np.random.default_rng(cols + qt + T)
+    base = O.quantize(qt, (rng.standard_normal((700, cols)) * 0.02).astype(np.float32)).reshape(700, -1)
+    raw = np.ascontiguousarray(base[np.arange(rows) % 700])
+    x = rng.standard_normal((T, cols)).astype(np.float32)
+    w = cai.QWeight(qt, rows, cols, raw.reshape(-1))
+    got = w.gemm(x)
+    want = x.astype(np.float64) @ O.dequant(qt, base.reshape(-1), 700 * cols).reshape(700, cols).astype(np.float64).T
+    assert rel_err(got, want[:, np.arange(rows) % 700]) < TIGHT
+    w.close()
+
+
 @pytest.mark.parametrize("experts,T", [(130, 40), (500, 70)])
 def test_prompt_of_a_mixture_of_more_experts_than_a_wave(experts, T):
     """slots grouped by expert where the sums over the experts before one run over several waves: a prompt equals its tokens one by one"""
