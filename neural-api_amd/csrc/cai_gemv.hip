@@ -9,7 +9,7 @@
 // Semantics of the layer this implements: Out[b*NumAs + a] = act(dot(W[a], X[b]) + bias[a])
 // (reference: neural/neuralvolume.pas:12127-12423, 12693-12745; fused tail neural/neural.cl:111-146).
 #include "cai_internal.hpp"
-#include "cai_gemv_common.hpp"
+#include "cai_router.hpp"
 #include <type_traits>
 #include "cai_blocks_raw.hpp"
 
@@ -462,8 +462,9 @@ __global__ __launch_bounds__(256) void gemv_fast(const GemvParams p)
 // in a step 3.5 | 3.0, 6144 x 2048 normed 7.6 | 6.3, 8 experts of 2048 x 2048 10.8 | 9.7, 49152 x 576 14.8 | 10.7; back to back 12000 x 3584 11.7 | 9.3, 36000 x 2048 17.1 | 13.5.
 // The leading scalar arguments are what these requests need of a launch of one matrix; they arrive preloaded (see the Makefile).
 // ------------------------------------------------------------------------------------------
-template <int QT, int R, int MODE, bool BANK, int SV>
-__global__ __launch_bounds__(256) void gemv_one(const float* hx, const uint8_t* hw0, const uint8_t* haux0, const float* hgain, const float* hres, const int hcols, const int hrows0, const int hgrp0, const int hnseg, const GemvParams p)
+constexpr int BANK_NONE = 0, BANK_SLOTS = 1, BANK_ROUTED = 2;
+template <int QT, int R, int MODE, int BANK, int SV>
+__global__ __launch_bounds__(256) void gemv_one(const float* hx, const uint8_t* hw0, const uint8_t* haux0, const float* hgain, const float* hres, const int hcols, const int hrows0, const int hgrp0, const int hnseg, const std::conditional_t<BANK == BANK_ROUTED, GemvRouted, GemvParams> p)
 {
   extern __shared__ float4 xs4[];          // [kp/4]
   const unsigned long long tl0 = timeline_now();
@@ -474,7 +475,7 @@ __global__ __launch_bounds__(256) void gemv_one(const float* hx, const uint8_t* 
   const int grp = blockIdx.x * 4 + wave, cols = hcols;
   const float* xin = hx; float* yout = p.y;
   int64_t bank_row = 0;
-  if constexpr (BANK) { xin += (int64_t)blockIdx.y * p.x_slot_stride; yout += (int64_t)blockIdx.y * p.y_slot_stride; }
+  if constexpr (BANK != BANK_NONE) { xin += (int64_t)blockIdx.y * p.x_slot_stride; yout += (int64_t)blockIdx.y * p.y_slot_stride; }
   // the activation (up to 1024 SV columns)
   typedef float f4 __attribute__((ext_vector_type(4)));
   const int n4 = cols >> 2;
@@ -492,7 +493,25 @@ __global__ __launch_bounds__(256) void gemv_one(const float* hx, const uint8_t* 
   if (s) { data = p.seg[s].data; aux = p.seg[s].aux; rows = p.seg[s].rows; }
   const int row_first = (grp - grp0) * R;
   const bool wave_live = s ? grp < p.seg[hnseg - 1].grp_end : grp < hgrp0;
-  if constexpr (BANK)
+  if constexpr (BANK == BANK_ROUTED) {
+    // The slot's expert: by the first wave of every work-group, while the activation is on its way (a selection of the last work-group of the router's
+    // launch to arrive was three more round trips.  8 of 64 experts of 2048 x 2048 Q8_0: 8.1 us of router + 9.5 here -> 3.8 + 9.8)
+    __shared__ int s_expert;
+    if (wave == 0) {
+      const int slot = blockIdx.y, k = gridDim.y;
+      const float prob = router_softmax64(p.route.logits[min(lane, p.route.n - 1)], p.route.n, lane);
+      int ej; float pj;
+      const int e = router_pick64(prob, p.route.n, slot, lane, ej, pj);
+      if (lane == 0) s_expert = e;
+      if (slot == k - 1 && blockIdx.x == 0) {
+        float sum = 0.0f;
+        for (int j = 0; j < k; j++) sum += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, pj), j));
+        if (lane < k) { p.route.experts[lane] = ej; p.route.gates[lane] = p.route.renorm ? (sum > 0.0f ? pj * (1.0f / sum) : 0.0f) : pj; }
+      }
+    }
+    __syncthreads();
+    bank_row = (int64_t)min(s_expert, p.bank_experts - 1) * p.expert_rows;
+  } else if constexpr (BANK == BANK_SLOTS)
     bank_row = (int64_t)min(max(p.slot_expert[blockIdx.y], 0), p.bank_experts - 1) * p.expert_rows;   // an id outside the bank (a router fed NaN) must not address memory
   int64_t row_bytes, aux_row_bytes = 0;
   if (QT == CAI_Q4_K) row_bytes = (int64_t)(cols >> 8) * 144;
@@ -767,6 +786,13 @@ bool gemv_fuses_swiglu(const cai_qw_s* w, int n_b, bool expert_bank)
   if (w->qtype == CAI_Q4_K || w->qtype == CAI_Q4_0 || w->qtype == CAI_Q8_0) return true;
   return raw_block_type(w->qtype) && n_b == 1 && !expert_bank && gemv_hands_off_ssq(w, 1);   // (integer-dot kernel only)
 }
+// (longer rows: what is held of them would be registers, and read in panels behind the weights they take longer than before them: 2000 x 12800
+// of Q8_0 12.4 us, 9.8 as gemv_fast)
+constexpr int ONE_COLS = 4096;
+bool gemv_routes(const cai_qw_s* bank, int n_experts, int k)
+{
+  return (bank->qtype == CAI_Q4_K || bank->qtype == CAI_Q4_0 || bank->qtype == CAI_Q8_0) && bank->cols <= ONE_COLS && n_experts <= 64 && k >= 1 && k <= n_experts;
+}
 static bool fast_type(int qt) { return qt == CAI_Q4_K || qt == CAI_Q4_0 || qt == CAI_Q8_0; }
 
 static int panel_len(int cols, int nb)
@@ -778,25 +804,23 @@ static int panel_len(int cols, int nb)
   return kp;
 }
 
-// (longer rows: what is held of them would be registers, and read in panels behind the weights they take longer than before them: 2000 x 12800
-// of Q8_0 12.4 us, 9.8 as gemv_fast)
-constexpr int ONE_COLS = 4096;
 template <int QT, int NB, int MODE>
-static int launch_fast_r(const GemvParams& p0, int n_groups_r, int R, int n_slots, hipStream_t st)
+static int launch_fast_r(const GemvParams& p0, const GemvRoute* route, int n_groups_r, int R, int n_slots, hipStream_t st)
 {
   GemvParams p = p0;
   const size_t lds = (size_t)NB * p.kp_lds * 4;
   const dim3 grid((n_groups_r + 3) / 4, n_slots);
   p.timeline = timeline_next((int)(grid.x * grid.y));
   if constexpr (NB == 1) if (p.cols <= ONE_COLS) {
-    auto go = [&](auto kern) {
-      hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, p.x, p.seg[0].data, p.seg[0].aux, p.norm_gain, p.residual, p.cols, p.seg[0].rows, p.seg[0].grp_end, p.n_seg, p);
+    auto go = [&](auto kern, const auto& args) {
+      hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, p.x, p.seg[0].data, p.seg[0].aux, p.norm_gain, p.residual, p.cols, p.seg[0].rows, p.seg[0].grp_end, p.n_seg, args);
     };
     auto rows = [&](auto bank, auto sv) {
-      constexpr bool BANK = decltype(bank)::value;
+      constexpr int BANK = decltype(bank)::value;
       constexpr int SV = decltype(sv)::value;
-      if constexpr (MODE == 0) { if (R == 4) { go(gemv_one<QT, 4, MODE, BANK, SV>); return; } }
-      if (R == 2) go(gemv_one<QT, 2, MODE, BANK, SV>); else go(gemv_one<QT, 1, MODE, BANK, SV>);
+      auto args = [&] { if constexpr (BANK == BANK_ROUTED) return GemvRouted{p, *route}; else return p; }();
+      if constexpr (MODE == 0) { if (R == 4) { go(gemv_one<QT, 4, MODE, BANK, SV>, args); return; } }
+      if (R == 2) go(gemv_one<QT, 2, MODE, BANK, SV>, args); else go(gemv_one<QT, 1, MODE, BANK, SV>, args);
     };
     auto width = [&](auto bank) {
       using std::integral_constant;
@@ -804,7 +828,10 @@ static int launch_fast_r(const GemvParams& p0, int n_groups_r, int R, int n_slot
       else if (p.cols <= 2048) rows(bank, integral_constant<int, 2>());
       else rows(bank, integral_constant<int, 4>());
     };
-    if (p.slot_expert) width(std::true_type()); else width(std::false_type());
+    if (route) {
+      if constexpr (MODE == 1) width(std::integral_constant<int, BANK_ROUTED>());
+      else return set_error(CAI_ERR_INVALID, "gemv: only the gated launch of a bank chooses its experts");
+    } else if (p.slot_expert) width(std::integral_constant<int, BANK_SLOTS>()); else width(std::integral_constant<int, BANK_NONE>());
     return CAI_OK;
   }
   if constexpr (NB == 1 && MODE == 0) {
@@ -827,7 +854,7 @@ static int pick_r(int64_t total_rows, int nb, int mode)
 
 
 template <int QT, int MODE>
-static int launch_fast_nb(GemvParams& p, const MultiGemv& m, int nb, hipStream_t st)
+static int launch_fast_nb(GemvParams& p, const GemvRoute* route, const MultiGemv& m, int nb, hipStream_t st)
 {
   int64_t total = 0;
   for (int i = 0; i < m.n; i++) total += m.rows[i];
@@ -839,14 +866,14 @@ static int launch_fast_nb(GemvParams& p, const MultiGemv& m, int nb, hipStream_t
     p.seg[i].grp_end = cum;
   }
   switch (nb) {
-    case 1: return launch_fast_r<QT, 1, MODE>(p, cum, R, ns, st);
-    case 2: return launch_fast_r<QT, 2, MODE>(p, cum, R, ns, st);
-    case 3: return launch_fast_r<QT, 3, MODE>(p, cum, R, ns, st);
-    case 4: return launch_fast_r<QT, 4, MODE>(p, cum, R, ns, st);
-    case 5: return launch_fast_r<QT, 5, MODE>(p, cum, R, ns, st);
-    case 6: return launch_fast_r<QT, 6, MODE>(p, cum, R, ns, st);
-    case 7: return launch_fast_r<QT, 7, MODE>(p, cum, R, ns, st);
-    case 8: return launch_fast_r<QT, 8, MODE>(p, cum, R, ns, st);
+    case 1: return launch_fast_r<QT, 1, MODE>(p, route, cum, R, ns, st);
+    case 2: return launch_fast_r<QT, 2, MODE>(p, route, cum, R, ns, st);
+    case 3: return launch_fast_r<QT, 3, MODE>(p, route, cum, R, ns, st);
+    case 4: return launch_fast_r<QT, 4, MODE>(p, route, cum, R, ns, st);
+    case 5: return launch_fast_r<QT, 5, MODE>(p, route, cum, R, ns, st);
+    case 6: return launch_fast_r<QT, 6, MODE>(p, route, cum, R, ns, st);
+    case 7: return launch_fast_r<QT, 7, MODE>(p, route, cum, R, ns, st);
+    case 8: return launch_fast_r<QT, 8, MODE>(p, route, cum, R, ns, st);
   }
   return set_error(CAI_ERR_INVALID, "gemv: n_b %d out of range 1..8", nb);
 }
@@ -885,10 +912,15 @@ int launch_gemv_multi(const MultiGemv& m, const float* x, int n_b, float* y, int
   p.ssq_in = nullptr; p.ssq_out = nullptr;
   p.slot_expert = m.slot_expert; p.expert_rows = m.expert_rows; p.x_slot_stride = m.x_slot_stride; p.y_slot_stride = m.y_slot_stride;
   const int n_slots = m.slot_expert ? m.n_slots : 1;
+  GemvRoute chosen; const GemvRoute* route = nullptr;
   if (m.slot_expert) {
     if (m.n != 1 || m.expert_rows <= 0 || w0->rows % m.expert_rows || m.row0[0] != 0 || m.rows[0] > m.expert_rows)
       return set_error(CAI_ERR_INVALID, "gemv: expert bank of %lld rows does not divide into windows of %lld", (long long)w0->rows, (long long)m.expert_rows);
     p.bank_experts = (int)(w0->rows / m.expert_rows);
+    if (m.route_logits) {
+      if (!swiglu_half || n_b != 1 || p.bank_experts != m.route_n || !gemv_routes(w0, m.route_n, n_slots)) return set_error(CAI_ERR_UNSUPPORTED, "gemv: a bank of type %d with %d experts does not choose by itself", w0->qtype, p.bank_experts);
+      chosen = GemvRoute{m.route_logits, m.route_n, m.route_renorm, const_cast<int32_t*>(m.slot_expert), m.route_gates}; route = &chosen;
+    }
   }
   for (int i = 0; i < m.n; i++) {
     const cai_qw_s* w = m.w[i];
@@ -919,23 +951,23 @@ int launch_gemv_multi(const MultiGemv& m, const float* x, int n_b, float* y, int
       if (m.n != 1) return set_error(CAI_ERR_INVALID, "gemv: swiglu takes one matrix");
       p.seg[0].rows = swiglu_half;
       MultiGemv mm = m; mm.rows[0] = swiglu_half;
-      if (qt == CAI_Q4_K) return launch_fast_nb<CAI_Q4_K, 1>(p, mm, n_b, c.stream);
-      if (qt == CAI_Q4_0) return launch_fast_nb<CAI_Q4_0, 1>(p, mm, n_b, c.stream);
-      return launch_fast_nb<CAI_Q8_0, 1>(p, mm, n_b, c.stream);
+      if (qt == CAI_Q4_K) return launch_fast_nb<CAI_Q4_K, 1>(p, route, mm, n_b, c.stream);
+      if (qt == CAI_Q4_0) return launch_fast_nb<CAI_Q4_0, 1>(p, route, mm, n_b, c.stream);
+      return launch_fast_nb<CAI_Q8_0, 1>(p, route, mm, n_b, c.stream);
     }
-    if (qt == CAI_Q4_K) return launch_fast_nb<CAI_Q4_K, 0>(p, m, n_b, c.stream);
-    if (qt == CAI_Q4_0) return launch_fast_nb<CAI_Q4_0, 0>(p, m, n_b, c.stream);
-    return launch_fast_nb<CAI_Q8_0, 0>(p, m, n_b, c.stream);
+    if (qt == CAI_Q4_K) return launch_fast_nb<CAI_Q4_K, 0>(p, nullptr, m, n_b, c.stream);
+    if (qt == CAI_Q4_0) return launch_fast_nb<CAI_Q4_0, 0>(p, nullptr, m, n_b, c.stream);
+    return launch_fast_nb<CAI_Q8_0, 0>(p, nullptr, m, n_b, c.stream);
   }
   if (qt == CAI_I8ROW && p.cols % 32 == 0 && !swiglu_half) {   // per-row int8 of a width the 16-byte walk covers; other widths below
     p.kp = panel_len(p.cols, n_b);
     p.kp_lds = (p.kp + 511) / 512 * 512;
-    return launch_fast_nb<CAI_I8ROW, 0>(p, m, n_b, c.stream);
+    return launch_fast_nb<CAI_I8ROW, 0>(p, nullptr, m, n_b, c.stream);
   }
   if (qt == CAI_Q6_K && !swiglu_half) {
     p.kp = panel_len(p.cols, n_b);
     p.kp_lds = (p.kp + 511) / 512 * 512;
-    return launch_fast_nb<CAI_Q6_K, 0>(p, m, n_b, c.stream);
+    return launch_fast_nb<CAI_Q6_K, 0>(p, nullptr, m, n_b, c.stream);
   }
   if (swiglu_half) return set_error(CAI_ERR_UNSUPPORTED, "gemv: fused swiglu needs a block-quantized matrix");
   if (raw_block_type(qt)) {

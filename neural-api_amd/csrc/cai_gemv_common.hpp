@@ -75,6 +75,10 @@ struct GemvParams {
   const uint8_t* seg_aux2[3];
   unsigned long long* timeline;   // stamps of this launch's work-groups (null: none)
 };
+// A bank whose slots' experts the launch chooses itself: soft-max over n logits, the most probable one a slot; the last slot's first work-group leaves ids and
+// gates for the launches behind.  (A record of its own: every launch copies its arguments.)
+struct GemvRoute { const float* logits; int n, renorm; int32_t* experts; float* gates; };
+struct GemvRouted : GemvParams { GemvRoute route; };
 
 __device__ __forceinline__ float cvt_ub0(uint32_t v) { return (float)(v & 0xffu); }
 __device__ __forceinline__ float cvt_ub1(uint32_t v) { return (float)((v >> 8) & 0xffu); }

@@ -259,7 +259,10 @@ struct MultiGemv {
   // RMSNorm hand-off between consecutive batch-1 Q4_K layers: the producer leaves per-work-group partials of
   // sum(y^2) (1024 floats) that the consumer sums instead of re-reducing its input.  Both optional.
   const float* ssq_in; float* ssq_out;
+  // expert bank whose launch chooses the slots' experts from router logits by itself (gemv_routes); ids (slot_expert) and gates are then results
+  const float* route_logits; int route_n, route_renorm; float* route_gates;
 };
+bool gemv_routes(const cai_qw_s* bank, int n_experts, int k);      // whether the gathered gate|up launch of one token can
 // norm_gain != null fuses RMSNorm(eps) of x into the staging; swiglu_half > 0 computes
 // y[i] = up_i * silu(gate_i) from rows i and swiglu_half + i of the (single) matrix.
 int launch_gemv_multi(const MultiGemv& m, const float* x, int n_b, float* y, int64_t y_stride, int act,
@@ -277,6 +280,7 @@ int noalloc_setup(int device);   // resolves the device address of the fixed scr
 int launch_embed(const cai_qw_s* w, const int32_t* tokens_dev, int n_tokens, float* out);
 int launch_router_topk(const float* logits, int n, int k, int renorm, int n_tokens, int32_t* expert_out, float* gate_out, float* probs_scratch);
 // ... and the router's matrix-vector product, RMSNorm and selection in one launch (Q8_0 router rows, up to 64 experts)
+bool router_in_launch();
 bool router_fused_supported(const cai_qw_s* w, int k);
 int launch_router_fused(const cai_qw_s* w, const float* x, int64_t x_stride, const float* gain, float eps, int k, int renorm, int n_tokens,
                         float* logits_out, int32_t* expert_out, float* gate_out, float* probs_scratch, unsigned* counters);   // counters: one per token, zero before the first launch (they wrap back to zero)

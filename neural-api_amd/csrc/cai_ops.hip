@@ -1,21 +1,11 @@
 // Elementwise layer math, block dequantization, embedding gather, arg-max and the MoE router for gfx950.
 #include "cai_layered.hpp"
 #include "cai_blocks_raw.hpp"
-#include "cai_gemv_common.hpp"
+#include "cai_router.hpp"
 #include <string.h>
 #include <math.h>
 
 namespace cai {
-
-__device__ __forceinline__ float last_lane(float v) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63)); }
-// maximum of the wave, valid in lane 63 (wave_sum's steps; a lane without a partner keeps its own)
-__device__ __forceinline__ float wave_max(float v)
-{
-#define STEP(ctrl, rows) { const int t = __builtin_bit_cast(int, v); v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(t, t, ctrl, rows, 0xf, false))); }
-  STEP(0x111, 0xf) STEP(0x112, 0xf) STEP(0x114, 0xf) STEP(0x118, 0xf) STEP(0x142, 0xa) STEP(0x143, 0xc)
-#undef STEP
-  return v;
-}
 
 __device__ __forceinline__ float wave_sum_all(float v)
 {
@@ -462,29 +452,13 @@ int noalloc_setup(int device)
 // One wave per token; lane i owns experts i, i+64, ...  Selection is k rounds of a wave-wide arg-max in which the
 // larger probability wins and, between equals, the lower expert index (the reference scans upwards with '>').
 constexpr int ROUTER_MAX_PER_LANE = 8;   // up to 512 experts
-// Selection key of a probability: larger key = selected earlier.  A total order whatever the value: lanes that hold no expert
-// get 0, a NaN (a poisoned activation row reaches the router as NaN logits) ranks below every number, and probabilities are
-// non-negative, so their bit patterns order like their values.  With a total order the k selected experts are always k
-// distinct ids inside [0, n); the gates still carry the NaN to the outputs.
-__device__ __forceinline__ uint32_t router_key(float p, bool candidate)
-{
-  if (!candidate) return 0u;
-  if (!(p == p)) return 1u;
-  return __builtin_bit_cast(uint32_t, fmaxf(p, 0.0f)) + 2u;
-}
 // Soft-max over n <= 64 logits and the k largest probabilities, by ONE wave (lane i owns expert i and brings its logit): every lane ranks its own
 // probability against the 64 broadcast ones (larger first, lower index between equals) - a permutation of 0..63 - and the lanes
 // of rank 0..k-1 are the selection, in order.  Returns the probability of the lane's expert; lane j < k gets the j-th selected
 // expert and its gate (divided by the sum of the k selected when renorm is set).
 __device__ __forceinline__ float router_select64(float logit, int n, int k, int renorm, int lane, int& expert_j, float& gate_j)
 {
-  float v = lane < n ? logit : -3.0e38f;
-  const float mx = last_lane(wave_max(v));
-  float a = v - mx; a = a > 4000.0f ? 4000.0f : (a < -4000.0f ? -4000.0f : a);
-  v = lane < n ? expf(a) : 0.0f;
-  const float tot = last_lane(wave_sum(v));
-  const float inv = tot > 0.0f ? 1.0f / tot : 1.0f;
-  v *= inv;
+  const float v = router_softmax64(logit, n, lane);
   const float pv = lane < n ? v : -1.0f;      // -1 marks "not a candidate"
   const uint32_t key = router_key(pv, lane < n);
   int rank = 0;
@@ -634,10 +608,14 @@ __global__ __launch_bounds__(256) void router_fused_kernel(const float* x, const
   if (lane < k) { expert_out[t * k + lane] = ej; gate_out[t * k + lane] = gj; }
 }
 
+bool router_in_launch()
+{
+  static const bool on = []() { const char* e = getenv("CAIHIP_ROUTER_LAUNCHES"); return !(e && e[0] == '1'); }();   // (1: product and selection are launches of their own)
+  return on;
+}
 bool router_fused_supported(const cai_qw_s* w, int k)
 {
-  static const bool off = []() { const char* e = getenv("CAIHIP_ROUTER_LAUNCHES"); return e && e[0] == '1'; }();   // keep the two launches
-  return !off && w->qtype == CAI_Q8_0 && !w->bias && w->rows >= 1 && w->rows <= 64 && k >= 1 && k <= w->rows && w->cols % 32 == 0;
+  return router_in_launch() && w->qtype == CAI_Q8_0 && !w->bias && w->rows >= 1 && w->rows <= 64 && k >= 1 && k <= w->rows && w->cols % 32 == 0;
 }
 int launch_router_fused(const cai_qw_s* w, const float* x, int64_t x_stride, const float* gain, float eps, int k, int renorm, int n_tokens,
                         float* logits_out, int32_t* expert_out, float* gate_out, float* probs_scratch, unsigned* counters)

@@ -217,6 +217,25 @@ def test_batched_decode_of_q4k_q6k_and_q8_matrices_equals_single(types, d, heads
                 assert np.max(np.abs(lg[b] - singles[b][p])) <= 2e-5 * np.max(np.abs(singles[b][p])), (n, p, b)
 
 
+@pytest.mark.parametrize("experts,top_k,norm_topk,qtype,d_model", [
+    (1, 1, 0, O.Q8_0, 256), (5, 5, 1, O.Q8_0, 1056), (64, 8, 0, O.Q4_0, 256), (63, 1, 1, O.Q4_K, 2304), (33, 8, 1, O.Q8_0, 4096),   # chosen by the gate|up launch
+    (33, 3, 1, O.Q8_0, 4128), (65, 2, 1, O.Q8_0, 256)])                                                                          # rows too long, experts too many: chosen before it
+def test_one_token_steps_choose_their_experts(experts, top_k, norm_topk, qtype, d_model):
+    """Both sides of the rule that lets the gathered gate|up launch choose the experts of a one-token step, at the edges of expert counts, places, bank types and
+    the three widths its kernel holds: the logits of the oracle, within the bound of the other quantized decoders."""
+    from helpers.device import dev, rel_err
+    cai = dev()
+    cfg = dict(n_layers=2, d_model=d_model, n_q_heads=4, n_kv_heads=2, head_dim=64, ffn=256 if qtype == O.Q4_K else 96, vocab=300, max_ctx=16, eps=1e-5, rope_theta=1e4,
+               n_experts=experts, top_k=top_k, norm_topk=norm_topk)
+    spec = synthetic_spec(cfg, qtype, std=0.05)
+    om = oracle_model(spec, acc64=1)
+    dec = cai.Decoder(spec)
+    for p, t in enumerate([3, 14, 299, 0, 65, 35]):
+        _, lo = om.step(t, p); _, ld = dec.step(t, p)
+        assert rel_err(ld[0], lo) < 1e-3, (p, rel_err(ld[0], lo))
+    dec.close()
+
+
 @pytest.mark.parametrize("name,n", [("olmoe_like_q8", 11), ("olmoe_like_q8", 45), ("moe_like_q6k", 29)])
 def test_moe_prefill_equals_sequential_steps(name, n):
     """Mixture-of-experts prompts: attention half on the whole chunk, routed half per group of rows (router and top-k once
