@@ -77,8 +77,8 @@ int  ensure_host_stage(size_t need);   // grows ctx().h_stage; only for calls th
 // An event goes out behind the last launch, while it runs: without one the runtime asks for the stream's end when the host program next
 // synchronises the device, later and at more cost.  us, 40 / 8 heads behind 8191 int8 rows, call after call | one call and hipDeviceSynchronize: hipStreamSynchronize in
 // the call 24.1 | 27.1, the flag alone 20.9 | 32, flag and event 22.1 | 25.6; a step of the 135M shape 583 | 586, 575 | 595, 575 | 584.
-// (The samplers' candidates leave in single words from many work-groups and wait for the end of the stream: with host_store and the flag 300 of 50000 took 69 us instead of 54, 905 of
-// 188977 68 instead of 59, 40 of 152064 the same.)
+// (Candidates that a launch of many work-groups ranks leave in single words and wait for the end of the stream: with host_store and the flag 300 of 50000 took 69 us instead of 54, 905 of
+// 188977 68 instead of 59.  Those that one work-group ranks take the flag.)
 constexpr int HOST_SIGNALS = 8;            // of one call
 struct HostSignal { uint32_t* flag = nullptr; unsigned* arrive = nullptr; uint32_t value = 0; };      // flag null: none
 HostSignal host_signal_next(int k = 0);    // the k-th of this call

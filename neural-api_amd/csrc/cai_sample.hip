@@ -8,11 +8,12 @@
 // The draw stays with the host and its own random generator: it gets m (token, probability) pairs instead of the row.
 //
 // The row is cut into at most 256 slices, one work-group each, and every stage that needs a number of the whole row is a launch
-// boundary: slice maxima and sums -> [penalised probabilities] -> last values and a histogram of their leading 12 bits -> the few
-// values at or above the bin that holds the m-th largest -> their ranking, by one work-group up to 32 candidates and sixteen for more.
-// What bounds it is launches (five, four without a penalty), not bytes: a 152k row with penalties, temperature and 40 candidates takes 44 us a call, 284 as
-// one work-group that walked the row ten times out of L2 at the 40 GB/s one compute unit gets.
-#include "cai_internal.hpp"
+// boundary: slice maxima and sums (and the history, out of pinned memory) -> penalised probabilities and the largest of each group of 4 to 64 -> last values, and
+// the few whose probability is at or above the bin that holds the m-th largest of those maxima -> their ranking, by the third launch's last work-group up to
+// 128 candidates and by a launch of sixteen for more.
+// What bounds it is launches and round trips, not bytes.  us a call, five launches and a copy with a histogram of the last values, waiting for the end of the stream | this: 40 of 152064
+// behind a history of 512, penalties and temperature 44.4 | 29.9; without penalties 36.1 | 27.7; 5 of 152064 42.1 | 27.8; 300 of 50000 behind 3000 54.0 | 37; 905 of 152064 57.6 | 41.
+#include "cai_router.hpp"
 #include <algorithm>
 #include <string.h>
 
@@ -23,15 +24,17 @@ constexpr int SMP_MAX_M = 1024;
 constexpr int SL_T = 256;         // threads of a slice's work-group
 constexpr int SL_MAX = 256;       // slices: a thread of a work-group folds one slice's number
 constexpr int SMP_BINS = 4096;
+constexpr int TOP_MAX = 8192;     // maxima of groups
 constexpr int RANK_MAX = 2048;    // values ranked by comparison with each other; more go through a radix select first
+constexpr int SMP_FOLD_M = 128;   // candidates that the third launch ranks itself: 32.5 us a call for 128; a launch of sixteen work-groups 35.4 for 200, 36.7 for 500
 constexpr int RANK_WG = 16;       // work-groups that share the ranking
 
 template <int NT>
 __device__ __forceinline__ float smp_max(float v, float* red)
 {
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+  v = wave_max(v);
   __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  if ((threadIdx.x & 63) == 63) red[threadIdx.x >> 6] = v;
   __syncthreads();
   float r = red[0];
 #pragma unroll
@@ -42,9 +45,9 @@ __device__ __forceinline__ float smp_max(float v, float* red)
 template <int NT>
 __device__ __forceinline__ float smp_sum(float v, float* red)
 {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  v = wave_sum(v);
   __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  if ((threadIdx.x & 63) == 63) red[threadIdx.x >> 6] = v;
   __syncthreads();
   float r = 0.0f;
 #pragma unroll
@@ -57,8 +60,10 @@ template <int NT>
 __device__ __forceinline__ int smp_excl_scan(int v, int* red, int* total)
 {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  int inc = v;
-  for (int o = 1; o < 64; o <<= 1) { const int t = __shfl_up(inc, o, 64); if (lane >= o) inc += t; }
+  int inc = v;                                   // (wave_sum's steps leave every lane the sum up to itself)
+#define STEP(ctrl, rows) inc += __builtin_amdgcn_update_dpp(0, inc, ctrl, rows, 0xf, true);
+  STEP(0x111, 0xf) STEP(0x112, 0xf) STEP(0x114, 0xf) STEP(0x118, 0xf) STEP(0x142, 0xa) STEP(0x143, 0xc)
+#undef STEP
   __syncthreads();
   if (lane == 63) red[w] = inc;
   __syncthreads();
@@ -78,7 +83,11 @@ __device__ __forceinline__ void smp_crossing(const int* hist, int need, int* red
   const int b0 = SMP_BINS - 1 - PER * (int)threadIdx.x;
   int own[PER], sum = 0, total;
 #pragma unroll
-  for (int k = 0; k < PER; k++) { own[k] = hist[b0 - k]; sum += own[k]; }
+  for (int k = 0; k < PER; k += 4) {
+    const int4 t = *reinterpret_cast<const int4*>(hist + b0 - k - 3);
+    own[k] = t.w; own[k + 1] = t.z; own[k + 2] = t.y; own[k + 3] = t.x;
+    sum += t.x + t.y + t.z + t.w;
+  }
   int acc = smp_excl_scan<NT>(sum, redi, &total);
   if (acc < need && need <= acc + sum) {        // exactly one thread: the crossing lies in its bins
 #pragma unroll
@@ -92,17 +101,41 @@ __device__ __forceinline__ void smp_crossing(const int* hist, int need, int* red
 
 struct SampleParams {
   const float* logits; int n;
-  const int32_t* hist_ids; const int32_t* hist_counts; int n_hist;
+  int32_t* hist_ids; int32_t* hist_counts; int n_hist;      // ... behind each other
+  const int32_t* hist_src;           // pinned host memory
   float repetition, frequency, presence, temperature;
   int m;
   int slice, n_slices;               // values of a slice (a multiple of 256); slices
-  int penalty;                       // some token of the history lies in the row and a penalty is set
   float* val;                        // [n] probabilities on the way
   float* cand_v; int32_t* cand_t;    // [n_slices][slice] the slice's values in reach of the m largest, in token order
-  int* bins;                         // [4096] values per leading 12 bits
+  uint32_t* top; int n_top, groups;  // bits of the maxima of the slices' groups of values (`groups` of every slice), or of a short row's values themselves
   float *st_max, *st_sum, *st_tot, *st_pmax, *st_sum2; int* st_cnt;   // [256] per slice
   int32_t* tok_out; float* p_out;    // host memory
+  HostSignal done;                   // set where the last work-group of the third launch ranks
 };
+
+// where the e-th value in reach lies: in the last slice that starts at or before it
+__device__ __forceinline__ int smp_slot(const int* start, int e, int slice)
+{
+  int s = 0;
+#pragma unroll
+  for (int step = SL_MAX / 2; step > 0; step >>= 1) if (start[s + step] <= e) s += step;
+  return s * slice + e - start[s];
+}
+// A value and its token as one number: descending values, equal ones by token.  (Values are not negative, so their bits order like they do; a NaN is the largest and has
+// a place like any other.)
+__device__ __forceinline__ uint64_t smp_key(float v, int32_t t) { return (uint64_t)__float_as_uint(v) << 32 | ~(uint32_t)t; }
+__device__ __forceinline__ int32_t smp_token(uint64_t k) { return (int32_t)~(uint32_t)k; }
+__device__ __forceinline__ float smp_value(uint64_t k) { return __uint_as_float((uint32_t)(k >> 32)); }
+// the place of a key among `total`, by eight neighbouring lanes
+__device__ __forceinline__ int smp_rank(const uint64_t* key, int total, uint64_t own)
+{
+  int rank = 0;
+#pragma unroll 8
+  for (int j = threadIdx.x & 7; j < total; j += 8) rank += key[j] > own;
+  rank += __shfl_xor(rank, 1); rank += __shfl_xor(rank, 2); rank += __shfl_xor(rank, 4);
+  return rank;
+}
 
 // the same clamps as the host row soft-max (a NaN counts as far below the maximum)
 __device__ __forceinline__ float smp_exp(float v, float mx) { return expf(fminf(fmaxf(v - mx, -4000.0f), 4000.0f)); }
@@ -117,133 +150,218 @@ __device__ __forceinline__ void smp_row_stats(const SampleParams& p, float* red,
   inv = sum > 0.0f ? 1.0f / sum : 0.0f;
 }
 
+// A slice of up to HELD x 256 values stays in registers over a launch
+constexpr int HELD = 8;
+// the work-groups behind the slices': the history, 8 x SL_T words each (as a copy of the stream's own it was one more launch)
+constexpr int HIST_PER = 8 * SL_T;
 __global__ __launch_bounds__(SL_T) void candidates_stats_kernel(const SampleParams p)
 {
   __shared__ float red[SL_T / 64];
+  if ((int)blockIdx.x >= p.n_slices) {
+    const int i0 = ((int)blockIdx.x - p.n_slices) * HIST_PER + threadIdx.x, n = 2 * p.n_hist;
+    int32_t t[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) t[u] = __hip_atomic_load(p.hist_src + min(i0 + u * SL_T, n - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+#pragma unroll
+    for (int u = 0; u < 8; u++) if (i0 + u * SL_T < n) p.hist_ids[i0 + u * SL_T] = t[u];
+    return;
+  }
   const int i0 = blockIdx.x * p.slice, len = min(p.slice, p.n - i0);
-  for (int b = blockIdx.x * SL_T + threadIdx.x; b < SMP_BINS; b += p.n_slices * SL_T) p.bins[b] = 0;
-  float mx = -3.0e38f;
-  for_strided8(p.logits + i0, threadIdx.x, len, SL_T, [&](float v, int) { mx = fmaxf(mx, v); });
+  const float* x = p.logits + i0;
+  float mx = -3.0e38f, sum = 0.0f, t[HELD];
+#pragma unroll
+  for (int u = 0; u < HELD; u++) { t[u] = x[min((int)threadIdx.x + u * SL_T, len - 1)]; mx = fmaxf(mx, t[u]); }
+  for_strided8(x, threadIdx.x + HELD * SL_T, len, SL_T, [&](float v, int) { mx = fmaxf(mx, v); });
   mx = smp_max<SL_T>(mx, red);
-  float sum = 0.0f;
-  for_strided8(p.logits + i0, threadIdx.x, len, SL_T, [&](float v, int) { sum += smp_exp(v, mx); });
+#pragma unroll
+  for (int u = 0; u < HELD; u++) if ((int)threadIdx.x + u * SL_T < len) sum += smp_exp(t[u], mx);
+  for_strided8(x, threadIdx.x + HELD * SL_T, len, SL_T, [&](float v, int) { sum += smp_exp(v, mx); });
   sum = smp_sum<SL_T>(sum, red);
   if (threadIdx.x == 0) { p.st_max[blockIdx.x] = mx; p.st_sum[blockIdx.x] = sum; }
 }
 
-// probabilities with the history penalty: p^r, * exp(-(f * count + presence)) on the distinct context tokens
+// Probabilities with the history penalty: p^r, * exp(-(f * count + presence)) on the distinct context tokens.  What follows keeps their order, but for its
+// rounding, so the largest ones of groups of values, found here, tell the next launch where the m-th largest lies (a histogram of the row by atomics: 8.7 us of launch, 5.5 so).
+template <bool SHORT>                            // slices of up to HELD x 256 values
 __global__ __launch_bounds__(SL_T) void candidates_penalty_kernel(const SampleParams p)
 {
   __shared__ float red[SL_T / 64];
-  const int i0 = blockIdx.x * p.slice, len = min(p.slice, p.n - i0);
+  __shared__ float held[SHORT ? HELD * SL_T : 1];
+  const int i0 = blockIdx.x * p.slice, len = min(p.slice, p.n - i0), tid = threadIdx.x;
+  constexpr int ID = 4;
+  int id[ID], count[ID];                         // (the first of the history on their way beside the row)
+  float t[HELD];
+#pragma unroll
+  for (int u = 0; u < ID; u++) if (p.n_hist) { const int k = min(tid + u * SL_T, p.n_hist - 1); id[u] = p.hist_ids[k]; count[u] = p.hist_counts[k]; }
+  if (SHORT) {
+#pragma unroll
+    for (int u = 0; u < HELD; u++) t[u] = p.logits[i0 + min(tid + u * SL_T, len - 1)];
+  }
   float mx, inv;
   smp_row_stats(p, red, mx, inv);
-  float* val = p.val + i0;
-  for_strided8(p.logits + i0, threadIdx.x, len, SL_T, [&](float v, int i) { const float e = smp_exp(v, mx); val[i] = inv > 0.0f ? e * inv : e; });
-  __syncthreads();
-  for (int k = threadIdx.x; k < p.n_hist; k += SL_T) {
-    const int t = p.hist_ids[k] - i0;
-    if (t < 0 || t >= len) continue;
-    float v = val[t];
-    if (p.repetition != 1.0f && v > 0.0f) v = powf(v, p.repetition);
-    if (p.frequency != 0.0f || p.presence != 0.0f) v *= expf(-(p.frequency * (float)p.hist_counts[k] + p.presence));
-    val[t] = v;
+  float* const out = p.val + i0;
+  float* const val = SHORT ? held : out;
+  auto prob = [&](float v) { const float e = smp_exp(v, mx); return inv > 0.0f ? e * inv : e; };
+  if (SHORT) {
+#pragma unroll
+    for (int u = 0; u < HELD; u++) if (tid + u * SL_T < len) held[tid + u * SL_T] = prob(t[u]);
+  } else
+    for_strided8(p.logits + i0, tid, len, SL_T, [&](float v, int i) { out[i] = prob(v); });
+  if (p.n_hist) {
+    __syncthreads();
+    auto penalise = [&](int t, int c) {
+      float v = val[t];
+      if (p.repetition != 1.0f && v > 0.0f) v = powf(v, p.repetition);
+      if (p.frequency != 0.0f || p.presence != 0.0f) v *= expf(-(p.frequency * (float)c + p.presence));
+      val[t] = v;
+    };
+#pragma unroll
+    for (int u = 0; u < ID; u++) { const int j = id[u] - i0; if (tid + u * SL_T < p.n_hist && j >= 0 && j < len) penalise(j, count[u]); }
+    for (int k = tid + ID * SL_T; k < p.n_hist; k += SL_T) { const int j = p.hist_ids[k] - i0; if (j >= 0 && j < len) penalise(j, p.hist_counts[k]); }
+    __syncthreads();
   }
-  __syncthreads();
   float tot = 0.0f, top = 0.0f;
-  for_strided8(val, threadIdx.x, len, SL_T, [&](float v, int) { tot += v; top = fmaxf(top, v); });
+  uint32_t own = 0;
+  for_strided8(val, tid, len, SL_T, [&](float v, int i) {
+    tot += v; top = fmaxf(top, v); own = max(own, __float_as_uint(v));
+    if (SHORT) out[i] = v;
+  });
   tot = smp_sum<SL_T>(tot, red);
   top = smp_max<SL_T>(top, red);
-  if (threadIdx.x == 0) { p.st_tot[blockIdx.x] = tot; p.st_pmax[blockIdx.x] = top; }
+  if (tid == 0) { p.st_tot[blockIdx.x] = tot; p.st_pmax[blockIdx.x] = top; }
+  if (p.groups == 0) return;
+  // groups of SL_T / groups neighbouring threads: 16, 4 or 1
+  if (p.groups <= SL_T / 4) { own = max(own, (uint32_t)__shfl_xor((int)own, 1)); own = max(own, (uint32_t)__shfl_xor((int)own, 2)); }
+  if (p.groups <= SL_T / 16) { own = max(own, (uint32_t)__shfl_xor((int)own, 4)); own = max(own, (uint32_t)__shfl_xor((int)own, 8)); }
+  const int of = SL_T / p.groups;
+  if (tid % of == 0) p.top[blockIdx.x * p.groups + tid / of] = own;
 }
 
-// last values: the probabilities, or with a temperature exp(ln(max(p, 1e-30)) / T - ln(max p) / T) still to be divided by its sum
-__global__ __launch_bounds__(SL_T) void candidates_value_kernel(const SampleParams p)
-{
-  __shared__ float red[SL_T / 64];
-  __shared__ int bins[SMP_BINS];
-  const int i0 = blockIdx.x * p.slice, len = min(p.slice, p.n - i0), g = threadIdx.x;
-  for (int b = g; b < SMP_BINS; b += SL_T) bins[b] = 0;
-  float mx = 0.0f, inv = 0.0f, tot = 0.0f, pm;
-  if (p.penalty) {
-    tot = smp_sum<SL_T>(g < p.n_slices ? p.st_tot[g] : 0.0f, red);
-    pm = smp_max<SL_T>(g < p.n_slices ? p.st_pmax[g] : 0.0f, red);
-    if (tot > 0.0f) pm = pm / tot;
-  } else {
-    smp_row_stats(p, red, mx, inv);
-    pm = inv;                                   // the maximum's exponential is 1
-  }
-  const bool warm = p.temperature != 1.0f && pm > 0.0f;
-  const float lm = logf(fmaxf(pm, 1e-30f)), inv_t = 1.0f / fmaxf(p.temperature, 1e-6f);
-  __syncthreads();
-  float sum2 = 0.0f;
-  const float* src = p.penalty ? p.val + i0 : p.logits + i0;
-  for_strided8(src, g, len, SL_T, [&](float v, int i) {
-    if (p.penalty) { if (tot > 0.0f) v = v / tot; }
-    else { v = smp_exp(v, mx); if (inv > 0.0f) v *= inv; }
-    if (warm) { v = expf(logf(fmaxf(v, 1e-30f)) * inv_t - lm * inv_t); sum2 += v; }
-    p.val[i0 + i] = v;
-    atomicAdd(&bins[__float_as_uint(v) >> 20], 1);
-  });
-  sum2 = smp_sum<SL_T>(sum2, red);
-  if (g == 0) p.st_sum2[blockIdx.x] = warm ? sum2 : -1.0f;      // (< 0: nothing to divide by)
-  __syncthreads();
-  for (int b = g; b < SMP_BINS; b += SL_T) { const int c = bins[b]; if (c) atomicAdd(&p.bins[b], c); }
-}
-
-// the slice's values that can be among the m largest, in token order
+// Last values: the probabilities, or with a temperature exp(ln(max(p, 1e-30)) / T - ln(max p) / T) still to be divided by its sum.  The slice's values that
+// can be among the m largest are kept in token order.  FOLDED: the work-group that arrives last ranks them (the hand-over of the attention's merge) and
+// leaves them to the host, or a token of -1 if they are more than it takes; a launch less, and the host reads the flag before the end of the stream.
+constexpr int FOLD_MAX = 512;
+template <typename T> __device__ __forceinline__ void part_put(T* q, T v) { __hip_atomic_store(q, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+template <typename T> __device__ __forceinline__ T part_get(const T* q) { return __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+template <bool FOLDED>
 __global__ __launch_bounds__(SL_T) void candidates_reach_kernel(const SampleParams p)
 {
   __shared__ float red[SL_T / 64];
   __shared__ int redi[SL_T / 64];
   __shared__ int sel[2];
-  const int i0 = blockIdx.x * p.slice, g = threadIdx.x, per = p.slice / SL_T;
-  const float s2 = g < p.n_slices ? p.st_sum2[g] : 0.0f;
-  const bool warm = !(p.st_sum2[0] < 0.0f);
-  float inv = smp_sum<SL_T>(s2, red);
-  inv = warm ? 1.0f / (inv <= 0.0f ? 1.0f : inv) : 1.0f;
-  smp_crossing<SL_T>(p.bins, min(p.m, p.n), redi, sel);
-  // A division by the sum keeps the order but can make neighbours equal, and equal ones go by token: a quotient rounds two steps of its
-  // dividend together at most, and with the rounding of the reciprocal values up to four steps below the bin are still in reach.  Where the quotients lose bits to the end of the number range everything is.
-  uint32_t floor_bits = (uint32_t)sel[0] << 20;
-  floor_bits = warm && __uint_as_float(floor_bits) * inv < 1.0e-36f ? 0u : floor_bits < 4u ? 0u : floor_bits - 4u;
-  int mine = 0, total;
-  const int j0 = g * per;
-  for (int k = 0; k < per; k++) mine += i0 + j0 + k < p.n && __float_as_uint(p.val[i0 + j0 + k]) >= floor_bits;
-  int at = smp_excl_scan<SL_T>(mine, redi, &total);
-  for (int k = 0; mine > 0 && k < per; k++) {
-    const int i = i0 + j0 + k;
-    if (i >= p.n) break;
-    const float v = p.val[i];
-    if (__float_as_uint(v) >= floor_bits) { p.cand_v[i0 + at] = v * inv; p.cand_t[i0 + at] = i; at++; }
+  __shared__ alignas(16) int bins[SMP_BINS];
+  const int i0 = blockIdx.x * p.slice, g = threadIdx.x, per = p.slice / SL_T, j0 = i0 + g * per;
+  float v[4];                                    // (a slice has four values a thread at least; past the row any values)
+#pragma unroll
+  for (int k = 0; k < 4; k++) v[k] = p.val[j0 + k];
+  const float own_tot = g < p.n_slices ? p.st_tot[g] : 0.0f, own_max = g < p.n_slices ? p.st_pmax[g] : 0.0f;
+  // where the m-th largest of the maxima lies: at least as many values lie there or above
+  constexpr int TOPS = 12;
+  uint32_t t[TOPS];
+#pragma unroll
+  for (int u = 0; u < TOPS; u++) t[u] = p.top[min(g + u * SL_T, p.n_top - 1)];
+#pragma unroll
+  for (int b = 0; b < SMP_BINS / SL_T / 4; b++) reinterpret_cast<int4*>(bins)[g + b * SL_T] = int4{0, 0, 0, 0};
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < TOPS; u++) if (g + u * SL_T < p.n_top) atomicAdd(&bins[t[u] >> 20], 1);
+  for_strided8(reinterpret_cast<const float*>(p.top), g + TOPS * SL_T, p.n_top, SL_T, [&](float w, int) { atomicAdd(&bins[__float_as_uint(w) >> 20], 1); });
+  float pm, tot = 0.0f;
+  if (p.n_hist) {
+    tot = smp_sum<SL_T>(own_tot, red);
+    pm = smp_max<SL_T>(own_max, red);
+    if (tot > 0.0f) pm = pm / tot;
+  } else {
+    float mx;
+    smp_row_stats(p, red, mx, pm);              // the maximum's exponential is 1
   }
-  if (g == 0) p.st_cnt[blockIdx.x] = total;
+  const bool warm = p.temperature != 1.0f && pm > 0.0f;
+  const float lm = logf(fmaxf(pm, 1e-30f)), inv_t = 1.0f / fmaxf(p.temperature, 1e-6f);
+  auto last = [&](float v) {
+    if (tot > 0.0f) v = v / tot;
+    return warm ? expf(logf(fmaxf(v, 1e-30f)) * inv_t - lm * inv_t) : v;
+  };
+  smp_crossing<SL_T>(bins, min(p.m, p.n), redi, sel);      // (behind the barriers of the sums)
+  // The steps after the maxima keep the order but can make neighbours equal, and equal ones go by token.  A quotient rounds two steps of its dividend together at
+  // most: four steps below the bin are still in reach.  With a temperature a whole bin is, 6 % of the value at least: 0.06 / T of the exponent, whose own
+  // errors are 3e-5 / T (of logarithms up to 69) and 1e-6.  Where values lose bits to the end of the number range, meet the logarithm's floor or have no finite sum, everything is.
+  uint32_t floor_bits = (uint32_t)sel[0] << 20;
+  const uint32_t slack = warm ? 1u << 20 : 4u;
+  floor_bits = floor_bits < slack ? 0u : floor_bits - slack;
+  const float low = __uint_as_float(floor_bits), lowest = last(low);
+  const bool clear = warm ? tot < 3.0e38f && (tot > 0.0f ? low / tot : low) > 1.0e-29f && lowest > 1.0e-35f * (float)p.n && p.temperature < 1000.0f : lowest > 1.0e-36f;
+  if (!clear) floor_bits = 0u;
+  int mine = 0, total;
+  float sum2 = 0.0f;
+#pragma unroll
+  for (int k = 0; k < 4; k++) if (j0 + k < p.n) { mine += __float_as_uint(v[k]) >= floor_bits; if (warm) sum2 += last(v[k]); }
+  for (int k = 4; k < per && j0 + k < p.n; k++) { const float t = p.val[j0 + k]; mine += __float_as_uint(t) >= floor_bits; if (warm) sum2 += last(t); }
+  sum2 = smp_sum<SL_T>(sum2, red);
+  int at = smp_excl_scan<SL_T>(mine, redi, &total);
+  if (!warm) sum2 = -1.0f;                       // (< 0: nothing to divide by)
+  auto put = [](auto* q, auto v) { if constexpr (FOLDED) part_put(q, v); else *q = v; };
+  if (g == 0) { put(p.st_sum2 + blockIdx.x, sum2); put(p.st_cnt + blockIdx.x, total); }
+  for (int k = 0; mine > 0 && k < per && j0 + k < p.n; k++) {
+    const float t = p.val[j0 + k];
+    if (__float_as_uint(t) >= floor_bits) { put(p.cand_v + i0 + at, last(t)); put(p.cand_t + i0 + at, (int32_t)(j0 + k)); at++; }
+  }
+  if constexpr (FOLDED) {
+    __shared__ int s_is_last;
+    __shared__ int start[SL_MAX];
+    __shared__ uint64_t key[FOLD_MAX], place[SMP_FOLD_M];
+    __builtin_amdgcn_s_waitcnt(0x0F70);          // vmcnt(0): this thread's values have been acknowledged
+    __syncthreads();
+    if (g == 0) s_is_last = __builtin_amdgcn_atomic_inc32(p.done.arrive, gridDim.x - 1, __ATOMIC_RELAXED, "agent") == gridDim.x - 1;
+    __syncthreads();
+    if (!s_is_last) return;
+    const int m = min(p.m, p.n), own = g < p.n_slices ? part_get(p.st_cnt + g) : 0;
+    float inv = smp_sum<SL_T>(g < p.n_slices ? part_get(p.st_sum2 + g) : 0.0f, red);
+    inv = !warm ? 1.0f : 1.0f / (inv <= 0.0f ? 1.0f : inv);
+    start[g] = smp_excl_scan<SL_T>(own, redi, &total);
+    __syncthreads();
+    if (total <= FOLD_MAX) {
+      for (int e = g; e < total; e += SL_T) {
+        const int j = smp_slot(start, e, p.slice);
+        key[e] = smp_key(part_get(p.cand_v + j) * inv, part_get(p.cand_t + j));
+      }
+      __syncthreads();
+      for (int e = g >> 3; e < total; e += SL_T / 8) {
+        const uint64_t k = key[e];
+        const int rank = smp_rank(key, total, k);
+        if ((g & 7) == 0 && rank < m) place[rank] = k;
+      }
+      __syncthreads();
+      for (int r = g; r < m; r += SL_T) { host_store(p.tok_out + r, smp_token(place[r])); host_store(p.p_out + r, smp_value(place[r])); }
+    } else if (g == 0) host_store(p.tok_out, (int32_t)-1);
+    host_signal(p.done, 1);
+  }
 }
 
 // descending probability, equal ones by token.  Every work-group gathers the whole list (a few thousand values from the L2) and ranks its
-// share of it: the comparisons, not the gathering, were the time of one work-group (of 152064 logits,
-// a whole call: 1000 candidates 185 -> 59 us, 256 65 -> 48, 40 46.8 -> 44.2; up to about 32 there is little to compare, and one is enough: 5 42.4, 42.3).
+// share of it: the comparisons, not the gathering, were the time of one work-group (1000 candidates of 152064, a whole call, 185 -> 59 us).  Where the third launch left more
+// than it takes (equal values in reach) up to 32 wanted are found by one work-group.
 __global__ __launch_bounds__(SMP_T) void candidates_rank_kernel(const SampleParams p)
 {
   __shared__ int redi[SMP_T / 64];
-  __shared__ int hist[SMP_BINS];
+  __shared__ float redf[SMP_T / 64];
+  __shared__ alignas(16) int hist[SMP_BINS];
   __shared__ int cnt[SL_MAX], start[SL_MAX];
   __shared__ int sel[2];
   __shared__ int n_gt;
-  __shared__ float cp[RANK_MAX];
-  __shared__ int32_t ct[RANK_MAX];
+  __shared__ uint64_t key[RANK_MAX];
   __shared__ uint16_t mine[RANK_MAX];
   __shared__ int n_own;
   const int tid = threadIdx.x, m = min(p.m, p.n);
   const int own = tid < p.n_slices ? p.st_cnt[tid] : 0;
+  float inv = smp_sum<SMP_T>(tid < p.n_slices ? p.st_sum2[tid] : 0.0f, redf);
+  inv = p.st_sum2[0] < 0.0f ? 1.0f : 1.0f / (inv <= 0.0f ? 1.0f : inv);
   int total;
   const int before = smp_excl_scan<SMP_T>(own, redi, &total);
   if (tid < SL_MAX) { cnt[tid] = own; start[tid] = before; }
   if (tid == 0) n_gt = 0;
   __syncthreads();
   if (total <= RANK_MAX) {
-    for (int s = tid >> 6; s < p.n_slices; s += SMP_T / 64)      // a wave per slice
-      for (int j = tid & 63; j < cnt[s]; j += 64) { cp[start[s] + j] = p.cand_v[s * p.slice + j]; ct[start[s] + j] = p.cand_t[s * p.slice + j]; }
+    for (int e = tid; e < total; e += SMP_T) { const int j = smp_slot(start, e, p.slice); key[e] = smp_key(p.cand_v[j] * inv, p.cand_t[j]); }
   } else {
     // many equal or nearly equal values: the m-th largest exactly, 12 + 12 + 8 bits at a time
     const int slots = p.n_slices * p.slice;
@@ -255,7 +373,7 @@ __global__ __launch_bounds__(SMP_T) void candidates_rank_kernel(const SamplePara
       for (int b = tid; b < SMP_BINS; b += SMP_T) hist[b] = 0;
       __syncthreads();
       for_strided8(p.cand_v, tid, slots, SMP_T, [&](float v, int i) {
-        const uint32_t u = __float_as_uint(v);
+        const uint32_t u = __float_as_uint(v * inv);
         const int s = i / p.slice;
         if (i - s * p.slice < cnt[s] && (u & mask) == prefix) atomicAdd(&hist[(u >> shifts[lvl]) & widths[lvl]], 1);
       });
@@ -268,17 +386,17 @@ __global__ __launch_bounds__(SMP_T) void candidates_rank_kernel(const SamplePara
     // everything above it (any order), then `need` of its copies in token order
     for_strided8(p.cand_v, tid, slots, SMP_T, [&](float v, int i) {
       const int s = i / p.slice;
-      if (i - s * p.slice < cnt[s] && __float_as_uint(v) > prefix) { const int k = atomicAdd(&n_gt, 1); cp[k] = v; ct[k] = p.cand_t[i]; }
+      if (i - s * p.slice < cnt[s] && __float_as_uint(v * inv) > prefix) { const int k = atomicAdd(&n_gt, 1); key[k] = smp_key(v * inv, p.cand_t[i]); }
     });
     __syncthreads();
     const int base = n_gt;                       // = m - need
     const int chunk = (slots + SMP_T - 1) / SMP_T, c0 = tid * chunk, c1 = min(slots, c0 + chunk);
     int ties = 0;
-    for (int i = c0; i < c1; i++) { const int s = i / p.slice; ties += i - s * p.slice < cnt[s] && __float_as_uint(p.cand_v[i]) == prefix; }
+    for (int i = c0; i < c1; i++) { const int s = i / p.slice; ties += i - s * p.slice < cnt[s] && __float_as_uint(p.cand_v[i] * inv) == prefix; }
     int all, rank = smp_excl_scan<SMP_T>(ties, redi, &all);
     for (int i = c0; ties > 0 && rank < need && i < c1; i++) {
       const int s = i / p.slice;
-      if (i - s * p.slice < cnt[s] && __float_as_uint(p.cand_v[i]) == prefix) { cp[base + rank] = p.cand_v[i]; ct[base + rank] = p.cand_t[i]; rank++; }
+      if (i - s * p.slice < cnt[s] && __float_as_uint(p.cand_v[i] * inv) == prefix) { key[base + rank] = smp_key(p.cand_v[i] * inv, p.cand_t[i]); rank++; }
     }
     total = m;
   }
@@ -287,16 +405,12 @@ __global__ __launch_bounds__(SMP_T) void candidates_rank_kernel(const SamplePara
   // lanes rank a value together.
   if (tid == 0) n_own = 0;
   __syncthreads();
-  for (int e = tid; e < total; e += SMP_T) if ((unsigned)ct[e] % gridDim.x == blockIdx.x) mine[atomicAdd(&n_own, 1)] = (uint16_t)e;
+  for (int e = tid; e < total; e += SMP_T) if ((unsigned)smp_token(key[e]) % gridDim.x == blockIdx.x) mine[atomicAdd(&n_own, 1)] = (uint16_t)e;
   __syncthreads();
   for (int o = tid >> 3; o < n_own; o += SMP_T / 8) {
-    const int e = mine[o], t = ct[e];
-    const float v = cp[e];
-    const uint32_t u = __float_as_uint(v);       // (values are not negative, so their bits order like they do; a NaN is the largest and has a rank like any other)
-    int rank = 0;
-    for (int j = tid & 7; j < total; j += 8) { const uint32_t w = __float_as_uint(cp[j]); rank += w > u || (w == u && ct[j] < t); }
-    rank += __shfl_xor(rank, 1); rank += __shfl_xor(rank, 2); rank += __shfl_xor(rank, 4);
-    if ((tid & 7) == 0 && rank < m) { p.tok_out[rank] = t; p.p_out[rank] = v; }
+    const uint64_t k = key[mine[o]];
+    const int rank = smp_rank(key, total, k);
+    if ((tid & 7) == 0 && rank < m) { p.tok_out[rank] = smp_token(k); p.p_out[rank] = smp_value(k); }
   }
 }
 
@@ -311,36 +425,49 @@ int run_candidates(const float* logits_dev, int n, const int32_t* hist_ids, cons
   if (m > n) m = n;
   SampleParams p{};
   p.logits = logits_dev; p.n = n; p.repetition = repetition; p.frequency = frequency; p.presence = presence; p.temperature = temperature; p.m = m;
+  bool penalty = false;              // some token of the history lies in the row and a penalty is set
   if (repetition != 1.0f || frequency != 0.0f || presence != 0.0f)
-    for (int k = 0; k < n_hist && !p.penalty; k++) p.penalty = hist_ids[k] >= 0 && hist_ids[k] < n;
+    for (int k = 0; k < n_hist && !penalty; k++) penalty = hist_ids[k] >= 0 && hist_ids[k] < n;
   // four values per thread of a slice (149 work-groups for a 152k row) until there are 256 slices
   p.slice = std::max(4 * SL_T, ((n + SL_MAX - 1) / SL_MAX + SL_T - 1) / SL_T * SL_T);
   p.n_slices = (n + p.slice - 1) / p.slice;
   const size_t slots = (size_t)p.n_slices * p.slice;
-  int rc = ensure_stage(&c.stage_out, &c.stage_out_cap, (3 * slots + SMP_BINS + 6 * SL_MAX) * 4); if (rc) return rc;
+  int rc = ensure_stage(&c.stage_out, &c.stage_out_cap, (3 * slots + TOP_MAX + 6 * SL_MAX) * 4); if (rc) return rc;
   p.val = (float*)c.stage_out; p.cand_v = p.val + slots; p.cand_t = (int32_t*)(p.cand_v + slots);
-  p.bins = (int*)(p.cand_t + slots);
-  p.st_max = (float*)(p.bins + SMP_BINS); p.st_sum = p.st_max + SL_MAX; p.st_tot = p.st_sum + SL_MAX; p.st_pmax = p.st_tot + SL_MAX;
+  // groups of 64 values of an ordinary slice, or of 16 or 4 where there would not be twice as many of them as are wanted; the values themselves of short rows
+  p.groups = n <= TOP_MAX ? 0 : p.n_slices * 16 >= 2 * m ? 16 : p.n_slices * 64 >= 2 * m ? 64 : 256;
+  p.top = p.groups ? (uint32_t*)(p.cand_t + slots) : (uint32_t*)p.val;
+  p.n_top = p.groups ? p.n_slices * p.groups : n;
+  p.st_max = (float*)((uint32_t*)(p.cand_t + slots) + TOP_MAX); p.st_sum = p.st_max + SL_MAX; p.st_tot = p.st_sum + SL_MAX; p.st_pmax = p.st_tot + SL_MAX;
   p.st_sum2 = p.st_pmax + SL_MAX; p.st_cnt = (int*)(p.st_sum2 + SL_MAX);
   // host side: [tokens 1024 | probabilities 1024 | history ids | history counts]; the last launch writes the first two where they lie
-  const size_t hist = p.penalty ? (size_t)n_hist : 0;
+  const size_t hist = penalty ? (size_t)n_hist : 0;
   if ((rc = ensure_host_stage((2 * (size_t)SMP_MAX_M + 2 * hist) * 4))) return rc;
   int32_t* h = (int32_t*)c.h_stage;
   p.tok_out = h; p.p_out = (float*)(h + SMP_MAX_M);
-  if (p.penalty) {
+  if (hist) {
     if ((rc = ensure_stage(&c.stage_in, &c.stage_in_cap, 2 * hist * 4))) return rc;
     memcpy(h + 2 * SMP_MAX_M, hist_ids, hist * 4); memcpy(h + 2 * SMP_MAX_M + hist, hist_counts, hist * 4);
-    CAI_HIP(hipMemcpyAsync(c.stage_in, h + 2 * SMP_MAX_M, 2 * hist * 4, hipMemcpyHostToDevice, c.stream));
-    p.hist_ids = (const int32_t*)c.stage_in; p.hist_counts = p.hist_ids + hist; p.n_hist = n_hist;
+    p.hist_src = h + 2 * SMP_MAX_M; p.hist_ids = (int32_t*)c.stage_in; p.hist_counts = p.hist_ids + hist; p.n_hist = n_hist;
   }
   const dim3 grid(p.n_slices), block(SL_T);
-  hipLaunchKernelGGL(candidates_stats_kernel, grid, block, 0, c.stream, p);
-  if (p.penalty) hipLaunchKernelGGL(candidates_penalty_kernel, grid, block, 0, c.stream, p);
-  hipLaunchKernelGGL(candidates_value_kernel, grid, block, 0, c.stream, p);
-  hipLaunchKernelGGL(candidates_reach_kernel, grid, block, 0, c.stream, p);
-  hipLaunchKernelGGL(candidates_rank_kernel, dim3(m > 32 ? RANK_WG : 1), dim3(SMP_T), 0, c.stream, p);
-  CAI_HIP(hipGetLastError());
-  CAI_HIP(hipStreamSynchronize(c.stream));
+  hipLaunchKernelGGL(candidates_stats_kernel, dim3(p.n_slices + (2 * hist + HIST_PER - 1) / HIST_PER), block, 0, c.stream, p);
+  if (p.slice <= HELD * SL_T) hipLaunchKernelGGL(candidates_penalty_kernel<true>, grid, block, 0, c.stream, p);
+  else hipLaunchKernelGGL(candidates_penalty_kernel<false>, grid, block, 0, c.stream, p);
+  bool ranked = false;
+  if (m <= SMP_FOLD_M) {
+    p.done = host_signal_next();
+    hipLaunchKernelGGL(candidates_reach_kernel<true>, grid, block, 0, c.stream, p);
+    CAI_HIP(hipGetLastError());
+    if ((rc = host_signal_wait(p.done))) return rc;
+    ranked = h[0] >= 0;
+  } else
+    hipLaunchKernelGGL(candidates_reach_kernel<false>, grid, block, 0, c.stream, p);
+  if (!ranked) {
+    hipLaunchKernelGGL(candidates_rank_kernel, dim3(m > 32 ? RANK_WG : 1), dim3(SMP_T), 0, c.stream, p);
+    CAI_HIP(hipGetLastError());
+    CAI_HIP(hipStreamSynchronize(c.stream));
+  }
   memcpy(tokens_out, h, (size_t)m * 4);
   memcpy(probs_out, h + SMP_MAX_M, (size_t)m * 4);
   if (count_out) *count_out = m;

@@ -116,3 +116,33 @@ def test_a_probability_that_overflows_leaves_the_other_ranks_alone(m):
     assert tok[0] == 4321 and np.isnan(p[0])
     np.testing.assert_array_equal(tok[1:], np.arange(m - 1))
     np.testing.assert_array_equal(p[1:], np.zeros(m - 1))
+
+
+@pytest.mark.parametrize("n,m,n_hist", [(8192, 128, 1025), (8193, 129, 1024), (9000, 1024, 1), (12289, 100, 5000), (33000, 256, 4097), (262145, 128, 2048), (600000, 33, 3000)])
+def test_the_groups_whose_maxima_bound_the_candidates(n, m, n_hist):
+    """rows whose values are binned themselves and rows in groups of 4, 16 and 64; candidates ranked by the third launch's last work-group and by a launch of their own; histories
+    that fill the copying work-groups and go past what the penalties hold in registers; temperatures on both sides of the bounds"""
+    from helpers.device import dev
+    cai = dev()
+    rng = np.random.default_rng(n + m + n_hist)
+    logits = (rng.standard_normal(n) * 3).astype(np.float32)
+    hist = rng.integers(0, n, n_hist).tolist() + [int(np.argmax(logits))] * 2
+    for kw in (dict(), dict(temperature=1500.0), dict(temperature=999.0, history=hist, presence=0.3), dict(temperature=1.3, history=hist, repetition=0.8, frequency=-0.4),
+               dict(history=hist, repetition=1.2, presence=0.5)):
+        check(cai.sample_candidates(logits, m, **kw), O.sample_candidates(logits, m, **kw))
+    # probabilities down to the end of the number range: an exponent is the difference of two products up to 20 / T, rounded on both sides: 4 x 2^-24 x 400
+    got, want = cai.sample_candidates(logits, m, temperature=0.05), O.sample_candidates(logits, m, temperature=0.05)
+    np.testing.assert_allclose(got[1], want[1], rtol=1e-4, atol=1e-30)
+
+
+def test_more_in_reach_than_the_third_launch_ranks():
+    """512 equal values and one more: the former are ranked by the launch that finds them, the latter by the launch behind it; both sides of the bound give token order"""
+    from helpers.device import dev
+    cai = dev()
+    for tied in (511, 512, 513, 3000):
+        logits = np.full(20000, -3.0, np.float32)
+        at = np.sort(np.random.default_rng(tied).permutation(20000)[:tied]); logits[at] = 2.0
+        for m in (1, 7, 128):
+            tok, p = cai.sample_candidates(logits, m)
+            np.testing.assert_array_equal(tok, at[:m]); assert np.all(p == p[0])
+            check(cai.sample_candidates(logits, m, temperature=0.7), O.sample_candidates(logits, m, temperature=0.7))
