@@ -12,12 +12,16 @@
 //     hi + lo and keeps the operands in 64 registers for the whole launch - no activation planes in memory, no LDS traffic
 //     in the product loop, no barrier before the first product;
 //   * a work-group = the waves that together cover the columns (7 waves for 3584) walks 32-row pairs of row sets; per pair
-//     every wave leaves its share in LDS, one barrier, and ONE wave (taking turns) adds the shares in wave order and
-//     finishes the rows: 1/rms of the token (sums of squares exchanged through LDS), bias, residual, or SwiGLU when the two
+//     every wave leaves its share in LDS, and after up to 16 pairs the waves meet and each finishes every n-th pair: adds the shares in wave
+//     order, 1/rms of the token (sums of squares exchanged through LDS), bias, residual, or SwiGLU when the two
 //     row sets of a pair are 16 up rows and their 16 gate rows - written once, as fp32, where the next launch reads them;
 //   * a width of more than 16 super-blocks (the 18944-wide down projection) is cut into column slices = work-groups of
 //     blockIdx.y; the slices' shares meet in a partial buffer and the LAST slice work-group of a row group to arrive (an
 //     arrival counter, as in the attention merge) adds them in slice order with bias and residual.
+// What bounds it: the arithmetic of the operands (two waves a SIMD, 250 instructions an item of 32 rows and a super-block) beside the requests, of which more on their
+// way are slower.  us a launch, 8 tokens, a meeting per pair, addresses by lane and up to three items on their way | this: 7B gate|up 27.4 | 23.0, down 20.1 | 17.5
+// (Q6_K 25.2 | 22.5), q|k|v 12.5 | 11.3, o 9.8 | 8.5, Q6_K head 121 | 106; alone the meetings were 1.2 of gate|up's, a second item on its way cost 2.5, requests past the
+// last item 0.5.
 // Fixed orders everywhere: the result does not depend on timing.
 #include "cai_internal.hpp"
 #include "cai_gemv_common.hpp"
@@ -42,6 +46,7 @@ constexpr int RA_BB = 144;       // bytes of a Q4_K super-block
 constexpr int RA_B6 = 192;       // bytes of a Q6_K record of codes (16 scales and d lie in planes of their own)
 constexpr int RA_PART_BATCH = 8; // slices of an element the last arriver requests at once (times 2 elements, times 2 for SwiGLU)
 constexpr int RA_XLD = RA_SBW * 256 + 8;          // halfs per operand column in LDS (+8: 16 columns x 16-byte reads tile the banks)
+constexpr int RA_PAIRS = 16;      // pairs that a wave leaves its shares of before the waves meet (a KB each, over its operand columns)
 constexpr int RA_WAVE_LDS = 16 * RA_XLD * 2 + 16 * 16 * 2 + RA_SBW * RA_TK * 4 + 192;   // = 17408 bytes per wave
 
 struct RaSeg { const uint8_t* w; const uint8_t* aux; const uint8_t* aux2; const float* bias; int rows; int y_off; int pair_end; };   // pair_end: cumulative 32-row pairs
@@ -115,16 +120,16 @@ __device__ __forceinline__ uint32_t ra_ror8(uint32_t v) { return (uint32_t)__bui
 // (what the first requests need travels as leading scalar arguments, preloaded in scalar registers)
 // Q6_K: see gemm_q6k_nb for which bytes make which group; the operands of group g are columns 16 g + 4 kg .. + 3, in the order 0, 2, 1, 3.
 // HH: 16-row sets per unit of rows (2: pairs - what SwiGLU needs and what long walks take; 1 halves the unit, for products
-// with fewer pairs than compute units or an uneven number per work-group).  GAIN: the activations carry an RMSNorm gain.
+// with fewer pairs than compute units or an uneven number per work-group).  GAIN: the activations carry an RMSNorm gain.  HQ: four tokens, or
+// two times four, are converted (2 sequences of a 7B shape 318 -> 308 us of four layers; as a branch of one kernel eight lost 1 %).
 #define RA_ARGS const float* hsrc, const long long hstride, const float* hgain, const int hcols, const int hntok, const int hnpairs, const int hS
-template <int QT, int HH, bool GAIN>
+template <int QT, int HH, bool GAIN, int HQ>
 __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, const RaParams& p)      // row group bx of n_bx
 {
   // per wave RA_WAVE_LDS bytes: the operand columns [16][RA_XLD] halfs while the activations are converted (each wave converts
   // and reads back only its own columns: no work-group barrier), their sub-block sums [16][16] halfs and 1 / scale [2][8]; once
-  // the operands are in registers the first 2 KB are the wave's shares of the pair in hand: [2 parities][32 lanes][8]
+  // the operands are in registers the first 16 KB are the wave's shares of its pairs: [RA_PAIRS][32 lanes][8]
   extern __shared__ __align__(16) unsigned char ra_dyn[];
-  __shared__ __align__(16) float s_d[RA_NW][2][32];         // d, 32 * dmin per row of the item in hand
   __shared__ float ssq_s[RA_SMAX][RA_TK];
   __shared__ int s_is_last;
   const unsigned long long tl0 = timeline_now();
@@ -135,7 +140,7 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
   const int nwa = (nS + RA_SBW - 1) / RA_SBW;                              // waves of this work-group with columns to cover
   const int nsw = max(0, min(RA_SBW, nS - RA_SBW * wave));                  // super-blocks of this wave
   const int sbw0 = sb0 + min(RA_SBW * wave, nS - 1);                        // its first one (an idle wave re-reads the last)
-  constexpr bool Q6 = QT == CAI_Q6_K, Q8 = QT == CAI_Q8_0, SWAPPED = Q6 || Q8;      // SWAPPED: the activations are the rows of a result
+  constexpr bool Q6 = QT == CAI_Q6_K, Q8 = QT == CAI_Q8_0, Q4 = QT == CAI_Q4_K;
   const int npw = bx < hnpairs ? (hnpairs - bx + n_bx - 1) / n_bx : 0;   // pairs of this work-group
   const int nq = RA_SBW * npw;                                              // (pair, super-block) items of a wave
   const int tok = n & (RA_TK - 1), tokc = min(tok, hntok - 1);
@@ -156,35 +161,38 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
   struct W6 { u32x4_t ql[HH][2], qh[HH], sc[HH]; uint32_t d[HH]; };
   struct W8 { u32x4_t q[HH][4], sc[HH]; };
   using WRegs = std::conditional_t<Q6, W6, std::conditional_t<Q8, W8, W4>>;
-  // weights of item q = (pair q / 2, super-block q % 2 of this wave): for the rows n of both row sets the header and this
-  // lane's 2 x 16 quant bytes.  Loads are never conditional: past the last item the last one is fetched again (a cache hit).
+  // Weights of item q = (pair q / 2, super-block q % 2 of this wave): for the rows n of both row sets the header and this
+  // lane's 2 x 16 quant bytes.  Loads are never under a branch.
+  // A scalar base and an offset that a lane keeps for the whole launch (row sets are whole, so no row is clamped).
+  constexpr int WB = Q6 ? RA_B6 : Q8 ? 256 : RA_BB;
+  uint32_t w_off = (uint32_t)(n * nsb) * WB + 16 * kg, h_off = (uint32_t)(n * nsb) * (Q4 ? WB : 16), d_off = (uint32_t)(n * nsb) * 2;
   auto load_w = [&](int q, WRegs& r) __attribute__((always_inline)) {
+    asm volatile("" : "+v"(w_off), "+v"(h_off), "+v"(d_off));      // (32-bit offsets beside a scalar base: kept as 64-bit sums the addresses were the registers that spilled)
     const int qc = max(min(q, nq - 1), 0);
     const int pair = min(bx + (qc >> 1) * n_bx, hnpairs - 1), sb = sbw0 + min(qc & 1, max(nsw, 1) - 1);
     const RaSeg* sg; int r0, r1; locate(pair, sg, r0, r1);
 #pragma unroll
     for (int hh = 0; hh < HH; hh++) {
-      const int64_t b = (int64_t)min((hh ? r1 : r0) + n, sg->rows - 1) * nsb + sb;   // tail rows: re-read the last row
+      const int64_t b = (int64_t)(hh ? r1 : r0) * nsb + sb;
+      const uint8_t* blk = sg->w + b * WB + w_off;
       if constexpr (Q6) {
-        const uint8_t* blk = sg->w + b * RA_B6;
-        r.ql[hh][0] = *reinterpret_cast<const u32x4_t*>(blk + 16 * kg);
-        r.ql[hh][1] = *reinterpret_cast<const u32x4_t*>(blk + 64 + 16 * kg);
-        r.qh[hh] = *reinterpret_cast<const u32x4_t*>(blk + 128 + 16 * kg);
-        r.sc[hh] = *reinterpret_cast<const u32x4_t*>(sg->aux + b * 16);
-        r.d[hh] = *reinterpret_cast<const uint16_t*>(sg->aux2 + b * 2);
+        r.ql[hh][0] = *reinterpret_cast<const u32x4_t*>(blk);
+        r.ql[hh][1] = *reinterpret_cast<const u32x4_t*>(blk + 64);
+        r.qh[hh] = *reinterpret_cast<const u32x4_t*>(blk + 128);
+        r.sc[hh] = *reinterpret_cast<const u32x4_t*>(sg->aux + b * 16 + h_off);
+        r.d[hh] = *reinterpret_cast<const uint16_t*>(sg->aux2 + b * 2 + d_off);
       } else if constexpr (Q8) {           // 256 codes; the scales of their eight blocks
 #pragma unroll
-        for (int i = 0; i < 4; i++) r.q[hh][i] = *reinterpret_cast<const u32x4_t*>(sg->w + b * 256 + 64 * i + 16 * kg);
-        r.sc[hh] = *reinterpret_cast<const u32x4_t*>(sg->aux + b * 16);
+        for (int i = 0; i < 4; i++) r.q[hh][i] = *reinterpret_cast<const u32x4_t*>(blk + 64 * i);
+        r.sc[hh] = *reinterpret_cast<const u32x4_t*>(sg->aux + b * 16 + h_off);
       } else {
-        const uint8_t* blk = sg->w + b * RA_BB;
-        r.h[hh] = *reinterpret_cast<const uint4*>(blk);
-        r.q[hh][0] = *reinterpret_cast<const uint4*>(blk + 16 + 16 * kg);
-        r.q[hh][1] = *reinterpret_cast<const uint4*>(blk + 80 + 16 * kg);
+        r.h[hh] = *reinterpret_cast<const uint4*>(sg->w + b * WB + h_off);
+        r.q[hh][0] = *reinterpret_cast<const uint4*>(blk + 16);
+        r.q[hh][1] = *reinterpret_cast<const uint4*>(blk + 80);
       }
     }
   };
-  WRegs wa, wb, wc, wd;
+  WRegs wa, wb;
 
   // ---- this wave's activations: 8 tokens x its super-blocks, requested before the first weights ----
   // Requests in memory order: lane (r = lane / 16, i = lane % 16) asks for floats 64 m + 4 i .. + 3 (m = 0..3) of super-block j
@@ -195,11 +203,11 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
   _Float16* sxw = xw + 16 * RA_XLD;                                        // [16 columns][16 sub-blocks]
   float* sinvw = reinterpret_cast<float*>(sxw + 16 * 16);                  // [RA_SBW][8 tokens]
   const int rr = lane >> 4, ii = lane & 15;
-  float4 xr[RA_SBW][2][4];
+  float4 xr[RA_SBW][HQ][4];
 #pragma unroll
   for (int j = 0; j < RA_SBW; j++)
 #pragma unroll
-    for (int hq = 0; hq < 2; hq++) {
+    for (int hq = 0; hq < HQ; hq++) {
       const float* px = hsrc + (int64_t)min(4 * hq + rr, hntok - 1) * hstride + (int64_t)(sbw0 + min(j, max(nsw, 1) - 1)) * 256 + 4 * ii;
 #pragma unroll
       for (int m = 0; m < 4; m++) xr[j][hq][m] = *reinterpret_cast<const float4*>(px + 64 * m);
@@ -219,6 +227,16 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
 #pragma unroll
     for (int hq = 0; hq < 2; hq++) {
       const int t8 = 4 * hq + rr;                 // the row's token
+      if (hq >= HQ) {                              // four absent tokens: zeros
+#pragma unroll
+        for (int m = 0; m < 4; m++) {
+          *reinterpret_cast<uint2*>(xw + t8 * RA_XLD + j * 256 + 64 * m + 4 * ii) = make_uint2(0u, 0u);
+          *reinterpret_cast<uint2*>(xw + (8 + t8) * RA_XLD + j * 256 + 64 * m + 4 * ii) = make_uint2(0u, 0u);
+          if (Q4 && (ii & 7) == 0) sxw[t8 * 16 + j * 8 + 2 * m + (ii >> 3)] = sxw[(8 + t8) * 16 + j * 8 + 2 * m + (ii >> 3)] = (_Float16)0.0f;
+        }
+        if (ii == 0) { sinvw[j * RA_TK + t8] = 0.0f; if (j < nsw) ssq_s[RA_SBW * wave + j][t8] = 0.0f; }
+        continue;
+      }
       float v[4][4];
       float amax = 0.0f, ss = 0.0f;
 #pragma unroll
@@ -244,11 +262,11 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
 #pragma unroll
         for (int u = 0; u < 4; u++) { vs[u] = v[m][u] * s; sm += vs[u]; }
         const half2_t h02 = ra_halves(vs[0], vs[2]), h13 = ra_halves(vs[1], vs[3]);
-        const half2_t l02 = ra_halves(vs[0] - (float)h02.x, vs[2] - (float)h02.y), l13 = ra_halves(vs[1] - (float)h13.x, vs[3] - (float)h13.y);
+        const half2_t l02 = ra_halves(fmaf((float)h02.x, -1.0f, vs[0]), fmaf((float)h02.y, -1.0f, vs[2])), l13 = ra_halves(fmaf((float)h13.x, -1.0f, vs[1]), fmaf((float)h13.y, -1.0f, vs[3]));      // (one v_fma_mix_f32 each)
         *reinterpret_cast<uint2*>(xw + t8 * RA_XLD + j * 256 + 64 * m + 4 * ii) = make_uint2(__builtin_bit_cast(uint32_t, h02), __builtin_bit_cast(uint32_t, h13));
         *reinterpret_cast<uint2*>(xw + (8 + t8) * RA_XLD + j * 256 + 64 * m + 4 * ii) = make_uint2(__builtin_bit_cast(uint32_t, l02), __builtin_bit_cast(uint32_t, l13));
         // sub-block 2 m + i / 8 of the block: the sum of 8 lanes' values, / 32, hi + lo
-        if constexpr (SWAPPED) continue;
+        if constexpr (!Q4) continue;
         sm = ra_oct_sum(sm) * 0.03125f;
         const _Float16 qh = (_Float16)sm, ql = (_Float16)(sm - (float)qh);
         if ((ii & 7) == 0) { sxw[t8 * 16 + j * 8 + 2 * m + (ii >> 3)] = qh; sxw[(8 + t8) * 16 + j * 8 + 2 * m + (ii >> 3)] = ql; }
@@ -260,31 +278,27 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
     }
   __builtin_amdgcn_wave_barrier();    // LDS operations of a wave complete in order: its own columns are there
   // the operands in MFMA order: column n, this lane's 8 k of every step
-  half8_t Bx[Q6 ? 1 : RA_SBW][8]; half4_t Xg[Q6 ? RA_SBW : 1][16]; half2_t bm[RA_SBW]; float sinv[RA_SBW]; float4 sinv4[RA_SBW];
+  half8_t Bx[Q6 ? 1 : RA_SBW][8]; half4_t Xg[Q6 ? RA_SBW : 1][16]; half2_t bm[RA_SBW]; float4 sinv4[RA_SBW];
 #pragma unroll
   for (int j = 0; j < RA_SBW; j++) {
     if constexpr (Q6) {
 #pragma unroll
       for (int gi = 0; gi < 16; gi++) Xg[j][gi] = *reinterpret_cast<const half4_t*>(xw + n * RA_XLD + j * 256 + 16 * gi + 4 * kg);
-      sinv4[j] = *reinterpret_cast<const float4*>(sinvw + j * RA_TK + 4 * c1);      // row 4 kg + i of a result: token (4 kg + i) % 8
     } else if constexpr (Q8) {             // block t: what the exchange of halves below leaves in this lane, weights 16 c1 + 8 g .. + 7
 #pragma unroll
       for (int t = 0; t < 8; t++) Bx[j][t] = *reinterpret_cast<const half8_t*>(xw + n * RA_XLD + j * 256 + 32 * t + 16 * c1 + 8 * g);
-      sinv4[j] = *reinterpret_cast<const float4*>(sinvw + j * RA_TK + 4 * c1);
     } else {
 #pragma unroll
       for (int t = 0; t < 8; t++)
         Bx[j][t] = *reinterpret_cast<const half8_t*>(xw + n * RA_XLD + j * 256 + 64 * g + 16 * c1 + 128 * (t >> 2) + 32 * ((t >> 1) & 1) + 8 * (t & 1));
       bm[j] = *reinterpret_cast<const half2_t*>(sxw + n * 16 + j * 8 + 2 * g + 4 * c1);    // sub-blocks 2 g + 4 c1, + 1
     }
-    sinv[j] = sinvw[j * RA_TK + tok];
+    sinv4[j] = *reinterpret_cast<const float4*>(sinvw + j * RA_TK + 4 * c1);      // row 4 kg + i of a result: token (4 kg + i) % 8
   }
   __builtin_amdgcn_wave_barrier();    // (the region is written again as the wave's shares of a pair)
-  if constexpr (!SWAPPED) load_w(2, wc);
-  timeline_stamp_after(p.timeline, 3, sinv[RA_SBW - 1]);
+  timeline_stamp_after(p.timeline, 3, sinv4[RA_SBW - 1].x);
   timeline_stamp(p.timeline, 4);
-  // what the finishing wave of a pair adds to the rows (bias, residual) is requested when the pair starts: by every wave, so
-  // that the requests stay unconditional (a kilobyte per wave and pair), and from a harmless address when there is none
+  // what a wave adds to the rows of the first pair that it finishes (bias, residual) is requested before the walk; from a harmless address when there is none
   struct Extra { float4 bias[HH], res[HH]; };
   auto prefetch = [&](int i, Extra& f) __attribute__((always_inline)) {
     const int pair = min(bx + min(i, max(npw, 1) - 1) * n_bx, hnpairs - 1);
@@ -298,7 +312,7 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
       f.res[hh] = *reinterpret_cast<const float4*>(rp);
     }
   };
-  Extra ea, eb;
+  Extra ex;
   float acc[HH][4];
   const _Float16 k1024 = (_Float16)1024.0f, kz = (_Float16)0.0f;
   uint32_t kreg = 0x64006400u;                 // 1024.0 twice, kept in a register the compiler cannot fold (see ra_weights)
@@ -331,7 +345,8 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
         }
         const float d = __half2float(__ushort_as_half((unsigned short)r.d[hh]));
         const uint32_t scw[4] = {r.sc[hh].x, r.sc[hh].y, r.sc[hh].z, r.sc[hh].w};
-        float gs[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        float gs[4] = {0.0f, 0.0f, 0.0f, 0.0f}, s_before = 0.0f;
+        float4_t c_before = z4;            // (a result is taken while the next product runs)
 #pragma unroll
         for (int gi = 0; gi < 16; gi++) {
           const int nh = gi >> 3, jq = (gi >> 1) & 3, h = gi & 1;
@@ -342,20 +357,23 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
           const half2_t w02 = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, c, 0x04020400u)) + o2;
           const half2_t w13 = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, c, 0x04030401u)) + o2;
           const half4_t W = {w02.x, w02.y, w13.x, w13.y};
-          const float ds = d * (float)(int)(int8_t)((scw[gi >> 2] >> (8 * (gi & 3))) & 0xffu);
           const float4_t C = __builtin_amdgcn_mfma_f32_16x16x16f16(Xg[j][gi], W, z4, 0, 0, 0);
 #pragma unroll
-          for (int i = 0; i < 4; i++) gs[i] = fmaf(ds, C[i], gs[i]);
+          for (int i = 0; i < 4; i++) gs[i] = gi ? fmaf(s_before, c_before[i], gs[i]) : 0.0f;
+          s_before = (float)(int)(int8_t)((scw[gi >> 2] >> (8 * (gi & 3))) & 0xffu);
+          c_before = C;
         }
-        acc[hh][0] = fmaf(sinv4[j].x, gs[0], acc[hh][0]); acc[hh][1] = fmaf(sinv4[j].y, gs[1], acc[hh][1]);
-        acc[hh][2] = fmaf(sinv4[j].z, gs[2], acc[hh][2]); acc[hh][3] = fmaf(sinv4[j].w, gs[3], acc[hh][3]);
+        const float si[4] = {sinv4[j].x, sinv4[j].y, sinv4[j].z, sinv4[j].w};
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc[hh][i] = fmaf(si[i] * d, fmaf(s_before, c_before[i], gs[i]), acc[hh][i]);
       }
     } else if constexpr (Q8) {
       const float4_t z4 = {0.0f, 0.0f, 0.0f, 0.0f};
       const half2_t o2 = {(_Float16)(-1152.0f), (_Float16)(-1152.0f)};   // 1024 + (code + 128) - 1152
 #pragma unroll
       for (int hh = 0; hh < HH; hh++) {
-        float gs[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        float gs[4] = {0.0f, 0.0f, 0.0f, 0.0f}, s_before = 0.0f;
+        float4_t c_before = z4;            // (a result is taken while the next product runs)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
           // lanes kg 0, 1 asked for block 2 i, kg 2, 3 for block 2 i + 1: the halves change places, and each block is in all four
@@ -372,11 +390,13 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
             const float ds = __half2float(__ushort_as_half((unsigned short)(e ? scw >> 16 : scw & 0xffffu)));
             const float4_t C = __builtin_amdgcn_mfma_f32_16x16x32_f16(Bx[j][2 * i + e], W, z4, 0, 0, 0);
 #pragma unroll
-            for (int k = 0; k < 4; k++) gs[k] = fmaf(ds, C[k], gs[k]);
+            for (int k = 0; k < 4; k++) gs[k] = i + e ? fmaf(s_before, c_before[k], gs[k]) : 0.0f;
+            s_before = ds; c_before = C;
           }
         }
-        acc[hh][0] = fmaf(sinv4[j].x, gs[0], acc[hh][0]); acc[hh][1] = fmaf(sinv4[j].y, gs[1], acc[hh][1]);
-        acc[hh][2] = fmaf(sinv4[j].z, gs[2], acc[hh][2]); acc[hh][3] = fmaf(sinv4[j].w, gs[3], acc[hh][3]);
+        const float si[4] = {sinv4[j].x, sinv4[j].y, sinv4[j].z, sinv4[j].w};
+#pragma unroll
+        for (int k = 0; k < 4; k++) acc[hh][k] = fmaf(si[k], fmaf(s_before, c_before[k], gs[k]), acc[hh][k]);
       }
     } else {
     float4_t C[HH], Cm[HH];
@@ -398,15 +418,10 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
         s2[hh][2 * c] = half2_t{sch.x, sch.x}; s2[hh][2 * c + 1] = half2_t{sch.y, sch.y};
         c2[hh][2 * c] = half2_t{cch.x, cch.x}; c2[hh][2 * c + 1] = half2_t{cch.y, cch.y};
       }
-      if (kg == 0) {
-        const float d = __half2float(__ushort_as_half((unsigned short)(h.x & 0xffffu)));
-        const float dmin = __half2float(__ushort_as_half((unsigned short)(h.x >> 16)));
-        s_d[wave][0][16 * hh + n] = d; s_d[wave][1][16 * hh + n] = dmin * 32.0f;
-      }
       // - dmin * mn * (sum of the sub-block's activations): k = this lane's two sub-blocks, the other six k stay zero
       const half8_t Am = {mnh.x, mnh.y, kz, kz, kz, kz, kz, kz}, Bm = {bm[j].x, bm[j].y, kz, kz, kz, kz, kz, kz};
       const float4_t z4 = {0.0f, 0.0f, 0.0f, 0.0f};
-      Cm[hh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Am, Bm, z4, 0, 0, 0);
+      Cm[hh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Bm, Am, z4, 0, 0, 0);
       C[hh] = z4;
     }
 #pragma unroll
@@ -417,49 +432,40 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
         const uint4& qq = r.q[hh][c];
         const uint32_t d0 = jj ? qq.z : qq.x, d1 = jj ? qq.w : qq.y;
         const half8_t A = nib ? ra_weights<true>(d0, d1, s2[hh][2 * c + 1], c2[hh][2 * c + 1], kreg) : ra_weights<false>(d0, d1, s2[hh][2 * c], c2[hh][2 * c], kreg);
-        C[hh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, Bx[j][t], C[hh], 0, 0, 0);
+        C[hh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Bx[j][t], A, C[hh], 0, 0, 0);
       }
     }
-    __builtin_amdgcn_wave_barrier();   // s_d was written by this wave's own lanes above; LDS operations of a wave complete in order
 #pragma unroll
     for (int hh = 0; hh < HH; hh++) {
-      const float4 d4 = *reinterpret_cast<const float4*>(&s_d[wave][0][16 * hh + 4 * kg]);
-      const float4 m4 = *reinterpret_cast<const float4*>(&s_d[wave][1][16 * hh + 4 * kg]);
-      acc[hh][0] += sinv[j] * (d4.x * C[hh][0] - m4.x * Cm[hh][0]);
-      acc[hh][1] += sinv[j] * (d4.y * C[hh][1] - m4.y * Cm[hh][1]);
-      acc[hh][2] += sinv[j] * (d4.z * C[hh][2] - m4.z * Cm[hh][2]);
-      acc[hh][3] += sinv[j] * (d4.w * C[hh][3] - m4.w * Cm[hh][3]);
+      const uint32_t dd = r.h[hh].x;
+      const float d = __half2float(__ushort_as_half((unsigned short)(dd & 0xffffu))), dmin = __half2float(__ushort_as_half((unsigned short)(dd >> 16))) * 32.0f;
+      const float si[4] = {sinv4[j].x, sinv4[j].y, sinv4[j].z, sinv4[j].w};
+#pragma unroll
+      for (int i = 0; i < 4; i++) acc[hh][i] += si[i] * (d * C[hh][i] - dmin * Cm[hh][i]);
     }
-    __builtin_amdgcn_wave_barrier();
     }
   };
 
-  // ---- end of a pair: every wave leaves its share (column t hi + column 8 + t lo), one wave finishes the rows ----
-  auto pair_end = [&](int i, const Extra& f) __attribute__((always_inline)) {
-    const int slot = i & 1;
-    if (SWAPPED && nsw > 0) {     // result row 4 kg + i = token (4 kg + i) % 8, hi (kg < 2) or lo: they meet across kg ^ 2; column n = weight row n
+  // ---- end of a pair: every wave leaves its share (column t hi + column 8 + t lo) ----
+  auto share = [&](int i) __attribute__((always_inline)) {
+    const int slot = i % RA_PAIRS;
+    if (nsw > 0) {     // result row 4 kg + i = token (4 kg + i) % 8, hi (kg < 2) or lo: they meet across kg ^ 2; column n = weight row n
 #pragma unroll
       for (int hh = 0; hh < HH; hh++)
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-          const float t = acc[hh][k] + __shfl_xor(acc[hh][k], 32, 64);
+          const uint32_t v = __builtin_bit_cast(uint32_t, acc[hh][k]);
+          const uint2_t hl = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+          const uint32_t hi = hl.x, lo = hl.y;      // (of an element in place __builtin_bit_cast takes the first)
+          const float t = __builtin_bit_cast(float, hi) + __builtin_bit_cast(float, lo);
           if (kg < 2) reinterpret_cast<float*>(wl)[(slot * 32 + (n >> 2) * 8 + 4 * kg + k) * 8 + 4 * hh + (n & 3)] = t;
         }
     }
-    if (!SWAPPED && nsw > 0) {
-      float tot[4 * HH];
-#pragma unroll
-      for (int hh = 0; hh < HH; hh++)
-#pragma unroll
-        for (int k = 0; k < 4; k++) tot[4 * hh + k] = acc[hh][k] + ra_ror8(acc[hh][k]);
-      if (!lo_col) {
-        float* dst = reinterpret_cast<float*>(wl) + (slot * 32 + kg * 8 + n) * 8;
-        *reinterpret_cast<float4*>(dst) = make_float4(tot[0], tot[1], tot[2], tot[3]);
-        if constexpr (HH == 2) *reinterpret_cast<float4*>(dst + 4) = make_float4(tot[4], tot[5], tot[6], tot[7]);
-      }
-    }
-    __syncthreads();     // (the slot is written again two pairs on: after the next barrier, which the finishing wave reaches after its reads)
-    if (wave != i % nwa || lo_col) return;
+  };
+  // ---- one wave finishes the rows of a pair ----
+  auto finish = [&](int i, const Extra& f) __attribute__((always_inline)) {
+    const int slot = i % RA_PAIRS;
+    if (lo_col) return;
     float t8[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     for (int w = 0; w < nwa; w++) {       // wave order: fixed
       const float* src = reinterpret_cast<const float*>(ra_dyn + (size_t)w * RA_WAVE_LDS) + (slot * 32 + kg * 8 + n) * 8;
@@ -513,22 +519,22 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
     }
   };
 
-  if constexpr (SWAPPED)       // (two items on their way are what the registers hold)
-    for (int i = 0; i < npw; i++) {
-      prefetch(i, ea);
+  const int nwb = blockDim.x >> 6;
+  for (int i0 = 0; i0 < npw; i0 += RA_PAIRS) {
+    const int i1 = min(npw, i0 + RA_PAIRS);
+    prefetch(i0 + wave, ex);
+    for (int i = i0; i < min(i1, npw - 1); i++) {
       compute(wa, 0); load_w(2 * i + 2, wa);
       compute(wb, 1); load_w(2 * i + 3, wb);
-      pair_end(i, ea);
+      share(i);
     }
-  else for (int q = 0; q < nq; q += 4) {
-    prefetch(q >> 1, ea);
-    load_w(q + 3, wd); compute(wa, 0);
-    load_w(q + 4, wa); compute(wb, 1);
-    if (q == 0 && p.n_slices == 1) timeline_stamp_after(p.timeline, 6, acc[0][0]);
-    pair_end(q >> 1, ea);
-    prefetch((q >> 1) + 1, eb);
-    load_w(q + 5, wb); if (q + 2 < nq) compute(wc, 0);      // (requests stay unconditional)
-    load_w(q + 6, wc); if (q + 2 < nq) { compute(wd, 1); pair_end((q >> 1) + 1, eb); }
+    if (i1 == npw) { compute(wa, 0); compute(wb, 1); share(npw - 1); }
+    __syncthreads();
+    for (int i = i0 + wave; i < i1; i += nwb) {
+      if (i != i0 + wave) prefetch(i, ex);
+      finish(i, ex);
+    }
+    if (i1 < npw) __syncthreads();      // (the slots are written again)
   }
   timeline_stamp(p.timeline, 5);
   if (p.n_slices > 1) {
@@ -579,18 +585,19 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
   timeline_stamp(p.timeline, 7);
 }
 
-template <int QT, int HH, bool GAIN>
+template <int QT, int HH, bool GAIN, int HQ>
 __global__ __launch_bounds__(64 * RA_NW) void gemm_ra(RA_ARGS, const RaParams p)
 {
-  ra_body<QT, HH, GAIN>(hsrc, hstride, hgain, hcols, hntok, hnpairs, hS, blockIdx.x, gridDim.x, p);
+  ra_body<QT, HH, GAIN, HQ>(hsrc, hstride, hgain, hcols, hntok, hnpairs, hS, blockIdx.x, gridDim.x, p);
 }
 // Normed products over the same activations whose matrices are of both types (attn_q and attn_k beside the attn_v of a mixed file): the first
 // hn4 work-groups take the Q4_K rows in pairs of row sets, the others the Q6_K rows.  Both launches by themselves spend most of their time on
 // the activations (7B shape, eight sequences: 11.1 + 11.2 us, 12.9 here).
+template <int HQ>
 __global__ __launch_bounds__(64 * RA_NW) void gemm_ra_two(RA_ARGS, const int hnpairs6, const int hn4, const RaParams p, const RaParams p6)
 {
-  if ((int)blockIdx.x < hn4) ra_body<CAI_Q4_K, 2, true>(hsrc, hstride, hgain, hcols, hntok, hnpairs, hS, blockIdx.x, hn4, p);
-  else ra_body<CAI_Q6_K, 1, true>(hsrc, hstride, hgain, hcols, hntok, hnpairs6, hS, blockIdx.x - hn4, gridDim.x - hn4, p6);
+  if ((int)blockIdx.x < hn4) ra_body<CAI_Q4_K, 2, true, HQ>(hsrc, hstride, hgain, hcols, hntok, hnpairs, hS, blockIdx.x, hn4, p);
+  else ra_body<CAI_Q6_K, 1, true, HQ>(hsrc, hstride, hgain, hcols, hntok, hnpairs6, hS, blockIdx.x - hn4, gridDim.x - hn4, p6);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -704,9 +711,13 @@ static int ra_two(const cai_qw_s* const* ws, const int* y_off, int n_w, int n_to
   const int nsb = (int)(ws[0]->cols >> 8), nw = (nsb + RA_SBW - 1) / RA_SBW, all = units[0] + units[1], slots = std::max(2, ctx().n_cu * (RA_NW / nw));
   const int n4 = all <= slots ? units[0] : std::max(1, std::min(slots - 1, (int)((int64_t)slots * units[0] / all))), n6 = all <= slots ? units[1] : std::max(1, std::min(units[1], slots - n4));
   p[0].timeline = p[1].timeline = timeline_next(n4 + n6);
-  static bool attr_done = false;
-  if (!attr_done) { CAI_HIP(hipFuncSetAttribute((const void*)gemm_ra_two, hipFuncAttributeMaxDynamicSharedMemorySize, RA_NW * RA_WAVE_LDS)); attr_done = true; }
-  hipLaunchKernelGGL(gemm_ra_two, dim3(n4 + n6), dim3(64 * nw), (size_t)nw * RA_WAVE_LDS, ctx().stream, x, (long long)x_stride, gain, (int)ws[0]->cols, n_tok, units[0], nsb, units[1], n4, p[0], p[1]);
+  auto launch = [&](auto kern, bool& attr_done) -> int {
+    if (!attr_done) { CAI_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, RA_NW * RA_WAVE_LDS)); attr_done = true; }
+    hipLaunchKernelGGL(kern, dim3(n4 + n6), dim3(64 * nw), (size_t)nw * RA_WAVE_LDS, ctx().stream, x, (long long)x_stride, gain, (int)ws[0]->cols, n_tok, units[0], nsb, units[1], n4, p[0], p[1]);
+    return CAI_OK;
+  };
+  static bool attr_done[2] = {false, false};
+  if ((rc = n_tok <= 4 ? launch(gemm_ra_two<1>, attr_done[0]) : launch(gemm_ra_two<2>, attr_done[1]))) return rc;
   return CAI_OK;
 }
 
@@ -764,19 +775,21 @@ int ra_gemm(const cai_qw_s* const* ws, const int* y_off, int n_w, int n_tok, con
   p.timeline = timeline_next(gx * n_slices);
   const dim3 grid(gx, n_slices), block(64 * nw);
   const size_t lds = (size_t)nw * RA_WAVE_LDS;
-#define RA_LAUNCH(QTv, HHv, GAINv) do { \
+#define RA_LAUNCH(QTv, HHv, GAINv, HQv) do { \
     static bool attr_done = false; \
-    if (!attr_done) { CAI_HIP(hipFuncSetAttribute((const void*)gemm_ra<QTv, HHv, GAINv>, hipFuncAttributeMaxDynamicSharedMemorySize, RA_NW * RA_WAVE_LDS)); attr_done = true; } \
-    hipLaunchKernelGGL((gemm_ra<QTv, HHv, GAINv>), grid, block, lds, ctx().stream, x, (long long)x_stride, gain, cols, n_tok, units, S, p); } while (0)
-#define RA_TYPE(QTv) do { \
-    if (HH == 2 && gain) RA_LAUNCH(QTv, 2, true); \
-    else if (HH == 2) RA_LAUNCH(QTv, 2, false); \
-    else if (gain) RA_LAUNCH(QTv, 1, true); \
-    else RA_LAUNCH(QTv, 1, false); } while (0)
+    if (!attr_done) { CAI_HIP(hipFuncSetAttribute((const void*)gemm_ra<QTv, HHv, GAINv, HQv>, hipFuncAttributeMaxDynamicSharedMemorySize, RA_NW * RA_WAVE_LDS)); attr_done = true; } \
+    hipLaunchKernelGGL((gemm_ra<QTv, HHv, GAINv, HQv>), grid, block, lds, ctx().stream, x, (long long)x_stride, gain, cols, n_tok, units, S, p); } while (0)
+#define RA_FORM(QTv, HQv) do { \
+    if (HH == 2 && gain) RA_LAUNCH(QTv, 2, true, HQv); \
+    else if (HH == 2) RA_LAUNCH(QTv, 2, false, HQv); \
+    else if (gain) RA_LAUNCH(QTv, 1, true, HQv); \
+    else RA_LAUNCH(QTv, 1, false, HQv); } while (0)
+#define RA_TYPE(QTv) do { if (n_tok <= 4) RA_FORM(QTv, 1); else RA_FORM(QTv, 2); } while (0)
   if (ws[0]->qtype == CAI_Q6_K) RA_TYPE(CAI_Q6_K);
   else if (ws[0]->qtype == CAI_Q8_0) RA_TYPE(CAI_Q8_0);
   else RA_TYPE(CAI_Q4_K);
 #undef RA_TYPE
+#undef RA_FORM
 #undef RA_LAUNCH
   return CAI_OK;
 }

@@ -105,6 +105,25 @@ def test_q4_k_one_launch_small_batch_form_on_awkward_shapes(rows, cols):
     w.close()
 
 
+@pytest.mark.parametrize("qt", [O.Q4_K, O.Q6_K, O.Q8_0])
+@pytest.mark.parametrize("rows", [16 * (16 * 1024 + 1), 32 * (16 * 1024 + 2)])
+def test_one_launch_small_batch_form_over_more_pairs_than_a_meeting(qt, rows):
+    """Work-groups that walk 17 units of rows, one more than they keep the shares of between two meetings of their waves (1024 work-groups at most; units of 16 rows where their
+    number is odd, else of 32), with four tokens converted (2, 4) and eight (5, 8)."""
+    from helpers.device import dev, rel_err
+    cai = dev()
+    cols = 256
+    raw, rng = big_matrix(qt, rows, cols, rows + qt)
+    w = cai.QWeight(qt, rows, cols, raw)
+    x = rng.standard_normal((8, cols)).astype(np.float32)
+    want = O.gemv(qt, raw, rows, cols, x, None, 0, 1)
+    for nb in (2, 4, 5, 8):
+        got = w.gemv(x[:nb])
+        for b in range(nb):
+            assert rel_err(got[b], want[b], floor=0.02 * cols ** 0.5) < TIGHT, (nb, b)
+    w.close()
+
+
 @pytest.mark.parametrize("qt", [O.Q8_0, O.Q4_0])
 @pytest.mark.parametrize("rows,cols", [(18944, 3584), (152064, 3584)])
 def test_q8_0_q4_0_gemv_at_the_large_sweep_shapes(qt, rows, cols):
