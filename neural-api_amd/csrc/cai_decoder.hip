@@ -393,14 +393,22 @@ static int moe_ffn_prompt(cai_decoder_s* d, const cai_decoder_s::Layer& L, int n
   const cai_decoder_config& c = d->cfg;
   const int dm = c.d_model, I = c.ffn, E = c.n_experts, K = c.top_k, slots = n * K;
   int rc;
-  // (the router and the banks read the same normalised rows: one pre-pass where the router takes planes too)
-  const bool shared_prep = prompt_route(L.w[CAI_W_ROUTER], n) == 2;
-  if (shared_prep && (rc = prefill_prep(d->px, dm, L.v[CAI_V_MLP_NORM], c.eps, dm, n))) return rc;
-  if ((rc = linear_rows(L.w[CAI_W_ROUTER], shared_prep, d->px, dm, L.v[CAI_V_MLP_NORM], c.eps, n, d->pm_logits, E, nullptr))) return rc;
-  if ((rc = launch_router_topk(d->pm_logits, E, K, c.norm_topk, n, d->pm_expert, d->pm_gate, d->pm_probs))) return rc;
+  // (the router and the banks read the same normalised rows: one pre-pass where the router takes planes too, and none where its launch leaves them)
+  const bool rows = router_fused_supported(L.w[CAI_W_ROUTER], K) && L.w[CAI_W_ROUTER]->rows == E, shared_prep = !rows && prompt_route(L.w[CAI_W_ROUTER], n) == 2;
+  bool prepped = shared_prep;
+  if (rows) {
+    _Float16 *rhi = nullptr, *rlo = nullptr; float* rsinv = nullptr;
+    prepped = router_rows_planes(L.w[CAI_W_ROUTER]);
+    if (prepped && (rc = prefill_planes_for(n, dm, &rhi, &rlo, &rsinv))) return rc;
+    if ((rc = launch_router_rows(L.w[CAI_W_ROUTER], d->px, dm, L.v[CAI_V_MLP_NORM], c.eps, K, c.norm_topk, n, d->pm_expert, d->pm_gate, rhi, rlo, rsinv))) return rc;
+  } else {
+    if (shared_prep && (rc = prefill_prep(d->px, dm, L.v[CAI_V_MLP_NORM], c.eps, dm, n))) return rc;
+    if ((rc = linear_rows(L.w[CAI_W_ROUTER], shared_prep, d->px, dm, L.v[CAI_V_MLP_NORM], c.eps, n, d->pm_logits, E, nullptr))) return rc;
+    if ((rc = launch_router_topk(d->pm_logits, E, K, c.norm_topk, n, d->pm_expert, d->pm_gate, d->pm_probs))) return rc;
+  }
   if ((rc = launch_moe_group(d->pm_expert, slots, E, d->pm_perm, d->pm_tiles))) return rc;
   const _Float16 *hi, *lo; const float* sinv;
-  if (!shared_prep && (rc = prefill_prep(d->px, dm, L.v[CAI_V_MLP_NORM], c.eps, dm, n))) return rc;
+  if (!prepped && (rc = prefill_prep(d->px, dm, L.v[CAI_V_MLP_NORM], c.eps, dm, n))) return rc;
   prefill_planes(&hi, &lo, &sinv);
   if ((rc = launch_gemm_blk_grouped(L.w[CAI_W_GATEUP], 2 * (int64_t)I, hi, lo, sinv, K, slots, E, d->pm_perm, d->pm_tiles, d->pm_gu, 2 * I))) return rc;
   if ((rc = prefill_prep_swiglu(d->pm_gu, 2 * I, I, slots))) return rc;   // SwiGLU inside the pre-pass of the down projection

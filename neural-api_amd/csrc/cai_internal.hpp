@@ -280,6 +280,10 @@ int noalloc_setup(int device);   // resolves the device address of the fixed scr
 int launch_embed(const cai_qw_s* w, const int32_t* tokens_dev, int n_tokens, float* out);
 int launch_router_topk(const float* logits, int n, int k, int renorm, int n_tokens, int32_t* expert_out, float* gate_out, float* probs_scratch);
 // ... and the router's matrix-vector product, RMSNorm and selection in one launch (Q8_0 router rows, up to 64 experts)
+// ... for a prompt's tokens (router_fused_supported)
+bool router_rows_planes(const cai_qw_s* w);      // ... whether it leaves the normed rows as planes (hi not null)
+int launch_router_rows(const cai_qw_s* w, const float* x, int64_t x_stride, const float* gain, float eps, int k, int renorm, int n_tokens, int32_t* expert_out, float* gate_out,
+                       _Float16* hi, _Float16* lo, float* sinv);
 bool router_in_launch();
 bool router_fused_supported(const cai_qw_s* w, int k);
 int launch_router_fused(const cai_qw_s* w, const float* x, int64_t x_stride, const float* gain, float eps, int k, int renorm, int n_tokens,
@@ -362,6 +366,7 @@ int  launch_blk_planes(const cai_qw_s* w, const float* x, const float* gain, int
 int  launch_gemm_blk_short(const cai_qw_s* const* ws, const int* y_off, int n_w, const BlkPlanes& x, float eps, int n_tok, float* y, int64_t y_stride, const float* residual, int half,
                            const BlkPlanes& out, const float* gain, const KvRows& kv = KvRows());
 void prefill_planes(const _Float16** hi, const _Float16** lo, const float** sinv);   // what the last prefill_prep filled
+int  prefill_planes_for(int n_tok, int K, _Float16** hi, _Float16** lo, float** sinv);
 int  prompt_route(const cai_qw_s* w, int n_tok);   // 0 matrix-vector passes, 1 small-batch kernel, 2 prompt kernel
 bool nb_supported(const cai_qw_s* w);          // 2..8-token matrix-core kernel
 // split pre-pass / product form: prep once, then any number of matrices of that width

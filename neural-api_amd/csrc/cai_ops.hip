@@ -608,6 +608,113 @@ __global__ __launch_bounds__(256) void router_fused_kernel(const float* x, const
   if (lane < k) { expert_out[t * k + lane] = ej; gate_out[t * k + lane] = gj; }
 }
 
+// The same for the tokens of a prompt: a work-group of eight waves per token, a wave every eighth expert, the row in registers (a lane 16 of every 1024 columns, so a router row is
+// one contiguous KB a request), the selection by the first wave from LDS; and, of rows that a wave holds whole, the normed planes that the banks read.
+// What bounds it: round trips and, per token, the router out of the L2 (139 KB of 64 x 2048).  255 tokens of 2048, 64 experts: planes 5.6, product on the matrix cores 8.8 and selection
+// 6.0 us as launches of their own, 11.4 here (8.5 without the planes).  The
+// router's bytes a token stay cheaper than its planes: 2048 tokens, four layers of 32 experts 4440 -> 4380 us, eight of 1536 at width 4096 5730 -> 5560, 1500 of width 512 1575 -> 1482.
+// EPW: experts a wave; U: runs of 1024 columns that a wave holds.
+constexpr int RR_WAVES = 8;
+template <int EPW, int U>
+__global__ __launch_bounds__(64 * RR_WAVES) void router_rows_kernel(const float* x, const long long x_stride, const float* gain, const float eps, const int8_t* wq, const uint16_t* wsc,
+                                                                    const int n, const int cols, const int k, const int renorm, int32_t* expert_out, float* gate_out,
+                                                                    _Float16* hi, _Float16* lo, float* sinv)
+{
+  __shared__ float s_logit[64];
+  const int t = blockIdx.x, lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const float* const xb = x + (int64_t)t * x_stride;
+  const int nblk = cols >> 5;
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+  float acc[EPW], ss = 0.0f;
+  f4 v[U][4], g[U][4];
+#pragma unroll
+  for (int e = 0; e < EPW; e++) acc[e] = 0.0f;
+  for (int b0 = 0; b0 < cols; b0 += 1024 * U) {
+    int c[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      c[u] = min(b0 + 1024 * u + 16 * lane, cols - 16);
+#pragma unroll
+      for (int i = 0; i < 4; i++) { v[u][i] = *reinterpret_cast<const f4*>(xb + c[u] + 4 * i); g[u][i] = *reinterpret_cast<const f4*>(gain + c[u] + 4 * i); }
+    }
+    u4 q[EPW][U]; uint16_t sc[EPW][U];
+#pragma unroll
+    for (int e = 0; e < EPW; e++) {
+      const int r = min(w + RR_WAVES * e, n - 1);       // (past the last expert that one again, not used)
+#pragma unroll
+      for (int u = 0; u < U; u++) { q[e][u] = *reinterpret_cast<const u4*>(wq + (int64_t)r * cols + c[u]); sc[e][u] = wsc[(int64_t)r * nblk + (c[u] >> 5)]; }
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const bool on = b0 + 1024 * u + 16 * lane < cols;
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) { const float xv = on ? v[u][i][j] : 0.0f; ss = fmaf(xv, xv, ss); v[u][i][j] = on ? g[u][i][j] * xv : 0.0f; }
+    }
+#pragma unroll
+    for (int e = 0; e < EPW; e++)
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        float d = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int c4 = (int)q[e][u][i];
+          d = fmaf(v[u][i][0], (float)((c4 << 24) >> 24), d); d = fmaf(v[u][i][1], (float)((c4 << 16) >> 24), d);
+          d = fmaf(v[u][i][2], (float)((c4 << 8) >> 24), d); d = fmaf(v[u][i][3], (float)(c4 >> 24), d);
+        }
+        acc[e] = fmaf(d, __half2float(__ushort_as_half(sc[e][u])), acc[e]);
+      }
+  }
+  const float inv = 1.0f / sqrtf(last_lane(wave_sum(ss)) / (float)cols + eps);
+#pragma unroll
+  for (int e = 0; e < EPW; e++) {
+    const float a = wave_sum(acc[e]) * inv;
+    if (lane == 63) s_logit[w + RR_WAVES * e] = a;
+  }
+  if (hi) {                                             // (cols <= 1024 U) a wave writes an eighth of the row
+    float m = 0.0f;
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) { v[u][i][j] *= inv; m = fmaxf(m, finite_abs(v[u][i][j])); }
+    const int e = plane_exponent(last_lane(wave_max(m)));
+    const float s = ldexpf(1.0f, e);
+    if (threadIdx.x == 0) sinv[t] = ldexpf(1.0f, -e);
+    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        if (w % (4 * U) != 4 * u + i) continue;
+        const int at = 1024 * u + 16 * lane + 4 * i;
+        if (at >= cols || w >= 4 * U) continue;
+        h4 h, l;
+#pragma unroll
+        for (int j = 0; j < 4; j++) { _Float16 a16, b16; split_plane(v[u][i][j] * s, a16, b16); h[j] = a16; l[j] = b16; }
+        *reinterpret_cast<h4*>(hi + (int64_t)t * cols + at) = h; *reinterpret_cast<h4*>(lo + (int64_t)t * cols + at) = l;
+      }
+  }
+  __syncthreads();
+  if (w != 0) return;
+  const float lg = s_logit[min(lane, n - 1)];
+  int ej; float pj, gate;
+  if (k > 20) router_select64(lg, n, k, renorm, lane, ej, gate);
+  else {
+    router_pick64(router_softmax64(lg, n, lane), n, k - 1, lane, ej, pj);
+    gate = pj;
+    if (renorm) {
+      float sum = 0.0f;
+      for (int j = 0; j < k; j++) sum += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, pj), j));
+      gate = sum > 0.0f ? pj * (1.0f / sum) : 0.0f;
+    }
+  }
+  if (lane < k) { expert_out[(int64_t)t * k + lane] = ej; gate_out[(int64_t)t * k + lane] = gate; }
+}
+
 bool router_in_launch()
 {
   static const bool on = []() { const char* e = getenv("CAIHIP_ROUTER_LAUNCHES"); return !(e && e[0] == '1'); }();   // (1: product and selection are launches of their own)
@@ -624,6 +731,23 @@ int launch_router_fused(const cai_qw_s* w, const float* x, int64_t x_stride, con
   if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(gain) | (uintptr_t)(x_stride * 4)) & 15) return set_error(CAI_ERR_INVALID, "router: activation rows and gain must be 16-byte aligned");
   hipLaunchKernelGGL(router_fused_kernel, dim3((unsigned)((w->rows + 3) / 4), n_tokens), dim3(256), 0, ctx().stream, x, (long long)x_stride, gain, eps, (const int8_t*)w->data, (const __half*)w->aux,
                      (int)w->rows, (int)w->cols, k, renorm, logits_out, expert_out, gate_out, probs_scratch, counters);
+  return CAI_OK;
+}
+
+bool router_rows_planes(const cai_qw_s* w) { return w->cols <= 2048; }
+int launch_router_rows(const cai_qw_s* w, const float* x, int64_t x_stride, const float* gain, float eps, int k, int renorm, int n_tokens, int32_t* expert_out, float* gate_out,
+                       _Float16* hi, _Float16* lo, float* sinv)
+{
+  if (!router_fused_supported(w, k) || !gain || (hi && !router_rows_planes(w))) return set_error(CAI_ERR_UNSUPPORTED, "router: the one-launch form takes a Q8_0 router of up to 64 experts with a norm gain");
+  if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(gain) | (uintptr_t)(x_stride * 4)) & 15) return set_error(CAI_ERR_INVALID, "router: activation rows and gain must be 16-byte aligned");
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(n_tokens), dim3(64 * RR_WAVES), 0, ctx().stream, x, (long long)x_stride, gain, eps, (const int8_t*)w->data, (const uint16_t*)w->aux,
+                       (int)w->rows, (int)w->cols, k, renorm, expert_out, gate_out, hi, lo, sinv);
+  };
+  const int epw = ((int)w->rows + RR_WAVES - 1) / RR_WAVES;
+#define RR(E) do { if (w->cols <= 1024) go(router_rows_kernel<E, 1>); else go(router_rows_kernel<E, 2>); } while (0)
+  if (epw == 1) RR(1); else if (epw == 2) RR(2); else if (epw <= 4) RR(4); else RR(8);
+#undef RR
   return CAI_OK;
 }
 

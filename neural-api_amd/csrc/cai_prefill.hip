@@ -787,6 +787,14 @@ int prefill_gemm_swiglu(const cai_qw_s* w, int n_tok, float* y, int64_t y_stride
   const int zero = 0;
   return launch_gemm_q4k_multi(&w, &zero, 1, g_pws.hi, g_pws.lo, g_pws.sxhi, g_pws.sxlo, g_pws.sinv, n_tok, y, y_stride, nullptr, (int)(w->rows / 2));
 }
+// room for the planes of n_tok rows that another launch writes
+int prefill_planes_for(int n_tok, int K, _Float16** hi, _Float16** lo, float** sinv)
+{
+  int rc;
+  if ((rc = prefill_reserve(n_tok, K))) return rc;
+  *hi = g_pws.hi; *lo = g_pws.lo; *sinv = g_pws.sinv;
+  return CAI_OK;
+}
 void prefill_planes(const _Float16** hi, const _Float16** lo, const float** sinv) { *hi = g_pws.hi; *lo = g_pws.lo; *sinv = g_pws.sinv; }
 int prefill_gemm(const cai_qw_s* w, int n_tok, float* y, int64_t y_stride, const float* residual)
 {

@@ -236,6 +236,24 @@ def test_one_token_steps_choose_their_experts(experts, top_k, norm_topk, qtype, 
     dec.close()
 
 
+@pytest.mark.parametrize("experts,top_k,norm_topk,d_model", [(1, 1, 0, 256), (9, 9, 1, 1024), (17, 2, 0, 1056), (64, 21, 1, 2048), (33, 20, 0, 2016), (64, 3, 1, 2080)])
+def test_prompt_tokens_choose_their_experts(experts, top_k, norm_topk, d_model):
+    """The router of a prompt's tokens in one launch, at the edges of what a wave takes (1, 2, 4, 8 experts; one and two runs of 1024 columns, rows that it walks and whose planes another
+    launch makes) and of the selection (every expert; more than twenty): the last row's logits of the oracle."""
+    from helpers.device import dev, rel_err
+    cai = dev()
+    cfg = dict(n_layers=2, d_model=d_model, n_q_heads=4, n_kv_heads=2, head_dim=64, ffn=96, vocab=300, max_ctx=64, eps=1e-5, rope_theta=1e4, n_experts=experts, top_k=top_k, norm_topk=norm_topk)
+    spec = synthetic_spec(cfg, O.Q8_0, std=0.05)
+    om = oracle_model(spec, acc64=1)
+    dec = cai.Decoder(spec)
+    toks = [int(t) for t in np.random.default_rng(experts + d_model).integers(0, 300, 37)]
+    for p, t in enumerate(toks):
+        _, lo = om.step(t, p)
+    _, lg = dec.prefill(toks, 0)
+    assert rel_err(lg, lo) < 1e-3
+    dec.close()
+
+
 @pytest.mark.parametrize("name,n", [("olmoe_like_q8", 11), ("olmoe_like_q8", 45), ("moe_like_q6k", 29)])
 def test_moe_prefill_equals_sequential_steps(name, n):
     """Mixture-of-experts prompts: attention half on the whole chunk, routed half per group of rows (router and top-k once
