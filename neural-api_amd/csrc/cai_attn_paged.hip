@@ -8,7 +8,7 @@
 // and a matrix-core form for prompts, whose key tile is one page.  Scores, soft-max and weights are 32-bit in both; the
 // matrix-core form hands its float weights to the value product as three bfloat16 parts that add up to all 24 bits.
 #include "cai_layered.hpp"
-#include "cai_gemv_common.hpp"
+#include "cai_router.hpp"
 
 #include <algorithm>
 
@@ -17,17 +17,49 @@ namespace cai {
 constexpr int SLICE = 64;                  // keys per work-group of the row form: a slice lies in at most two pages
 
 template <typename T> __device__ __forceinline__ float round_to(float v) { return (float)(T)v; }
-template <typename T> __device__ __forceinline__ void load8(const T* p, float* v)
+// eight elements as they lie, and as floats
+template <typename T> struct Raw8 { u32x4 a; };
+template <> struct Raw8<float> { f32x4 a, c; };
+template <typename T> __device__ __forceinline__ void load8(const T* p, Raw8<T>& r)
+{
+  if constexpr (sizeof(T) == 2) r.a = *reinterpret_cast<const u32x4*>(p);
+  else { r.a = *reinterpret_cast<const f32x4*>(p); r.c = *reinterpret_cast<const f32x4*>(p + 4); }
+}
+template <typename T> __device__ __forceinline__ void floats8(const Raw8<T>& r, float* v)
 {
   if constexpr (sizeof(T) == 2) {
-    const u32x4 u = *reinterpret_cast<const u32x4*>(p);
 #pragma unroll
-    for (int j = 0; j < 4; j++) { v[2 * j] = bf16_lo(u[j]); v[2 * j + 1] = bf16_hi(u[j]); }
+    for (int j = 0; j < 4; j++) { v[2 * j] = bf16_lo(r.a[j]); v[2 * j + 1] = bf16_hi(r.a[j]); }
   } else {
-    const f32x4 a = *reinterpret_cast<const f32x4*>(p), c = *reinterpret_cast<const f32x4*>(p + 4);
 #pragma unroll
-    for (int j = 0; j < 4; j++) { v[j] = a[j]; v[4 + j] = c[j]; }
+    for (int j = 0; j < 4; j++) { v[j] = r.a[j]; v[4 + j] = r.c[j]; }
   }
+}
+// sums in the vector unit (a shuffle goes through the LDS crossbar): of the 16 lanes of a row, in all of them
+__device__ __forceinline__ float row16_total(float v)
+{
+#define STEP(ctrl) v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, 0xf, 0xf, false));
+  STEP(0xb1) STEP(0x4e) STEP(0x141) STEP(0x140)      // lane ^ 1, lane ^ 2, the mirror images within 8 and 16
+#undef STEP
+  return v;
+}
+// ... and of the lanes that agree modulo `apart` (a power of two)
+__device__ __forceinline__ float lanes_apart_total(float v, int apart)
+{
+  typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+  for (int o = apart; o < 8; o <<= 1) v += __shfl_xor(v, o);
+  if (apart <= 8) v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xf, 0xf, false));      // row_ror:8
+  if (apart <= 16) {
+    const u2 t = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
+    const uint32_t a = t.x, b = t.y;                 // (of an element in place __builtin_bit_cast takes the first)
+    v = __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
+  }
+  if (apart <= 32) {
+    const u2 t = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
+    const uint32_t a = t.x, b = t.y;
+    v = __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
+  }
+  return v;
 }
 template <typename T> __device__ __forceinline__ T* kv_page(const KvView& kv, int slot, int key)
 {
@@ -65,33 +97,44 @@ __device__ __forceinline__ float sigmoid_weight(const AttnDims& d, int h, float 
 // A query or key head of `dim` values by one wave, lane holds x[lane + 64 i]: RMS norm (gain null: none) with the factor `inv` or, without
 // whole_norm, one of its own, then the rotation at position pos, then `times`.  The angle is reduced in turns with double precision
 // before sine and cosine.
-__device__ __forceinline__ void head_vector(const float* x, const float* gain, float inv, const float times, const AttnDims& d, int pos, int lane, float* v)
+// HC: 64s of a head.  In two steps: what a head needs, requested without a condition, and the arithmetic.
+template <int HC> struct HeadRequest { float x[HC], o[HC], gx[HC], go[HC]; double turns[HC]; };
+template <int HC> __device__ __forceinline__ void request_head(HeadRequest<HC>& q, const float* x, const float* gain, const AttnDims& d, const float* any, int lane)
+{
+  const int half = d.rot / 2;
+  const float* const gp = gain ? gain : x;                             // (none: any readable values)
+  const double* const tp = half ? d.turns : reinterpret_cast<const double*>(any);
+#pragma unroll
+  for (int i = 0; i < HC; i++) {
+    const int c = min(lane + 64 * i, d.dim - 1), j = c < half ? c : min(max(c - half, 0), max(half - 1, 0)), other = c < half ? c + half : c < d.rot ? c - half : c;
+    q.x[i] = x[c]; q.o[i] = x[other]; q.gx[i] = gp[c]; q.go[i] = gp[other]; q.turns[i] = tp[j];
+  }
+}
+template <int HC> __device__ __forceinline__ void finish_head(const HeadRequest<HC>& q, bool normed, float inv, const float times, const AttnDims& d, int pos, int lane, float* v)
 {
   float s = 0.0f;
 #pragma unroll
-  for (int i = 0; i < 4; i++) { const int c = lane + 64 * i; v[i] = c < d.dim ? x[c] : 0.0f; s = fmaf(v[i], v[i], s); }
-  if (gain) {
+  for (int i = 0; i < HC; i++) { const int c = lane + 64 * i; v[i] = c < d.dim ? q.x[i] : 0.0f; s = fmaf(v[i], v[i], s); }
+  if (normed) {
     s = wave_sum(s);
     if (!d.whole_norm) inv = 1.0f / sqrtf(__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, s), 63)) / (float)d.dim + d.eps);
 #pragma unroll
-    for (int i = 0; i < 4; i++) { const int c = lane + 64 * i; if (c < d.dim) v[i] *= inv * gain[c]; }
+    for (int i = 0; i < HC; i++) { const int c = lane + 64 * i; if (c < d.dim) v[i] *= inv * q.gx[i]; }
   }
   const int half = d.rot / 2;
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
+  for (int i = 0; i < HC; i++) {
     const int c = lane + 64 * i;
     if (c >= d.rot) continue;
-    const bool lo = c < half;
-    const int j = lo ? c : c - half, other = lo ? c + half : j;
-    float o = x[other];
-    if (gain) o *= inv * gain[other];
-    const double t = (double)pos * d.turns[j];
+    float o = q.o[i];
+    if (normed) o *= inv * q.go[i];
+    const double t = (double)pos * q.turns[i];
     float sn, cs;
     sincospif((float)(2.0 * (t - rint(t))), &sn, &cs);
-    v[i] = lo ? v[i] * cs - o * sn : v[i] * cs + o * sn;
+    v[i] = c < half ? v[i] * cs - o * sn : v[i] * cs + o * sn;
   }
 #pragma unroll
-  for (int i = 0; i < 4; i++) v[i] *= times;
+  for (int i = 0; i < HC; i++) v[i] *= times;
 }
 __device__ __forceinline__ float out_gate(const AttnIn& in, int64_t row, int c)
 {
@@ -113,7 +156,9 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(const AttnDims d, const 
     const bool is_q = u < d.heads; const int hh = is_q ? u : u - d.heads;
     const float* gain = is_q ? in.qn : in.kn;
     float v[4];
-    head_vector(p + (is_q ? in.oq : in.ok) + hh * d.dim, gain ? gain + hh * by_head : nullptr, is_q ? f.inv_q : f.inv_k, is_q ? f.temp : 1.0f, d, pos, lane, v);
+    HeadRequest<4> hr;
+    request_head<4>(hr, p + (is_q ? in.oq : in.ok) + hh * d.dim, gain ? gain + hh * by_head : nullptr, d, in.proj, lane);
+    finish_head<4>(hr, gain != nullptr, is_q ? f.inv_q : f.inv_k, is_q ? f.temp : 1.0f, d, pos, lane, v);
     T* dst = is_q ? qbuf + ((int64_t)row * d.heads + hh) * d.dim_p : page + ((int64_t)hh * PAGE_TOKENS + tp) * d.dim_p;
 #pragma unroll
     for (int i = 0; i < 4; i++) { const int c = lane + 64 * i; if (c < d.dim_p) dst[c] = (T)v[i]; }
@@ -130,7 +175,10 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(const AttnDims d, const 
 // run has filled the pages).
 // part (more than one slice): per (row, head, slice) vdim_p weighted sums, the maximum and the normaliser (of a soft-max).
 // ------------------------------------------------------------------------------------------
-template <typename T, int HT, bool SINGLE>
+// NC: 128s of a key or value.  What bounds it: round trips, one after another, so what lies at known places (the heads' numbers of a single row) is requested before the
+// position has arrived, and the slice's values with its keys; sums over lanes stay in the vector unit.  Four rows of 16 / 4 heads of 128 behind 48 to 180 keys 14.7 us a launch as they came to
+// their use, 12.8 requested so, 12.3 with the sums.
+template <typename T, int HT, bool SINGLE, int NC>
 __global__ __launch_bounds__(256) void attn_rows_kernel(const AttnDims d, const KvView kv, const AttnIn in, const StepRows r, const T* qbuf, T* out, const int64_t ldo, float* part)
 {
   __shared__ float sq[HT][256], nk[256], nv[256];
@@ -140,6 +188,15 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(const AttnDims d, const 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hg = d.heads / d.kv_heads, hblk = (hg + HT - 1) / HT;
   const int row = blockIdx.z, g = blockIdx.y / hblk, h0 = g * hg + blockIdx.y % hblk * HT, nh = min(HT, (g + 1) * hg - h0);
+  // a wave's query head, and the new key's, which one wave works out
+  const float* const p = SINGLE ? in.proj + row * in.ldp : nullptr;
+  HeadRequest<2 * NC> rq, rk;
+  const bool gq = SINGLE && in.qn, gk = SINGLE && in.kn;
+  if constexpr (SINGLE) {
+    const int by_head = d.whole_norm ? d.dim : 0, hq = h0 + min(wave, nh - 1), ok = in.ok >= 0 ? in.ok : in.oq;
+    request_head<2 * NC>(rq, p + in.oq + hq * d.dim, gq ? in.qn + hq * by_head : nullptr, d, in.proj, lane);
+    request_head<2 * NC>(rk, p + ok + g * d.dim, gk ? in.kn + g * by_head : nullptr, d, in.proj, lane);
+  }
   const int pos = r.pos[row], slot = r.slot[row];
   const int lo = d.first_key(pos), k0 = lo + blockIdx.x * SLICE, nkeys = min(SLICE, pos + 1 - k0);
   const int n_sl = gridDim.x;
@@ -153,32 +210,45 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(const AttnDims d, const 
   const int l16 = lane & 15, kb = wave * 4 + (lane >> 4);
   const int pk = (k0 / PAGE_TOKENS + 1) * PAGE_TOKENS;                 // first key of the second page
   const T* pg0 = kv_page<T>(kv, slot, k0), *pg1 = kv_page<T>(kv, slot, k0 + nkeys - 1);
-  float kx[4][2][8];
+  Raw8<T> kx[4][NC];
 #pragma unroll
   for (int u = 0; u < 4; u++) {
     const int key = k0 + max(0, min(kb + 16 * u, nkeys - 1 - (own_new ? 1 : 0)));
     const T* kp = (key < pk ? pg0 : pg1) + ((int64_t)g * PAGE_TOKENS + key % PAGE_TOKENS) * d.dim_p;
 #pragma unroll
-    for (int t = 0; t < 2; t++) {
-      if (t && d.dim_p <= 128) continue;
+    for (int t = 0; t < NC; t++) {
       const int c = l16 * 8 + t * 128;
       load8<T>(kp + (c < d.dim_p ? c : 0), kx[u][t]);
     }
   }
-  if (SINGLE) {
-    const float* p = in.proj + row * in.ldp;
-    const RowFactors f = row_factors(d, in, p, pos, own_new, rf);
-    for (int u = wave; u < nh + (own_new ? 1 : 0); u += 4) {
-      float v[4];
-      const bool is_q = u < nh;
-      const int hh = is_q ? h0 + u : g;
-      const float* gain = is_q ? in.qn : in.kn;
-      head_vector(p + (is_q ? in.oq : in.ok) + hh * d.dim, gain && d.whole_norm ? gain + hh * d.dim : gain, is_q ? f.inv_q : f.inv_k, is_q ? f.temp : 1.0f, d, pos, lane, v);
-      float* dst = is_q ? sq[u] : nk;
+  // its values: CB lanes along the columns (eight each), the rest of the work-group along the keys
+  const int chunks = d.vdim_p / 8;
+  int cb_log = 0; while ((1 << cb_log) < chunks) cb_log++;
+  const int cbl = 1 << cb_log, cc = tid & (cbl - 1), kg = tid >> cb_log, nkg = 256 >> cb_log;
+  Raw8<T> vx[4];
+  auto load_values = [&](int kb) {
 #pragma unroll
-      for (int i = 0; i < 4; i++) dst[lane + 64 * i] = is_q ? v[i] : round_to<T>(v[i]);
+    for (int u = 0; u < 4; u++) {
+      const int key = k0 + min(kb + nkg * u, nkeys - 1);
+      load8<T>((key < pk ? pg0 : pg1) + kv.v_off + ((int64_t)g * PAGE_TOKENS + key % PAGE_TOKENS) * d.vdim_p + min(cc, chunks - 1) * 8, vx[u]);
     }
-    if (own_new) for (int c = tid; c < 256; c += 256) nv[c] = c < d.vdim ? round_to<T>(p[in.ov + g * d.vdim + c]) : 0.0f;
+  };
+  load_values(kg);
+  if constexpr (SINGLE) {
+    const float fresh_v = p[in.ok >= 0 ? in.ov + g * d.vdim + min(tid, d.vdim - 1) : in.oq];
+    const RowFactors f = row_factors(d, in, p, pos, own_new, rf);
+    float v[2 * NC];
+    if (wave < nh) {
+      finish_head<2 * NC>(rq, gq, f.inv_q, f.temp, d, pos, lane, v);
+#pragma unroll
+      for (int i = 0; i < 2 * NC; i++) sq[wave][lane + 64 * i] = v[i];
+    }
+    if (own_new && wave == (nh & 3)) {
+      finish_head<2 * NC>(rk, gk, f.inv_k, 1.0f, d, pos, lane, v);
+#pragma unroll
+      for (int i = 0; i < 2 * NC; i++) nk[lane + 64 * i] = round_to<T>(v[i]);
+    }
+    if (own_new) nv[tid] = tid < d.vdim ? round_to<T>(fresh_v) : 0.0f;
   } else {
     for (int i = tid; i < nh * 256; i += 256) {
       const int hh = i >> 8, c = i & 255;
@@ -198,21 +268,22 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(const AttnDims d, const 
     if (hh >= nh) break;
     float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int t = 0; t < 2; t++) {
-      if (t && d.dim_p <= 128) continue;
+    for (int t = 0; t < NC; t++) {
       float q[8];
       *reinterpret_cast<f32x4*>(q) = *reinterpret_cast<const f32x4*>(&sq[hh][l16 * 8 + t * 128]);
       *reinterpret_cast<f32x4*>(q + 4) = *reinterpret_cast<const f32x4*>(&sq[hh][l16 * 8 + t * 128 + 4]);
 #pragma unroll
       for (int u = 0; u < 4; u++) {
         const bool fresh = own_new && kb + 16 * u == nkeys - 1;
+        float kf[8];
+        floats8<T>(kx[u][t], kf);
 #pragma unroll
-        for (int i = 0; i < 8; i++) s[u] = fmaf(q[i], fresh ? nk[l16 * 8 + t * 128 + i] : kx[u][t][i], s[u]);
+        for (int i = 0; i < 8; i++) s[u] = fmaf(q[i], fresh ? nk[l16 * 8 + t * 128 + i] : kf[i], s[u]);
       }
     }
 #pragma unroll
     for (int u = 0; u < 4; u++) {
-      s[u] += __shfl_xor(s[u], 8); s[u] += __shfl_xor(s[u], 4); s[u] += __shfl_xor(s[u], 2); s[u] += __shfl_xor(s[u], 1);
+      s[u] = row16_total(s[u]);
       if (l16 == 0) sc[hh][kb + 16 * u] = s[u] * d.scale;
     }
   }
@@ -231,20 +302,15 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(const AttnDims d, const 
     float v[SLICE / 64], m = -INFINITY;
 #pragma unroll
     for (int i = 0; i < SLICE / 64; i++) { v[i] = lane + 64 * i < nkeys ? sc[hh][lane + 64 * i] : -INFINITY; m = fmaxf(m, v[i]); }
-#pragma unroll
-    for (int o = 32; o; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+    m = last_lane(wave_max(m));
     float s = 0.0f;
 #pragma unroll
     for (int i = 0; i < SLICE / 64; i++) { v[i] = expf(v[i] - m); s += v[i]; sc[hh][lane + 64 * i] = v[i]; }
-#pragma unroll
-    for (int o = 32; o; o >>= 1) s += __shfl_xor(s, o);
+    s = last_lane(wave_sum(s));
     if (lane == 0) { smax[hh] = m; ssum[hh] = d.sink && n_sl == 1 ? s + expf(d.sink[h0 + hh] - m) : s; }
   }
   __syncthreads();
-  // weighted values: CB lanes along the columns (eight each), the rest of the work-group along the keys
-  const int chunks = d.vdim_p / 8;
-  int cb_log = 0; while ((1 << cb_log) < chunks) cb_log++;
-  const int cbl = 1 << cb_log, cc = tid & (cbl - 1), kg = tid >> cb_log, nkg = 256 >> cb_log;
+  // weighted values
   float acc[HT][8];
 #pragma unroll
   for (int hh = 0; hh < HT; hh++)
@@ -252,14 +318,14 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(const AttnDims d, const 
     for (int i = 0; i < 8; i++) acc[hh][i] = 0.0f;
   if (cc < chunks) {
     for (int kb = kg; kb < nkeys; kb += nkg * 4) {
-      float vx[4][8];
+      if (kb != kg) load_values(kb);
+      float vf[4][8];
 #pragma unroll
       for (int u = 0; u < 4; u++) {
-        const int key = k0 + min(kb + nkg * u, nkeys - 1);
-        if (own_new && key == pos) {
+        if (own_new && k0 + min(kb + nkg * u, nkeys - 1) == pos) {
 #pragma unroll
-          for (int i = 0; i < 8; i++) vx[u][i] = nv[cc * 8 + i];
-        } else load8<T>((key < pk ? pg0 : pg1) + kv.v_off + ((int64_t)g * PAGE_TOKENS + key % PAGE_TOKENS) * d.vdim_p + cc * 8, vx[u]);
+          for (int i = 0; i < 8; i++) vf[u][i] = nv[cc * 8 + i];
+        } else floats8<T>(vx[u], vf[u]);
       }
 #pragma unroll
       for (int hh = 0; hh < HT; hh++) {
@@ -267,9 +333,9 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(const AttnDims d, const 
 #pragma unroll
         for (int u = 0; u < 4; u++) {
           const int kk = kb + nkg * u;
-          const float p = kk < nkeys ? sc[hh][kk] : 0.0f;
+          const float w = kk < nkeys ? sc[hh][kk] : 0.0f;
 #pragma unroll
-          for (int i = 0; i < 8; i++) acc[hh][i] = fmaf(p, vx[u][i], acc[hh][i]);
+          for (int i = 0; i < 8; i++) acc[hh][i] = fmaf(w, vf[u][i], acc[hh][i]);
         }
       }
     }
@@ -277,9 +343,8 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(const AttnDims d, const 
 #pragma unroll
   for (int hh = 0; hh < HT; hh++) {
     if (hh >= nh) break;
-    for (int o = cbl; o < 64; o <<= 1)
 #pragma unroll
-      for (int i = 0; i < 8; i++) acc[hh][i] += __shfl_xor(acc[hh][i], o);
+    for (int i = 0; i < 8; i++) acc[hh][i] = lanes_apart_total(acc[hh][i], cbl);
     if (lane < cbl && cc < chunks) {
       *reinterpret_cast<f32x4*>(&red[wave][hh][cc * 8]) = f32x4{acc[hh][0], acc[hh][1], acc[hh][2], acc[hh][3]};
       *reinterpret_cast<f32x4*>(&red[wave][hh][cc * 8 + 4]) = f32x4{acc[hh][4], acc[hh][5], acc[hh][6], acc[hh][7]};
@@ -550,22 +615,23 @@ size_t attn_paged_part_floats(const AttnDims& d, int n_rows)
   return ns > 1 ? std::max(part_row(d, ns), std::min(PART_FLOATS, (size_t)n_rows * part_row(d, ns))) : 0;
 }
 
-template <typename T, int HT>
+template <typename T, int HT, int NC>
 static void run_rows(const AttnDims& d, const KvView& kv, const AttnIn& in, const StepRows& r, const T* qbuf, T* out, int64_t ldo, float* part, bool single)
 {
   const int hg = d.heads / d.kv_heads, ns = n_slices(d, r.reach);
   const dim3 grid(ns, d.kv_heads * ((hg + HT - 1) / HT), r.n_rows);
-  if (single) hipLaunchKernelGGL((attn_rows_kernel<T, HT, true>), grid, dim3(256), 0, ctx().stream, d, kv, in, r, qbuf, out, ldo, part);
-  else hipLaunchKernelGGL((attn_rows_kernel<T, HT, false>), grid, dim3(256), 0, ctx().stream, d, kv, in, r, qbuf, out, ldo, part);
+  if (single) hipLaunchKernelGGL((attn_rows_kernel<T, HT, true, NC>), grid, dim3(256), 0, ctx().stream, d, kv, in, r, qbuf, out, ldo, part);
+  else hipLaunchKernelGGL((attn_rows_kernel<T, HT, false, NC>), grid, dim3(256), 0, ctx().stream, d, kv, in, r, qbuf, out, ldo, part);
   if (ns > 1) hipLaunchKernelGGL(attn_rows_merge_kernel<T>, dim3(d.heads, r.n_rows), dim3(256), 0, ctx().stream, d, in, r, ns, part, out, ldo);
 }
 template <typename T>
 static void run_rows_t(const AttnDims& d, const KvView& kv, const AttnIn& in, const StepRows& r, const void* qbuf, void* out, int64_t ldo, float* part, bool single)
 {
   const int hg = d.heads / d.kv_heads;
-  if (hg == 1) run_rows<T, 1>(d, kv, in, r, (const T*)qbuf, (T*)out, ldo, part, single);
-  else if (hg == 2) run_rows<T, 2>(d, kv, in, r, (const T*)qbuf, (T*)out, ldo, part, single);
-  else run_rows<T, 4>(d, kv, in, r, (const T*)qbuf, (T*)out, ldo, part, single);
+#define ROWS(HT) do { if (d.dim_p <= 128 && d.vdim_p <= 128) run_rows<T, HT, 1>(d, kv, in, r, (const T*)qbuf, (T*)out, ldo, part, single); \
+                      else run_rows<T, HT, 2>(d, kv, in, r, (const T*)qbuf, (T*)out, ldo, part, single); } while (0)
+  if (hg == 1) ROWS(1); else if (hg == 2) ROWS(2); else ROWS(4);
+#undef ROWS
 }
 int attn_paged_rows(const AttnDims& d, const KvView& kv, int act_t, const void* qbuf, const StepRows& r, void* out, int64_t ldo, float* part, size_t part_floats, bool single, const AttnIn& in)
 {

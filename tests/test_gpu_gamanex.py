@@ -240,6 +240,19 @@ def test_wide_layers_in_small_batches(cai, wide, rows, dt):
     dec.close()
 
 
+@DT
+@pytest.mark.parametrize("heads,dim,vdim", [(2, 128, 128), (4, 136, 128), (6, 128, 136), (8, 40, 256), (2, 256, 8)])
+def test_single_tokens_of_heads_at_the_edges_of_a_lane_group(cai, tmp_path, heads, dim, vdim, dt):
+    """one and two runs of 128 columns of a key or a value, one to four query heads of a key head, a layer that reads an earlier layer's keys (its projections hold no key and
+    no value of its own), single tokens in the first slice of keys and past it"""
+    layers = [B.glayer(B.sig(heads=heads, kv_heads=2, dim=dim, vdim=vdim, scale=0.1, kv_from=0 if i else None), 24) for i in range(2)]
+    m = Model(tmp_path, B.gconfig(layers, width=72, vocab=60), seed=heads + dim)
+    t = m.tokens(70, dim + vdim)
+    dec = m.open(cai, 128, 1, dt)
+    check(feed(dec, t, [3, 1, 1, 59, 1, 1, 1, 1, 1, 1]), m.ref(t), dt)
+    dec.close()
+
+
 def test_batches_agree_with_each_request_alone_to_rounding(cai, models):
     m = models["f32"]
     reqs = [m.tokens(n, 60 + n) for n in (21, 90, 2, 1)]
