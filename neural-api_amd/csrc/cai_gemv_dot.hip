@@ -134,7 +134,7 @@ template <> struct DotRegs<CAI_Q5_1> { using type = Q51Regs; };
 
 // PK > 1 packs PK rows into one wave: a wave then holds 16 / PK super-blocks of PK different row-group streams (lane
 // quarter-groups of 64 / PK lanes), so a width that is not a multiple of 4096 columns leaves no lanes idle - 5120 columns
-// are five waves of 4 super-blocks x 4 rows instead of two waves of 16 + 4 super-blocks x 1 row.  The row a lane works on
+// are five waves of 4 super-blocks x 4 rows instead of two waves of 16 + 4 super-blocks x 1 row, 2048 one wave of two rows.  The row a lane works on
 // then differs inside the wave (addresses and group indices are vector values), sums are taken per lane group and the
 // outputs always finish through LDS.
 // The arguments every work-group needs before it can issue its first requests travel as leading scalar kernel arguments:
@@ -817,22 +817,28 @@ int launch_q4k_dot(GemvParams& p, const MultiGemv& m, int swiglu_half, hipStream
   const bool q6k = m.w[0]->qtype == CAI_Q6_K;
   if (q6k && (swiglu_half || m.n != 1)) return CAI_ERR_UNSUPPORTED;
   constexpr int W = 12;   // resident waves per CU
+  int64_t total = 0;
+  for (int i = 0; i < m.n; i++) total += swiglu_half ? swiglu_half : m.rows[i];
   // Rows packed per wave: a width of 17..24 super-blocks, whose second 4096-column slice would be mostly empty (5120 columns:
   // 20 of 32 lane quads at work), is cut into five or six slices of 4 super-blocks instead, four rows to a wave.  Measured
   // on 55296 x 5120: 40.7 -> 32.5 us, 6144 columns 42.9 -> 38.2; widths that fill one wave lose to the exchange through LDS
-  // (2048 columns: 4.2 -> 4.9 us, 3584: 18.1 -> 19.6) and keep one row per wave.
-  constexpr int PKW = 4;
-  const bool packed = !q6k && nsb > 16 && nsb <= 24;
-  if (packed) nsw = (nsb + 16 / PKW - 1) / (16 / PKW);
+  // (3584: 18.1 -> 19.6) and keep one row per wave.
+  // Up to 8 super-blocks a wave of one row has half its lanes (and requests) idle: two or four whole rows to a wave, where there are more rows than
+  // waves (below that a launch is one row a wave either way, and this many work-groups fewer).  us, one row | so: 32000 x 2048 Q3_K 17.4 | 11.7, Q2_K 16.0 | 9.7,
+  // Q4_1 13.6 | 8.9, Q5_1 16.3 | 10.4, Q4_K 11.3 | 7.2, Q4_0 10.4 | 7.0, Q5_K 14.3 | 10.4; 49152 x 1024, four rows: 24.6 | 9.3, 22.5 | 7.9, 19.2 | 7.4, 23.0 | 8.4, 15.3 | 5.8, 13.7 | 5.3,
+  // 19.5 | 7.6 (two: 14.7, 12.9, 11.2, 13.2, 8.9, 8.1, 11.1); 11008 x 2048 Q4_K 5.9 | 4.6; 4096 x 2048 Q3_K 5.0 | 4.5; 2304 to 3000 rows the same.
+  // 9 to 12 super-blocks: three slices of four, four rows, from two turns of that on: 32000 x 2304 Q3_K 17.6 | 15.1, Q4_K 11.4 | 9.5; 8192 x 2560 7.1 | 6.7, 5.2 | 4.7;
+  // 14336 x 3072 9.7 | 9.4, 7.4 | 6.0 (3072 x 3072 Q3_K 5.3 | 5.8; pairs of gate and up rows, a step of six layers Q3_K 306 | 294, Q4_1 267 | 271: one row).
+  const int pkw = q6k ? 1 : nsb > 16 ? (nsb <= 24 ? 4 : 1) : nsb <= 8 && total > (int64_t)c.n_cu * 8 ? (nsb <= 4 ? 4 : 2) : nsb > 8 && nsb <= 12 && !swiglu_half && total >= (int64_t)c.n_cu * 32 ? 4 : 1;
+  const bool packed = pkw > 1;
+  if (packed) nsw = (nsb + 16 / pkw - 1) / (16 / pkw);
   // waves per work-group: short rows (one or two waves span the columns) use ONE work-group of 8 waves per CU - the
   // activation is quantised once per CU instead of once per 4 waves, which outweighs the lower wave count (measured:
   // 3 work-groups of 4 waves 537 tok/s, 1 of 12 waves 544, 1 of 8 waves 561 on the 7B shape); long rows fill the CU
   // with a single work-group of up to 12 waves
   int gwv = nsw >= 3 ? std::max(1, W / nsw) : 8 / nsw;   // the kernel is built for at most 12 waves per work-group
   int gquads = gwv;                                        // waves along the rows
-  if (packed) { gquads = W / nsw; gwv = gquads * PKW; }   // two waves along the rows (one measured 6 % slower)
-  int64_t total = 0;
-  for (int i = 0; i < m.n; i++) total += swiglu_half ? swiglu_half : m.rows[i];
+  if (packed) { gquads = nsw == 1 ? 8 : W / nsw; gwv = gquads * pkw; }   // five or six slices: two waves along the rows (one measured 6 % slower)
   const int waves_per_wg = nsw * gquads;
   const bool stream = raw_block_type(m.w[0]->qtype) && m.w[0]->qtype != CAI_Q5_K;
   const size_t lds = (size_t)((cols + 1023) / 1024 * 1024) * 4 + (stream ? cols / 32 * 4 : 0);   // 16 uint4 per 64 activations; scales of the four-digit form
@@ -903,13 +909,13 @@ int launch_q4k_dot(GemvParams& p, const MultiGemv& m, int swiglu_half, hipStream
         default: pick_stream(std::integral_constant<int, CAI_Q5_1>(), pk); break;
       }
     };
-    if (packed) type(std::integral_constant<int, PKW>()); else type(std::integral_constant<int, 1>());
+    if (pkw == 4) type(std::integral_constant<int, 4>()); else if (pkw == 2) type(std::integral_constant<int, 2>()); else type(std::integral_constant<int, 1>());
     return CAI_OK;
   }
   auto pick = [&](auto ns) {
     constexpr int NSV = decltype(ns)::value;
     if (q6k) go(gemv_q6k_dot<1, NSV>);
-    else if (packed) pick_pk(ns, std::integral_constant<int, PKW>());
+    else if (pkw == 4) pick_pk(ns, std::integral_constant<int, 4>()); else if (pkw == 2) pick_pk(ns, std::integral_constant<int, 2>());
     else pick_pk(ns, std::integral_constant<int, 1>());
   };
   pick(std::integral_constant<int, 2>());   // two row groups per wave: one in flight while one is reduced (three or four, also for the one-row walks alone, measured slower on every shape)

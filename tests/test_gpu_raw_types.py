@@ -409,3 +409,48 @@ def test_prompt_products_of_arbitrary_bytes(qt, cols):
     ok = np.abs(got - want) <= (0.0 if qt in (O.Q3_K, O.Q5_0) else 4e-6) * size
     assert ok.all(), (int((~ok).sum()), float((np.abs(got - want) / size).max()))
     w.close()
+
+
+PACKED = [(2049, 256), (2051, 1024), (2050, 1280), (4099, 2048), (8192, 2304), (8195, 3072), (40001, 512)]
+
+
+@pytest.mark.parametrize("rows,cols", PACKED)
+@pytest.mark.parametrize("qt", [O.Q2_K, O.Q3_K, O.Q4_1, O.Q5_0, O.Q5_1, O.Q4_0, O.Q4_K, O.Q5_K])
+def test_one_token_of_short_rows_that_share_a_wave(qt, rows, cols):
+    """Two and four rows a wave, whole or in three slices: one more row than waves, no whole number of rows a wave, lanes past the width, several turns.
+    The same products as one row a wave makes, to the same bound; and the front half of a feed-forward layer over such rows."""
+    import ctypes as C
+    from helpers.device import dev, rel_err
+    cai = dev()
+    rng = np.random.default_rng(rows + cols + qt)
+    raw = O.quantize(qt, (rng.standard_normal((2 * rows, cols)) * 0.02).astype(np.float32))
+    bias = (rng.standard_normal(2 * rows) * 0.1).astype(np.float32)
+    x = rng.standard_normal((1, cols)).astype(np.float32)
+    want = O.gemv(qt, raw, 2 * rows, cols, x, bias, 0, 1)
+    w = cai.QWeight(qt, rows, cols, raw[:rows * O.row_bytes(qt, cols)], bias[:rows])
+    assert rel_err(w.gemv(x), want[:, :rows], floor=0.02 * cols ** 0.5) < TIGHT
+    w.close()
+    if qt not in (O.Q4_0, O.Q4_K, O.Q5_K):       # (the front half alone takes no other type)
+        return
+    w = cai.QWeight(qt, 2 * rows, cols, raw)
+    gain = (1.0 + 0.2 * rng.standard_normal(cols)).astype(np.float32)
+    h, front, L = np.empty(cols, np.float32), np.empty(rows, np.float32), O.lib()
+    L.orc_rmsnorm(C.c_void_p(x.ctypes.data), C.c_void_p(gain.ctypes.data), cols, C.c_float(1e-6), C.c_void_p(h.ctypes.data))
+    ug = O.gemv(qt, raw, 2 * rows, cols, h, None, 0, 1)[0]
+    L.orc_swiglu(C.c_void_p(ug.ctypes.data), rows, C.c_void_p(front.ctypes.data))
+    # (a product of two sums, each within TIGHT of its scale s = 0.02 sqrt(cols): twice that, over s s)
+    assert rel_err(w.ffn_gateup(x, gain, 1e-6)[0], front, floor=(0.02 * cols ** 0.5) ** 2) < 2 * TIGHT
+    w.close()
+
+
+@pytest.mark.parametrize("qt", [O.Q3_K, O.Q4_K, O.Q5_1])
+def test_decoder_whose_projections_share_waves(qt):
+    from helpers.device import dev, rel_err
+    cai = dev()
+    cfg = dict(n_layers=2, d_model=512, n_q_heads=24, n_kv_heads=6, head_dim=64, ffn=2304, vocab=2500, max_ctx=48, eps=1e-5, rope_theta=1e4)
+    spec = synthetic_spec(cfg, qt, seed=77 + qt, std=0.05)
+    om, dec = oracle_model(spec, acc64=1), cai.Decoder(spec)
+    for p, t in enumerate([3, 2499, 17, 17, 250, 9]):
+        n_o, lo = om.step(t, p); am, ld = dec.step(t, p)
+        assert rel_err(ld[0], lo) < TOL and int(am[0]) == n_o
+    dec.close()
