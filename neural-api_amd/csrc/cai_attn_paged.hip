@@ -35,30 +35,38 @@ template <typename T> __device__ __forceinline__ void floats8(const Raw8<T>& r, 
     for (int j = 0; j < 4; j++) { v[j] = r.a[j]; v[4 + j] = r.c[j]; }
   }
 }
-// sums in the vector unit (a shuffle goes through the LDS crossbar): of the 16 lanes of a row, in all of them
+// Sums in the vector unit (a shuffle goes through the LDS crossbar), in the order of lane ^ 32, 16, 8, 4, 2, 1: lanes half a row apart first, so values that cancel half a head apart
+// do so before anything is added to them.  Of the 16 lanes of a row, in all of them (once lanes 8 apart agree, a rotation by 4 is lane ^ 4, and so on)
 __device__ __forceinline__ float row16_total(float v)
 {
 #define STEP(ctrl) v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, 0xf, 0xf, false));
-  STEP(0xb1) STEP(0x4e) STEP(0x141) STEP(0x140)      // lane ^ 1, lane ^ 2, the mirror images within 8 and 16
+  STEP(0x128) STEP(0x124) STEP(0x122) STEP(0x121)      // row_ror:8, 4, 2, 1
 #undef STEP
   return v;
 }
-// ... and of the lanes that agree modulo `apart` (a power of two)
-__device__ __forceinline__ float lanes_apart_total(float v, int apart)
+__device__ __forceinline__ float rows_16_apart(float v)
 {
   typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+  const u2 t = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
+  const uint32_t a = t.x, b = t.y;                     // (of an element in place __builtin_bit_cast takes the first)
+  return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
+}
+__device__ __forceinline__ float rows_32_apart(float v)
+{
+  typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+  const u2 t = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
+  const uint32_t a = t.x, b = t.y;
+  return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
+}
+// ... of the wave, in all lanes
+__device__ __forceinline__ float wave_total(float v) { return row16_total(rows_16_apart(rows_32_apart(v))); }
+// ... of the lanes that agree modulo `apart` (a power of two), the nearest first
+__device__ __forceinline__ float lanes_apart_total(float v, int apart)
+{
   for (int o = apart; o < 8; o <<= 1) v += __shfl_xor(v, o);
   if (apart <= 8) v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xf, 0xf, false));      // row_ror:8
-  if (apart <= 16) {
-    const u2 t = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
-    const uint32_t a = t.x, b = t.y;                 // (of an element in place __builtin_bit_cast takes the first)
-    v = __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
-  }
-  if (apart <= 32) {
-    const u2 t = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
-    const uint32_t a = t.x, b = t.y;
-    v = __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
-  }
+  if (apart <= 16) v = rows_16_apart(v);
+  if (apart <= 32) v = rows_32_apart(v);
   return v;
 }
 template <typename T> __device__ __forceinline__ T* kv_page(const KvView& kv, int slot, int key)
@@ -306,7 +314,7 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(const AttnDims d, const 
     float s = 0.0f;
 #pragma unroll
     for (int i = 0; i < SLICE / 64; i++) { v[i] = expf(v[i] - m); s += v[i]; sc[hh][lane + 64 * i] = v[i]; }
-    s = last_lane(wave_sum(s));
+    s = wave_total(s);
     if (lane == 0) { smax[hh] = m; ssum[hh] = d.sink && n_sl == 1 ? s + expf(d.sink[h0 + hh] - m) : s; }
   }
   __syncthreads();

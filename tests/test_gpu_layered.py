@@ -370,6 +370,31 @@ def test_repeated_layers(cai, tmp_path, loop):
 
 
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("dim", [128, 136, 256])
+def test_scores_of_single_tokens_add_columns_half_a_row_apart_first(cai, tmp_path, dim, dt):
+    """Keys whose 2^25 and -2^25 lie 64 columns apart, beside two ones 8 columns behind each: a score of 2 (the oracle's) where these are the first that meet, of 0 where neighbouring
+    groups of eight do, since 2^25 + 1 has no place in 32 bits.  Token 1's key is the negative of the others'."""
+    cfg = B.config([B.layer((B.attn(heads=2, kv_heads=1, dim=dim, vdim=24, window=64, scale=1.0), B.delta()), ff=None)], width=64, vocab=40)
+
+    def edit(w):
+        w["embed"][:, 0] = 4.0; w["embed"][1::2, 0] = -4.0; w["embed"][:, 1] = 4.0
+        w["l0.norm1.alpha"] = np.asarray(8.0); w["l0.norm1"][:2] = 1.0; w["l0.norm1.b"][:2] = 0.0        # tanh(32) = 1 in 32 bits
+        p = "l0.mix.left."
+        for n, col in (("q", 1), ("k", 0)):
+            w[p + n][:] = 0.0; w[p + n][:, col] = 1.0
+        w[p + "q.norm"][:] = 1.0; w[p + "k.norm"][:] = 0.0
+        w[p + "k.norm"][[0, 64, 8, 72]] = [2.0 ** 25, -2.0 ** 25, 1.0, 1.0]
+    m = Model(tmp_path, cfg, seed=dim, edit=edit)
+    t = [1 + i % 2 for i in range(24)]
+    want, flat = m.ref(t), {n: a.copy() for n, a in m.w.items()}
+    flat["l0.mix.left.k.norm"][[8, 72]] = 0.0
+    assert err(R.forward(cfg, flat, np.array(t))[4:], want[4:]) > 0.1           # (scores of 0 are seen)
+    dec = m.open(cai, 64, 1, dt)
+    check(feed(dec, t, [1]), want, dt)
+    dec.close()
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
 def test_a_window_wider_than_the_pool(cai, tmp_path, dt):
     m = Model(tmp_path, B.config([B.layer((B.attn(heads=3, kv_heads=1, dim=40, vdim=72, window=1 << 29), B.delta()))]), seed=6)
     tok = m.tokens(384, 2)
