@@ -156,36 +156,12 @@ __device__ __forceinline__ float lane_value(float v, int lane) { return __builti
 __device__ __forceinline__ void part_store(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ float part_load(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
-// Hand-over of the partial results.  The form built by default relies on what gfx942 / gfx950 do, not on the language's
-// memory model: the partials are stored with agent-scope atomic stores (written through to memory, bypassing the
-// non-coherent caches), vmcnt(0) returns only when those stores have been acknowledged, the work-group barrier orders every
-// wave's acknowledgement before thread 0's agent-scope increment, and the last arriver reads with agent-scope atomic loads
-// issued after the barrier that publishes s_is_last (atomic loads are not moved above it by the compiler).  It breaks if
-// the partials are accessed with ordinary loads or stores, or on a target where an acknowledged agent-scope store may still
-// be invisible to another compute unit.  -DCAI_MERGE_RELACQ builds the form the memory model guarantees (release increment,
-// acquire fence in the last arriver); it writes back and invalidates the L2 of the XCD on every hand-over and takes the
-// 7B batch-1 step from 1.52 to 1.60 ms.
-#if defined(__HIP_DEVICE_COMPILE__) && !defined(CAI_MERGE_RELACQ) && !defined(__gfx950__) && !defined(__gfx942__)
-#error "merge_if_last: the relaxed hand-over is only valid on gfx942 / gfx950; build with -DCAI_MERGE_RELACQ"
-#endif
-// head qh of sequence `seq`; every thread of the work-group calls it after its partial stores
+// The slices of head qh of sequence `seq`; every thread of the work-group calls it after its partial stores
 __device__ __forceinline__ void merge_if_last(const AttnParams& p, int seq, int qh, int s_first, int n_active, int counter)
 {
-  __shared__ int s_is_last;
-  __builtin_amdgcn_s_waitcnt(0x0F70);           // vmcnt(0): this thread's partial stores have been acknowledged
-  __syncthreads();
-  if (threadIdx.x == 0)
-#ifdef CAI_MERGE_RELACQ
-    s_is_last = __builtin_amdgcn_atomic_inc32(p.merge_cnt + counter, (unsigned)n_active - 1, __ATOMIC_RELEASE, "agent") == (unsigned)n_active - 1;
-#else
-    s_is_last = __builtin_amdgcn_atomic_inc32(p.merge_cnt + counter, (unsigned)n_active - 1, __ATOMIC_RELAXED, "agent") == (unsigned)n_active - 1;
-#endif
-  __syncthreads();
+  const bool last = arrives_last(p.merge_cnt + counter, (unsigned)n_active);
   timeline_stamp(p.timeline, 6);
-  if (!s_is_last) return;
-#ifdef CAI_MERGE_RELACQ
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-#endif
+  if (!last) return;
   // One round trip per MB slices: every thread requests its value of each slice, lane u of every wave the maximum and the sum of slice u.  The
   // slices are folded in order with a running maximum; what that scales by depends on the maxima alone, so lane u works it out for slice u
   // and the fold reads it from there (every thread by itself, two exponentials a slice: half a microsecond at ten slices).

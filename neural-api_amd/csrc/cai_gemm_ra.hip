@@ -131,7 +131,6 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
   // the operands are in registers the first 16 KB are the wave's shares of its pairs: [RA_PAIRS][32 lanes][8]
   extern __shared__ __align__(16) unsigned char ra_dyn[];
   __shared__ float ssq_s[RA_SMAX][RA_TK];
-  __shared__ int s_is_last;
   const unsigned long long tl0 = timeline_now();
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 15, kg = lane >> 4, g = kg >> 1, c1 = kg & 1;
@@ -538,15 +537,10 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
   }
   timeline_stamp(p.timeline, 5);
   if (p.n_slices > 1) {
-    // the slices of a row group meet: shares stored with agent-scope stores and acknowledged (vmcnt(0)) before the barrier and
-    // the work-group's arrival; the last arriver reads them with agent-scope loads, in slice order
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-    if (threadIdx.x == 0)
-      s_is_last = __builtin_amdgcn_atomic_inc32(p.counters + bx, (unsigned)p.n_slices - 1, __ATOMIC_RELAXED, "agent") == (unsigned)p.n_slices - 1;
-    __syncthreads();
+    // the slices of a row group meet (shares stored and read at agent scope); the last to arrive adds them in slice order
+    const bool last = arrives_last(p.counters + bx, (unsigned)p.n_slices);
     timeline_stamp(p.timeline, 6);
-    if (!s_is_last) { timeline_stamp(p.timeline, 7); return; }
+    if (!last) { timeline_stamp(p.timeline, 7); return; }
     // the elements EB at a time: all slices' shares of a batch of elements (and their bias and residual) are requested before
     // the first addition; the additions run in slice order
     const int rpu = 16 * HH;                                  // rows per unit

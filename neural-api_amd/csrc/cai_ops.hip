@@ -547,18 +547,13 @@ int launch_router_topk(const float* logits, int n, int k, int renorm, int n_toke
 // the rows measured slower than the two launches it replaced: a single CU streams the 128 KB of a 64 x 2048 router at about
 // 20 GB/s).  Every wave sums the squares of the row itself (no meeting before the products), takes one Q8_0 router row (a lane
 // four of every 256 columns: with a block of 32 to a lane each request touched 64 lines, 9.6 us a launch of 64 x 2048, 8.7 here; the factor 1 / rms multiplies the finished sum) and stores its logit at agent scope; the
-// work-group that arrives last (wrapping counter per token, the hand-over of the attention merge: agent-scope stores
-// acknowledged under vmcnt(0), work-group barrier, agent-scope increment, agent-scope loads) selects (router_select64).  Takes the
+// work-group that arrives last (arrives_last, a counter per token) selects (router_select64).  Takes the
 // place of the matrix-vector launch and the selection launch of a decode step (TNNetPointwiseSoftMax + TNNetTopKGate behind the
 // router's TNNetPointwiseConvLinear, neural/neuralpretrained.pas:15331-15348).
-#if defined(__HIP_DEVICE_COMPILE__) && !defined(CAI_MERGE_RELACQ) && !defined(__gfx950__) && !defined(__gfx942__)
-#error "router_fused_kernel: the relaxed hand-over is only valid on gfx942 / gfx950; build with -DCAI_MERGE_RELACQ"
-#endif
 __global__ __launch_bounds__(256) void router_fused_kernel(const float* x, const long long x_stride, const float* gain, const float eps,
                                                            const int8_t* wq, const __half* wsc, const int n, const int cols, const int k, const int renorm,
                                                            float* logits_out, int32_t* expert_out, float* gate_out, float* probs, unsigned* counters)
 {
-  __shared__ int s_is_last;
   const int t = blockIdx.y, tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int r_own = blockIdx.x * 4 + w, r = min(r_own, n - 1);
   const float* xb = x + (int64_t)t * x_stride;
@@ -588,19 +583,7 @@ __global__ __launch_bounds__(256) void router_fused_kernel(const float* x, const
   ss = last_lane(wave_sum(ss)); acc = last_lane(wave_sum(acc));
   const float logit = acc * (1.0f / sqrtf(ss / (float)cols + eps));
   if (lane == 0 && r_own < n) __hip_atomic_store(logits_out + (int64_t)t * n + r_own, logit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __builtin_amdgcn_s_waitcnt(0x0F70);           // vmcnt(0): the logit store has been acknowledged
-  __syncthreads();
-  if (tid == 0)
-#ifdef CAI_MERGE_RELACQ
-    s_is_last = __builtin_amdgcn_atomic_inc32(counters + t, gridDim.x - 1, __ATOMIC_RELEASE, "agent") == gridDim.x - 1;
-#else
-    s_is_last = __builtin_amdgcn_atomic_inc32(counters + t, gridDim.x - 1, __ATOMIC_RELAXED, "agent") == gridDim.x - 1;
-#endif
-  __syncthreads();
-  if (!s_is_last || w != 0) return;
-#ifdef CAI_MERGE_RELACQ
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-#endif
+  if (!arrives_last(counters + t, gridDim.x) || w != 0) return;
   const float lg = __hip_atomic_load(logits_out + (int64_t)t * n + min(lane, n - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   int ej; float gj;
   const float pr = router_select64(lg, n, k, renorm, lane, ej, gj);

@@ -238,7 +238,7 @@ __global__ __launch_bounds__(SL_T) void candidates_penalty_kernel(const SamplePa
 }
 
 // Last values: the probabilities, or with a temperature exp(ln(max(p, 1e-30)) / T - ln(max p) / T) still to be divided by its sum.  The slice's values that
-// can be among the m largest are kept in token order.  FOLDED: the work-group that arrives last ranks them (the hand-over of the attention's merge) and
+// can be among the m largest are kept in token order.  FOLDED: the work-group that arrives last ranks them and
 // leaves them to the host, or a token of -1 if they are more than it takes; a launch less, and the host reads the flag before the end of the stream.
 constexpr int FOLD_MAX = 512;
 template <typename T> __device__ __forceinline__ void part_put(T* q, T v) { __hip_atomic_store(q, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
@@ -306,14 +306,9 @@ __global__ __launch_bounds__(SL_T) void candidates_reach_kernel(const SamplePara
     if (__float_as_uint(t) >= floor_bits) { put(p.cand_v + i0 + at, last(t)); put(p.cand_t + i0 + at, (int32_t)(j0 + k)); at++; }
   }
   if constexpr (FOLDED) {
-    __shared__ int s_is_last;
     __shared__ int start[SL_MAX];
     __shared__ uint64_t key[FOLD_MAX], place[SMP_FOLD_M];
-    __builtin_amdgcn_s_waitcnt(0x0F70);          // vmcnt(0): this thread's values have been acknowledged
-    __syncthreads();
-    if (g == 0) s_is_last = __builtin_amdgcn_atomic_inc32(p.done.arrive, gridDim.x - 1, __ATOMIC_RELAXED, "agent") == gridDim.x - 1;
-    __syncthreads();
-    if (!s_is_last) return;
+    if (!arrives_last(p.done.arrive, gridDim.x)) return;
     const int m = min(p.m, p.n), own = g < p.n_slices ? part_get(p.st_cnt + g) : 0;
     float inv = smp_sum<SL_T>(g < p.n_slices ? part_get(p.st_sum2 + g) : 0.0f, red);
     inv = !warm ? 1.0f : 1.0f / (inv <= 0.0f ? 1.0f : inv);
