@@ -237,9 +237,38 @@ __global__ __launch_bounds__(SL_T) void candidates_penalty_kernel(const SamplePa
   if (tid % of == 0) p.top[blockIdx.x * p.groups + tid / of] = own;
 }
 
+// The last step of a probability v of a row with the sum tot (0: it is 1) and the largest probability of logarithm lm: itself, or warmed or cooled and still to be
+// divided by the row's sum.
+__host__ __device__ inline float smp_last(float v, float tot, bool warm, float lm, float inv_t)
+{
+  if (tot > 0.0f) v = v / tot;
+  return warm ? expf(logf(fmaxf(v, 1e-30f)) * inv_t - lm * inv_t) : v;
+}
+__host__ __device__ inline float smp_bits_float(uint32_t u) { return __builtin_bit_cast(float, u); }
+// The bits from which on a probability is in reach of the m largest, where the m-th largest of the groups' maxima lies in `bin` (its leading 12 bits).
+// The steps after the maxima keep the order but can make neighbours equal, and equal ones go by token.  A quotient rounds two steps of its dividend together at
+// most: four steps below the bin are still in reach.  With a temperature a whole bin is, 6 % of the value at least: 0.06 / T of the exponent, whose own
+// errors are 3e-5 / T (of logarithms up to 69) and 1e-6.  Everything is (0) where the row has no finite sum, where what lies below would meet the logarithm's floor, and where the m-th
+// value itself, divided by the row's sum, would have lost bits to the end of the number range (what is smaller may: it stays smaller).  That sum is at most n, and up to T = 1 at
+// most 1 / (the largest probability), since (v / top)^(1 / T) <= v / top.  Of 152064 values at T = 0.1 this reaches to an m-th value 9 nats below the first (a call 26 us; with everything in
+// reach 350).
+__host__ __device__ inline uint32_t smp_reach_floor(int bin, bool warm, float tot, float pm, float lm, float inv_t, float temperature, int n, bool divided)
+{
+  const uint32_t at = (uint32_t)bin << 20, slack = warm ? 1u << 20 : 4u, low = at < slack ? 0u : at - slack;
+  const float quotient = tot > 0.0f ? smp_bits_float(low) / tot : smp_bits_float(low);
+  bool clear;
+  if (warm) {
+    const float sum = temperature < 1.0f ? fminf((float)n, 1.0f / pm) : (float)n;
+    clear = tot < 3.0e38f && quotient > 1.0e-30f && temperature < 1000.0f && smp_last(smp_bits_float(at), tot, warm, lm, inv_t) > 1.0e-40f * sum;
+  } else
+    clear = !divided || quotient > 1.2e-38f;
+  return clear ? low : 0u;
+}
+
 // Last values: the probabilities, or with a temperature exp(ln(max(p, 1e-30)) / T - ln(max p) / T) still to be divided by its sum.  The slice's values that
 // can be among the m largest are kept in token order.  FOLDED: the work-group that arrives last ranks them and
-// leaves them to the host, or a token of -1 if they are more than it takes; a launch less, and the host reads the flag before the end of the stream.
+// leaves them to the host, or a token of -1 if they are more than it takes; a launch less, and the host reads the flag before the end of the stream.  Where all values of a
+// row are in reach every work-group knows that they are too many: nothing is handed over, and the first one tells the host at once.
 constexpr int FOLD_MAX = 512;
 template <typename T> __device__ __forceinline__ void part_put(T* q, T v) { __hip_atomic_store(q, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 template <typename T> __device__ __forceinline__ T part_get(const T* q) { return __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
@@ -277,20 +306,14 @@ __global__ __launch_bounds__(SL_T) void candidates_reach_kernel(const SamplePara
   }
   const bool warm = p.temperature != 1.0f && pm > 0.0f;
   const float lm = logf(fmaxf(pm, 1e-30f)), inv_t = 1.0f / fmaxf(p.temperature, 1e-6f);
-  auto last = [&](float v) {
-    if (tot > 0.0f) v = v / tot;
-    return warm ? expf(logf(fmaxf(v, 1e-30f)) * inv_t - lm * inv_t) : v;
-  };
+  auto last = [&](float v) { return smp_last(v, tot, warm, lm, inv_t); };
   smp_crossing<SL_T>(bins, min(p.m, p.n), redi, sel);      // (behind the barriers of the sums)
-  // The steps after the maxima keep the order but can make neighbours equal, and equal ones go by token.  A quotient rounds two steps of its dividend together at
-  // most: four steps below the bin are still in reach.  With a temperature a whole bin is, 6 % of the value at least: 0.06 / T of the exponent, whose own
-  // errors are 3e-5 / T (of logarithms up to 69) and 1e-6.  Where values lose bits to the end of the number range, meet the logarithm's floor or have no finite sum, everything is.
-  uint32_t floor_bits = (uint32_t)sel[0] << 20;
-  const uint32_t slack = warm ? 1u << 20 : 4u;
-  floor_bits = floor_bits < slack ? 0u : floor_bits - slack;
-  const float low = __uint_as_float(floor_bits), lowest = last(low);
-  const bool clear = warm ? tot < 3.0e38f && (tot > 0.0f ? low / tot : low) > 1.0e-29f && lowest > 1.0e-35f * (float)p.n && p.temperature < 1000.0f : lowest > 1.0e-36f;
-  if (!clear) floor_bits = 0u;
+  const uint32_t floor_bits = smp_reach_floor(sel[0], warm, tot, pm, lm, inv_t, p.temperature, p.n, p.n_hist > 0);
+  const bool whole = FOLDED && floor_bits == 0u && p.n > FOLD_MAX;
+  if (whole && blockIdx.x == 0) {
+    if (g == 0) host_store(p.tok_out, (int32_t)-1);
+    host_signal(p.done, 1);
+  }
   int mine = 0, total;
   float sum2 = 0.0f;
 #pragma unroll
@@ -299,7 +322,7 @@ __global__ __launch_bounds__(SL_T) void candidates_reach_kernel(const SamplePara
   sum2 = smp_sum<SL_T>(sum2, red);
   int at = smp_excl_scan<SL_T>(mine, redi, &total);
   if (!warm) sum2 = -1.0f;                       // (< 0: nothing to divide by)
-  auto put = [](auto* q, auto v) { if constexpr (FOLDED) part_put(q, v); else *q = v; };
+  auto put = [&](auto* q, auto v) { if (FOLDED && !whole) part_put(q, v); else *q = v; };
   if (g == 0) { put(p.st_sum2 + blockIdx.x, sum2); put(p.st_cnt + blockIdx.x, total); }
   for (int k = 0; mine > 0 && k < per && j0 + k < p.n; k++) {
     const float t = p.val[j0 + k];
@@ -308,7 +331,7 @@ __global__ __launch_bounds__(SL_T) void candidates_reach_kernel(const SamplePara
   if constexpr (FOLDED) {
     __shared__ int start[SL_MAX];
     __shared__ uint64_t key[FOLD_MAX], place[SMP_FOLD_M];
-    if (!arrives_last(p.done.arrive, gridDim.x)) return;
+    if (whole || !arrives_last(p.done.arrive, gridDim.x)) return;
     const int m = min(p.m, p.n), own = g < p.n_slices ? part_get(p.st_cnt + g) : 0;
     float inv = smp_sum<SL_T>(g < p.n_slices ? part_get(p.st_sum2 + g) : 0.0f, red);
     inv = !warm ? 1.0f : 1.0f / (inv <= 0.0f ? 1.0f : inv);
@@ -472,6 +495,16 @@ int run_candidates(const float* logits_dev, int n, const int32_t* hist_ids, cons
 }  // namespace cai
 
 using namespace cai;
+
+// For the tests of the rule; host only, not part of the interface in caihip.h: the bits from which on values are in reach (0: all), in a row whose largest probability is pm and whose
+// values are, with a history, probabilities times tot.
+extern "C" int cai_candidates_floor(int bin, float tot, float pm, float temperature, int n, int divided)
+{
+  CAI_ENTER();
+  CAI_REQUIRE(bin >= 0 && bin < SMP_BINS && n >= 1, "cai_candidates_floor: bad argument");
+  const bool warm = temperature != 1.0f && pm > 0.0f;
+  return (int)smp_reach_floor(bin, warm, tot, pm, logf(fmaxf(pm, 1e-30f)), 1.0f / fmaxf(temperature, 1e-6f), temperature, n, divided != 0);
+}
 
 extern "C" int cai_sample_candidates(const float* logits, int n, const int32_t* hist_ids, const int32_t* hist_counts, int n_hist,
                                      float repetition, float frequency, float presence, float temperature, int m,
