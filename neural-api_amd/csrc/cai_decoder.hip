@@ -89,6 +89,24 @@ static int check_ready(cai_decoder_s* d)
 }
 
 
+// How a block of a mixture gets from its rows to their experts.
+// Steps (up to 8 rows): for one token the gate|up launch chooses the experts (every work-group its slot's) from logits that an ordinary product leaves.  For several the selection
+// in the router's launch is shared by as many: a layer of 64 experts, routing here against there, 251 against 255 us of four layers for two tokens, 519 against
+// 495 for five.  And a slot's work-groups pick the experts of the places before theirs too, so up to 24 of a token (20 of banks of 4 bits, which
+// have less to wait for).  us of eight layers of 64 experts, chosen by the gate|up launch : by the
+// router's, width 2048 and 1024 wide experts, of 8 a token 324 : 358, 20 458 : 478, 24 490 : 511, 32 590 : 584, 64 1017 : 889; Q4_0 355 : 385, 480 : 486, 531 : 515, 625 : 579, 1069 : 828;
+// width 512 258 : 291, 297 : 321, 308 : 329, 356 : 356, 530 : 445; width 4096 365 : 407, 499 : 544, 563 : 591, 637 : 667, 1042 : 985.
+// Prompts: one launch whose work-groups read the router once a token.
+enum RouterForm { ROUTER_LAUNCHES = 0, ROUTER_FUSED = 1, ROUTER_IN_BANK = 2, ROUTER_ROWS = 3 };
+static int router_form(const cai_qw_s* router, const cai_qw_s* gateup, int E, int K, int I, int n_tok, bool prompt)
+{
+  if (router->rows != E) return ROUTER_LAUNCHES;
+  const bool one = router_fused_supported(router, K);
+  if (prompt) return one ? ROUTER_ROWS : ROUTER_LAUNCHES;
+  if (n_tok == 1 && K <= (gateup->qtype == CAI_Q8_0 ? 24 : 20) && router_in_launch() && gemv_routes(gateup, E, K) && gateup->rows == 2 * (int64_t)I * E) return ROUTER_IN_BANK;
+  return one ? ROUTER_FUSED : ROUTER_LAUNCHES;
+}
+
 // Expert half of a block for n_b (<= 8) activation rows x[b][d_model], in place: router -> soft-max -> top-k
 // gates -> gathered gate|up (RMSNorm and SwiGLU fused) -> gathered down -> gate-weighted mixture added to the row
 // (neural/neuralpretrained.pas:15331-15388; neural/neural.cl:2689-2752).
@@ -98,14 +116,12 @@ static int moe_ffn_rows(cai_decoder_s* d, const cai_decoder_s::Layer& L, float* 
   const int dm = c.d_model, I = c.ffn;
   int rc;
   const int E = c.n_experts, K = c.top_k;
-  // One token: the gate|up launch chooses the experts (every work-group its slot's) from logits that an ordinary product leaves.  For several the selection
-  // in the router's launch is shared by as many: a layer of 64 experts, routing here against there, 251 against 255 us of four layers for two tokens, 519 against
-  // 495 for five.
-  const bool routes = n_b == 1 && router_in_launch() && gemv_routes(L.w[CAI_W_GATEUP], E, K) && L.w[CAI_W_ROUTER]->rows == E && L.w[CAI_W_GATEUP]->rows == 2 * (int64_t)I * E;
+  const int form = router_form(L.w[CAI_W_ROUTER], L.w[CAI_W_GATEUP], E, K, I, n_b, false);
+  const bool routes = form == ROUTER_IN_BANK;
   if (routes) {
     MultiGemv r{}; r.n = 1; r.w[0] = L.w[CAI_W_ROUTER]; r.rows[0] = E;
     if ((rc = launch_gemv_multi(r, x, 1, d->router_logits, E, CAI_ACT_NONE, nullptr, L.v[CAI_V_MLP_NORM], c.eps, 0))) return rc;
-  } else if (router_fused_supported(L.w[CAI_W_ROUTER], K) && L.w[CAI_W_ROUTER]->rows == E && dm % 4 == 0) {
+  } else if (form == ROUTER_FUSED) {
     if ((rc = launch_router_fused(L.w[CAI_W_ROUTER], x, dm, L.v[CAI_V_MLP_NORM], c.eps, K, c.norm_topk, n_b, d->router_logits, d->moe_expert, d->moe_gate, d->router_probs, reinterpret_cast<unsigned*>(d->moe_expert + 8 * K)))) return rc;
   } else {
     MultiGemv r{}; r.n = 1; r.w[0] = L.w[CAI_W_ROUTER]; r.rows[0] = E;
@@ -394,7 +410,7 @@ static int moe_ffn_prompt(cai_decoder_s* d, const cai_decoder_s::Layer& L, int n
   const int dm = c.d_model, I = c.ffn, E = c.n_experts, K = c.top_k, slots = n * K;
   int rc;
   // (the router and the banks read the same normalised rows: one pre-pass where the router takes planes too, and none where its launch leaves them)
-  const bool rows = router_fused_supported(L.w[CAI_W_ROUTER], K) && L.w[CAI_W_ROUTER]->rows == E, shared_prep = !rows && prompt_route(L.w[CAI_W_ROUTER], n) == 2;
+  const bool rows = router_form(L.w[CAI_W_ROUTER], L.w[CAI_W_GATEUP], E, K, I, n, true) == ROUTER_ROWS, shared_prep = !rows && prompt_route(L.w[CAI_W_ROUTER], n) == 2;
   bool prepped = shared_prep;
   if (rows) {
     _Float16 *rhi = nullptr, *rlo = nullptr; float* rsinv = nullptr;
@@ -663,6 +679,17 @@ using namespace cai;
 // what a layered decoder has no use for
 #define NOT_LAYERED(d, name) \
   do { if ((d)->net) return set_error(CAI_ERR_UNSUPPORTED, name ": not available for a layered decoder"); } while (0)
+
+// For the tests of the rule; host only, not part of the interface in caihip.h.
+extern "C" int cai_router_form(int router_type, int bank_type, int experts, int top_k, int width, int ffn, int n_tok, int prompt)
+{
+  CAI_ENTER();
+  CAI_REQUIRE(experts >= 1 && top_k >= 1 && top_k <= experts && width >= 1 && ffn >= 1 && n_tok >= 1, "cai_router_form: bad argument");
+  cai_qw_s router{}, bank{};
+  router.qtype = router_type; router.rows = experts; router.cols = width;
+  bank.qtype = bank_type; bank.rows = 2 * (int64_t)ffn * experts; bank.cols = width;
+  return router_form(&router, &bank, experts, top_k, ffn, n_tok, prompt != 0);
+}
 
 extern "C" int cai_decoder_create(const cai_decoder_config* cfg, cai_decoder_t* out)
 {

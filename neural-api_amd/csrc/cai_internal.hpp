@@ -311,15 +311,15 @@ int argmax_scratch_entries(int n, int n_rows);
 int noalloc_setup(int device);   // resolves the device address of the fixed scratch array (cai_init, device current)
 int launch_embed(const cai_qw_s* w, const int32_t* tokens_dev, int n_tokens, float* out);
 int launch_router_topk(const float* logits, int n, int k, int renorm, int n_tokens, int32_t* expert_out, float* gate_out, float* probs_scratch);
+bool router_in_launch();      // (CAIHIP_ROUTER_LAUNCHES=1: product and selection stay launches of their own)
 // ... and the router's matrix-vector product, RMSNorm and selection in one launch (Q8_0 router rows, up to 64 experts)
-// ... for a prompt's tokens (router_fused_supported)
-bool router_rows_planes(const cai_qw_s* w);      // ... whether it leaves the normed rows as planes (hi not null)
-int launch_router_rows(const cai_qw_s* w, const float* x, int64_t x_stride, const float* gain, float eps, int k, int renorm, int n_tokens, int32_t* expert_out, float* gate_out,
-                       _Float16* hi, _Float16* lo, float* sinv);
-bool router_in_launch();
 bool router_fused_supported(const cai_qw_s* w, int k);
 int launch_router_fused(const cai_qw_s* w, const float* x, int64_t x_stride, const float* gain, float eps, int k, int renorm, int n_tokens,
                         float* logits_out, int32_t* expert_out, float* gate_out, float* probs_scratch, unsigned* counters);   // counters: one per token, zero before the first launch (they wrap back to zero)
+// ... the same for a prompt's tokens.  hi, lo and sinv (all three, or all null): the normed rows as operand planes, of rows up to 2048 wide (router_rows_planes).
+bool router_rows_planes(const cai_qw_s* w);
+int launch_router_rows(const cai_qw_s* w, const float* x, int64_t x_stride, const float* gain, float eps, int k, int renorm, int n_tokens, int32_t* expert_out, float* gate_out,
+                       _Float16* hi, _Float16* lo, float* sinv);
 int launch_rmsnorm_strided(const float* x, const float* gain, int n, int n_tokens, float eps, float* y, int64_t x_stride, int64_t y_stride);
 void decoder_adopt_weight(cai_decoder_s* d, cai_qw_s* w);   // the decoder destroys w with itself
 int launch_rmsnorm_pair(float* x, const float* gain_a, int n_a, const float* gain_b, int n_b, int n_tokens, float eps, int64_t stride);
