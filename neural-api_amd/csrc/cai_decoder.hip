@@ -96,13 +96,15 @@ static int check_ready(cai_decoder_s* d)
 // have less to wait for).  us of eight layers of 64 experts, chosen by the gate|up launch : by the
 // router's, width 2048 and 1024 wide experts, of 8 a token 324 : 358, 20 458 : 478, 24 490 : 511, 32 590 : 584, 64 1017 : 889; Q4_0 355 : 385, 480 : 486, 531 : 515, 625 : 579, 1069 : 828;
 // width 512 258 : 291, 297 : 321, 308 : 329, 356 : 356, 530 : 445; width 4096 365 : 407, 499 : 544, 563 : 591, 637 : 667, 1042 : 985.
-// Prompts: one launch whose work-groups read the router once a token.
+// Prompts: one launch whose work-groups read the router once a token.  Past 2048 columns the planes are a launch of their own all the same, and products on the matrix
+// cores, which read the router once a tile, catch up with more than 32 experts: four layers of 64 experts, one launch : three, width 2080 255 tokens 893 : 908, 400 1142 : 1123,
+// 2048 5094 : 5042; width 4096 255 1316 : 1340, 400 1651 : 1635, 2048 7207 : 7156; of 48 2048 tokens 7103 : 7053, of 32 4718 : 4796; width 2048, 64 experts, 1024 2204 : 2219, 2048 4488 : 4530.
 enum RouterForm { ROUTER_LAUNCHES = 0, ROUTER_FUSED = 1, ROUTER_IN_BANK = 2, ROUTER_ROWS = 3 };
 static int router_form(const cai_qw_s* router, const cai_qw_s* gateup, int E, int K, int I, int n_tok, bool prompt)
 {
   if (router->rows != E) return ROUTER_LAUNCHES;
   const bool one = router_fused_supported(router, K);
-  if (prompt) return one ? ROUTER_ROWS : ROUTER_LAUNCHES;
+  if (prompt) return one && (router_rows_planes(router) || E <= 32 || n_tok <= 256) ? ROUTER_ROWS : ROUTER_LAUNCHES;
   if (n_tok == 1 && K <= (gateup->qtype == CAI_Q8_0 ? 24 : 20) && router_in_launch() && gemv_routes(gateup, E, K) && gateup->rows == 2 * (int64_t)I * E) return ROUTER_IN_BANK;
   return one ? ROUTER_FUSED : ROUTER_LAUNCHES;
 }

@@ -256,6 +256,22 @@ def test_prompt_tokens_choose_their_experts(experts, top_k, norm_topk, d_model):
     dec.close()
 
 
+def test_long_prompts_on_both_sides_of_the_router_s_line():
+    """more than 32 experts of rows past 2048 columns: the router in one launch for 256 tokens, products on the matrix cores for one more"""
+    from helpers.device import dev, rel_err
+    cai = dev()
+    cfg = dict(n_layers=2, d_model=2080, n_q_heads=4, n_kv_heads=2, head_dim=64, ffn=96, vocab=300, max_ctx=320, eps=1e-5, rope_theta=1e4, n_experts=33, top_k=3, norm_topk=1)
+    spec = synthetic_spec(cfg, O.Q8_0, std=0.05)
+    om, dec = oracle_model(spec, acc64=1), cai.Decoder(spec)
+    toks = [int(t) for t in np.random.default_rng(33).integers(0, 300, 257)]
+    for p, t in enumerate(toks):
+        _, lo = om.step(t, p)
+        if p + 1 in (256, 257):
+            dec.reset()
+            assert rel_err(dec.prefill(toks[:p + 1], 0)[1], lo) < 1e-3, p
+    dec.close()
+
+
 @pytest.mark.parametrize("name,n", [("olmoe_like_q8", 11), ("olmoe_like_q8", 45), ("moe_like_q6k", 29)])
 def test_moe_prefill_equals_sequential_steps(name, n):
     """Mixture-of-experts prompts: attention half on the whole chunk, routed half per group of rows (router and top-k once

@@ -15,3 +15,11 @@ LAUNCHES, FUSED, IN_BANK, ROWS = range(4)
     (Q8_0, Q8_0, 64, 8, 2048, 2, FUSED), (Q8_0, Q8_0, 64, 64, 2048, 8, FUSED), (Q4_0, Q4_0, 64, 8, 2048, 2, LAUNCHES)])
 def test_how_a_step_finds_its_experts(router, bank, experts, top_k, width, n_tok, want):
     assert cai.load().cai_router_form(router, bank, experts, top_k, width, 1024, n_tok, 0) == want
+
+
+@pytest.mark.parametrize("router,experts,top_k,width,n_tok,want", [
+    # rows whose planes the launch leaves; longer ones of up to 32 experts, or of up to 256 tokens
+    (Q8_0, 64, 8, 2048, 2048, ROWS), (Q8_0, 64, 64, 512, 2048, ROWS), (Q8_0, 32, 8, 4096, 2048, ROWS), (Q8_0, 33, 8, 4096, 256, ROWS), (Q8_0, 33, 8, 4096, 257, LAUNCHES), (Q8_0, 64, 8, 2080, 2048, LAUNCHES),
+    (Q8_0, 65, 8, 2048, 100, LAUNCHES), (Q4_0, 64, 8, 2048, 100, LAUNCHES)])
+def test_how_a_prompt_finds_its_experts(router, experts, top_k, width, n_tok, want):
+    assert cai.load().cai_router_form(router, router, experts, top_k, width, 1024, n_tok, 1) == want
