@@ -272,6 +272,67 @@ def test_long_prompts_on_both_sides_of_the_router_s_line():
     dec.close()
 
 
+def router_rows_edit(spec, edit):
+    """edits the Q8_0 router rows (uint8 [experts][blocks][34]) of every layer"""
+    for (layer, slot), t in spec["tensors"].items():
+        if slot == O.W_ROUTER:
+            t["raw"] = np.array(t["raw"], np.uint8)
+            edit(t["raw"].reshape(t["rows"], -1, 34))
+
+
+@pytest.mark.parametrize("what", ["all alike", "pairs", "one is not a number"])
+@pytest.mark.parametrize("experts,top_k,norm_topk", [(64, 7, 0), (64, 7, 1), (9, 5, 1), (64, 23, 0), (64, 25, 1)])
+def test_equal_and_absent_scores_of_experts(what, experts, top_k, norm_topk):
+    """Experts whose scores are equal to the bit are taken in the order of their numbers, one whose score is no number last: one-token steps and prompts like the oracle, up to the places
+    that the gate|up launch picks and past them, and past what a prompt's router picks one by one."""
+    from helpers.device import dev, rel_err
+    cai = dev()
+    cfg = dict(n_layers=2, d_model=544, n_q_heads=4, n_kv_heads=2, head_dim=64, ffn=96, vocab=300, max_ctx=16, eps=1e-5, rope_theta=1e4, n_experts=experts, top_k=top_k, norm_topk=norm_topk)
+    spec = synthetic_spec(cfg, O.Q8_0, std=0.05, seed=experts + top_k)
+
+    def edit(r):
+        if what == "all alike":
+            r[:] = r[0]
+        elif what == "pairs":                # (an odd number of places: one pair is parted)
+            r[1::2] = r[0:len(r) // 2 * 2:2]
+        else:
+            r[3, 0, :2] = (0x00, 0x7e)
+    router_rows_edit(spec, edit)
+    om, dec = oracle_model(spec, acc64=1), cai.Decoder(spec)
+    toks, rows = [3, 14, 299, 0, 65, 35, 7], []
+    for p, t in enumerate(toks):
+        _, lo = om.step(t, p); _, ld = dec.step(t, p)
+        assert np.isfinite(lo).all() and rel_err(ld[0], lo) < 1e-3, (p, rel_err(ld[0], lo))
+        rows.append(lo)
+    for n in range(2, len(toks) + 1):
+        dec.reset()
+        assert rel_err(dec.prefill(toks[:n], 0)[1], rows[n - 1]) < 1e-3, n
+    dec.close()
+
+
+@pytest.mark.parametrize("top_k", [4, 24, 25])
+def test_a_poisoned_row_stays_inside_the_bank_and_leaves_the_next_sequence_alone(top_k):
+    """a token whose embedding is not a number reaches every router as scores that are none: its logits show it, in a step and in a prompt, and a sequence after it is the oracle's again"""
+    from helpers.device import dev, rel_err
+    cai = dev()
+    cfg = dict(n_layers=2, d_model=544, n_q_heads=4, n_kv_heads=2, head_dim=64, ffn=96, vocab=300, max_ctx=16, eps=1e-5, rope_theta=1e4, n_experts=64, top_k=top_k, norm_topk=1)
+    spec = synthetic_spec(cfg, O.Q8_0, std=0.05, seed=top_k)
+    e = spec["tensors"][(-1, O.W_EMBED)]
+    e["raw"] = np.array(e["raw"], np.uint8)
+    e["raw"].reshape(300, -1, 34)[7, 2, :2] = (0x00, 0x7e)
+    om, dec = oracle_model(spec, acc64=1), cai.Decoder(spec)
+    for poisoned in (lambda: dec.step(7, 0)[1][0], lambda: dec.prefill([5, 7], 0)[1], lambda: dec.prefill([3, 5, 9, 7], 0)[1]):
+        dec.reset()
+        assert np.isnan(poisoned()).all()
+    dec.reset()
+    for p, t in enumerate([3, 14, 299]):
+        _, lo = om.step(t, p); _, ld = dec.step(t, p)
+        assert rel_err(ld[0], lo) < 1e-3
+    dec.reset()
+    assert rel_err(dec.prefill([3, 14, 299], 0)[1], lo) < 1e-3
+    dec.close()
+
+
 @pytest.mark.parametrize("name,n", [("olmoe_like_q8", 11), ("olmoe_like_q8", 45), ("moe_like_q6k", 29)])
 def test_moe_prefill_equals_sequential_steps(name, n):
     """Mixture-of-experts prompts: attention half on the whole chunk, routed half per group of rows (router and top-k once
