@@ -443,14 +443,20 @@ def test_one_token_of_short_rows_that_share_a_wave(qt, rows, cols):
     w.close()
 
 
-@pytest.mark.parametrize("qt", [O.Q3_K, O.Q4_K, O.Q5_1])
-def test_decoder_whose_projections_share_waves(qt):
+SHARED = {"four rows": dict(n_layers=2, d_model=512, n_q_heads=24, n_kv_heads=6, head_dim=64, ffn=2304, vocab=2500),
+          "two rows": dict(n_layers=2, d_model=1280, n_q_heads=20, n_kv_heads=10, head_dim=64, ffn=2304, vocab=2500),
+          "four rows in three slices": dict(n_layers=1, d_model=2304, n_q_heads=64, n_kv_heads=32, head_dim=64, ffn=256, vocab=2500)}
+
+
+@pytest.mark.parametrize("shape", list(SHARED))
+@pytest.mark.parametrize("qt", [O.Q2_K, O.Q3_K, O.Q4_1, O.Q5_0, O.Q5_1, O.Q4_0, O.Q4_K, O.Q5_K])
+def test_decoder_whose_projections_share_waves(qt, shape):
+    """q | k | v, gate | up pairs and the head of decoders whose rows share a wave, in every type that does"""
     from helpers.device import dev, rel_err
     cai = dev()
-    cfg = dict(n_layers=2, d_model=512, n_q_heads=24, n_kv_heads=6, head_dim=64, ffn=2304, vocab=2500, max_ctx=48, eps=1e-5, rope_theta=1e4)
-    spec = synthetic_spec(cfg, qt, seed=77 + qt, std=0.05)
+    spec = synthetic_spec(dict(SHARED[shape], max_ctx=48, eps=1e-5, rope_theta=1e4), qt, seed=77 + qt, std=0.05)
     om, dec = oracle_model(spec, acc64=1), cai.Decoder(spec)
-    for p, t in enumerate([3, 2499, 17, 17, 250, 9]):
+    for p, t in enumerate([3, 2499, 17, 17, 250, 9][:3 if "slices" in shape else 6]):
         n_o, lo = om.step(t, p); am, ld = dec.step(t, p)
         assert rel_err(ld[0], lo) < TOL and int(am[0]) == n_o
     dec.close()
