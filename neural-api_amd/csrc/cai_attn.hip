@@ -4,10 +4,9 @@
 // appended to a head-major cache (row (g, p) at (g*MaxCtx + p)*Dk), then for each query head h (KV head
 // g = h / group) out_h = softmax(q_h . K_g / sqrt(Dk)) V_g over the live rows [jStart, len).
 //
-// Device formulation: split-K over the key axis; a slice of the live rows per work-group, a small second kernel
-// (one work-group per query head) merges the slices.  (Merging inside the first kernel through an arrival counter was
-// measured slower: every device-coherent hand-off between work-groups costs a memory round trip of ~2.5 us.)  RoPE of
-// q and of the new k row and the cache append happen inside the split kernel.  Two split kernels:
+// Device formulation: split-K over the key axis; a slice of the live rows per work-group, and the slices of a head merged by the last of its work-groups to
+// arrive (the per-head kernel: 8.0 + 4.9 -> 9.8 us on the 7B shape) or by a small second kernel, one work-group per query head (the kernels of a whole group of heads: merged in place 37.7 us on
+// the 32B shape, 21.5 + 5 so).  RoPE of q and of the new k row and the cache append happen inside the split kernel.  Two split kernels:
 //   attn_group_kernel       one work-group per (slice, KV head) serves the whole group of query heads, so K and V are
 //                           fetched once; three phases per slice (scores -> LDS, softmax, value sum).  Used when the
 //                           grid fills the chip by itself (long caches, several sequences, prompt ingestion).

@@ -105,9 +105,6 @@ __device__ __forceinline__ float ra_oct_sum(float v)
   v += RA_DPP(v, 0xb1); v += RA_DPP(v, 0x4e); v += RA_DPP(v, 0x141);
   return v;
 }
-// the value of lane ^ 8 (the other half of a 16-lane row: the hi / lo column of the same token)
-__device__ __forceinline__ float ra_ror8(float v) { return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xf, 0xf, false)); }
-__device__ __forceinline__ uint32_t ra_ror8(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, false); }
 }  // namespace
 
 // v_mfma_f32_16x16x32_f16: lane (m = lane % 16, kg = lane / 16) supplies 8 consecutive k of row m (A) / column m (B); the
@@ -485,7 +482,7 @@ __device__ __forceinline__ void ra_body(RA_ARGS, const int bx, const int n_bx, c
       return;
     }
     float inv = 1.0f;
-    if (GAIN) {   // (a product with a gain is one slice: the work-group has seen the whole row; every wave has passed this pair's barrier)
+    if (GAIN) {   // (a product with a gain is one slice: the work-group has seen the whole row, and its waves have met since)
       float t = 0.0f;
       for (int sb = 0; sb < nS; sb++) t += ssq_s[sb][tok];     // fixed order
       inv = 1.0f / sqrtf(t / (float)K + p.eps);
