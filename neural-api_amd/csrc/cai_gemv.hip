@@ -463,8 +463,10 @@ __global__ __launch_bounds__(256) void gemv_fast(const GemvParams p)
 // The leading scalar arguments are what these requests need of a launch of one matrix; they arrive preloaded (see the Makefile).
 // ------------------------------------------------------------------------------------------
 constexpr int BANK_NONE = 0, BANK_SLOTS = 1, BANK_ROUTED = 2;
-template <int QT, int R, int MODE, int BANK, int SV>
-__global__ __launch_bounds__(256) void gemv_one(const float* hx, const uint8_t* hw0, const uint8_t* haux0, const float* hgain, const float* hres, const int hcols, const int hrows0, const int hgrp0, const int hnseg, const std::conditional_t<BANK == BANK_ROUTED, GemvRouted, GemvParams> p)
+// P: GemvRouted where the launch chooses its experts, else GemvParams, as a parameter and not worked out in the signature: a type spelled there doubles the kernel's mangled name, and the
+// host pays for the names of a graph's nodes on every launch (151 of them, 135M shape: 574.9 us a step with names of 150 characters, 570.0 with 90).
+template <int QT, int R, int MODE, int BANK, int SV, class P>
+__global__ __launch_bounds__(256) void gemv_one(const float* hx, const uint8_t* hw0, const uint8_t* haux0, const float* hgain, const float* hres, const int hcols, const int hrows0, const int hgrp0, const int hnseg, const P p)
 {
   extern __shared__ float4 xs4[];          // [kp/4]
   const unsigned long long tl0 = timeline_now();
@@ -819,8 +821,8 @@ static int launch_fast_r(const GemvParams& p0, const GemvRoute* route, int n_gro
       constexpr int BANK = decltype(bank)::value;
       constexpr int SV = decltype(sv)::value;
       auto args = [&] { if constexpr (BANK == BANK_ROUTED) return GemvRouted{p, *route}; else return p; }();
-      if constexpr (MODE == 0) { if (R == 4) { go(gemv_one<QT, 4, MODE, BANK, SV>, args); return; } }
-      if (R == 2) go(gemv_one<QT, 2, MODE, BANK, SV>, args); else go(gemv_one<QT, 1, MODE, BANK, SV>, args);
+      if constexpr (MODE == 0) { if (R == 4) { go(gemv_one<QT, 4, MODE, BANK, SV, decltype(args)>, args); return; } }
+      if (R == 2) go(gemv_one<QT, 2, MODE, BANK, SV, decltype(args)>, args); else go(gemv_one<QT, 1, MODE, BANK, SV, decltype(args)>, args);
     };
     auto width = [&](auto bank) {
       using std::integral_constant;
