@@ -826,7 +826,8 @@ int launch_q4k_dot(GemvParams& p, const MultiGemv& m, int swiglu_half, hipStream
   // Up to 8 super-blocks a wave of one row has half its lanes (and requests) idle: two or four whole rows to a wave, where there are more rows than
   // waves (below that a launch is one row a wave either way, and this many work-groups fewer).  us, one row | so: 32000 x 2048 Q3_K 17.4 | 11.7, Q2_K 16.0 | 9.7,
   // Q4_1 13.6 | 8.9, Q5_1 16.3 | 10.4, Q4_K 11.3 | 7.2, Q4_0 10.4 | 7.0, Q5_K 14.3 | 10.4; 49152 x 1024, four rows: 24.6 | 9.3, 22.5 | 7.9, 19.2 | 7.4, 23.0 | 8.4, 15.3 | 5.8, 13.7 | 5.3,
-  // 19.5 | 7.6 (two: 14.7, 12.9, 11.2, 13.2, 8.9, 8.1, 11.1); 11008 x 2048 Q4_K 5.9 | 4.6; 4096 x 2048 Q3_K 5.0 | 4.5; 2304 to 3000 rows the same.
+  // 19.5 | 7.6 (two: 14.7, 12.9, 11.2, 13.2, 8.9, 8.1, 11.1); 11008 x 2048 Q4_K 5.9 | 4.6; 4096 x 2048 Q3_K 5.0 | 4.5.  From the
+  // first row past the waves on (by trace, Q3_K, one | two | four): 2049 x 1024 5.3 | 4.9 | 4.9, 4096 x 1024 5.8 | 5.0 | 5.0, 8192 x 1024 7.7 | 5.9 | 5.2, 2560 x 2048 5.8 | 5.1 | 5.0; Q4_K, Q4_0 and Q5_1 alike.
   // 9 to 12 super-blocks: three slices of four, four rows, from two turns of that on: 32000 x 2304 Q3_K 17.6 | 15.1, Q4_K 11.4 | 9.5; 8192 x 2560 7.1 | 6.7, 5.2 | 4.7;
   // 14336 x 3072 9.7 | 9.4, 7.4 | 6.0 (3072 x 3072 Q3_K 5.3 | 5.8; pairs of gate and up rows, a step of six layers Q3_K 306 | 294, Q4_1 267 | 271: one row).
   const int pkw = q6k ? 1 : nsb > 16 ? (nsb <= 24 ? 4 : 1) : nsb <= 8 && total > (int64_t)c.n_cu * 8 ? (nsb <= 4 ? 4 : 2) : nsb > 8 && nsb <= 12 && !swiglu_half && total >= (int64_t)c.n_cu * 32 ? 4 : 1;
